@@ -179,6 +179,8 @@ MIXERS_SIGNATURES = {
     "aphro_silu_gate_part_rms_norm": (I, [P, L, P, P, L, P, L, I, I, F, F, I, P]),
     "aphro_qk_row_norm_kv_write": (I, [P, L, P, P, P, L, P, L, P, L, P, L, P, P, L, I, I, I, F, I, P]),
     "aphro_outer_memory_scan": (I, [P, P, L, P, L, P, L, P, P, L, P, P, P, P, I, P, P, P, I, L, I, I, I, I, P, F, F, I, P, P, P, I, I, P]),
+    "aphro_outer_memory_chunked_workspace": (L, [I, L, I, I, I, I, I]),
+    "aphro_outer_memory_chunked": (I, [P, P, L, P, L, P, L, P, P, L, P, P, P, P, I, P, P, P, I, L, I, I, I, I, P, F, F, I, P, P, P, I, P, L, I, P]),
     "aphro_depth_residual_rms_norm": (I, [P, P, P, L, P, L, I, P, F, P, P, L, I, F, I, P]),
     "aphro_poly_norm": (I, [P, P, L, L, I, F, F, F, F, F, I, P]),
     "aphro_differential_norm_gate": (I, [P, L, P, L, P, L, L, I, I, I, F, F, F, I, P]),

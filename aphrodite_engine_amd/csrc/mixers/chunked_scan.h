@@ -1,0 +1,107 @@
+// Helpers of the recurrences that run in chunks of 64 tokens (outer_memory_chunked.hip, delta_rule_chunked.hip): which chunk a
+// workgroup owns, cumulative log decays, 16-byte loads, fp32 matrix-core products.
+#pragma once
+#include "mixers_common.h"
+
+namespace aphro {
+
+constexpr int CHUNK = 64;
+
+// fp32 product on the matrix cores: D[i][j] += sum over four k of A[i][k] B[k][j].  Lane l gives A[l % 16][k] and B[k][l % 16] for k =
+// l / 16 and holds D[4 (l / 16) + r][l % 16].  Which four of the k a call covers is the caller's choice as long as A and B agree:
+// here lane group g = l / 16 brings four (or eight) NEIGHBOURING k per load and one of them per call.
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+__device__ __forceinline__ int wave_incl_sum(int v, int lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(v, o, 64);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
+
+__device__ __forceinline__ int chunks_of(int n, int min_len) { return n >= min_len ? (n + CHUNK - 1) / CHUNK : 0; }
+
+// Chunk ``id`` of the batch's segments of at least min_len tokens, counted in order -> segment s and chunk c of it; false: there are
+// fewer.  Every wave of a workgroup works it out for itself (64 segments a step).
+__device__ __forceinline__ bool locate_chunk(int id, const int32_t* __restrict__ q_len, int num_seqs, int min_len, int& s, int& c) {
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  for (int s0 = 0; s0 < num_seqs; s0 += 64) {
+    const int cnt = s0 + lane < num_seqs ? chunks_of(q_len[s0 + lane], min_len) : 0;
+    const int incl = wave_incl_sum(cnt, lane) + before;
+    const uint64_t past = __ballot(incl > id);
+    if (past) {
+      const int l = __ffsll((unsigned long long)past) - 1;
+      s = __builtin_amdgcn_readfirstlane(s0 + l);
+      c = __builtin_amdgcn_readfirstlane(id - (__shfl(incl, l, 64) - __shfl(cnt, l, 64)));
+      return true;
+    }
+    before = __shfl(incl, 63, 64);
+  }
+  return false;
+}
+
+// Number of chunks ahead of segment s.
+__device__ __forceinline__ int chunks_before(int s, const int32_t* __restrict__ q_len, int min_len) {
+  const int lane = threadIdx.x & 63;
+  int sum = 0;
+  for (int s0 = 0; s0 < s; s0 += 64) sum += __shfl(wave_incl_sum(s0 + lane < s ? chunks_of(q_len[s0 + lane], min_len) : 0, lane), 63, 64);
+  return __builtin_amdgcn_readfirstlane(sum);
+}
+
+// The most chunks that num_tokens rows in num_seqs segments can hold.
+inline int64_t max_chunks(int64_t num_tokens, int num_seqs, int min_len) {
+  const int64_t longs = num_tokens / min_len;
+  return num_tokens / CHUNK + (longs < num_seqs ? longs : num_seqs);
+}
+
+// Inclusive prefix sum over the wave, in 64 bits: differences of two prefixes keep a small decay exact behind a large one.
+__device__ __forceinline__ double wave_incl_sum(double v, int lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double u = __shfl_up(v, o, 64);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
+
+// 2^t for a difference of two prefixes.  Rounding t to fp32 costs |t| 2^-24 of a factor of size 2^t: half an ulp of one at the most.
+__device__ __forceinline__ float exp2_d(double t) { return __builtin_amdgcn_exp2f((float)t); }
+
+// A log decay as it enters a prefix: in units of ln 2, and finite (2^-1e5 is zero however it is split).
+__device__ __forceinline__ double log2_decay(float la) { return 1.4426950408889634 * (double)(la < -1e5f ? -1e5f : la); }
+
+// Eight neighbouring numbers of a row, as fp32; zeros from ``limit`` on.  VEC: the address is a multiple of 16 bytes and the row's
+// length a multiple of eight.
+template <typename T, bool VEC>
+__device__ __forceinline__ void load8(const typename T::storage* __restrict__ row, int at, int limit, float (&x)[8]) {
+  if constexpr (VEC) {
+    if (at < limit) {
+      if constexpr (sizeof(typename T::storage) == 2) {
+        const u16x8 w = *reinterpret_cast<const u16x8*>(row + at);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = T::to_f32(w[i]);
+      } else {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(row + at), b = *reinterpret_cast<const f32x4*>(row + at + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = a[i], x[4 + i] = b[i];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = 0.f;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = at + i < limit ? T::to_f32(row[at + i]) : 0.f;
+  }
+}
+
+inline bool rows_of_16_bytes(const void* p, int64_t stride, int head, int elem) {
+  return ((uintptr_t)p & 15) == 0 && (stride * elem) % 16 == 0 && head % 8 == 0;
+}
+
+__device__ __forceinline__ bool finite_f(float x) { return fabsf(x) <= 3.402823466e38f; }
+
+}  // namespace aphro

@@ -14,7 +14,7 @@
 // their activations applied (the next 16 tokens' raw values are already in flight in registers), the per-token partial dot products are folded over the slices with DPP moves.  The
 // mLSTM gate recurrence of a 16-token stage runs in wave 0 (lane = token for the transcendental parts, a 16-step max-plus
 // loop for m) before the stage is released to all waves.
-#include "mixers_common.h"
+#include "outer_memory.h"
 
 namespace aphro {
 
@@ -27,7 +27,7 @@ __global__ __launch_bounds__(256) void outer_memory_scan_kernel(
     const typename T::storage* __restrict__ gate_i, const typename T::storage* __restrict__ gate_f, int64_t gate_stride,
     float* __restrict__ state_s, float* __restrict__ state_n, float* __restrict__ state_m,
     const int32_t* __restrict__ slot_of_seq, int num_slots, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ q_len, const int32_t* __restrict__ ctx_len, int heads, int dim, int vdim,
+    const int32_t* __restrict__ q_len, const int32_t* __restrict__ ctx_len, int below, int heads, int dim, int vdim,
     const float* __restrict__ decay, float q_scale, float gate_cap, int qk_heads, const float* __restrict__ a_log,
     const float* __restrict__ dt_bias, const float* __restrict__ skip) {
   constexpr int NS = 1 << SLOG;        // slices of the key dimension = lanes that share a column
@@ -43,7 +43,7 @@ __global__ __launch_bounds__(256) void outer_memory_scan_kernel(
   const int hq = MODE == 2 ? h / (heads / qk_heads) : h;    // head of q and k
   const int n = q_len[s];
   const int slot = slot_of_seq[s];
-  if (n <= 0 || slot < 0 || slot >= num_slots) return;
+  if (n <= 0 || n >= below || slot < 0 || slot >= num_slots) return;
   const int64_t t0 = q_start[s];
   const bool fresh = ctx_len[s] == 0;
   float S[DPT], nv[DPT];
@@ -175,6 +175,55 @@ __global__ __launch_bounds__(256) void outer_memory_scan_kernel(
     for (int cp = 0; cp < TW / 16 && copy0 + cp < ncopy; ++cp) mptr[cp] = m;
 }
 
+int outer_memory_check(const OuterMemory& p) {
+  APHRO_CHECK(p.out && p.q && p.k && p.v && p.state_s && p.slot_of_seq && p.q_start && p.q_len && p.ctx_len, "outer_memory_scan: null argument");
+  APHRO_CHECK(p.mode >= 0 && p.mode <= 2, "outer_memory_scan: mode %d", p.mode);
+  APHRO_CHECK(p.qk_heads > 0 && p.heads % p.qk_heads == 0 && (p.mode == 2 || p.qk_heads == p.heads), "outer_memory_scan: %d heads over %d query/key heads", p.heads, p.qk_heads);
+  APHRO_CHECK(p.mode == 0 ? p.decay != nullptr : p.mode == 2 ? (p.gate_i && p.a_log && p.dt_bias && p.skip && p.gate_stride >= p.heads) : (p.gate_i && p.gate_f && p.state_n && p.state_m && p.gate_cap > 0.f && p.gate_stride >= p.heads),
+              "outer_memory_scan: mode %d lacks its gate arguments", p.mode);
+  APHRO_CHECK(p.heads > 0 && p.heads <= 65535 && p.dim > 0 && p.dim <= 256 && p.vdim > 0 && p.vdim <= 64 * 65535 && p.num_slots > 0 && p.num_seqs > 0,
+              "outer_memory_scan: heads %d dim %d (<= 256) vdim %d", p.heads, p.dim, p.vdim);
+  APHRO_CHECK(p.q_stride >= (int64_t)p.qk_heads * p.dim && p.k_stride >= (int64_t)p.qk_heads * p.dim && p.v_stride >= (int64_t)p.heads * p.vdim,
+              "outer_memory_scan: row strides smaller than the rows");
+  return APHRO_OK;
+}
+
+// Prompt portions: 16 lanes per value column (16 columns per workgroup), so that a long sequential scan spreads over four
+// times as many waves with a quarter of the work per token and lane.  Single tokens: 4 lanes per column (64 columns per
+// workgroup), whose state loads and stores come in 64-byte pieces.
+int outer_memory_scan_launch(const OuterMemory& p, int below, bool wide) {
+  const int tw = wide ? 16 : 64;
+  const dim3 grid((unsigned)p.num_seqs, (unsigned)p.heads, (unsigned)((p.vdim + tw - 1) / tw));
+#define OMS_LAUNCH(MODE, DPT, SLOG)                                                                                         \
+  hipLaunchKernelGGL((outer_memory_scan_kernel<T, MODE, DPT, SLOG>), grid, dim3(256), 0, p.stream, p.out, (const S*)p.q,         \
+                     p.q_stride, (const S*)p.k, p.k_stride, (const S*)p.v, p.v_stride, (const S*)p.gate_i, (const S*)p.gate_f, p.gate_stride, \
+                     p.state_s, p.state_n, p.state_m, p.slot_of_seq, p.num_slots, p.q_start, p.q_len, p.ctx_len, below, p.heads, p.dim, p.vdim, \
+                     p.decay, p.q_scale, p.gate_cap, p.qk_heads, p.a_log, p.dt_bias, p.skip)
+#define OMS_BY_DIM(MODE)                               \
+  do {                                                 \
+    if (wide) {                                        \
+      if (p.dim <= 64) OMS_LAUNCH(MODE, 4, 4);         \
+      else if (p.dim <= 128) OMS_LAUNCH(MODE, 8, 4);   \
+      else OMS_LAUNCH(MODE, 16, 4);                    \
+    } else if (p.dim <= 32) OMS_LAUNCH(MODE, 8, 2);    \
+    else if (p.dim <= 48) OMS_LAUNCH(MODE, 12, 2);     \
+    else if (p.dim <= 64) OMS_LAUNCH(MODE, 16, 2);     \
+    else if (p.dim <= 96) OMS_LAUNCH(MODE, 24, 2);     \
+    else if (p.dim <= 128) OMS_LAUNCH(MODE, 32, 2);    \
+    else OMS_LAUNCH(MODE, 64, 2);                      \
+  } while (0)
+  MIX_DISPATCH_DTYPE(p.dtype, {
+    typedef typename T::storage S;
+    if (p.mode == 0) OMS_BY_DIM(0);
+    else if (p.mode == 1) OMS_BY_DIM(1);
+    else OMS_BY_DIM(2);
+  });
+#undef OMS_BY_DIM
+#undef OMS_LAUNCH
+  APHRO_LAUNCH_CHECK();
+  return APHRO_OK;
+}
+
 }  // namespace aphro
 
 using namespace aphro;
@@ -188,47 +237,9 @@ extern "C" int aphro_outer_memory_scan(float* out, const void* q, int64_t q_stri
                                        const float* a_log, const float* dt_bias, const float* skip, int max_q_len, int dtype,
                                        void* stream) {
   if (num_tokens == 0 || num_seqs == 0) return APHRO_OK;
-  APHRO_CHECK(out && q && k && v && state_s && slot_of_seq && q_start && q_len && ctx_len, "outer_memory_scan: null argument");
-  APHRO_CHECK(mode >= 0 && mode <= 2, "outer_memory_scan: mode %d", mode);
-  APHRO_CHECK(qk_heads > 0 && heads % qk_heads == 0 && (mode == 2 || qk_heads == heads), "outer_memory_scan: %d heads over %d query/key heads", heads, qk_heads);
-  APHRO_CHECK(mode == 0 ? decay != nullptr : mode == 2 ? (gate_i && a_log && dt_bias && skip && gate_stride >= heads) : (gate_i && gate_f && state_n && state_m && gate_cap > 0.f && gate_stride >= heads),
-              "outer_memory_scan: mode %d lacks its gate arguments", mode);
-  APHRO_CHECK(heads > 0 && heads <= 65535 && dim > 0 && dim <= 256 && vdim > 0 && vdim <= 64 * 65535 && num_slots > 0 && num_seqs > 0,
-              "outer_memory_scan: heads %d dim %d (<= 256) vdim %d", heads, dim, vdim);
-  APHRO_CHECK(q_stride >= (int64_t)qk_heads * dim && k_stride >= (int64_t)qk_heads * dim && v_stride >= (int64_t)heads * vdim,
-              "outer_memory_scan: row strides smaller than the rows");
-  // Prompt portions: 16 lanes per value column (16 columns per workgroup), so that a long sequential scan spreads over four
-  // times as many waves with a quarter of the work per token and lane.  Single tokens: 4 lanes per column (64 columns per
-  // workgroup), whose state loads and stores come in 64-byte pieces.
-  const bool wide = max_q_len >= 32;
-  const int tw = wide ? 16 : 64;
-  const dim3 grid((unsigned)num_seqs, (unsigned)heads, (unsigned)((vdim + tw - 1) / tw));
-#define OMS_LAUNCH(MODE, DPT, SLOG)                                                                                         \
-  hipLaunchKernelGGL((outer_memory_scan_kernel<T, MODE, DPT, SLOG>), grid, dim3(256), 0, (hipStream_t)stream, out, (const S*)q, \
-                     q_stride, (const S*)k, k_stride, (const S*)v, v_stride, (const S*)gate_i, (const S*)gate_f, gate_stride, \
-                     state_s, state_n, state_m, slot_of_seq, num_slots, q_start, q_len, ctx_len, heads, dim, vdim, decay,     \
-                     q_scale, gate_cap, qk_heads, a_log, dt_bias, skip)
-#define OMS_BY_DIM(MODE)                               \
-  do {                                                 \
-    if (wide) {                                        \
-      if (dim <= 64) OMS_LAUNCH(MODE, 4, 4);           \
-      else if (dim <= 128) OMS_LAUNCH(MODE, 8, 4);     \
-      else OMS_LAUNCH(MODE, 16, 4);                    \
-    } else if (dim <= 32) OMS_LAUNCH(MODE, 8, 2);      \
-    else if (dim <= 48) OMS_LAUNCH(MODE, 12, 2);       \
-    else if (dim <= 64) OMS_LAUNCH(MODE, 16, 2);       \
-    else if (dim <= 96) OMS_LAUNCH(MODE, 24, 2);       \
-    else if (dim <= 128) OMS_LAUNCH(MODE, 32, 2);      \
-    else OMS_LAUNCH(MODE, 64, 2);                      \
-  } while (0)
-  MIX_DISPATCH_DTYPE(dtype, {
-    typedef typename T::storage S;
-    if (mode == 0) OMS_BY_DIM(0);
-    else if (mode == 1) OMS_BY_DIM(1);
-    else OMS_BY_DIM(2);
-  });
-#undef OMS_BY_DIM
-#undef OMS_LAUNCH
-  APHRO_LAUNCH_CHECK();
-  return APHRO_OK;
+  const OuterMemory p = {out, q, k, v, gate_i, gate_f, q_stride, k_stride, v_stride, gate_stride, state_s, state_n, state_m, slot_of_seq,
+                         num_slots, q_start, q_len, ctx_len, num_seqs, num_tokens, heads, dim, vdim, mode, decay, q_scale, gate_cap, qk_heads,
+                         a_log, dt_bias, skip, max_q_len, dtype, (hipStream_t)stream};
+  const int rc = outer_memory_check(p);
+  return rc != APHRO_OK ? rc : outer_memory_scan_launch(p, 0x7fffffff, max_q_len >= 32);
 }

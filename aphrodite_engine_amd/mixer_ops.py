@@ -254,6 +254,15 @@ def memory_state_shapes(slots: int, heads: int, dim: int, vdim: int, mode: int):
     return (s, ) if mode != MEMORY_MLSTM else (s, (slots, heads, tiles, dim), (slots, heads, tiles))
 
 
+# A batch whose longest segment has at least MEMORY_CHUNKED_FROM tokens runs its segments of MEMORY_CHUNKED_MIN and more in chunks of 64 on the
+# matrix cores, and token by token what is shorter; any other batch is scanned.  One segment, scan / chunks in us: 64 tokens 21 / 24 (decay), 33 / 34
+# (mLSTM), 23 / 33 (state space); 96 tokens 30 / 24, 47 / 35, 33 / 34; where the launches are made anyway, shorter segments cost little in them
+# and would keep the token form's wide split, which single tokens beside them are slower in.  The chunked forms keep every chunk's state for
+# the length of the call; a batch that would need more than the bound is scanned.
+MEMORY_CHUNKED_FROM, MEMORY_CHUNKED_MIN = 96, 32
+CHUNKED_WORKSPACE_MAX = 8 << 30
+
+
 def outer_memory_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state, slot_of_seq: torch.Tensor,
                       q_start: torch.Tensor, q_len: torch.Tensor, ctx_len: torch.Tensor, heads: int, mode: int,
                       decay: Optional[torch.Tensor] = None, gate_i: Optional[torch.Tensor] = None,
@@ -290,13 +299,19 @@ def outer_memory_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state, 
         gs = _rows(gate_i, heads, "gate_i")
         _need(_rows(gate_f, heads, "gate_f") == gs, "outer_memory_scan: the two gates share a row stride")
     out = torch.empty(T, heads * e, dtype=torch.float32, device=q.device)
-    check(_lib.mixers_lib().aphro_outer_memory_scan(
-        out.data_ptr(), q.data_ptr(), _rows(q, qk_heads * d, "q"), k.data_ptr(), _rows(k, qk_heads * d, "k"), v.data_ptr(),
-        _rows(v, heads * e, "v"), _p(gate_i), _p(gate_f), gs, state[0].data_ptr(),
-        state[1].data_ptr() if len(state) > 1 else None, state[2].data_ptr() if len(state) > 2 else None,
-        slot_of_seq.data_ptr(), slots, q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(), S, T, heads, d, e, int(mode),
-        _p(decay), float(q_scale), float(gate_cap), qk_heads, _p(a_log), _p(dt_bias), _p(skip), int(max_q_len), _dt(q), _stream()),
-        "outer_memory_scan")
+    lib = _lib.mixers_lib()
+    args = (out.data_ptr(), q.data_ptr(), _rows(q, qk_heads * d, "q"), k.data_ptr(), _rows(k, qk_heads * d, "k"), v.data_ptr(),
+            _rows(v, heads * e, "v"), _p(gate_i), _p(gate_f), gs, state[0].data_ptr(),
+            state[1].data_ptr() if len(state) > 1 else None, state[2].data_ptr() if len(state) > 2 else None,
+            slot_of_seq.data_ptr(), slots, q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(), S, T, heads, d, e, int(mode),
+            _p(decay), float(q_scale), float(gate_cap), qk_heads, _p(a_log), _p(dt_bias), _p(skip))
+    if max_q_len >= MEMORY_CHUNKED_FROM and d <= 128 and S <= 65535:
+        need = lib.aphro_outer_memory_chunked_workspace(S, T, heads, d, e, int(mode), MEMORY_CHUNKED_MIN)
+        if need <= CHUNKED_WORKSPACE_MAX:
+            ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
+            check(lib.aphro_outer_memory_chunked(*args, MEMORY_CHUNKED_MIN, ws.data_ptr(), need, _dt(q), _stream()), "outer_memory_scan")
+            return out
+    check(lib.aphro_outer_memory_scan(*args, int(max_q_len), _dt(q), _stream()), "outer_memory_scan")
     return out
 
 

@@ -123,6 +123,18 @@ int aphro_outer_memory_scan(float* out, const void* q, int64_t q_stride, const v
                             int64_t num_tokens, int heads, int dim, int vdim, int mode, const float* decay, float q_scale,
                             float gate_cap, int qk_heads, const float* a_log, const float* dt_bias, const float* skip, int max_q_len, int dtype, void* stream);
 
+/* The same with segments of at least min_len tokens in chunks of 64 on the matrix cores (fp32 products); shorter ones token by token; a
+ * single segment always in chunks.  dim <= 128, num_seqs <= 65535.  workspace: 16-byte aligned, of at least
+ * aphro_outer_memory_chunked_workspace(...) bytes (0: sizes that are not served), in use until the stream has passed the call. */
+int64_t aphro_outer_memory_chunked_workspace(int num_seqs, int64_t num_tokens, int heads, int dim, int vdim, int mode, int min_len);
+int aphro_outer_memory_chunked(float* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                               int64_t v_stride, const void* gate_i, const void* gate_f, int64_t gate_stride, float* state_s,
+                               float* state_n, float* state_m, const int32_t* slot_of_seq, int num_slots,
+                               const int32_t* q_start, const int32_t* q_len, const int32_t* ctx_len, int num_seqs,
+                               int64_t num_tokens, int heads, int dim, int vdim, int mode, const float* decay, float q_scale,
+                               float gate_cap, int qk_heads, const float* a_log, const float* dt_bias, const float* skip, int min_len,
+                               float* workspace, int64_t workspace_bytes, int dtype, void* stream);
+
 /* ---- an fp32 residual stream joined over depth, scalar-gain RMS norm ---------------------------------------------------
  * One launch, every step optional:
  *   1. r = x_in + y                                       y [T, width] of `dtype` (row stride y_stride), NULL: r = x_in

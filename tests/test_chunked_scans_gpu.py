@@ -1,0 +1,125 @@
+"""The recurrences in chunks of 64 tokens against plain 64-bit recurrences, at the edges of chunks and tiles: lengths about 16, 32 and 64,
+several segments of one batch, states carried in, rows that are not 16-byte aligned, numbers that are not finite."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def mops():
+    from aphrodite_engine_amd import mixer_ops
+    return mixer_ops
+
+
+def i32(xs):
+    return torch.tensor(list(xs), dtype=torch.int32, device=DEV)
+
+
+def part(g, rows, cols, dtype, pad):
+    """Random rows behind ``pad`` other columns of a wider tensor."""
+    return torch.randn(rows, cols + pad, generator=g, device=DEV).to(dtype)[:, pad:]
+
+
+def memory_reference(mops, mode, q, k, v, S, n, m, decay, gi, gf, q_scale, cap, a_log, dt_bias, skip):
+    """One head, one segment, token by token in 64 bits."""
+    out = torch.empty(v.shape, dtype=torch.float64)
+    silu = torch.nn.functional.silu
+    for t in range(q.shape[0]):
+        qt, kt, vt, den = q[t], k[t], v[t], 1.0
+        if mode == mops.MEMORY_DECAY:
+            qt, kt, vt, a, b = silu(qt), silu(kt), silu(vt), decay, 1.0
+        elif mode == mops.MEMORY_MLSTM:
+            i, f = cap * torch.tanh(gi[t] / cap), torch.nn.functional.logsigmoid(cap * torch.tanh(gf[t] / cap))
+            now = max(float(f) + m, float(i))
+            a, b, m = np.exp(float(f) + m - now), np.exp(float(i) - now), now
+            qt = qt * q_scale
+            n = a * n + b * kt
+            den = max(abs(float(n @ qt)), np.exp(-m)) + 1e-6
+        else:
+            dt = torch.nn.functional.softplus(gi[t] + dt_bias)
+            a, b = torch.exp(-torch.exp(a_log) * dt), dt
+        S = a * S + b * kt[:, None] * vt[None, :]
+        out[t] = S.T @ qt / den + (skip * vt if mode == mops.MEMORY_STATE_SPACE else 0.0)
+    return out, S, n, m
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("dtype,pad", [(torch.bfloat16, 0), (torch.bfloat16, 3), (torch.float32, 4)])
+@pytest.mark.parametrize("d,e", [(64, 128), (128, 64), (24, 72), (100, 20)])
+def test_memory_chunks(mops, mode, dtype, pad, d, e):
+    H, lens, ctx = 2, [64, 1, 33, 129, 31], [0, 7, 5, 0, 9]
+    g = torch.Generator(device=DEV).manual_seed(d * 3 + e + mode)
+    T, S = sum(lens), len(lens)
+    q, k, v = part(g, T, H * d, dtype, pad), part(g, T, H * d, dtype, pad), part(g, T, H * e, dtype, pad)
+    gates = torch.randn(T, 2 * H + 1, generator=g, device=DEV).to(dtype)
+    gi, gf = gates[:, 1:H + 1], gates[:, H + 1:]
+    decay = torch.tensor([0.97, -0.8], device=DEV)
+    a_log, dt_bias, skip = (torch.randn(H, generator=g, device=DEV) for _ in range(3))
+    state = tuple(torch.randn(s, generator=g, device=DEV) for s in mops.memory_state_shapes(S + 1, H, d, e, mode))
+    if mode == mops.MEMORY_MLSTM:                       # every 16 columns hold the same n and m
+        state[1][:], state[2][:] = state[1][:, :, :1].clone(), state[2][:, :, :1].abs().clone()
+    slots, start = [3, 5, 0, 2, 4], np.concatenate([[0], np.cumsum(lens)[:-1]])
+    before = [s.double().cpu() for s in state]
+    kw = {0: dict(decay=decay), 1: dict(gate_i=gi, gate_f=gf, q_scale=d ** -0.5, gate_cap=6.0),
+          2: dict(gate_i=gi, a_log=a_log, dt_bias=dt_bias, skip=skip)}[mode]
+    out = mops.outer_memory_scan(q, k, v, state, i32(slots), i32(start), i32(lens), i32(ctx), H, mode, max_q_len=max(lens), **kw)
+    Q, K, V, GI, GF = (x.double().cpu() for x in (q, k, v, gi, gf))
+    for s in range(S):
+        rows = slice(start[s], start[s] + lens[s])
+        for h in range(H):
+            S0 = before[0][slots[s], h] if ctx[s] else torch.zeros(d, e, dtype=torch.float64)
+            n0, m0 = torch.zeros(d, dtype=torch.float64), 0.0
+            if mode == mops.MEMORY_MLSTM and ctx[s]:
+                n0, m0 = before[1][slots[s], h, 0], float(before[2][slots[s], h, 0])
+            want, Sw, nw, mw = memory_reference(
+                mops, mode, Q[rows, h * d:(h + 1) * d], K[rows, h * d:(h + 1) * d], V[rows, h * e:(h + 1) * e], S0, n0, m0, float(decay[h]),
+                GI[rows, h], GF[rows, h], d ** -0.5, 6.0, float(a_log[h]) * torch.ones((), dtype=torch.float64), float(dt_bias[h]), float(skip[h]))
+            got = out[rows, h * e:(h + 1) * e].double().cpu()
+            # fp32 sums of up to 129 + d products behind a few exponentials of 1 ulp; silu and the mLSTM's division as the scan has them
+            assert torch.allclose(got, want, rtol=1e-4, atol=3e-5 * float(want.abs().max())), (s, h, (got - want).abs().max())
+            assert torch.allclose(state[0][slots[s], h].double().cpu(), Sw, rtol=1e-4, atol=3e-5 * float(Sw.abs().max()))
+            if mode == mops.MEMORY_MLSTM:
+                for c in range(state[1].shape[2]):
+                    assert torch.allclose(state[1][slots[s], h, c].double().cpu(), nw, rtol=1e-4, atol=3e-5 * float(nw.abs().max()))
+                    assert abs(float(state[2][slots[s], h, c]) - mw) < 1e-4 * max(1.0, abs(mw))
+    assert torch.equal(state[0][1].double().cpu(), before[0][1])          # a slot that no segment names
+
+
+def test_memory_chunks_long_gates(mops):
+    """More tokens than the gate launch folds at a time; strong and weak decays in turn."""
+    T, H, d, e = 4096 + 77, 1, 16, 16
+    g = torch.Generator(device=DEV).manual_seed(5)
+    q, k, v = part(g, T, d, torch.float32, 0), part(g, T, d, torch.float32, 0), part(g, T, e, torch.float32, 0)
+    gi, gf = part(g, T, 1, torch.float32, 0) * 4, part(g, T, 1, torch.float32, 0) * 9
+    state = tuple(torch.zeros(s, device=DEV) for s in mops.memory_state_shapes(1, H, d, e, 1))
+    out = mops.outer_memory_scan(q, k, v, state, i32([0]), i32([0]), i32([T]), i32([0]), H, 1, gate_i=gi, gate_f=gf, q_scale=0.25,
+                                 gate_cap=15.0, max_q_len=T).double().cpu()
+    z = torch.zeros(d, dtype=torch.float64)
+    want, S, n, m = memory_reference(mops, 1, q.double().cpu(), k.double().cpu(), v.double().cpu(), torch.zeros(d, e, dtype=torch.float64), z, 0.0,
+                                     0.0, gi[:, 0].double().cpu(), gf[:, 0].double().cpu(), 0.25, 15.0, None, None, None)
+    rel = (out - want).norm(dim=1) / want.norm(dim=1)
+    assert float(rel.median()) < 1e-6 and float(rel.max()) < 2e-3, (float(rel.median()), float(rel.max()))   # (a normaliser near zero)
+    assert torch.allclose(state[0][0, 0].double().cpu(), S, rtol=1e-4, atol=1e-5 * float(S.abs().max()))
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_memory_chunks_keep_the_tokens_ahead_of_a_bad_value(mops, mode, bad):
+    T, H, d, e, at = 100, 1, 32, 24, 70
+    g = torch.Generator(device=DEV).manual_seed(9)
+    q, k, v = (part(g, T, n, torch.float32, 0) for n in (d, d, e))
+    gi, gf, one = part(g, T, 1, torch.float32, 0), part(g, T, 1, torch.float32, 0), torch.ones(1, device=DEV)
+    kw = {0: dict(decay=0.9 * one), 1: dict(gate_i=gi, gate_f=gf), 2: dict(gate_i=gi, a_log=one, dt_bias=one, skip=one)}[mode]
+
+    def go(vv):
+        state = tuple(torch.zeros(s, device=DEV) for s in mops.memory_state_shapes(1, H, d, e, mode))
+        return mops.outer_memory_scan(q, k, vv, state, i32([0]), i32([0]), i32([T]), i32([0]), H, mode, max_q_len=T, **kw)
+    want, w = go(v), v.clone()
+    w[at, 3] = bad
+    got = go(w)
+    cols = [c for c in range(e) if c != 3]
+    assert torch.allclose(got[:at], want[:at], rtol=1e-4, atol=1e-5) and torch.allclose(got[:, cols], want[:, cols], rtol=1e-4, atol=1e-5)
+    assert not torch.isfinite(got[at:, 3]).any()
