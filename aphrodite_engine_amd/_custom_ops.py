@@ -1930,6 +1930,54 @@ def wna16_gemm_grouped(a_packed: torch.Tensor, m_pad: int, k: int, qweight: torc
     return out
 
 
+def moe_route_align_blocks(gating_output: torch.Tensor, topk: int, renormalize: bool, num_experts: int, block_size: int):
+    """moe_route_align (with the inverse) for any number of tokens and <= 16 experts, in two launches."""
+    _require_cuda(gating_output)
+    t_, e = gating_output.shape
+    if e != num_experts or gating_output.stride(1) != 1:
+        raise RuntimeError("moe_route_align_blocks: gating_output must be [tokens, num_experts] with contiguous rows")
+    numel = t_ * topk
+    max_padded = numel + num_experts * (block_size - 1)
+    i32 = dict(dtype=torch.int32, device=gating_output.device)
+    topk_weights = torch.empty((t_, topk), dtype=torch.float32, device=gating_output.device)
+    topk_ids, inv, counts = torch.empty((t_, topk), **i32), torch.empty(numel, **i32), torch.empty((t_ + 255) // 256 * 16, **i32)
+    sorted_ids, expert_ids, post_pad = (torch.empty(n, **i32) for n in (max_padded, (max_padded + block_size - 1) // block_size, 1))
+    check(_lib.lib().aphro_moe_route_align_blocks(
+        topk_weights.data_ptr(), topk_ids.data_ptr(), gating_output.data_ptr(), gating_output.stride(0), counts.data_ptr(),
+        sorted_ids.data_ptr(), expert_ids.data_ptr(), post_pad.data_ptr(), inv.data_ptr(), t_, num_experts, topk, 1 if renormalize else 0,
+        block_size, _dt(gating_output), _stream()), "moe_route_align_blocks")
+    return topk_weights, topk_ids, sorted_ids, expert_ids, post_pad, inv
+
+
+def wna16_moe_tile_ksplit(blocks: int, n: int, k: int, groups: int, block_m: int, silu: bool) -> int:
+    """K slices of wna16_moe_tile for a shape (0: not served)."""
+    return int(_lib.lib().aphro_wna16_moe_tile_ksplit(blocks, n, k, groups, block_m, 1 if silu else 0))
+
+
+def wna16_moe_tile(a: torch.Tensor, sorted_slots: Optional[torch.Tensor], numel: int, topk: int, qweight: torch.Tensor, qzeros: torch.Tensor,
+                   scales: torch.Tensor, expert_ids: torch.Tensor, num_tokens_post_pad: torch.Tensor, m_pad: int, block_m: int,
+                   zero_offset: int, silu: bool) -> torch.Tensor:
+    """Grouped expert GEMM of prompt-sized batches (csrc/wna16_moe_tile.hip): a [rows, K] f16 (or bf16 with bf16 scales, widened first);
+    silu -> f16 activations [m_pad, N/2], else fp32 slabs [S, m_pad, N]."""
+    lib = _lib.lib()
+    k, n, groups = qweight.shape[1] * 8, qweight.shape[2], scales.shape[1]
+    ks = wna16_moe_tile_ksplit(m_pad // block_m, n, k, groups, block_m, silu)
+    if ks <= 0:
+        raise RuntimeError(f"wna16_moe_tile: shape N={n} K={k} not served")
+    if a.stride(1) != 1 or a.stride(0) % 8 != 0 or a.data_ptr() % 16 != 0:
+        a = a.contiguous()
+    if a.dtype == torch.bfloat16:
+        f = torch.empty(a.shape, dtype=torch.float16, device=a.device)
+        check(lib.aphro_moe_rows_to_f16(a.data_ptr(), f.data_ptr(), a.shape[0], k, a.stride(0), _stream()), "moe_rows_to_f16")
+        a = f
+    act = torch.empty((m_pad, n // 2), dtype=torch.float16, device=a.device) if silu else None
+    out = None if silu else torch.empty((ks, m_pad, n), dtype=torch.float32, device=a.device)
+    check(lib.aphro_wna16_moe_tile(a.data_ptr(), a.shape[0], a.stride(0), _ptr(sorted_slots), numel, topk, qweight.data_ptr(), qzeros.data_ptr(),
+                                   scales.data_ptr(), expert_ids.data_ptr(), num_tokens_post_pad.data_ptr(), _ptr(act), _ptr(out), m_pad, n, k,
+                                   groups, ks, block_m, zero_offset, _dt(scales), _stream()), "wna16_moe_tile")
+    return act if silu else out
+
+
 def moe_combine(slabs: torch.Tensor, inv_pos: torch.Tensor, topk_weights: torch.Tensor,
                 out_dtype: torch.dtype) -> torch.Tensor:
     """out[t] = sum_k round(w[t,k] * y[inv_pos[t,k]]), y = sum of the split-K slabs."""

@@ -336,6 +336,101 @@ __global__ __launch_bounds__(1024) void moe_route_align_kernel(
   }
 }
 
+// fused_topk + moe_align_block_size for PROMPT-sized batches with <= 16 experts: the one-workgroup form ranks its slots in one wave (118 us at
+// 6000 slots of 8 experts); here a workgroup routes 256 tokens, thread = token with moe_route_row16's arithmetic, and counts its experts; the
+// second launch sums the counts ahead of it and places its slots.  A token names an expert once, so a slot's rank among its workgroup's is
+// the number of earlier threads that name the expert: a ballot per expert and wave.  Same weights, ids and slot order.
+constexpr int MRB_TOKENS = 256;
+template <typename T>
+__global__ __launch_bounds__(MRB_TOKENS) void moe_route_blocks_kernel(float* __restrict__ topk_weights, int32_t* __restrict__ topk_ids,
+                                                                      const typename T::storage* __restrict__ gating, int64_t gating_stride,
+                                                                      int32_t* __restrict__ counts, int num_tokens, int num_experts, int k,
+                                                                      int renormalize) {
+  __shared__ int32_t cnt[16];
+  if (threadIdx.x < 16) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int tok = blockIdx.x * MRB_TOKENS + threadIdx.x;
+  if (tok < num_tokens) {
+    float wk[8];
+    int we[8];
+    float wsum;
+    moe_route_row16<T>(gating + (size_t)tok * gating_stride, num_experts, k, wk, we, wsum);
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+      if (kk < k) {
+        topk_ids[(size_t)tok * k + kk] = we[kk];
+        topk_weights[(size_t)tok * k + kk] = renormalize ? wk[kk] / wsum : wk[kk];
+        atomicAdd(&cnt[we[kk]], 1);
+      }
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 16) counts[blockIdx.x * 16 + threadIdx.x] = cnt[threadIdx.x];
+}
+
+__global__ __launch_bounds__(MRB_TOKENS) void moe_align_blocks_kernel(const int32_t* __restrict__ topk_ids, const int32_t* __restrict__ counts,
+                                                                      int32_t* __restrict__ sorted_token_ids, int32_t* __restrict__ expert_ids,
+                                                                      int32_t* __restrict__ num_tokens_post_pad, int32_t* __restrict__ inv_pos,
+                                                                      int num_tokens, int num_experts, int k, int block_size, int max_padded,
+                                                                      int max_blocks) {
+  __shared__ int32_t all[16], ahead[16], start[17], wcnt[MRB_TOKENS / 64][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, numel = num_tokens * k;
+  if (tid < 16) all[tid] = ahead[tid] = 0;
+  __syncthreads();
+  {
+    int a = 0, b = 0;
+    for (int blk = tid >> 4; blk < (int)gridDim.x; blk += MRB_TOKENS / 16) {
+      const int c = counts[blk * 16 + (tid & 15)];
+      a += c;
+      if (blk < (int)blockIdx.x) b += c;
+    }
+    atomicAdd(&all[tid & 15], a);
+    atomicAdd(&ahead[tid & 15], b);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    start[0] = 0;
+    for (int e = 0; e < num_experts; ++e) start[e + 1] = start[e] + (all[e] + block_size - 1) / block_size * block_size;
+  }
+  const int tok = blockIdx.x * MRB_TOKENS + tid;
+  int mine[8], rank[8];
+  unsigned chosen = 0;                                  // experts of the token, one bit each
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) {
+    mine[kk] = kk < k && tok < num_tokens ? topk_ids[(size_t)tok * k + kk] : -1;
+    if (mine[kk] >= 0) chosen |= 1u << mine[kk];
+    rank[kk] = 0;
+  }
+  for (int e = 0; e < num_experts; ++e) {
+    const unsigned long long mask = __ballot((chosen >> e) & 1);
+    if (lane == 0) wcnt[wave][e] = __popcll(mask);
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk)
+      if (mine[kk] == e) rank[kk] = __popcll(mask & ((1ull << lane) - 1ull));
+  }
+  __syncthreads();
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk)
+    if (mine[kk] >= 0) {
+      const int e = mine[kk];
+      int pos = start[e] + ahead[e] + rank[kk];
+      for (int w = 0; w < wave; ++w) pos += wcnt[w][e];
+      sorted_token_ids[pos] = tok * k + kk;
+      if (inv_pos) inv_pos[(size_t)tok * k + kk] = pos;
+    }
+  if (blockIdx.x != 0) return;                          // what is left: padding, the blocks' experts, the padded total
+  if (tid == 0) *num_tokens_post_pad = start[num_experts];
+  for (int e = 0; e < num_experts; ++e)
+    for (int i = start[e] + all[e] + tid; i < start[e + 1]; i += MRB_TOKENS) sorted_token_ids[i] = numel;
+  for (int i = start[num_experts] + tid; i < max_padded; i += MRB_TOKENS) sorted_token_ids[i] = numel;
+  for (int i = tid; i < max_blocks; i += MRB_TOKENS) {
+    int e = -1;
+    for (int x = 0; x < num_experts; ++x)
+      if (i * block_size >= start[x] && i * block_size < start[x + 1]) e = x;
+    expert_ids[i] = e;
+  }
+}
+
 // Fragment-major pack (see pack_a_kernel, wna16_gemm.hip) of the rows selected by sorted_token_ids:
 // packed row r <- a[sorted[r] / topk] (a zero row for padding entries and for rows beyond
 // *num_tokens_post_pad).
@@ -525,6 +620,31 @@ extern "C" int aphro_moe_route_align(float* topk_weights, int32_t* topk_ids, con
                      inv_pos, (int)num_tokens, num_experts, topk, renormalize, block_size, max_padded, max_blocks)
   if (dtype == APHRO_F16) L(Half); else if (dtype == APHRO_BF16) L(BFloat); else L(Float);
 #undef L
+  APHRO_LAUNCH_CHECK();
+  return APHRO_OK;
+}
+
+// The same results in two launches of ceil(num_tokens / 256) workgroups: <= 16 experts, any number of tokens.  counts: scratch of 16 int32 per
+// workgroup.
+extern "C" int aphro_moe_route_align_blocks(float* topk_weights, int32_t* topk_ids, const void* gating, int64_t gating_stride,
+                                            int32_t* counts, int32_t* sorted_token_ids, int32_t* expert_ids, int32_t* num_tokens_post_pad,
+                                            int32_t* inv_pos, int64_t num_tokens, int num_experts, int topk, int renormalize,
+                                            int block_size, int dtype, void* stream) {
+  APHRO_CHECK(num_experts >= 1 && num_experts <= 16 && block_size >= 1, "moe_route_align_blocks: %d experts (<= 16)", num_experts);
+  APHRO_CHECK(topk >= 1 && topk <= 8 && topk <= num_experts, "moe_route_align_blocks: topk=%d (1..8 supported)", topk);
+  APHRO_CHECK(num_tokens >= 1 && num_tokens * topk < (1 << 24), "moe_route_align_blocks: %ld tokens", (long)num_tokens);
+  APHRO_CHECK(dtype >= APHRO_F16 && dtype <= APHRO_F32, "moe_route_align_blocks: unsupported gating dtype %d", dtype);
+  const int numel = (int)num_tokens * topk;
+  const int max_padded = numel + num_experts * (block_size - 1);
+  const int max_blocks = (max_padded + block_size - 1) / block_size;
+  const dim3 grid((unsigned)((num_tokens + MRB_TOKENS - 1) / MRB_TOKENS));
+#define L(TT)                                                                                                             \
+  hipLaunchKernelGGL((moe_route_blocks_kernel<TT>), grid, dim3(MRB_TOKENS), 0, (hipStream_t)stream, topk_weights, topk_ids, \
+                     (const typename TT::storage*)gating, gating_stride, counts, (int)num_tokens, num_experts, topk, renormalize)
+  if (dtype == APHRO_F16) L(Half); else if (dtype == APHRO_BF16) L(BFloat); else L(Float);
+#undef L
+  hipLaunchKernelGGL(moe_align_blocks_kernel, grid, dim3(MRB_TOKENS), 0, (hipStream_t)stream, topk_ids, counts, sorted_token_ids, expert_ids,
+                     num_tokens_post_pad, inv_pos, (int)num_tokens, num_experts, topk, block_size, max_padded, max_blocks);
   APHRO_LAUNCH_CHECK();
   return APHRO_OK;
 }

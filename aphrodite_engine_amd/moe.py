@@ -127,6 +127,39 @@ class Wna16Experts:
         self.inter = self.w2[0].shape[1] * 8
 
 
+# Prompt-sized batches: from MOE_TILE_ROWS slots per expert on (the average) the experts run on the tile GEMM, in blocks of 64 rows, and of 128
+# from MOE_TILE_WIDE on.  Mixtral-8x7B's experts (8, top 2), decode kernel / 64 / 128 in us: 64 tokens 251 / 280 / 475, 96 tokens 325 / 257 / 434,
+# 160 tokens 451 / 258 / 448, 512 tokens 1268 / 540 / 632, 2048 tokens 4900 / 1760 / 1806, 4096 tokens - / 3354 / 3334.
+MOE_TILE_ROWS, MOE_TILE_WIDE = 24, 768
+
+
+def moe_tile_block(slots: int, experts: Wna16Experts, dtype: torch.dtype) -> int:
+    """Rows of a block of the tile GEMM for a batch of ``slots`` (token, expert) pairs; 0: the decode kernel's batch or shape."""
+    e = experts.num_experts
+    if slots < MOE_TILE_ROWS * e or dtype != experts.w13[2].dtype:
+        return 0
+    bm = 64 if slots < MOE_TILE_WIDE * e else 128
+    blocks = (slots + e * (bm - 1) + bm - 1) // bm
+    for (qw, _, sc), k, silu in ((experts.w13, experts.hidden, True), (experts.w2, experts.inter, False)):
+        # (what the decode kernel refuses stays refused whatever the batch)
+        if ops.wna16_moe_tile_ksplit(blocks, qw.shape[2], k, sc.shape[1], bm, silu) <= 0 \
+                or ops.wna16_grouped_ksplit(blocks * bm, qw.shape[2], k, sc.shape[1]) <= 0:
+            return 0
+    return bm
+
+
+def _tile_experts(hidden_states, experts: Wna16Experts, topk: int, topk_weights, sorted_ids, expert_ids, post_pad, inv, bm: int,
+                  defer_combine: bool):
+    """Both expert GEMMs on the tile kernel, rows aligned in blocks of ``bm``."""
+    m_pad = (sorted_ids.numel() + bm - 1) // bm * bm
+    numel = hidden_states.shape[0] * topk
+    act = ops.wna16_moe_tile(hidden_states, sorted_ids, numel, topk, *experts.w13, expert_ids, post_pad, m_pad, bm, experts.zero_offset, True)
+    slabs = ops.wna16_moe_tile(act, None, numel, topk, *experts.w2, expert_ids, post_pad, m_pad, bm, experts.zero_offset, False)
+    if defer_combine:
+        return DeferredCombine(slabs, inv, topk_weights.contiguous(), hidden_states.dtype)
+    return ops.moe_combine(slabs, inv, topk_weights.contiguous(), hidden_states.dtype)
+
+
 def fused_wna16_moe(hidden_states: torch.Tensor, experts: Wna16Experts, gating_output: torch.Tensor,
                     topk: int, renormalize: bool = True,
                     topk_weights: Optional[torch.Tensor] = None,
@@ -138,6 +171,18 @@ def fused_wna16_moe(hidden_states: torch.Tensor, experts: Wna16Experts, gating_o
     m = hidden_states.shape[0]
     e = experts.num_experts
     packed = None
+    bm = moe_tile_block(m * topk, experts, hidden_states.dtype) if aligned is None else 0
+    if bm:
+        if topk_ids is not None:
+            sorted_ids, expert_ids, post_pad, inv = moe_align_block_size(topk_ids, bm, e, want_inverse=True)
+        elif (e <= 16 and topk <= 8 and topk <= e and gating_output.stride(1) == 1
+              and gating_output.dtype in (torch.float16, torch.bfloat16, torch.float32) and m * topk < 1 << 24
+              and not switch("APHRO_MOE_NO_ROUTE_ALIGN")):
+            topk_weights, topk_ids, sorted_ids, expert_ids, post_pad, inv = ops.moe_route_align_blocks(gating_output, topk, renormalize, e, bm)
+        else:
+            topk_weights, topk_ids = fused_topk(hidden_states, gating_output, topk, renormalize)
+            sorted_ids, expert_ids, post_pad, inv = moe_align_block_size(topk_ids, bm, e, want_inverse=True)
+        return _tile_experts(hidden_states, experts, topk, topk_weights, sorted_ids, expert_ids, post_pad, inv, bm, defer_combine)
     if aligned is not None:
         sorted_ids, expert_ids, post_pad, inv = aligned
     elif topk_ids is None:

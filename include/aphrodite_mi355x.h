@@ -829,6 +829,23 @@ int aphro_wna16_gemm_grouped(const void* a_packed, const uint32_t* q_weight,
                              void* act_packed, int64_t m_pad, int64_t N, int64_t K,
                              int64_t groups, int zero_offset, int dtype, void* stream);
 
+/* Grouped expert GEMM for prompt-sized batches: blocks of block_m (64 or 128) rows of one expert (aphro_moe_align_block_size with that
+ * block size) x 256 columns.  a: f16 [rows, lda]; sorted_slots given: row r of a block is token sorted_slots[r] / topk of `a` (numel: the
+ * valid slots), else row r itself.  Weights as aphro_wna16_gemm_grouped.  Exactly one of: act = f16 [m_pad, N / 2], SiluAndMul of the
+ * interleaved (gate, up) columns rounded as `dtype` rounds; out = fp32 [ksplit, m_pad, N] slabs.  N % 256 == 0, group size % 128 == 0;
+ * ksplit: aphro_wna16_moe_tile_ksplit (0: not served).  Rows past *num_tokens_post_pad are not written. */
+int aphro_wna16_moe_tile_ksplit(int64_t blocks, int64_t N, int64_t K, int64_t groups, int block_m, int silu);
+int aphro_wna16_moe_tile(const void* a, int64_t rows, int64_t lda, const int32_t* sorted_slots, int64_t numel, int topk,
+                         const uint32_t* q_weight, const uint32_t* qzeros, const void* scales, const int32_t* expert_ids,
+                         const int32_t* num_tokens_post_pad, void* act, float* out, int64_t m_pad, int64_t N, int64_t K,
+                         int64_t groups, int ksplit, int block_m, int zero_offset, int dtype, void* stream);
+/* bf16 rows as f16, saturating, dense [rows, K]. */
+int aphro_moe_rows_to_f16(const void* a, void* out, int64_t rows, int64_t K, int64_t lda, void* stream);
+/* aphro_moe_route_align in two launches over 256 tokens a workgroup: <= 16 experts, any number of tokens.  counts: 16 int32 per 256 tokens. */
+int aphro_moe_route_align_blocks(float* topk_weights, int32_t* topk_ids, const void* gating, int64_t gating_stride, int32_t* counts,
+                                 int32_t* sorted_token_ids, int32_t* expert_ids, int32_t* num_tokens_post_pad, int32_t* inv_pos,
+                                 int64_t num_tokens, int num_experts, int topk, int renormalize, int block_size, int dtype, void* stream);
+
 /* out[t] = sum_k round(w[t][k] * y[inv_pos[t*topk+k]]) with y = sum of the nslab fp32 slabs
  * [nslab][m_pad][N] of the second expert GEMM (fused_moe.py:520-542). */
 int aphro_moe_combine(void* out, const float* slabs, int nslab, int64_t m_pad,
