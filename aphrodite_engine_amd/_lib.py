@@ -214,6 +214,8 @@ MIXERS_SIGNATURES = {
     "aphro_experts_route_topk": (I, [P, P, P, P, L, I, I, P]),
     "aphro_hyper_residual_rms_norm": (I, [P, P, L, P, P, P, F, P, P, P, P, L, I, I, F, I, P]),
     "aphro_logit_softcap": (I, [P, P, L, F, F, I, P]),
+    "aphro_gated_delta_chunked_workspace": (L, [I, L, I, I, I, I]),
+    "aphro_gated_delta_chunked": (I, [P, P, L, P, L, P, L, P, L, P, L, P, P, P, P, I, P, P, P, I, L, I, I, I, I, I, F, F, I, P, L, I, P]),
     "aphro_gated_delta_scan": (I, [P, P, L, P, L, P, L, P, L, P, L, P, P, P, P, I, P, P, P, I, L, I, I, I, I, I, F, F, I, I, P]),
     "aphro_gated_head_rms_norm": (I, [P, L, P, P, P, L, L, I, I, F, I, I, P]),
     "aphro_conv_rotary_supported": (I, [I, I, I]),

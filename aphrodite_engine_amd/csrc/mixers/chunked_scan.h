@@ -12,6 +12,13 @@ constexpr int CHUNK = 64;
 // here lane group g = l / 16 brings four (or eight) NEIGHBOURING k per load and one of them per call.
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
+// A barrier for what lies in LDS only: __syncthreads() also waits for the loads from memory that are still on their way.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 __device__ __forceinline__ int wave_incl_sum(int v, int lane) {
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {

@@ -17,7 +17,7 @@
 // registers meanwhile.  The per-token partial dot products are folded over the slices with DPP moves.
 //
 // gated_head_rms_norm: out = o / rms(o over the head's vdim) * weight[vdim] * act(gate), one wave per (token, head).
-#include "mixers_common.h"
+#include "delta_rule.h"
 
 namespace aphro {
 
@@ -30,7 +30,7 @@ __global__ __launch_bounds__(256) void gated_delta_scan_kernel(
     const typename T::storage* __restrict__ b, int64_t b_stride, const typename T::storage* __restrict__ a, int64_t a_stride,
     const float* __restrict__ a_log, const float* __restrict__ dt_bias, float* __restrict__ state,
     const int32_t* __restrict__ slot_of_seq, int num_slots, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ q_len, const int32_t* __restrict__ ctx_len, int heads, int kv_heads, int dim, int vdim,
+    const int32_t* __restrict__ q_len, const int32_t* __restrict__ ctx_len, int below, int heads, int kv_heads, int dim, int vdim,
     float q_scale, float norm_eps) {
   constexpr int NS = 1 << SLOG;        // slices of the key dimension = lanes that share a column
   constexpr int TW = 256 >> SLOG;      // value columns per workgroup
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void gated_delta_scan_kernel(
   const int tid = threadIdx.x, c = tid >> SLOG, sl = tid & (NS - 1), col = c0 + c;
   const int n = q_len[s];
   const int slot = slot_of_seq[s];
-  if (n <= 0 || slot < 0 || slot >= num_slots) return;
+  if (n <= 0 || n >= below || slot < 0 || slot >= num_slots) return;
   const int64_t t0 = q_start[s];
   const bool fresh = ctx_len[s] == 0;
   float S[DPT];
@@ -197,6 +197,46 @@ __global__ __launch_bounds__(256) void gated_head_rms_norm_kernel(typename T::st
   }
 }
 
+int gated_delta_check(const GatedDelta& p) {
+  APHRO_CHECK(p.out && p.q && p.k && p.v && p.b && p.a && p.a_log && p.dt_bias && p.state && p.slot_of_seq && p.q_start && p.q_len && p.ctx_len,
+              "gated_delta_scan: null argument");
+  APHRO_CHECK(p.heads > 0 && p.heads <= 65535 && p.kv_heads > 0 && p.heads % p.kv_heads == 0 && p.dim > 0 && p.dim <= 256 && p.vdim > 0 &&
+                  p.vdim <= 16 * 65535 && p.num_slots > 0,
+              "gated_delta_scan: heads %d over %d key heads, dim %d (<= 256), vdim %d", p.heads, p.kv_heads, p.dim, p.vdim);
+  APHRO_CHECK(p.q_stride >= (int64_t)p.kv_heads * p.dim && p.k_stride >= (int64_t)p.kv_heads * p.dim && p.v_stride >= (int64_t)p.heads * p.vdim &&
+                  p.b_stride >= p.heads && p.a_stride >= (p.channel_decay ? (int64_t)p.heads * p.dim : (int64_t)p.heads), "gated_delta_scan: row strides smaller than the rows");
+  return APHRO_OK;
+}
+
+int gated_delta_scan_launch(const GatedDelta& p, int below, bool wide) {
+  const int tw = wide ? 16 : 64;
+  const dim3 grid((unsigned)p.num_seqs, (unsigned)p.heads, (unsigned)((p.vdim + tw - 1) / tw));
+#define GDR_LAUNCH1(DPT, SLOG, CHANNEL)                                                                                                \
+  hipLaunchKernelGGL((gated_delta_scan_kernel<T, DPT, SLOG, CHANNEL>), grid, dim3(256), 0, p.stream, p.out, (const S*)p.q, p.q_stride, \
+                     (const S*)p.k, p.k_stride, (const S*)p.v, p.v_stride, (const S*)p.b, p.b_stride, (const S*)p.a, p.a_stride, p.a_log, p.dt_bias, \
+                     p.state, p.slot_of_seq, p.num_slots, p.q_start, p.q_len, p.ctx_len, below, p.heads, p.kv_heads, p.dim, p.vdim, p.q_scale, p.norm_eps)
+#define GDR_LAUNCH(DPT, SLOG)                             \
+  do {                                                    \
+    if (p.channel_decay) GDR_LAUNCH1(DPT, SLOG, true);    \
+    else GDR_LAUNCH1(DPT, SLOG, false);                   \
+  } while (0)
+  MIX_DISPATCH_DTYPE(p.dtype, {
+    typedef typename T::storage S;
+    if (wide) {
+      if (p.dim <= 64) GDR_LAUNCH(4, 4);
+      else if (p.dim <= 128) GDR_LAUNCH(8, 4);
+      else GDR_LAUNCH(16, 4);
+    } else if (p.dim <= 32) GDR_LAUNCH(8, 2);
+    else if (p.dim <= 64) GDR_LAUNCH(16, 2);
+    else if (p.dim <= 128) GDR_LAUNCH(32, 2);
+    else GDR_LAUNCH(64, 2);
+  });
+#undef GDR_LAUNCH
+#undef GDR_LAUNCH1
+  APHRO_LAUNCH_CHECK();
+  return APHRO_OK;
+}
+
 }  // namespace aphro
 
 using namespace aphro;
@@ -208,40 +248,11 @@ extern "C" int aphro_gated_delta_scan(float* out, const void* q, int64_t q_strid
                                       int num_seqs, int64_t num_tokens, int heads, int kv_heads, int dim, int vdim, int channel_decay,
                                       float q_scale, float norm_eps, int max_q_len, int dtype, void* stream) {
   if (num_tokens == 0 || num_seqs == 0) return APHRO_OK;
-  APHRO_CHECK(out && q && k && v && b && a && a_log && dt_bias && state && slot_of_seq && q_start && q_len && ctx_len,
-              "gated_delta_scan: null argument");
-  APHRO_CHECK(heads > 0 && heads <= 65535 && kv_heads > 0 && heads % kv_heads == 0 && dim > 0 && dim <= 256 && vdim > 0 &&
-                  vdim <= 16 * 65535 && num_slots > 0,
-              "gated_delta_scan: heads %d over %d key heads, dim %d (<= 256), vdim %d", heads, kv_heads, dim, vdim);
-  APHRO_CHECK(q_stride >= (int64_t)kv_heads * dim && k_stride >= (int64_t)kv_heads * dim && v_stride >= (int64_t)heads * vdim &&
-                  b_stride >= heads && a_stride >= (channel_decay ? (int64_t)heads * dim : (int64_t)heads), "gated_delta_scan: row strides smaller than the rows");
-  const bool wide = max_q_len >= 32;
-  const int tw = wide ? 16 : 64;
-  const dim3 grid((unsigned)num_seqs, (unsigned)heads, (unsigned)((vdim + tw - 1) / tw));
-#define GDR_LAUNCH1(DPT, SLOG, CHANNEL)                                                                                                \
-  hipLaunchKernelGGL((gated_delta_scan_kernel<T, DPT, SLOG, CHANNEL>), grid, dim3(256), 0, (hipStream_t)stream, out, (const S*)q, q_stride, \
-                     (const S*)k, k_stride, (const S*)v, v_stride, (const S*)b, b_stride, (const S*)a, a_stride, a_log, dt_bias,  \
-                     state, slot_of_seq, num_slots, q_start, q_len, ctx_len, heads, kv_heads, dim, vdim, q_scale, norm_eps)
-#define GDR_LAUNCH(DPT, SLOG)                             \
-  do {                                                    \
-    if (channel_decay) GDR_LAUNCH1(DPT, SLOG, true);      \
-    else GDR_LAUNCH1(DPT, SLOG, false);                   \
-  } while (0)
-  MIX_DISPATCH_DTYPE(dtype, {
-    typedef typename T::storage S;
-    if (wide) {
-      if (dim <= 64) GDR_LAUNCH(4, 4);
-      else if (dim <= 128) GDR_LAUNCH(8, 4);
-      else GDR_LAUNCH(16, 4);
-    } else if (dim <= 32) GDR_LAUNCH(8, 2);
-    else if (dim <= 64) GDR_LAUNCH(16, 2);
-    else if (dim <= 128) GDR_LAUNCH(32, 2);
-    else GDR_LAUNCH(64, 2);
-  });
-#undef GDR_LAUNCH
-#undef GDR_LAUNCH1
-  APHRO_LAUNCH_CHECK();
-  return APHRO_OK;
+  const GatedDelta p = {out, q, k, v, b, a, q_stride, k_stride, v_stride, b_stride, a_stride, a_log, dt_bias, state, slot_of_seq, num_slots,
+                        q_start, q_len, ctx_len, num_seqs, num_tokens, heads, kv_heads, dim, vdim, channel_decay, q_scale, norm_eps, dtype,
+                        (hipStream_t)stream};
+  const int rc = gated_delta_check(p);
+  return rc != APHRO_OK ? rc : gated_delta_scan_launch(p, 0x7fffffff, max_q_len >= 32);
 }
 
 extern "C" int aphro_gated_head_rms_norm(void* out, int64_t out_stride, const float* x, const void* weight, const void* gate,

@@ -305,7 +305,7 @@ def outer_memory_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state, 
             state[1].data_ptr() if len(state) > 1 else None, state[2].data_ptr() if len(state) > 2 else None,
             slot_of_seq.data_ptr(), slots, q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(), S, T, heads, d, e, int(mode),
             _p(decay), float(q_scale), float(gate_cap), qk_heads, _p(a_log), _p(dt_bias), _p(skip))
-    if max_q_len >= MEMORY_CHUNKED_FROM and d <= 128 and S <= 65535:
+    if max_q_len >= MEMORY_CHUNKED_FROM and d <= 128 and 0 < S <= 65535:
         need = lib.aphro_outer_memory_chunked_workspace(S, T, heads, d, e, int(mode), MEMORY_CHUNKED_MIN)
         if need <= CHUNKED_WORKSPACE_MAX:
             ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
@@ -832,6 +832,12 @@ def logit_softcap(z: torch.Tensor, scale: float = 1.0, cap: float = 0.0) -> torc
     return out
 
 
+# The delta rule's own line between the forms: a chunk's preparation is a chain of its own (a triangle of 64 tokens), 50 us however few there
+# are.  Scan / chunks in us, 16 heads of 128: one segment of 128 tokens 67 / 61 (a decay per channel), 48 / 52 (one per head), of 512 246 / 88,
+# 175 / 78; eight segments of 128 131 / 130, 83 / 111.
+DELTA_CHUNKED_FROM, DELTA_CHUNKED_MIN = 160, 32
+
+
 def gated_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, b: torch.Tensor, a: torch.Tensor, a_log: torch.Tensor,
                      dt_bias: torch.Tensor, state: torch.Tensor, slot_of_seq: torch.Tensor, q_start: torch.Tensor,
                      q_len: torch.Tensor, ctx_len: torch.Tensor, heads: int, kv_heads: int, q_scale: float, norm_eps: float = 1e-6,
@@ -854,11 +860,18 @@ def gated_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, b: torch
     for t, nm in ((slot_of_seq, "slot_of_seq"), (q_start, "q_start"), (q_len, "q_len"), (ctx_len, "ctx_len")):
         _i32(t, S, nm)
     out = torch.empty(T, heads * e, dtype=torch.float32, device=q.device)
-    check(_lib.mixers_lib().aphro_gated_delta_scan(
-        out.data_ptr(), q.data_ptr(), _rows(q, kv_heads * d, "q"), k.data_ptr(), _rows(k, kv_heads * d, "k"), v.data_ptr(),
-        _rows(v, heads * e, "v"), b.data_ptr(), _rows(b, heads, "b"), a.data_ptr(), _rows(a, na, "a"), a_log.data_ptr(),
-        dt_bias.data_ptr(), state.data_ptr(), slot_of_seq.data_ptr(), slots, q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(),
-        S, T, heads, kv_heads, d, e, int(channel), float(q_scale), float(norm_eps), int(max_q_len), _dt(q), _stream()), "gated_delta_scan")
+    lib = _lib.mixers_lib()
+    args = (out.data_ptr(), q.data_ptr(), _rows(q, kv_heads * d, "q"), k.data_ptr(), _rows(k, kv_heads * d, "k"), v.data_ptr(),
+            _rows(v, heads * e, "v"), b.data_ptr(), _rows(b, heads, "b"), a.data_ptr(), _rows(a, na, "a"), a_log.data_ptr(),
+            dt_bias.data_ptr(), state.data_ptr(), slot_of_seq.data_ptr(), slots, q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(),
+            S, T, heads, kv_heads, d, e, int(channel), float(q_scale), float(norm_eps))
+    if max_q_len >= DELTA_CHUNKED_FROM and d <= 128 and 0 < S <= 65535:
+        need = lib.aphro_gated_delta_chunked_workspace(S, T, heads, d, e, DELTA_CHUNKED_MIN)
+        if need <= CHUNKED_WORKSPACE_MAX:
+            ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
+            check(lib.aphro_gated_delta_chunked(*args, DELTA_CHUNKED_MIN, ws.data_ptr(), need, _dt(q), _stream()), "gated_delta_scan")
+            return out
+    check(lib.aphro_gated_delta_scan(*args, int(max_q_len), _dt(q), _stream()), "gated_delta_scan")
     return out
 
 

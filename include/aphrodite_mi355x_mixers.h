@@ -340,6 +340,17 @@ int aphro_gated_delta_scan(float* out, const void* q, int64_t q_stride, const vo
                            const float* dt_bias, float* state, const int32_t* slot_of_seq, int num_slots, const int32_t* q_start,
                            const int32_t* q_len, const int32_t* ctx_len, int num_seqs, int64_t num_tokens, int heads, int kv_heads,
                            int dim, int vdim, int channel_decay, float q_scale, float norm_eps, int max_q_len, int dtype, void* stream);
+/* aphro_gated_delta_scan with segments of at least min_len tokens in chunks of 64 on the matrix cores (fp32 products), shorter ones token by
+ * token; a single segment always in chunks.  dim <= 128, num_seqs <= 65535; workspace as aphro_outer_memory_chunked's. */
+int64_t aphro_gated_delta_chunked_workspace(int num_seqs, int64_t num_tokens, int heads, int dim, int vdim, int min_len);
+int aphro_gated_delta_chunked(float* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
+                              int64_t v_stride, const void* b, int64_t b_stride, const void* a, int64_t a_stride,
+                              const float* a_log, const float* dt_bias, float* state, const int32_t* slot_of_seq,
+                              int num_slots, const int32_t* q_start, const int32_t* q_len, const int32_t* ctx_len,
+                              int num_seqs, int64_t num_tokens, int heads, int kv_heads, int dim, int vdim, int channel_decay,
+                              float q_scale, float norm_eps, int min_len, float* workspace, int64_t workspace_bytes,
+                              int dtype, void* stream);
+
 /* out[t, h, i] = x[t, h, i] / sqrt(mean_i x^2 + eps) * weight[i] * act(gate[t, h, i]); x fp32 [T, heads * vdim] contiguous;
  * weight [vdim] (shared by the heads; NULL: ones), gate (row stride; NULL: none) and out (row stride) of `dtype`;
  * act 0: sigmoid, 1: silu. */

@@ -123,3 +123,74 @@ def test_memory_chunks_keep_the_tokens_ahead_of_a_bad_value(mops, mode, bad):
     cols = [c for c in range(e) if c != 3]
     assert torch.allclose(got[:at], want[:at], rtol=1e-4, atol=1e-5) and torch.allclose(got[:, cols], want[:, cols], rtol=1e-4, atol=1e-5)
     assert not torch.isfinite(got[at:, 3]).any()
+
+
+def delta_reference(q, k, v, beta, g, S):
+    """One head, one segment, token by token in 64 bits; g [T, d]."""
+    out = torch.empty(v.shape, dtype=torch.float64)
+    for t in range(q.shape[0]):
+        S = g[t][:, None] * S
+        S = S + k[t][:, None] * (beta[t] * (v[t] - S.T @ k[t]))[None, :]
+        out[t] = S.T @ q[t]
+    return out, S
+
+
+@pytest.mark.parametrize("channel", [True, False])
+@pytest.mark.parametrize("dtype,pad", [(torch.bfloat16, 0), (torch.bfloat16, 3), (torch.float32, 4)])
+@pytest.mark.parametrize("d,e", [(128, 128), (64, 72), (24, 20), (100, 200)])
+@pytest.mark.parametrize("strong", [False, True])
+def test_delta_chunks(mops, channel, dtype, pad, d, e, strong):
+    H, G, lens, ctx = 2, 1, [64, 1, 33, 193, 31], [0, 7, 5, 0, 9]
+    g = torch.Generator(device=DEV).manual_seed(d * 3 + e + channel)
+    T, S = sum(lens), len(lens)
+    q, k, v = part(g, T, G * d, dtype, pad), part(g, T, G * d, dtype, pad), part(g, T, H * e, dtype, pad)
+    b = part(g, T, H, dtype, 1)
+    na = H * d if channel else H
+    a = part(g, T, na, dtype, pad) * (4.0 if strong else 1.0)
+    a_log, dt_bias = torch.randn(H, generator=g, device=DEV), torch.randn(na, generator=g, device=DEV) - (0.0 if strong else 3.0)
+    state = torch.randn(S + 1, H, d, e, generator=g, device=DEV)
+    slots, start = [3, 5, 0, 2, 4], np.concatenate([[0], np.cumsum(lens)[:-1]])
+    before = state.double().cpu()
+    out = mops.gated_delta_scan(q, k, v, b, a, a_log, dt_bias, state, i32(slots), i32(start), i32(lens), i32(ctx), H, G, d ** -0.5,
+                                max_q_len=max(lens))
+    Q, K, V, B, A, AL, DT = (x.double().cpu() for x in (q, k, v, b, a, a_log, dt_bias))
+    for s in range(S):
+        rows = slice(start[s], start[s] + lens[s])
+        for h in range(H):
+            qh, kh = (x[rows, :d] / torch.sqrt((x[rows, :d] ** 2).sum(1, keepdim=True) + 1e-6) for x in (Q, K))
+            ah = A[rows, h * d:(h + 1) * d] + DT[h * d:(h + 1) * d] if channel else (A[rows, h] + DT[h])[:, None].expand(-1, d)
+            gh = torch.exp(-torch.exp(AL[h]) * torch.nn.functional.softplus(ah))
+            S0 = before[slots[s], h] if ctx[s] else torch.zeros(d, e, dtype=torch.float64)
+            want, Sw = delta_reference(qh * d ** -0.5, kh, V[rows, h * e:(h + 1) * e], torch.sigmoid(B[rows, h]), gh, S0)
+            got = out[rows, h * e:(h + 1) * e].double().cpu()
+            # fp32 sums of d + 64 products through a triangle of 64 corrections of size below one
+            assert torch.allclose(got, want, rtol=1e-4, atol=2e-5 * float(want.abs().max())), (s, h, (got - want).abs().max())
+            assert torch.allclose(state[slots[s], h].double().cpu(), Sw, rtol=1e-4, atol=2e-5 * float(Sw.abs().max()))
+    assert torch.equal(state[1].double().cpu(), before[1])                # a slot that no segment names
+
+
+@pytest.mark.parametrize("where", ["v", "k", "q", "b"])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_delta_chunks_keep_the_tokens_ahead_of_a_bad_value(mops, where, bad):
+    T, H, d, e, at = 170, 1, 32, 24, 70
+    g = torch.Generator(device=DEV).manual_seed(9)
+    x = {n: part(g, T, w, torch.float32, 0).contiguous() for n, w in (("q", d), ("k", d), ("v", e), ("b", 1), ("a", d))}
+
+    def go(y):
+        state = torch.zeros(1, H, d, e, device=DEV)
+        o = mops.gated_delta_scan(y["q"], y["k"], y["v"], y["b"], y["a"], torch.zeros(1, device=DEV), torch.zeros(d, device=DEV) - 2, state,
+                                  i32([0]), i32([0]), i32([T]), i32([0]), H, H, 1.0, max_q_len=T)
+        return o, state
+    want, w = go(x)[0], {n: t.clone() for n, t in x.items()}
+    w[where][at, 0 if where == "b" else 3] = bad
+    got, state = go(w)
+    assert torch.allclose(got[:at], want[:at], rtol=1e-4, atol=1e-5)
+    old = mops.DELTA_CHUNKED_FROM
+    try:
+        mops.DELTA_CHUNKED_FROM = 1 << 30
+        scanned, state2 = go(w)
+    finally:
+        mops.DELTA_CHUNKED_FROM = old
+    assert torch.equal(torch.isfinite(got), torch.isfinite(scanned)) and torch.equal(torch.isfinite(state), torch.isfinite(state2))
+    fine = torch.isfinite(scanned)
+    assert torch.allclose(got[fine], scanned[fine], rtol=1e-4, atol=1e-5)
