@@ -86,8 +86,6 @@ class ModelRunner:
     def execute(self, segments: Sequence[Tuple[Request, Sequence[int]]], want: Sequence[Sequence[int]]) -> torch.Tensor:
         """Run the segments as one batch from the caches earlier steps left; returns fp32 logits [sum(len(w)), vocab] for
         the wanted places (indices into each segment's tokens), in segment order."""
-        batch = StepBatch.build([list(t) for _, t in segments], [r.num_computed for r, _ in segments],
-                                [r.pages for r, _ in segments], [r.slot for r, _ in segments], self.block_size, self.device)
         rows, a = [], 0
         for (_, toks), w in zip(segments, want):
             for i in w:
@@ -95,11 +93,11 @@ class ModelRunner:
                     raise ValueError("a wanted place outside its segment")
                 rows.append(a + i)
             a += len(toks)
-        if not rows:                  # the step still has to advance caches and states
-            rows = [0]
-            logits = self.model.step(batch, self.caches, torch.tensor(rows, dtype=torch.int64, device=self.device))
-            return logits[:0]
-        return self.model.step(batch, self.caches, torch.tensor(rows, dtype=torch.int64, device=self.device))
+        # (built and used on the current stream: nothing to wait for.  The step has to advance caches and states also where nobody wants a row)
+        batch = StepBatch.build([t for _, t in segments], [r.num_computed for r, _ in segments], [r.pages for r, _ in segments],
+                                [r.slot for r, _ in segments], self.block_size, self.device, rows=rows or [0], wait=False)
+        logits = self.model.step(batch, self.caches, batch.rows)
+        return logits if rows else logits[:0]
 
 
 class Scheduler:

@@ -10,6 +10,24 @@ import numpy as np
 import torch
 
 
+def _to_device(arrays: List[np.ndarray], device, wait: bool) -> List[torch.Tensor]:
+    """The arrays on the device, as parts (16-byte aligned) of one buffer that one copy from pinned memory fills: a copy per array from
+    pageable memory is ten round trips that wait for everything the stream still has to do."""
+    device = torch.device(device)
+    if device.type == "cpu":
+        return [torch.from_numpy(np.ascontiguousarray(a)) for a in arrays]
+    at = np.cumsum([0] + [(a.nbytes + 15) // 16 * 16 for a in arrays]).tolist()
+    host = torch.empty(max(16, at[-1]), dtype=torch.uint8, pin_memory=True)
+    image = host.numpy()
+    for a, i in zip(arrays, at):
+        image[i:i + a.nbytes] = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
+    buf = host.to(device, non_blocking=True)
+    if wait:
+        torch.cuda.current_stream(device).synchronize()
+    kinds = {np.dtype(np.int64): torch.int64, np.dtype(np.int32): torch.int32}
+    return [buf[i:i + a.nbytes].view(kinds[a.dtype]).view(a.shape) for a, i in zip(arrays, at)]
+
+
 @dataclass
 class StepBatch:
     num_tokens: int
@@ -26,44 +44,47 @@ class StepBatch:
     block_size: int
     q_lens: List[int] = field(default_factory=list)      # host copies
     ctx_lens: List[int] = field(default_factory=list)
+    rows: Optional[torch.Tensor] = None                  # int64, rows of the batch asked for
+    seq_lens_tensor: Optional[torch.Tensor] = None       # int32 [S] ctx_len + q_len
+    query_start_loc: Optional[torch.Tensor] = None       # int32, first rows of the leading prompt portions and their end
+    seq_start_loc: Optional[torch.Tensor] = None         # int32, the same of their whole sequences
 
     @staticmethod
     def build(tokens: Sequence[Sequence[int]], ctx_lens: Sequence[int], block_tables: Sequence[Sequence[int]],
-              state_slots: Sequence[int], block_size: int, device) -> "StepBatch":
-        """From host lists, one entry per segment.  Every index the kernels will follow is checked here."""
+              state_slots: Sequence[int], block_size: int, device, rows: Optional[Sequence[int]] = None, wait: bool = True) -> "StepBatch":
+        """From host lists, one entry per segment.  Every index the kernels will follow is checked here.  ``rows``: rows of the batch the
+        caller will ask for (``StepBatch.rows``).  All arrays travel in one copy; ``wait`` False: without waiting for it -- for a caller who
+        uses the batch on the current stream."""
         S = len(tokens)
         q_lens = [len(t) for t in tokens]
         if S == 0 or min(q_lens) <= 0:
             raise ValueError("a step batch needs at least one segment and no empty one")
-        T = sum(q_lens)
-        starts = np.zeros(S, np.int32)
-        starts[1:] = np.cumsum(q_lens)[:-1]
-        width = max(1, max(len(b) for b in block_tables))
-        bt = np.zeros((S, width), np.int32)
-        pos = np.empty(T, np.int64)
-        slots = np.empty(T, np.int64)
-        seq_of = np.empty(T, np.int32)
-        for s in range(S):
-            n, c, a = q_lens[s], int(ctx_lens[s]), int(starts[s])
-            need = (c + n + block_size - 1) // block_size
-            if len(block_tables[s]) < need:
-                raise ValueError(f"segment {s}: {len(block_tables[s])} pages for {c + n} tokens")
-            bt[s, :len(block_tables[s])] = block_tables[s]
-            p = np.arange(c, c + n, dtype=np.int64)
-            pos[a:a + n] = p
-            slots[a:a + n] = bt[s, p // block_size].astype(np.int64) * block_size + p % block_size
-            seq_of[a:a + n] = s
+        n, c = np.asarray(q_lens, np.int64), np.asarray([int(x) for x in ctx_lens], np.int64)
+        pages = np.asarray([len(b) for b in block_tables], np.int64)
+        need = (c + n + block_size - 1) // block_size
+        for s in np.nonzero(pages < need)[0]:
+            raise ValueError(f"segment {s}: {pages[s]} pages for {c[s] + n[s]} tokens")
         if len(set(int(x) for x in state_slots)) != S:
             raise ValueError("two segments of one step share a state slot")
-
-        def dev(a):
-            return torch.from_numpy(a).to(device)
+        T = int(n.sum())
+        starts = np.cumsum(n) - n
+        bt = np.zeros((S, max(1, int(pages.max()))), np.int32)
+        for s, b in enumerate(block_tables):
+            bt[s, :len(b)] = b
+        seq_of = np.repeat(np.arange(S), n)
+        pos = np.arange(T) - np.repeat(starts - c, n)
+        slots = bt[seq_of, pos // block_size].astype(np.int64) * block_size + pos % block_size
         ids = np.concatenate([np.asarray(t, np.int64) for t in tokens])
-        return StepBatch(num_tokens=T, num_seqs=S, input_ids=dev(ids), positions=dev(pos), q_start=dev(starts),
-                         q_len=dev(np.asarray(q_lens, np.int32)), ctx_len=dev(np.asarray(ctx_lens, np.int32)),
-                         seq_of_token=dev(seq_of), block_tables=dev(bt), slot_mapping=dev(slots),
-                         state_slots=dev(np.asarray(state_slots, np.int32)), block_size=block_size, q_lens=q_lens,
-                         ctx_lens=[int(c) for c in ctx_lens])
+        # prompt portions lead (decode_split checks that): their rows and lengths, summed up
+        seq_lens, i32 = c + n, np.int32
+        k = next((s for s in range(S) if q_lens[s] == 1 and c[s] > 0), S)
+        loc, sloc = (np.concatenate([[0], np.cumsum(x[:k])]).astype(i32) for x in (n, seq_lens))
+        d = _to_device([ids, pos, slots, np.asarray([] if rows is None else rows, np.int64), starts.astype(i32), n.astype(i32), c.astype(i32),
+                        seq_of.astype(i32), bt, np.asarray(state_slots, i32), seq_lens.astype(i32), loc, sloc], device, wait)
+        return StepBatch(num_tokens=T, num_seqs=S, input_ids=d[0], positions=d[1], q_start=d[4], q_len=d[5], ctx_len=d[6],
+                         seq_of_token=d[7], block_tables=d[8], slot_mapping=d[2], state_slots=d[9], block_size=block_size, q_lens=q_lens,
+                         ctx_lens=[int(x) for x in c], rows=None if rows is None else d[3], seq_lens_tensor=d[10], query_start_loc=d[11],
+                         seq_start_loc=d[12])
 
     def last_rows(self) -> List[int]:
         """Row of the last token of every segment."""
@@ -86,18 +107,13 @@ class StepBatch:
         """The same batch as MI355XAttentionMetadata (prefill rows first, decode rows after)."""
         from .attention.backend import MI355XAttentionMetadata
         k = self.decode_split()
-        dev = self.input_ids.device
         seq_lens = [c + n for c, n in zip(self.ctx_lens, self.q_lens)]
         npt = sum(self.q_lens[:k])
-        loc = np.zeros(k + 1, np.int32)
-        loc[1:] = np.cumsum(self.q_lens[:k])
-        sloc = np.zeros(k + 1, np.int32)
-        sloc[1:] = np.cumsum(seq_lens[:k])
         return MI355XAttentionMetadata(
             num_prefills=k, num_prefill_tokens=npt, num_decode_tokens=self.num_tokens - npt, slot_mapping=self.slot_mapping,
-            seq_lens=seq_lens, seq_lens_tensor=torch.tensor(seq_lens, dtype=torch.int32, device=dev),
+            seq_lens=seq_lens, seq_lens_tensor=self.seq_lens_tensor,
             max_query_len=max(self.q_lens), max_prefill_seq_len=max(seq_lens[:k], default=0),
             max_decode_seq_len=max(seq_lens[k:], default=0),
-            query_start_loc=torch.from_numpy(loc).to(dev), seq_start_loc=torch.from_numpy(sloc).to(dev),
+            query_start_loc=self.query_start_loc, seq_start_loc=self.seq_start_loc,
             context_lens_tensor=self.ctx_len[:k] if k else self.ctx_len[:0], block_tables=self.block_tables,
             use_cuda_graph=False, max_context_len=max(self.ctx_lens[:k], default=0))
