@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "wna16_rows.h"
 
 namespace aphro {
 
@@ -1039,6 +1040,19 @@ static bool large_eight(const LargePlan& pl, int64_t K) {
   return pl.wm == 2 && pl.wn == 4 && pl.streamk && eight;
 }
 
+// The tile of wna16_gemm_rows.hip, up to 4096 rows: always where this file would take one workgroup per tile (4096 x 4096: 150 rows
+// 27.3 -> 18.3 us, 1300 rows 78 -> 56 us), and beside the stream-K form where its last round is full enough (28672 x 4096: 300 rows
+// 127 -> 82 us, 1300 rows 341 -> 326 us; 2048 rows 450 against 489 us: stays).  Its slabs fit the workspace of this file's
+// plan; a call that is not sliced here is not sliced there: the SiluAndMul form and the plain GEMM have the same bits.
+static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs) {
+  int64_t other_ns = -1;
+  if (pl.streamk) {            // 1.9 us per 256 x 256 x 64 of a CU's even share, 18 us around them
+    const int64_t units = (M + 255) / 256 * ((N + 255) / 256) * (K / 64);
+    other_ns = 18000 + units * 1900 / pl.grid;
+  }
+  return wna16_rows_plan(M, N, K, gs, pl.streamk ? 0 : (int64_t)large_scratch_bytes(pl, M, N), other_ns < 0 ? -1 : other_ns * 97 / 100);
+}
+
 static size_t large_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype, int strip_m) {
   if (groups <= 0 || K % groups != 0) return 0;
   const LargePlan pl = large_plan(M, N, K, K / groups);
@@ -1117,6 +1131,16 @@ static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const 
     for (uint32_t x = 0; x < segs; ++x)
       APHRO_CHECK(((x * p.st_inv_nseg) >> 16) == x / p.st_nseg && ((x * p.st_inv_nwv) >> 16) == x / p.st_nwv,
                   "wna16_gemm_large_strip: multiply-shift division fails at %u (nseg %d, nwv %d)", x, p.st_nseg, p.st_nwv);
+  }
+  const Wna16RowsPlan rp = rows_plan(pl, M, N, K, gs);
+  if (rp.mb > 0) {
+    Wna16RowsParams q = {};
+    q.a = p.a; q.lda = p.lda; q.qw = p.qw; q.qz = p.qz; q.sc = p.sc; q.c = p.c; q.partial = (float*)ws;
+    q.M = p.M; q.N = p.N; q.K = p.K; q.group_size = p.group_size; q.zero_offset = zero_offset;
+    q.ksplit = rp.ksplit; q.silu = silu; q.bf16 = p.out_bf16;
+    APHRO_CHECK(strip_m == 0 || wna16_strip_fill(q.strip, strip_m, N, K, groups),
+                "wna16_gemm_large_strip: no strip-major form for M class %d, N=%ld, K=%ld, groups=%ld", strip_m, (long)N, (long)K, (long)groups);
+    return wna16_rows_launch(q, rp, st);
   }
   if (large_two_pass(pl, M, N, K, gs)) {
     // pass 1: the weights dequantised once into f16 W^T [N, K] (same numerics as the in-loop dequantisation: same bits out)

@@ -1,0 +1,384 @@
+// W4A16 (GPTQ / AWQ-repacked int4) GEMM for 65 rows and more on gfx950: large decode batches and prompts up to a few thousand tokens, where
+// the 256-row tiles of wna16_gemm_large.hip are half empty or too few for the chip.
+//
+//   * tile = 32 MB rows (MB = 3, 4, 5: the height fits the batch) x 128 columns, K tile 128, 8 waves: 2 column groups of 64 x 4 K groups
+//     of 32.  D^T[n][m] = W^T[n][k] . A^T[k][m] with v_mfma_f32_32x32x16_f16, an exllama dword being a lane's weight fragment; every
+//     dword is fetched and unpacked by ONE wave of the chip per row tile, for all its rows: 13 VALU against MB MFMAs of 32 cycles.
+//     The four K groups meet in LDS at the end, in fixed order.
+//   * weights, scales and zero points go global -> VGPR (8 bytes a lane: two adjacent columns, so that a lane ends with 8 adjacent columns
+//     of its row); the activations go direct to LDS, 256-byte rows XOR-swizzled on the source address.  Four stages, three tiles ahead.
+//   * int4 -> f16 in registers with the numerics of wna16_gemm_large.hip: (q - z) exact, one rounding in the multiply by the group scale.
+//   * a step's MFMAs run while the next step's fragments are read and unpacked, and the loads go out BETWEEN the MFMAs: all eight
+//     waves' at once, behind the barrier, made the waves wait for the address unit with the matrix cores idle (28672 x 4096, 150 rows:
+//     48.9 -> 41.8 us).
+//   * K slices write the accumulators as they lie in the registers, 1 KiB a store; a second kernel sums them in the order of K.
+// Bound by the activations' way into LDS and the MFMAs together: 1.2 us per K tile of 160 rows on every CU, 0.53 us of it MFMA.
+// Layer of Llama-3-8B at 150 rows, four GEMMs with their slab sums: 192 -> 114 us (qkv 40.4 -> 24, o 27.3 -> 17, gate_up 76 -> 42,
+// down 48 -> 31); at 65 rows 128 -> 79; at 1300 rows 756 -> 629 us.
+#include <type_traits>
+
+#include "common.h"
+#include "wna16_rows.h"
+
+namespace aphro {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) void* lds_void_ptr;
+
+__device__ __forceinline__ uint32_t rw_and_or(uint32_t a, uint32_t mask, uint32_t orv) {
+  uint32_t r;
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(mask), "v"(orv));
+  return r;
+}
+// one exllama dword -> 8 scaled f16: ((1024 + q) - (1024 + z)) * s  (exact difference, one rounding)
+__device__ __forceinline__ f16x8 rw_dq8(uint32_t w, f16x2 zh, f16x2 zh16, f16x2 sc) {
+  const f16x2 inv16 = {(f16)0.0625f, (f16)0.0625f};
+  const uint32_t magic = 0x64006400u;
+  const uint32_t q0 = rw_and_or(w, 0x000f000fu, magic);
+  const uint32_t q1 = rw_and_or(w, 0x00f000f0u, magic);
+  const uint32_t w8 = w >> 8;
+  const uint32_t q2 = rw_and_or(w8, 0x000f000fu, magic);
+  const uint32_t q3 = rw_and_or(w8, 0x00f000f0u, magic);
+  const f16x2 d0 = (__builtin_bit_cast(f16x2, q0) - zh) * sc;
+  const f16x2 d1 = (__builtin_bit_cast(f16x2, q1) * inv16 + zh16) * sc;
+  const f16x2 d2 = (__builtin_bit_cast(f16x2, q2) - zh) * sc;
+  const f16x2 d3 = (__builtin_bit_cast(f16x2, q3) * inv16 + zh16) * sc;
+  u32x4 r = {__builtin_bit_cast(uint32_t, d0), __builtin_bit_cast(uint32_t, d1), __builtin_bit_cast(uint32_t, d2),
+             __builtin_bit_cast(uint32_t, d3)};
+  return __builtin_bit_cast(f16x8, r);
+}
+
+constexpr int RW_BN = 128, RW_BK = 128, RW_STAGES = 4;
+constexpr int rw_pass(int mb) { return (mb + 1) / 2; }      // 32-row blocks whose K groups meet in LDS at a time
+constexpr size_t rw_lds(int mb) {
+  const size_t stages = (size_t)RW_STAGES * mb * 32 * RW_BK * 2, meet = (size_t)8 * 3 * rw_pass(mb) * 2048;
+  return stages > meet ? stages : meet;
+}
+
+// Slabs of K slices are images of the accumulators: [ksplit][tile][32-row block][16-column group] of 2 KiB, a lane's two quads 1 KiB apart.
+__device__ __forceinline__ size_t rw_image(const Wna16RowsParams& p, int MB, int ks, int tile, int mb, int group) {
+  return (((size_t)ks * (p.tiles_m * p.tiles_n) + tile) * MB + mb) * 4096 + (size_t)group * 512;
+}
+
+template <int MB, bool BF16, bool STRIP>
+__global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p) {
+  constexpr int STAGE = MB * 32 * RW_BK * 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wn = wave & 1, kg = wave >> 1;
+  const int kh = lane >> 5, l31 = lane & 31;
+  // ---- which tile: contiguous ranges per XCD, the column tiles of one K slice and row tile next to each other -------------------
+  int lin;
+  {
+    const int n = gridDim.x, q = n / 8, r = n % 8, xcd = blockIdx.x % 8, k = blockIdx.x / 8;
+    lin = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + k;
+  }
+  const int tn = lin % p.tiles_n, rest = lin / p.tiles_n, tm = rest % p.tiles_m, ks = rest / p.tiles_m;
+  const int m0 = tm * MB * 32, n0 = tn * RW_BN;
+  const int T = p.K / RW_BK, t0 = ks * T / p.ksplit, t1 = (ks + 1) * T / p.ksplit;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a) + (size_t)m0 * p.lda, 0,
+                                                                      (uint32_t)((size_t)(p.M - m0) * p.lda * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qw), 0, (uint32_t)((size_t)(p.K >> 3) * p.N * 4), 0x00020000);
+  // ---- activations: one DMA instruction = 4 rows of 256 B, rows 32 apart from one to the next; LDS slot s of row r holds the row's
+  // slot s ^ (r & 15).  Rows from M on read zeros (the buffer ends there) or, where the offset wraps, some row: nobody stores theirs. ---
+  const int row0 = wave * 4 + (lane >> 4);
+  const int a_voff = (int)((uint32_t)row0 * (uint32_t)p.lda * 2u + (((lane & 15) ^ (row0 & 15)) << 4));
+  // ---- weights: the lane's columns are col and col + 1 (MFMA row i of block nb is column 2 i + nb) -------------------------------
+  const int col = n0 + wn * 64 + 2 * l31;
+  uint32_t w_voff, mult = 0;
+  if constexpr (STRIP) w_voff = wna16_strip_col(p.strip, col & ~3, mult) + (uint32_t)(col & 3) + mult * 64u * (uint32_t)kh;
+  else w_voff = (uint32_t)((kg * 4 + kh) * p.N + col);
+  w_voff *= 4u;
+  const uint32_t* scp = reinterpret_cast<const uint32_t*>(p.sc + col);
+  const uint32_t* zp = p.qz + (col >> 3);
+  const int zshift = (col & 7) * 4;
+  const int first_k = t0 * RW_BK + kg * 32, first_grp = first_k / p.group_size, first_in = first_k - first_grp * p.group_size;
+  int t_load = t0, grp = first_grp, in_group = first_in;  // the tile the next load fetches; its group, the k inside the group
+  const int grp_step = RW_BK / p.group_size, grp_rest = RW_BK - grp_step * p.group_size;
+  u32x2 wr[3][2];
+  uint32_t scr[3], zr[3];
+  auto load_w = [&](auto set) {
+    constexpr int S = decltype(set)::value;
+    scr[S] = scp[(size_t)grp * (p.N >> 1)];
+    zr[S] = zp[(size_t)grp * (p.N >> 3)];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if constexpr (STRIP) {
+        uint32_t chunk, R;
+        wna16_strip_row(p.strip, (uint32_t)(t_load * 16 + kg * 4), chunk, R);
+        wr[S][j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, (int)(w_voff + mult * (R + 128u * j) * 4u), (int)(chunk * 4u), 0));
+      } else {
+        wr[S][j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, (int)w_voff, (t_load * 16 + 2 * j) * p.N * 4, 0));
+      }
+    }
+  };
+  auto load_a = [&](int st, int i) {
+    const int voff = a_voff;                               // (a local copy: see wna16_gemm_large.hip)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_ptr)(smem + st * STAGE + (i * 8 + wave) * 1024), 16, voff,
+                                             (int)((uint32_t)t_load * (RW_BK * 2) + (uint32_t)i * 64u * (uint32_t)p.lda), 0, 0);
+  };
+  auto advance = [&] {
+    ++t_load;
+    grp += grp_step;
+    in_group += grp_rest;
+    if (in_group >= p.group_size) { in_group -= p.group_size; ++grp; }
+    if (t_load == t1) { t_load = t0; grp = first_grp; in_group = first_in; }      // (behind the last tile: straight-line code)
+  };
+  auto load = [&](auto set, int st) {
+    load_w(set);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) load_a(st, i);
+    advance();
+  };
+  constexpr int LOADS = MB + 4;                            // memory instructions of one load()
+  f32x16 acc[2][MB];
+#pragma unroll
+  for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[nb][mb][r] = 0.f;
+  // ---- K loop.  While a step's (16 k) MFMAs run, the next step's activations come from LDS and its weights are unpacked, across the
+  // tiles' borders too: halfway through a tile the next one has to be there -----------------------------------------------------------
+  u32x4 af[2][MB];
+  f16x8 wf[2][2];
+  f16x2 zh[2], zh16[2], sv[2];
+  const uint32_t a_base = (uint32_t)l31 * 256u;
+  auto read_a = [&](int stage, int j, u32x4 (&x)[MB]) {
+    const unsigned char* sa = smem + stage * STAGE + (a_base + (((uint32_t)(kg * 4 + 2 * j + kh) ^ (uint32_t)(l31 & 15)) << 4));
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) x[mb] = *reinterpret_cast<const u32x4*>(sa + mb * 8192);
+  };
+  auto meta = [&](auto set) {
+    constexpr int S = decltype(set)::value;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      const uint16_t sb = (uint16_t)(nb ? scr[S] >> 16 : scr[S]);
+      const int z = (int)((zr[S] >> (zshift + 4 * nb)) & 0xf) + p.zero_offset;
+      const f16 s16 = BF16 ? (f16)bf16_bits_to_f32(sb) : __builtin_bit_cast(f16, sb);
+      const f16 a16 = __builtin_bit_cast(f16, (uint16_t)(0x6400 | z));       // 1024 + z
+      const f16 b16 = (f16)960.f - a16;                                      // -64 - z
+      sv[nb] = f16x2{s16, s16};
+      zh[nb] = f16x2{a16, a16};
+      zh16[nb] = f16x2{b16, b16};
+    }
+  };
+  auto unpack = [&](auto set, auto step) {
+    constexpr int S = decltype(set)::value, J = decltype(step)::value;
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) wf[J][nb] = rw_dq8(wr[S][J][nb], zh[nb], zh16[nb], sv[nb]);
+  };
+  auto multiply = [&](auto step) {
+    constexpr int J = decltype(step)::value;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+        acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[J][nb], __builtin_bit_cast(f16x8, af[J][mb]), acc[nb][mb], 0, 0, 0);
+  };
+  int stage = 0;                                           // of the tile being multiplied
+  auto tile = [&](auto set, auto more) {
+    constexpr int S = decltype(set)::value;
+    read_a(stage, 1, af[1]);
+    unpack(set, std::integral_constant<int, 1>{});
+    multiply(std::integral_constant<int, 0>{});
+    if constexpr (decltype(more)::value) {
+      // the next tile has landed once at most the loads of ONE load(), the tile after it, are outstanding; past the barrier every wave
+      // is through with the tile BEFORE this one, whose stage the loads issued now take
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(LOADS) : "memory");
+      __builtin_amdgcn_s_barrier();
+    }
+    const int fetch = (stage + 3) & 3;
+    stage = (stage + 1) & 3;
+    read_a(stage, 0, af[0]);
+    meta(std::integral_constant<int, (S + 1) % 3>{});
+    unpack(std::integral_constant<int, (S + 1) % 3>{}, std::integral_constant<int, 0>{});
+    if constexpr (decltype(more)::value) {
+      // the loads go out between the MFMAs: all waves' at once would wait for one another with the matrix cores idle
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+          acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[1][nb], __builtin_bit_cast(f16x8, af[1][mb]), acc[nb][mb], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0x86);
+        if (mb == 0) load_w(set);
+        load_a(fetch, mb);
+        __builtin_amdgcn_sched_barrier(0x86);
+      }
+      advance();
+    } else {
+      multiply(std::integral_constant<int, 1>{});
+    }
+  };
+  constexpr std::integral_constant<int, 0> set0{};
+  constexpr std::integral_constant<int, 1> set1{};
+  constexpr std::integral_constant<int, 2> set2{};
+  load(set0, 0);
+  asm volatile("" ::: "memory");                           // (the counted waits rely on the order of the loads)
+  load(set1, 1);
+  asm volatile("" ::: "memory");
+  load(set2, 2);
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * LOADS) : "memory");
+  __builtin_amdgcn_s_barrier();
+  read_a(0, 0, af[0]);
+  meta(set0);
+  unpack(set0, std::integral_constant<int, 0>{});
+  int left = t1 - t0;
+  for (; left >= 3; left -= 3) {
+    tile(set0, std::true_type{});
+    tile(set1, std::true_type{});
+    tile(set2, std::true_type{});
+  }
+  // The last one or two tiles, in flight or landed.  They issue no loads: ones that nobody reads are dropped by the compiler, and a
+  // counted wait behind them would let a tile's own activations be outstanding.
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  if (left > 0) tile(set0, std::false_type{});
+  if (left > 1) tile(set1, std::false_type{});
+  // ---- the four K groups meet in LDS: the wave of group g ends with quad g of every block, columns 16 g + 8 kh + 2 r + nb ----------
+  constexpr int RM = rw_pass(MB);
+#pragma unroll
+  for (int m1 = 0; m1 < MB; m1 += RM) {
+    __syncthreads();
+    f32x4 own[2][RM];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (q != kg) {
+        unsigned char* dst = smem + (size_t)(((q * 2 + wn) * 3 + (kg ^ q) - 1) * RM) * 2048 + lane * 16;
+#pragma unroll
+        for (int i = 0; i < RM; ++i)
+          if (m1 + i < MB)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+              const f32x16& x = acc[nb][m1 + i < MB ? m1 + i : 0];
+              *reinterpret_cast<f32x4*>(dst + (i * 2 + nb) * 1024) = f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+            }
+      } else {
+#pragma unroll
+        for (int i = 0; i < RM; ++i)
+          if (m1 + i < MB)
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+              const f32x16& x = acc[nb][m1 + i < MB ? m1 + i : 0];
+              own[nb][i] = f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+            }
+      }
+    }
+    __syncthreads();
+    const unsigned char* src = smem + (size_t)((kg * 2 + wn) * 3 * RM) * 2048 + lane * 16;
+    // (v0 + v1) + (v2 + v3) whichever group the wave is: a column's bits do not depend on its place
+#pragma unroll
+    for (int i = 0; i < RM; ++i)
+      if (m1 + i < MB)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb) {
+          f32x4 v[3];
+#pragma unroll
+          for (int s = 0; s < 3; ++s) v[s] = *reinterpret_cast<const f32x4*>(src + (size_t)((s * RM + i) * 2 + nb) * 1024);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) own[nb][i][r] = (own[nb][i][r] + v[0][r]) + (v[1][r] + v[2][r]);
+        }
+#pragma unroll
+    for (int i = 0; i < RM; ++i) {
+      if (m1 + i >= MB) continue;
+      const int row = m0 + (m1 + i) * 32 + l31;
+      if (row >= p.M) continue;
+      const int c0 = n0 + wn * 64 + 16 * kg + 8 * kh;
+      const f32x4 x = own[0][i], y = own[1][i];
+      if (p.ksplit > 1) {
+        float* o = p.partial + rw_image(p, MB, ks, tm * p.tiles_n + tn, m1 + i, wn * 4 + kg) + lane * 4;
+        *reinterpret_cast<f32x4*>(o) = x;
+        *reinterpret_cast<f32x4*>(o + 256) = y;
+      } else if (p.silu) {
+        using T16 = std::conditional_t<BF16, BFloat, Half>;
+        u16x4 o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = silu_mul_bits<T16>(T16::to_f32(T16::from_f32(x[r])), T16::to_f32(T16::from_f32(y[r])));
+        *reinterpret_cast<u16x4*>(p.c + (size_t)row * (p.N / 2) + c0 / 2) = o;
+      } else {
+        const u32x4 o = {pack2_16<BF16>(x[0], y[0]), pack2_16<BF16>(x[1], y[1]), pack2_16<BF16>(x[2], y[2]), pack2_16<BF16>(x[3], y[3])};
+        *reinterpret_cast<u32x4*>(p.c + (size_t)row * p.N + c0) = o;
+      }
+    }
+  }
+}
+
+// The slabs summed in the order of K, one wave per image, and rounded.
+template <bool BF16>
+__global__ __launch_bounds__(256) void wna16_rows_reduce_kernel(Wna16RowsParams p, int MB) {
+  const int lane = threadIdx.x & 63, kh = lane >> 5, l31 = lane & 31;
+  const int img = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int group = img & 7, rest = img >> 3, mb = rest % MB, tile = rest / MB;
+  const int row = (tile / p.tiles_n * MB + mb) * 32 + l31;
+  if (row >= p.M) return;
+  const float* src = p.partial + rw_image(p, MB, 0, tile, mb, group) + lane * 4;
+  const size_t slab = (size_t)p.tiles_m * p.tiles_n * MB * 4096;
+  f32x4 x = *reinterpret_cast<const f32x4*>(src), y = *reinterpret_cast<const f32x4*>(src + 256);
+#pragma unroll 4
+  for (int s = 1; s < p.ksplit; ++s) {
+    x += *reinterpret_cast<const f32x4*>(src + s * slab);
+    y += *reinterpret_cast<const f32x4*>(src + s * slab + 256);
+  }
+  const u32x4 o = {pack2_16<BF16>(x[0], y[0]), pack2_16<BF16>(x[1], y[1]), pack2_16<BF16>(x[2], y[2]), pack2_16<BF16>(x[3], y[3])};
+  *reinterpret_cast<u32x4*>(p.c + (size_t)row * p.N + tile % p.tiles_n * RW_BN + group * 16 + kh * 8) = o;
+}
+
+// Tile height and K slices by the time they are expected to take (MI355X, ns; within 10 % of what was measured for 65 .. 4096 rows of
+// Llama-3-8B's and -70B's matrices): rounds of workgroups over the CUs, each 170 + 200 per 32-row block and K tile and 4.7 us around
+// them, and the slabs written and read again at 2.2 TB/s behind 3 us.  4096 x 14336, 150 rows: one slice 115 us, two 56, four 35, eight
+// 30; 4096 x 4096, 150 rows: five blocks and five slices 20.7, twice three blocks and four slices 18.0 us.
+Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t gs, int64_t slab_bytes, int64_t other_ns) {
+  Wna16RowsPlan best = {0, 1};
+  if (M <= 64 || M > 4096 || N % RW_BN || K % RW_BK || gs % 64) return best;
+  const int cus = device_cu_count();
+  const int64_t T = K / RW_BK;
+  int64_t best_ns = other_ns;
+  for (int mb = 3; mb <= 5; ++mb) {
+    const int64_t tiles_m = (M + mb * 32 - 1) / (mb * 32), tiles = tiles_m * (N / RW_BN);
+    for (int ks = 1; ks <= 16 && (ks == 1 || T / ks >= 4); ++ks) {
+      const int64_t slabs = tiles_m * mb * 32 * N * 4 * ks;
+      if (ks > 1 && slabs > slab_bytes) break;
+      const int64_t rounds = (tiles * ks + cus - 1) / cus;
+      const int64_t ns = rounds * ((T + ks - 1) / ks * (170 + 200 * mb) + 4700) + (ks > 1 ? 3000 + slabs * 45 / 100000 : 0);
+      if (best_ns < 0 || ns < best_ns) { best = {mb, ks}; best_ns = ns; }
+    }
+  }
+  return best;
+}
+
+template <int MB, bool BF16, bool STRIP>
+static int rows_launch(Wna16RowsParams p, hipStream_t st) {
+  p.tiles_m = (p.M + MB * 32 - 1) / (MB * 32);
+  p.tiles_n = p.N / RW_BN;
+  static bool attr_set_dev[APHRO_MAX_DEVICES] = {}; bool& attr_set = attr_set_dev[device_slot()];
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)wna16_gemm_rows_kernel<MB, BF16, STRIP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            160 * 1024) != hipSuccess) {
+      set_error("wna16_gemm_rows: cannot raise the dynamic LDS limit");
+      return APHRO_ERR_LAUNCH;
+    }
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((wna16_gemm_rows_kernel<MB, BF16, STRIP>), dim3(p.tiles_m * p.tiles_n * p.ksplit), dim3(512), rw_lds(MB), st, p);
+  APHRO_LAUNCH_CHECK();
+  if (p.ksplit > 1) {
+    hipLaunchKernelGGL(wna16_rows_reduce_kernel<BF16>, dim3(p.tiles_m * p.tiles_n * MB * 2), dim3(256), 0, st, p, MB);
+    APHRO_LAUNCH_CHECK();
+  }
+  return APHRO_OK;
+}
+
+template <int MB>
+static int rows_launch_mb(const Wna16RowsParams& p, hipStream_t st) {
+  if (p.bf16) return p.strip.on ? rows_launch<MB, true, true>(p, st) : rows_launch<MB, true, false>(p, st);
+  return p.strip.on ? rows_launch<MB, false, true>(p, st) : rows_launch<MB, false, false>(p, st);
+}
+
+int wna16_rows_launch(const Wna16RowsParams& p, const Wna16RowsPlan& plan, hipStream_t st) {
+  if (plan.mb == 3) return rows_launch_mb<3>(p, st);
+  if (plan.mb == 4) return rows_launch_mb<4>(p, st);
+  return rows_launch_mb<5>(p, st);
+}
+
+}  // namespace aphro

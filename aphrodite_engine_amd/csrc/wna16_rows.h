@@ -1,0 +1,29 @@
+// Host interface of wna16_gemm_rows.hip: int4 GEMM for 65 rows and more, tile heights that fit the batch.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "wna16_strip.h"
+
+namespace aphro {
+
+struct Wna16RowsParams {
+  const uint16_t* a;      // f16 [M, lda]
+  const uint32_t* qw;     // [K/8, N] exllama order, or the strip-major copy
+  const uint32_t* qz;     // [G, N/8]
+  const uint16_t* sc;     // [G, N]
+  uint16_t* c;            // [M, N], [M, N / 2] with SiluAndMul
+  float* partial;         // slabs when ksplit > 1
+  int M, N, K, lda;
+  int group_size, zero_offset, ksplit, silu;
+  int bf16;               // scales and results are bf16 (else f16)
+  int tiles_m, tiles_n;   // (filled by the launch)
+  Wna16StripGeom strip;
+};
+
+// 32-row blocks of a workgroup's tile (0: the kernel does not take the call, or needs longer than other_ns >= 0) and K slices, whose
+// slabs, ksplit x M rounded up to tiles x N floats, fit slab_bytes
+struct Wna16RowsPlan { int mb, ksplit; };
+Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t slab_bytes, int64_t other_ns);
+int wna16_rows_launch(const Wna16RowsParams& p, const Wna16RowsPlan& plan, hipStream_t st);
+
+}  // namespace aphro
