@@ -96,6 +96,10 @@ inline int aphro_lab_env_int(const char* name, int dflt) { const char* e = geten
 // and the shape takes the one-workgroup-per-tile + split-K plan, which has no cross-workgroup wait.
 inline int device_coresident_cu_count() { return knobs().cu_masked ? 0 : device_cu_count(); }
 
+// One block's words set to zero in front of a kernel that counts on them.  A kernel, not hipMemsetAsync: a caller may capture the
+// call, and memset nodes of a captured graph have left wrong values on replays after the first.
+static __global__ void clear_words_kernel(unsigned* words) { words[threadIdx.x] = 0u; }
+
 // Pair-major 16-bit activations between a fused producer and the AQ GEMM: element (row m, column k) of [M, K] sits at
 //   ((((k / 64) * mtiles + m / 16) * 2 + (k % 16) / 8) * 64 + ((k % 64) / 16) * 16 + m % 16) * 8 + k % 8      (16-bit elements)
 // i.e. for every (k-pair, 16-row tile, half) the 64 lanes' 16-byte pieces are one contiguous KiB in lane order: the consumer's

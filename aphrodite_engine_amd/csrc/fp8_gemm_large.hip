@@ -768,10 +768,8 @@ extern "C" int aphro_scaled_mm_fp8_large(void* out, const void* a, const void* b
   if (pl.streamk) {
     p.flags = (unsigned*)workspace;
     p.partial = (float*)((char*)workspace + FP8_LARGE_FLAG_BYTES);
-    if (hipMemsetAsync(p.flags, 0, FP8_LARGE_FLAG_BYTES, st) != hipSuccess) {
-      set_error("scaled_mm_fp8_large: cannot clear the stream-K flags");
-      return APHRO_ERR_LAUNCH;
-    }
+    hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(FP8_LARGE_FLAG_BYTES / 4), 0, st, p.flags);
+    APHRO_LAUNCH_CHECK();
   }
   int rc;
   // eight-phase schedule from 16 K tiles per output tile up: below that the longer prologue (seven half-tiles, the stagger

@@ -1018,16 +1018,14 @@ static size_t large_scratch_bytes(const LargePlan& pl, int64_t M, int64_t N) {
   return pl.ksplit > 1 ? (size_t)pl.ksplit * M * N * sizeof(float) : 0;
 }
 
-// stream-K: clear the flag words (a memset node in front of the kernel: replays in HIP graphs), point the kernel at them
+// stream-K: clear the flag words, point the kernel at them
 static int large_bind_scratch(Wna16LargeParams& p, const LargePlan& pl, char* ws, hipStream_t st) {
   p.streamk = pl.streamk; p.grid = pl.grid; p.ksplit = pl.ksplit; p.flags = nullptr; p.partial = (float*)ws;
   if (pl.streamk) {
     p.flags = (unsigned*)ws;
     p.partial = (float*)(ws + LARGE_FLAG_BYTES);
-    if (hipMemsetAsync(p.flags, 0, LARGE_FLAG_BYTES, st) != hipSuccess) {
-      set_error("wna16_gemm_large: cannot clear the stream-K flags");
-      return APHRO_ERR_LAUNCH;
-    }
+    hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(LARGE_FLAG_BYTES / 4), 0, st, p.flags);
+    APHRO_LAUNCH_CHECK();
   }
   return APHRO_OK;
 }
