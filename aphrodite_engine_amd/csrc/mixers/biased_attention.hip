@@ -220,6 +220,7 @@ extern "C" int aphro_distance_bias_attention(void* out, int64_t out_stride, cons
     p.lut_len = lut_len; p.temp_every = temp_every; p.scale = scale; p.temp_coef = temp_coef; p.out_scale = out_scale;
     p.ws = workspace;
     p.max_tiles = 0;
+    p.num_seqs = num_seqs; p.snake = 0;
     p.window = window; p.chunk = chunk; p.softcap = softcap; p.sink = sink; p.gate_cols = gate_cols;
     p.cap_in = softcap > 0.f ? 2.0f / softcap : 0.f;
     p.cap_out = softcap * 1.4426950408889634f;
@@ -233,9 +234,9 @@ extern "C" int aphro_distance_bias_attention(void* out, int64_t out_stride, cons
     const bool all_long = min_q_len >= DBA_MFMA_MIN_LEN;
     if (pf && (all_long || dc)) {
       p.min_len = DBA_MFMA_MIN_LEN;
-      if (form == DBA_MASKED) dba_prefill_launch<DBA_MASKED>(p, max_q_len, num_seqs, (hipStream_t)stream);
-      else if (form == DBA_GATED) dba_prefill_launch<DBA_GATED>(p, max_q_len, num_seqs, (hipStream_t)stream);
-      else dba_prefill_launch<DBA_PLAIN>(p, max_q_len, num_seqs, (hipStream_t)stream);
+      if (form == DBA_MASKED) dba_prefill_launch<DBA_MASKED>(p, num_tokens, max_q_len, num_seqs, (hipStream_t)stream);
+      else if (form == DBA_GATED) dba_prefill_launch<DBA_GATED>(p, num_tokens, max_q_len, num_seqs, (hipStream_t)stream);
+      else dba_prefill_launch<DBA_PLAIN>(p, num_tokens, max_q_len, num_seqs, (hipStream_t)stream);
       if (!all_long) {
         if (form == DBA_MASKED) dba_decode_launch<DBA_MASKED>(p, num_tokens, nsplit, (hipStream_t)stream);
         else if (form == DBA_GATED) dba_decode_launch<DBA_GATED>(p, num_tokens, nsplit, (hipStream_t)stream);

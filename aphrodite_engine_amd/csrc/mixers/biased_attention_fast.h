@@ -12,6 +12,7 @@
 //    S^T = K Q^T on v_mfma_f32_16x16x32_bf16, so that the probabilities come out in the B-operand layout of O^T = V^T P^T
 //    (keys of the two 16-key halves interleaved per lane group, V fragments read in the same order); temperature, bias,
 //    mask and the online softmax are fp32 on the accumulator registers.
+//  * dba_prefill32_kernel: the same for rows of 128 values, see there.
 //  * dba_decode_kernel<QH, CHL>: the other rows (single decoded tokens, short portions), one workgroup per (row, kv head)
 //    serving QH query heads of that kv head from one pass over the keys.  A key row is read by 2^CHL lanes x 16 bytes,
 //    64 / 2^CHL keys per load instruction (fully coalesced); the partial dot products fold over the lanes of a key with
@@ -516,6 +517,316 @@ __global__ void dba_merge_kernel(DBAParams p, int nsplit) {
   }
 }
 
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef short dba_s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* dba_lds_ptr;
+typedef const __attribute__((address_space(1))) void* dba_glb_ptr;
+
+constexpr int P32_BN = 64, P32_TILE = P32_BN * 256;          // keys of a tile, bytes of its K (or V) rows
+constexpr int p32_rows(int qt) { return 128 / qt; }
+constexpr int p32_pitch(int qt) { return p32_rows(qt) + 72; } // floats of a bias window: rows + 64, 32 bytes past a multiple of 128
+constexpr size_t p32_lds(int qt) { return 4 * P32_TILE + (size_t)2 * qt * 4 * p32_pitch(qt) * 4; }
+
+// The same attention for rows of 128 (the width of the models), on 32x32x16 products: a workgroup owns 128 / QT consecutive rows of QT
+// query heads of one kv head (QT = 4, 2, 1: as many as divide its heads), a wave 32 rows of one head.  Against dba_prefill_kernel a
+// fragment read from LDS feeds 32 columns instead of 16, K and V go from the cache to LDS without a stop in registers (V by whole rows,
+// its transpose is the transposing LDS read's), the temperature and the bias are one FMA on a score whose four biases are one aligned
+// LDS read, the output is rescaled only when some row's maximum moved, and one barrier a tile does.  Two workgroups share a CU.
+// Workgroups are numbered over the row tiles that the segments have, not over the longest segment's times their number: decoded rows
+// beside a prompt portion cost none.
+// Bound by a tile's chain of steps (products, softmax, products, 2 us) more than by any unit: without its exponentials, its products or its
+// loads it is 5 to 30 % faster each.  us before / after: 16 heads on 4, 4096 rows with bias 327 / 160, without 317 / 137; 2000 rows
+// behind 1024 keys, window 1024 84 / 42, with cap and bias 151 / 99; 32 heads on 8, three segments of 900 to 1400 rows with gate 147 / 86,
+// eight of 9 rows 35 / 23; 48 rows 20 / 20 (the launch).  V in the order [4 keys][16 bytes] of flash_attn.hip, for which four neighbouring
+// lanes read four rows: 192 for 164; fragments as hipcc orders them: 164 for 160; tiles begun at another key by every workgroup: no change.
+template <int QT, int FORM>
+__global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
+  constexpr bool EXT = FORM == DBA_MASKED;
+  constexpr int D = 128, R = p32_rows(QT), BP = p32_pitch(QT), NB = (QT * (R + 63) + 255) / 256;
+  constexpr float LOG2E = 1.4426950408889634f;
+  extern __shared__ __attribute__((aligned(16))) unsigned char dba_smem[];
+  float* bias_lds = reinterpret_cast<float*>(dba_smem + 4 * P32_TILE);      // [2][QT][4 copies][BP]
+  const int lane = threadIdx.x & 63, kh = lane >> 5, l31 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // ---- head unit and rank among the row tiles (numbering over the XCDs: see dba_prefill_kernel) ------------------------------------
+  int unit, rank;
+  {
+    constexpr int NX = 8;
+    const int G = p.kv_heads, QU = p.heads / p.kv_heads / QT, x = blockIdx.x % NX, j = blockIdx.x / NX;
+    if (G % NX == 0) {
+      const int ux = (G / NX) * QU, ul = j % ux;
+      rank = j / ux;
+      unit = ((ul / QU) * NX + x) * QU + ul % QU;
+    } else if (NX % G == 0) {
+      const int share = NX / G, pair = j * share + x / G;
+      rank = pair / QU;
+      unit = (x % G) * QU + pair % QU;
+    } else {
+      rank = blockIdx.x / (p.heads / QT);
+      unit = blockIdx.x % (p.heads / QT);
+    }
+  }
+  // ---- segment and row tile of the rank: the tiles of the segments one after the other, 64 segments a step ----------------------------
+  int seq = -1, ntiles = 0;
+  for (int base = 0; base < p.num_seqs && seq < 0; base += 64) {
+    const int len = base + lane < p.num_seqs ? p.q_len[base + lane] : 0;
+    const int n = len >= p.min_len ? (len + R - 1) / R : 0;
+    int sum = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(sum, d, 64);
+      if (lane >= d) sum += up;
+    }
+    const unsigned long long past = __builtin_amdgcn_ballot_w64(sum > rank);
+    if (past) {
+      const int at = __builtin_ctzll(past);
+      seq = base + at;
+      ntiles = __builtin_amdgcn_readlane(n, at);
+      rank -= __builtin_amdgcn_readlane(sum, at) - ntiles;
+    } else {
+      rank -= __builtin_amdgcn_readlane(sum, 63);
+    }
+  }
+  if (seq < 0) return;
+  // longest key ranges first; where every workgroup is resident at once, the second half shortest first: the two of a CU even out
+  int tile = ntiles - 1 - rank;
+  if (p.snake && rank >= (ntiles + 1) / 2) tile = rank - (ntiles + 1) / 2;
+  const int len = p.q_len[seq], ctx = p.ctx_len[seq], s0 = p.q_start[seq];
+  const int t = wave % QT, head = unit * QT + t, kvh = unit * QT / (p.heads / p.kv_heads);
+  const int q0 = tile * R, row0 = q0 + 32 * (wave / QT), qrow = row0 + l31, qpos = ctx + qrow;
+  const float qs = p.scale * dba_temp(p, qpos) * LOG2E;      // scores in units of ln 2: the exponentials are exp2
+  u32x4 qf[8];
+  {
+    const uint16_t* qp = p.q + (int64_t)(s0 + min(qrow, len - 1)) * p.q_stride + head * D + 8 * kh;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const u32x4*>(qp + 16 * ks);
+  }
+  const int32_t* bt = p.block_tables + (int64_t)seq * p.max_blocks;
+  const int nk = ctx + min(len, q0 + R);                     // keys the tile's last row sees
+  const int lo_row = EXT ? dba_first_key(p, qpos) : 0;
+  const int lo_wave0 = EXT ? dba_first_key(p, ctx + row0) : 0, lo_wave1 = EXT ? dba_first_key(p, ctx + row0 + 31) : 0;
+  const int t_first = EXT ? dba_first_key(p, ctx + q0) & ~(P32_BN - 1) : 0;
+  // ---- staging: a wave fetches 16 keys of a tile, 4 keys an instruction, lane L -> key L >> 4: a row's 64-byte lines are asked for by
+  // neighbouring lanes.  LDS slot L & 15 holds K's piece slot ^ (key & 15), V's piece slot ^ 4 (key & 3): fragment reads and transposing
+  // reads find their banks free -------------------------------------------------------------------------------------------------------
+  const int64_t row_bytes = (int64_t)p.kv_heads * D * 2;
+  const unsigned char* kb = reinterpret_cast<const unsigned char*>(p.k_cache) + kvh * D * 2;
+  const int64_t v_off = reinterpret_cast<const unsigned char*>(p.v_cache) - reinterpret_cast<const unsigned char*>(p.k_cache) +
+                        (((lane & 15) ^ ((lane >> 4) << 2)) << 4);
+  // block of the wave's 16 keys of the tile at t0 where they share one (past the last key: the last key's)
+  auto block_of = [&](int t0) {
+    if (p.bs_shift < 4) return 0;
+    const int blk = bt[min(t0 + 16 * wave, (nk - 1) & ~15) >> p.bs_shift];
+    return blk < 0 || blk >= p.num_blocks ? 0 : blk;         // never read outside the pool
+  };
+  auto fetch = [&](int buf, int t0, int blk, int j) {        // four keys of K and of V
+    const int key = min(t0 + 16 * wave + 4 * j + (lane >> 4), nk - 1);
+    const int64_t slot = p.bs_shift >= 4 ? ((int64_t)blk << p.bs_shift) + (key & (p.block_size - 1)) : dba_slot(p, bt, key);
+    const unsigned char* src = kb + slot * row_bytes;
+    unsigned char* dst = dba_smem + buf * 2 * P32_TILE + wave * 4096 + j * 1024;
+    __builtin_amdgcn_global_load_lds((dba_glb_ptr)(src + (((lane & 15) ^ (4 * j + (lane >> 4))) << 4)), (dba_lds_ptr)dst, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((dba_glb_ptr)(src + v_off), (dba_lds_ptr)(dst + P32_TILE), 16, 0, 0);
+  };
+  // ---- bias of a tile: entry x of a head's window is the distance (ctx + q0 - t0 + R - 1) - x; a row reads 4 neighbours at a time, and
+  // the copy shifted by its own misalignment makes them 16 aligned bytes -----------------------------------------------------------------
+  float bias_reg[NB];
+  auto bias_load = [&](int t0) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int x = threadIdx.x + 256 * i, h = x / (R + 63), e = x - h * (R + 63);
+      const int dist = ctx + q0 - t0 + R - 1 - e;
+      bias_reg[i] = h < QT ? p.bias_lut[(int64_t)(unit * QT + h) * p.lut_len + min(max(dist, 0), p.lut_len - 1)] * LOG2E : 0.f;
+    }
+  };
+  auto bias_store = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int x = threadIdx.x + 256 * i, h = x / (R + 63), e = x - h * (R + 63);
+      if (h < QT)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (e >= c) bias_lds[((buf * QT + h) * 4 + c) * BP + e - c] = bias_reg[i];
+    }
+  };
+  const int bx = R - 1 - (qrow - q0), bias_at = (t * 4 + (bx & 3)) * BP + (bx & ~3) + 4 * kh;
+  f32x16 o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+  float m_run = -1e28f, l_run = 0.f;                         // above a masked score: a row without a visible key so far adds nothing
+  const int kaddr = l31 * 256 + ((kh ^ (l31 & 15)) << 4);
+  // transposing read of 4 keys x 16 columns by 16 lanes: lane i asks for 8 bytes of key i >> 2 and gets column i of the four keys
+  const int vk = (lane & 15) >> 2;
+  const int vaddr = P32_TILE + kh * 1024 + vk * 256 + (vk << 6) + (((lane >> 4) & 1) << 5) + ((lane & 3) << 3);
+  {
+    const int b0 = block_of(t_first);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) fetch(0, t_first, b0, j);
+  }
+  if (p.bias_lut) {
+    bias_load(t_first);
+    bias_store(0);
+  }
+  int blk = block_of(t_first + P32_BN), buf = 0;
+  for (int t0 = t_first; t0 < nk; t0 += P32_BN, buf ^= 1) {
+    // this wave's part of the tile is there, and it is through with the other buffer
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    const bool more = t0 + P32_BN < nk;
+    if (more) {                                              // in flight during this tile's products
+      if (p.bias_lut) bias_load(t0 + P32_BN);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) fetch(buf ^ 1, t0 + P32_BN, blk, j);
+      blk = block_of(t0 + 2 * P32_BN);
+    }
+    if (t0 <= ctx + row0 + 31 && !(EXT && t0 + P32_BN <= lo_wave0)) {      // some key of the tile is seen by some row of the wave
+      const unsigned char* sb = dba_smem + buf * 2 * P32_TILE;
+      // (the order is fixed by hand: left to itself hipcc reads one pair of fragments, waits for it, multiplies, and so on)
+      f32x16 s[2];
+      u32x4 kf[8][2];
+      auto read_k = [&](int k0) {
+#pragma unroll
+        for (int ks = k0; ks < k0 + 4; ++ks)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) kf[ks][b] = *reinterpret_cast<const u32x4*>(sb + b * 8192 + (kaddr ^ (ks << 5)));
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto multiply_k = [&](int k0) {
+#pragma unroll
+        for (int ks = k0; ks < k0 + 4; ++ks)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+            const f32x16 zero = {};
+            s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[ks][b]), __builtin_bit_cast(bf16x8, qf[ks]), ks == 0 ? zero : s[b], 0, 0, 0);
+          }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      read_k(0);
+      read_k(4);
+      multiply_k(0);
+      multiply_k(4);
+      // lane's scores: row l31, keys t0 + 32 b + 8 q + 4 kh + r
+      if (EXT && p.softcap > 0.f) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[b][i] = dba_cap2(p, s[b][i] * qs);
+        if (p.bias_lut) {
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const f32x4 w = *reinterpret_cast<const f32x4*>(bias_lds + buf * QT * 4 * BP + bias_at + 32 * b + 8 * q);
+#pragma unroll
+              for (int r = 0; r < 4; ++r) s[b][4 * q + r] += w[r];
+            }
+        }
+      } else if (p.bias_lut) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x4 w = *reinterpret_cast<const f32x4*>(bias_lds + buf * QT * 4 * BP + bias_at + 32 * b + 8 * q);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[b][4 * q + r] = __builtin_fmaf(s[b][4 * q + r], qs, w[r]);
+          }
+      } else {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[b][i] *= qs;
+      }
+      if (t0 + P32_BN - 1 > ctx + row0) {                    // some key of the tile is ahead of some row of the wave
+        const int last = qpos - t0 - 4 * kh;
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[b][i] = 32 * b + 8 * (i >> 2) + (i & 3) <= last ? s[b][i] : -1e30f;
+      }
+      if (EXT && t0 < lo_wave1) {                            // ... or older than what some row of the wave sees
+        const int first = lo_row - t0 - 4 * kh;
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[b][i] = 32 * b + 8 * (i >> 2) + (i & 3) >= first ? s[b][i] : -1e30f;
+      }
+      float mx = -1e30f;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[b][i]);
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      float lsum = 0.f;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          s[b][i] = __builtin_amdgcn_exp2f(s[b][i] - m_new);      // a masked score is 1e30 below: exactly 0
+          lsum += s[b][i];
+        }
+      l_run = l_run * alpha + lsum;
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
+      }
+      // O^T += V^T P^T, 16 keys a step: k slots 4 h .. + 3 of lane half kh are keys 16 ks + 8 h + 4 kh .. + 3, the ones it has
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const f32x16& e = s[ks >> 1];
+        const int i0 = 8 * (ks & 1);
+        const u32x4 pf = {pack2_16<true>(e[i0], e[i0 + 1]), pack2_16<true>(e[i0 + 2], e[i0 + 3]), pack2_16<true>(e[i0 + 4], e[i0 + 5]),
+                          pack2_16<true>(e[i0 + 6], e[i0 + 7])};
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+          const unsigned char* va = sb + (vaddr ^ (db << 6)) + 4 * ks * 1024;
+          const dba_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((dba_s16x4 __attribute__((address_space(3)))*)va);
+          const dba_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((dba_s16x4 __attribute__((address_space(3)))*)(va + 2048));
+          const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+          o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, u32x4{l2[0], l2[1], h2[0], h2[1]}),
+                                                          __builtin_bit_cast(bf16x8, pf), o[db], 0, 0, 0);
+        }
+      }
+    }
+    if (more && p.bias_lut) bias_store(buf ^ 1);
+  }
+  float l = l_run + __shfl_xor(l_run, 32, 64);
+  if (qrow >= len) return;
+  float f = (l > 0.f ? 1.f / l : 0.f) * p.out_scale;
+  if (EXT && p.sink) {                                       // one more term of the denominator, without a value
+    const float s2 = p.sink[head] * LOG2E, M = fmaxf(m_run, s2), a = __builtin_amdgcn_exp2f(m_run - M);
+    f = a / (l * a + __builtin_amdgcn_exp2f(s2 - M)) * p.out_scale;
+  }
+  if (p.gate && !(FORM != DBA_PLAIN && p.gate_cols)) f *= sigmoid_f(BFloat::to_f32(p.gate[(int64_t)(s0 + qrow) * p.gate_stride + head]));
+  uint16_t* op = p.out + (int64_t)(s0 + qrow) * p.out_stride + head * D + 4 * kh;
+  const uint16_t* gp = FORM != DBA_PLAIN && p.gate && p.gate_cols ? p.gate + (int64_t)(s0 + qrow) * p.gate_stride + head * D + 4 * kh : nullptr;
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c0 = 32 * db + 8 * q;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = o[db][4 * q + r] * f;
+      if (p.vec4) {                                          // rows of out and gate are 8-byte aligned
+        if (FORM != DBA_PLAIN && gp) {
+          const u16x4 gv = *reinterpret_cast<const u16x4*>(gp + c0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] *= sigmoid_f(BFloat::to_f32(gv[r]));
+        }
+        *reinterpret_cast<u16x4*>(op + c0) = u16x4{BFloat::from_f32(v[0]), BFloat::from_f32(v[1]), BFloat::from_f32(v[2]), BFloat::from_f32(v[3])};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) op[c0 + r] = BFloat::from_f32(FORM != DBA_PLAIN && gp ? v[r] * sigmoid_f(BFloat::to_f32(gp[c0 + r])) : v[r]);
+      }
+    }
+}
+
 template <int DK, int QT, int FORM>
 static void launch_prefill_dv(const DBAParams& p, dim3 grid, hipStream_t st) {
   switch (p.vdim) {
@@ -536,8 +847,30 @@ static void launch_prefill_dk(const DBAParams& p, dim3 grid, hipStream_t st) {
   }
 }
 
+template <int QT, int FORM>
+static void launch_prefill32(const DBAParams& p0, int64_t num_tokens, int num_seqs, hipStream_t st) {
+  DBAParams p = p0;
+  constexpr int R = p32_rows(QT);
+  const int64_t most = num_tokens / R + (num_tokens / p.min_len < num_seqs ? num_tokens / p.min_len : num_seqs);     // row tiles there can be
+  const int64_t blocks = (most * (p.heads / QT) + 7) / 8 * 8;
+  p.num_seqs = num_seqs;
+  p.snake = num_seqs == 1 && blocks <= 2 * device_cu_count();
+  static bool attr_set_dev[APHRO_MAX_DEVICES] = {}; bool& attr_set = attr_set_dev[device_slot()];
+  if (!attr_set)
+    attr_set = hipFuncSetAttribute((const void*)dba_prefill32_kernel<QT, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p32_lds(QT)) == hipSuccess;
+  hipLaunchKernelGGL((dba_prefill32_kernel<QT, FORM>), dim3((unsigned)blocks), dim3(256), p32_lds(QT), st, p);
+}
+
 template <int FORM>
-void dba_prefill_launch(const DBAParams& p0, int max_q_len, int num_seqs, hipStream_t st) {
+void dba_prefill_launch(const DBAParams& p0, int64_t num_tokens, int max_q_len, int num_seqs, hipStream_t st) {
+  // (16-byte loads into LDS want 16-byte aligned rows: of 256 bytes times the kv heads, so aligned caches)
+  if (p0.dim == 128 && p0.vdim == 128 && (((uintptr_t)p0.k_cache | (uintptr_t)p0.v_cache) & 15) == 0) {
+    const int per_kv = p0.heads / p0.kv_heads;
+    if (per_kv % 4 == 0) launch_prefill32<4, FORM>(p0, num_tokens, num_seqs, st);
+    else if (per_kv % 2 == 0) launch_prefill32<2, FORM>(p0, num_tokens, num_seqs, st);
+    else launch_prefill32<1, FORM>(p0, num_tokens, num_seqs, st);
+    return;
+  }
   DBAParams p = p0;
   p.max_tiles = (max_q_len + PF_BM - 1) / PF_BM;
   const int qt = (p.heads / p.kv_heads) % 2 == 0 ? 2 : 1;   // two query heads of a kv head per workgroup where they pair up
