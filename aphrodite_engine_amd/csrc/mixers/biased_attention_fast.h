@@ -520,7 +520,6 @@ __global__ void dba_merge_kernel(DBAParams p, int nsplit) {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short dba_s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* dba_lds_ptr;
-typedef const __attribute__((address_space(1))) void* dba_glb_ptr;
 
 constexpr int P32_BN = 64, P32_TILE = P32_BN * 256;          // keys of a tile, bytes of its K (or V) rows
 constexpr int p32_rows(int qt) { return 128 / qt; }
@@ -535,9 +534,10 @@ constexpr size_t p32_lds(int qt) { return 4 * P32_TILE + (size_t)2 * qt * 4 * p3
 // Workgroups are numbered over the row tiles that the segments have, not over the longest segment's times their number: decoded rows
 // beside a prompt portion cost none.
 // Bound by a tile's chain of steps (products, softmax, products, 2 us) more than by any unit: without its exponentials, its products or its
-// loads it is 5 to 30 % faster each.  us before / after: 16 heads on 4, 4096 rows with bias 327 / 160, without 317 / 137; 2000 rows
-// behind 1024 keys, window 1024 84 / 42, with cap and bias 151 / 99; 32 heads on 8, three segments of 900 to 1400 rows with gate 147 / 86,
-// eight of 9 rows 35 / 23; 48 rows 20 / 20 (the launch).  V in the order [4 keys][16 bytes] of flash_attn.hip, for which four neighbouring
+// loads it is 5 to 30 % faster each.  us before / after: 16 heads on 4, 4096 rows with bias 327 / 152, without 317 / 125; 2000 rows
+// behind 1024 keys, window 1024 84 / 42, with cap and bias 151 / 97; 32 heads on 8, three segments of 900 to 1400 rows with gate 147 / 79,
+// eight of 9 rows 35 / 20; 48 rows 20 / 20 (the launch).  Loads by 64-bit addresses instead of buffer offsets: 160 for 152; loads between the
+// products: 170 to 208 (hipcc waits for them in front of the next LDS read).  V in the order [4 keys][16 bytes] of flash_attn.hip, for which four neighbouring
 // lanes read four rows: 192 for 164; fragments as hipcc orders them: 164 for 160; tiles begun at another key by every workgroup: no change.
 template <int QT, int FORM>
 __global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
@@ -609,10 +609,12 @@ __global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
   // ---- staging: a wave fetches 16 keys of a tile, 4 keys an instruction, lane L -> key L >> 4: a row's 64-byte lines are asked for by
   // neighbouring lanes.  LDS slot L & 15 holds K's piece slot ^ (key & 15), V's piece slot ^ 4 (key & 3): fragment reads and transposing
   // reads find their banks free -------------------------------------------------------------------------------------------------------
-  const int64_t row_bytes = (int64_t)p.kv_heads * D * 2;
+  // rows are addressed inside their block (or, in blocks of fewer than 16 keys, inside the whole cache, which then is below 4 GiB)
+  const uint32_t row_bytes = (uint32_t)p.kv_heads * D * 2;
+  const bool in_block = p.bs_shift >= 4;
+  const uint32_t span = (uint32_t)(in_block ? p.block_size : p.num_blocks * p.block_size) * row_bytes - kvh * D * 2;
   const unsigned char* kb = reinterpret_cast<const unsigned char*>(p.k_cache) + kvh * D * 2;
-  const int64_t v_off = reinterpret_cast<const unsigned char*>(p.v_cache) - reinterpret_cast<const unsigned char*>(p.k_cache) +
-                        (((lane & 15) ^ ((lane >> 4) << 2)) << 4);
+  const unsigned char* vb = reinterpret_cast<const unsigned char*>(p.v_cache) + kvh * D * 2;
   // block of the wave's 16 keys of the tile at t0 where they share one (past the last key: the last key's)
   auto block_of = [&](int t0) {
     if (p.bs_shift < 4) return 0;
@@ -621,11 +623,14 @@ __global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
   };
   auto fetch = [&](int buf, int t0, int blk, int j) {        // four keys of K and of V
     const int key = min(t0 + 16 * wave + 4 * j + (lane >> 4), nk - 1);
-    const int64_t slot = p.bs_shift >= 4 ? ((int64_t)blk << p.bs_shift) + (key & (p.block_size - 1)) : dba_slot(p, bt, key);
-    const unsigned char* src = kb + slot * row_bytes;
+    const uint32_t at = (uint32_t)(in_block ? key & (p.block_size - 1) : dba_slot(p, bt, key)) * row_bytes;
+    const int64_t base = in_block ? (int64_t)blk * p.block_size * row_bytes : 0;
     unsigned char* dst = dba_smem + buf * 2 * P32_TILE + wave * 4096 + j * 1024;
-    __builtin_amdgcn_global_load_lds((dba_glb_ptr)(src + (((lane & 15) ^ (4 * j + (lane >> 4))) << 4)), (dba_lds_ptr)dst, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((dba_glb_ptr)(src + v_off), (dba_lds_ptr)(dst + P32_TILE), 16, 0, 0);
+    const int ko = (int)(at + (((lane & 15) ^ (4 * j + (lane >> 4))) << 4)), vo = (int)(at + (((lane & 15) ^ ((lane >> 4) << 2)) << 4));
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(kb + base), 0, span, 0x00020000),
+                                             (dba_lds_ptr)dst, 16, ko, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(vb + base), 0, span, 0x00020000),
+                                             (dba_lds_ptr)(dst + P32_TILE), 16, vo, 0, 0, 0);
   };
   // ---- bias of a tile: entry x of a head's window is the distance (ctx + q0 - t0 + R - 1) - x; a row reads 4 neighbours at a time, and
   // the copy shifted by its own misalignment makes them 16 aligned bytes -----------------------------------------------------------------
@@ -863,8 +868,10 @@ static void launch_prefill32(const DBAParams& p0, int64_t num_tokens, int num_se
 
 template <int FORM>
 void dba_prefill_launch(const DBAParams& p0, int64_t num_tokens, int max_q_len, int num_seqs, hipStream_t st) {
-  // (16-byte loads into LDS want 16-byte aligned rows: of 256 bytes times the kv heads, so aligned caches)
-  if (p0.dim == 128 && p0.vdim == 128 && (((uintptr_t)p0.k_cache | (uintptr_t)p0.v_cache) & 15) == 0) {
+  // 16-byte loads into LDS want aligned caches (rows are 256 bytes times the kv heads); their 32-bit offsets a block below 4 GiB, or the
+  // whole cache where blocks are no multiples of 16 keys
+  const int64_t span = (p0.bs_shift >= 4 ? 1 : p0.num_blocks) * p0.block_size * (int64_t)p0.kv_heads * 256;
+  if (p0.dim == 128 && p0.vdim == 128 && (((uintptr_t)p0.k_cache | (uintptr_t)p0.v_cache) & 15) == 0 && span < (1ll << 32)) {
     const int per_kv = p0.heads / p0.kv_heads;
     if (per_kv % 4 == 0) launch_prefill32<4, FORM>(p0, num_tokens, num_seqs, st);
     else if (per_kv % 2 == 0) launch_prefill32<2, FORM>(p0, num_tokens, num_seqs, st);
