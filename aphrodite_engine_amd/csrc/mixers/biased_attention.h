@@ -22,7 +22,9 @@ struct DBAParams {
   float* ws;          // decode split partials [T, heads, nsplit, 2 + vdim]
   int bs_shift;       // log2(block_size), or -1 when it is no power of two
   int max_tiles;      // prompt kernel: 64-row tiles of the longest segment
-  int num_seqs, snake;     // 128-wide prompt kernel: segments; its workgroups are all resident at once
+  int num_seqs;       // segments
+  int snake;          // 128-wide prompt kernel: its workgroups are all resident at once
+  int mixed;          // decode kernel: its rows lie beside prompt portions'
   // the forms with a mask, a soft cap, a sink or an elementwise gate
   int window, chunk;  // 0: none
   float softcap;      // 0: none
@@ -36,14 +38,14 @@ bool dba_prefill_supported(int dim, int vdim);
 bool dba_decode_supported(int heads, int kv_heads, int dim, int vdim);
 // workgroups per decoded row (before the key range is split)
 int dba_decode_units(int heads, int kv_heads, int dim, int vdim);
-int dba_decode_splits(int64_t num_tokens, int units, int max_kv_len, int64_t ws_floats, int heads, int vdim);
+int dba_decode_splits(int64_t rows, int64_t num_tokens, int units, int max_kv_len, int64_t ws_floats, int heads, int vdim);
 // The forms of the kernels, a translation unit each: causal with a gate per head at most; window / chunk, soft cap, sink and elementwise
 // gate, chosen at run time; causal with an elementwise gate.
 enum DBAForm { DBA_PLAIN = 0, DBA_MASKED = 1, DBA_GATED = 2 };
 template <int FORM>
 void dba_prefill_launch(const DBAParams& p, int64_t num_tokens, int max_q_len, int num_seqs, hipStream_t st);
 template <int FORM>
-void dba_decode_launch(const DBAParams& p, int64_t num_tokens, int nsplit, hipStream_t st);
+void dba_decode_launch(const DBAParams& p, int64_t rows, int nsplit, hipStream_t st);
 constexpr int DBA_MFMA_MIN_LEN = 8;     // segments at least this long go to the matrix-core kernel
 
 }  // namespace aphro

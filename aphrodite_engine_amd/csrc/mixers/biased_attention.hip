@@ -220,7 +220,7 @@ extern "C" int aphro_distance_bias_attention(void* out, int64_t out_stride, cons
     p.lut_len = lut_len; p.temp_every = temp_every; p.scale = scale; p.temp_coef = temp_coef; p.out_scale = out_scale;
     p.ws = workspace;
     p.max_tiles = 0;
-    p.num_seqs = num_seqs; p.snake = 0;
+    p.num_seqs = num_seqs; p.snake = 0; p.mixed = 0;
     p.window = window; p.chunk = chunk; p.softcap = softcap; p.sink = sink; p.gate_cols = gate_cols;
     p.cap_in = softcap > 0.f ? 2.0f / softcap : 0.f;
     p.cap_out = softcap * 1.4426950408889634f;
@@ -228,19 +228,27 @@ extern "C" int aphro_distance_bias_attention(void* out, int64_t out_stride, cons
     p.bs_shift = -1;
     for (int sft = 0; sft < 20; ++sft)
       if ((1 << sft) == block_size) p.bs_shift = sft;
-    const int nsplit = workspace ? dba_decode_splits(num_tokens, dba_decode_units(heads, kv_heads, dim, vdim), visible, workspace_floats, heads, vdim) : 1;
     const bool pf = dba_prefill_supported(dim, vdim) && max_q_len >= DBA_MFMA_MIN_LEN;
     const bool dc = dba_decode_supported(heads, kv_heads, dim, vdim);
     const bool all_long = min_q_len >= DBA_MFMA_MIN_LEN;
+    // rows the decode kernel can have: all, or beside prompt portions those of shorter segments (mostly one token each: the key ranges
+    // are split for as many rows as there are segments)
+    int64_t rows = num_tokens, likely = num_tokens;
+    if (pf && dc && !all_long) {
+      p.mixed = 1;
+      rows = min(num_tokens, (int64_t)(DBA_MFMA_MIN_LEN - 1) * num_seqs);
+      likely = min(num_tokens, (int64_t)num_seqs);
+    }
+    const int nsplit = workspace ? dba_decode_splits(likely, num_tokens, dba_decode_units(heads, kv_heads, dim, vdim), visible, workspace_floats, heads, vdim) : 1;
     if (pf && (all_long || dc)) {
       p.min_len = DBA_MFMA_MIN_LEN;
       if (form == DBA_MASKED) dba_prefill_launch<DBA_MASKED>(p, num_tokens, max_q_len, num_seqs, (hipStream_t)stream);
       else if (form == DBA_GATED) dba_prefill_launch<DBA_GATED>(p, num_tokens, max_q_len, num_seqs, (hipStream_t)stream);
       else dba_prefill_launch<DBA_PLAIN>(p, num_tokens, max_q_len, num_seqs, (hipStream_t)stream);
       if (!all_long) {
-        if (form == DBA_MASKED) dba_decode_launch<DBA_MASKED>(p, num_tokens, nsplit, (hipStream_t)stream);
-        else if (form == DBA_GATED) dba_decode_launch<DBA_GATED>(p, num_tokens, nsplit, (hipStream_t)stream);
-        else dba_decode_launch<DBA_PLAIN>(p, num_tokens, nsplit, (hipStream_t)stream);
+        if (form == DBA_MASKED) dba_decode_launch<DBA_MASKED>(p, rows, nsplit, (hipStream_t)stream);
+        else if (form == DBA_GATED) dba_decode_launch<DBA_GATED>(p, rows, nsplit, (hipStream_t)stream);
+        else dba_decode_launch<DBA_PLAIN>(p, rows, nsplit, (hipStream_t)stream);
       }
       APHRO_LAUNCH_CHECK();
       return APHRO_OK;

@@ -43,6 +43,43 @@ __device__ __forceinline__ float dba_temp(const DBAParams& p, int pos) {
   return p.temp_coef != 0.f ? 1.0f + p.temp_coef * logf((float)((pos + 1) / p.temp_every + 1)) : 1.0f;
 }
 
+// Segment of a rank among items that the segments have `count(q_len)` of, one segment's after the other's (-1: there are fewer); rank
+// becomes the item's number in its segment, mine the segment's items.  One wave, 64 segments a step.
+template <typename F>
+__device__ __forceinline__ int dba_segment(const DBAParams& p, int& rank, int& mine, F count) {
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < p.num_seqs; base += 64) {
+    const int n = base + lane < p.num_seqs ? count(p.q_len[base + lane]) : 0;
+    int sum = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(sum, d, 64);
+      if (lane >= d) sum += up;
+    }
+    const unsigned long long past = __builtin_amdgcn_ballot_w64(sum > rank);
+    if (past) {
+      const int at = __builtin_ctzll(past);
+      mine = __builtin_amdgcn_readlane(n, at);
+      rank -= __builtin_amdgcn_readlane(sum, at) - mine;
+      return base + at;
+    }
+    rank -= __builtin_amdgcn_readlane(sum, 63);
+  }
+  return -1;
+}
+
+// Row and segment of the decode kernel's workgroup number `x` (-1: none).  Beside prompt portions only the rows of short segments are
+// numbered: 2000 portion rows would otherwise start and end thousands of workgroups, and the key ranges be split for their number.
+__device__ __forceinline__ int dba_short_row(const DBAParams& p, int x, int& seq) {
+  if (!p.mixed) {
+    seq = p.seq_of_token[x];
+    return p.q_len[seq] >= p.min_len ? -1 : x;
+  }
+  int mine;
+  seq = dba_segment(p, x, mine, [&](int len) { return len < p.min_len ? len : 0; });
+  return seq < 0 ? -1 : p.q_start[seq] + x;
+}
+
 // Oldest key the row at `pos` sees: its window's first key, its chunk's first key, or key 0.
 __device__ __forceinline__ int dba_first_key(const DBAParams& p, int pos) {
   int lo = 0;
@@ -357,9 +394,10 @@ __global__ __launch_bounds__(256) void dba_decode_kernel(DBAParams p) {
   // grid y: the kv heads, each with the groups of QH query heads that cover its own (the last group may be partly empty:
   // its surplus lanes repeat the kv head's last query head and write nothing)
   const int per_kv = p.heads / p.kv_heads, groups = (per_kv + QH - 1) / QH;
-  const int t = blockIdx.x, kvh = blockIdx.y / groups, sub0 = (blockIdx.y % groups) * QH, hbase = kvh * per_kv;
-  const int seq = p.seq_of_token[t];
-  if (p.q_len[seq] >= p.min_len) return;                   // the prompt kernel's share
+  const int kvh = blockIdx.y / groups, sub0 = (blockIdx.y % groups) * QH, hbase = kvh * per_kv;
+  int seq;
+  const int t = dba_short_row(p, blockIdx.x, seq);
+  if (t < 0) return;                                       // the prompt kernel's share
   const int pos = p.ctx_len[seq] + (t - p.q_start[seq]);
   const int k0 = EXT ? dba_first_key(p, pos) : 0;          // oldest visible key
   const int nkeys = pos + 1;
@@ -497,8 +535,10 @@ __global__ __launch_bounds__(256) void dba_decode_kernel(DBAParams p) {
 
 template <int FORM>
 __global__ void dba_merge_kernel(DBAParams p, int nsplit) {
-  const int t = blockIdx.x, head = blockIdx.y;
-  if (p.q_len[p.seq_of_token[t]] >= p.min_len) return;
+  const int head = blockIdx.y;
+  int seq;
+  const int t = dba_short_row(p, blockIdx.x, seq);
+  if (t < 0) return;
   const float* w = p.ws + ((int64_t)t * p.heads + head) * nsplit * (2 + p.vdim);
   float M = -INFINITY;
   for (int z = 0; z < nsplit; ++z) M = fmaxf(M, w[z * (2 + p.vdim)]);
@@ -566,27 +606,9 @@ __global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
       unit = blockIdx.x % (p.heads / QT);
     }
   }
-  // ---- segment and row tile of the rank: the tiles of the segments one after the other, 64 segments a step ----------------------------
-  int seq = -1, ntiles = 0;
-  for (int base = 0; base < p.num_seqs && seq < 0; base += 64) {
-    const int len = base + lane < p.num_seqs ? p.q_len[base + lane] : 0;
-    const int n = len >= p.min_len ? (len + R - 1) / R : 0;
-    int sum = n;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int up = __shfl_up(sum, d, 64);
-      if (lane >= d) sum += up;
-    }
-    const unsigned long long past = __builtin_amdgcn_ballot_w64(sum > rank);
-    if (past) {
-      const int at = __builtin_ctzll(past);
-      seq = base + at;
-      ntiles = __builtin_amdgcn_readlane(n, at);
-      rank -= __builtin_amdgcn_readlane(sum, at) - ntiles;
-    } else {
-      rank -= __builtin_amdgcn_readlane(sum, 63);
-    }
-  }
+  // ---- segment and row tile of the rank: the tiles of the segments one after the other ------------------------------------------------
+  int ntiles = 0;
+  const int seq = dba_segment(p, rank, ntiles, [&](int len) { return len >= p.min_len ? (len + R - 1) / R : 0; });
   if (seq < 0) return;
   // longest key ranges first; where every workgroup is resident at once, the second half shortest first: the two of a CU even out
   int tile = ntiles - 1 - rank;
@@ -858,7 +880,6 @@ static void launch_prefill32(const DBAParams& p0, int64_t num_tokens, int num_se
   constexpr int R = p32_rows(QT);
   const int64_t most = num_tokens / R + (num_tokens / p.min_len < num_seqs ? num_tokens / p.min_len : num_seqs);     // row tiles there can be
   const int64_t blocks = (most * (p.heads / QT) + 7) / 8 * 8;
-  p.num_seqs = num_seqs;
   p.snake = num_seqs == 1 && blocks <= 2 * device_cu_count();
   static bool attr_set_dev[APHRO_MAX_DEVICES] = {}; bool& attr_set = attr_set_dev[device_slot()];
   if (!attr_set)
@@ -904,8 +925,8 @@ static int decode_qh(int heads, int kv_heads, int chl) {
 }
 
 template <int FORM>
-void dba_decode_launch(const DBAParams& p, int64_t num_tokens, int nsplit, hipStream_t st) {
-  const dim3 grid((unsigned)num_tokens, (unsigned)dba_decode_units(p.heads, p.kv_heads, p.dim, p.vdim), (unsigned)nsplit);
+void dba_decode_launch(const DBAParams& p, int64_t rows, int nsplit, hipStream_t st) {
+  const dim3 grid((unsigned)rows, (unsigned)dba_decode_units(p.heads, p.kv_heads, p.dim, p.vdim), (unsigned)nsplit);
   const int chl = decode_chl(p.dim, p.vdim), qh = decode_qh(p.heads, p.kv_heads, chl);
 #define DEC(QH, CHL) hipLaunchKernelGGL((dba_decode_kernel<QH, CHL, FORM>), grid, dim3(256), 0, st, p)
 #define DEC_BY_CHL(QH)                          \
@@ -924,7 +945,7 @@ void dba_decode_launch(const DBAParams& p, int64_t num_tokens, int nsplit, hipSt
 #undef DEC_BY_CHL
 #undef DEC
   if (nsplit > 1)
-    hipLaunchKernelGGL((dba_merge_kernel<FORM>), dim3((unsigned)num_tokens, (unsigned)p.heads), dim3(64), 0, st, p, nsplit);
+    hipLaunchKernelGGL((dba_merge_kernel<FORM>), dim3((unsigned)rows, (unsigned)p.heads), dim3(64), 0, st, p, nsplit);
 }
 
 }  // namespace aphro

@@ -18,9 +18,9 @@ int dba_decode_units(int heads, int kv_heads, int dim, int vdim) {
 }
 
 // Key splits of the decode kernel: enough workgroups to fill the chip, at least four 64-key tiles (one per wave) each.
-int dba_decode_splits(int64_t num_tokens, int units, int max_kv_len, int64_t ws_floats, int heads, int vdim) {
+int dba_decode_splits(int64_t rows, int64_t num_tokens, int units, int max_kv_len, int64_t ws_floats, int heads, int vdim) {
   const int tiles = (max_kv_len + 63) / 64;
-  int64_t n = (1024 + num_tokens * units - 1) / (num_tokens * units);
+  int64_t n = (1024 + rows * units - 1) / (rows * units);
   if (n > tiles / 4) n = tiles / 4;
   if (n > 8) n = 8;
   while (n > 1 && num_tokens * heads * n * (2 + vdim) > ws_floats) --n;

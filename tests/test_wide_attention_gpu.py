@@ -96,10 +96,13 @@ def test_forms(heads, kv_heads, kw):
     run([200, 9, 70], [33, 300, 0], heads, kv_heads, 16, seed=heads, **kw)
 
 
-def test_rows_shorter_than_a_segment_go_the_other_way_beside_it():
-    """Decoded rows among prompt portions, more than 64 segments of them."""
-    lens = [1] * 70 + [90] + [3] * 5 + [40]
-    run(lens, [i % 37 + 8 for i in range(len(lens))], 8, 2, 16, bias=64, fill=0.0)
+@pytest.mark.parametrize("kw", [dict(bias=64), dict(window=600, sink=True), dict(gate="columns", pad=1)])
+@pytest.mark.parametrize("block,ctx", [(16, 8), (24, 700)])
+def test_short_segments_beside_prompt_portions(kw, block, ctx):
+    """Decoded rows and portions of up to 7 tokens before, among and behind prompt portions, more than 64 segments of them; with the longer
+    contexts their key ranges are split."""
+    lens = [2] + [1] * 70 + [90] + [3] * 5 + [40, 7, 1]
+    run(lens, [i * 13 % 37 + ctx for i in range(len(lens))], 8, 2, block, fill=0.0, **kw)
 
 
 def test_a_column_s_bits_do_not_depend_on_the_batch():
