@@ -574,9 +574,9 @@ constexpr size_t p32_lds(int qt) { return 4 * P32_TILE + (size_t)2 * qt * 4 * p3
 // Workgroups are numbered over the row tiles that the segments have, not over the longest segment's times their number: decoded rows
 // beside a prompt portion cost none.
 // Bound by a tile's chain of steps (products, softmax, products, 2 us) more than by any unit: without its exponentials, its products or its
-// loads it is 5 to 30 % faster each.  us before / after: 16 heads on 4, 4096 rows with bias 327 / 152, without 317 / 125; 2000 rows
-// behind 1024 keys, window 1024 84 / 42, with cap and bias 151 / 97; 32 heads on 8, three segments of 900 to 1400 rows with gate 147 / 79,
-// eight of 9 rows 35 / 20; 48 rows 20 / 20 (the launch).  Loads by 64-bit addresses instead of buffer offsets: 160 for 152; loads between the
+// loads it is 5 to 30 % faster each.  us before / after: 16 heads on 4, 4096 rows with bias 327 / 157, without 317 / 135; 2000 rows
+// behind 1024 keys, window 1024 84 / 42, with cap and bias 151 / 98; 32 heads on 8, three segments of 900 to 1400 rows with gate 147 / 82,
+// eight of 9 rows 35 / 21; 48 rows 20 / 20 (the launch).  Loads by 64-bit addresses instead of buffer offsets: 160 for 157; loads between the
 // products: 170 to 208 (hipcc waits for them in front of the next LDS read).  V in the order [4 keys][16 bytes] of flash_attn.hip, for which four neighbouring
 // lanes read four rows: 192 for 164; fragments as hipcc orders them: 164 for 160; tiles begun at another key by every workgroup: no change.
 template <int QT, int FORM>
