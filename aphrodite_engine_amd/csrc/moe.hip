@@ -338,8 +338,9 @@ __global__ __launch_bounds__(1024) void moe_route_align_kernel(
 
 // fused_topk + moe_align_block_size for PROMPT-sized batches with <= 16 experts: the one-workgroup form ranks its slots in one wave (118 us at
 // 6000 slots of 8 experts); here a workgroup routes 256 tokens, thread = token with moe_route_row16's arithmetic, and counts its experts; the
-// second launch sums the counts ahead of it and places its slots.  A token names an expert once, so a slot's rank among its workgroup's is
-// the number of earlier threads that name the expert: a ballot per expert and wave.  Same weights, ids and slot order.
+// second launch sums the counts ahead of it and places its slots.  A slot's rank among its workgroup's is the number of earlier slots that
+// name the expert: a ballot per expert, choice and wave.  (Not one per expert: where a row's logits are not finite no probability compares
+// greater, and the token names expert 0 with every choice.)  Same weights, ids and slot order.
 constexpr int MRB_TOKENS = 256;
 template <typename T>
 __global__ __launch_bounds__(MRB_TOKENS) void moe_route_blocks_kernel(float* __restrict__ topk_weights, int32_t* __restrict__ topk_ids,
@@ -394,19 +395,23 @@ __global__ __launch_bounds__(MRB_TOKENS) void moe_align_blocks_kernel(const int3
   }
   const int tok = blockIdx.x * MRB_TOKENS + tid;
   int mine[8], rank[8];
-  unsigned chosen = 0;                                  // experts of the token, one bit each
 #pragma unroll
   for (int kk = 0; kk < 8; ++kk) {
     mine[kk] = kk < k && tok < num_tokens ? topk_ids[(size_t)tok * k + kk] : -1;
-    if (mine[kk] >= 0) chosen |= 1u << mine[kk];
     rank[kk] = 0;
   }
   for (int e = 0; e < num_experts; ++e) {
-    const unsigned long long mask = __ballot((chosen >> e) & 1);
-    if (lane == 0) wcnt[wave][e] = __popcll(mask);
+    int below = 0, total = 0;
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+      const unsigned long long mask = __ballot(mine[kk] == e);
+      below += __popcll(mask & ((1ull << lane) - 1ull));
+      total += __popcll(mask);
+    }
+    if (lane == 0) wcnt[wave][e] = total;
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk)
-      if (mine[kk] == e) rank[kk] = __popcll(mask & ((1ull << lane) - 1ull));
+      if (mine[kk] == e) rank[kk] = below++;
   }
   __syncthreads();
 #pragma unroll

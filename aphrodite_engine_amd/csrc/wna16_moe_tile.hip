@@ -37,6 +37,7 @@ struct MoeTileParams {
   const int32_t* num_post_pad;
   uint16_t* act;              // SiluAndMul output f16 [m_pad, N / 2], or
   float* out;                 // [ksplit, m_pad, N]
+  uint32_t a_bytes;           // of a, its last row to K
   int numel, topk, lda, N, K, group_size, zero_offset;
   int m_pad, ksplit;
 };
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(WM * 256) void wna16_moe_tile_kernel(MoeTileParams 
   const uint32_t* qz = p.qz + ((size_t)e * G_all + g_begin) * (p.N >> 3) + (n0 >> 3);
   const uint16_t* sc = p.sc + ((size_t)e * G_all + g_begin) * p.N + n0;
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(qw), 0, (uint32_t)((size_t)(p.K >> 3) * p.N * 4), 0x00020000);
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a), 0, 0xffffffffu, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a), 0, p.a_bytes, 0x00020000);
   // ---- scales and zero points of the columns for the K range ----------------------------------------------------------------------
   uint16_t* meta_sc = reinterpret_cast<uint16_t*>(smem + STAGES * STAGE);
   uint32_t* meta_z = reinterpret_cast<uint32_t*>(smem + STAGES * STAGE + G * MT_BN * 2);
@@ -119,7 +120,7 @@ __global__ __launch_bounds__(WM * 256) void wna16_moe_tile_kernel(MoeTileParams 
     int src = m0 + row;
     if (p.slots != nullptr) {
       const int sl = p.slots[src];
-      src = (sl < p.numel ? sl : 0) / p.topk;               // (a padding row multiplies some token's row; nobody reads the result)
+      src = ((uint32_t)sl < (uint32_t)p.numel ? sl : 0) / p.topk;               // (a padding row multiplies some token's row; nobody reads the result)
     }
     a_voff[i] = ((uint32_t)src * (uint32_t)p.lda + slot * 8) * 2;
   }
@@ -376,6 +377,7 @@ extern "C" int aphro_wna16_moe_tile(const void* a, int64_t rows, int64_t lda, co
               "wna16_moe_tile: operand exceeds 4 GiB");
   APHRO_CHECK(sorted_slots != nullptr ? numel >= 1 && (numel - 1) / topk < rows : m_pad <= rows, "wna16_moe_tile: rows outside the activations");
   MoeTileParams p;
+  p.a_bytes = (uint32_t)(((rows - 1) * lda + K) * 2);
   p.a = (const uint16_t*)a; p.slots = sorted_slots; p.qw = q_weight; p.qz = qzeros; p.sc = (const uint16_t*)scales;
   p.expert_ids = expert_ids; p.num_post_pad = num_tokens_post_pad; p.act = (uint16_t*)act; p.out = out;
   p.numel = (int)numel; p.topk = topk; p.lda = (int)lda; p.N = (int)N; p.K = (int)K; p.group_size = (int)(K / groups);

@@ -83,6 +83,39 @@ def test_route_align_blocks_is_route_align(tokens, e, topk, block, dtype):
             assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("e,topk,block", [(8, 2, 64), (16, 8, 128), (3, 3, 64)])
+def test_routing_places_every_slot_of_rows_that_are_not_finite(e, topk, block):
+    """A row with a NaN, a +inf, or of -inf only names expert 0 with every choice: in several waves and workgroups, first and last."""
+    from aphrodite_engine_amd import _custom_ops as ops
+    tokens = 700
+    logits = torch.randn(tokens, e, device=DEV)
+    for i, t in enumerate((0, 1, 63, 64, 100, 255, 256, 400, 401, 699)):
+        logits[t] = (float("nan"), -float("inf"))[i % 2]
+        if i % 3 == 0:
+            logits[t] = 0.5
+            logits[t, i % e] = (float("inf"), float("nan"))[i % 2]
+    a = ops.moe_route_align_blocks(logits, topk, True, e, block)
+    b = ops.moe_route_align(logits, topk, True, e, block, True)
+    for x, y in zip(a, b):
+        assert torch.equal(x.nan_to_num(-1.0), y.nan_to_num(-1.0))
+    order = a[2][: int(a[4])].tolist()
+    assert sorted(i for i in order if i < tokens * topk) == list(range(tokens * topk))
+    assert all(order[p] == i for i, p in enumerate(a[5].tolist()))
+
+
+def test_a_token_without_a_finite_logit_leaves_the_others():
+    """The prompt-sized experts with such tokens in the batch: everyone else's output is what it is without them."""
+    from aphrodite_engine_amd import moe as M
+    experts, _, _ = experts_of(8, 512, 512, torch.float16, "gptq", 11)
+    x, logits = torch.randn(300, 512, device=DEV).half(), torch.randn(300, 8, device=DEV).half()
+    want = M.fused_wna16_moe(x, experts, logits, 2, True)
+    assert M.moe_tile_block(600, experts, torch.float16)
+    logits[17], logits[64, 5], logits[299] = float("nan"), float("inf"), -float("inf")
+    got = M.fused_wna16_moe(x, experts, logits, 2, True)
+    rest = [t for t in range(300) if t not in (17, 64, 299)]
+    assert torch.equal(got[rest], want[rest])
+
+
 def test_route_align_blocks_many_tokens():
     """More slots than the one-workgroup form holds: against the separate ops."""
     from aphrodite_engine_amd import _custom_ops as ops
