@@ -342,7 +342,8 @@ __device__ __forceinline__ void ar_norm_row(const u32x4 (&xs)[2], const uint16_t
       if (res_row) *reinterpret_cast<u16x8*>(res_row + 8 * i) = rs;
       if (res_pub) *reinterpret_cast<u16x8*>(res_pub + 8 * i) = rs;
       {
-        // squares rounded, then added (what hipcc emits for add_rms_norm_pack_kernel's input path: v_pk_mul_f32 + adds)
+        // squares, then their sum in add_rms_norm_pack_kernel's order; squares of 16-bit numbers are exact in fp32, so the bits are
+        // those of its input path whether hipcc contracts there or not
 #pragma clang fp contract(off)
 #pragma unroll
         for (int j = 0; j < 8; ++j) ss += v[it][j] * v[it][j];

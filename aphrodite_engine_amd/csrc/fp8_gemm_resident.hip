@@ -30,8 +30,8 @@
 //     A fragment is quantised in registers in front of its MFMAs: fp8(x / scale) with the IEEE quotient.  The quotient is
 //     hipcc's own fp32 division sequence (v_rcp, one Newton step on the reciprocal, q = n r, residual corrections) with
 //     the per-ROW part -- reciprocal + its refinement -- hoisted and ONE residual correction (proven sufficient for every
-//     (input, scale) pair that can occur, see F8R_DIV_STEPS): 3 VALU per element, packed two at a time (v_pk_mul_f32 /
-//     v_pk_fma_f32), on |x| with the sign put back on the packed bytes (-0 stays -0 as v_div_fixup_f32 would leave it).
+//     (input, scale) pair that can occur, see F8R_DIV_STEPS): 3 VALU per element
+//     (v_mul_f32, two v_fma_f32), on |x| with the sign put back on the packed bytes (-0 stays -0 as v_div_fixup_f32 would leave it).
 //     v_div_scale_f32 is the identity for every finite 16-bit x and scale in [1 / (448 * 512), 65504 / 448]; the clamp to
 //     +-448 is a no-op when |x| <= absmax.  tests: aphro_fp8_quant_rows_aq runs the same device function over all 65 536
 //     f16 / bf16 inputs x adversarial scales against x / scale.

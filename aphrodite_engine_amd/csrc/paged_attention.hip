@@ -648,7 +648,10 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t*
 #pragma unroll
           for (int w = 0; w < NW; ++w) {
             float wt = __expf(ml[(w * 16 + h) * 2] - M);
-            L += ml[(w * 16 + h) * 2 + 1] * wt;
+            {   // products rounded, then added: the outputs must not depend on what hipcc contracts
+#pragma clang fp contract(off)
+              L += ml[(w * 16 + h) * 2 + 1] * wt;
+            }
             acc += *reinterpret_cast<const f32x4*>(&ov[((size_t)w * p.nh_lds + h) * HD + d]) * wt;
           }
           st_wt_f32x4(slot + h * HD + d, acc);

@@ -381,8 +381,8 @@ __global__ __launch_bounds__(NWV * 64, NWV <= 4 ? 1 : 2) void wna16_gemm_residen
         const float nzs = -z * sf;
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-          // (packed f32 FMAs: the scalar-FMA form VERDICT r4 asked about -- 945 v_fma_f32 instead of 437 v_pk_fma_f32 in the
-          //  gate_up instantiation -- measured the same to +-0.1 us on all four projections, profiles/r5_decode_experiments.txt)
+          // (945 v_fma_f32 in the gate_up instantiation; 437 v_pk_fma_f32, which the library is built without, measured the same to
+          //  +-0.1 us on all four projections, profiles/r5_decode_experiments.txt)
           cacc[i][t] = __builtin_elementwise_fma(acc[i][t], f32x4{s24, s24, s24, s24}, cacc[i][t]);
           cacc[i][t] = __builtin_elementwise_fma(rs[i], f32x4{nzs, nzs, nzs, nzs}, cacc[i][t]);
         }
