@@ -500,12 +500,14 @@ def wna16_large_ok(m: int, n: int, k: int, groups: int) -> bool:
         and (k // 8) * n * 4 < 2 ** 32 and m * k * 2 < 2 ** 32
 
 
-def wna16_prefers_large(m: int, n: int, k: int, dtype=None) -> bool:
-    """Which of 65 to 128 rows leave the decode kernel (two 64-row passes over the weights).  float16, K a multiple of 128: all of them,
-    for the tile whose height fits the batch (csrc/wna16_gemm_rows.hip; 6144 x 4096 at 65 / 128 rows 20.5 / 25.1 -> 16.2 / 22 us, 4096 x
-    4096 19.1 / 24.6 -> 15.5 / 23 us, errors 2.9e-4 -> 2.1e-4).  Else the large matrices only: the decode kernel applies the group
-    scales in fp32, the tiles round scale and weight to float16, which a bfloat16 scale below 6e-5 would not survive unchanged."""
-    return m > 128 or n * k >= 2 ** 25 or (dtype == torch.float16 and k % 128 == 0)
+def wna16_prefers_large(m: int, n: int, k: int) -> bool:
+    """Between 65 and 128 rows the small projections (weights < 16 MiB) stay with the decode kernel (two 64-row passes over the weights):
+    it multiplies exact integers and applies the group scales to fp32 sums, where the tiles round every scaled weight to 16 bits --
+    a float16 result's error against 64 bits grows from 2.1e-4 (its own rounding) to 2.9e-4.  In time the tile whose height fits the
+    batch (csrc/wna16_gemm_rows.hip) would win: 6144 x 4096 at 65 / 128 rows 16.2 / 22 against 20.5 / 25.1 us, 4096 x 4096 15.5 / 23
+    against 19.1 / 24.6 us.  The large matrices go to the tiles (gate_up 59 vs 52 us, down 43 vs 35 us at 96 rows before that
+    tile; tools/mid_gemm_bench.py, profiles/r2_mid_gemm.txt)."""
+    return m > 128 or n * k >= 2 ** 25
 
 
 def _wna16_large(a, qweight, qzeros, scales, perm, zero_offset):
@@ -592,7 +594,7 @@ def wna16_linear_strip(a: torch.Tensor, strip: torch.Tensor, qzeros: torch.Tenso
     if m == 0:
         return torch.empty((0, n), dtype=a.dtype, device=a.device)
     large = wna16_large_ok(m, n, k, groups) and not switch("APHRO_WNA16_NO_LARGE")
-    if large and wna16_prefers_large(m, n, k, a.dtype):
+    if large and wna16_prefers_large(m, n, k):
         return wna16_gemm_large_strip(a, strip, qzeros, scales, zero_offset, strip_m=strip_m)
     if wna16_prefers_mid(m, n, k) and wna16_mid_ok(m, n, k, groups) and a.dtype == scales.dtype and not switch("APHRO_WNA16_NO_MID"):
         # 33..64 rows on the big matrices: ONE pass of the 32x32x16 kernel over the strip-major words (the generic op's own rule)
@@ -660,7 +662,7 @@ def _wna16_mid(a, qweight, qzeros, scales, perm, zero_offset):
 def _wna16(a, qweight, qzeros, scales, perm, zero_offset):
     m, k = a.shape
     n = qweight.shape[1]
-    if wna16_large_ok(m, n, k, scales.shape[0]) and wna16_prefers_large(m, n, k, a.dtype) \
+    if wna16_large_ok(m, n, k, scales.shape[0]) and wna16_prefers_large(m, n, k) \
             and not switch("APHRO_WNA16_NO_LARGE"):
         return _wna16_large(a, qweight, qzeros, scales, perm, zero_offset)
     if wna16_prefers_mid(m, n, k) and wna16_mid_ok(m, n, k, scales.shape[0]) and not switch("APHRO_WNA16_NO_MID"):
@@ -701,7 +703,7 @@ def gptq_gemm(a: torch.Tensor, b_q_weight: torch.Tensor,
         raise RuntimeError(f"gptq_gemm: weight width {bit} is not one of 2, 3, 4, 8")
     m = a.shape[0]
     large = use_exllama and wna16_large_ok(m, b_q_weight.shape[1], a.shape[1], b_gptq_scales.shape[0]) \
-        and wna16_prefers_large(m, b_q_weight.shape[1], a.shape[1], a.dtype) and not switch("APHRO_WNA16_NO_LARGE")
+        and wna16_prefers_large(m, b_q_weight.shape[1], a.shape[1]) and not switch("APHRO_WNA16_NO_LARGE")
     if not use_exllama or (m >= GPTQ_DEQUANT_MIN_M and not large):
         w = gptq_dequant(b_q_weight, b_gptq_qzeros, b_gptq_scales, b_g_idx,
                          use_exllama, bit)

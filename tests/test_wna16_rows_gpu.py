@@ -44,7 +44,7 @@ def test_rows_gemm(dtype, group, m, k, n):
     for _ in range(3):
         assert torch.equal(ops._wna16_large(a, qw, qz, sc, None, 1), got)
     assert torch.equal(ops.gptq_gemm(a, qw, qz, sc, torch.empty(0, dtype=torch.int32, device=DEV), True, 4), got) \
-        or not ops.wna16_prefers_large(m, n, k, dtype)
+        or not ops.wna16_prefers_large(m, n, k)
     if ops.wna16_gemm_large_silu_supported(m, n, k, k // group):
         act = ops.wna16_gemm_large_silu(a, qw, qz, sc, 1)
         gate, up = got[:, 0::2].contiguous(), got[:, 1::2].contiguous()
@@ -54,8 +54,24 @@ def test_rows_gemm(dtype, group, m, k, n):
     if group == 128 and ops.wna16_resident_ksplit(32, n, k, k // 128) > 0:
         strip = ops.wna16_strip_relayout(qw, 32, k // 128)
         assert torch.equal(ops.wna16_gemm_large_strip(a, strip, qz, sc, 1), got)
-        if m > 128 or ops.wna16_prefers_large(m, n, k, dtype):
+        if m > 128 or ops.wna16_prefers_large(m, n, k):
             assert torch.equal(ops.wna16_linear_strip(a, strip, qz, sc, 1), got)
+
+
+@pytest.mark.parametrize("m", [65, 96, 97, 128])
+@pytest.mark.parametrize("k,n", [(4096, 4096), (4096, 6144), (2048, 4096)])
+def test_small_projections_do_not_round_their_weights(m, k, n):
+    """float16, 65 to 128 rows, by the public entries: no further from 64 bits than the rounding of the exact result is (the fp32 sums add
+    a hundredth of it; weights rounded to float16 as well add four tenths)."""
+    from aphrodite_engine_amd import _custom_ops as ops
+    qw, qz, sc, g = weights(k, n, 128, torch.float16, m + n)
+    a = torch.randn(m, k, generator=g, device=DEV).half()
+    want = a.double() @ dense(qw, qz, sc, 1)
+    bound = 1.02 * float((want.half().double() - want).norm())
+    got = [ops.gptq_gemm(a, qw, qz, sc, torch.empty(0, dtype=torch.int32, device=DEV), True, 4)]
+    if ops.wna16_resident_ksplit(32, n, k, k // 128) > 0:
+        got.append(ops.wna16_linear_strip(a, ops.wna16_strip_relayout(qw, 32, k // 128), qz, sc, 1))
+    assert all(float((x.double() - want).norm()) < bound for x in got)
 
 
 def test_rows_gemm_keeps_a_row_s_infinities_and_nans_to_itself():
