@@ -1040,15 +1040,16 @@ static bool large_eight(const LargePlan& pl, int64_t K) {
 
 // The tile of wna16_gemm_rows.hip, up to 4096 rows: always where this file would take one workgroup per tile (4096 x 4096: 150 rows
 // 27.3 -> 18.3 us, 1300 rows 78 -> 56 us), and beside the stream-K form where its last round is full enough (28672 x 4096: 300 rows
-// 127 -> 82 us, 1300 rows 341 -> 326 us; 2048 rows 450 against 489 us: stays).  Its slabs fit the workspace of this file's
-// plan; a call that is not sliced here is not sliced there: the SiluAndMul form and the plain GEMM have the same bits.
+// 127 -> 82 us, 1300 rows 341 -> 326 us; 2048 rows 450 against 489 us: stays).  Its K slices are its own, of any whole K tiles up to 36 MiB of slabs;
+// this file's are ranges of whole groups, of which 11008 or 9728 rows of K have few divisors and one group per column none (4096 x 11008 at 65
+// / 150 / 300 rows with slices bound to this file's 53 / 54 / 54 us, without 21 / 28 / 40 us).
 static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs) {
   int64_t other_ns = -1;
   if (pl.streamk) {            // 1.9 us per 256 x 256 x 64 of a CU's even share, 18 us around them
     const int64_t units = (M + 255) / 256 * ((N + 255) / 256) * (K / 64);
     other_ns = 18000 + units * 1900 / pl.grid;
   }
-  return wna16_rows_plan(M, N, K, gs, pl.streamk ? 0 : (int64_t)large_scratch_bytes(pl, M, N), other_ns < 0 ? -1 : other_ns * 97 / 100);
+  return wna16_rows_plan(M, N, K, gs, pl.streamk ? 0 : 36ll << 20, other_ns < 0 ? -1 : other_ns * 97 / 100);
 }
 
 static size_t large_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype, int strip_m) {
@@ -1057,7 +1058,8 @@ static size_t large_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t gro
   size_t b = dtype == APHRO_BF16 ? ((size_t)M * K * 2 + 255) / 256 * 256 : 0;
   if (large_two_pass(pl, M, N, K, K / groups)) b += ((size_t)N * K * 2 + 255) / 256 * 256;      // f16 W^T of the two-pass form
   (void)strip_m;              // (every plan addresses the strip-major copy in place: nothing is rebuilt)
-  return b + large_scratch_bytes(pl, M, N);
+  const size_t slabs = wna16_rows_slab_bytes(rows_plan(pl, M, N, K, K / groups), M, N), other = large_scratch_bytes(pl, M, N);
+  return b + (slabs > other ? slabs : other);
 }
 
 // Bytes of scratch aphro_wna16_gemm_large needs: the f16 copy of bf16 activations + the fp32 split-K slabs.

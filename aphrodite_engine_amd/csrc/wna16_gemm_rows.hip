@@ -304,7 +304,7 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   }
 }
 
-// The slabs summed in the order of K, one wave per image, and rounded.
+// The slabs summed in the order of K, one wave per image, and rounded (SiluAndMul behind it as in the kernel itself).
 template <bool BF16>
 __global__ __launch_bounds__(256) void wna16_rows_reduce_kernel(Wna16RowsParams p, int MB) {
   const int lane = threadIdx.x & 63, kh = lane >> 5, l31 = lane & 31;
@@ -320,8 +320,17 @@ __global__ __launch_bounds__(256) void wna16_rows_reduce_kernel(Wna16RowsParams 
     x += *reinterpret_cast<const f32x4*>(src + s * slab);
     y += *reinterpret_cast<const f32x4*>(src + s * slab + 256);
   }
+  const int c0 = tile % p.tiles_n * RW_BN + group * 16 + kh * 8;
+  if (p.silu) {
+    using T16 = std::conditional_t<BF16, BFloat, Half>;
+    u16x4 a;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) a[r] = silu_mul_bits<T16>(T16::to_f32(T16::from_f32(x[r])), T16::to_f32(T16::from_f32(y[r])));
+    *reinterpret_cast<u16x4*>(p.c + (size_t)row * (p.N / 2) + c0 / 2) = a;
+    return;
+  }
   const u32x4 o = {pack2_16<BF16>(x[0], y[0]), pack2_16<BF16>(x[1], y[1]), pack2_16<BF16>(x[2], y[2]), pack2_16<BF16>(x[3], y[3])};
-  *reinterpret_cast<u32x4*>(p.c + (size_t)row * p.N + tile % p.tiles_n * RW_BN + group * 16 + kh * 8) = o;
+  *reinterpret_cast<u32x4*>(p.c + (size_t)row * p.N + c0) = o;
 }
 
 // Tile height and K slices by the time they are expected to take (MI355X, ns; within 10 % of what was measured for 65 .. 4096 rows of
@@ -373,6 +382,11 @@ template <int MB>
 static int rows_launch_mb(const Wna16RowsParams& p, hipStream_t st) {
   if (p.bf16) return p.strip.on ? rows_launch<MB, true, true>(p, st) : rows_launch<MB, true, false>(p, st);
   return p.strip.on ? rows_launch<MB, false, true>(p, st) : rows_launch<MB, false, false>(p, st);
+}
+
+size_t wna16_rows_slab_bytes(const Wna16RowsPlan& plan, int64_t M, int64_t N) {
+  const int64_t bm = plan.mb * 32;
+  return plan.mb > 0 && plan.ksplit > 1 ? (size_t)((M + bm - 1) / bm * bm * N * 4 * plan.ksplit) : 0;
 }
 
 int wna16_rows_launch(const Wna16RowsParams& p, const Wna16RowsPlan& plan, hipStream_t st) {

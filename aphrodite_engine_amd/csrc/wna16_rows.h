@@ -24,6 +24,8 @@ struct Wna16RowsParams {
 // slabs, ksplit x M rounded up to tiles x N floats, fit slab_bytes
 struct Wna16RowsPlan { int mb, ksplit; };
 Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t slab_bytes, int64_t other_ns);
+// bytes of Wna16RowsParams::partial
+size_t wna16_rows_slab_bytes(const Wna16RowsPlan& plan, int64_t M, int64_t N);
 int wna16_rows_launch(const Wna16RowsParams& p, const Wna16RowsPlan& plan, hipStream_t st);
 
 }  // namespace aphro

@@ -49,6 +49,9 @@ def test_int4_gemm_plans_through_their_workspace_sizes():
     # round 6, from 6144 rows: + the f16 W^T [N, K] of the two-pass form (dequantised once per call instead of once per row tile)
     assert large(8192, 28672, 4096) == 28672 * 4096 * 2 + 4096 + 256 * 8 * 32 * 1024
     assert large(256, 28672, 4096, ) % 256 == 0
+    # up to 4096 rows the row tile takes K slices of its own, whatever divisors the number of groups has (11008 / 128 = 2 x 43; one group)
+    assert large(65, 4096, 11008) == 8 * slab(96, 4096) and large(150, 4096, 11008) == 8 * slab(160, 4096)
+    assert L.aphro_wna16_gemm_large_workspace_bytes(150, 4096, 4096, 1, 0) >= 4 * slab(150, 4096)
     mid_ok = lambda m, n, k: L.aphro_wna16_gemm_mid_supported(m, n, k, k // 128)
     mid = lambda m, n, k: L.aphro_wna16_gemm_mid_workspace_bytes(m, n, k, k // 128)
     assert mid_ok(64, 28672, 4096) and mid_ok(1, 128, 512) and not mid_ok(65, 28672, 4096)
