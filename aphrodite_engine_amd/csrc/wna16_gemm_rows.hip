@@ -81,8 +81,9 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
                                                                       (uint32_t)((size_t)(p.M - m0) * p.lda * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qw), 0, (uint32_t)((size_t)(p.K >> 3) * p.N * 4), 0x00020000);
   // ---- activations: one DMA instruction = 4 rows of 256 B, rows 32 apart from one to the next; LDS slot s of row r holds the row's
-  // slot s ^ (r & 15).  Rows from M on read zeros (the buffer ends there) or, where the offset wraps, some row: nobody stores theirs. ---
-  const int row0 = wave * 4 + (lane >> 4);
+  // slot s ^ (r & 15).  Rows from M on read zeros (the buffer ends there); 32-row blocks that begin behind M read the last one that does
+  // not, because a scalar offset past the buffer's end is not certain to fail the range check.  Nobody stores either. ------------------
+  const int row0 = wave * 4 + (lane >> 4), last_block = (p.M - m0 - 1) >> 5;
   const int a_voff = (int)((uint32_t)row0 * (uint32_t)p.lda * 2u + (((lane & 15) ^ (row0 & 15)) << 4));
   // ---- weights: the lane's columns are col and col + 1 (MFMA row i of block nb is column 2 i + nb) -------------------------------
   const int col = n0 + wn * 64 + 2 * l31;
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   auto load_a = [&](int st, int i) {
     const int voff = a_voff;                               // (a local copy: see wna16_gemm_large.hip)
     __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_ptr)(smem + st * STAGE + (i * 8 + wave) * 1024), 16, voff,
-                                             (int)((uint32_t)t_load * (RW_BK * 2) + (uint32_t)i * 64u * (uint32_t)p.lda), 0, 0);
+                                             (int)((uint32_t)t_load * (RW_BK * 2) + (uint32_t)min(i, last_block) * 64u * (uint32_t)p.lda), 0, 0);
   };
   auto advance = [&] {
     ++t_load;
