@@ -133,13 +133,16 @@ class Wna16Experts:
 MOE_TILE_ROWS, MOE_TILE_WIDE = 24, 768
 
 
-def moe_tile_block(slots: int, experts: Wna16Experts, dtype: torch.dtype) -> int:
-    """Rows of a block of the tile GEMM for a batch of ``slots`` (token, expert) pairs; 0: the decode kernel's batch or shape."""
+def moe_tile_block(slots: int, experts: Wna16Experts, dtype: torch.dtype, a_bytes: int = 0) -> int:
+    """Rows of a block of the tile GEMM for a batch of ``slots`` (token, expert) pairs whose activations span ``a_bytes``; 0: the decode
+    kernel's batch or shape."""
     e = experts.num_experts
     if slots < MOE_TILE_ROWS * e or dtype != experts.w13[2].dtype:
         return 0
     bm = 64 if slots < MOE_TILE_WIDE * e else 128
     blocks = (slots + e * (bm - 1) + bm - 1) // bm
+    if max(a_bytes, blocks * bm * experts.inter * 2) >= 2 ** 32 - 1:       # rows of either GEMM by 32-bit offsets: Mixtral's from 74 000 tokens on
+        return 0
     for (qw, _, sc), k, silu in ((experts.w13, experts.hidden, True), (experts.w2, experts.inter, False)):
         # (what the decode kernel refuses stays refused whatever the batch)
         if ops.wna16_moe_tile_ksplit(blocks, qw.shape[2], k, sc.shape[1], bm, silu) <= 0 \
@@ -171,7 +174,7 @@ def fused_wna16_moe(hidden_states: torch.Tensor, experts: Wna16Experts, gating_o
     m = hidden_states.shape[0]
     e = experts.num_experts
     packed = None
-    bm = moe_tile_block(m * topk, experts, hidden_states.dtype) if aligned is None else 0
+    bm = moe_tile_block(m * topk, experts, hidden_states.dtype, m * hidden_states.stride(0) * 2) if aligned is None else 0
     if bm:
         if topk_ids is not None:
             sorted_ids, expert_ids, post_pad, inv = moe_align_block_size(topk_ids, bm, e, want_inverse=True)

@@ -758,3 +758,16 @@ def test_lab_patches_apply_to_the_product_sources():
         with open(pf) as f:
             r = subprocess.run(["patch", "--dry-run", "-s", "-p0", target], stdin=f, capture_output=True, text=True)
         assert r.returncode == 0, (os.path.basename(pf), r.stdout[-400:], r.stderr[-400:])
+
+
+def test_expert_tile_leaves_batches_beyond_32_bit_offsets_to_the_decode_kernel():
+    """moe.moe_tile_block at the sizes its kernel refuses: 4 GiB of activations in front of either GEMM."""
+    from types import SimpleNamespace
+    from aphrodite_engine_amd import moe as M
+    hidden, inter, e = 4096, 14336, 8
+    w = lambda k, n: tuple(torch.empty(e, r, c, dtype=t, device="meta") for r, c, t in
+                           ((k // 8, n, torch.int32), (k // 128, n // 8, torch.int32), (k // 128, n, torch.float16)))
+    experts = SimpleNamespace(num_experts=e, hidden=hidden, inter=inter, w13=w(hidden, 2 * inter), w2=w(inter, hidden))
+    most = (2 ** 32 - 2) // (inter * 2) // 128 * 128 - e * 127           # slots whose blocks of 128 rows just fit
+    assert M.moe_tile_block(most, experts, torch.float16) == 128 and M.moe_tile_block(most + 128, experts, torch.float16) == 0
+    assert M.moe_tile_block(6000, experts, torch.float16, 2 ** 32 - 2) == 64 and M.moe_tile_block(6000, experts, torch.float16, 2 ** 32 - 1) == 0
