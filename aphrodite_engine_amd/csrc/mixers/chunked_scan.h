@@ -64,6 +64,35 @@ inline int64_t max_chunks(int64_t num_tokens, int num_seqs, int min_len) {
   return num_tokens / CHUNK + (longs < num_seqs ? longs : num_seqs);
 }
 
+// A call's chunks run in spans of as many as the workspace holds, the state between them in the state tensors (fp32, as the chunks carry it: the
+// span's length does not show in the results).  Chunks [begin, end) of segment s in the span from chunk id ``chunk0`` on; ``first``: where
+// the segment's chunk 0 would lie in the span's arrays.
+constexpr int64_t SPAN_BYTES = 256 << 20;       // 38 chunks of 32 heads of the delta rule's 128 x 128, the widest: enough for the chip.  16384 tokens in spans
+// against all at once: delta rule 16 / 32 heads 1712 / 2687 -> 1748 / 2682 us, state space of 64 heads 1227 -> 1310 us
+__device__ __forceinline__ bool span_of(int s, int nc, const int32_t* __restrict__ q_len, int min_len, int chunk0, int span, int& begin, int& end, int64_t& first) {
+  const int64_t rel = (int64_t)chunks_before(s, q_len, min_len) - chunk0;
+  first = rel;
+  begin = rel < 0 ? (int)-rel : 0;
+  end = rel + nc > span ? (int)(span - rel) : nc;
+  return begin < end;
+}
+
+// The most of ``chunks`` chunks whose parts, floats(n) floats of n chunks, fit ``bytes``.
+template <typename F>
+inline int64_t span_chunks(int64_t chunks, int64_t bytes, F floats) {
+  const int64_t fixed = floats(0), four = floats(4) - fixed;
+  int64_t n = (bytes / 4 - fixed) / four * 4 + 4;
+  if (n > chunks) n = chunks;
+  while (n > 0 && floats(n) * 4 > bytes) --n;
+  return n;
+}
+template <typename F>
+inline int64_t span_workspace(int64_t chunks, F floats) {
+  int64_t n = span_chunks(chunks, floats(0) * 4 + SPAN_BYTES, floats);
+  if (n < 1) n = chunks < 1 ? chunks : 1;
+  return floats(n) * 4;
+}
+
 // Inclusive prefix sum over the wave, in 64 bits: differences of two prefixes keep a small decay exact behind a large one.
 __device__ __forceinline__ double wave_incl_sum(double v, int lane) {
 #pragma unroll

@@ -29,6 +29,7 @@ constexpr int GDC_P = CHUNK + 4;         // pitch of [.., 64] rows in LDS: 4 flo
 struct GDChunk {
   GatedDelta p;
   int min_len;
+  int chunk0, span;        // the chunks of these launches (below: [chunks] of one span)
   int vpad;                // vdim rounded up to 16
   float* w;                // [chunks, heads, 64, DP]  T (Pi K)
   float* qg;               // [chunks, heads, 64, DP]  Pi Q
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
   int* bad_tok = bad_col + CHUNK;          // [1]
   const GatedDelta& p = a.p;
   int s, c;
-  if (!locate_chunk(blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
   const int slot = p.slot_of_seq[s];
   if (slot < 0 || slot >= p.num_slots) return;
   const int h = blockIdx.y, hk = h / (p.heads / p.kv_heads);
@@ -393,12 +394,14 @@ __global__ __launch_bounds__(256) void gd_chunk_carry_kernel(GDChunk a) {
   const int s = blockIdx.z, h = blockIdx.x, c0 = blockIdx.y * 16;
   const int n = p.q_len[s], slot = p.slot_of_seq[s];
   if (n < a.min_len || slot < 0 || slot >= p.num_slots) return;
-  const int nc = (n + CHUNK - 1) / CHUNK;
-  const int64_t first = chunks_before(s, p.q_len, a.min_len);
+  int begin, nc;
+  int64_t first;
+  if (!span_of(s, (n + CHUNK - 1) / CHUNK, p.q_len, a.min_len, a.chunk0, a.span, begin, nc, first)) return;
+  first += begin, nc -= begin;                             // (chunks are numbered from the span's first from here on)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
   const int col = c0 + li;
   float* sb = p.state + ((int64_t)slot * p.heads + h) * p.dim * (int64_t)p.vdim + col;
-  const bool fresh = p.ctx_len[s] == 0;
+  const bool fresh = begin == 0 && p.ctx_len[s] == 0;
   f32x4 S[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -495,7 +498,7 @@ template <int DP>
 __global__ __launch_bounds__(256) void gd_chunk_out_kernel(GDChunk a) {
   const GatedDelta& p = a.p;
   int s, c;
-  if (!locate_chunk(blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
   const int slot = p.slot_of_seq[s];
   if (slot < 0 || slot >= p.num_slots) return;
   const int h = blockIdx.y, c0 = blockIdx.z * 64;
@@ -553,9 +556,9 @@ __global__ __launch_bounds__(256) void gd_chunk_out_kernel(GDChunk a) {
   }
 }
 
-// Sizes of the workspace's parts, in floats.
-static void gd_chunk_parts(const GatedDelta& p, int min_len, int64_t (&n)[9]) {
-  const int64_t units = max_chunks(p.num_tokens, p.num_seqs, min_len) * p.heads, dp = p.dim <= 64 ? 64 : 128, vpad = (p.vdim + 15) / 16 * 16;
+// Sizes of the workspace's parts for so many chunks, in floats.
+static void gd_chunk_parts(const GatedDelta& p, int64_t chunks, int64_t (&n)[9]) {
+  const int64_t units = chunks * p.heads, dp = p.dim <= 64 ? 64 : 128, vpad = (p.vdim + 15) / 16 * 16;
   n[0] = n[1] = n[2] = units * CHUNK * dp;
   n[3] = units * CHUNK * CHUNK;
   n[4] = units * vpad * CHUNK;
@@ -564,9 +567,15 @@ static void gd_chunk_parts(const GatedDelta& p, int min_len, int64_t (&n)[9]) {
   n[7] = (units + 3) / 4 * 4;
   n[8] = units * vpad;
 }
+static int64_t gd_chunk_floats(const GatedDelta& p, int64_t chunks) {
+  int64_t n[9], sum = 0;
+  gd_chunk_parts(p, chunks, n);
+  for (int64_t x : n) sum += x;
+  return sum;
+}
 
 template <typename T, int DP, bool CHANNEL, bool VEC>
-static int gd_chunk_launch(const GDChunk& a, unsigned chunks) {
+static int gd_chunk_launch(GDChunk a, int64_t chunks) {
   const GatedDelta& p = a.p;
   constexpr size_t lds = gd_prepare_lds<DP>();
   static bool attr_set_dev[APHRO_MAX_DEVICES] = {};
@@ -578,9 +587,12 @@ static int gd_chunk_launch(const GDChunk& a, unsigned chunks) {
     }
     attr_set = true;
   }
-  hipLaunchKernelGGL((gd_chunk_prepare_kernel<T, DP, CHANNEL, VEC>), dim3(chunks, (unsigned)p.heads), dim3(DP * 4), lds, p.stream, a);
-  hipLaunchKernelGGL((gd_chunk_carry_kernel<DP>), dim3((unsigned)p.heads, (unsigned)a.vpad / 16, (unsigned)p.num_seqs), dim3(256), 0, p.stream, a);
-  hipLaunchKernelGGL((gd_chunk_out_kernel<DP>), dim3(chunks, (unsigned)p.heads, (unsigned)((p.vdim + 63) / 64)), dim3(256), 0, p.stream, a);
+  const unsigned span = (unsigned)a.span;
+  for (; a.chunk0 < chunks; a.chunk0 += a.span) {
+    hipLaunchKernelGGL((gd_chunk_prepare_kernel<T, DP, CHANNEL, VEC>), dim3(span, (unsigned)p.heads), dim3(DP * 4), lds, p.stream, a);
+    hipLaunchKernelGGL((gd_chunk_carry_kernel<DP>), dim3((unsigned)p.heads, (unsigned)a.vpad / 16, (unsigned)p.num_seqs), dim3(256), 0, p.stream, a);
+    hipLaunchKernelGGL((gd_chunk_out_kernel<DP>), dim3(span, (unsigned)p.heads, (unsigned)((p.vdim + 63) / 64)), dim3(256), 0, p.stream, a);
+  }
   APHRO_LAUNCH_CHECK();
   return APHRO_OK;
 }
@@ -593,10 +605,7 @@ extern "C" int64_t aphro_gated_delta_chunked_workspace(int num_seqs, int64_t num
   if (num_seqs <= 0 || num_tokens <= 0 || heads <= 0 || dim <= 0 || dim > 128 || vdim <= 0 || min_len <= 0) return 0;
   GatedDelta p = {};
   p.num_seqs = num_seqs, p.num_tokens = num_tokens, p.heads = heads, p.dim = dim, p.vdim = vdim;
-  int64_t n[9], sum = 0;
-  gd_chunk_parts(p, num_seqs == 1 ? 1 : min_len, n);
-  for (int64_t x : n) sum += x;
-  return sum * 4;
+  return span_workspace(max_chunks(num_tokens, num_seqs, num_seqs == 1 ? 1 : min_len), [&](int64_t n) { return gd_chunk_floats(p, n); });
 }
 
 extern "C" int aphro_gated_delta_chunked(float* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
@@ -615,13 +624,14 @@ extern "C" int aphro_gated_delta_chunked(float* out, const void* q, int64_t q_st
   if (rc != APHRO_OK) return rc;
   APHRO_CHECK(dim <= 128 && min_len > 0 && num_seqs > 0 && num_seqs <= 65535, "gated_delta_chunked: dim %d (<= 128), %d segments (<= 65535) from %d tokens on", dim, num_seqs, min_len);
   if (num_seqs == 1) min_len = 1;
-  int64_t n[9], sum = 0;
-  gd_chunk_parts(p, min_len, n);
-  for (int64_t y : n) sum += y;
-  APHRO_CHECK(workspace && ((uintptr_t)workspace & 15) == 0 && ((uintptr_t)out & 15) == 0 && workspace_bytes >= sum * 4,
-              "gated_delta_chunked: a workspace of %lld bytes, 16-byte aligned, is needed", (long long)(sum * 4));
   const int64_t chunks = max_chunks(num_tokens, num_seqs, min_len);
-  APHRO_CHECK(chunks <= 0x7fffffff, "gated_delta_chunked: too many tokens");
+  APHRO_CHECK(chunks <= 0x3fffffff, "gated_delta_chunked: too many tokens");
+  const int64_t span = span_chunks(chunks, workspace_bytes, [&](int64_t m) { return gd_chunk_floats(p, m); });
+  APHRO_CHECK(((uintptr_t)out & 15) == 0 && (chunks == 0 || (workspace && ((uintptr_t)workspace & 15) == 0 && span > 0)),
+              "gated_delta_chunked: a workspace of %lld bytes at least, 16-byte aligned, is needed", (long long)gd_chunk_floats(p, 1) * 4);
+  int64_t n[9];
+  gd_chunk_parts(p, span, n);
+  x.chunk0 = 0, x.span = (int)span;
   x.min_len = min_len;
   x.vpad = (vdim + 15) / 16 * 16;
   float* at = workspace;
@@ -636,7 +646,7 @@ extern "C" int aphro_gated_delta_chunked(float* out, const void* q, int64_t q_st
   const int elem = dtype == APHRO_BF16 ? 2 : 4;
   const bool vec = rows_of_16_bytes(q, q_stride, dim, elem) && rows_of_16_bytes(k, k_stride, dim, elem) && rows_of_16_bytes(v, v_stride, vdim, elem) &&
                    (!channel_decay || rows_of_16_bytes(a, a_stride, dim, elem));
-#define GDC_LAUNCH(DP, CH) (vec ? gd_chunk_launch<T, DP, CH, true>(x, (unsigned)chunks) : gd_chunk_launch<T, DP, CH, false>(x, (unsigned)chunks))
+#define GDC_LAUNCH(DP, CH) (vec ? gd_chunk_launch<T, DP, CH, true>(x, chunks) : gd_chunk_launch<T, DP, CH, false>(x, chunks))
   MIX_DISPATCH_DTYPE(dtype, {
     if (dim <= 64) return channel_decay ? GDC_LAUNCH(64, true) : GDC_LAUNCH(64, false);
     return channel_decay ? GDC_LAUNCH(128, true) : GDC_LAUNCH(128, false);

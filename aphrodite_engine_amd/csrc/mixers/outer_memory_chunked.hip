@@ -28,6 +28,7 @@ constexpr int OMC_PITCH = CHUNK + 4;
 struct OMChunk {
   OuterMemory p;
   int min_len;            // segments shorter than this are the scan's
+  int chunk0, span;       // the chunks of these launches (below: [chunks] of one span)
   int vpad;               // vdim rounded up to 16
   float* u;               // [chunks, heads, vpad, DP] U, then the state ahead of the chunk
   float* un;              // mLSTM: [chunks, heads, DP], the same of the normaliser
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(256) void om_chunk_update_kernel(OMChunk a) {
   __shared__ __attribute__((aligned(16))) float vt[OMC_COLS * OMC_PITCH];
   const OuterMemory& p = a.p;
   int s, c;
-  if (!locate_chunk(blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
   const int slot = p.slot_of_seq[s];
   if (slot < 0 || slot >= p.num_slots) return;
   const int h = blockIdx.y, c0 = blockIdx.z * OMC_COLS, hk = MODE == 2 ? h / (p.heads / p.qk_heads) : h;
@@ -222,9 +223,11 @@ __global__ __launch_bounds__(64) void om_chunk_carry_kernel(OMChunk a) {
   const int s = blockIdx.z, h = blockIdx.y;
   const int n = p.q_len[s], slot = p.slot_of_seq[s];
   if (n < a.min_len || slot < 0 || slot >= p.num_slots) return;
-  const int nc = (n + CHUNK - 1) / CHUNK;
-  const int64_t first = chunks_before(s, p.q_len, a.min_len);
-  const bool fresh = p.ctx_len[s] == 0;
+  int begin, nc;
+  int64_t first;
+  if (!span_of(s, (n + CHUNK - 1) / CHUNK, p.q_len, a.min_len, a.chunk0, a.span, begin, nc, first)) return;
+  const bool fresh = begin == 0 && p.ctx_len[s] == 0;
+  first += begin, nc -= begin;                             // (chunks are numbered from the span's first from here on)
   const int x = blockIdx.x * 64 + threadIdx.x, quads = a.vpad * (DP / 4);
   const float* tot = a.total + first * p.heads + h;
   if (MODE == 1 && x >= quads && x < quads + DP) {
@@ -295,7 +298,7 @@ __global__ __launch_bounds__(256) void om_chunk_out_kernel(OMChunk a) {
   __shared__ float bs[CHUNK];
   const OuterMemory& p = a.p;
   int s, c;
-  if (!locate_chunk(blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
   const int slot = p.slot_of_seq[s];
   if (slot < 0 || slot >= p.num_slots) return;
   const int h = blockIdx.y, c0 = blockIdx.z * OMC_COLS, hk = MODE == 2 ? h / (p.heads / p.qk_heads) : h;
@@ -470,24 +473,31 @@ __global__ __launch_bounds__(256) void om_chunk_out_kernel(OMChunk a) {
   }
 }
 
-// Sizes of the workspace's parts, in floats: U, the normaliser's, decays, gates.
-static void om_chunk_parts(const OuterMemory& p, int min_len, int64_t (&n)[4]) {
-  const int64_t chunks = max_chunks(p.num_tokens, p.num_seqs, min_len), dp = p.dim <= 64 ? 64 : 128, vpad = (p.vdim + 15) / 16 * 16;
+// Sizes of the workspace's parts for so many chunks, in floats: U, the normaliser's, decays, gates (of all tokens).
+static void om_chunk_parts(const OuterMemory& p, int64_t chunks, int64_t (&n)[4]) {
+  const int64_t dp = p.dim <= 64 ? 64 : 128, vpad = (p.vdim + 15) / 16 * 16;
   n[0] = chunks * p.heads * vpad * dp;
   n[1] = p.mode == 1 ? chunks * p.heads * dp : 0;
   n[2] = (chunks * p.heads + 3) / 4 * 4;
   n[3] = p.mode == 1 ? 3 * p.heads * p.num_tokens : 0;
 }
+static int64_t om_chunk_floats(const OuterMemory& p, int64_t chunks) {
+  int64_t n[4];
+  om_chunk_parts(p, chunks, n);
+  return n[0] + n[1] + n[2] + n[3];
+}
 
 template <typename T, int MODE, int DP, bool VEC>
-static void om_chunk_launch(const OMChunk& a, unsigned chunks) {
+static void om_chunk_launch(OMChunk a, int64_t chunks) {
   const OuterMemory& p = a.p;
-  const dim3 grid(chunks, (unsigned)p.heads, (unsigned)((p.vdim + OMC_COLS - 1) / OMC_COLS));
+  const dim3 grid((unsigned)a.span, (unsigned)p.heads, (unsigned)((p.vdim + OMC_COLS - 1) / OMC_COLS));
   const unsigned items = (unsigned)a.vpad * (DP / 4) + (MODE == 1 ? DP : 0);
   if (MODE == 1) hipLaunchKernelGGL((om_gates_kernel<T>), dim3((unsigned)p.num_seqs, (unsigned)p.heads), dim3(1024), 0, p.stream, a);
-  hipLaunchKernelGGL((om_chunk_update_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
-  hipLaunchKernelGGL((om_chunk_carry_kernel<MODE, DP>), dim3((items + 63) / 64, (unsigned)p.heads, (unsigned)p.num_seqs), dim3(64), 0, p.stream, a);
-  hipLaunchKernelGGL((om_chunk_out_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
+  for (; a.chunk0 < chunks; a.chunk0 += a.span) {
+    hipLaunchKernelGGL((om_chunk_update_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
+    hipLaunchKernelGGL((om_chunk_carry_kernel<MODE, DP>), dim3((items + 63) / 64, (unsigned)p.heads, (unsigned)p.num_seqs), dim3(64), 0, p.stream, a);
+    hipLaunchKernelGGL((om_chunk_out_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
+  }
 }
 
 }  // namespace aphro
@@ -498,9 +508,7 @@ extern "C" int64_t aphro_outer_memory_chunked_workspace(int num_seqs, int64_t nu
   if (num_seqs <= 0 || num_tokens <= 0 || heads <= 0 || dim <= 0 || dim > 128 || vdim <= 0 || mode < 0 || mode > 2 || min_len <= 0) return 0;
   OuterMemory p = {};
   p.num_seqs = num_seqs, p.num_tokens = num_tokens, p.heads = heads, p.dim = dim, p.vdim = vdim, p.mode = mode;
-  int64_t n[4];
-  om_chunk_parts(p, num_seqs == 1 ? 1 : min_len, n);
-  return (n[0] + n[1] + n[2] + n[3]) * 4;
+  return span_workspace(max_chunks(num_tokens, num_seqs, num_seqs == 1 ? 1 : min_len), [&](int64_t n) { return om_chunk_floats(p, n); });
 }
 
 extern "C" int aphro_outer_memory_chunked(float* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride,
@@ -521,12 +529,14 @@ extern "C" int aphro_outer_memory_chunked(float* out, const void* q, int64_t q_s
   if (rc != APHRO_OK) return rc;
   APHRO_CHECK(dim <= 128 && min_len > 0 && num_seqs <= 65535, "outer_memory_chunked: dim %d (<= 128), %d segments (<= 65535) from %d tokens on", dim, num_seqs, min_len);
   if (num_seqs == 1) min_len = 1;
-  int64_t n[4];
-  om_chunk_parts(p, min_len, n);
-  APHRO_CHECK(workspace && ((uintptr_t)workspace & 15) == 0 && ((uintptr_t)out & 15) == 0 && workspace_bytes >= (n[0] + n[1] + n[2] + n[3]) * 4,
-              "outer_memory_chunked: a workspace of %lld bytes, 16-byte aligned, is needed", (long long)((n[0] + n[1] + n[2] + n[3]) * 4));
   const int64_t chunks = max_chunks(num_tokens, num_seqs, min_len);
-  APHRO_CHECK(chunks <= 0x7fffffff, "outer_memory_chunked: too many tokens");
+  APHRO_CHECK(chunks <= 0x3fffffff, "outer_memory_chunked: too many tokens");
+  const int64_t span = span_chunks(chunks, workspace_bytes, [&](int64_t m) { return om_chunk_floats(p, m); });
+  APHRO_CHECK(((uintptr_t)out & 15) == 0 && (chunks == 0 || (workspace && ((uintptr_t)workspace & 15) == 0 && span > 0)),
+              "outer_memory_chunked: a workspace of %lld bytes at least, 16-byte aligned, is needed", (long long)om_chunk_floats(p, 1) * 4);
+  int64_t n[4];
+  om_chunk_parts(p, span, n);
+  a.chunk0 = 0, a.span = (int)span;
   a.min_len = min_len;
   a.vpad = (vdim + 15) / 16 * 16;
   a.u = workspace;
@@ -544,11 +554,11 @@ extern "C" int aphro_outer_memory_chunked(float* out, const void* q, int64_t q_s
 #define OMC_LAUNCH(MODE)                                                                  \
   do {                                                                                    \
     if (dim <= 64) {                                                                      \
-      if (vec) om_chunk_launch<T, MODE, 64, true>(a, (unsigned)chunks);                   \
-      else om_chunk_launch<T, MODE, 64, false>(a, (unsigned)chunks);                      \
+      if (vec) om_chunk_launch<T, MODE, 64, true>(a, chunks);                   \
+      else om_chunk_launch<T, MODE, 64, false>(a, chunks);                      \
     } else {                                                                              \
-      if (vec) om_chunk_launch<T, MODE, 128, true>(a, (unsigned)chunks);                  \
-      else om_chunk_launch<T, MODE, 128, false>(a, (unsigned)chunks);                     \
+      if (vec) om_chunk_launch<T, MODE, 128, true>(a, chunks);                  \
+      else om_chunk_launch<T, MODE, 128, false>(a, chunks);                     \
     }                                                                                     \
   } while (0)
   MIX_DISPATCH_DTYPE(dtype, {

@@ -257,10 +257,8 @@ def memory_state_shapes(slots: int, heads: int, dim: int, vdim: int, mode: int):
 # A batch whose longest segment has at least MEMORY_CHUNKED_FROM tokens runs its segments of MEMORY_CHUNKED_MIN and more in chunks of 64 on the
 # matrix cores, and token by token what is shorter; any other batch is scanned.  One segment, scan / chunks in us: 64 tokens 21 / 24 (decay), 33 / 34
 # (mLSTM), 23 / 33 (state space); 96 tokens 30 / 24, 47 / 35, 33 / 34; where the launches are made anyway, shorter segments cost little in them
-# and would keep the token form's wide split, which single tokens beside them are slower in.  The chunked forms keep every chunk's state for
-# the length of the call; a batch that would need more than the bound is scanned.
+# and would keep the token form's wide split, which single tokens beside them are slower in.
 MEMORY_CHUNKED_FROM, MEMORY_CHUNKED_MIN = 96, 32
-CHUNKED_WORKSPACE_MAX = 8 << 30
 
 
 def outer_memory_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state, slot_of_seq: torch.Tensor,
@@ -307,10 +305,9 @@ def outer_memory_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state, 
             _p(decay), float(q_scale), float(gate_cap), qk_heads, _p(a_log), _p(dt_bias), _p(skip))
     if max_q_len >= MEMORY_CHUNKED_FROM and d <= 128 and 0 < S <= 65535:
         need = lib.aphro_outer_memory_chunked_workspace(S, T, heads, d, e, int(mode), MEMORY_CHUNKED_MIN)
-        if need <= CHUNKED_WORKSPACE_MAX:
-            ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
-            check(lib.aphro_outer_memory_chunked(*args, MEMORY_CHUNKED_MIN, ws.data_ptr(), need, _dt(q), _stream()), "outer_memory_scan")
-            return out
+        ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
+        check(lib.aphro_outer_memory_chunked(*args, MEMORY_CHUNKED_MIN, ws.data_ptr(), need, _dt(q), _stream()), "outer_memory_scan")
+        return out
     check(lib.aphro_outer_memory_scan(*args, int(max_q_len), _dt(q), _stream()), "outer_memory_scan")
     return out
 
@@ -867,10 +864,9 @@ def gated_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, b: torch
             S, T, heads, kv_heads, d, e, int(channel), float(q_scale), float(norm_eps))
     if max_q_len >= DELTA_CHUNKED_FROM and d <= 128 and 0 < S <= 65535:
         need = lib.aphro_gated_delta_chunked_workspace(S, T, heads, d, e, DELTA_CHUNKED_MIN)
-        if need <= CHUNKED_WORKSPACE_MAX:
-            ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
-            check(lib.aphro_gated_delta_chunked(*args, DELTA_CHUNKED_MIN, ws.data_ptr(), need, _dt(q), _stream()), "gated_delta_scan")
-            return out
+        ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
+        check(lib.aphro_gated_delta_chunked(*args, DELTA_CHUNKED_MIN, ws.data_ptr(), need, _dt(q), _stream()), "gated_delta_scan")
+        return out
     check(lib.aphro_gated_delta_scan(*args, int(max_q_len), _dt(q), _stream()), "gated_delta_scan")
     return out
 

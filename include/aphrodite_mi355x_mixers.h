@@ -124,8 +124,10 @@ int aphro_outer_memory_scan(float* out, const void* q, int64_t q_stride, const v
                             float gate_cap, int qk_heads, const float* a_log, const float* dt_bias, const float* skip, int max_q_len, int dtype, void* stream);
 
 /* The same with segments of at least min_len tokens in chunks of 64 on the matrix cores (fp32 products); shorter ones token by token; a
- * single segment always in chunks.  dim <= 128, num_seqs <= 65535.  workspace: 16-byte aligned, of at least
- * aphro_outer_memory_chunked_workspace(...) bytes (0: sizes that are not served), in use until the stream has passed the call. */
+ * single segment always in chunks.  dim <= 128, num_seqs <= 65535.  workspace: 16-byte aligned, of
+ * aphro_outer_memory_chunked_workspace(...) bytes (0: sizes that are not served; up to 256 MiB beside mode 1's three numbers a head and
+ * token), in use until the stream has passed the call.  The chunks run in spans of as many as it holds; less serves, down to one chunk's,
+ * in more launches and with the same results. */
 int64_t aphro_outer_memory_chunked_workspace(int num_seqs, int64_t num_tokens, int heads, int dim, int vdim, int mode, int min_len);
 int aphro_outer_memory_chunked(float* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
                                int64_t v_stride, const void* gate_i, const void* gate_f, int64_t gate_stride, float* state_s,

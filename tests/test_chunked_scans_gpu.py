@@ -194,3 +194,44 @@ def test_delta_chunks_keep_the_tokens_ahead_of_a_bad_value(mops, where, bad):
     assert torch.equal(torch.isfinite(got), torch.isfinite(scanned)) and torch.equal(torch.isfinite(state), torch.isfinite(state2))
     fine = torch.isfinite(scanned)
     assert torch.allclose(got[fine], scanned[fine], rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, "delta"])
+@pytest.mark.parametrize("chunks", [1, 3])
+def test_chunks_in_spans(mops, monkeypatch, mode, chunks):
+    """A workspace of one or three chunks instead of all: segments cut at any of theirs, the same bits."""
+    H, d, e, lens, ctx = 2, 100, 72, [200, 1, 33, 500, 64, 7], [0, 4, 6, 3, 0, 0]
+    g = torch.Generator(device=DEV).manual_seed(7)
+    T, S = sum(lens), len(lens)
+    start = i32(np.concatenate([[0], np.cumsum(lens)[:-1]]))
+    q, k, v = (part(g, T, H * n, torch.bfloat16, 0) for n in (d, d, e))
+    gi, gf, one = part(g, T, H, torch.bfloat16, 0), part(g, T, H, torch.bfloat16, 0), torch.ones(H, device=DEV)
+    shapes = [(S, H, d, e)] if mode == "delta" else mops.memory_state_shapes(S, H, d, e, mode)
+    first = [torch.randn(s, generator=g, device=DEV) for s in shapes]
+    if mode == 1:
+        first[1][:], first[2][:] = first[1][:, :, :1].clone(), first[2][:, :, :1].clone()
+    lib = mops._lib.mixers_lib()
+    query = "aphro_gated_delta_chunked_workspace" if mode == "delta" else "aphro_outer_memory_chunked_workspace"
+
+    def go():
+        state = tuple(s.clone() for s in first)
+        if mode == "delta":
+            out = mops.gated_delta_scan(q, k, v, gi, gf, one, one, state[0], i32(range(S)), start, i32(lens), i32(ctx), H, H, 1.0, max_q_len=500)
+        else:
+            kw = {0: dict(decay=0.9 * one), 1: dict(gate_i=gi, gate_f=gf), 2: dict(gate_i=gi, a_log=one, dt_bias=one, skip=one)}[mode]
+            out = mops.outer_memory_scan(q, k, v, state, i32(range(S)), start, i32(lens), i32(ctx), H, mode, max_q_len=500, **kw)
+        return (out, ) + state
+    want, full = go(), getattr(lib, query)
+    one_chunk = (lambda *a: full(1, 64, *a[2:-1], 64)) if mode != 1 else (lambda *a: full(1, 64, *a[2:-1], 64) + 12 * H * (T - 64))
+    monkeypatch.setattr(lib, query, lambda *a: one_chunk(*a) if chunks == 1 else 3 * one_chunk(*a) - (24 * H * T if mode == 1 else 0))
+    for x, y in zip(go(), want):
+        assert torch.equal(x, y)
+
+
+def test_chunks_do_not_take_memory_with_the_prompt(mops):
+    """The workspace of prompts of a hundred thousand tokens: 256 MiB, and mode 1's three numbers a head and token."""
+    lib, T = mops._lib.mixers_lib(), 100_000
+    assert 200 << 20 < lib.aphro_gated_delta_chunked_workspace(1, T, 32, 128, 128, 32) <= 256 << 20
+    for mode in (0, 1, 2):
+        extra = 12 * 32 * T if mode == 1 else 0
+        assert 200 << 20 < lib.aphro_outer_memory_chunked_workspace(1, T, 32, 128, 256, mode, 32) - extra <= 256 << 20
