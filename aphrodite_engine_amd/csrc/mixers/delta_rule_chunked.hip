@@ -12,7 +12,8 @@
 // blocks as (from the block's start) x (whole blocks between) x (to the block's end) -- factors of at most one, as exact as the scan's.
 //
 // A token whose k, beta or g is not finite, and a value that is not, would reach tokens ahead of it in the products (zero times NaN): they are
-// entered as a token without effect, and the chunk says from where on outputs and state are NaN (`bad_token`, `bad_value`).
+// entered as a token without effect, and the chunk says from where on outputs and state are NaN (`bad_token`, `bad_value`).  So is a u
+// that overflows.
 //
 // What bounds it: the scan is bound by the latency of its token chain; here launch 2's chain is one of 64-token steps (two products of 64 x
 // dim x 16 and two barriers each), launches 1 and 3 have all chunks to fill the chip (launch 1 one workgroup a CU:
@@ -39,7 +40,7 @@ struct GDChunk {
   float* st;               // [chunks, heads, vpad, DP] the state ahead of the chunk
   float* gam;              // [chunks, heads, DP]      Pi_63
   int32_t* bad_token;      // [chunks, heads]          first token that is not finite (64: none)
-  int32_t* bad_value;      // [chunks, heads, vpad]    first value of the column that is not finite (64: none)
+  int32_t* bad_value;      // [chunks, heads, vpad]    first value, or u, of the column that is not finite (64: none)
 };
 
 template <int DP>
@@ -454,6 +455,14 @@ __global__ __launch_bounds__(256) void gd_chunk_carry_kernel(GDChunk a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) uv[r] = x.ut[r] - (acc[0][r] + acc[1][r]);
     *reinterpret_cast<f32x4*>(&us[li * GDC_P + wave * 16 + 4 * lg]) = uv;
+    if (!(finite_f(uv[0]) && finite_f(uv[1]) && finite_f(uv[2]) && finite_f(uv[3]))) {      // (overflowed: the state takes it as it is)
+#pragma unroll
+      for (int r = 3; r >= 0; --r)
+        if (!finite_f(uv[r])) {
+          atomicMin(&a.bad_value[unit * a.vpad + col], wave * 16 + 4 * lg + r);
+          uv[r] = 0.f;
+        }
+    }
     *reinterpret_cast<f32x4*>(a.ut + (unit * a.vpad + col) * CHUNK + wave * 16 + 4 * lg) = uv;
     lds_barrier();
 #pragma unroll

@@ -169,7 +169,7 @@ def test_delta_chunks(mops, channel, dtype, pad, d, e, strong):
     assert torch.equal(state[1].double().cpu(), before[1])                # a slot that no segment names
 
 
-@pytest.mark.parametrize("where", ["v", "k", "q", "b"])
+@pytest.mark.parametrize("where", ["v", "k", "q", "b", "u"])
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_delta_chunks_keep_the_tokens_ahead_of_a_bad_value(mops, where, bad):
     T, H, d, e, at = 170, 1, 32, 24, 70
@@ -182,7 +182,11 @@ def test_delta_chunks_keep_the_tokens_ahead_of_a_bad_value(mops, where, bad):
                                   i32([0]), i32([0]), i32([T]), i32([0]), H, H, 1.0, max_q_len=T)
         return o, state
     want, w = go(x)[0], {n: t.clone() for n, t in x.items()}
-    w[where][at, 0 if where == "b" else 3] = bad
+    if where == "u":                                     # finite values whose correction is beyond fp32: v against what the same key holds
+        w["k"][at], w["b"][at - 1:at + 1], w["v"][at - 1, 3], w["v"][at, 3] = w["k"][at - 1], 20.0, 3e38, -3e38
+        want = go({**w, "v": torch.cat([w["v"][:at], x["v"][at:]])})[0]
+    else:
+        w[where][at, 0 if where == "b" else 3] = bad
     got, state = go(w)
     assert torch.allclose(got[:at], want[:at], rtol=1e-4, atol=1e-5)
     old = mops.DELTA_CHUNKED_FROM
