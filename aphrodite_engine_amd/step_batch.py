@@ -109,11 +109,16 @@ class StepBatch:
         k = self.decode_split()
         seq_lens = [c + n for c, n in zip(self.ctx_lens, self.q_lens)]
         npt = sum(self.q_lens[:k])
+        dev = self.input_ids.device
+        # (build() sent these along; a batch put together by hand has none)
+        sums = lambda x: torch.from_numpy(np.concatenate([[0], np.cumsum(x[:k], dtype=np.int64)]).astype(np.int32)).to(dev)
+        seq_lens_tensor = torch.tensor(seq_lens, dtype=torch.int32, device=dev) if self.seq_lens_tensor is None else self.seq_lens_tensor
         return MI355XAttentionMetadata(
             num_prefills=k, num_prefill_tokens=npt, num_decode_tokens=self.num_tokens - npt, slot_mapping=self.slot_mapping,
-            seq_lens=seq_lens, seq_lens_tensor=self.seq_lens_tensor,
+            seq_lens=seq_lens, seq_lens_tensor=seq_lens_tensor,
             max_query_len=max(self.q_lens), max_prefill_seq_len=max(seq_lens[:k], default=0),
             max_decode_seq_len=max(seq_lens[k:], default=0),
-            query_start_loc=self.query_start_loc, seq_start_loc=self.seq_start_loc,
+            query_start_loc=sums(self.q_lens) if self.query_start_loc is None else self.query_start_loc,
+            seq_start_loc=sums(seq_lens) if self.seq_start_loc is None else self.seq_start_loc,
             context_lens_tensor=self.ctx_len[:k] if k else self.ctx_len[:0], block_tables=self.block_tables,
             use_cuda_graph=False, max_context_len=max(self.ctx_lens[:k], default=0))

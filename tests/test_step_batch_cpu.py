@@ -1,4 +1,6 @@
 """StepBatch.build against the same arrays made segment by segment."""
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -34,6 +36,9 @@ def test_build(segs, block):
     assert m.seq_lens_tensor.tolist() == [c + n for c, n in segs] and m.num_prefill_tokens == sum(n for _, n in segs[:k])
     assert m.query_start_loc.tolist() == [0] + np.cumsum([n for _, n in segs[:k]]).tolist()
     assert m.seq_start_loc.tolist() == [0] + np.cumsum([c + n for c, n in segs[:k]]).tolist()
+    by_hand = dataclasses.replace(b, rows=None, seq_lens_tensor=None, query_start_loc=None, seq_start_loc=None).attention_metadata()
+    for name in ("seq_lens_tensor", "query_start_loc", "seq_start_loc"):
+        assert torch.equal(getattr(by_hand, name), getattr(m, name)) and getattr(by_hand, name).dtype == torch.int32
     assert m.query_start_loc.dtype == m.seq_start_loc.dtype == m.seq_lens_tensor.dtype == torch.int32
 
 
