@@ -59,8 +59,10 @@ class StepBatch:
         q_lens = [len(t) for t in tokens]
         if S == 0 or min(q_lens) <= 0:
             raise ValueError("a step batch needs at least one segment and no empty one")
-        n, c = np.asarray(q_lens, np.int64), np.asarray([int(x) for x in ctx_lens], np.int64)
-        pages = np.asarray([len(b) for b in block_tables], np.int64)
+        if min(len(ctx_lens), len(block_tables)) < S:
+            raise ValueError(f"{S} segments, but {len(ctx_lens)} contexts and {len(block_tables)} page lists")
+        n, c = np.asarray(q_lens, np.int64), np.asarray([int(x) for x in ctx_lens[:S]], np.int64)
+        pages = np.asarray([len(b) for b in block_tables[:S]], np.int64)
         need = (c + n + block_size - 1) // block_size
         for s in np.nonzero(pages < need)[0]:
             raise ValueError(f"segment {s}: {pages[s]} pages for {c[s] + n[s]} tokens")
@@ -69,7 +71,7 @@ class StepBatch:
         T = int(n.sum())
         starts = np.cumsum(n) - n
         bt = np.zeros((S, max(1, int(pages.max()))), np.int32)
-        for s, b in enumerate(block_tables):
+        for s, b in enumerate(block_tables[:S]):
             bt[s, :len(b)] = b
         seq_of = np.repeat(np.arange(S), n)
         pos = np.arange(T) - np.repeat(starts - c, n)

@@ -46,6 +46,8 @@ def test_build_refuses():
     ok = dict(tokens=[[1, 2]], ctx_lens=[15], block_tables=[[3, 4]], state_slots=[0], block_size=16, device="cpu")
     StepBatch.build(**ok)
     for bad, what in ((dict(tokens=[]), "at least one"), (dict(tokens=[[]]), "at least one"), (dict(block_tables=[[3]]), "1 pages for 17 tokens"),
-                      (dict(tokens=[[1], [2]], ctx_lens=[0, 0], block_tables=[[1], [2]], state_slots=[4, 4]), "share a state slot")):
+                      (dict(tokens=[[1], [2]], ctx_lens=[0, 0], block_tables=[[1], [2]], state_slots=[4, 4]), "share a state slot"),
+                      (dict(tokens=[[1], [2]], ctx_lens=[0], block_tables=[[1], [2]], state_slots=[0, 1]), "1 contexts"),
+                      (dict(tokens=[[1], [2]], ctx_lens=[0, 0], block_tables=[[1]], state_slots=[0, 1]), "1 page lists")):
         with pytest.raises(ValueError, match=what):
             StepBatch.build(**{**ok, **bad})
