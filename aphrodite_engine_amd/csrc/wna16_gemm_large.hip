@@ -1044,6 +1044,7 @@ static bool large_eight(const LargePlan& pl, int64_t K) {
 // this file's are ranges of whole groups, of which 11008 or 9728 rows of K have few divisors and one group per column none (4096 x 11008 at 65
 // / 150 / 300 rows with slices bound to this file's 53 / 54 / 54 us, without 21 / 28 / 40 us).
 static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs) {
+  if (knobs().wna16_large_8phase >= 0 || knobs().wna16_large_two_pass >= 0) return {0, 1};      // a switch names this file's forms
   int64_t other_ns = -1;
   if (pl.streamk) {            // 1.9 us per 256 x 256 x 64 of a CU's even share, 18 us around them
     const int64_t units = (M + 255) / 256 * ((N + 255) / 256) * (K / 64);

@@ -234,7 +234,7 @@ def test_config2_prefill_sized_fp8_scaled_mm_vs_oracle(ops, K, N, M, per_token, 
 
 
 def test_prefill_sized_fp8_scaled_mm_under_graph_capture(ops):
-    """The stream-K form clears its flag words with a memset node in front of the kernel: capture it, replay it twice."""
+    """The stream-K form clears its flag words with a kernel of its own in front: capture it, replay it twice."""
     g_ = torch.Generator(device=DEV).manual_seed(3)
     M, K, N = 2304, 1024, 6144
     a = torch.randn(M, K, generator=g_, device=DEV).to(torch.float8_e4m3fn)

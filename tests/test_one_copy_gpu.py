@@ -100,9 +100,10 @@ def test_plans_outside_the_eight_phase_kernel_read_it_in_place_too(ops, M_, K, N
     st = ops.wna16_strip_relayout(qw, 32, K // 128)
     from aphrodite_engine_amd import _lib
     lib = _lib.lib()
-    assert lib.aphro_wna16_gemm_large_strip_workspace_bytes(M_, N, K, K // 128, 0, 32) == \
-        lib.aphro_wna16_gemm_large_workspace_bytes(M_, N, K, K // 128, 0)
-    assert torch.equal(ops.wna16_gemm_large_strip(a, st, qz, sc, 1), ops._wna16_large(a, qw, qz, sc, None, 1))
+    with ops.knob("APHRO_WNA16_LARGE_8PHASE", 0):          # (else the row tile takes these)
+        assert lib.aphro_wna16_gemm_large_strip_workspace_bytes(M_, N, K, K // 128, 0, 32) == \
+            lib.aphro_wna16_gemm_large_workspace_bytes(M_, N, K, K // 128, 0)
+        assert torch.equal(ops.wna16_gemm_large_strip(a, st, qz, sc, 1), ops._wna16_large(a, qw, qz, sc, None, 1))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

@@ -139,7 +139,7 @@ def test_gptq_gemm_large_m_path(ops):
 
 @pytest.mark.parametrize("M,N,K,G", [(2048, 4096, 2048, 128), (2000, 4096, 2304, 128), (4096, 2048, 4096, 64)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_wna16_large_eight_phase(ops, monkeypatch, M, N, K, G, dtype):
+def test_wna16_large_eight_phase(ops, M, N, K, G, dtype):
     """Prefill-sized W4A16 on the 256 x 256 stream-K tile (>= 128 tiles, K >= 2048: wna16_gemm_large8_kernel, weights built
     in the LDS from one packed row piece per thread) against the oracle's gptq_gemm on sampled rows (all columns) and sampled
     columns (all rows), and bit-equal to the staged kernel it replaces (same K order, same dequantisation)."""
@@ -148,11 +148,11 @@ def test_wna16_large_eight_phase(ops, monkeypatch, M, N, K, G, dtype):
     shuf = oq.gptq_shuffle(qweight)
     a = rng.standard_normal((M, K)).astype(np.float16)
     ta, ts = t(a).to(dtype), t(s, torch.float16).to(dtype)
-    got_t = ops._wna16_large(ta, t(shuf), t(qzeros), ts, None, 1)
+    with ops.knob("APHRO_WNA16_LARGE_8PHASE", 1):          # (up to 4096 rows the row tile may take the call where neither is named)
+        got_t = ops._wna16_large(ta, t(shuf), t(qzeros), ts, None, 1)
     assert got_t.shape == (M, N) and got_t.dtype == dtype
-    monkeypatch.setenv("APHRO_WNA16_LARGE_8PHASE", "0"); ops.reload_env()
-    old_t = ops._wna16_large(ta, t(shuf), t(qzeros), ts, None, 1)
-    monkeypatch.delenv("APHRO_WNA16_LARGE_8PHASE"); ops.reload_env()
+    with ops.knob("APHRO_WNA16_LARGE_8PHASE", 0):
+        old_t = ops._wna16_large(ta, t(shuf), t(qzeros), ts, None, 1)
     assert torch.equal(got_t, old_t)
     got = got_t.float().cpu().numpy()
     a16 = ta.float().cpu().numpy().astype(np.float16)

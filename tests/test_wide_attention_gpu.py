@@ -8,7 +8,7 @@ DEV = "cuda"
 D = 128
 
 
-def run(lens, ctxs, heads, kv_heads, block, bias=0, temp=0.0, window=0, chunk=0, softcap=0.0, sink=False, gate=None, pad=0, seed=0, fill=None):
+def run(lens, ctxs, heads, kv_heads, block, bias=0, temp=0.0, window=0, chunk=0, softcap=0.0, sink=False, gate=None, pad=0, seed=0, fill=None, shift=0):
     from aphrodite_engine_amd import mixer_ops as mops
     g = torch.Generator(device=DEV).manual_seed(seed)
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
@@ -20,8 +20,8 @@ def run(lens, ctxs, heads, kv_heads, block, bias=0, temp=0.0, window=0, chunk=0,
     for i, k in enumerate(need):
         tables[i, :k] = order[at:at + k]
         at += k
-    kc = rnd(len(order), block, kv_heads, D).bfloat16()
-    vc = rnd(len(order), block, kv_heads, D).bfloat16()
+    size = len(order) * block * kv_heads * D
+    kc, vc = (rnd(size + shift).bfloat16()[shift:].view(len(order), block, kv_heads, D) for _ in range(2))
     if fill is not None:                                     # what lies in blocks and slots that no key has
         used = torch.zeros(len(order), block, dtype=torch.bool, device=DEV)
         for i, k in enumerate(need):
@@ -105,7 +105,33 @@ def test_short_segments_beside_prompt_portions(kw, block, ctx):
     run(lens, [i * 13 % 37 + ctx for i in range(len(lens))], 8, 2, block, fill=0.0, **kw)
 
 
-def test_a_column_s_bits_do_not_depend_on_the_batch():
-    a = run([257], [0], 8, 2, 16, seed=1)
-    b = run([257], [0], 8, 2, 16, seed=1)
-    assert torch.equal(a, b)
+@pytest.mark.parametrize("kw", [dict(), dict(bias=64, gate="heads"), dict(window=100, sink=True), dict(gate="columns", pad=1)])
+@pytest.mark.parametrize("block", [16, 24])
+def test_caches_that_are_not_16_byte_aligned(kw, block):
+    """The older prompt kernel, which loads through registers, has these."""
+    run([200, 9, 70], [33, 300, 0], 8, 2, block, fill=0.0, shift=4, **kw)
+
+
+def test_a_row_s_bits_do_not_depend_on_the_batch():
+    """A segment by itself and between others, its rows cut at the same places: workgroups are numbered and ordered otherwise, the sums are not."""
+    from aphrodite_engine_amd import mixer_ops as mops
+    heads, G, block, lens, ctxs = 8, 2, 16, [70, 257, 1, 400], [33, 90, 500, 0]
+    g = torch.Generator(device=DEV).manual_seed(1)
+    kc, vc = (torch.randn(128, block, G, D, generator=g, device=DEV).bfloat16() for _ in range(2))
+    q = torch.randn(sum(lens), heads * D, generator=g, device=DEV).bfloat16()
+    lut = torch.randn(heads, 64, generator=g, device=DEV)
+    tables = torch.randperm(128, generator=g, device=DEV).to(torch.int32)[:4 * 32].view(4, 32)
+
+    def go(segs):
+        rows = torch.cat([torch.arange(sum(lens[:s]), sum(lens[:s + 1]), device=DEV) for s in segs])
+        n = [lens[s] for s in segs]
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+        out = torch.empty(len(rows), heads * D, device=DEV).bfloat16()
+        mops.distance_bias_attention(out, q[rows], None, kc, vc, tables[segs].contiguous(), i32([sum(n[:i]) for i in range(len(n))]), i32(n),
+                                     i32([ctxs[s] for s in segs]), torch.repeat_interleave(torch.arange(len(n), device=DEV, dtype=torch.int32), i32(n)),
+                                     (min(n), max(n)), heads, D ** -0.5, lut, max_kv_len=501)
+        at = sum(n[:segs.index(1)])
+        return out[at:at + lens[1]]
+    want = go([1])
+    for segs in ([0, 1, 2, 3], [3, 1], [1, 2]):
+        assert torch.equal(go(segs), want)

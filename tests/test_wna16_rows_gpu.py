@@ -74,6 +74,17 @@ def test_small_projections_do_not_round_their_weights(m, k, n):
     assert all(float((x.double() - want).norm()) < bound for x in got)
 
 
+@pytest.mark.parametrize("m,k,n", [(65, 576, 256), (150, 4160, 4096), (300, 4160, 1024), (513, 2112, 8192)])
+def test_k_that_the_row_tile_does_not_take(m, k, n):
+    """K = 64 (mod 128): the few-tile plans of csrc/wna16_gemm_large.hip, K slices of whole groups among them."""
+    from aphrodite_engine_amd import _custom_ops as ops
+    qw, qz, sc, g = weights(k, n, 64, torch.float16, m + k + n)
+    a = torch.randn(m, k, generator=g, device=DEV).half()
+    want, got = a.double() @ dense(qw, qz, sc, 1), ops._wna16_large(a, qw, qz, sc, None, 1)
+    assert float((got.double() - want).norm() / want.norm()) < BOUND[torch.float16]
+    assert torch.equal(ops._wna16_large(a, qw, qz, sc, None, 1), got)
+
+
 def test_rows_gemm_keeps_a_row_s_infinities_and_nans_to_itself():
     from aphrodite_engine_amd import _custom_ops as ops
     qw, qz, sc, g = weights(1024, 512, 128, torch.float16, 3)
