@@ -445,8 +445,12 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t*
           lsum += e;
         }
       l_run = l_run * alpha + lsum;
+      // (only where some lane's maximum moved: a step's 32 multiplies, one by one in this library, for a factor that is mostly 1; 32 rows of
+      //  Llama-3-8B, 16 layers: a decode step 1407.5 -> 1403.4 us, same bits)
+      if (__ballot(alpha != 1.0f)) {
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) o[dt] *= alpha;
+        for (int dt = 0; dt < NDT; ++dt) o[dt] *= alpha;
+      }
       u32x4 pf;  // B operand of the PV MFMA: k = (jj, 4g + r)
       pf[0] = pack2<T>(pv[0][0], pv[0][1]);
       pf[1] = pack2<T>(pv[0][2], pv[0][3]);
