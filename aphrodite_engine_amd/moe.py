@@ -127,17 +127,27 @@ class Wna16Experts:
         self.inter = self.w2[0].shape[1] * 8
 
 
-# Prompt-sized batches: from MOE_TILE_ROWS slots per expert on (the average) the experts run on the tile GEMM, in blocks of 64 rows, and of 128
+# Prompt-sized batches: from MOE_TILE_ROWS slots per expert on (the average; moe_tile_rows) the experts run on the tile GEMM, in blocks of 64 rows, and of 128
 # from MOE_TILE_WIDE on.  Mixtral-8x7B's experts (8, top 2), decode kernel / 64 / 128 in us: 64 tokens 251 / 280 / 475, 96 tokens 325 / 257 / 434,
 # 160 tokens 451 / 258 / 448, 512 tokens 1268 / 540 / 632, 2048 tokens 4900 / 1760 / 1806, 4096 tokens - / 3354 / 3334.
 MOE_TILE_ROWS, MOE_TILE_WIDE = 24, 768
+
+
+def moe_tile_rows(experts: "Wna16Experts") -> int:
+    """Slots per expert from which the tile GEMM is the faster: MOE_TILE_ROWS, and more where up to 16 experts are small, because its chain over K
+    then outlasts the decode kernel's few blocks (more experts are routed by the separate ops, in blocks of 16 rows slower than anything
+    behind them).  us, decode kernel / tile at 24, 32, 48 slots: 2^27 weights of hidden x inter and more 169 / 164, 204 / 157, 254 / 158 (4 x 4096
+    x 14336), 191 / 164 (16 x 4096 x 4096); fewer 87 / 98, 102 / 95, 129 / 96 (8 x 4096 x 3584), 56 / 67, 63 / 66, 79 / 67 (4 x 2048 x 8192); 2^23
+    54 / 59, 54 / 60, 52 / 59 and at 192 slots 70 / 61 (8 x 1024 x 1024); 60 x 2048 x 1024 356 / 107, 128 x 1024 x 512 314 / 109."""
+    weights = experts.num_experts * experts.hidden * experts.inter
+    return MOE_TILE_ROWS * (1 if experts.num_experts > 16 or weights >= 2 ** 27 else 2 if weights >= 2 ** 25 else 8)
 
 
 def moe_tile_block(slots: int, experts: Wna16Experts, dtype: torch.dtype, a_bytes: int = 0) -> int:
     """Rows of a block of the tile GEMM for a batch of ``slots`` (token, expert) pairs whose activations span ``a_bytes``; 0: the decode
     kernel's batch or shape."""
     e = experts.num_experts
-    if slots < MOE_TILE_ROWS * e or dtype != experts.w13[2].dtype:
+    if slots < moe_tile_rows(experts) * e or dtype != experts.w13[2].dtype:
         return 0
     bm = 64 if slots < MOE_TILE_WIDE * e else 128
     blocks = (slots + e * (bm - 1) + bm - 1) // bm

@@ -760,8 +760,8 @@ def test_lab_patches_apply_to_the_product_sources():
         assert r.returncode == 0, (os.path.basename(pf), r.stdout[-400:], r.stderr[-400:])
 
 
-def test_expert_tile_leaves_batches_beyond_32_bit_offsets_to_the_decode_kernel():
-    """moe.moe_tile_block at the sizes its kernel refuses: 4 GiB of activations in front of either GEMM."""
+def test_which_batches_the_expert_tile_takes():
+    """moe.moe_tile_block by slots per expert and at the sizes its kernel refuses: 4 GiB of activations in front of either GEMM."""
     from types import SimpleNamespace
     from aphrodite_engine_amd import moe as M
     hidden, inter, e = 4096, 14336, 8
@@ -770,4 +770,7 @@ def test_expert_tile_leaves_batches_beyond_32_bit_offsets_to_the_decode_kernel()
     experts = SimpleNamespace(num_experts=e, hidden=hidden, inter=inter, w13=w(hidden, 2 * inter), w2=w(inter, hidden))
     most = (2 ** 32 - 2) // (inter * 2) // 128 * 128 - e * 127           # slots whose blocks of 128 rows just fit
     assert M.moe_tile_block(most, experts, torch.float16) == 128 and M.moe_tile_block(most + 128, experts, torch.float16) == 0
+    for e, hidden, inter, rows in ((8, 4096, 14336, 24), (4, 4096, 14336, 24), (64, 2048, 1536, 24), (128, 1024, 512, 24), (8, 4096, 3584, 48), (8, 1024, 1024, 192)):
+        small = SimpleNamespace(num_experts=e, hidden=hidden, inter=inter, w13=w(hidden, 2 * inter), w2=w(inter, hidden))
+        assert M.moe_tile_block(rows * e, small, torch.float16) == 64 and M.moe_tile_block(rows * e - 1, small, torch.float16) == 0
     assert M.moe_tile_block(6000, experts, torch.float16, 2 ** 32 - 2) == 64 and M.moe_tile_block(6000, experts, torch.float16, 2 ** 32 - 1) == 0

@@ -103,10 +103,11 @@ def test_routing_places_every_slot_of_rows_that_are_not_finite(e, topk, block):
     assert all(order[p] == i for i, p in enumerate(a[5].tolist()))
 
 
-def test_a_token_without_a_finite_logit_leaves_the_others():
+def test_a_token_without_a_finite_logit_leaves_the_others(monkeypatch):
     """The prompt-sized experts with such tokens in the batch: everyone else's output is what it is without them."""
     from aphrodite_engine_amd import moe as M
     experts, _, _ = experts_of(8, 512, 512, torch.float16, "gptq", 11)
+    monkeypatch.setattr(M, "MOE_TILE_ROWS", 1)
     x, logits = torch.randn(300, 512, device=DEV).half(), torch.randn(300, 8, device=DEV).half()
     want = M.fused_wna16_moe(x, experts, logits, 2, True)
     assert M.moe_tile_block(600, experts, torch.float16)
