@@ -2,6 +2,7 @@
 ``_custom_ops``: every wrapper checks on the host what the kernel and its grid assume (shapes, strides, dtypes, devices)
 before it launches, issues on the current stream, allocates only its result, and raises on CPU tensors -- there is no
 fallback."""
+import math
 from typing import Optional
 
 import torch
@@ -254,11 +255,14 @@ def memory_state_shapes(slots: int, heads: int, dim: int, vdim: int, mode: int):
     return (s, ) if mode != MEMORY_MLSTM else (s, (slots, heads, tiles, dim), (slots, heads, tiles))
 
 
-# A batch whose longest segment has at least MEMORY_CHUNKED_FROM tokens runs its segments of MEMORY_CHUNKED_MIN and more in chunks of 64 on the
-# matrix cores, and token by token what is shorter; any other batch is scanned.  One segment, scan / chunks in us: 64 tokens 21 / 24 (decay), 33 / 34
-# (mLSTM), 23 / 33 (state space); 96 tokens 30 / 24, 47 / 35, 33 / 34; where the launches are made anyway, shorter segments cost little in them
+# A batch whose longest segment has at least MEMORY_CHUNKED_FROM[mode] tokens (a single segment, several) runs its segments of MEMORY_CHUNKED_MIN and
+# more in chunks of 64 on the matrix cores, and token by token what is shorter; any other batch is scanned.  Scan / chunks in us: one segment of
+# 96 tokens 30 / 24 (decay, 8 heads of 64 x 128), 47 / 35 (mLSTM, 4 x 128 x 256), 33 / 35 (state space, 64 x 128 x 64), of 160 47 / 26, 74 / 37, 51 / 36; with
+# several the scan fills the chip and a chunk that is half empty costs as much as a full one: 4 of 160 91 / 94 (decay, 32 x 128 x 128), 8 of
+# 96 54 / 57 (mLSTM, 4 x 128 x 256), 4 of 192 92 / 100 (state space).  Where the launches are made anyway, shorter segments cost little in them
 # and would keep the token form's wide split, which single tokens beside them are slower in.
-MEMORY_CHUNKED_FROM, MEMORY_CHUNKED_MIN = 96, 32
+MEMORY_CHUNKED_FROM = {MEMORY_DECAY: (96, 193), MEMORY_MLSTM: (96, 128), MEMORY_STATE_SPACE: (160, 193)}
+MEMORY_CHUNKED_MIN = 32
 
 
 def outer_memory_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state, slot_of_seq: torch.Tensor,
@@ -303,7 +307,7 @@ def outer_memory_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state, 
             state[1].data_ptr() if len(state) > 1 else None, state[2].data_ptr() if len(state) > 2 else None,
             slot_of_seq.data_ptr(), slots, q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(), S, T, heads, d, e, int(mode),
             _p(decay), float(q_scale), float(gate_cap), qk_heads, _p(a_log), _p(dt_bias), _p(skip))
-    if max_q_len >= MEMORY_CHUNKED_FROM and d <= 128 and 0 < S <= 65535:
+    if max_q_len >= MEMORY_CHUNKED_FROM.get(int(mode), (1 << 30, ) * 2)[S > 1] and d <= 128 and 0 < S <= 65535:
         need = lib.aphro_outer_memory_chunked_workspace(S, T, heads, d, e, int(mode), MEMORY_CHUNKED_MIN)
         ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
         check(lib.aphro_outer_memory_chunked(*args, MEMORY_CHUNKED_MIN, ws.data_ptr(), need, _dt(q), _stream()), "outer_memory_scan")
@@ -829,10 +833,25 @@ def logit_softcap(z: torch.Tensor, scale: float = 1.0, cap: float = 0.0) -> torc
     return out
 
 
-# The delta rule's own line between the forms: a chunk's preparation is a chain of its own (a triangle of 64 tokens), 50 us however few there
-# are.  Scan / chunks in us, 16 heads of 128: one segment of 128 tokens 67 / 61 (a decay per channel), 48 / 52 (one per head), of 512 246 / 88,
-# 175 / 78; eight segments of 128 131 / 130, 83 / 111.
-DELTA_CHUNKED_FROM, DELTA_CHUNKED_MIN = 160, 32
+# The delta rule's own line between the forms.
+DELTA_CHUNKED_FROM, DELTA_CHUNKED_MIN = 128, 32
+
+
+def delta_chunks_pay(tokens: int, segments: int, longest: int, heads: int, dim: int, vdim: int, channel: bool) -> bool:
+    """Whether the chunked delta rule is expected to be the faster by a tenth, from times measured on MI355X (420 batches of 1 to 64 segments of 96 to
+    2048 tokens, 4 to 48 heads of 64 x 64 to 96 x 192: none of those it takes is slower than the scan).  The scan is bound by the longest segment's
+    chain of tokens or, where there are many segments and heads, by what all tokens take of the vector ALUs; the chunks by their preparation,
+    a workgroup a CU, and their products, more work than the scan's but with a chain a tenth as long.  Scan / chunks in us: one segment of
+    512 tokens, 16 heads of 128, a decay per channel 246 / 88, per head 175 / 78; sixteen of 256 444 / 336, 274 / 298; sixteen of 256, 48 heads of
+    64 382 / 554, 284 / 455."""
+    wide = dim > 64
+    chain = longest * ((0.48 if channel else 0.35) if wide else (0.34 if channel else 0.29))
+    work = tokens * heads * ((vdim + 15) // 16) * ((0.81 if channel else 0.50) if wide else (0.49 if channel else 0.35)) * 1e-3
+    scan = 8 + (chain ** 4 + work ** 4) ** 0.25
+    units = (tokens / 64 + min(segments, tokens / 32) / 2) * heads              # (segments that end in half a chunk, on the average)
+    prepare = (27.5 + 10 * channel if wide else 16 + 8 * channel) * math.ceil(units / 256)
+    chunks = 17.5 + (1.2 if wide else 0.6) * ((longest + 63) // 64) + prepare + (23 if wide else 17) * units * ((vdim + 63) // 64) / 256
+    return 1.1 * chunks < scan
 
 
 def gated_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, b: torch.Tensor, a: torch.Tensor, a_log: torch.Tensor,
@@ -862,7 +881,7 @@ def gated_delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, b: torch
             _rows(v, heads * e, "v"), b.data_ptr(), _rows(b, heads, "b"), a.data_ptr(), _rows(a, na, "a"), a_log.data_ptr(),
             dt_bias.data_ptr(), state.data_ptr(), slot_of_seq.data_ptr(), slots, q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(),
             S, T, heads, kv_heads, d, e, int(channel), float(q_scale), float(norm_eps))
-    if max_q_len >= DELTA_CHUNKED_FROM and d <= 128 and 0 < S <= 65535:
+    if max_q_len >= DELTA_CHUNKED_FROM and d <= 128 and 0 < S <= 65535 and delta_chunks_pay(T, S, int(max_q_len), heads, d, e, channel):
         need = lib.aphro_gated_delta_chunked_workspace(S, T, heads, d, e, DELTA_CHUNKED_MIN)
         ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
         check(lib.aphro_gated_delta_chunked(*args, DELTA_CHUNKED_MIN, ws.data_ptr(), need, _dt(q), _stream()), "gated_delta_scan")

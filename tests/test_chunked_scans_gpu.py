@@ -14,6 +14,13 @@ def mops():
     return mixer_ops
 
 
+@pytest.fixture(autouse=True)
+def chunks_whatever_pays(mops, monkeypatch):
+    monkeypatch.setattr(mops, "MEMORY_CHUNKED_FROM", {m: (1, 1) for m in mops.MEMORY_CHUNKED_FROM})
+    monkeypatch.setattr(mops, "DELTA_CHUNKED_FROM", 1)
+    monkeypatch.setattr(mops, "delta_chunks_pay", lambda *a: True)
+
+
 def i32(xs):
     return torch.tensor(list(xs), dtype=torch.int32, device=DEV)
 

@@ -774,3 +774,12 @@ def test_which_batches_the_expert_tile_takes():
         small = SimpleNamespace(num_experts=e, hidden=hidden, inter=inter, w13=w(hidden, 2 * inter), w2=w(inter, hidden))
         assert M.moe_tile_block(rows * e, small, torch.float16) == 64 and M.moe_tile_block(rows * e - 1, small, torch.float16) == 0
     assert M.moe_tile_block(6000, experts, torch.float16, 2 ** 32 - 2) == 64 and M.moe_tile_block(6000, experts, torch.float16, 2 ** 32 - 1) == 0
+
+
+def test_when_the_delta_rule_runs_in_chunks():
+    """mixer_ops.delta_chunks_pay at batches far from its line: long single portions, and many segments of many heads, which fill the chip token by
+    token."""
+    from aphrodite_engine_amd.mixer_ops import delta_chunks_pay as pay
+    assert pay(2000, 1, 2000, 16, 128, 128, True) and pay(2000, 1, 2000, 16, 128, 128, False) and pay(4096, 1, 4096, 48, 64, 64, False)
+    assert pay(2024, 25, 2000, 16, 128, 128, True)                       # a portion with decoded tokens beside it
+    assert not pay(4096, 16, 256, 48, 64, 64, True) and not pay(8192, 32, 256, 32, 128, 128, False) and not pay(512, 4, 128, 32, 128, 128, False)
