@@ -155,18 +155,22 @@ __device__ __forceinline__ void wna16_large_finish(const Wna16LargeParams& p, f3
         }
       }
       __syncthreads();
+      // eight loads at a time, by hand: left to itself hipcc loads, waits, adds (32 round trips: 6144 x 4096,
+      // 1500 rows 100.3 us, so 91 us)
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
+      for (int h = 0; h < 4; ++h) {
+        u32x4 raw[8];
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb)
+        for (int i = 0; i < 8; ++i)
+          raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rp, ((j * NWAVE + wave) * 32 + h * 8 + i) * 1024 + lane * 16, 0, 17);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const u32x4 raw = __builtin_amdgcn_raw_buffer_load_b128(
-                rp, ((j * NWAVE + wave) * 32 + (nb * 4 + mb) * 4 + q) * 1024 + lane * 16, 0, 17);
-            const f32x4 v = __builtin_bit_cast(f32x4, raw);
+        for (int i = 0; i < 8; ++i) {
+          const f32x4 v = __builtin_bit_cast(f32x4, raw[i]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[nb][mb][4 * q + r] += v[r];
-          }
+          for (int r = 0; r < 4; ++r) acc[h >> 1][(h & 1) * 2 + (i >> 2)][4 * (i & 3) + r] += v[r];
+        }
+      }
     }
   }
   if (!p.streamk && p.ksplit > 1) {          // fp32 slab of this K range; summed by splitk_reduce_large_kernel
