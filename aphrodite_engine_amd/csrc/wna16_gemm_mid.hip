@@ -77,53 +77,11 @@ __device__ __forceinline__ f16x8 mid_dq8(uint32_t w, f16x2 zh, f16x2 zh16, f16x2
   return __builtin_bit_cast(f16x8, r);
 }
 
-// ---- butterfly pieces: static register indices only (a runtime quad index would put the accumulators in scratch) -----
-// send / receive quads [Q0, Q0 + NQ) of n-blocks [NB0, NB0 + NNB)
-template <int MB, int NQ, int Q0, int NB0 = 0, int NNB = 4>
-__device__ __forceinline__ void mid_send(const f32x16 (&acc)[4][MB], float* red, int wave, int lane) {
-#pragma unroll
-  for (int nbi = 0; nbi < NNB; ++nbi)
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int qi = 0; qi < NQ; ++qi) {
-        const int q = Q0 + qi, nb = NB0 + nbi;
-        const f32x4 v = {acc[nb][mb][4 * q], acc[nb][mb][4 * q + 1], acc[nb][mb][4 * q + 2], acc[nb][mb][4 * q + 3]};
-        *reinterpret_cast<f32x4*>(&red[(((wave * (NNB * MB * NQ)) + (nbi * MB + mb) * NQ + qi) * 64 + lane) * 4]) = v;
-      }
-}
-template <int MB, int NQ, int Q0, int NB0 = 0, int NNB = 4>
-__device__ __forceinline__ void mid_recv(f32x16 (&acc)[4][MB], const float* red, int partner, int lane) {
-#pragma unroll
-  for (int nbi = 0; nbi < NNB; ++nbi)
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int qi = 0; qi < NQ; ++qi) {
-        const int q = Q0 + qi, nb = NB0 + nbi;
-        const f32x4 v = *reinterpret_cast<const f32x4*>(&red[(((partner * (NNB * MB * NQ)) + (nbi * MB + mb) * NQ + qi) * 64 + lane) * 4]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[nb][mb][4 * q + r] += v[r];
-      }
-}
-// wave owns quad Q (of n-blocks NB0 .. NB0 + NNB - 1): row m = mb * 32 + l31, columns 32 Q + 16 kh + (4 r + nb) of the
+// The wave that owns quad q of n-blocks nb0 .. holds row m = mb * 32 + l31, columns 32 q + 16 kh + (4 r + nb) of the
 // workgroup's 128.  Stored straight from the registers every instruction would scatter 16-byte pieces over 32 rows
 // (measured: 10 us of a 28 us kernel); the tile goes through LDS ([32 MB][128 + 4] fp32, conflict-free both ways) and
 // leaves as whole 512-byte rows.
 constexpr int MID_LDT = 132;
-template <int MB, int Q, int NB0 = 0, int NNB = 4>
-__device__ __forceinline__ void mid_put(const f32x16 (&acc)[4][MB], float* tile, int l31, int kh) {
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float* dst = &tile[(mb * 32 + l31) * MID_LDT + 32 * Q + 16 * kh + 4 * r + NB0];
-      if constexpr (NNB == 4)
-        *reinterpret_cast<f32x4*>(dst) = f32x4{acc[0][mb][4 * Q + r], acc[1][mb][4 * Q + r], acc[2][mb][4 * Q + r], acc[3][mb][4 * Q + r]};
-      else
-        *reinterpret_cast<f32x2*>(dst) = f32x2{acc[NB0][mb][4 * Q + r], acc[NB0 + 1][mb][4 * Q + r]};
-    }
-}
 template <int MB, int NWK>
 __device__ __forceinline__ void mid_flush(const float* tile, const Wna16MidParams& p, int n0, int wave, int lane) {
   constexpr int ROWS = 32 * MB / NWK;           // rows per wave
@@ -314,58 +272,63 @@ __global__ __launch_bounds__(64 * NWK, 2) void wna16_gemm_mid_kernel(Wna16MidPar
     p.partial[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * (64 * NWK) + threadIdx.x] = t;
     return;
   }
-  // ---- K reduction: butterfly over the wave index.  Quad rounds on bits SH+1 and SH (two quads each way, then one);
-  // with 8 waves a last round on bit 0 splits the n-blocks.  Fixed pairing -> fixed summation order. ---------------------
+  // ---- K reduction: butterfly over the wave index.  Rounds on bits SH + 1 and SH of it exchange two of the quads and then one; with
+  // 8 waves a last round on bit 0 splits the n-blocks.  Fixed pairing -> fixed summation order.  What a round keeps goes into an array of
+  // its own: merged back into the accumulators behind branches, all 128 of them met there and 81 were spilled (28672 x 4096, 64 rows:
+  // 42 us, so 26.6).  Piece i of a wave in a round of n: red[((wave * n + i) * 64 + lane) * 4]. ----------------------------------------
   constexpr int SH = NWK == 8 ? 1 : 0;
   const int wq = wave >> SH;                     // the quad this wave ends up owning
-  if (wq & 2) mid_send<MB, 2, 0>(acc, red, wave, lane); else mid_send<MB, 2, 2>(acc, red, wave, lane);
+  auto at = [&](int w, int n, int i) -> f32x4& { return *reinterpret_cast<f32x4*>(&red[((w * n + i) * 64 + lane) * 4]); };
+  auto quad = [&](int nb, int mb, int q) { return f32x4{acc[nb][mb][4 * q], acc[nb][mb][4 * q + 1], acc[nb][mb][4 * q + 2], acc[nb][mb][4 * q + 3]}; };
+  auto send = [&](auto q0) {
+#pragma unroll
+    for (int i = 0; i < 8 * MB; ++i) at(wave, 8 * MB, i) = quad(i / (2 * MB), i / 2 % MB, decltype(q0)::value + i % 2);
+  };
+  f32x4 two[8 * MB];                             // quads 2 (wq >> 1) and the next, [nb][mb][2]
+  auto keep = [&](auto q0) {
+#pragma unroll
+    for (int i = 0; i < 8 * MB; ++i) two[i] = quad(i / (2 * MB), i / 2 % MB, decltype(q0)::value + i % 2) + at(wave ^ (2 << SH), 8 * MB, i);
+  };
+  constexpr std::integral_constant<int, 0> low{};
+  constexpr std::integral_constant<int, 2> high{};
+  if (wq & 2) send(low); else send(high);
   __syncthreads();
-  if (wq & 2) mid_recv<MB, 2, 2>(acc, red, wave ^ (2 << SH), lane); else mid_recv<MB, 2, 0>(acc, red, wave ^ (2 << SH), lane);
+  if (wq & 2) keep(high); else keep(low);
   __syncthreads();
-  switch (wq) {
-    case 0: mid_send<MB, 1, 1>(acc, red, wave, lane); break;
-    case 1: mid_send<MB, 1, 0>(acc, red, wave, lane); break;
-    case 2: mid_send<MB, 1, 3>(acc, red, wave, lane); break;
-    default: mid_send<MB, 1, 2>(acc, red, wave, lane); break;
+  const bool odd = wq & 1;
+  f32x4 one[4 * MB];                             // quad wq, [nb][mb]
+#pragma unroll
+  for (int i = 0; i < 4 * MB; ++i) {
+    at(wave, 4 * MB, i) = odd ? two[2 * i] : two[2 * i + 1];
+    one[i] = odd ? two[2 * i + 1] : two[2 * i];
   }
   __syncthreads();
-  float* tile = red + 4096 * MB;                 // behind the last round's buffers (16 MB KiB): no barrier between recv and put
+#pragma unroll
+  for (int i = 0; i < 4 * MB; ++i) one[i] += at(wave ^ (1 << SH), 4 * MB, i);
+  float* tile = red + 4096 * MB;                 // behind the last round's buffers (16 MB KiB): no barrier between its reads and the tile
+  float* dst = &tile[l31 * MID_LDT + 32 * wq + 16 * kh];
   if constexpr (NWK == 4) {
-    switch (wq) {
-      case 0: mid_recv<MB, 1, 0>(acc, red, wave ^ 1, lane); mid_put<MB, 0>(acc, tile, l31, kh); break;
-      case 1: mid_recv<MB, 1, 1>(acc, red, wave ^ 1, lane); mid_put<MB, 1>(acc, tile, l31, kh); break;
-      case 2: mid_recv<MB, 1, 2>(acc, red, wave ^ 1, lane); mid_put<MB, 2>(acc, tile, l31, kh); break;
-      default: mid_recv<MB, 1, 3>(acc, red, wave ^ 1, lane); mid_put<MB, 3>(acc, tile, l31, kh); break;
-    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<f32x4*>(dst + mb * 32 * MID_LDT + 4 * r) = f32x4{one[mb][r], one[MB + mb][r], one[2 * MB + mb][r], one[3 * MB + mb][r]};
   } else {
-    switch (wq) {
-      case 0: mid_recv<MB, 1, 0>(acc, red, wave ^ 2, lane); break;
-      case 1: mid_recv<MB, 1, 1>(acc, red, wave ^ 2, lane); break;
-      case 2: mid_recv<MB, 1, 2>(acc, red, wave ^ 2, lane); break;
-      default: mid_recv<MB, 1, 3>(acc, red, wave ^ 2, lane); break;
+    __syncthreads();
+    const bool upper = wave & 1;                 // keeps n-blocks 2 and 3
+    f32x4 half[2 * MB];
+#pragma unroll
+    for (int i = 0; i < 2 * MB; ++i) {
+      at(wave, 2 * MB, i) = upper ? one[i] : one[2 * MB + i];
+      half[i] = upper ? one[2 * MB + i] : one[i];
     }
     __syncthreads();
-    switch (wave) {       // quad wq: the even wave keeps n-blocks 0, 1, the odd one 2, 3
-      case 0: mid_send<MB, 1, 0, 2, 2>(acc, red, wave, lane); break;
-      case 1: mid_send<MB, 1, 0, 0, 2>(acc, red, wave, lane); break;
-      case 2: mid_send<MB, 1, 1, 2, 2>(acc, red, wave, lane); break;
-      case 3: mid_send<MB, 1, 1, 0, 2>(acc, red, wave, lane); break;
-      case 4: mid_send<MB, 1, 2, 2, 2>(acc, red, wave, lane); break;
-      case 5: mid_send<MB, 1, 2, 0, 2>(acc, red, wave, lane); break;
-      case 6: mid_send<MB, 1, 3, 2, 2>(acc, red, wave, lane); break;
-      default: mid_send<MB, 1, 3, 0, 2>(acc, red, wave, lane); break;
-    }
-    __syncthreads();
-    switch (wave) {
-      case 0: mid_recv<MB, 1, 0, 0, 2>(acc, red, 1, lane); mid_put<MB, 0, 0, 2>(acc, tile, l31, kh); break;
-      case 1: mid_recv<MB, 1, 0, 2, 2>(acc, red, 0, lane); mid_put<MB, 0, 2, 2>(acc, tile, l31, kh); break;
-      case 2: mid_recv<MB, 1, 1, 0, 2>(acc, red, 3, lane); mid_put<MB, 1, 0, 2>(acc, tile, l31, kh); break;
-      case 3: mid_recv<MB, 1, 1, 2, 2>(acc, red, 2, lane); mid_put<MB, 1, 2, 2>(acc, tile, l31, kh); break;
-      case 4: mid_recv<MB, 1, 2, 0, 2>(acc, red, 5, lane); mid_put<MB, 2, 0, 2>(acc, tile, l31, kh); break;
-      case 5: mid_recv<MB, 1, 2, 2, 2>(acc, red, 4, lane); mid_put<MB, 2, 2, 2>(acc, tile, l31, kh); break;
-      case 6: mid_recv<MB, 1, 3, 0, 2>(acc, red, 7, lane); mid_put<MB, 3, 0, 2>(acc, tile, l31, kh); break;
-      default: mid_recv<MB, 1, 3, 2, 2>(acc, red, 6, lane); mid_put<MB, 3, 2, 2>(acc, tile, l31, kh); break;
-    }
+#pragma unroll
+    for (int i = 0; i < 2 * MB; ++i) half[i] += at(wave ^ 1, 2 * MB, i);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) *reinterpret_cast<f32x2*>(dst + mb * 32 * MID_LDT + 4 * r + 2 * upper) = f32x2{half[mb][r], half[MB + mb][r]};
   }
   __syncthreads();
   mid_flush<MB, NWK>(tile, p, n0, wave, lane);
