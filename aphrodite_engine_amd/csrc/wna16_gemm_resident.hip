@@ -614,8 +614,10 @@ __device__ __forceinline__ void res_reduce_store(const Wna16ResParams& p, float*
 // that -amdgpu-kernarg-preload-count (Makefile) has the dispatcher deliver it in SGPRs -- a by-value struct is fetched by
 // s_load at entry, one scalar-cache miss in front of every address (profiles/r5_decode_experiments.txt (2)).  p_in carries the rest;
 // its copies of the leading fields are not read.
+// Two m-tiles: 256 registers, so that the two halves of 33..64 rows share a CU.  (Left free, gate_up's instance takes 257 where fp32 has no packed
+// instructions: Llama-3-8B, 16 layers, a decode step of 33 / 64 rows 2333 / 2640 us, so 1978 / 2262.)
 template <int MT, int NWV, int NSEG, int NP4, int REM, int D>
-__global__ __launch_bounds__(NWV * 64, 1) void wna16_gemm_stream_kernel(const uint32_t* qw, const uint16_t* apk, int strips,
+__global__ __launch_bounds__(NWV * 64, MT) void wna16_gemm_stream_kernel(const uint32_t* qw, const uint16_t* apk, int strips,
                                                                         int xcd_shift, int strips_per_xcd, int ksplit, int M,
                                                                         int N, int K, int gshift, const uint16_t* sc,
                                                                         const uint32_t* qz, Wna16ResParams p_in) {
