@@ -535,7 +535,7 @@ __global__ __launch_bounds__(NWV * 64, NWV <= 4 ? 1 : 2) void wna16_gemm_residen
   }
 }
 
-// K reduction over the waves (LDS tile [wave][row][column]) + the three output forms; shared by the two kernels.
+// K reduction over the waves (LDS tile [wave][row][column], of sums times 2^-24) + the three output forms.
 template <int MT, int NWV, int NP4, int REM, int NTHREADS = NWV * 64>
 __device__ __forceinline__ void res_reduce_store(const Wna16ResParams& p, float* red, int WP, int ky, int cb, int mtiles,
                                                  int row0 = 0) {
@@ -554,7 +554,8 @@ __device__ __forceinline__ void res_reduce_store(const Wna16ResParams& p, float*
         f32x4 sum = zero4;
 #pragma unroll
         for (int w2 = 0; w2 < NWV; ++w2) sum += *reinterpret_cast<const f32x4*>(&red[w2 * WP + row * CWP + 16 * ch + 4 * q]);
-        v[4 * q] = sum[0]; v[4 * q + 1] = sum[1]; v[4 * q + 2] = sum[2]; v[4 * q + 3] = sum[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * q + e] = sum[e] * 16777216.f;
       }
       uint16_t o[8];
 #pragma unroll
@@ -578,7 +579,7 @@ __device__ __forceinline__ void res_reduce_store(const Wna16ResParams& p, float*
       f32x4 sum = zero4;
 #pragma unroll
       for (int w2 = 0; w2 < NWV; ++w2) sum += *reinterpret_cast<const f32x4*>(&red[w2 * WP + row * CWP + 4 * c4]);
-      if (row0 + row < p.M) *reinterpret_cast<f32x4*>(p.partial + ((size_t)ky * p.M + row0 + row) * p.N + cb + 4 * c4) = sum;
+      if (row0 + row < p.M) *reinterpret_cast<f32x4*>(p.partial + ((size_t)ky * p.M + row0 + row) * p.N + cb + 4 * c4) = sum * 16777216.f;
     }
   } else {
     constexpr int UNITS = ROWS * (CW / 8);
@@ -590,6 +591,8 @@ __device__ __forceinline__ void res_reduce_store(const Wna16ResParams& p, float*
         s0 += *reinterpret_cast<const f32x4*>(&red[w2 * WP + row * CWP + 8 * c8]);
         s1 += *reinterpret_cast<const f32x4*>(&red[w2 * WP + row * CWP + 8 * c8 + 4]);
       }
+      s0 *= 16777216.f;
+      s1 *= 16777216.f;
       uint16_t o[8];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -614,9 +617,15 @@ __device__ __forceinline__ void res_reduce_store(const Wna16ResParams& p, float*
 // that -amdgpu-kernarg-preload-count (Makefile) has the dispatcher deliver it in SGPRs -- a by-value struct is fetched by
 // s_load at entry, one scalar-cache miss in front of every address (profiles/r5_decode_experiments.txt (2)).  p_in carries the rest;
 // its copies of the leading fields are not read.
+// Everything a group adds carries the products' factor 2^-24 (weights enter them as subnormals) until the waves have met: the scale then
+// goes into the FMA as the f16 it is (v_fma_mix_f32), zero points convert a byte at a time and are scaled in the FMA that adds their
+// offset, and bf16 is an instantiation.  All factors are powers of two: the resident kernel's bits.  That is 2843 VALU instead of 3502 in gate_up's
+// two-tile instance (3032 with packed fp32, which the library is built without); Llama-3-8B, 16 layers, a decode step of 1 / 32 rows
+// 992.8 / 1407.9 -> 982.8 / 1401.8 us with the norm's squares as FMAs (fused_decode.hip).  The row sums keep ones that are normal
+// numbers: with 2^-24 in their place the products lose low bits.
 // Two m-tiles: 256 registers, so that the two halves of 33..64 rows share a CU.  (Left free, gate_up's instance takes 257 where fp32 has no packed
 // instructions: Llama-3-8B, 16 layers, a decode step of 33 / 64 rows 2333 / 2640 us, so 1978 / 2262.)
-template <int MT, int NWV, int NSEG, int NP4, int REM, int D>
+template <int MT, int NWV, int NSEG, int NP4, int REM, int D, bool BF16>
 __global__ __launch_bounds__(NWV * 64, MT) void wna16_gemm_stream_kernel(const uint32_t* qw, const uint16_t* apk, int strips,
                                                                         int xcd_shift, int strips_per_xcd, int ksplit, int M,
                                                                         int N, int K, int gshift, const uint16_t* sc,
@@ -624,6 +633,7 @@ __global__ __launch_bounds__(NWV * 64, MT) void wna16_gemm_stream_kernel(const u
   Wna16ResParams p = p_in;
   p.qw = qw; p.apk = apk; p.strips = strips; p.xcd_shift = xcd_shift; p.strips_per_xcd = strips_per_xcd; p.ksplit = ksplit;
   p.M = M; p.N = N; p.K = K; p.gshift = gshift; p.sc = sc; p.qz = qz;
+  p.is_bf16 = BF16;
   constexpr int NST = NSEG * 4;
   constexpr int CW = 64 * NP4 + 16 * REM;
   constexpr int CWP = CW + 4;
@@ -668,7 +678,7 @@ __global__ __launch_bounds__(NWV * 64, MT) void wna16_gemm_stream_kernel(const u
   const int voff_s4 = col4 * 2, voff_z4 = (col4 >> 3) * 4, zshift4 = (col4 & 7) * 4;
   const int voff_sr = colr * 2, voff_zr0 = (colr >> 3) * 4, voff_zr1 = ((colr + (REM > 0 ? REM - 1 : 0)) >> 3) * 4;
   const int zshiftr = (colr & 7) * 4;
-  const float zoff = (float)p.zero_offset;
+  const float nzoff = (float)p.zero_offset * -0x1p-24f;
   const f16x8 ones = {(f16)1.f, (f16)1.f, (f16)16.f, (f16)16.f, (f16)1.f, (f16)1.f, (f16)16.f, (f16)16.f};
   const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
 
@@ -766,29 +776,41 @@ __global__ __launch_bounds__(NWV * 64, MT) void wna16_gemm_stream_kernel(const u
     });
     if constexpr (u == 3) {
       const Meta& m = meta[s & 1];
-      res_static_for<0, NT>([&](auto T_) {
-        constexpr int t = decltype(T_)::value;
+      // even and odd nibbles as bytes, which convert in one instruction each
+      uint32_t z4[NP4 > 0 ? NP4 : 1][2], zr[2] = {0u, 0u};
+#pragma unroll
+      for (int pp = 0; pp < NP4; ++pp) {
+        const uint32_t zb = m.z[pp] >> zshift4;
+        z4[pp][0] = zb & 0x0f0fu;
+        z4[pp][1] = (zb >> 4) & 0x0f0fu;
+      }
+      if constexpr (REM > 0) {
         uint32_t zb;
-        uint16_t sb;
+        if constexpr (REM == 3) zb = __builtin_amdgcn_alignbit(m.zr1, m.zr0, zshiftr);
+        else zb = m.zr0 >> zshiftr;
+        zr[0] = zb & 0x0f0fu;
+        zr[1] = (zb >> 4) & 0x0f0fu;
+      }
+      res_static_for<0, NT>([&](auto T_) {
+        constexpr int t = decltype(T_)::value, tr = t < 4 * NP4 ? t % 4 : t - 4 * NP4;
+        uint32_t zb, word;          // the word that holds the column's scale
+        bool high;
         if constexpr (t < 4 * NP4) {
-          zb = (m.z[t / 4] >> zshift4) >> (4 * (t % 4));
-          sb = (uint16_t)(m.sc[2 * (t / 4) + ((t % 4) >> 1)] >> (16 * (t & 1)));
+          zb = z4[t / 4][tr & 1];
+          word = m.sc[2 * (t / 4) + (tr >> 1)], high = t & 1;
         } else {
-          constexpr int tr = t - 4 * NP4;
-          uint32_t zbits;
-          if constexpr (REM == 3) zbits = __builtin_amdgcn_alignbit(m.zr1, m.zr0, zshiftr);
-          else zbits = m.zr0 >> zshiftr;
-          zb = zbits >> (4 * tr);
-          if constexpr (REM == 2) sb = (uint16_t)(m.scr[0] >> (16 * tr));
-          else sb = (uint16_t)m.scr[tr];
+          zb = zr[tr & 1];
+          if constexpr (REM == 2) word = m.scr[0], high = tr;
+          else word = m.scr[tr], high = false;
         }
-        const float z = (float)(zb & 0xf) + zoff;
-        const float sf = p.is_bf16 ? bf16_bits_to_f32(sb) : f16_bits_to_f32(sb);
-        const float s24 = sf * 16777216.f;
-        const float nzs = -z * sf;
+        const float nz = __builtin_fmaf((float)((zb >> (8 * (tr >> 1))) & 0xffu), -0x1p-24f, nzoff);
+        float sf;
+        if constexpr (BF16) sf = __builtin_bit_cast(float, high ? word & 0xffff0000u : word << 16);
+        else sf = f16_bits_to_f32((uint16_t)(high ? word >> 16 : word));
+        const float nzs = nz * sf;
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-          cacc[i][t] = __builtin_elementwise_fma(acc[i][t], f32x4{s24, s24, s24, s24}, cacc[i][t]);
+          cacc[i][t] = __builtin_elementwise_fma(acc[i][t], f32x4{sf, sf, sf, sf}, cacc[i][t]);
           cacc[i][t] = __builtin_elementwise_fma(rs[i], f32x4{nzs, nzs, nzs, nzs}, cacc[i][t]);
         }
       });
@@ -924,12 +946,12 @@ static int res_launch(const Wna16ResParams& p, hipStream_t st) {
   return APHRO_OK;
 }
 
-template <int MT, int NWV, int NSEG, int NP4, int REM, int D>
-static int res_launch_stream(const Wna16ResParams& p, hipStream_t st) {
+template <int MT, int NWV, int NSEG, int NP4, int REM, int D, bool BF16>
+static int res_launch_stream_t(const Wna16ResParams& p, hipStream_t st) {
   constexpr int CW = 64 * NP4 + 16 * REM;
   constexpr size_t LDS = (size_t)NWV * 16 * MT * (CW + 4) * sizeof(float);
   static_assert(LDS <= 160 * 1024, "the K-reduce tile exceeds the LDS");
-  auto kern = wna16_gemm_stream_kernel<MT, NWV, NSEG, NP4, REM, D>;
+  auto kern = wna16_gemm_stream_kernel<MT, NWV, NSEG, NP4, REM, D, BF16>;
   if (LDS > 64 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS) != hipSuccess) {
     set_error("wna16_gemm_stream: cannot raise the dynamic LDS limit to %zu", LDS);
     return APHRO_ERR_LAUNCH;
@@ -941,6 +963,11 @@ static int res_launch_stream(const Wna16ResParams& p, hipStream_t st) {
                      q.K, q.gshift, q.sc, q.qz, q);
   APHRO_LAUNCH_CHECK();
   return APHRO_OK;
+}
+
+template <int MT, int NWV, int NSEG, int NP4, int REM, int D>
+static int res_launch_stream(const Wna16ResParams& p, hipStream_t st) {
+  return p.is_bf16 ? res_launch_stream_t<MT, NWV, NSEG, NP4, REM, D, true>(p, st) : res_launch_stream_t<MT, NWV, NSEG, NP4, REM, D, false>(p, st);
 }
 
 // ---- the instantiated configurations ------------------------------------------------------------------------------------

@@ -78,6 +78,25 @@ def test_resident_strip_layout_is_bit_identical(ops, K, N, M):
     np.testing.assert_allclose(s1.double().sum(0).cpu().numpy(), ref, rtol=1e-4, atol=2e-5 * np.abs(ref).max())
 
 
+@pytest.mark.parametrize("zero_offset", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,N", SHAPES)
+def test_stream_kernel_has_the_resident_kernel_s_bits(ops, K, N, dtype, zero_offset):
+    """Its sums carry 2^-24 until the waves have met, its zero points convert as bytes: every nibble, scales and rows over many
+    binades."""
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    qw = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 8, N), generator=g, device=DEV, dtype=torch.int32)
+    qz = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 128, N // 8), generator=g, device=DEV, dtype=torch.int32)
+    sc = (torch.rand(K // 128, N, generator=g, device=DEV) * torch.exp2(-12 * torch.rand(K // 128, 1, generator=g, device=DEV))).to(dtype)
+    strip = ops.wna16_strip_relayout(qw, 32, K // 128)
+    for M in (1, 17):
+        a = (torch.randn(M, K, generator=g, device=DEV) * torch.exp2(-20 * torch.rand(M, 1, generator=g, device=DEV))).to(dtype)
+        pk = ops.wna16_pack_a(a)
+        s0, _ = ops.wna16_gemm_resident(pk, M, K, qw, qz, sc, zero_offset, mode="slabs")
+        s1, _ = ops.wna16_gemm_resident(pk, M, K, strip, qz, sc, zero_offset, mode="slabs", strip_layout=True)
+        assert torch.equal(s0, s1), M
+
+
 @pytest.mark.parametrize("strip", [False, True])
 @pytest.mark.parametrize("M", [1, 17, 32])
 def test_resident_gate_up_silu_epilogue_vs_oracle(ops, M, strip):

@@ -34,10 +34,10 @@ def mean(xs):
     return sum(xs) / len(xs)
 
 
-ROLE = {"wna16_gemm_stream_kernel<2, 4, 8, 1, 3, 4>": "int4 gate_up + SiluAndMul (step kernel)",
-        "wna16_gemm_stream_kernel<2, 4, 7, 1, 0, 6>": "int4 down (step kernel)",
-        "wna16_gemm_stream_kernel<2, 4, 4, 1, 0, 6>": "int4 qkv (step kernel)",
-        "wna16_gemm_stream_kernel<2, 4, 2, 1, 0, 4>": "int4 o (step kernel)",
+ROLE = {"wna16_gemm_stream_kernel<2, 4, 8, 1, 3, 4, false>": "int4 gate_up + SiluAndMul (step kernel)",
+        "wna16_gemm_stream_kernel<2, 4, 7, 1, 0, 6, false>": "int4 down (step kernel)",
+        "wna16_gemm_stream_kernel<2, 4, 4, 1, 0, 6, false>": "int4 qkv (step kernel)",
+        "wna16_gemm_stream_kernel<2, 4, 2, 1, 0, 4, false>": "int4 o (step kernel)",
         "paged_attention_kernel<aphro::Half, 0, 128, 16, 8, 1, false>": "decode attention ctx 1100 (fused rope form)",
         "add_rms_norm_pack_kernel<aphro::Half, false, false, 4>": "norm + pack",
         "lm_head_argmax_kernel<aphro::Half, 2, 4>": "LM head + argmax",
