@@ -146,11 +146,9 @@ __global__ void add_rms_norm_pack_kernel(const uint16_t* __restrict__ input, con
         }
         if (residual) *reinterpret_cast<u16x8*>(residual + off) = rs2;
         {
-          // squares rounded, then added -- pinned: the norm-in-consumer GEMM launch (wna16_gemm_resident.hip, res_norm_finish)
-          // reproduces this row bit for bit and must not depend on which of the two loops hipcc contracts into FMAs
-#pragma clang fp contract(off)
+          // (squares of 16-bit numbers are exact in fp32: one FMA each has the bits of multiply and add)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) ss += v[it][j] * v[it][j];
+          for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(v[it][j], v[it][j], ss);
         }
         continue;
       } else if (slabs) {
