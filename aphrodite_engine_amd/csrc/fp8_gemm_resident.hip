@@ -31,7 +31,8 @@
 //     hipcc's own fp32 division sequence (v_rcp, one Newton step on the reciprocal, q = n r, residual corrections) with
 //     the per-ROW part -- reciprocal + its refinement -- hoisted and ONE residual correction (proven sufficient for every
 //     (input, scale) pair that can occur, see F8R_DIV_STEPS): 3 VALU per element
-//     (v_mul_f32, two v_fma_f32), on |x| with the sign put back on the packed bytes (-0 stays -0 as v_div_fixup_f32 would leave it).
+//     (FMAs, of which the two that take x read the f16 as it is: v_fma_mix_f32; with conversions in front of a multiply down's instance had 2649
+//     vector instructions, so 2201: 32 rows of 8192 keys, 8 layers, a decode step 1450.2 -> 1445.9 us), on |x| with the sign put back on the packed bytes (-0 stays -0 as v_div_fixup_f32 would leave it).
 //     v_div_scale_f32 is the identity for every finite 16-bit x and scale in [1 / (448 * 512), 65504 / 448]; the clamp to
 //     +-448 is a no-op when |x| <= absmax.  tests: aphro_fp8_quant_rows_aq runs the same device function over all 65 536
 //     f16 / bf16 inputs x adversarial scales against x / scale.
@@ -95,32 +96,26 @@ typedef f16 f16x8_t __attribute__((ext_vector_type(8)));
 // 8 consecutive 16-bit values (one 16-byte load) -> 8 e4m3 bytes (lo: elements 0..3, hi: 4..7)
 template <typename T>
 __device__ __forceinline__ void f8r_quant8(const u32x4 h, const F8Rcp rc, uint32_t& lo, uint32_t& hi) {
-  const f32x2 nd = {-rc.s, -rc.s}, rr = {rc.r, rc.r};
-  f32x2 q[4];
-  // (a bit-cast of ONE element of an ext-vector may read element 0 -- DESIGN 3: cast the whole vector)
+  float q[8];
+  // (a bit-cast of ONE element of an ext-vector may read element 0: cast the whole vector)
   const f16x8_t hv = __builtin_bit_cast(f16x8_t, h);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    f32x2 n;
-    if constexpr (__is_same(T, Half)) {
-      n = f32x2{__builtin_fabsf((float)hv[2 * j]), __builtin_fabsf((float)hv[2 * j + 1])};
-    } else {
-      n = f32x2{__builtin_bit_cast(float, (h[j] << 16) & 0x7fffffffu), __builtin_bit_cast(float, h[j] & 0x7fff0000u)};
-    }
-    const f32x2 q0 = n * rr;
-    const f32x2 e1 = __builtin_elementwise_fma(nd, q0, n);
-    const f32x2 q1 = __builtin_elementwise_fma(e1, rr, q0);
+  for (int j = 0; j < 8; ++j) {
+    float n;
+    if constexpr (__is_same(T, Half)) n = __builtin_fabsf((float)hv[j]);
+    else n = __builtin_bit_cast(float, (j & 1 ? h[j / 2] : h[j / 2] << 16) & 0x7fffffffu & (j & 1 ? 0xffff0000u : ~0u));
+    const float q0 = __builtin_fmaf(n, rc.r, 0.f);         // (an FMA reads the f16 as it is, a multiply does not: v_fma_mix_f32)
+    const float e1 = __builtin_fmaf(-rc.s, q0, n);
+    q[j] = __builtin_fmaf(e1, rc.r, q0);
 #if F8R_DIV_STEPS >= 2
-    const f32x2 e2 = __builtin_elementwise_fma(nd, q1, n);
-    q[j] = __builtin_elementwise_fma(e2, rr, q1);
-#else
-    q[j] = q1;
+    const float e2 = __builtin_fmaf(-rc.s, q[j], n);
+    q[j] = __builtin_fmaf(e2, rc.r, q[j]);
 #endif
   }
-  int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(q[0][0], q[0][1], 0, false);
-  w0 = __builtin_amdgcn_cvt_pk_fp8_f32(q[1][0], q[1][1], w0, true);
-  int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(q[2][0], q[2][1], 0, false);
-  w1 = __builtin_amdgcn_cvt_pk_fp8_f32(q[3][0], q[3][1], w1, true);
+  int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
+  w0 = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], w0, true);
+  int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], 0, false);
+  w1 = __builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], w1, true);
   // signs: the high byte of every 16-bit element, gathered by one v_perm_b32 per four
   const uint32_t s01 = __builtin_amdgcn_perm(h[1], h[0], 0x07050301u);
   const uint32_t s23 = __builtin_amdgcn_perm(h[3], h[2], 0x07050301u);
