@@ -500,14 +500,20 @@ def wna16_large_ok(m: int, n: int, k: int, groups: int) -> bool:
         and (k // 8) * n * 4 < 2 ** 32 and m * k * 2 < 2 ** 32
 
 
-def wna16_prefers_large(m: int, n: int, k: int) -> bool:
-    """Between 65 and 128 rows the small projections (weights < 16 MiB) stay with the decode kernel (two 64-row passes over the weights):
-    it multiplies exact integers and applies the group scales to fp32 sums, where the tiles round every scaled weight to 16 bits --
-    a float16 result's error against 64 bits grows from 2.1e-4 (its own rounding) to 2.9e-4.  In time the tile whose height fits the
-    batch (csrc/wna16_gemm_rows.hip) would win: 6144 x 4096 at 65 / 128 rows 16.2 / 22 against 20.5 / 25.1 us, 4096 x 4096 15.5 / 23
-    against 19.1 / 24.6 us.  The large matrices go to the tiles (gate_up 59 vs 52 us, down 43 vs 35 us at 96 rows before that
-    tile; tools/mid_gemm_bench.py, profiles/r2_mid_gemm.txt)."""
-    return m > 128 or n * k >= 2 ** 25
+def wna16_prefers_large(m: int, n: int, k: int, dtype: Optional[torch.dtype] = None, groups: int = 0, strip: bool = False) -> bool:
+    """Which of 65 to 128 rows leave the decode kernels: the large matrices (gate_up 59 vs 52 us, down 43 vs 35 us at 96 rows before there
+    was a tile whose height fits the batch; tools/mid_gemm_bench.py, profiles/r2_mid_gemm.txt), and below 2^25 weights float16 calls for
+    the form of that tile which rounds no weight (csrc/wna16_gemm_rows.hip, EXACT; the decode kernels multiply exact integers too).
+    Against the decode kernel's two 64-row passes by how many K tiles a CU has to do: us at 65 / 96 / 128 rows, up to 15 tiles 17.3 / 20.3 / 22
+    -> 15 / 15.8 / 17.3 (4096 x 4096), 25.7 / 28.4 / 33.5 -> 18 / 18.4 / 19 (5120 x 5120), 14 / 15 / 15 -> 10 (1024 x 1024); 16 tiles 18.9 / 20.4 / 21.8 ->
+    20.8 / 20.3 / 21.5 (4096 x 6144): from 96 rows; two rounds of 8 14.8 / 16.3 -> 19.6 (1024 x 24576): never.  Against the strip-major copy's
+    32-row passes always: 28 / 30.1 / 38.3 -> 21 / 20.6 / 21.7 (4096 x 6144).  bfloat16 stays with the decode kernels."""
+    if m > 128 or n * k >= 2 ** 25:
+        return True
+    if dtype != torch.float16 or m <= WNA16_LARGE_MIN_M or k % 128 != 0 or groups <= 0:
+        return False
+    tiles = _lib.lib().aphro_wna16_rows_exact_tiles(m, n, k, groups)
+    return tiles > 0 and (strip or tiles < 16 or (tiles == 16 and m >= 96))
 
 
 def _wna16_large(a, qweight, qzeros, scales, perm, zero_offset):
@@ -594,7 +600,7 @@ def wna16_linear_strip(a: torch.Tensor, strip: torch.Tensor, qzeros: torch.Tenso
     if m == 0:
         return torch.empty((0, n), dtype=a.dtype, device=a.device)
     large = wna16_large_ok(m, n, k, groups) and not switch("APHRO_WNA16_NO_LARGE")
-    if large and wna16_prefers_large(m, n, k):
+    if large and wna16_prefers_large(m, n, k, a.dtype, groups, strip=True):
         return wna16_gemm_large_strip(a, strip, qzeros, scales, zero_offset, strip_m=strip_m)
     if wna16_prefers_mid(m, n, k) and wna16_mid_ok(m, n, k, groups) and a.dtype == scales.dtype and not switch("APHRO_WNA16_NO_MID"):
         # 33..64 rows on the big matrices: ONE pass of the 32x32x16 kernel over the strip-major words (the generic op's own rule)
@@ -662,7 +668,7 @@ def _wna16_mid(a, qweight, qzeros, scales, perm, zero_offset):
 def _wna16(a, qweight, qzeros, scales, perm, zero_offset):
     m, k = a.shape
     n = qweight.shape[1]
-    if wna16_large_ok(m, n, k, scales.shape[0]) and wna16_prefers_large(m, n, k) \
+    if wna16_large_ok(m, n, k, scales.shape[0]) and wna16_prefers_large(m, n, k, a.dtype if perm is None else None, scales.shape[0]) \
             and not switch("APHRO_WNA16_NO_LARGE"):
         return _wna16_large(a, qweight, qzeros, scales, perm, zero_offset)
     if wna16_prefers_mid(m, n, k) and wna16_mid_ok(m, n, k, scales.shape[0]) and not switch("APHRO_WNA16_NO_MID"):

@@ -1042,13 +1042,23 @@ static bool large_eight(const LargePlan& pl, int64_t K) {
   return pl.wm == 2 && pl.wn == 4 && pl.streamk && eight;
 }
 
+// 65 to 128 float16 rows of a matrix below 2^25 weights belong to the decode kernels otherwise, which round no weight: nor does the tile's EXACT form.
+static Wna16RowsPlan rows_exact_plan(int64_t M, int64_t N, int64_t K, int64_t gs) {
+  if (M > 128 || N * K >= (1 << 25) || knobs().wna16_large_8phase >= 0 || knobs().wna16_large_two_pass >= 0) return {0, 1, false};
+  return wna16_rows_plan_exact(M, N, K, gs, 36ll << 20);
+}
+
 // The tile of wna16_gemm_rows.hip, up to 4096 rows: always where this file would take one workgroup per tile (4096 x 4096: 150 rows
 // 27.3 -> 18.3 us, 1300 rows 78 -> 56 us), and beside the stream-K form where its last round is full enough (28672 x 4096: 300 rows
 // 127 -> 82 us, 1300 rows 341 -> 326 us; 2048 rows 450 against 489 us: stays).  Its K slices are its own, of any whole K tiles up to 36 MiB of slabs;
 // this file's are ranges of whole groups, of which 11008 or 9728 rows of K have few divisors and one group per column none (4096 x 11008 at 65
 // / 150 / 300 rows with slices bound to this file's 53 / 54 / 54 us, without 21 / 28 / 40 us).
-static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs) {
-  if (knobs().wna16_large_8phase >= 0 || knobs().wna16_large_two_pass >= 0) return {0, 1};      // a switch names this file's forms
+static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype) {
+  if (knobs().wna16_large_8phase >= 0 || knobs().wna16_large_two_pass >= 0) return {0, 1, false};      // a switch names this file's forms
+  if (dtype == APHRO_F16) {
+    const Wna16RowsPlan exact = rows_exact_plan(M, N, K, gs);
+    if (exact.mb > 0) return exact;
+  }
   int64_t other_ns = -1;
   if (pl.streamk) {            // 1.9 us per 256 x 256 x 64 of a CU's even share, 18 us around them
     const int64_t units = (M + 255) / 256 * ((N + 255) / 256) * (K / 64);
@@ -1063,8 +1073,16 @@ static size_t large_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t gro
   size_t b = dtype == APHRO_BF16 ? ((size_t)M * K * 2 + 255) / 256 * 256 : 0;
   if (large_two_pass(pl, M, N, K, K / groups)) b += ((size_t)N * K * 2 + 255) / 256 * 256;      // f16 W^T of the two-pass form
   (void)strip_m;              // (every plan addresses the strip-major copy in place: nothing is rebuilt)
-  const size_t slabs = wna16_rows_slab_bytes(rows_plan(pl, M, N, K, K / groups), M, N), other = large_scratch_bytes(pl, M, N);
+  const size_t slabs = wna16_rows_slab_bytes(rows_plan(pl, M, N, K, K / groups, dtype), M, N), other = large_scratch_bytes(pl, M, N);
   return b + (slabs > other ? slabs : other);
+}
+
+extern "C" int aphro_wna16_rows_exact_tiles(int64_t M, int64_t N, int64_t K, int64_t groups) {
+  if (groups <= 0 || K % groups != 0) return 0;
+  const Wna16RowsPlan pl = rows_exact_plan(M, N, K, K / groups);
+  if (pl.mb == 0) return 0;
+  const int64_t cus = device_cu_count(), rounds = (2 * (N / 128) * pl.ksplit + cus - 1) / cus;
+  return (int)(rounds * ((K / 128 + pl.ksplit - 1) / pl.ksplit) + (rounds - 1) * 8);
 }
 
 // Bytes of scratch aphro_wna16_gemm_large needs: the f16 copy of bf16 activations + the fp32 split-K slabs.
@@ -1137,7 +1155,7 @@ static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const 
       APHRO_CHECK(((x * p.st_inv_nseg) >> 16) == x / p.st_nseg && ((x * p.st_inv_nwv) >> 16) == x / p.st_nwv,
                   "wna16_gemm_large_strip: multiply-shift division fails at %u (nseg %d, nwv %d)", x, p.st_nseg, p.st_nwv);
   }
-  const Wna16RowsPlan rp = rows_plan(pl, M, N, K, gs);
+  const Wna16RowsPlan rp = rows_plan(pl, M, N, K, gs, dtype);
   if (rp.mb > 0) {
     Wna16RowsParams q = {};
     q.a = p.a; q.lda = p.lda; q.qw = p.qw; q.qz = p.qz; q.sc = p.sc; q.c = p.c; q.partial = (float*)ws;

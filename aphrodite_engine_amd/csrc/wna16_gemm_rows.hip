@@ -30,7 +30,8 @@ __device__ __forceinline__ uint32_t rw_and_or(uint32_t a, uint32_t mask, uint32_
   asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(mask), "v"(orv));
   return r;
 }
-// one exllama dword -> 8 scaled f16: ((1024 + q) - (1024 + z)) * s  (exact difference, one rounding)
+// one exllama dword -> 8 f16: (1024 + q) - (1024 + z), exact, and times the scale where SCALED (one rounding)
+template <bool SCALED>
 __device__ __forceinline__ f16x8 rw_dq8(uint32_t w, f16x2 zh, f16x2 zh16, f16x2 sc) {
   const f16x2 inv16 = {(f16)0.0625f, (f16)0.0625f};
   const uint32_t magic = 0x64006400u;
@@ -39,10 +40,11 @@ __device__ __forceinline__ f16x8 rw_dq8(uint32_t w, f16x2 zh, f16x2 zh16, f16x2 
   const uint32_t w8 = w >> 8;
   const uint32_t q2 = rw_and_or(w8, 0x000f000fu, magic);
   const uint32_t q3 = rw_and_or(w8, 0x00f000f0u, magic);
-  const f16x2 d0 = (__builtin_bit_cast(f16x2, q0) - zh) * sc;
-  const f16x2 d1 = (__builtin_bit_cast(f16x2, q1) * inv16 + zh16) * sc;
-  const f16x2 d2 = (__builtin_bit_cast(f16x2, q2) - zh) * sc;
-  const f16x2 d3 = (__builtin_bit_cast(f16x2, q3) * inv16 + zh16) * sc;
+  f16x2 d0 = __builtin_bit_cast(f16x2, q0) - zh;
+  f16x2 d1 = __builtin_bit_cast(f16x2, q1) * inv16 + zh16;
+  f16x2 d2 = __builtin_bit_cast(f16x2, q2) - zh;
+  f16x2 d3 = __builtin_bit_cast(f16x2, q3) * inv16 + zh16;
+  if constexpr (SCALED) d0 *= sc, d1 *= sc, d2 *= sc, d3 *= sc;
   u32x4 r = {__builtin_bit_cast(uint32_t, d0), __builtin_bit_cast(uint32_t, d1), __builtin_bit_cast(uint32_t, d2),
              __builtin_bit_cast(uint32_t, d3)};
   return __builtin_bit_cast(f16x8, r);
@@ -50,7 +52,9 @@ __device__ __forceinline__ f16x8 rw_dq8(uint32_t w, f16x2 zh, f16x2 zh16, f16x2 
 
 constexpr int RW_BN = 128, RW_BK = 128, RW_STAGES = 4;
 constexpr int rw_pass(int mb) { return (mb + 1) / 2; }      // 32-row blocks whose K groups meet in LDS at a time
-constexpr size_t rw_lds(int mb) {
+constexpr int RW_EXACT_GROUPS = 64;                         // of a K slice, whose scales EXACT keeps in LDS behind the stages
+constexpr size_t rw_lds(int mb, bool exact = false) {
+  if (exact) return (size_t)RW_STAGES * mb * 32 * RW_BK * 2 + RW_EXACT_GROUPS * RW_BN * 2;
   const size_t stages = (size_t)RW_STAGES * mb * 32 * RW_BK * 2, meet = (size_t)8 * 3 * rw_pass(mb) * 2048;
   return stages > meet ? stages : meet;
 }
@@ -60,8 +64,14 @@ __device__ __forceinline__ size_t rw_image(const Wna16RowsParams& p, int MB, int
   return (((size_t)ks * (p.tiles_m * p.tiles_n) + tile) * MB + mb) * 4096 + (size_t)group * 512;
 }
 
-template <int MB, bool BF16, bool STRIP>
+// EXACT: the numerics of the decode kernels -- the integers q - z enter the products, and a K tile's fp32 sum is added times its group's
+// fp32 scale, one FMA an accumulator element (with the f16 scale as it is: v_fma_mix_f32).  An accumulator's columns are other lanes'
+// weights, so the scales come from LDS, 16 bytes a quad.  Twice the accumulators, so two 32-row blocks at most.  float16, 65 / 128 rows, 4096 x 4096:
+// 15.0 / 17.3 us, error against 64 bits 2.08e-4, a float16 result's own rounding; the form that rounds weights 15.5 / 23 us, 2.87e-4; the
+// decode kernel, two passes of 64 rows, 17.3 / 22.0 us.
+template <int MB, bool BF16, bool STRIP, bool EXACT>
 __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p) {
+  static_assert(!EXACT || (MB <= 2 && !BF16), "registers; bf16 stays with the decode kernels");
   constexpr int STAGE = MB * 32 * RW_BK * 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63;
@@ -101,7 +111,7 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   uint32_t scr[3], zr[3];
   auto load_w = [&](auto set) {
     constexpr int S = decltype(set)::value;
-    scr[S] = scp[(size_t)grp * (p.N >> 1)];
+    if constexpr (!EXACT) scr[S] = scp[(size_t)grp * (p.N >> 1)];
     zr[S] = zp[(size_t)grp * (p.N >> 3)];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -132,14 +142,51 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
     for (int i = 0; i < MB; ++i) load_a(st, i);
     advance();
   };
-  constexpr int LOADS = MB + 4;                            // memory instructions of one load()
-  f32x16 acc[2][MB];
+  constexpr int LOADS = MB + (EXACT ? 3 : 4);              // memory instructions of one load()
+  f32x16 acc[2][MB], total[EXACT ? 2 : 1][EXACT ? MB : 1];
 #pragma unroll
   for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[nb][mb][r] = 0.f;
+      for (int r = 0; r < 16; ++r) {
+        acc[nb][mb][r] = 0.f;
+        if constexpr (EXACT) total[nb][mb][r] = 0.f;
+      }
+  // EXACT: scales of the slice's groups, [group][128 columns]; the accumulators' columns 16 q + 8 kh + 2 r + nb are 16 bytes for a quad
+  constexpr int SC_LOADS = RW_EXACT_GROUPS * (RW_BN / 2) / 512;
+  unsigned char* sc_lds = smem + RW_STAGES * STAGE;
+  const int slice_grp = t0 * RW_BK / p.group_size;
+  uint32_t sc_reg[SC_LOADS];
+  if constexpr (EXACT) {
+    const int dwords = ((t1 * RW_BK - 1) / p.group_size + 1 - slice_grp) * (RW_BN / 2);
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(p.sc + (size_t)slice_grp * p.N + n0);
+#pragma unroll
+    for (int i = 0; i < SC_LOADS; ++i) {
+      const int x = threadIdx.x + 512 * i;
+      sc_reg[i] = x < dwords ? src[(size_t)(x >> 6) * (p.N >> 1) + (x & 63)] : 0u;
+    }
+    asm volatile("" ::: "memory");                         // (ahead of the loads that are counted)
+  }
+  int tile_grp = first_grp, tile_in = first_in;             // of the tile being multiplied
+  auto fold = [&] {
+    const unsigned char* row = sc_lds + (tile_grp - slice_grp) * (RW_BN * 2) + wn * 128 + kh * 16;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f16x8 s8 = *reinterpret_cast<const f16x8*>(row + q * 32);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            total[EXACT ? nb : 0][EXACT ? mb : 0][4 * q + r] =
+                __builtin_fmaf(acc[nb][mb][4 * q + r], (float)s8[2 * r + nb], total[EXACT ? nb : 0][EXACT ? mb : 0][4 * q + r]);
+    }
+    tile_grp += grp_step;
+    tile_in += grp_rest;
+    if (tile_in >= p.group_size) { tile_in -= p.group_size; ++tile_grp; }
+  };
   // ---- K loop.  While a step's (16 k) MFMAs run, the next step's activations come from LDS and its weights are unpacked, across the
   // tiles' borders too: halfway through a tile the next one has to be there -----------------------------------------------------------
   u32x4 af[2][MB];
@@ -155,7 +202,8 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
     constexpr int S = decltype(set)::value;
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
-      const uint16_t sb = (uint16_t)(nb ? scr[S] >> 16 : scr[S]);
+      uint16_t sb = 0;
+      if constexpr (!EXACT) sb = (uint16_t)(nb ? scr[S] >> 16 : scr[S]);
       const int z = (int)((zr[S] >> (zshift + 4 * nb)) & 0xf) + p.zero_offset;
       const f16 s16 = BF16 ? (f16)bf16_bits_to_f32(sb) : __builtin_bit_cast(f16, sb);
       const f16 a16 = __builtin_bit_cast(f16, (uint16_t)(0x6400 | z));       // 1024 + z
@@ -168,15 +216,16 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   auto unpack = [&](auto set, auto step) {
     constexpr int S = decltype(set)::value, J = decltype(step)::value;
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) wf[J][nb] = rw_dq8(wr[S][J][nb], zh[nb], zh16[nb], sv[nb]);
+    for (int nb = 0; nb < 2; ++nb) wf[J][nb] = rw_dq8<!EXACT>(wr[S][J][nb], zh[nb], zh16[nb], sv[nb]);
   };
   auto multiply = [&](auto step) {
     constexpr int J = decltype(step)::value;
+    const f32x16 zero = {};
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
-        acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[J][nb], __builtin_bit_cast(f16x8, af[J][mb]), acc[nb][mb], 0, 0, 0);
+        acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[J][nb], __builtin_bit_cast(f16x8, af[J][mb]), EXACT && J == 0 ? zero : acc[nb][mb], 0, 0, 0);
   };
   int stage = 0;                                           // of the tile being multiplied
   auto tile = [&](auto set, auto more) {
@@ -211,6 +260,10 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
     } else {
       multiply(std::integral_constant<int, 1>{});
     }
+    if constexpr (EXACT) {
+      fold();
+      __builtin_amdgcn_sched_barrier(0);                   // (the next tile's sums would be a second set of accumulators)
+    }
   };
   constexpr std::integral_constant<int, 0> set0{};
   constexpr std::integral_constant<int, 1> set1{};
@@ -220,7 +273,11 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   load(set1, 1);
   asm volatile("" ::: "memory");
   load(set2, 2);
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * LOADS) : "memory");
+  if constexpr (EXACT) {
+#pragma unroll
+    for (int i = 0; i < SC_LOADS; ++i) reinterpret_cast<uint32_t*>(sc_lds)[threadIdx.x + 512 * i] = sc_reg[i];
+  }
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(2 * LOADS) : "memory");
   __builtin_amdgcn_s_barrier();
   read_a(0, 0, af[0]);
   meta(set0);
@@ -239,6 +296,10 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   if (left > 1) tile(set1, std::false_type{});
   // ---- the four K groups meet in LDS: the wave of group g ends with quad g of every block, columns 16 g + 8 kh + 2 r + nb ----------
   constexpr int RM = rw_pass(MB);
+  auto& sum = [&]() -> f32x16 (&)[2][MB] {
+    if constexpr (EXACT) return total;
+    else return acc;
+  }();
 #pragma unroll
   for (int m1 = 0; m1 < MB; m1 += RM) {
     __syncthreads();
@@ -252,7 +313,7 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
           if (m1 + i < MB)
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
-              const f32x16& x = acc[nb][m1 + i < MB ? m1 + i : 0];
+              const f32x16& x = sum[nb][m1 + i < MB ? m1 + i : 0];
               *reinterpret_cast<f32x4*>(dst + (i * 2 + nb) * 1024) = f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
             }
       } else {
@@ -261,7 +322,7 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
           if (m1 + i < MB)
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb) {
-              const f32x16& x = acc[nb][m1 + i < MB ? m1 + i : 0];
+              const f32x16& x = sum[nb][m1 + i < MB ? m1 + i : 0];
               own[nb][i] = f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
             }
       }
@@ -339,7 +400,7 @@ __global__ __launch_bounds__(256) void wna16_rows_reduce_kernel(Wna16RowsParams 
 // them, and the slabs written and read again at 2.2 TB/s behind 3 us.  4096 x 14336, 150 rows: one slice 115 us, two 56, four 35, eight
 // 30; 4096 x 4096, 150 rows: five blocks and five slices 20.7, twice three blocks and four slices 18.0 us.
 Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t gs, int64_t slab_bytes, int64_t other_ns) {
-  Wna16RowsPlan best = {0, 1};
+  Wna16RowsPlan best = {0, 1, false};
   if (M <= 64 || M > 4096 || N % RW_BN || K % RW_BK || gs % 64) return best;
   const int cus = device_cu_count();
   const int64_t T = K / RW_BK;
@@ -351,26 +412,45 @@ Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t gs, int64
       if (ks > 1 && slabs > slab_bytes) break;
       const int64_t rounds = (tiles * ks + cus - 1) / cus;
       const int64_t ns = rounds * ((T + ks - 1) / ks * (170 + 200 * mb) + 4700) + (ks > 1 ? 3000 + slabs * 45 / 100000 : 0);
-      if (best_ns < 0 || ns < best_ns) { best = {mb, ks}; best_ns = ns; }
+      if (best_ns < 0 || ns < best_ns) { best = {mb, ks, false}; best_ns = ns; }
     }
   }
   return best;
 }
 
-template <int MB, bool BF16, bool STRIP>
+// The EXACT form, 65 to 128 rows: two tiles of 64.  K slices by the time they are expected to take, as above; a slice's groups fit its LDS.
+Wna16RowsPlan wna16_rows_plan_exact(int64_t M, int64_t N, int64_t K, int64_t gs, int64_t slab_bytes) {
+  Wna16RowsPlan best = {0, 1, true};
+  if (M <= 64 || M > 128 || N % RW_BN || K % RW_BK || gs % 64) return best;
+  const int cus = device_cu_count();
+  const int64_t T = K / RW_BK, tiles = 2 * (N / RW_BN);
+  int64_t best_ns = -1;
+  for (int ks = 1; ks <= 16 && (ks == 1 || T / ks >= 4); ++ks) {
+    const int64_t slabs = 128 * N * 4 * ks;
+    if (ks > 1 && slabs > slab_bytes) break;
+    bool fits = true;
+    for (int i = 0; i < ks; ++i) fits = fits && ((i + 1) * T / ks * RW_BK - 1) / gs - i * T / ks * RW_BK / gs < RW_EXACT_GROUPS;
+    if (!fits) continue;
+    const int64_t ns = (tiles * ks + cus - 1) / cus * ((T + ks - 1) / ks * 700 + 4700) + (ks > 1 ? 3000 + slabs * 45 / 100000 : 0);
+    if (best_ns < 0 || ns < best_ns) { best = {2, ks, true}; best_ns = ns; }
+  }
+  return best;
+}
+
+template <int MB, bool BF16, bool STRIP, bool EXACT>
 static int rows_launch(Wna16RowsParams p, hipStream_t st) {
   p.tiles_m = (p.M + MB * 32 - 1) / (MB * 32);
   p.tiles_n = p.N / RW_BN;
   static bool attr_set_dev[APHRO_MAX_DEVICES] = {}; bool& attr_set = attr_set_dev[device_slot()];
   if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)wna16_gemm_rows_kernel<MB, BF16, STRIP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)wna16_gemm_rows_kernel<MB, BF16, STRIP, EXACT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             160 * 1024) != hipSuccess) {
       set_error("wna16_gemm_rows: cannot raise the dynamic LDS limit");
       return APHRO_ERR_LAUNCH;
     }
     attr_set = true;
   }
-  hipLaunchKernelGGL((wna16_gemm_rows_kernel<MB, BF16, STRIP>), dim3(p.tiles_m * p.tiles_n * p.ksplit), dim3(512), rw_lds(MB), st, p);
+  hipLaunchKernelGGL((wna16_gemm_rows_kernel<MB, BF16, STRIP, EXACT>), dim3(p.tiles_m * p.tiles_n * p.ksplit), dim3(512), rw_lds(MB, EXACT), st, p);
   APHRO_LAUNCH_CHECK();
   if (p.ksplit > 1) {
     hipLaunchKernelGGL(wna16_rows_reduce_kernel<BF16>, dim3(p.tiles_m * p.tiles_n * MB * 2), dim3(256), 0, st, p, MB);
@@ -381,8 +461,8 @@ static int rows_launch(Wna16RowsParams p, hipStream_t st) {
 
 template <int MB>
 static int rows_launch_mb(const Wna16RowsParams& p, hipStream_t st) {
-  if (p.bf16) return p.strip.on ? rows_launch<MB, true, true>(p, st) : rows_launch<MB, true, false>(p, st);
-  return p.strip.on ? rows_launch<MB, false, true>(p, st) : rows_launch<MB, false, false>(p, st);
+  if (p.bf16) return p.strip.on ? rows_launch<MB, true, true, false>(p, st) : rows_launch<MB, true, false, false>(p, st);
+  return p.strip.on ? rows_launch<MB, false, true, false>(p, st) : rows_launch<MB, false, false, false>(p, st);
 }
 
 size_t wna16_rows_slab_bytes(const Wna16RowsPlan& plan, int64_t M, int64_t N) {
@@ -391,6 +471,7 @@ size_t wna16_rows_slab_bytes(const Wna16RowsPlan& plan, int64_t M, int64_t N) {
 }
 
 int wna16_rows_launch(const Wna16RowsParams& p, const Wna16RowsPlan& plan, hipStream_t st) {
+  if (plan.exact) return p.strip.on ? rows_launch<2, false, true, true>(p, st) : rows_launch<2, false, false, true>(p, st);
   if (plan.mb == 3) return rows_launch_mb<3>(p, st);
   if (plan.mb == 4) return rows_launch_mb<4>(p, st);
   return rows_launch_mb<5>(p, st);

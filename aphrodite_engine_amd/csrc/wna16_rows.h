@@ -22,8 +22,10 @@ struct Wna16RowsParams {
 
 // 32-row blocks of a workgroup's tile (0: the kernel does not take the call, or needs longer than other_ns >= 0) and K slices, whose
 // slabs, ksplit x M rounded up to tiles x N floats, fit slab_bytes
-struct Wna16RowsPlan { int mb, ksplit; };
+struct Wna16RowsPlan { int mb, ksplit; bool exact; };
 Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t slab_bytes, int64_t other_ns);
+// the same of the form that multiplies exact integers and scales fp32 sums: 65 to 128 rows, float16
+Wna16RowsPlan wna16_rows_plan_exact(int64_t M, int64_t N, int64_t K, int64_t group_size, int64_t slab_bytes);
 // bytes of Wna16RowsParams::partial
 size_t wna16_rows_slab_bytes(const Wna16RowsPlan& plan, int64_t M, int64_t N);
 int wna16_rows_launch(const Wna16RowsParams& p, const Wna16RowsPlan& plan, hipStream_t st);

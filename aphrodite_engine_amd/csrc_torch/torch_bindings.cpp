@@ -477,7 +477,9 @@ torch::Tensor wna16_dispatch(torch::Tensor a, const torch::Tensor& qweight, cons
   const int64_t gs = groups > 0 ? k / groups : 0;
   const bool large_ok = m > 64 && n % 128 == 0 && k % 64 == 0 && groups > 0 && k % groups == 0 && gs % 64 == 0 &&
                         (k / 8) * n * 4 < (int64_t(1) << 32) && m * k * 2 < (int64_t(1) << 32);
-  const bool prefers_large = m > 128 || n * k >= (int64_t(1) << 25);
+  // (_custom_ops.wna16_prefers_large has the reasons)
+  const int exact = dt == APHRO_F16 && !has_perm && m > 64 && k % 128 == 0 ? aphro_wna16_rows_exact_tiles(m, n, k, groups) : 0;
+  const bool prefers_large = m > 128 || n * k >= (int64_t(1) << 25) || (exact > 0 && exact < 16) || (exact == 16 && m >= 96);
   auto out = torch::empty({m, n}, a.options());
   auto gathered = [&]() {
     torch::Tensor x = has_perm ? a.index_select(1, perm.to(torch::kLong)) : a;

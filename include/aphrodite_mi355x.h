@@ -639,6 +639,9 @@ int aphro_custom_ar_init_loopback(void** fa_out, void* signal, void* scratch, si
  * workspace: aphro_wna16_gemm_large_workspace_bytes (f16 copy of bf16 activations, saturating; fp32 split-K slabs when
  * the tile grid alone would not cover the chip). */
 size_t aphro_wna16_gemm_large_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype);
+/* 65 to 128 float16 rows of a matrix below 2^25 weights: K tiles of 128 that a CU has to do (a further round of workgroups counts as
+ * eight) in the form of aphro_wna16_gemm_large that multiplies exact integers and scales fp32 sums; 0: no such form for the call. */
+int aphro_wna16_rows_exact_tiles(int64_t M, int64_t N, int64_t K, int64_t groups);
 int aphro_wna16_gemm_large(const void* a, const uint32_t* q_weight, const uint32_t* qzeros, const void* scales,
                            void* c, void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K,
                            int64_t groups, int64_t lda, int zero_offset, int dtype, void* stream);

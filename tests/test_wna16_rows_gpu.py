@@ -74,6 +74,20 @@ def test_small_projections_do_not_round_their_weights(m, k, n):
     assert all(float((x.double() - want).norm()) < bound for x in got)
 
 
+@pytest.mark.parametrize("m", [65, 97, 128])
+@pytest.mark.parametrize("k,n,group", [(128, 128, 128), (640, 384, 64), (4224, 256, 128), (1536, 2048, 192), (8192, 1024, 64), (16384, 512, 64), (4096, 1024, 4096)])
+def test_tiles_that_round_no_weight(m, k, n, group):
+    """The form for 65 to 128 float16 rows: groups inside, across and beside K tiles, more of them than one slice's scales fit."""
+    from aphrodite_engine_amd import _custom_ops as ops, _lib
+    assert _lib.lib().aphro_wna16_rows_exact_tiles(m, n, k, k // group) > 0
+    qw, qz, sc, g = weights(k, n, group, torch.float16, m + n)
+    a = torch.randn(m, k + 8, generator=g, device=DEV).half()[:, :k]
+    want = a.double() @ dense(qw, qz, sc, 0)
+    got = ops._wna16_large(a, qw, qz, sc, None, 0)
+    assert float((got.double() - want).norm()) < 1.02 * float((want.half().double() - want).norm())
+    assert torch.equal(ops._wna16_large(a, qw, qz, sc, None, 0), got)
+
+
 @pytest.mark.parametrize("m,k,n", [(65, 576, 256), (150, 4160, 4096), (300, 4160, 1024), (513, 2112, 8192)])
 def test_k_that_the_row_tile_does_not_take(m, k, n):
     """K = 64 (mod 128): the few-tile plans of csrc/wna16_gemm_large.hip, K slices of whole groups among them."""
