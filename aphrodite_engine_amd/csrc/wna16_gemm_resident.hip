@@ -622,7 +622,7 @@ __device__ __forceinline__ void res_reduce_store(const Wna16ResParams& p, float*
 // offset, and bf16 is an instantiation.  All factors are powers of two: the resident kernel's bits.  That is 2843 VALU instead of 3502 in gate_up's
 // two-tile instance (3032 with packed fp32, which the library is built without); Llama-3-8B, 16 layers, a decode step of 1 / 32 rows
 // 992.8 / 1407.9 -> 982.8 / 1401.8 us with the norm's squares as FMAs (fused_decode.hip).  The row sums keep ones that are normal
-// numbers: with 2^-24 in their place the products lose low bits.
+// numbers: with 2^-24 in their place the sums' last bits changed.
 // Two m-tiles: 256 registers, so that the two halves of 33..64 rows share a CU.  (Left free, gate_up's instance takes 257 where fp32 has no packed
 // instructions: Llama-3-8B, 16 layers, a decode step of 33 / 64 rows 2333 / 2640 us, so 1978 / 2262.)
 template <int MT, int NWV, int NSEG, int NP4, int REM, int D, bool BF16>
