@@ -782,4 +782,5 @@ def test_when_the_delta_rule_runs_in_chunks():
     from aphrodite_engine_amd.mixer_ops import delta_chunks_pay as pay
     assert pay(2000, 1, 2000, 16, 128, 128, True) and pay(2000, 1, 2000, 16, 128, 128, False) and pay(4096, 1, 4096, 48, 64, 64, False)
     assert pay(2024, 25, 2000, 16, 128, 128, True)                       # a portion with decoded tokens beside it
+    assert pay(2228, 28, 551, 32, 128, 128, True)                        # ... and four: the rows are not portions that end in half a chunk
     assert not pay(4096, 16, 256, 48, 64, 64, True) and not pay(8192, 32, 256, 32, 128, 128, False) and not pay(512, 4, 128, 32, 128, 128, False)
