@@ -261,6 +261,9 @@ def memory_state_shapes(slots: int, heads: int, dim: int, vdim: int, mode: int):
 # several the scan fills the chip and a chunk that is half empty costs as much as a full one: 4 of 160 91 / 94 (decay, 32 x 128 x 128), 8 of
 # 96 54 / 57 (mLSTM, 4 x 128 x 256), 4 of 192 92 / 100 (state space).  Where the launches are made anyway, shorter segments cost little in them
 # and would keep the token form's wide split, which single tokens beside them are slower in.
+# Beside many segments that are much shorter -- decoded rows, scanned either way -- the scan has no such chip to fill and the line is MEMORY_CHUNKED_BESIDE:
+# one of 128 beside 24 single tokens 44 / 34, 102 / 79 (decay, 8 heads of 64 x 128, 32 of 128 x 128), 95 / 83 (state space); two of 190 141 / 105.
+MEMORY_CHUNKED_BESIDE = 128
 MEMORY_CHUNKED_FROM = {MEMORY_DECAY: (96, 193), MEMORY_MLSTM: (96, 128), MEMORY_STATE_SPACE: (160, 193)}
 MEMORY_CHUNKED_MIN = 32
 
@@ -307,7 +310,10 @@ def outer_memory_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state, 
             state[1].data_ptr() if len(state) > 1 else None, state[2].data_ptr() if len(state) > 2 else None,
             slot_of_seq.data_ptr(), slots, q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(), S, T, heads, d, e, int(mode),
             _p(decay), float(q_scale), float(gate_cap), qk_heads, _p(a_log), _p(dt_bias), _p(skip))
-    if max_q_len >= MEMORY_CHUNKED_FROM.get(int(mode), (1 << 30, ) * 2)[S > 1] and d <= 128 and 0 < S <= 65535:
+    line = MEMORY_CHUNKED_FROM.get(int(mode), (1 << 30, ) * 2)[S > 1]
+    if S * max_q_len > 2 * T and int(mode) in MEMORY_CHUNKED_FROM:
+        line = min(line, MEMORY_CHUNKED_BESIDE)
+    if max_q_len >= line and d <= 128 and 0 < S <= 65535:
         need = lib.aphro_outer_memory_chunked_workspace(S, T, heads, d, e, int(mode), MEMORY_CHUNKED_MIN)
         ws = torch.empty(need // 4, dtype=torch.float32, device=q.device)
         check(lib.aphro_outer_memory_chunked(*args, MEMORY_CHUNKED_MIN, ws.data_ptr(), need, _dt(q), _stream()), "outer_memory_scan")
