@@ -1733,6 +1733,72 @@ def argmax_rows(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Te
     return out
 
 
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_transforms, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+_raw_stream, _current_device = torch._C._cuda_getCurrentRawStream, torch.cuda.current_device
+
+
+def _launchable(*tensors) -> bool:
+    """Tensors whose memory a kernel may be launched on right away: nothing records, traces or batches what happens to them."""
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad):
+            return False
+    return not (_dispatch_modes() or _function_modes() or _transforms() or _tracing() or torch.compiler.is_compiling())
+
+
+def dense_rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, act: int = -1,
+               out: Optional[torch.Tensor] = None, f32: bool = False) -> Optional[torch.Tensor]:
+    """x [M, K] . weight [N, K]^T (+ bias) for few rows on the weight-stream kernel (csrc/dense_rows.hip); ``act`` 0 (silu) / 1 (gelu, tanh
+    form): act(x . weight[:N/2]^T) * (x . weight[N/2:]^T); ``f32``: the 16-bit result widened.  None, without a launch, where the form is not
+    served (rows, sizes, types, strides, alignment, device, anything that traces): the caller has a general path."""
+    if x.dim() != 2 or x.shape[0] > 192 or not x.is_cuda or weight.dim() != 2:
+        return None
+    dt = _DT.get(x.dtype)
+    if dt is None or dt == _lib.F32 or not _launchable(x, weight):
+        return None
+    (M, K), (N, kw), (lda, one), (ldw, onew) = x.shape, weight.shape, x.stride(), weight.stride()
+    dev = x.get_device()
+    if M == 0 or kw != K or one != 1 or onew != 1 or weight.dtype != x.dtype or weight.get_device() != dev \
+            or dev != _current_device():
+        return None
+    if act >= 0:
+        if N % 2 or bias is not None:
+            return None
+        N //= 2
+    if M == 1:
+        lda = K
+    need = _lib.lib().aphro_dense_rows_slab_floats(M, N, K, lda, ldw, act)
+    xp, wp, bp = x.data_ptr(), weight.data_ptr(), None
+    if need < 0 or (xp | wp) & 15:
+        return None
+    if bias is not None:
+        bp = bias.data_ptr()
+        if bias.dtype != x.dtype or bias.get_device() != dev or not bias.is_contiguous() or bias.numel() != N or bp & 7 or not _launchable(bias):
+            return None
+    if out is None:
+        out = torch.empty(M, N, dtype=torch.float32 if f32 else x.dtype, device=x.device)
+    elif out.dtype != (torch.float32 if f32 else x.dtype) or out.shape != (M, N) or out.stride(1) != 1 or out.get_device() != dev or not _launchable(out) \
+            or out.stride(0) % 4 or (M > 1 and out.stride(0) < N) or out.data_ptr() % (16 if f32 else 8):
+        return None
+    slabs = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
+    check(_lib.lib().aphro_dense_rows(out.data_ptr(), max(out.stride(0), N), xp, lda, wp, ldw, bp, None if slabs is None else slabs.data_ptr(), need,
+                                      M, N, K, act, int(f32), dt, _raw_stream(dev)), "dense_rows")
+    return out
+
+
+def dense_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """torch.nn.functional.linear, on ``dense_rows`` where that serves the call."""
+    out = dense_rows(x, weight, bias)
+    return torch.nn.functional.linear(x, weight, bias) if out is None else out
+
+
+def dense_logits(hidden: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """A head's product in the activation type, widened to fp32."""
+    out = dense_rows(hidden, weight, f32=True)
+    return torch.nn.functional.linear(hidden, weight).float() if out is None else out
+
+
 def lm_head_argmax_supported(m: int, k: int, v: int, ldw: int, dtype: torch.dtype) -> bool:
     return dtype in (torch.float16, torch.bfloat16) and \
         bool(_lib.lib().aphro_lm_head_argmax_supported(m, k, v, ldw, _DT[dtype]))

@@ -110,6 +110,8 @@ SIGNATURES = {
     "aphro_wna16_gemm_large_strip_workspace_bytes": (Z, [L, L, L, L, I, L]),
     "aphro_wna16_gemm_large_strip": (I, [P, P, P, P, P, P, Z, L, L, L, L, L, I, I, I, L, P]),
     "aphro_wna16_gemm_rowmajor_supported": (I, [L, L, L, L, I]),
+    "aphro_dense_rows_slab_floats": (L, [L, L, L, L, L, I]),
+    "aphro_dense_rows": (I, [P, L, P, L, P, L, P, P, L, L, L, L, I, I, I, P]),
     "aphro_lm_head_argmax_supported": (I, [L, L, L, L, I]),
     "aphro_fp8_moe_gemm": (I, [P, P, P, P, P, P, P, P, P, L, L, L, L, I, I, P]),
     "aphro_moe_route_align": (I, [P, P, P, L, P, P, P, P, L, I, I, I, I, I, P]),

@@ -17,8 +17,8 @@ from typing import Any, Dict, Iterable, List, Optional, Tuple
 
 import torch
 from torch import nn
-from torch.nn import functional as F
 
+from . import _custom_ops as ops
 from . import mixer_ops as mops
 from .mixers import DistanceBiasAttention, GatedMLP, LayerNormParams, OuterProductMemory
 from .step_batch import StepBatch
@@ -215,7 +215,7 @@ class FatudraForCausalLM(nn.Module):
         y, post, yb = pend
         h = mops.residual_layer_norm(xs, y=y.index_select(0, rows), post=post, y_bias=yb, pre=self.final_norm.pair(),
                                      eps=self.cfg.eps)
-        return F.linear(h, self.head).float()
+        return ops.dense_logits(h, self.head)
 
     def forward(self, batch: StepBatch, caches):
         """Returns the residual stream and the last sublayer's still-unadded output (y, its norm, its fp32 bias): every

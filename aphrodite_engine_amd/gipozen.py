@@ -18,8 +18,8 @@ from typing import Any, Dict, Iterable, List, Optional, Tuple
 
 import torch
 from torch import nn
-from torch.nn import functional as F
 
+from . import _custom_ops as ops
 from . import mixer_ops as mops
 from .mixers import PolyNormMLP, RoutedExperts, WindowedMapsAttention
 from .step_batch import StepBatch
@@ -164,7 +164,7 @@ class GipozenForCausalLM(nn.Module):
         return self.logits(h.index_select(0, rows))
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(h, self.head).float() * self.cfg.logit_scale
+        return ops.dense_logits(h, self.head) * self.cfg.logit_scale
 
     def forward(self, batch: StepBatch, caches) -> torch.Tensor:
         """The final norm's output for every row of the batch."""

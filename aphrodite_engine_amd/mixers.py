@@ -45,6 +45,7 @@ from typing import List, Optional, Tuple
 import torch
 from torch import nn
 
+from . import _custom_ops as ops
 from . import mixer_ops as mops
 from .step_batch import StepBatch
 
@@ -208,7 +209,8 @@ class GatedMLP(nn.Module):
 
     def inner(self, h: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """What the output product reads, into ``out`` [T, ff] (dense rows, any row stride) if given."""
-        return mops.act_and_mul(self.gate_up(h), self.act, out)
+        few = ops.dense_rows(h, self.gate_up.weight, act=self.act, out=out)
+        return mops.act_and_mul(self.gate_up(h), self.act, out) if few is None else few
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         return self.down(self.inner(h))

@@ -121,7 +121,7 @@ class QuantLinear(nn.Module):
         (RowParallelLinear.forward, linear.py:1136-1150)."""
         bias = self.bias if add_bias else None
         if self.quant_method is None:
-            return torch.nn.functional.linear(x, self.weight, bias)
+            return ops.dense_linear(x, self.weight, bias)
         if getattr(self, "qweight_strip_major", False):
             # DecoderLayer.enable_one_copy: ``qweight`` holds the strip-major order of the decode kernels, the only resident
             # copy -- any M through the kernels that read it (ops.wna16_linear_strip), never through the quant method's op
@@ -1075,7 +1075,7 @@ class LlamaForCausalLM(nn.Module):
         return self.compute_logits(hidden.index_select(0, rows)).float()
 
     def compute_logits(self, hidden):
-        logits = torch.matmul(hidden, self.lm_head.t())
+        logits = ops.dense_linear(hidden, self.lm_head)
         if get_tensor_model_parallel_world_size() > 1:
             from .distributed import tensor_model_parallel_all_gather
             logits = tensor_model_parallel_all_gather(logits, dim=-1)

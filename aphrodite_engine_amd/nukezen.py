@@ -20,8 +20,8 @@ from typing import Any, Dict, Iterable, List, Optional, Tuple
 
 import torch
 from torch import nn
-from torch.nn import functional as F
 
+from . import _custom_ops as ops
 from . import mixer_ops as mops
 from .mixers import GatedDeltaMixer, GatedMLP, GroupedQueryAttention, RotaryFrequencies, SelectiveStateSpace
 from .step_batch import StepBatch
@@ -274,7 +274,7 @@ class NukezenForCausalLM(nn.Module):
         return self.logits(self.forward(batch, caches, rows))
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(h, self.embed).float()
+        return ops.dense_logits(h, self.embed)
 
     def forward(self, batch: StepBatch, caches, rows: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The final norm's output for the rows asked for (all rows if ``rows`` is None).  In the last layer everything behind the

@@ -22,8 +22,8 @@ from typing import Any, Dict, Iterable, List, Optional, Tuple
 
 import torch
 from torch import nn
-from torch.nn import functional as F
 
+from . import _custom_ops as ops
 from . import mixer_ops as mops
 from .mixers import (GatedDeltaMixer, LatentAttention, RotaryFrequencies, RotaryGQAttention, RoutedExperts, StreamedResidual,
                      interleaved_to_half)
@@ -172,7 +172,7 @@ class PagulixForCausalLM(nn.Module):
         return self.logits(h)
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        return mops.logit_softcap(F.linear(h, self.embed), 1.0, self.cfg.logit_softcap)
+        return mops.logit_softcap(ops.dense_linear(h, self.embed), 1.0, self.cfg.logit_softcap)
 
     def _sublayers(self):
         out = []

@@ -21,8 +21,8 @@ from typing import Any, Dict, Iterable, List, Optional, Tuple
 
 import torch
 from torch import nn
-from torch.nn import functional as F
 
+from . import _custom_ops as ops
 from . import mixer_ops as mops
 from .mixers import (DynamicTanh, GatedMLP, GroupedQueryAttention, JoinedOutput, LatentAttention, RotaryFrequencies, looped_layers)
 from .step_batch import StepBatch
@@ -212,7 +212,7 @@ class VivisunForCausalLM(nn.Module):
         return self.logits(self.forward(batch, caches, rows))
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(h, self.head).float()
+        return ops.dense_logits(h, self.head)
 
     def forward(self, batch: StepBatch, caches, rows: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The final norm's output for the rows asked for (all rows if ``rows`` is None).  In the last layer run everything behind the

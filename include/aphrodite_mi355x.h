@@ -975,6 +975,14 @@ int aphro_lm_head_argmax_supported(int64_t M, int64_t K, int64_t V, int64_t ldw,
 int aphro_lm_head_argmax(const void* hidden, int64_t lda, const void* weight, int64_t ldw, void* logits, int64_t ldl,
                          int64_t* out_ids, int64_t M, int64_t K, int64_t V, int dtype, void* stream);
 
+/* out[M, N] = x[M, K] . weight[N, K]^T (+ bias[N]) for up to 192 rows, 16-bit operands, fp32 sums rounded once (out_f32: the rounded
+ * values widened).  act 0 (silu) / 1 (gelu, tanh form): weight is [2 N, K] and out = act(x . weight[:N]^T) * (x . weight[N:]^T), no bias;
+ * act -1: none.  K % 64 == 0, N % 8 == 0, strides in elements, lda and ldw multiples of 8, operands 16-byte aligned.
+ * aphro_dense_rows_slab_floats: fp32 scratch the call needs (0: none), -1 where the form is not served. */
+int64_t aphro_dense_rows_slab_floats(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int act);
+int aphro_dense_rows(void* out, int64_t ldo, const void* x, int64_t lda, const void* weight, int64_t ldw, const void* bias, float* slabs,
+                     int64_t slab_floats, int64_t M, int64_t N, int64_t K, int act, int out_f32, int dtype, void* stream);
+
 /* Greedy sampling: out[r] = argmax_c x[r][c] (lowest index on ties) -- the torch.argmax of
  * modeling/layers/sampler.py:_greedy_sample as one pass over each logits row. */
 int aphro_argmax_rows(int64_t* out, const void* x, int64_t rows, int64_t cols,
