@@ -210,6 +210,7 @@ MIXERS_SIGNATURES = {
     "aphro_latent_prep": (I, [P, P, L, P, L, I, I, P, P, P, P, P, P, P, F, L, I, I, I, I, F, I, P]),
     "aphro_latent_attention_plain": (I, [P, L, L, P, L, L, P, L, L, P, P, I, L, I, P, P, P, P, F, L, I, I, I, I, F, I, P, P, L, I, P]),
     "aphro_latent_attention_fast_supported": (I, [I, I, I, I]),
+    "aphro_latent_gather": (I, [P, L, P, I, P, P, I, L, I, P, P, I, I, I, P]),
     "aphro_latent_attention_splits": (I, [L, I, I, I, I]),
     "aphro_latent_attention": (I, [P, L, L, P, L, L, P, L, L, P, P, I, L, I, P, P, P, P, P, F, L, I, I, I, I, I, I, I, F, I, P, P, L, P, L, I, P]),
     "aphro_sigmoid_gate_mul": (I, [P, L, P, L, P, L, L, I, I, P]),

@@ -658,6 +658,26 @@ def latent_prep(proj: torch.Tensor, q_at: int, q_rank: int, kv_at: int, kv_rank:
     return cq
 
 
+def latent_gather(cache: torch.Tensor, block_tables: torch.Tensor, q_len: torch.Tensor, ctx_len: torch.Tensor, lens) -> tuple:
+    """(rows [N, D], tables int32 [S, blocks]): the cache rows that segments see, bf16 [blocks, block, D], one segment after the other from
+    multiples of 16 rows on, and their numbers as blocks of 16.  ``lens``: every segment's ctx_len + q_len, known on the host."""
+    _cuda(cache, block_tables, q_len, ctx_len)
+    S, (nb, bs, D) = len(lens), cache.shape
+    _need(cache.dtype == torch.bfloat16 and cache.is_contiguous() and D % 8 == 0, "latent_gather: cache bf16 [blocks, block, D], contiguous")
+    _need(block_tables.dtype == torch.int32 and block_tables.dim() == 2 and block_tables.shape[0] == S and block_tables.is_contiguous(),
+          "latent_gather: block_tables int32 [S, max_blocks]")
+    _i32(q_len, S, "q_len")
+    _i32(ctx_len, S, "ctx_len")
+    _need(S > 0 and min(lens) > 0 and max(lens) <= block_tables.shape[1] * bs, "latent_gather: lengths beyond the tables")
+    blocks = [(n + 15) // 16 for n in lens]
+    rows = torch.empty(16 * sum(blocks), D, dtype=cache.dtype, device=cache.device)
+    tables = torch.empty(S, max(blocks), dtype=torch.int32, device=cache.device)
+    check(_lib.mixers_lib().aphro_latent_gather(rows.data_ptr(), rows.shape[0], tables.data_ptr(), tables.shape[1], cache.data_ptr(),
+                                                block_tables.data_ptr(), block_tables.shape[1], nb, bs, q_len.data_ptr(), ctx_len.data_ptr(),
+                                                S, D, _dt(cache), _stream()), "latent_gather")
+    return rows, tables
+
+
 def _head_view(t: torch.Tensor, T: int, heads: int, n: int, what: str):
     """(token stride, head stride) of a [T, heads, n] view whose last axis is dense."""
     _need(t.dim() == 3 and tuple(t.shape) == (T, heads, n) and (t.stride(2) == 1 or n == 1), f"{what}: [T, heads, {n}] with a dense last axis")

@@ -430,6 +430,12 @@ def interleaved_to_half(t: torch.Tensor, dims: int, at: int = 0) -> torch.Tensor
     return t.index_select(0, idx.to(t.device))
 
 
+# Latents are expanded where prompt portions have LATENT_EXPAND_ROWS rows in all and either half of the keys they see are their own, or a key is
+# seen often enough to pay for its expansion (heads * kv_rank * pairs of a row and a key, over keys); up to LATENT_EXPAND_MOST numbers of
+# keys and values (512 MiB).
+LATENT_EXPAND_ROWS, LATENT_EXPAND_PAIRS, LATENT_EXPAND_MOST = 96, 2.5e6, 1 << 28
+
+
 class LatentAttention(nn.Module):
     """Causal softmax attention whose keys and values are products of a cached low-rank latent.
 
@@ -439,7 +445,8 @@ class LatentAttention(nn.Module):
 
     Every projection that reads h -- W_dq, W_dkv, W_g -- is one product.  The attention itself runs in the latent (the cache
     holds [c | rot(k_r)] per token and nothing per head): q_lat,a = W_uk,a^T q_n,a is a batched product over heads, the kernel
-    returns sum_j p_ij c_j per head, and W_uv,a is applied to that, again batched over heads."""
+    returns sum_j p_ij c_j per head, and W_uv,a is applied to that, again batched over heads.  Prompt portions without a rotary part
+    make keys and values per head instead (expanded_segments)."""
 
     def __init__(self, width: int, heads: int, dim: int, rot_dim: int, vdim: int, q_rank: int, kv_rank: int, scale: float,
                  rotary: RotaryFrequencies, eps: float, dtype, prefix: str = "", gate=True, window: int = 0,
@@ -490,6 +497,23 @@ class LatentAttention(nn.Module):
     def finalize(self) -> None:
         self.rotary.to(self.w_uk.device)
 
+    def expanded_segments(self, batch: StepBatch) -> int:
+        """Number of leading prompt portions that attend over keys and values per head, made for this call, instead of in the latent: 4 dim
+        operations a (row, key, head) instead of 4 kv_rank, for one more product of every latent seen.  kv_rank 512, attention and the products
+        around it, us in the latent / expanded: fresh prompts of 96, 512, 4096 tokens 61 / 60, 116 / 87, 1817 / 382 (32 heads), 54 / 51, 98 / 71,
+        992 / 237 (16); eight of 256 235 / 139; behind 2048 cached tokens 128 tokens 131 / 152, 256 279 / 159 (32), 131 / 127 (16); behind 8192 256
+        827 / 453 (32), 268 / 360 (16)."""
+        if self.rot_dim or self.dim != 128 or self.vdim != 128 or self.kv_rank % 8 or self.w_uv.dtype != torch.bfloat16 or not self.w_uv.is_cuda:
+            return 0
+        k = batch.portions()
+        lens = batch.q_lens[:k]
+        rows, seen = sum(lens), [c + n for c, n in zip(batch.ctx_lens, lens)]
+        keys = sum(seen)
+        if rows < LATENT_EXPAND_ROWS or keys * self.heads * (self.dim + self.vdim) > LATENT_EXPAND_MOST:
+            return 0
+        pairs = sum(n * (min(self.window, s) if self.window else s - n // 2) for n, s in zip(lens, seen))
+        return k if 2 * rows >= keys or self.heads * self.kv_rank * pairs >= LATENT_EXPAND_PAIRS * keys else 0
+
     def attend(self, h: torch.Tensor, cache: torch.Tensor, batch: StepBatch, out: Optional[torch.Tensor] = None,
                rows: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The gated heads [T, heads * vdim], into ``out`` (dense rows, any row stride) if given; ``rows``: of these rows only."""
@@ -503,23 +527,56 @@ class LatentAttention(nn.Module):
         else:
             q = proj.as_strided((T, H, d + P), (proj.stride(0), d + P, 1))
         g_at = self.splits[0] + R + P
-        q_lat = torch.empty(T, H, R, dtype=h.dtype, device=h.device)
-        torch.bmm(q[:, :, :d].transpose(0, 1), self.w_uk, out=q_lat.transpose(0, 1))
-        o_lat = torch.empty(T, H, R, dtype=h.dtype, device=h.device)
-        mops.latent_attention(o_lat, q_lat, q[:, :, d:] if P else None, cache, batch.block_tables, batch.q_start, batch.q_len,
-                              batch.ctx_len, batch.seq_of_token, (min(batch.q_lens), max(batch.q_lens)), rot.inv_freq, rot.mscale,
-                              rot.dims, self.scale, max_kv_len=max(c + n for c, n in zip(batch.ctx_lens, batch.q_lens)),
-                              window=self.window, sink=self.sink, gate=proj[:, g_at:g_at + H] if self.head_gate else None)
-        if rows is not None:
-            o_lat = o_lat.index_select(0, rows)
-        n = o_lat.shape[0]
-        if out is None:
-            out = torch.empty(n, H * e, dtype=h.dtype, device=h.device)
-        torch.bmm(o_lat.transpose(0, 1), self.w_uv, out=out.as_strided((H, n, e), (e, out.stride(0), 1)))
+        gate = proj[:, g_at:g_at + H] if self.head_gate else None
+        k = self.expanded_segments(batch)
+        if k:
+            o = torch.empty(T, H * e, dtype=h.dtype, device=h.device) if out is None or rows is not None else out
+            n = sum(batch.q_lens[:k])
+            self._attend_expanded(o[:n], q[:n], cache, batch, k, n, None if gate is None else gate[:n])
+            if n < T:
+                self._attend_latent(o[n:], q[n:], cache, batch.block_tables[k:], batch.q_start[k:] - n, batch.q_len[k:], batch.ctx_len[k:],
+                                    batch.seq_of_token[n:] - k, batch.q_lens[k:], batch.ctx_lens[k:], None if gate is None else gate[n:])
+            if rows is not None:
+                out = o.index_select(0, rows) if out is None else out.copy_(o.index_select(0, rows))
+            else:
+                out = o
+        else:
+            out = self._attend_latent(out, q, cache, batch.block_tables, batch.q_start, batch.q_len, batch.ctx_len, batch.seq_of_token,
+                                      batch.q_lens, batch.ctx_lens, gate, rows)
         if self.gated and not self.head_gate:
             gate = proj[:, g_at:g_at + H * e]
             mops.sigmoid_gate_mul(out, gate if rows is None else gate.index_select(0, rows), out=out)
         return out
+
+    def _attend_latent(self, out, q, cache, block_tables, q_start, q_len, ctx_len, seq_of_token, q_lens, ctx_lens, gate, rows=None) -> torch.Tensor:
+        """Queries carried into the latent, attention over the cache rows, results carried out."""
+        T, H, d, P, e, R = q.shape[0], self.heads, self.dim, self.rot_dim, self.vdim, self.kv_rank
+        rot = self.rotary
+        q_lat = torch.empty(T, H, R, dtype=q.dtype, device=q.device)
+        torch.bmm(q[:, :, :d].transpose(0, 1), self.w_uk, out=q_lat.transpose(0, 1))
+        o_lat = torch.empty(T, H, R, dtype=q.dtype, device=q.device)
+        mops.latent_attention(o_lat, q_lat, q[:, :, d:] if P else None, cache, block_tables, q_start, q_len, ctx_len, seq_of_token,
+                              (min(q_lens), max(q_lens)), rot.inv_freq, rot.mscale, rot.dims, self.scale,
+                              max_kv_len=max(c + n for c, n in zip(ctx_lens, q_lens)), window=self.window, sink=self.sink, gate=gate)
+        if rows is not None:
+            o_lat = o_lat.index_select(0, rows)
+        n = o_lat.shape[0]
+        if out is None:
+            out = torch.empty(n, H * e, dtype=q.dtype, device=q.device)
+        torch.bmm(o_lat.transpose(0, 1), self.w_uv, out=out.as_strided((H, n, e), (e, out.stride(0), 1)))
+        return out
+
+    def _attend_expanded(self, out, q, cache, batch: StepBatch, k: int, n: int, gate) -> None:
+        """The first ``k`` segments, ``n`` rows: the latents they see times W_uk and W_uv are keys and values of every head."""
+        H, d, e = self.heads, self.dim, self.vdim
+        seen = [c + m for c, m in zip(batch.ctx_lens[:k], batch.q_lens)]
+        c, tables = mops.latent_gather(cache, batch.block_tables[:k], batch.q_len[:k], batch.ctx_len[:k], seen)
+        keys = ops.dense_linear(c, self.w_uk.view(H * d, self.kv_rank)).view(-1, 16, H, d)
+        # (W_uv's rows, copied each time -- 5 us for 4 MB -- so that no second set of weights can fall behind the first)
+        values = ops.dense_linear(c, self.w_uv.transpose(1, 2).reshape(H * e, self.kv_rank)).view(-1, 16, H, e)
+        mops.distance_bias_attention(out, q.as_strided((n, H * d), (q.stride(0), 1)), gate, keys, values, tables, batch.q_start[:k], batch.q_len[:k],
+                                     batch.ctx_len[:k], batch.seq_of_token[:n], (min(batch.q_lens[:k]), max(batch.q_lens[:k])), H, self.scale,
+                                     None, max_kv_len=max(seen), window=self.window, sink=self.sink)
 
     def forward(self, h: torch.Tensor, cache: torch.Tensor, batch: StepBatch) -> torch.Tensor:
         return self.out_proj(self.attend(h, cache, batch))

@@ -96,6 +96,13 @@ class StepBatch:
             out.append(a - 1)
         return out
 
+    def portions(self) -> int:
+        """Number of leading segments that are prompt portions (anything but a single token with a context)."""
+        for s, (n, c) in enumerate(zip(self.q_lens, self.ctx_lens)):
+            if n == 1 and c > 0:
+                return s
+        return len(self.q_lens)
+
     def decode_split(self) -> int:
         """Number of leading segments that are prompt portions when the batch is ordered portions first, single tokens
         with a context last (the order the reference's metadata assumes); raises if it is not."""

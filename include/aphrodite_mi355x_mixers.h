@@ -292,6 +292,12 @@ int aphro_latent_attention_plain(void* out, int64_t out_stride, int64_t out_head
  * query rows of a segment flattened to (token, head) pairs, 64 per workgroup; everything else runs the kernel above.  min/max
  * segment lengths and the longest ctx_len + q_len come from the host.  Decode-sized launches split long key ranges over
  * aphro_latent_attention_splits(...) workgroups when `workspace` holds num_tokens * heads * splits * (2 + kv_rank) floats. */
+/* The cache rows (dim numbers, bf16) that the first num_seqs segments see, ctx_len + q_len of them each, one segment after the other from
+ * multiples of 16 rows on (padding repeats a segment's last row); tables [num_seqs, out_blocks] takes their numbers as blocks of 16 rows, so
+ * that `rows` -- or products of it -- can be read as a paged cache.  total_rows: the padded lengths' sum. */
+int aphro_latent_gather(void* rows, int64_t total_rows, int32_t* tables, int out_blocks, const void* cache, const int32_t* block_tables,
+                        int max_blocks, int64_t num_blocks, int block_size, const int32_t* q_len, const int32_t* ctx_len, int num_seqs,
+                        int dim, int dtype, void* stream);
 int aphro_latent_attention_fast_supported(int kv_rank, int rot_dim, int rot_dims, int dtype);
 int aphro_latent_attention_splits(int64_t num_tokens, int num_seqs, int max_q_len, int heads, int max_kv_len);
 int aphro_latent_attention(void* out, int64_t out_stride, int64_t out_head_stride, const void* q_lat, int64_t ql_stride,
