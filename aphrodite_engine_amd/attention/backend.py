@@ -200,7 +200,7 @@ class MI355XAttentionImpl:
 
         num_prefill_tokens = attn_metadata.num_prefill_tokens
         num_decode_tokens = attn_metadata.num_decode_tokens
-        output = torch.empty_like(query)
+        output = torch.empty((num_tokens, self.num_heads, self.head_size), dtype=query.dtype, device=query.device)
         decode_query = query[num_prefill_tokens:]
         query = query[:num_prefill_tokens]
         key = key[:num_prefill_tokens]
@@ -219,20 +219,19 @@ class MI355XAttentionImpl:
             if has_ctx:
                 # prefix-enabled attention (rocm_flash_attn.py:509-527)
                 assert key_cache is not None
-                output[:num_prefill_tokens] = PagedAttention.forward_prefix(
+                PagedAttention.forward_prefix(
                     query, key, value, self.kv_cache_dtype, key_cache, value_cache,
                     prefill_meta.block_tables, prefill_meta.query_start_loc,
                     prefill_meta.seq_lens_tensor, prefill_meta.context_lens_tensor,
                     prefill_meta.max_query_len, self.alibi_slopes, self.sliding_window[0],
                     k_scale, v_scale,
                     # host-side maxima of the prefill sequences (seq_lens is a Python list): no .item() per layer
-                    max_seq_len=max(prefill_meta.seq_lens), total_kv_tokens=sum(prefill_meta.seq_lens))
+                    max_seq_len=max(prefill_meta.seq_lens), total_kv_tokens=sum(prefill_meta.seq_lens), output=output[:num_prefill_tokens])
             else:
-                out = ops.flash_attn_varlen(
+                ops.flash_attn_varlen(
                     query, key, value, prefill_meta.seq_start_loc,
                     prefill_meta.max_prefill_seq_len, self.scale, causal=True,
-                    alibi_slopes=self.alibi_slopes, window_size=self.sliding_window)
-                output[:num_prefill_tokens] = out
+                    alibi_slopes=self.alibi_slopes, window_size=self.sliding_window, out=output[:num_prefill_tokens])
 
         if decode_meta := attn_metadata.decode_metadata:
             assert key_cache is not None

@@ -80,11 +80,12 @@ class PagedAttention:
                        block_tables, query_start_loc, seq_lens_tensor, context_lens,
                        max_query_len: int, alibi_slopes, sliding_window, k_scale: float,
                        v_scale: float, max_seq_len: Optional[int] = None,
-                       total_kv_tokens: Optional[int] = None) -> torch.Tensor:
+                       total_kv_tokens: Optional[int] = None, output: Optional[torch.Tensor] = None) -> torch.Tensor:
         """ops/paged_attn.py:192-231.  ``max_seq_len`` / ``total_kv_tokens``: host-side max / sum of the prefill
         sequences' lengths (the metadata holds them as a Python list): with them the long-prompt path of
         context_attention_fwd needs no device-to-host sync."""
-        output = torch.empty_like(query)
+        if output is None:
+            output = torch.empty_like(query)
         ops.context_attention_fwd(query, key, value, output, kv_cache_dtype, key_cache,
                                   value_cache, block_tables, query_start_loc, seq_lens_tensor,
                                   context_lens, max_query_len, k_scale, v_scale, alibi_slopes,

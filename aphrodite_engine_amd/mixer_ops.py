@@ -15,8 +15,11 @@ ACT_SILU, ACT_GELU_TANH = 0, 1
 MEMORY_DECAY, MEMORY_MLSTM, MEMORY_STATE_SPACE = 0, 1, 2
 
 
+_raw_stream, _current_device = torch._C._cuda_getCurrentRawStream, torch.cuda.current_device
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
 
 
 def _dt(t: torch.Tensor) -> int:
@@ -31,19 +34,23 @@ def _need(cond: bool, msg: str) -> None:
 
 
 def _cuda(*ts) -> None:
-    dev = None
+    dev = -1
     for t in ts:
         if t is None:
             continue
         if not t.is_cuda:
             raise RuntimeError("mixer ops run on the GPU only (no CPU fallback)")
-        dev = dev or t.device
-        _need(t.device == dev, "mixer ops: tensors on different devices")
+        at = t.get_device()
+        if dev < 0:
+            dev = at
+        elif at != dev:
+            raise RuntimeError("mixer ops: tensors on different devices")
 
 
 def _rows(t: torch.Tensor, cols: int, what: str) -> int:
     """Row stride (elements) of a [T, cols] view whose rows are dense."""
-    _need(t.dim() == 2 and t.shape[1] == cols and (t.stride(1) == 1 or cols == 1), f"{what}: expected dense rows of {cols}")
+    if t.dim() != 2 or t.shape[1] != cols or not (t.stride(1) == 1 or cols == 1):
+        raise RuntimeError(f"{what}: expected dense rows of {cols}")
     return t.stride(0) if t.shape[0] > 1 else max(t.stride(0), cols)
 
 
@@ -52,7 +59,8 @@ def _p(t: Optional[torch.Tensor]):
 
 
 def _i32(t: torch.Tensor, n: int, what: str) -> None:
-    _need(t.dtype == torch.int32 and t.is_contiguous() and t.numel() == n, f"{what}: int32 [{n}] expected")
+    if t.dtype != torch.int32 or not t.is_contiguous() or t.numel() != n:
+        raise RuntimeError(f"{what}: int32 [{n}] expected")
 
 
 def embed_scale(table: torch.Tensor, ids: torch.Tensor, scale: float, out: Optional[torch.Tensor] = None,
@@ -680,7 +688,8 @@ def latent_gather(cache: torch.Tensor, block_tables: torch.Tensor, q_len: torch.
 
 def _head_view(t: torch.Tensor, T: int, heads: int, n: int, what: str):
     """(token stride, head stride) of a [T, heads, n] view whose last axis is dense."""
-    _need(t.dim() == 3 and tuple(t.shape) == (T, heads, n) and (t.stride(2) == 1 or n == 1), f"{what}: [T, heads, {n}] with a dense last axis")
+    if t.dim() != 3 or tuple(t.shape) != (T, heads, n) or not (t.stride(2) == 1 or n == 1):
+        raise RuntimeError(f"{what}: [T, heads, {n}] with a dense last axis")
     return t.stride(0), t.stride(1)
 
 

@@ -10,22 +10,24 @@ import numpy as np
 import torch
 
 
-def _to_device(arrays: List[np.ndarray], device, wait: bool) -> List[torch.Tensor]:
-    """The arrays on the device, as parts (16-byte aligned) of one buffer that one copy from pinned memory fills: a copy per array from
-    pageable memory is ten round trips that wait for everything the stream still has to do."""
-    device = torch.device(device)
+def _to_device(longs: List[np.ndarray], ints: List[np.ndarray], device, wait: bool) -> List[torch.Tensor]:
+    """The int64 and int32 arrays (flat) on the device, as parts (16-byte aligned) of one buffer that one copy from pinned memory fills: a copy
+    per array from pageable memory is ten round trips that wait for everything the stream still has to do."""
     if device.type == "cpu":
-        return [torch.from_numpy(np.ascontiguousarray(a)) for a in arrays]
-    at = np.cumsum([0] + [(a.nbytes + 15) // 16 * 16 for a in arrays]).tolist()
-    host = torch.empty(max(16, at[-1]), dtype=torch.uint8, pin_memory=True)
+        return [torch.from_numpy(a) for a in longs + ints]
+    sizes = [[x for a in part for x in (a.size, -a.size % unit)] for part, unit in ((longs, 2), (ints, 4))]
+    split = sum(sizes[0])
+    host = torch.empty(2 * split + sum(sizes[1]), dtype=torch.int32, pin_memory=True)
     image = host.numpy()
-    for a, i in zip(arrays, at):
-        image[i:i + a.nbytes] = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
+    for part, into in ((longs, image[:2 * split].view(np.int64)), (ints, image[2 * split:])):
+        at = 0
+        for a in part:
+            into[at:at + a.size] = a
+            at += a.size + -a.size % (16 // a.itemsize)
     buf = host.to(device, non_blocking=True)
     if wait:
         torch.cuda.current_stream(device).synchronize()
-    kinds = {np.dtype(np.int64): torch.int64, np.dtype(np.int32): torch.int32}
-    return [buf[i:i + a.nbytes].view(kinds[a.dtype]).view(a.shape) for a, i in zip(arrays, at)]
+    return list(buf[:2 * split].view(torch.int64).split_with_sizes(sizes[0])[::2]) + list(buf[2 * split:].split_with_sizes(sizes[1])[::2])
 
 
 @dataclass
@@ -61,31 +63,40 @@ class StepBatch:
             raise ValueError("a step batch needs at least one segment and no empty one")
         if min(len(ctx_lens), len(block_tables)) < S:
             raise ValueError(f"{S} segments, but {len(ctx_lens)} contexts and {len(block_tables)} page lists")
-        n, c = np.asarray(q_lens, np.int64), np.asarray([int(x) for x in ctx_lens[:S]], np.int64)
-        pages = np.asarray([len(b) for b in block_tables[:S]], np.int64)
-        need = (c + n + block_size - 1) // block_size
-        for s in np.nonzero(pages < need)[0]:
-            raise ValueError(f"segment {s}: {pages[s]} pages for {c[s] + n[s]} tokens")
+        ctx = [int(x) for x in ctx_lens[:S]]
+        held = [len(b) for b in block_tables[:S]]
+        for s in range(S):
+            if held[s] * block_size < ctx[s] + q_lens[s]:
+                raise ValueError(f"segment {s}: {held[s]} pages for {ctx[s] + q_lens[s]} tokens")
         if len(set(int(x) for x in state_slots)) != S:
             raise ValueError("two segments of one step share a state slot")
+        n, c, i32 = np.array(q_lens, np.int64), np.array(ctx, np.int64), np.int32
         T = int(n.sum())
-        starts = np.cumsum(n) - n
-        bt = np.zeros((S, max(1, int(pages.max()))), np.int32)
-        for s, b in enumerate(block_tables[:S]):
-            bt[s, :len(b)] = b
-        seq_of = np.repeat(np.arange(S), n)
-        pos = np.arange(T) - np.repeat(starts - c, n)
-        slots = bt[seq_of, pos // block_size].astype(np.int64) * block_size + pos % block_size
-        ids = np.concatenate([np.asarray(t, np.int64) for t in tokens])
+        ends = np.cumsum(n)
+        starts = ends - n
+        wide = max(1, max(held))
+        bt = np.array([list(b) + [0] * (wide - len(b)) for b in block_tables[:S]], i32)
+        if T == S:                                           # (decoded tokens: no segment to lay out)
+            seq_of, pos, ids = np.arange(S, dtype=i32), c, np.array([t[0] for t in tokens], np.int64)
+        else:
+            seq_of = np.repeat(np.arange(S, dtype=i32), n)
+            pos = np.arange(T) - (starts - c)[seq_of]
+            ids = np.empty(T, np.int64)
+            for t, a, z in zip(tokens, starts.tolist(), ends.tolist()):
+                ids[a:z] = t
+        page = pos // block_size
+        slots = bt[seq_of, page].astype(np.int64) * block_size + (pos - page * block_size)
         # prompt portions lead (decode_split checks that): their rows and lengths, summed up
-        seq_lens, i32 = c + n, np.int32
-        k = next((s for s in range(S) if q_lens[s] == 1 and c[s] > 0), S)
-        loc, sloc = (np.concatenate([[0], np.cumsum(x[:k])]).astype(i32) for x in (n, seq_lens))
-        d = _to_device([ids, pos, slots, np.asarray([] if rows is None else rows, np.int64), starts.astype(i32), n.astype(i32), c.astype(i32),
-                        seq_of.astype(i32), bt, np.asarray(state_slots, i32), seq_lens.astype(i32), loc, sloc], device, wait)
+        seq_lens = c + n
+        k = next((s for s in range(S) if q_lens[s] == 1 and ctx[s] > 0), S)
+        loc = np.zeros((2, k + 1), i32)
+        loc[0, 1:], loc[1, 1:] = ends[:k], np.cumsum(seq_lens[:k])
+        wanted = np.array([] if rows is None else rows, np.int64)
+        d = _to_device([ids, pos, slots, wanted], [starts.astype(i32), n.astype(i32), c.astype(i32), seq_of, bt.reshape(-1),
+                                                   np.array(state_slots, i32).reshape(-1), seq_lens.astype(i32), loc[0], loc[1]], torch.device(device), wait)
         return StepBatch(num_tokens=T, num_seqs=S, input_ids=d[0], positions=d[1], q_start=d[4], q_len=d[5], ctx_len=d[6],
-                         seq_of_token=d[7], block_tables=d[8], slot_mapping=d[2], state_slots=d[9], block_size=block_size, q_lens=q_lens,
-                         ctx_lens=[int(x) for x in c], rows=None if rows is None else d[3], seq_lens_tensor=d[10], query_start_loc=d[11],
+                         seq_of_token=d[7], block_tables=d[8].view(S, wide), slot_mapping=d[2], state_slots=d[9], block_size=block_size,
+                         q_lens=q_lens, ctx_lens=ctx, rows=None if rows is None else d[3], seq_lens_tensor=d[10], query_start_loc=d[11],
                          seq_start_loc=d[12])
 
     def last_rows(self) -> List[int]:
