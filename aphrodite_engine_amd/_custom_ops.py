@@ -2173,7 +2173,10 @@ def cutlass_scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor,
         raise RuntimeError("b must be column-major [K,N] (weight.t())")
     if not a.is_contiguous():
         a = a.contiguous()
-    if m > SCALED_MM_LIBRARY_MIN_M and n % 128 == 0 and k % 128 == 0 and not switch("APHRO_FP8_NO_LARGE"):
+    # 65 to 192 rows in one pass of the weight-stream kernel where that is the faster one
+    rows = m > SCALED_MM_LIBRARY_MIN_M and not switch("APHRO_FP8_NO_LARGE") and (out is None or out.data_ptr() % 8 == 0) \
+        and bool(_lib.lib().aphro_fp8_gemm_rows_preferred(m, n, k))
+    if m > SCALED_MM_LIBRARY_MIN_M and not rows and n % 128 == 0 and k % 128 == 0 and not switch("APHRO_FP8_NO_LARGE"):
         # prefill-sized M: the MFMA-bound kernel of fp8_gemm_large.hip (scales + bias in its epilogue, f16 or bf16)
         lib = _lib.lib()
         if out is None:
@@ -2190,7 +2193,7 @@ def cutlass_scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor,
             ws.data_ptr(), ws.numel(), m, n, k, 1 if sa.numel() > 1 else 0, 1 if sb.numel() > 1 else 0,
             _lib.F16 if out_dtype == torch.float16 else _lib.BF16, _stream()), "cutlass_scaled_mm")
         return out
-    if m > SCALED_MM_LIBRARY_MIN_M:
+    if m > SCALED_MM_LIBRARY_MIN_M and not rows:
         # shapes the hand-written kernel does not tile (N or K not a multiple of 128): library GEMM: a plain library GEMM (hipBLASLt through torch._scaled_mm --
         # what the reference itself calls on ROCm, w8a8_utils.py:130,165; measured 1.9 PFLOP/s fp8 at
         # M = 8192).  Row-wise scaling needs both scale vectors; a scalar one is broadcast.
@@ -2232,9 +2235,10 @@ def cutlass_scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor,
     sb = scale_b.reshape(-1).float()
     a_tok = 1 if sa.numel() > 1 else 0
     b_ch = 1 if sb.numel() > 1 else 0
-    ws = _workspace(a.device, lib.aphro_fp8_gemm_workspace_bytes(min(m, 64), n, k))
-    for m0 in range(0, m, 64):
-        rows = min(64, m - m0)
+    most = m if rows else 64
+    ws = _workspace(a.device, lib.aphro_fp8_gemm_workspace_bytes(min(m, most), n, k))
+    for m0 in range(0, m, most):
+        rows = min(most, m - m0)
         sa_blk = sa[m0:] if a_tok else sa
         check(lib.aphro_scaled_mm_fp8(
             out[m0:].data_ptr(), a[m0:].data_ptr(), b.data_ptr(),

@@ -409,6 +409,10 @@ static int fp8_gemm_common(Fp8GemmParams p, bool a8, int dtype, void* workspace,
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "fp8 gemm: output dtype must be f16 or bf16");
   APHRO_CHECK(p.K % 128 == 0, "fp8 gemm: K=%d must be a multiple of 128", p.K);
   APHRO_CHECK(p.N % 16 == 0, "fp8 gemm: N=%d must be a multiple of 16", p.N);
+  // W8A8 from 33 rows on: one pass over the weight (fp8_gemm_rows.hip)
+  if (a8 && p.lda == p.K && aphro_fp8_gemm_rows_ksplit(p.M, p.N, p.K) > 0 && ((uintptr_t)p.c % 8) == 0 && ((uintptr_t)workspace % 16) == 0)
+    return aphro_fp8_gemm_rows(p.a, p.w, p.a_scales, p.b_scales, p.bias, p.force_partial ? nullptr : p.c, (float*)workspace, workspace_bytes,
+                               p.M, p.N, p.K, p.a_per_token, p.b_per_channel, dtype, (void*)st);
   APHRO_CHECK(p.M <= 64, "fp8 gemm: M=%d exceeds 64 rows per call", p.M);
   if (p.M == 0) return APHRO_OK;
   // W8A8 at <= 32 rows: the LDS-DMA streaming kernel (fp8_gemm_stream.hip) where it tiles the shape -- directly to `c` when
@@ -448,9 +452,9 @@ static int fp8_gemm_common(Fp8GemmParams p, bool a8, int dtype, void* workspace,
 using namespace aphro;
 
 extern "C" size_t aphro_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  (void)K;
-  int64_t m = M < 64 ? M : 64;
-  return (size_t)8 * m * N * sizeof(float);
+  const int64_t m = M < 64 ? M : 64;
+  const size_t few = (size_t)8 * m * N * sizeof(float), rows = (size_t)aphro_fp8_gemm_rows_ksplit(M, N, K) * M * N * sizeof(float);
+  return rows > few ? rows : few;
 }
 
 extern "C" int aphro_scaled_mm_fp8(void* out, const void* a, const void* b, const float* a_scales,
@@ -470,6 +474,7 @@ extern "C" int aphro_scaled_mm_fp8(void* out, const void* a, const void* b, cons
 // consumer (aphro_fused_add_rms_norm_quant_fp8, the rotary/attention kernel) which sums them and
 // applies a_scale * (b_scale * acc) itself -- no reduce launch, no fp16 round trip.
 extern "C" int aphro_fp8_gemm_ksplit(int64_t M, int64_t N, int64_t K) {
+  if (const int rows = aphro_fp8_gemm_rows_ksplit(M, N, K); rows > 0) return rows;      // (what fp8_gemm_common will run)
   if (M <= 0 || M > 64 || K % 128 != 0 || N % 16 != 0) return -1;
   const int split = aphro_fp8_gemm_stream_ksplit(M, N, K);     // (what fp8_gemm_common will run)
   if (split > 0) return split;

@@ -149,16 +149,18 @@ void cutlass_scaled_mm(torch::Tensor out, torch::Tensor a, torch::Tensor b, torc
   const int odt = act_dtype(out);
   const void* bp = bias ? bias->data_ptr() : nullptr;
   const int a_tok = a_scales.numel() > 1, b_ch = b_scales.numel() > 1;
-  if (m > 64 && n % 128 == 0 && k % 128 == 0) {         // prefill-sized: the MFMA-bound stream-K kernel
+  const bool few = m > 64 && ((uintptr_t)out.data_ptr() % 8) == 0 && aphro_fp8_gemm_rows_preferred(m, n, k);      // one pass of the weight-stream kernel
+  if (m > 64 && !few && n % 128 == 0 && k % 128 == 0) {         // prefill-sized: the MFMA-bound stream-K kernel
     auto ws = torch::empty({(int64_t)aphro_scaled_mm_fp8_large_workspace_bytes(m, n, k)}, a.options().dtype(torch::kUInt8));
     ok(aphro_scaled_mm_fp8_large(out.data_ptr(), a.data_ptr(), b.data_ptr(), a_scales.data_ptr<float>(), b_scales.data_ptr<float>(),
                                  bp, ws.data_ptr(), (size_t)ws.numel(), m, n, k, a_tok, b_ch, odt, cur_stream()),
        "cutlass_scaled_mm");
     return;
   }
-  auto ws = torch::empty({(int64_t)aphro_fp8_gemm_workspace_bytes(m < 64 ? m : 64, n, k)}, a.options().dtype(torch::kUInt8));
-  for (int64_t m0 = 0; m0 < m; m0 += 64) {
-    const int64_t rows = m - m0 < 64 ? m - m0 : 64;
+  const int64_t most = few ? m : 64;
+  auto ws = torch::empty({(int64_t)aphro_fp8_gemm_workspace_bytes(m < most ? m : most, n, k)}, a.options().dtype(torch::kUInt8));
+  for (int64_t m0 = 0; m0 < m; m0 += most) {
+    const int64_t rows = m - m0 < most ? m - m0 : most;
     ok(aphro_scaled_mm_fp8((char*)out.data_ptr() + m0 * n * out.element_size(), (const char*)a.data_ptr() + m0 * k, b.data_ptr(),
                            a_scales.data_ptr<float>() + (a_tok ? m0 : 0), b_scales.data_ptr<float>(), bp, ws.data_ptr(),
                            (size_t)ws.numel(), rows, n, k, a_tok, b_ch, odt, cur_stream()),

@@ -672,7 +672,7 @@ class LlamaDecoderLayer(nn.Module):
         inside the attention kernel.  The activation scheme -- dynamic per token, or the checkpoint's
         static per-tensor input_scale -- must be the same for the four projections of the layer."""
         from .quantization.fp8 import CompressedTensorsW8A8Fp8Method, CDNA4Fp8LinearMethod
-        if m > 64 or self.head_dim != 128 or not self.fuse_rope_attention or self.is_moe or self.has_bias:
+        if m > 192 or self.head_dim != 128 or not self.fuse_rope_attention or self.is_moe or self.has_bias:
             return False
         lins = self.linears()
         static = [getattr(lin, "input_scale", None) is not None for lin in lins]
@@ -1043,9 +1043,8 @@ class LlamaForCausalLM(nn.Module):
                 _, _, out = ops.fused_add_rms_norm_quant_fp8(None, prev[0], prev[1], prev[2], residual, True,
                                                              self.norm, self.cfg.rms_norm_eps, want_out=True)
             return out
-        if (attn_metadata.num_prefill_tokens > 0 and attn_metadata.num_decode_tokens == 0 and hidden.shape[0] > 64
-                and all(l.fused_prefill_fp8_ok() for l in self.layers)):
-            # prompt-sized FP8 W8A8 batches: norm + quant and SiluAndMul + quant fused (forward_prefill_fp8)
+        if hidden.shape[0] > 64 and all(l.fused_prefill_fp8_ok() for l in self.layers):
+            # FP8 W8A8 batches of prompts, or of more decoded rows than the fused decode step takes: norm + quant and SiluAndMul + quant fused (forward_prefill_fp8)
             residual = torch.empty_like(hidden)
             for i, layer in enumerate(self.layers):
                 hidden = layer.forward_prefill_fp8(positions, hidden, residual, i == 0, kv_caches[i], attn_metadata,

@@ -983,6 +983,15 @@ int64_t aphro_dense_rows_slab_floats(int64_t M, int64_t N, int64_t K, int64_t ld
 int aphro_dense_rows(void* out, int64_t ldo, const void* x, int64_t lda, const void* weight, int64_t ldw, const void* bias, float* slabs,
                      int64_t slab_floats, int64_t M, int64_t N, int64_t K, int act, int out_f32, int dtype, void* stream);
 
+/* FP8 W8A8 product of 33 to 192 rows (same arithmetic as aphro_scaled_mm_fp8[_slabs], which route to it by themselves): out [M, N] in `dtype`, or,
+ * out == NULL, raw fp32 slabs [ksplit][M][N].  aphro_fp8_gemm_rows_ksplit: K slices, 0 = not served; with more than one, slabs of
+ * ksplit * M * N floats are needed either way. */
+int aphro_fp8_gemm_rows_ksplit(int64_t M, int64_t N, int64_t K);
+int aphro_fp8_gemm_rows_preferred(int64_t M, int64_t N, int64_t K);   /* M > 64: rather than aphro_scaled_mm_fp8_large */
+int aphro_fp8_gemm_rows(const void* a, const void* w, const float* a_scales, const float* b_scales, const void* bias, void* out, float* slabs,
+                        size_t slabs_bytes, int64_t M, int64_t N, int64_t K, int a_scale_per_token, int b_scale_per_channel, int dtype,
+                        void* stream);
+
 /* Greedy sampling: out[r] = argmax_c x[r][c] (lowest index on ties) -- the torch.argmax of
  * modeling/layers/sampler.py:_greedy_sample as one pass over each logits row. */
 int aphro_argmax_rows(int64_t* out, const void* x, int64_t rows, int64_t cols,

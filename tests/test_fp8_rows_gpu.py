@@ -1,0 +1,45 @@
+"""The FP8 product of 33 to 192 rows: its row and column tiles and their remainders, K in one piece and split, scalar and vector scales,
+bias; raw slabs add up to the same bits.  Operands are eighths up to 15 / 8: their products' sums fit fp32 without a rounding, so that results
+are compared bit by bit."""
+import pytest
+import torch
+
+from aphrodite_engine_amd import _custom_ops as ops
+from aphrodite_engine_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(33, 16, 128), (48, 6144, 4096), (49, 4096, 14336), (64, 28672, 512), (65, 1040, 2048), (96, 10304, 1024), (97, 4096, 4096),
+          (128, 20496, 256), (150, 6144, 4096), (160, 4096, 14336), (161, 28672, 384), (192, 528, 8192), (192, 65552, 128)]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("vector", [False, True])
+def test_rows(m, n, k, dtype, vector):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = (torch.randint(-15, 16, (m, k), generator=g, device="cuda") / 8).to(torch.float8_e4m3fn)
+    w = (torch.randint(-15, 16, (n, k), generator=g, device="cuda") / 8).to(torch.float8_e4m3fn)
+    sa = torch.rand(m if vector else 1, 1, generator=g, device="cuda") * 0.02 + 0.01
+    sb = torch.rand(n if vector else 1, generator=g, device="cuda") * 0.02 + 0.01
+    bias = torch.randn(n, generator=g, device="cuda").to(dtype) if vector else None
+    assert ops.fp8_gemm_ksplit(m, n, k) == _lib.lib().aphro_fp8_gemm_rows_ksplit(m, n, k) > 0
+    got = torch.empty(m, n, dtype=dtype, device="cuda")
+    split = ops.fp8_gemm_ksplit(m, n, k)
+    ws = torch.empty(split * m * n, dtype=torch.float32, device="cuda")
+    rc = _lib.lib().aphro_scaled_mm_fp8(got.data_ptr(), a.data_ptr(), w.data_ptr(), sa.data_ptr(), sb.data_ptr(), None if bias is None else bias.data_ptr(),
+                                        ws.data_ptr(), ws.numel() * 4, m, n, k, int(vector), int(vector), _lib.F16 if dtype == torch.float16 else _lib.BF16,
+                                        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    exact = (a.double() @ w.double().t()).float()
+    scaled = sa * (sb * exact)
+    want = (scaled if bias is None else scaled + bias.float()).to(dtype)
+    assert torch.equal(got, want)
+    slabs = ops.scaled_mm_fp8_slabs(a, w.t())
+    assert slabs.shape == (split, m, n) and torch.equal(slabs.sum(0), exact)
+    assert torch.equal(got, ops.cutlass_scaled_mm(a, w.t(), sa, sb, dtype, bias)) or not (m <= 64 or _lib.lib().aphro_fp8_gemm_rows_preferred(m, n, k))
+
+
+def test_not_served():
+    for m, n, k in ((32, 4096, 4096), (193, 4096, 4096), (64, 4096, 4032), (64, 4104, 4096)):
+        assert _lib.lib().aphro_fp8_gemm_rows_ksplit(m, n, k) == 0
