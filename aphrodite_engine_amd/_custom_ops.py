@@ -1246,8 +1246,9 @@ def rope_cache(qkv: Optional[torch.Tensor], slabs: Optional[torch.Tensor], posit
                cos_sin_cache: torch.Tensor, is_neox: bool, key_cache: torch.Tensor,
                value_cache: torch.Tensor, slot_mapping: torch.Tensor, num_heads: int,
                num_kv_heads: int, head_size: int, kv_cache_dtype: str, k_scale: float,
-               v_scale: float) -> torch.Tensor:
-    """[slab reduce] + rotary_embedding(q, k) + reshape_and_cache(k, v); returns q [T, Hq*hd]."""
+               v_scale: float, row_scale: Optional[torch.Tensor] = None, col_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """[slab reduce] + rotary_embedding(q, k) + reshape_and_cache(k, v); returns q [T, Hq*hd].  ``row_scale`` [T] or None, ``col_scale``
+    [columns], fp32: the slabs are an FP8 projection's raw sums."""
     lib = _lib.lib()
     if slabs is not None:
         nslab, tokens, _ = slabs.shape
@@ -1259,7 +1260,7 @@ def rope_cache(qkv: Optional[torch.Tensor], slabs: Optional[torch.Tensor], posit
     q_out = torch.empty((tokens, num_heads * head_size), dtype=dtype, device=dev)
     if positions is not None and positions.dtype != torch.int64:
         positions = positions.long()
-    check(lib.aphro_rope_cache(_ptr(qkv), stride, _ptr(slabs), nslab, _ptr(positions),
+    check(lib.aphro_rope_cache_scaled(_ptr(qkv), stride, _ptr(slabs), nslab, _ptr(row_scale), _ptr(col_scale), _ptr(positions),
                                cos_sin_cache.data_ptr(), cos_sin_cache.shape[1], 1 if is_neox else 0,
                                q_out.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
                                slot_mapping.data_ptr(), tokens, num_heads, num_kv_heads, head_size,

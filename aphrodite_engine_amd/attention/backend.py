@@ -235,23 +235,29 @@ class MI355XAttentionImpl:
 
         if decode_meta := attn_metadata.decode_metadata:
             assert key_cache is not None
-            num_seqs = decode_query.shape[0]
-            block_size = value_cache.shape[3]
-            max_seq_len = decode_meta.max_decode_seq_len
-            max_num_partitions = ((max_seq_len + _PARTITION_SIZE_ROCM - 1)
-                                  // _PARTITION_SIZE_ROCM)
-            tmp_output = torch.empty(
-                size=(num_seqs, self.num_heads, max_num_partitions, self.head_size),
-                dtype=output.dtype, device=output.device)
-            exp_sums = torch.empty(size=(num_seqs, self.num_heads, max_num_partitions),
-                                   dtype=torch.float32, device=output.device)
-            max_logits = torch.empty_like(exp_sums)
-            ops.paged_attention_rocm(
-                output[num_prefill_tokens:], exp_sums, max_logits, tmp_output,
-                decode_query, key_cache, value_cache, self.num_kv_heads, self.scale,
-                decode_meta.block_tables, decode_meta.seq_lens_tensor, block_size,
-                max_seq_len, self.alibi_slopes, self.kv_cache_dtype, k_scale, v_scale)
+            self.decode(decode_query, key_cache, value_cache, decode_meta, k_scale, v_scale, output[num_prefill_tokens:])
         return output.view(num_tokens, hidden_size)
+
+    def decode(self, query: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, decode_meta: MI355XAttentionMetadata,
+               k_scale: float, v_scale: float, output: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """One query row [S, Hq, hd] a sequence over the paged cache, into ``output`` (contiguous) if given."""
+        if output is None:
+            output = torch.empty(query.shape, dtype=query.dtype, device=query.device)
+        num_seqs, max_seq_len = query.shape[0], decode_meta.max_decode_seq_len
+        max_num_partitions = ((max_seq_len + _PARTITION_SIZE_ROCM - 1)
+                              // _PARTITION_SIZE_ROCM)
+        tmp_output = torch.empty(
+            size=(num_seqs, self.num_heads, max_num_partitions, self.head_size),
+            dtype=output.dtype, device=output.device)
+        exp_sums = torch.empty(size=(num_seqs, self.num_heads, max_num_partitions),
+                               dtype=torch.float32, device=output.device)
+        max_logits = torch.empty_like(exp_sums)
+        ops.paged_attention_rocm(
+            output, exp_sums, max_logits, tmp_output,
+            query, key_cache, value_cache, self.num_kv_heads, self.scale,
+            decode_meta.block_tables, decode_meta.seq_lens_tensor, value_cache.shape[3],
+            max_seq_len, self.alibi_slopes, self.kv_cache_dtype, k_scale, v_scale)
+        return output
 
 
 # ---------------------------------------------------------------------------------------------------------------------

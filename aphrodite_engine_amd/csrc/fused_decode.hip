@@ -310,7 +310,7 @@ __global__ void rope_cache_kernel(const uint16_t* __restrict__ qkv, int64_t qkv_
                                   int rot_dim, uint16_t* __restrict__ q_out, void* __restrict__ key_cache,
                                   void* __restrict__ value_cache, const int64_t* __restrict__ slot_mapping,
                                   int num_heads, int num_kv_heads, int head_size, int block_size, int x,
-                                  float k_scale, float v_scale) {
+                                  float k_scale, float v_scale, const float* __restrict__ row_scale, const float* __restrict__ col_scale) {
   const int tok = blockIdx.x;
   const int nq = num_heads * head_size, nkv = num_kv_heads * head_size;
   const int ntot = nq + 2 * nkv;
@@ -319,7 +319,8 @@ __global__ void rope_cache_kernel(const uint16_t* __restrict__ qkv, int64_t qkv_
     if (slabs) {
       float s = slabs[(size_t)tok * ntot + j];
       for (int k = 1; k < nslab; ++k) s += slabs[k * slab_stride + (size_t)tok * ntot + j];
-      return T::to_f32(T::from_f32(s));
+      if (col_scale) s = (row_scale ? row_scale[tok] : 1.f) * (col_scale[j] * s);
+      return T::to_f32(from_f32_exact<T>(s));
     }
     return T::to_f32(qkv[(size_t)tok * qkv_stride + j]);
   };
@@ -384,7 +385,8 @@ __global__ void rope_cache_vec_kernel(const uint16_t* __restrict__ qkv, int64_t 
                                       uint16_t* __restrict__ q_out, void* __restrict__ key_cache,
                                       void* __restrict__ value_cache, const int64_t* __restrict__ slot_mapping,
                                       int num_heads, int num_kv_heads, int head_size, int block_size, int x,
-                                      float k_scale, float v_scale) {
+                                      float k_scale, float v_scale, const float* __restrict__ row_scale,
+                                      const float* __restrict__ col_scale) {
   const int tok = blockIdx.x;
   const int nq = num_heads * head_size, nkv = num_kv_heads * head_size;
   const int ntot = nq + 2 * nkv;
@@ -393,14 +395,23 @@ __global__ void rope_cache_vec_kernel(const uint16_t* __restrict__ qkv, int64_t 
     if (slabs) {
       const float* p0 = slabs + (size_t)tok * ntot + j;
       f32x4 a = *reinterpret_cast<const f32x4*>(p0), b = *reinterpret_cast<const f32x4*>(p0 + 4);
+#pragma unroll 4
       for (int k = 1; k < nslab; ++k) {
         a += *reinterpret_cast<const f32x4*>(p0 + k * slab_stride);
         b += *reinterpret_cast<const f32x4*>(p0 + k * slab_stride + 4);
       }
+      if (col_scale) {                                     // an FP8 projection's raw sums
+        const float rs = row_scale ? row_scale[tok] : 1.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          a[i] = rs * (col_scale[j + i] * a[i]);
+          b[i] = rs * (col_scale[j + 4 + i] * b[i]);
+        }
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        o[i] = T::to_f32(T::from_f32(a[i]));
-        o[4 + i] = T::to_f32(T::from_f32(b[i]));
+        o[i] = T::to_f32(from_f32_exact<T>(a[i]));
+        o[4 + i] = T::to_f32(from_f32_exact<T>(b[i]));
       }
     } else {
       u16x8 v = *reinterpret_cast<const u16x8*>(qkv + (size_t)tok * qkv_stride + j);
@@ -597,14 +608,15 @@ extern "C" int aphro_silu_and_mul_pack_slabs(const float* slabs, int nslab, void
   return APHRO_OK;
 }
 
-extern "C" int aphro_rope_cache(const void* qkv, int64_t qkv_stride, const float* slabs, int nslab,
-                                const int64_t* positions, const void* cos_sin_cache, int rot_dim, int is_neox,
-                                void* q_out, void* key_cache, void* value_cache, const int64_t* slot_mapping,
-                                int64_t tokens, int num_heads, int num_kv_heads, int head_size, int block_size,
-                                int x, int dtype, int kv_dtype, float k_scale, float v_scale, void* stream) {
+extern "C" int aphro_rope_cache_scaled(const void* qkv, int64_t qkv_stride, const float* slabs, int nslab, const float* row_scale,
+                                       const float* col_scale, const int64_t* positions, const void* cos_sin_cache, int rot_dim,
+                                       int is_neox, void* q_out, void* key_cache, void* value_cache, const int64_t* slot_mapping,
+                                       int64_t tokens, int num_heads, int num_kv_heads, int head_size, int block_size, int x, int dtype,
+                                       int kv_dtype, float k_scale, float v_scale, void* stream) {
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "rope_cache: dtype must be f16 or bf16");
   APHRO_CHECK(kv_dtype >= APHRO_KV_AUTO && kv_dtype <= APHRO_KV_FP8_E5M2, "Unsupported data type of kv cache: %d", kv_dtype);
   APHRO_CHECK((qkv != nullptr) != (slabs != nullptr), "rope_cache: exactly one of qkv / slabs");
+  APHRO_CHECK(slabs != nullptr || (row_scale == nullptr && col_scale == nullptr), "rope_cache: scales belong to slabs");
   APHRO_CHECK(rot_dim % 2 == 0 && rot_dim <= head_size && head_size % x == 0, "rope_cache: bad rot_dim / x");
   if (tokens == 0) return APHRO_OK;
   dim3 grid((unsigned)tokens), block(512);
@@ -616,7 +628,7 @@ extern "C" int aphro_rope_cache(const void* qkv, int64_t qkv_stride, const float
   hipLaunchKernelGGL((rope_cache_vec_kernel<TT, KVV>), grid, vblock, 0, (hipStream_t)stream, (const uint16_t*)qkv, \
                      qkv_stride, slabs, nslab, (int)tokens, positions, (const uint16_t*)cos_sin_cache,           \
                      (uint16_t*)q_out, key_cache, value_cache, slot_mapping, num_heads, num_kv_heads, head_size, \
-                     block_size, x, k_scale, v_scale)
+                     block_size, x, k_scale, v_scale, row_scale, col_scale)
 #define LVK(TT) { if (kv_dtype == APHRO_KV_AUTO) LV(TT, 0); else if (kv_dtype == APHRO_KV_FP8_E4M3) LV(TT, 1); else LV(TT, 2); }
     if (dtype == APHRO_F16) LVK(Half) else LVK(BFloat)
 #undef LVK
@@ -628,7 +640,7 @@ extern "C" int aphro_rope_cache(const void* qkv, int64_t qkv_stride, const float
   hipLaunchKernelGGL((rope_cache_kernel<TT, KVV, NX>), grid, block, 0, (hipStream_t)stream, (const uint16_t*)qkv, \
                      qkv_stride, slabs, nslab, (int)tokens, positions, (const uint16_t*)cos_sin_cache, rot_dim,  \
                      (uint16_t*)q_out, key_cache, value_cache, slot_mapping, num_heads, num_kv_heads, head_size, \
-                     block_size, x, k_scale, v_scale)
+                     block_size, x, k_scale, v_scale, row_scale, col_scale)
 #define LN(TT, KVV) { if (is_neox) L(TT, KVV, true); else L(TT, KVV, false); }
 #define LK(TT) { if (kv_dtype == APHRO_KV_AUTO) LN(TT, 0) else if (kv_dtype == APHRO_KV_FP8_E4M3) LN(TT, 1) else LN(TT, 2) }
   if (dtype == APHRO_F16) LK(Half) else LK(BFloat)
@@ -637,4 +649,14 @@ extern "C" int aphro_rope_cache(const void* qkv, int64_t qkv_stride, const float
 #undef L
   APHRO_LAUNCH_CHECK();
   return APHRO_OK;
+}
+
+extern "C" int aphro_rope_cache(const void* qkv, int64_t qkv_stride, const float* slabs, int nslab,
+                                const int64_t* positions, const void* cos_sin_cache, int rot_dim, int is_neox,
+                                void* q_out, void* key_cache, void* value_cache, const int64_t* slot_mapping,
+                                int64_t tokens, int num_heads, int num_kv_heads, int head_size, int block_size,
+                                int x, int dtype, int kv_dtype, float k_scale, float v_scale, void* stream) {
+  return aphro_rope_cache_scaled(qkv, qkv_stride, slabs, nslab, nullptr, nullptr, positions, cos_sin_cache, rot_dim, is_neox, q_out, key_cache,
+                                 value_cache, slot_mapping, tokens, num_heads, num_kv_heads, head_size, block_size, x, dtype, kv_dtype,
+                                 k_scale, v_scale, stream);
 }

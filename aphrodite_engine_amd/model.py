@@ -221,6 +221,12 @@ def _rope_cache(head_dim: int, max_pos: int, theta: float, dtype, device, rope_s
     return torch.cat((cos, sin), dim=-1).to(dtype)
 
 
+# Decoded rows from which an FP8 step's rotary embedding and cache write are a launch of their own in front of the attention, where they sum a
+# token's slabs once instead of in each of its kv heads' workgroups.  Four layers, us apart / inside: 33 rows 628 / 655, 64 668 / 696, 139
+# 938 / 1025, 190 874 / 927.  (Up to 32 rows, and for the int4 steps' rows, the launch costs more than it saves: 32 rows 527 / 513.)
+ROPE_APART_FROM = 33
+
+
 class LlamaDecoderLayer(nn.Module):
     def __init__(self, cfg: LlamaConfig, quant_config, dtype, kv_cache_dtype: str, layer_idx: int = 0):
         super().__init__()
@@ -672,7 +678,7 @@ class LlamaDecoderLayer(nn.Module):
         inside the attention kernel.  The activation scheme -- dynamic per token, or the checkpoint's
         static per-tensor input_scale -- must be the same for the four projections of the layer."""
         from .quantization.fp8 import CompressedTensorsW8A8Fp8Method, CDNA4Fp8LinearMethod
-        if m > 192 or self.head_dim != 128 or not self.fuse_rope_attention or self.is_moe or self.has_bias:
+        if m > 64 or self.head_dim != 128 or not self.fuse_rope_attention or self.is_moe or self.has_bias:
             return False
         lins = self.linears()
         static = [getattr(lin, "input_scale", None) is not None for lin in lins]
@@ -694,6 +700,11 @@ class LlamaDecoderLayer(nn.Module):
                 return False
         return True
 
+    def fused_decode_fp8_rows_ok(self, m: int) -> bool:
+        """``fused_decode_fp8_ok``, and beyond its 64 rows whatever the few-rows product leaves as slabs (up to 192)."""
+        return self.fused_decode_fp8_ok(min(m, 64)) and (m <= 64 or all(ops.fp8_gemm_ksplit(m, lin.out_features, lin.in_features) > 0
+                                                                        for lin in self.linears()))
+
     def _channel_scale(self, lin) -> torch.Tensor:
         ws = lin.weight_scale
         if ws.numel() == lin.out_features:
@@ -703,6 +714,13 @@ class LlamaDecoderLayer(nn.Module):
             cached = ws.reshape(1).expand(lin.out_features).contiguous()
             lin._weight_scale_channel = cached
         return cached
+
+    def _attend_apart(self, qkv_slabs, sx, positions, cos_sin, cos_sin_tok, key_cache, value_cache, attn_metadata):
+        """Rotary embedding and cache write of an FP8 projection's slabs in a launch of their own, then the attention."""
+        q = ops.rope_cache(None, qkv_slabs, None if cos_sin_tok is not None else positions, cos_sin_tok if cos_sin_tok is not None else cos_sin,
+                           True, key_cache, value_cache, attn_metadata.slot_mapping, self.num_heads, self.num_kv_heads, self.head_dim,
+                           self.attn.kv_cache_dtype, self.k_scale, self.v_scale, row_scale=sx, col_scale=self._channel_scale(self.qkv_proj))
+        return self.attn.decode(q.view(-1, self.num_heads, self.head_dim), key_cache, value_cache, attn_metadata, self.k_scale, self.v_scale)
 
     def forward_decode_fused_fp8(self, positions, x, prev, residual, first, kv_cache, attn_metadata, cos_sin,
                                  cos_sin_tok=None):
@@ -734,7 +752,9 @@ class LlamaDecoderLayer(nn.Module):
         aq_o = s_o is None and self.tp == 1 and o_st is not None and self.num_heads // self.num_kv_heads <= 16 and self.q_size % 64 == 0 \
             and ops.fp8_gemm_resident_aq_supported(m, self.o_proj.out_features, self.q_size, self.num_kv_heads) \
             and not switch("APHRO_FP8_NO_LAUNCH_DIET")
-        attn_res = ops.paged_attention_rope_scaled(
+        apart = m >= ROPE_APART_FROM
+        attn_res = self._attend_apart(qkv_slabs, sx, positions, cos_sin, cos_sin_tok, key_cache, value_cache, attn_metadata) if apart \
+            else ops.paged_attention_rope_scaled(
             qkv_slabs, sx, self._channel_scale(self.qkv_proj),
             None if cos_sin_tok is not None else positions,
             cos_sin_tok if cos_sin_tok is not None else cos_sin, attn_metadata.slot_mapping,
@@ -743,7 +763,7 @@ class LlamaDecoderLayer(nn.Module):
             attn_metadata.max_decode_seq_len, None, self.attn.kv_cache_dtype, self.k_scale, self.v_scale,
             out_q8_scale=s_o if fuse_static else None, want_out=False, want_absmax=aq_o, out_pairs=aq_o)
         o_slabs = None
-        if fuse_static:
+        if fuse_static and not apart:
             qa, sa = attn_res[1], s_o
             act_dtype = cos_sin.dtype if cos_sin_tok is None else cos_sin_tok.dtype
         elif aq_o:
@@ -1027,7 +1047,7 @@ class LlamaForCausalLM(nn.Module):
             return out
         if (self.use_fused_decode and attn_metadata.num_prefill_tokens == 0
                 and attn_metadata.num_decode_tokens > 0
-                and all(l.fused_decode_fp8_ok(hidden.shape[0]) for l in self.layers)):
+                and all(l.fused_decode_fp8_rows_ok(hidden.shape[0]) for l in self.layers)):
             residual = torch.empty_like(hidden)
             x, prev = hidden, None
             cos_sin_tok = self.cos_sin.index_select(0, positions)

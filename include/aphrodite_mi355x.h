@@ -379,6 +379,12 @@ int aphro_rope_cache(const void* qkv, int64_t qkv_stride, const float* slabs, in
                      const int64_t* slot_mapping, int64_t tokens, int num_heads,
                      int num_kv_heads, int head_size, int block_size, int x, int dtype,
                      int kv_dtype, float k_scale, float v_scale, void* stream);
+/* the same on an FP8 projection's raw slabs: an element is row_scale[token] * (col_scale[column] * sum) (row_scale NULL: 1) */
+int aphro_rope_cache_scaled(const void* qkv, int64_t qkv_stride, const float* slabs, int nslab, const float* row_scale,
+                            const float* col_scale, const int64_t* positions, const void* cos_sin_cache, int rot_dim,
+                            int is_neox, void* q_out, void* key_cache, void* value_cache, const int64_t* slot_mapping,
+                            int64_t tokens, int num_heads, int num_kv_heads, int head_size, int block_size, int x, int dtype,
+                            int kv_dtype, float k_scale, float v_scale, void* stream);
 
 /* ------------------------------------------------------------------------
  * Prefill attention (row a5): causal varlen flash attention on MFMA.

@@ -43,3 +43,31 @@ def test_rows(m, n, k, dtype, vector):
 def test_not_served():
     for m, n, k in ((32, 4096, 4096), (193, 4096, 4096), (64, 4096, 4032), (64, 4104, 4096)):
         assert _lib.lib().aphro_fp8_gemm_rows_ksplit(m, n, k) == 0
+
+
+@pytest.mark.parametrize("kv", ["auto", "fp8"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("nslab,rows", [(1, True), (5, True), (9, False)])
+def test_rope_cache_of_scaled_slabs(kv, dtype, nslab, rows):
+    """Scales over raw slabs: the bits of the scaled sums handed over in 16 bits."""
+    g = torch.Generator(device="cuda").manual_seed(nslab)
+    T, H, G, d, block = 37, 8, 2, 128, 16
+    n = (H + 2 * G) * d
+    slabs = torch.randn(nslab, T, n, generator=g, device="cuda") * 20
+    sa = torch.rand(T, 1, generator=g, device="cuda") * 0.1 if rows else None
+    sb = torch.rand(n, generator=g, device="cuda") * 0.1
+    total = slabs[0].clone()
+    for s in slabs[1:]:
+        total += s
+    qkv = ((sb * total) if sa is None else sa * (sb * total)).to(dtype)
+    cos_sin = torch.randn(T, d, generator=g, device="cuda").to(dtype)
+    slots = torch.randperm(64, generator=g, device="cuda")[:T]
+    results = []
+    for args in ((None, slabs, dict(row_scale=sa, col_scale=sb)), (qkv, None, {})):
+        kind, x = (torch.uint8, 16) if kv == "fp8" else (dtype, 8)
+        k = torch.zeros(4, G, d // x, block, x, dtype=kind, device="cuda")
+        v = torch.zeros(4, G, d, block, dtype=kind, device="cuda")
+        q = ops.rope_cache(args[0], args[1], None, cos_sin, True, k, v, slots, H, G, d, kv, 1.0, 1.0, **args[2])
+        results.append((q, k, v))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
