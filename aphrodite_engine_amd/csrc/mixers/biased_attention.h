@@ -46,6 +46,7 @@ template <int FORM>
 void dba_prefill_launch(const DBAParams& p, int64_t num_tokens, int max_q_len, int num_seqs, hipStream_t st);
 template <int FORM>
 void dba_decode_launch(const DBAParams& p, int64_t rows, int nsplit, hipStream_t st);
+constexpr int DBA_MAX_SPLITS = 8;       // workgroups that share a decoded row's keys
 constexpr int DBA_MFMA_MIN_LEN = 8;     // segments at least this long go to the matrix-core kernel
 
 }  // namespace aphro

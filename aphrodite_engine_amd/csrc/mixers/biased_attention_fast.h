@@ -20,6 +20,7 @@
 //    the V pass wants, so nothing is redistributed; K and V of a step are fetched together.  Four waves take the steps
 //    round-robin and merge their (max, sum, acc) in LDS; long key ranges are also split over workgroups (grid z), whose
 //    partial results dba_merge_kernel combines.
+//  * dba_decode128_kernel<QH>: the same for rows of 128 values in blocks of whole 16-key tiles, see there.
 #pragma once
 #include "biased_attention.h"
 
@@ -533,6 +534,186 @@ __global__ __launch_bounds__(256) void dba_decode_kernel(DBAParams p) {
   }
 }
 
+// The same rows where rows are 128 wide (the width of the models) and a cache block holds whole tiles of 16 keys.  A wave takes 16 keys a
+// step, aligned in the block, so that a step's block is one scalar lookup and every address a uniform base and a constant of the lane.
+// S = K Q^T is four v_mfma_f32_16x16x32_bf16: a lane ends with keys 4 g + r of head `lane % 16` (QH of the 16 columns are heads, the others
+// zeros), which makes temperature, cap, bias, mask and softmax of a step those of 4 numbers.  The V pass stays on the vector ALUs in fp32:
+// 16 lanes read a V row of key 4 g + i, and the weight of a head is broadcast to them inside their row of 16 lanes by DPP.  K of the next
+// step is asked for behind the products, V behind the V pass, so both are on their way during the softmax; nothing branches around a load.
+// Bound by memory latency: a wave has few steps.  us with dba_decode_kernel, whose loads wait for one another behind their masks and which
+// spends 660 instructions on a step of 16 keys, and here, merge included: 32 rows of up to 1040 keys, 32 heads on 8 with bias 52.9 / 25.4
+// (3.4 TB/s), 16 on 4 34.4 / 16.4; one row of 1000 keys 25.0 / 11.5; 128 rows of up to 2000 364 / 146 (4.3 TB/s); two of 16000 121 / 31;
+// 24 rows of up to 700, window 31.2 / 18.8, cap and bias 37.7 / 22.9.
+template <int H>
+__device__ __forceinline__ float row_bcast(float v) { return dpp_f<0x150 + H>(v); }       // lane H of every row of 16
+template <int QH, int H>
+__device__ __forceinline__ void dec128_scale(float (&acc)[QH][8], float alpha) {
+  const float a = row_bcast<H>(alpha);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc[H][j] *= a;
+  if constexpr (H + 1 < QH) dec128_scale<QH, H + 1>(acc, alpha);
+}
+template <int QH, int H>
+__device__ __forceinline__ void dec128_add(float (&acc)[QH][8], float prob, const float* vf) {
+  const float w = row_bcast<H>(prob);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc[H][j] += w * vf[j];
+  if constexpr (H + 1 < QH) dec128_add<QH, H + 1>(acc, prob, vf);
+}
+
+template <int QH, int FORM>
+__global__ __launch_bounds__(256, 4) void dba_decode128_kernel(DBAParams p) {
+  constexpr bool EXT = FORM == DBA_MASKED;
+  constexpr int D = 128;
+  __shared__ __attribute__((aligned(16))) float part[4][4][QH][D];      // [wave][lane group]: sums of e^(s - m) v
+  __shared__ float stat[4][QH][2];                                       // [wave]: m, l
+  const int per_kv = p.heads / p.kv_heads, groups = (per_kv + QH - 1) / QH;
+  const int kvh = blockIdx.y / groups, sub0 = (blockIdx.y % groups) * QH, hbase = kvh * per_kv;
+  int seq;
+  const int t = __builtin_amdgcn_readfirstlane(dba_short_row(p, blockIdx.x, seq));
+  if (t < 0) return;                                       // the prompt kernel's share
+  seq = __builtin_amdgcn_readfirstlane(seq);
+  const int pos = p.ctx_len[seq] + (t - p.q_start[seq]);
+  const int k0 = EXT ? dba_first_key(p, pos) : 0;          // oldest visible key
+  const int nkeys = pos + 1;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l15 = lane & 15, g = lane >> 4;
+  const float qs = p.scale * dba_temp(p, pos);
+  const int myhead = hbase + min(sub0 + min(l15, QH - 1), per_kv - 1);
+  u16x8 qf[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) {
+    qf[kk] = *reinterpret_cast<const u16x8*>(p.q + (int64_t)t * p.q_stride + myhead * D + 32 * kk + 8 * g);
+    if (l15 >= QH) qf[kk] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  }
+  const int32_t* bt = p.block_tables + (int64_t)seq * p.max_blocks;
+  const float* lut = p.bias_lut ? p.bias_lut + (int64_t)myhead * p.lut_len : nullptr;
+  const int row = p.kv_heads * D;                          // numbers of a cache row
+  const int koff = l15 * row + 8 * g, voff = 4 * g * row + 8 * l15;
+  const int first = k0 >> 4, ntiles = ((nkeys + 15) >> 4) - first;
+  const int nsplit = gridDim.z, tps = (ntiles + nsplit - 1) / nsplit;
+  const int tile_end = min(ntiles, ((int)blockIdx.z + 1) * tps);
+  int tile = (int)blockIdx.z * tps + wave;
+  float m = -INFINITY, l = 0.f, acc[QH][8], b[4] = {0.f, 0.f, 0.f, 0.f};
+  u16x8 kf[4], vv[4];
+#pragma unroll
+  for (int qh = 0; qh < QH; ++qh)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[qh][j] = 0.f;
+  // block of a tile (asked for two steps ahead), and numbers ahead of its first cache row of this kv head
+  auto block_of = [&](int tl) { return bt[((first + min(tl, tile_end - 1)) << 4) >> p.bs_shift]; };
+  auto base_of = [&](int tl, int blk) -> int64_t {
+    if (blk < 0 || blk >= p.num_blocks) blk = 0;           // never read outside the pool
+    return ((int64_t)blk * p.block_size + (((first + tl) << 4) & (p.block_size - 1))) * row + kvh * D;
+  };
+  auto load_k = [&](int tl, int64_t base) {
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) kf[kk] = *reinterpret_cast<const u16x8*>(p.k_cache + base + koff + 32 * kk);
+    if (lut) {
+      const int dist = pos - ((first + tl) << 4) - 4 * g;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) b[r] = lut[max(0, min(dist - r, p.lut_len - 1))];
+    }
+  };
+  auto load_v = [&](int64_t base) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) vv[i] = *reinterpret_cast<const u16x8*>(p.v_cache + base + voff + i * row);
+  };
+  if (tile < tile_end) {
+    const int64_t base = base_of(tile, block_of(tile));
+    load_k(tile, base);
+    load_v(base);
+    int blk = block_of(tile + 4);
+    while (true) {
+      const bool more = tile + 4 < tile_end;
+      const int64_t next = base_of(tile + 4, blk);
+      blk = block_of(tile + 8);
+      f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kf[kk]), __builtin_bit_cast(bf16x8, qf[kk]), s, 0, 0, 0);
+      const int key0 = (first + tile) << 4;
+      float x[4], mx = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = key0 + 4 * g + r;
+        x[r] = s[r] * qs;
+        if (EXT && p.softcap > 0.f) x[r] = p.softcap * tanhf(x[r] / p.softcap);
+        x[r] = key >= k0 && key < nkeys ? x[r] + b[r] : -INFINITY;       // slots that hold no key may hold anything
+        mx = fmaxf(mx, x[r]);
+      }
+      if (more) load_k(tile + 4, next);
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float m_new = fmaxf(m, mx);
+      if (__builtin_amdgcn_ballot_w64(m_new > m)) {
+        const float alpha = m == -INFINITY ? 0.f : __expf(m - m_new);
+        m = m_new;
+        l *= alpha;
+        dec128_scale<QH, 0>(acc, alpha);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x[r] = x[r] == -INFINITY ? 0.f : __expf(x[r] - m);
+        l += x[r];                                         // this lane group's share; groups are summed at the end
+      }
+      if (key0 < k0 || key0 + 16 > nkeys) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (key0 + 4 * g + i < k0 || key0 + 4 * g + i >= nkeys) vv[i] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float vf[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) vf[j] = BFloat::to_f32(vv[i][j]);
+        dec128_add<QH, 0>(acc, x[i], vf);
+      }
+      if (!more) break;
+      load_v(next);
+      tile += 4;
+    }
+  }
+  // the four lane groups of the four waves meet in LDS
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (g == 0 && l15 < QH) {
+    stat[wave][l15][0] = m;
+    stat[wave][l15][1] = l;
+  }
+#pragma unroll
+  for (int qh = 0; qh < QH; ++qh) {
+    *reinterpret_cast<f32x4*>(&part[wave][g][qh][8 * l15]) = f32x4{acc[qh][0], acc[qh][1], acc[qh][2], acc[qh][3]};
+    *reinterpret_cast<f32x4*>(&part[wave][g][qh][8 * l15 + 4]) = f32x4{acc[qh][4], acc[qh][5], acc[qh][6], acc[qh][7]};
+  }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < QH * D; idx += 256) {
+    const int qh = idx / D, col = idx % D;
+    if (sub0 + qh >= per_kv) continue;
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) M = fmaxf(M, stat[w][qh][0]);
+    float L = 0.f, o = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float f = (stat[w][qh][0] == -INFINITY) ? 0.f : __expf(stat[w][qh][0] - M);
+      L += stat[w][qh][1] * f;
+      o += ((part[w][0][qh][col] + part[w][1][qh][col]) + (part[w][2][qh][col] + part[w][3][qh][col])) * f;
+    }
+    const int head = hbase + sub0 + qh;
+    if (nsplit > 1) {                                       // this split's share; dba_merge_kernel finishes the row
+      float* w = p.ws + (((int64_t)t * p.heads + head) * nsplit + blockIdx.z) * (2 + D);
+      if (col == 0) {
+        w[0] = M;
+        w[1] = L;
+      }
+      w[2 + col] = o;
+      continue;
+    }
+    dba_finish<FORM>(p, t, head, col, M, L, o);
+  }
+}
+
+// the key ranges' shares of a row, all asked for at once (there are at most DBA_MAX_SPLITS)
 template <int FORM>
 __global__ void dba_merge_kernel(DBAParams p, int nsplit) {
   const int head = blockIdx.y;
@@ -540,19 +721,27 @@ __global__ void dba_merge_kernel(DBAParams p, int nsplit) {
   const int t = dba_short_row(p, blockIdx.x, seq);
   if (t < 0) return;
   const float* w = p.ws + ((int64_t)t * p.heads + head) * nsplit * (2 + p.vdim);
-  float M = -INFINITY;
-  for (int z = 0; z < nsplit; ++z) M = fmaxf(M, w[z * (2 + p.vdim)]);
-  float L = 0.f;
-  for (int z = 0; z < nsplit; ++z) {
-    const float mz = w[z * (2 + p.vdim)];
-    if (mz != -INFINITY) L += w[z * (2 + p.vdim) + 1] * __expf(mz - M);
+  float mz[DBA_MAX_SPLITS], lz[DBA_MAX_SPLITS], M = -INFINITY, L = 0.f;
+#pragma unroll
+  for (int z = 0; z < DBA_MAX_SPLITS; ++z) {
+    const float* wz = w + min(z, nsplit - 1) * (2 + p.vdim);
+    mz[z] = wz[0];
+    lz[z] = wz[1];
+  }
+#pragma unroll
+  for (int z = 0; z < DBA_MAX_SPLITS; ++z) M = fmaxf(M, mz[z]);
+#pragma unroll
+  for (int z = 0; z < DBA_MAX_SPLITS; ++z) {
+    mz[z] = z < nsplit && mz[z] != -INFINITY ? __expf(mz[z] - M) : 0.f;       // the share's weight
+    if (mz[z] != 0.f) L += lz[z] * mz[z];
   }
   for (int col = threadIdx.x; col < p.vdim; col += blockDim.x) {
-    float o = 0.f;
-    for (int z = 0; z < nsplit; ++z) {
-      const float mz = w[z * (2 + p.vdim)];
-      if (mz != -INFINITY) o += w[z * (2 + p.vdim) + 2 + col] * __expf(mz - M);
-    }
+    float oz[DBA_MAX_SPLITS], o = 0.f;
+#pragma unroll
+    for (int z = 0; z < DBA_MAX_SPLITS; ++z) oz[z] = w[min(z, nsplit - 1) * (2 + p.vdim) + 2 + col];
+#pragma unroll
+    for (int z = 0; z < DBA_MAX_SPLITS; ++z)
+      if (mz[z] != 0.f) o += oz[z] * mz[z];
     dba_finish<FORM>(p, t, head, col, M, L, o);
   }
 }
@@ -928,6 +1117,14 @@ template <int FORM>
 void dba_decode_launch(const DBAParams& p, int64_t rows, int nsplit, hipStream_t st) {
   const dim3 grid((unsigned)rows, (unsigned)dba_decode_units(p.heads, p.kv_heads, p.dim, p.vdim), (unsigned)nsplit);
   const int chl = decode_chl(p.dim, p.vdim), qh = decode_qh(p.heads, p.kv_heads, chl);
+  // rows of the models' width in blocks of whole 16-key tiles, 16-byte pieces aligned, a block's rows within 32-bit offsets
+  const bool wide = p.dim == 128 && p.vdim == 128 && p.bs_shift >= 4 && (((uintptr_t)p.k_cache | (uintptr_t)p.v_cache) & 15) == 0 &&
+                    (int64_t)p.kv_heads * 128 * 16 < (1ll << 30);
+  if (wide) {
+    if (qh == 4) hipLaunchKernelGGL((dba_decode128_kernel<4, FORM>), grid, dim3(256), 0, st, p);
+    else if (qh == 2) hipLaunchKernelGGL((dba_decode128_kernel<2, FORM>), grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((dba_decode128_kernel<1, FORM>), grid, dim3(256), 0, st, p);
+  } else {
 #define DEC(QH, CHL) hipLaunchKernelGGL((dba_decode_kernel<QH, CHL, FORM>), grid, dim3(256), 0, st, p)
 #define DEC_BY_CHL(QH)                          \
   switch (chl) {                                \
@@ -941,6 +1138,7 @@ void dba_decode_launch(const DBAParams& p, int64_t rows, int nsplit, hipStream_t
     case 2: DEC_BY_CHL(2); break;
     case 4: DEC_BY_CHL(4); break;
     case 8: DEC_BY_CHL(8); break;
+  }
   }
 #undef DEC_BY_CHL
 #undef DEC

@@ -22,7 +22,7 @@ int dba_decode_splits(int64_t rows, int64_t num_tokens, int units, int max_kv_le
   const int tiles = (max_kv_len + 63) / 64;
   int64_t n = (1024 + rows * units - 1) / (rows * units);
   if (n > tiles / 4) n = tiles / 4;
-  if (n > 8) n = 8;
+  if (n > DBA_MAX_SPLITS) n = DBA_MAX_SPLITS;
   while (n > 1 && num_tokens * heads * n * (2 + vdim) > ws_floats) --n;
   return n < 1 ? 1 : (int)n;
 }
