@@ -432,8 +432,10 @@ def interleaved_to_half(t: torch.Tensor, dims: int, at: int = 0) -> torch.Tensor
 
 # Latents are expanded where prompt portions have LATENT_EXPAND_ROWS rows in all and either half of the keys they see are their own, or a key is
 # seen often enough to pay for its expansion (heads * kv_rank * pairs of a row and a key, over keys); up to LATENT_EXPAND_MOST numbers of
-# keys and values (512 MiB).
-LATENT_EXPAND_ROWS, LATENT_EXPAND_PAIRS, LATENT_EXPAND_MOST = 96, 2.5e6, 1 << 28
+# keys and values (512 MiB).  It saves about 14 us of the GPU per 1e9 of heads * kv_rank * pairs and costs five more launches, 35 us of a host
+# that small steps wait for: from LATENT_EXPAND_WORK on (a step of two portions of 500 tokens behind 300 beside 12 decoded ones, 16 heads, 2.5e9:
+# 1230 us with it, 1000 without; three of 1400 tokens, 32 heads, 2e10: 3630 and 4260).
+LATENT_EXPAND_ROWS, LATENT_EXPAND_PAIRS, LATENT_EXPAND_MOST, LATENT_EXPAND_WORK = 96, 2.5e6, 1 << 28, 6e9
 
 
 class LatentAttention(nn.Module):
@@ -512,7 +514,8 @@ class LatentAttention(nn.Module):
         if rows < LATENT_EXPAND_ROWS or keys * self.heads * (self.dim + self.vdim) > LATENT_EXPAND_MOST:
             return 0
         pairs = sum(n * (min(self.window, s) if self.window else s - n // 2) for n, s in zip(lens, seen))
-        return k if 2 * rows >= keys or self.heads * self.kv_rank * pairs >= LATENT_EXPAND_PAIRS * keys else 0
+        work = self.heads * self.kv_rank * pairs
+        return k if work >= LATENT_EXPAND_WORK and (2 * rows >= keys or work >= LATENT_EXPAND_PAIRS * keys) else 0
 
     def attend(self, h: torch.Tensor, cache: torch.Tensor, batch: StepBatch, out: Optional[torch.Tensor] = None,
                rows: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -78,6 +78,7 @@ def test_expanded(heads, segments, block, form, monkeypatch):
     errors = []
     for pairs in (0.0, float("inf")):                          # every portion expanded, none
         monkeypatch.setattr(M, "LATENT_EXPAND_PAIRS", pairs)
+        monkeypatch.setattr(M, "LATENT_EXPAND_WORK", 0)
         monkeypatch.setattr(M, "LATENT_EXPAND_ROWS", 1 if pairs == 0.0 else 1 << 40)
         assert (m.expanded_segments(b) > 0) == (pairs == 0.0)
         wide = torch.full((b.num_tokens, heads * D + 16), 7.0, dtype=torch.bfloat16, device="cuda")
@@ -105,8 +106,11 @@ def test_gathered_rows():
         assert torch.equal(got, want)
 
 
-def test_when_it_runs():
+def test_when_it_runs(monkeypatch):
     m = _module(4)
+    assert m.expanded_segments(_batch([(0, 4100), (90, 1)], 16)[0]) == 1          # 6.5e9 of heads * kv_rank * pairs
+    assert m.expanded_segments(_batch([(0, 3900), (90, 1)], 16)[0]) == 0          # 5.8e9
+    monkeypatch.setattr(M, "LATENT_EXPAND_WORK", 0)
     assert m.expanded_segments(_batch([(0, 100), (90, 1)], 16)[0]) == 1
     assert m.expanded_segments(_batch([(0, 95)], 16)[0]) == 0                    # few rows
     assert m.expanded_segments(_batch([(2000, 100)], 16)[0]) == 0                 # few rows for the keys
