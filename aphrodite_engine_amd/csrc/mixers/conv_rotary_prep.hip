@@ -12,6 +12,9 @@
 // A thread owns 8 neighbouring channels of one head and TOK consecutive rows (TOK + TAPS - 1 input rows and its taps are read once, 16
 // bytes at a time); tph threads -- a power of two, within one wave -- share a head.  The angles of the workgroup's rows are worked out
 // once, in LDS, for all its heads; rotation partners meet in LDS too, so that half the rotated part may be any number.
+// Bound by the rows' way in and out and by the chain lookup, angles, rows ahead of it; the rows and weights need neither and are asked for
+// first.  With them asked for behind the angles, partners read number by number and 4 rows a thread, us before / here: 32 heads on 8 of 128,
+// 3000 rows in three segments 34.3 / 31.7, 2560 rows 29.6 / 26.4, 60 rows 11.5 / 9.5; 16 on 4, 900 rows 12.7 / 10.4, 20 single tokens 5.1 / 4.5.
 #include "mixers_common.h"
 
 extern "C" int aphro_short_conv_state(void* state, const void* u, int64_t u_stride, const int32_t* state_slots, const int32_t* q_start,
@@ -42,21 +45,6 @@ struct ConvRotaryParams {
 };
 
 template <typename T>
-__device__ __forceinline__ void cr_load8(const typename T::storage* p, float* o) {
-  if constexpr (sizeof(typename T::storage) == 2) {
-    const u16x8 v = *reinterpret_cast<const u16x8*>(p);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = T::to_f32(v[j]);
-  } else {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      o[j] = a[j];
-      o[4 + j] = b[j];
-    }
-  }
-}
-template <typename T>
 __device__ __forceinline__ void cr_store8(typename T::storage* p, const float* v) {
   if constexpr (sizeof(typename T::storage) == 2) {
     *reinterpret_cast<u32x4*>(p) = u32x4{pack2_16<true>(v[0], v[1]), pack2_16<true>(v[2], v[3]), pack2_16<true>(v[4], v[5]), pack2_16<true>(v[6], v[7])};
@@ -65,38 +53,6 @@ __device__ __forceinline__ void cr_store8(typename T::storage* p, const float* v
     *reinterpret_cast<f32x4*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
   }
 }
-
-// 8 numbers as they lie in memory (16 bytes of bf16, 32 of fp32): rows in flight take no more registers than that
-template <typename T>
-struct CRChunk {
-  u32x4 v[sizeof(typename T::storage) / 2];
-  __device__ __forceinline__ void load(const typename T::storage* p) {
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(typename T::storage) / 2); ++i) v[i] = reinterpret_cast<const u32x4*>(p)[i];
-  }
-  __device__ __forceinline__ void clear() {
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(typename T::storage) / 2); ++i) v[i] = u32x4{0, 0, 0, 0};
-  }
-  __device__ __forceinline__ void store(typename T::storage* p) const {
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(typename T::storage) / 2); ++i) reinterpret_cast<u32x4*>(p)[i] = v[i];
-  }
-  __device__ __forceinline__ void floats(float* o) const {
-    if constexpr (sizeof(typename T::storage) == 2) {
-      const u16x8 x = __builtin_bit_cast(u16x8, v[0]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = T::to_f32(x[j]);
-    } else {
-      const f32x4 a = __builtin_bit_cast(f32x4, v[0]), b = __builtin_bit_cast(f32x4, v[1]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        o[j] = a[j];
-        o[4 + j] = b[j];
-      }
-    }
-  }
-};
 
 constexpr int CR_THREADS = 256, CR_MAX_DIM = 512;
 
@@ -115,6 +71,29 @@ __global__ __launch_bounds__(CR_THREADS) void conv_rotary_qk_norm_kv_write_kerne
   f32x2* turn = reinterpret_cast<f32x2*>(cr_lds + 8 * CR_THREADS);      // (cos, sin) of [row of the tile][pair]
   const int64_t t0 = (int64_t)blockIdx.x * TOK;
   const int half = p.rot_dims >> 1;
+  const int tph = p.tph, H = p.heads, G = p.kv_heads;
+  const int unit = blockIdx.y * (CR_THREADS / tph) + threadIdx.x / tph, i0 = 8 * (threadIdx.x % tph);
+  const bool is_q = unit < H, is_v = unit >= H + G;
+  const int hd = is_q ? unit : (is_v ? unit - H - G : unit - H), n = is_v ? p.vdim : p.dim;
+  const int C = (H + G) * p.dim + G * p.vdim;
+  const int c0 = (is_v ? (H + G) * p.dim + hd * p.vdim : unit * p.dim) + i0;       // first channel (meaningful if work)
+  const bool unit_on = unit < H + 2 * G, work = unit_on && i0 < n;
+  // the rows and weights need no segment: they are on their way while the segments are looked up and the angles worked out
+  Chunk8<T> rows[TOK + TAPS - 1], wr[TAPS], nr;
+  nr.clear();
+#pragma unroll
+  for (int x = 0; x < TAPS; ++x) wr[x].clear();
+#pragma unroll
+  for (int x = 0; x < TOK + TAPS - 1; ++x) {
+    const int64_t gr = t0 - (TAPS - 1) + x;
+    if (work && gr >= 0 && gr < p.num_tokens) rows[x].load(p.u + gr * p.u_stride + c0);
+    else rows[x].clear();
+  }
+  if (work) {
+#pragma unroll
+    for (int x = 0; x < TAPS; ++x) wr[x].load(p.w + (int64_t)c0 * TAPS + 8 * x);
+    if (!is_v && p.q_weight) nr.load((is_q ? p.q_weight : p.k_weight) + i0);
+  }
   // what the rows of the tile are (uniform over the workgroup), asked for together
   int seq[TOK], back0[TOK], ctx[TOK], sslot[TOK];
   int64_t cslot[TOK];
@@ -140,37 +119,17 @@ __global__ __launch_bounds__(CR_THREADS) void conv_rotary_qk_norm_kv_write_kerne
     turn[i] = f32x2{c * p.mscale, sn * p.mscale};
   }
   __syncthreads();
-  const int tph = p.tph, H = p.heads, G = p.kv_heads;
-  const int unit = blockIdx.y * (CR_THREADS / tph) + threadIdx.x / tph, i0 = 8 * (threadIdx.x % tph);
-  if (unit >= H + 2 * G) return;                             // whole groups of tph lanes leave together
-  const bool is_q = unit < H, is_v = unit >= H + G;
-  const int hd = is_q ? unit : (is_v ? unit - H - G : unit - H), n = is_v ? p.vdim : p.dim;
-  const int C = (H + G) * p.dim + G * p.vdim;
-  const int c0 = (is_v ? (H + G) * p.dim + hd * p.vdim : unit * p.dim) + i0;       // first channel (meaningful if work)
-  const bool work = i0 < n;
+  if (!unit_on) return;                                      // whole groups of tph lanes leave together
   float wv[TAPS][8], nw[8];
-  CRChunk<T> rows[TOK + TAPS - 1];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) nw[i] = 1.f;
-#pragma unroll
-  for (int j = 0; j < TAPS; ++j)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) wv[j][i] = 0.f;
-  if (work) {
+  {
     float flat[8 * TAPS];
 #pragma unroll
-    for (int x = 0; x < TAPS; ++x) cr_load8<T>(p.w + (int64_t)c0 * TAPS + 8 * x, flat + 8 * x);
+    for (int x = 0; x < TAPS; ++x) wr[x].floats(flat + 8 * x);
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) wv[j][i] = flat[i * TAPS + j];
-    if (!is_v && p.q_weight) cr_load8<T>((is_q ? p.q_weight : p.k_weight) + i0, nw);
-  }
-#pragma unroll
-  for (int x = 0; x < TOK + TAPS - 1; ++x) {
-    const int64_t gr = t0 - (TAPS - 1) + x;
-    if (work && gr >= 0 && gr < p.num_tokens) rows[x].load(p.u + gr * p.u_stride + c0);
-    else rows[x].clear();
+    nr.floats(nw);
   }
 #pragma unroll
   for (int k = 0; k < TOK; ++k) {
@@ -178,7 +137,7 @@ __global__ __launch_bounds__(CR_THREADS) void conv_rotary_qk_norm_kv_write_kerne
     if (t >= p.num_tokens) break;
     S* st = TAPS > 1 && work ? p.state + (int64_t)sslot[k] * (TAPS - 1) * C + c0 : nullptr;
     float acc[8];
-    CRChunk<T> win[TAPS];
+    Chunk8<T> win[TAPS];
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) {
       const int back = back0[k] - TAPS + 1 + j;              // row of the segment, negative: before it
@@ -222,7 +181,19 @@ __global__ __launch_bounds__(CR_THREADS) void conv_rotary_qk_norm_kv_write_kerne
       *reinterpret_cast<f32x4*>(mine) = f32x4{acc[0], acc[1], acc[2], acc[3]};
       *reinterpret_cast<f32x4*>(mine + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
       cr_wave_fence();
-      if (i0 < 2 * half) {
+      if ((half & 7) == 0) {                                 // a thread's 8 numbers have one side, their partners lie together
+        if (i0 < 2 * half) {
+          const bool first = i0 < half;
+          const float* op = head + (first ? i0 + half : i0 - half);
+          const f32x4* tp = reinterpret_cast<const f32x4*>(turn + k * half + (first ? i0 : i0 - half));
+          const f32x4 o0 = *reinterpret_cast<const f32x4*>(op), o1 = *reinterpret_cast<const f32x4*>(op + 4);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const float c = tp[i >> 1][(i & 1) * 2], sn = tp[i >> 1][(i & 1) * 2 + 1], other = i < 4 ? o0[i] : o1[i - 4];
+            acc[i] = first ? acc[i] * c - other * sn : acc[i] * c + other * sn;
+          }
+        }
+      } else if (i0 < 2 * half) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int x = i0 + i;
@@ -275,11 +246,14 @@ extern "C" int aphro_conv_rotary_qk_norm_kv_write(void* q_out, int64_t q_out_str
   while (8 * tph < (dim > vdim ? dim : vdim)) tph *= 2;
   const int units = heads + 2 * kv_heads, per_block = CR_THREADS / tph;
   const bool single = max_q_len == 1;                        // every segment is one token: rows are tiled singly and advance their states
-  const int tok = single ? 1 : 4;
+  // rows a thread: 8 where that leaves four workgroups for every CU (each further row saves re-reading taps - 1 of them), else 4
+  const int64_t blocks8 = (num_tokens + 7) / 8 * ((units + per_block - 1) / per_block);
+  const int tok = single ? 1 : blocks8 >= 4 * device_cu_count() ? 8 : 4;
   const dim3 grid((unsigned)((num_tokens + tok - 1) / tok), (unsigned)((units + per_block - 1) / per_block));
   const size_t lds = (size_t)8 * CR_THREADS * sizeof(float) + (size_t)tok * (rot_dims / 2) * sizeof(f32x2);
 #define CR_LAUNCH(TAPS)                                                                                                               \
   if (single) hipLaunchKernelGGL((conv_rotary_qk_norm_kv_write_kernel<T, TAPS, 1>), grid, dim3(CR_THREADS), lds, (hipStream_t)stream, p); \
+  else if (tok == 8) hipLaunchKernelGGL((conv_rotary_qk_norm_kv_write_kernel<T, TAPS, 8>), grid, dim3(CR_THREADS), lds, (hipStream_t)stream, p); \
   else hipLaunchKernelGGL((conv_rotary_qk_norm_kv_write_kernel<T, TAPS, 4>), grid, dim3(CR_THREADS), lds, (hipStream_t)stream, p)
   MIX_DISPATCH_DTYPE(dtype, {
     typedef typename T::storage S;

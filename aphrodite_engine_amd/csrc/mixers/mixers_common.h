@@ -45,6 +45,38 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// 8 numbers as they lie in memory (16 bytes of bf16, 32 of fp32): rows in flight take no more registers than that
+template <typename T>
+struct Chunk8 {
+  u32x4 v[sizeof(typename T::storage) / 2];
+  __device__ __forceinline__ void load(const typename T::storage* p) {
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(typename T::storage) / 2); ++i) v[i] = reinterpret_cast<const u32x4*>(p)[i];
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(typename T::storage) / 2); ++i) v[i] = u32x4{0, 0, 0, 0};
+  }
+  __device__ __forceinline__ void store(typename T::storage* p) const {
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(typename T::storage) / 2); ++i) reinterpret_cast<u32x4*>(p)[i] = v[i];
+  }
+  __device__ __forceinline__ void floats(float* o) const {
+    if constexpr (sizeof(typename T::storage) == 2) {
+      const u16x8 x = __builtin_bit_cast(u16x8, v[0]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = T::to_f32(x[j]);
+    } else {
+      const f32x4 a = __builtin_bit_cast(f32x4, v[0]), b = __builtin_bit_cast(f32x4, v[1]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        o[j] = a[j];
+        o[4 + j] = b[j];
+      }
+    }
+  }
+};
+
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + __expf(-z)); }
 __device__ __forceinline__ float silu_f(float z) { return z / (1.0f + __expf(-z)); }
 __device__ __forceinline__ float gelu_tanh_f(float z) {
