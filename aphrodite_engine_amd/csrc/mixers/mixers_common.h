@@ -77,6 +77,41 @@ struct Chunk8 {
   }
 };
 
+// Sums over the four rows of 16 lanes of a wave, scattered: of four values a lane, the lane ends with the total of one over the lanes of its
+// column (lane % 16), without a shuffle through LDS: of value scatter_index4(lane).  (A bit cast of a vector's element, without the
+// conversion in between, reads element 0 whatever its index.)
+__device__ __forceinline__ float swap_add32(float a, float b) {          // lower half: a of both halves, upper half: b
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+__device__ __forceinline__ float swap_add16(float a, float b) {          // even rows: a of the two rows, odd rows: b
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+// the value whose total a lane ends with
+__device__ __forceinline__ float scatter_sum4(const float (&v)[4]) { return swap_add16(swap_add32(v[0], v[1]), swap_add32(v[2], v[3])); }
+__device__ __forceinline__ int scatter_index4(int lane) { return ((lane >> 5) & 1) | ((lane >> 3) & 2); }
+
+// NI neighbouring floats of LDS, in the widest pieces that NI allows
+template <int NI>
+__device__ __forceinline__ void lds_row(const float* p, float (&o)[NI]) {
+  if constexpr (NI % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < NI; i += 4) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(p + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[i + j] = x[j];
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NI; i += 2) {
+      const f32x2 x = *reinterpret_cast<const f32x2*>(p + i);
+      o[i] = x[0];
+      o[i + 1] = x[1];
+    }
+  }
+}
+
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + __expf(-z)); }
 __device__ __forceinline__ float silu_f(float z) { return z / (1.0f + __expf(-z)); }
 __device__ __forceinline__ float gelu_tanh_f(float z) {

@@ -176,11 +176,11 @@ __global__ __launch_bounds__(256) void outer_memory_scan_kernel(
 }
 
 // The same for short segments -- decoded tokens, one per request -- where the state's way through memory and back is the work: a thread
-// owns 4 neighbouring columns of every 16th row, so the state comes in 16-byte pieces, 256 contiguous bytes a row and workgroup, all of them
+// owns 4 neighbouring columns of NI rows, so the state comes in 16-byte pieces, 256 contiguous bytes a row and workgroup, all of them
 // in flight together with the first tokens' numbers; a token's partial sums meet in LDS once a stage, not once a token.
 // The split above with 4 lanes a column (4-byte pieces, 64 contiguous bytes, 160 to 210 registers: 2 or 3 waves a SIMD) took, in us against
-// here: single tokens of 32 sequences, decay 16 heads of 64 x 128 10.7 / 7.9, mLSTM 8 of 128 x 256 39.8 / 15.7 (4.3 TB/s), state space 128 of
-// 128 x 64 79.8 / 46.1 (5.8 TB/s); of one, 6.4 / 4.6 and 9.5 / 6.1; four segments of 8 tokens, mLSTM 22.4 / 13.0; three of 31, decay 17.3 / 16.8.
+// here: single tokens of 32 sequences, decay 16 heads of 64 x 128 10.7 / 7.8, mLSTM 8 of 128 x 256 39.8 / 15.5 (4.3 TB/s), state space 128 of
+// 128 x 64 79.8 / 46.3 (5.8 TB/s); of one, 6.4 / 4.4 and 9.5 / 5.9; four segments of 8 tokens, mLSTM 22.4 / 11.3; three of 31, decay 17.3 / 14.0.
 template <typename T, int MODE, int NI>
 __global__ __launch_bounds__(256, NI <= 8 ? 4 : 2) void outer_memory_rows_kernel(
     float* __restrict__ out, const typename T::storage* __restrict__ q, int64_t q_stride,
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256, NI <= 8 ? 4 : 2) void outer_memory_rows_kernel
   const bool in = col < vdim;                               // (vdim is a multiple of 4)
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int r = rr + 16 * i;
+    const int r = rr * NI + i;
     S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (!fresh && in && r < dim) S[i] = *reinterpret_cast<const f32x4*>(sbase + (int64_t)r * vdim + col);
   }
@@ -302,22 +302,18 @@ __global__ __launch_bounds__(256, NI <= 8 ? 4 : 2) void outer_memory_rows_kernel
       const float a = MODE != 0 ? a_s[tt] : dec;
       const float b = MODE != 0 ? b_s[tt] : 1.0f;
       const f32x4 v4 = *reinterpret_cast<const f32x4*>(&vs[tt][4 * cg]);
-      float part[4] = {0.f, 0.f, 0.f, 0.f};
+      float part[4] = {0.f, 0.f, 0.f, 0.f}, x[NI];
+      lds_row<NI>(&ks[tt][rr * NI], x);
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const float kk = ks[tt][rr + 16 * i], qq = qs[tt][rr + 16 * i];
+      for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          S[i][u] = a * S[i][u] + kk * (v4[u] * b);
-          part[u] += S[i][u] * qq;
-        }
-      }
+        for (int u = 0; u < 4; ++u) S[i][u] = a * S[i][u] + x[i] * (v4[u] * b);
+      lds_row<NI>(&qs[tt][rr * NI], x);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        part[u] += __shfl_xor(part[u], 16, 64);
-        part[u] += __shfl_xor(part[u], 32, 64);
-      }
-      if ((tid & 48) == 0) *reinterpret_cast<f32x4*>(&po_s[tt][wave][4 * cg]) = f32x4{part[0], part[1], part[2], part[3]};
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) part[u] += S[i][u] * x[i];
+      po_s[tt][wave][4 * cg + scatter_index4(tid)] = scatter_sum4(part);
       if (MODE == 1) {
         float pn = 0.f;
         if (tid < DP) {
@@ -344,7 +340,7 @@ __global__ __launch_bounds__(256, NI <= 8 ? 4 : 2) void outer_memory_rows_kernel
   }
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int r = rr + 16 * i;
+    const int r = rr * NI + i;
     if (in && r < dim) *reinterpret_cast<f32x4*>(sbase + (int64_t)r * vdim + col) = S[i];
   }
   if (MODE == 1 && tid < dim)
