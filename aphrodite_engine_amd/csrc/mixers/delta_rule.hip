@@ -432,6 +432,10 @@ extern "C" int aphro_gated_head_rms_norm(void* out, int64_t out_stride, const fl
   if (num_tokens == 0) return APHRO_OK;
   APHRO_CHECK(out && x && heads > 0 && vdim > 0 && out_stride >= (int64_t)heads * vdim && (!gate || gate_stride >= (int64_t)heads * vdim) &&
                   (act == 0 || act == 1), "gated_head_rms_norm: bad arguments (%d heads of %d)", heads, vdim);
+  if (group_rms_norm_launch(out, out_stride, x, weight, true, gate, gate_stride, num_tokens, heads * vdim, vdim, eps, 1.0f, act, dtype, (hipStream_t)stream)) {
+    APHRO_LAUNCH_CHECK();
+    return APHRO_OK;
+  }
   const int64_t units = num_tokens * heads;
   APHRO_CHECK((units + 3) / 4 <= 0x7fffffff, "gated_head_rms_norm: too many rows");
   MIX_DISPATCH_DTYPE(dtype, {

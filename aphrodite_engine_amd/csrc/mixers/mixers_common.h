@@ -27,6 +27,18 @@ __device__ __forceinline__ float wg_sum(float v, float* red) {
   return t;
 }
 
+// the same for an ``red`` that nothing in the kernel has used before: one barrier instead of two
+__device__ __forceinline__ float wg_sum_once(float v, float* red) {
+  v = wave_sum(v);
+  const int nw = (blockDim.x + 63) >> 6;
+  if (nw == 1) return v;
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float t = 0.f;
+  for (int w = 0; w < nw; ++w) t += red[w];
+  return t;
+}
+
 // Sums over groups of 2^LOG adjacent lanes with DPP moves (no LDS round trip): quad permutes for 2 and 4, the half-row and
 // row mirrors for 8 and 16 (after the quad steps every lane of a quad holds the quad's total, so the mirror partner brings
 // in the other half); every lane of a group ends with the group's total.  Wider groups finish with ds_bpermute shuffles.
@@ -111,6 +123,12 @@ __device__ __forceinline__ void lds_row(const float* p, float (&o)[NI]) {
     }
   }
 }
+
+// out [rows, n] = x / rms(x over its group) * out_scale * weight * act(gate), x fp32 dense, groups of neighbouring columns; weight [n], or
+// [group] shared by the groups (``shared``), or NULL; gate [rows, n] or NULL, act 0 sigmoid, 1 silu.  False: not a form that the launch serves
+// (groups of 8 to 512 numbers, a power of two, 16-byte pieces).
+bool group_rms_norm_launch(void* out, int64_t out_stride, const float* x, const void* weight, bool shared, const void* gate, int64_t gate_stride,
+                           int64_t rows, int n, int group, float eps, float out_scale, int act, int dtype, hipStream_t stream);
 
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + __expf(-z)); }
 __device__ __forceinline__ float silu_f(float z) { return z / (1.0f + __expf(-z)); }
