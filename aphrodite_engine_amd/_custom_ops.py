@@ -2350,6 +2350,38 @@ def rotary_embedding(positions: torch.Tensor, query: torch.Tensor,
         "rotary_embedding")
 
 
+@functools.lru_cache(maxsize=64)
+def _rotary_cache_served(head_size: int, rot_dim: int, is_neox: bool, block_size: int, x: int, dtype: int, kv_dtype: int) -> bool:
+    return bool(_lib.lib().aphro_rotary_cache_supported(head_size, rot_dim, 1 if is_neox else 0, block_size, x, dtype, kv_dtype))
+
+
+def rotary_embedding_and_cache(positions: torch.Tensor, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, head_size: int,
+                               cos_sin_cache: torch.Tensor, is_neox: bool, key_cache: torch.Tensor, value_cache: torch.Tensor,
+                               slot_mapping: torch.Tensor, kv_cache_dtype: str, k_scale: float, v_scale: float) -> bool:
+    """``rotary_embedding`` of query and key [T, heads * head_size] followed by ``reshape_and_cache`` of key and value, in one launch; False, and
+    nothing done, where that launch does not serve the geometry (heads of 64 or 128, all of it rotated in NeoX pairs, blocks of whole 16-token
+    pieces, rows of aligned 16-byte pieces)."""
+    _require_cuda(positions, query, key, value, cos_sin_cache, key_cache, value_cache, slot_mapping)
+    dt, kv = _dt(query), _kv(kv_cache_dtype)
+    slots = slot_mapping.flatten()
+    if not (query.dim() == key.dim() == value.dim() == 2 and query.dtype == key.dtype == value.dtype == cos_sin_cache.dtype
+            and slots.dtype == torch.int64 and positions.dtype == torch.int64 and positions.is_contiguous()
+            and query.stride(1) == key.stride(1) == value.stride(1) == 1 and cos_sin_cache.is_contiguous()
+            and key_cache.is_contiguous() and value_cache.is_contiguous() and value_cache.shape[3] == key_cache.shape[3]
+            and _rotary_cache_served(head_size, cos_sin_cache.shape[1], bool(is_neox), key_cache.shape[3], key_cache.shape[4], dt, kv)):
+        return False
+    qs, ks, vs = query.stride(0), key.stride(0), value.stride(0)
+    ptrs = [t.data_ptr() for t in (query, key, value, cos_sin_cache, key_cache, value_cache)]
+    num_tokens = positions.numel()
+    if (qs | ks | vs) & 7 or any(p & 15 for p in ptrs) or query.shape[0] != num_tokens or key.shape[0] != num_tokens or value.shape[0] != num_tokens \
+            or slots.numel() != num_tokens or key.shape[1] != value.shape[1] or key.shape[1] != key_cache.shape[1] * head_size:
+        return False
+    check(_lib.lib().aphro_rotary_cache(positions.data_ptr(), *ptrs, slots.data_ptr(), num_tokens, query.shape[1] // head_size,
+                                        key.shape[1] // head_size, head_size, key_cache.shape[3], qs, ks, vs, dt, kv, float(k_scale), float(v_scale),
+                                        _stream()), "rotary_embedding_and_cache")
+    return True
+
+
 # ---------------------------------------------------------------------------
 # _C_custom_ar::* (kernels/torch_bindings.cpp:506-536; aphrodite/_custom_ops.py:906-941) over
 # csrc/custom_all_reduce.hip.  Same names, argument order and meaning as the reference wrappers, so that

@@ -78,6 +78,8 @@ SIGNATURES = {
     "aphro_fused_add_rms_norm_pack": (I, [P, P, I, P, I, P, F, P, P, L, I, I, P]),
     "aphro_silu_and_mul_pack_slabs": (I, [P, I, P, P, L, I, I, P]),
     "aphro_silu_and_mul_pack": (I, [P, P, P, L, I, I, P]),
+    "aphro_rotary_cache_supported": (I, [I, I, I, I, I, I, I]),
+    "aphro_rotary_cache": (I, [P, P, P, P, P, P, P, P, L, I, I, I, I, L, L, L, I, I, F, F, P]),
     "aphro_rope_cache_scaled": (I, [P, L, P, I, P, P, P, P, I, I, P, P, P, P, L, I, I, I, I, I, I, I, F, F, P]),
     "aphro_rope_cache": (I, [P, L, P, I, P, P, I, I, P, P, P, P, L, I, I, I, I, I, I, I, F, F, P]),
     "aphro_gptq_dequant": (I, [P, P, P, P, P, L, L, L, I, I, I, P]),

@@ -177,8 +177,8 @@ class MI355XAttentionImpl:
 
     def forward(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
                 kv_cache: Optional[torch.Tensor], attn_metadata: MI355XAttentionMetadata,
-                k_scale: float = 1.0, v_scale: float = 1.0, attn_type=None) -> torch.Tensor:
-        """``attn_type``: the reference's Attention layer passes it by keyword (attention/layer.py:99-106); anything but
+                k_scale: float = 1.0, v_scale: float = 1.0, attn_type=None, cached: bool = False) -> torch.Tensor:
+        """``cached``: key and value are in the cache already (ops.rotary_embedding_and_cache).  ``attn_type``: the reference's Attention layer passes it by keyword (attention/layer.py:99-106); anything but
         AttentionType.DECODER is refused as by ROCmFlashAttentionImpl (rocm_flash_attn.py:395-399)."""
         if attn_type is not None and getattr(attn_type, "name", str(attn_type)) != "DECODER":
             raise NotImplementedError("Encoder self-attention and encoder/decoder cross-attention are not implemented for "
@@ -194,9 +194,10 @@ class MI355XAttentionImpl:
         if kv_cache is not None and kv_cache.numel() > 0:
             key_cache, value_cache = PagedAttention.split_kv_cache(
                 kv_cache, self.num_kv_heads, self.head_size)
-            PagedAttention.write_to_paged_cache(
-                key, value, key_cache, value_cache, attn_metadata.slot_mapping,
-                self.kv_cache_dtype, k_scale, v_scale)
+            if not cached:
+                PagedAttention.write_to_paged_cache(
+                    key, value, key_cache, value_cache, attn_metadata.slot_mapping,
+                    self.kv_cache_dtype, k_scale, v_scale)
 
         num_prefill_tokens = attn_metadata.num_prefill_tokens
         num_decode_tokens = attn_metadata.num_decode_tokens

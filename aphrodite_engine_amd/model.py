@@ -853,6 +853,18 @@ class LlamaDecoderLayer(nn.Module):
                 return False
         return True
 
+    def _attend(self, positions, q, k, v, kv_cache, attn_metadata, cos_sin):
+        """Rotary embedding, cache write and attention of a projection's rows."""
+        cached = False
+        if kv_cache is not None and kv_cache.numel() > 0:
+            from .attention.paged_attn import PagedAttention
+            key_cache, value_cache = PagedAttention.split_kv_cache(kv_cache, self.num_kv_heads, self.head_dim)
+            cached = ops.rotary_embedding_and_cache(positions, q, k, v, self.head_dim, cos_sin, True, key_cache, value_cache,
+                                                    attn_metadata.slot_mapping, self.attn.kv_cache_dtype, self.k_scale, self.v_scale)
+        if not cached:
+            ops.rotary_embedding(positions, q, k, self.head_dim, cos_sin, True)
+        return self.attn.forward(q, k, v, kv_cache, attn_metadata, self.k_scale, self.v_scale, cached=cached)
+
     def forward_prefill_fp8(self, positions, hidden, residual, first, kv_cache, attn_metadata, cos_sin):
         """One decoder layer on a prompt-sized batch, FP8 W8A8: returns the down_proj output (the next norm adds it to
         ``residual``, updated in place)."""
@@ -865,8 +877,7 @@ class LlamaDecoderLayer(nn.Module):
                                                      eps, static_scale=s_qkv)
         qkv = mm(qx, sx, self.qkv_proj)
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
-        ops.rotary_embedding(positions, q, k, self.head_dim, cos_sin, True)
-        attn_out = self.attn.forward(q, k, v, kv_cache, attn_metadata, self.k_scale, self.v_scale)
+        attn_out = self._attend(positions, q, k, v, kv_cache, attn_metadata, cos_sin)
         qa, sa = ops.scaled_fp8_quant(attn_out.view(attn_out.shape[0], self.q_size), s_o, use_per_token_if_dynamic=True)
         o = mm(qa, sa, self.o_proj)
         if self.tp > 1:
@@ -891,9 +902,7 @@ class LlamaDecoderLayer(nn.Module):
             ops.fused_add_rms_norm(hidden, residual, self.input_layernorm, eps)
         qkv = self.qkv_proj(hidden)
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
-        ops.rotary_embedding(positions, q, k, self.head_dim, cos_sin, True)
-        attn_out = self.attn.forward(q, k, v, kv_cache, attn_metadata,
-                                     self.k_scale, self.v_scale)
+        attn_out = self._attend(positions, q, k, v, kv_cache, attn_metadata, cos_sin)
         hidden = self._row_parallel(self.o_proj, attn_out)
         ops.fused_add_rms_norm(hidden, residual, self.post_attention_layernorm, eps)
         if self.is_moe:

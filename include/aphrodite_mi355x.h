@@ -379,6 +379,13 @@ int aphro_rope_cache(const void* qkv, int64_t qkv_stride, const float* slabs, in
                      const int64_t* slot_mapping, int64_t tokens, int num_heads,
                      int num_kv_heads, int head_size, int block_size, int x, int dtype,
                      int kv_dtype, float k_scale, float v_scale, void* stream);
+/* rotary_embedding of q and k in place and reshape_and_cache of k and v in one launch, any number of tokens (16-byte rows; the
+ * geometries of the first function: 1 served, 0 not) */
+int aphro_rotary_cache_supported(int head_size, int rot_dim, int is_neox, int block_size, int x, int dtype, int kv_dtype);
+int aphro_rotary_cache(const int64_t* positions, void* query, void* key, const void* value, const void* cos_sin_cache, void* key_cache,
+                       void* value_cache, const int64_t* slot_mapping, int64_t num_tokens, int num_heads, int num_kv_heads, int head_size,
+                       int block_size, int64_t q_stride, int64_t k_stride, int64_t v_stride, int dtype, int kv_dtype, float k_scale,
+                       float v_scale, void* stream);
 /* the same on an FP8 projection's raw slabs: an element is row_scale[token] * (col_scale[column] * sum) (row_scale NULL: 1) */
 int aphro_rope_cache_scaled(const void* qkv, int64_t qkv_stride, const float* slabs, int nslab, const float* row_scale,
                             const float* col_scale, const int64_t* positions, const void* cos_sin_cache, int rot_dim,
