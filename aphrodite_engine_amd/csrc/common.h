@@ -162,6 +162,24 @@ __device__ __forceinline__ typename T::storage from_f32_exact(float f) {
   return T::from_f32(f);
 }
 
+// Division of many numbers by one: the reciprocal once, then q = v r and two corrections by the exact remainder (Markstein's theorem: with r and
+// the first correction within half and one unit in the last place, the second is the rounded quotient) -- 6 operations for the 11 of a division
+// that has to scale its operands, one of them a quarter as fast.  The bits of v / s for finite v whose quotient is not below 2^-40 of all; smaller
+// ones stay as small, and keep their sign.  ``plain`` says that s is in the range where nothing overflows or underflows on the way.
+struct Divisor {
+  float s, r;
+  bool plain;
+};
+__device__ __forceinline__ Divisor divisor(float s, bool finite) {
+  return {s, 1.0f / s, (bool)__builtin_amdgcn_readfirstlane(finite && s >= 0x1p-60f && s <= 0x1p60f)};
+}
+__device__ __forceinline__ float divide_plain(float v, const Divisor& d) {
+  float q = v * d.r;
+  q = __builtin_fmaf(__builtin_fmaf(-q, d.s, v), d.r, q);
+  q = __builtin_fmaf(__builtin_fmaf(-q, d.s, v), d.r, q);
+  return __builtin_copysignf(q, v);
+}
+
 // ---- fp8 (OCP e4m3fn / e5m2, native on gfx950) ---------------------------------
 // word: 4 packed fp8; returns elements (2*hi_pair, 2*hi_pair+1) as f32.
 template <bool E5M2>

@@ -39,6 +39,22 @@ __device__ __forceinline__ uint32_t pack4_e4m3(const float (&v)[4], float s, boo
   return (uint32_t)w;
 }
 
+__device__ __forceinline__ uint32_t pack4_e4m3(const float (&v)[4], const Divisor& d) {
+  float a[4];
+  if (d.plain) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = divide_plain(v[i], d);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = v[i] / d.s;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) a[i] = __builtin_fmaxf(-FP8_MAX, __builtin_fminf(a[i], FP8_MAX));
+  int w = __builtin_amdgcn_cvt_pk_fp8_f32(a[0], a[1], 0, false);
+  w = __builtin_amdgcn_cvt_pk_fp8_f32(a[2], a[3], w, true);
+  return (uint32_t)w;
+}
+
 // out = fp8(x * (1 / *scale))   (common.cu:187-199)
 template <typename T>
 __global__ void static_quant_kernel(uint8_t* __restrict__ out, const typename T::storage* __restrict__ in,
@@ -206,15 +222,17 @@ __global__ __launch_bounds__(256) void per_token_quant_wave_kernel(uint8_t* __re
     }
   }
   m = wave_max(m);
+  const bool finite = m <= 3.402823466e38f;
   if (scale_ub) m = __builtin_fminf(m, *scale_ub);
   const float min_sf = 1.0f / (FP8_MAX * 512.f);
   const float s = __builtin_fmaxf(m / FP8_MAX, min_sf);
   if (lane == 0) scales[tok] = s;
+  const Divisor by = divisor(s, finite);
   uint32_t* o = reinterpret_cast<uint32_t*>(out + tok * hidden);
 #pragma unroll
   for (int j = 0; j < NQ; ++j) {
     const int q = j * 64 + lane;
-    if (q < quads) o[q] = pack4_e4m3(v[j], s, false);   // division: matches FBGemm (common.cu:243)
+    if (q < quads) o[q] = pack4_e4m3(v[j], by);   // division: matches FBGemm (common.cu:243)
   }
 }
 
