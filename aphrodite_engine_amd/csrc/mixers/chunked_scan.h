@@ -134,6 +134,36 @@ __device__ __forceinline__ void load8(const typename T::storage* __restrict__ ro
   }
 }
 
+// The same as they lie in memory: bf16 bits.
+template <bool VEC>
+__device__ __forceinline__ u16x8 load8_bits(const uint16_t* __restrict__ row, int at, int limit) {
+  u16x8 w = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  if constexpr (VEC) {
+    if (at < limit) w = *reinterpret_cast<const u16x8*>(row + at);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (at + i < limit) w[i] = row[at + i];
+  }
+  return w;
+}
+
+// An fp32 number as the sum of three bf16 ones, exactly (8 + 8 + 8 bits of its 24): a product with a bf16 number is then three products on the
+// 16-bit matrix cores, each exact, for a quarter of the time of the fp32 ones.  What is not finite stays in the first part.
+__device__ __forceinline__ void split3(float x, uint16_t (&p)[3]) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const bool fin = (u & 0x7f800000u) != 0x7f800000u;
+  const float h = __builtin_bit_cast(float, u & 0xffff0000u), r = fin ? x - h : 0.f;
+  const uint32_t ur = __builtin_bit_cast(uint32_t, r);
+  const float l = r - __builtin_bit_cast(float, ur & 0xffff0000u);
+  p[0] = (uint16_t)((u >> 16) | (x != x ? 0x40u : 0u));
+  p[1] = (uint16_t)(ur >> 16);
+  p[2] = (uint16_t)(__builtin_bit_cast(uint32_t, l) >> 16);
+}
+__device__ __forceinline__ f32x4 mfma16(u16x8 a, u16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
 inline bool rows_of_16_bytes(const void* p, int64_t stride, int head, int elem) {
   return ((uintptr_t)p & 15) == 0 && (stride * elem) % 16 == 0 && head % 8 == 0;
 }

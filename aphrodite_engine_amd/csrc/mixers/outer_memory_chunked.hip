@@ -13,7 +13,9 @@
 // What bounds it: the fp32 products (the matrix pipe is busy half of the time in launches 1 and 3) and the states between the chunks
 // (written once, read and written once, read once: dim x vdim x 4 bytes a chunk and head).  A scan is bound by the latency of its
 // token chain.  One portion of 4096 tokens, scan -> chunks: decay 8 x 64 x 128 1106 -> 60 us, mLSTM 4 x 128 x 256 2170 -> 113 us, state
-// space 64 x 128 x 64 1476 -> 274 us (128 heads: 1482 -> 575 us).
+// space 64 x 128 x 64 1476 -> 274 us (128 heads: 1482 -> 575 us).  With mLSTM's and the state space's bf16 inputs on the 16-bit units (the *16
+// kernels): mLSTM 4096 tokens 112 -> 95 us, state space 2000 tokens 146 -> 111, three portions of 300, 128 heads 171 -> 137; error against 64
+// bits 4.8e-7 -> 2.5e-7 and 1.05e-7 -> 0.94e-7.
 // Outputs lie as the products leave them: scores as K Q^T and results as V^T P^T, so that a score's registers are the next product's
 // operand and a lane holds four neighbouring value columns of one token.  Row pitches are 4 floats over a multiple of 32: the
 // eight lanes that a 16-byte LDS access serves at a time fall on all 32 banks.
@@ -209,6 +211,106 @@ __global__ __launch_bounds__(256) void om_chunk_update_kernel(OMChunk a) {
     for (int t = 0; t < CHUNK; t += 4) {
       const f32x4 x = *reinterpret_cast<const f32x4*>(&kt[tid * OMC_PITCH + t]);
       sum += (x[0] + x[1]) + (x[2] + x[3]);
+    }
+    a.un[((int64_t)blockIdx.x * p.heads + h) * DP + tid] = sum;
+  }
+}
+
+// The same where keys and values enter as the bf16 numbers they are (mLSTM, state space): U = sum_j k_j (w_j v_j)^T with the second factor in
+// three bf16 parts.  Keys that are not finite would meet a part that is zero: such a chunk multiplies in fp32, from the same LDS.
+template <int MODE, int DP, bool VEC>
+__global__ __launch_bounds__(256) void om_chunk_update16_kernel(OMChunk a) {
+  constexpr int PITCH = CHUNK + 8;
+  __shared__ __attribute__((aligned(16))) uint16_t kt[DP * PITCH];
+  __shared__ __attribute__((aligned(16))) uint16_t vt[3][OMC_COLS * PITCH];
+  __shared__ float ws[CHUNK];
+  const OuterMemory& p = a.p;
+  int s, c;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
+  const int slot = p.slot_of_seq[s];
+  if (slot < 0 || slot >= p.num_slots) return;
+  const int h = blockIdx.y, c0 = blockIdx.z * OMC_COLS, hk = MODE == 2 ? h / (p.heads / p.qk_heads) : h;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int cnt = min(CHUNK, p.q_len[s] - c * CHUNK);
+  const int64_t row0 = (int64_t)p.q_start[s] + c * CHUNK;
+  const int64_t row = row0 + min(lane, cnt - 1);
+  const uint16_t* kr = (const uint16_t*)p.k + row * p.k_stride + (int64_t)hk * p.dim;
+  const uint16_t* vr = (const uint16_t*)p.v + row * p.v_stride + (int64_t)h * p.vdim + c0;
+  u16x8 kx[DP / 32], vx[OMC_COLS / 32];
+#pragma unroll
+  for (int it = 0; it < DP / 32; ++it) kx[it] = load8_bits<VEC>(kr, wave * (DP / 4) + it * 8, p.dim);
+#pragma unroll
+  for (int it = 0; it < OMC_COLS / 32; ++it) vx[it] = load8_bits<VEC>(vr, wave * (OMC_COLS / 4) + it * 8, p.vdim - c0);
+  double la;
+  float b;
+  chunk_gate<BFloat, MODE>(a, h, row0, lane, cnt, la, b);
+  const double g = wave_incl_sum(la, lane), gend = __shfl(g, 63, 64);
+  const float w = exp2_d(gend - g) * b, all = exp2_d(gend);
+  if (blockIdx.z == 0 && tid == 0) a.total[(int64_t)blockIdx.x * p.heads + h] = all;
+  if (tid < CHUNK) ws[tid] = lane < cnt ? w : 0.f;
+  bool odd = false;                                                      // a key that is not finite
+#pragma unroll
+  for (int it = 0; it < DP / 32; ++it)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint16_t x = lane < cnt ? kx[it][i] : (uint16_t)0;
+      odd |= (x & 0x7f80u) == 0x7f80u;
+      kt[(wave * (DP / 4) + it * 8 + i) * PITCH + lane] = x;
+    }
+#pragma unroll
+  for (int it = 0; it < OMC_COLS / 32; ++it)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      uint16_t part[3];
+      split3(lane < cnt ? BFloat::to_f32(vx[it][i]) * w : 0.f, part);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) vt[n][(wave * (OMC_COLS / 4) + it * 8 + i) * PITCH + lane] = part[n];
+    }
+  odd = __syncthreads_or(odd);
+  const int li = lane & 15, lg = lane >> 4;
+  const int nct = min(OMC_COLS / 16, (p.vdim - c0 + 15) >> 4);
+  constexpr int DT = DP / 64;                              // 16-row tiles of a wave
+  f32x4 acc[DT][OMC_COLS / 16] = {};
+#pragma unroll
+  for (int kk = 0; kk < CHUNK / 32; ++kk) {
+    u16x8 av[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) av[dt] = *reinterpret_cast<const u16x8*>(&kt[((wave * DT + dt) * 16 + li) * PITCH + 32 * kk + 8 * lg]);
+#pragma unroll
+    for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
+      if (ct >= nct) break;
+      u16x8 bv[3];
+#pragma unroll
+      for (int n = 0; n < 3; ++n) bv[n] = *reinterpret_cast<const u16x8*>(&vt[n][(ct * 16 + li) * PITCH + 32 * kk + 8 * lg]);
+      if (!odd) {
+#pragma unroll
+        for (int n = 2; n >= 0; --n)
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) acc[dt][ct] = mfma16(av[dt], bv[n], acc[dt][ct]);
+      } else {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+          const float x = (BFloat::to_f32(bv[2][m]) + BFloat::to_f32(bv[1][m])) + BFloat::to_f32(bv[0][m]);
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) acc[dt][ct] = mfma4(BFloat::to_f32(av[dt][m]), x, acc[dt][ct]);
+        }
+      }
+    }
+  }
+  float* u = a.u + (((int64_t)blockIdx.x * p.heads + h) * a.vpad + c0) * DP;
+#pragma unroll
+  for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
+    if (ct >= nct) break;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      *reinterpret_cast<f32x4*>(&u[(ct * 16 + li) * DP + (wave * DT + dt) * 16 + 4 * lg]) = acc[dt][ct];
+  }
+  if (MODE == 1 && blockIdx.z == 0 && tid < DP) {
+    float sum = 0.f;
+    for (int t = 0; t < CHUNK; t += 8) {
+      const u16x8 x = *reinterpret_cast<const u16x8*>(&kt[tid * PITCH + t]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum += BFloat::to_f32(x[i]) * ws[t + i];
     }
     a.un[((int64_t)blockIdx.x * p.heads + h) * DP + tid] = sum;
   }
@@ -473,6 +575,179 @@ __global__ __launch_bounds__(256) void om_chunk_out_kernel(OMChunk a) {
   }
 }
 
+// The same where keys, queries and values enter as the bf16 numbers they are (mLSTM, state space): scores are bf16 products as they stand, the
+// weights that meet the values go in three bf16 parts; only the state's product stays on the fp32 units.
+template <int MODE, int DP, bool VEC>
+__global__ __launch_bounds__(256, MODE == 2 ? 4 : 3) void om_chunk_out16_kernel(OMChunk a) {
+  constexpr int KP = DP + 8, VP = CHUNK + 8, SCORES = CHUNK * (CHUNK + 1) * 4, KEYS = CHUNK * KP * 2;
+  __shared__ __attribute__((aligned(16))) unsigned char room[KEYS > SCORES ? KEYS : SCORES];      // keys; for values that are not finite, then: the scores
+  __shared__ __attribute__((aligned(16))) uint16_t vt[OMC_COLS * VP];
+  __shared__ double gs[CHUNK];
+  __shared__ float bs[CHUNK];
+  uint16_t* ks = reinterpret_cast<uint16_t*>(room);
+  const OuterMemory& p = a.p;
+  int s, c;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
+  const int slot = p.slot_of_seq[s];
+  if (slot < 0 || slot >= p.num_slots) return;
+  const int h = blockIdx.y, c0 = blockIdx.z * OMC_COLS, hk = MODE == 2 ? h / (p.heads / p.qk_heads) : h;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
+  const int cnt = min(CHUNK, p.q_len[s] - c * CHUNK);
+  const int64_t row0 = (int64_t)p.q_start[s] + c * CHUNK;
+  const int64_t row = row0 + min(lane, cnt - 1);
+  const uint16_t* kr = (const uint16_t*)p.k + row * p.k_stride + (int64_t)hk * p.dim;
+  const uint16_t* vr = (const uint16_t*)p.v + row * p.v_stride + (int64_t)h * p.vdim + c0;
+  u16x8 kx[DP / 32], vx[OMC_COLS / 32];
+#pragma unroll
+  for (int it = 0; it < DP / 32; ++it) kx[it] = load8_bits<VEC>(kr, wave * (DP / 4) + it * 8, p.dim);
+#pragma unroll
+  for (int it = 0; it < OMC_COLS / 32; ++it) vx[it] = load8_bits<VEC>(vr, wave * (OMC_COLS / 4) + it * 8, p.vdim - c0);
+  const int qt = (wave + blockIdx.x + blockIdx.y) & 3, qi = qt * 16 + li;      // (which queries a wave has: as above)
+  u16x8 q[DP / 32];
+  {
+    const uint16_t* qr = (const uint16_t*)p.q + (row0 + min(qi, cnt - 1)) * p.q_stride + (int64_t)hk * p.dim;
+#pragma unroll
+    for (int kk = 0; kk < DP / 32; ++kk) q[kk] = load8_bits<VEC>(qr, 32 * kk + 8 * lg, p.dim);
+  }
+  const int nct = min(OMC_COLS / 16, (p.vdim - c0 + 15) >> 4);
+  const float* st = a.u + (((int64_t)blockIdx.x * p.heads + h) * a.vpad + c0) * DP;
+  f32x4 acc[OMC_COLS / 16] = {};
+#pragma unroll
+  for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
+    if (ct >= nct) break;
+    const float* sr = st + (ct * 16 + li) * DP + 8 * lg;
+#pragma unroll
+    for (int kk = 0; kk < DP / 32; ++kk) {
+      const f32x4 s0 = *reinterpret_cast<const f32x4*>(sr + 32 * kk), s1 = *reinterpret_cast<const f32x4*>(sr + 32 * kk + 4);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) acc[ct] = mfma4(s0[m], BFloat::to_f32(q[kk][m]), acc[ct]);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) acc[ct] = mfma4(s1[m], BFloat::to_f32(q[kk][4 + m]), acc[ct]);
+    }
+  }
+  bool odd = false;                                                      // a value that is not finite
+#pragma unroll
+  for (int it = 0; it < DP / 32; ++it)
+    *reinterpret_cast<u16x8*>(&ks[lane * KP + wave * (DP / 4) + it * 8]) = lane < cnt ? kx[it] : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int it = 0; it < OMC_COLS / 32; ++it)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint16_t x = lane < cnt ? vx[it][i] : (uint16_t)0;
+      odd |= (x & 0x7f80u) == 0x7f80u;
+      vt[(wave * (OMC_COLS / 4) + it * 8 + i) * VP + lane] = x;
+    }
+  if (wave == 0) {
+    double la;
+    float b;
+    chunk_gate<BFloat, MODE>(a, h, row0, lane, cnt, la, b);
+    gs[lane] = wave_incl_sum(la, lane);
+    bs[lane] = b;
+  }
+  odd = __syncthreads_or(odd);
+  const double gq = gs[qi];
+  const float scale = MODE == 1 ? p.q_scale : 1.f, eq = exp2_d(gq) * scale;
+#pragma unroll
+  for (int ct = 0; ct < OMC_COLS / 16; ++ct)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[ct][r] *= eq;
+  float nq = 0.f;                                                       // mLSTM: the lane's part of n . q
+  if constexpr (MODE == 1) {
+    const float* nb = a.un + ((int64_t)blockIdx.x * p.heads + h) * DP + 8 * lg;
+#pragma unroll
+    for (int kk = 0; kk < DP / 32; ++kk)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) nq += BFloat::to_f32(q[kk][i]) * nb[32 * kk + i];
+    nq *= eq;
+  }
+  // the chunk's own tokens up to the query's, 32 a step: lane group lg has tokens 4 lg .. 4 lg + 3 of either half
+  f32x4 pr[CHUNK / 16];
+#pragma unroll
+  for (int jp = 0; jp < CHUNK / 32; ++jp) {
+    if (2 * jp > qt) break;
+    u16x8 part[3];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int jt = 2 * jp + half;
+      f32x4 sc = {};
+      if (jt <= qt) {
+#pragma unroll
+        for (int kk = 0; kk < DP / 32; ++kk) sc = mfma16(*reinterpret_cast<const u16x8*>(&ks[(jt * 16 + li) * KP + 32 * kk + 8 * lg]), q[kk], sc);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = jt * 16 + 4 * lg + r;
+        float w = 0.f;
+        if (j <= qi) w = sc[r] * scale * (exp2_d(gq - gs[j]) * bs[j]);
+        pr[jt][r] = w;
+        if (MODE == 1) nq += w;
+        uint16_t x[3];
+        split3(w, x);
+#pragma unroll
+        for (int n = 0; n < 3; ++n) part[n][4 * half + r] = x[n];
+      }
+    }
+    if (!odd) {
+#pragma unroll
+      for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
+        if (ct >= nct) break;
+        const uint16_t* vp = &vt[(ct * 16 + li) * VP + 32 * jp + 4 * lg];
+        const u32x2 lo = *reinterpret_cast<const u32x2*>(vp), hi = *reinterpret_cast<const u32x2*>(vp + 16);
+        const u16x8 vv = __builtin_bit_cast(u16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+#pragma unroll
+        for (int n = 2; n >= 0; --n) acc[ct] = mfma16(vv, part[n], acc[ct]);
+      }
+    }
+  }
+  if (odd) {
+    // zero times a value that is not finite is not zero: a token behind the query must not be multiplied at all
+    __syncthreads();                                                     // every wave is through with the keys
+    float* ps = reinterpret_cast<float*>(room);                          // [64 queries][64 + 1]
+#pragma unroll
+    for (int jt = 0; jt < CHUNK / 16; ++jt)
+      if (jt <= qt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ps[qi * (CHUNK + 1) + jt * 16 + 4 * lg + r] = pr[jt][r];
+    __syncthreads();
+#pragma unroll
+    for (int ct = 0; ct < OMC_COLS / 16; ++ct)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float sum = 0.f;
+        for (int j = 0; j <= qi; ++j) sum += ps[qi * (CHUNK + 1) + j] * BFloat::to_f32(vt[(ct * 16 + 4 * lg + r) * VP + j]);
+        acc[ct][r] += sum;
+      }
+  }
+  float inv = 1.f;
+  if constexpr (MODE == 1) {
+    nq += __shfl_xor(nq, 16, 64);
+    nq += __shfl_xor(nq, 32, 64);
+    const float em = a.em[(int64_t)h * p.num_tokens + row0 + min(qi, cnt - 1)];
+    inv = fmaxf(fabsf(nq), em) + 1e-6f;
+  }
+  if (qi >= cnt) return;
+  const float skip = MODE == 2 ? p.skip[h] : 0.f;
+  float* o = p.out + (row0 + qi) * ((int64_t)p.heads * p.vdim) + (int64_t)h * p.vdim + c0;
+#pragma unroll
+  for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
+    if (ct >= nct) break;
+    const int e = ct * 16 + 4 * lg;
+    f32x4 x = acc[ct];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (MODE == 1) x[r] = x[r] / inv;
+      if (MODE == 2) x[r] += skip * BFloat::to_f32(vt[(e + r) * VP + qi]);
+    }
+    if ((p.vdim & 3) == 0) {
+      if (c0 + e < p.vdim) *reinterpret_cast<f32x4*>(o + e) = x;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (c0 + e + r < p.vdim) o[e + r] = x[r];
+    }
+  }
+}
+
 // Sizes of the workspace's parts for so many chunks, in floats: U, the normaliser's, decays, gates (of all tokens).
 static void om_chunk_parts(const OuterMemory& p, int64_t chunks, int64_t (&n)[4]) {
   const int64_t dp = p.dim <= 64 ? 64 : 128, vpad = (p.vdim + 15) / 16 * 16;
@@ -494,9 +769,12 @@ static void om_chunk_launch(OMChunk a, int64_t chunks) {
   const unsigned items = (unsigned)a.vpad * (DP / 4) + (MODE == 1 ? DP : 0);
   if (MODE == 1) hipLaunchKernelGGL((om_gates_kernel<T>), dim3((unsigned)p.num_seqs, (unsigned)p.heads), dim3(1024), 0, p.stream, a);
   for (; a.chunk0 < chunks; a.chunk0 += a.span) {
-    hipLaunchKernelGGL((om_chunk_update_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
+    constexpr bool B16 = sizeof(typename T::storage) == 2 && MODE != 0;
+    if constexpr (B16) hipLaunchKernelGGL((om_chunk_update16_kernel<MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
+    else hipLaunchKernelGGL((om_chunk_update_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
     hipLaunchKernelGGL((om_chunk_carry_kernel<MODE, DP>), dim3((items + 63) / 64, (unsigned)p.heads, (unsigned)p.num_seqs), dim3(64), 0, p.stream, a);
-    hipLaunchKernelGGL((om_chunk_out_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
+    if constexpr (B16) hipLaunchKernelGGL((om_chunk_out16_kernel<MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
+    else hipLaunchKernelGGL((om_chunk_out_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
   }
 }
 
