@@ -26,6 +26,22 @@ __global__ void paged_kv_write_kernel(typename T::storage* __restrict__ k_cache,
   for (int i = threadIdx.x; i < vd; i += blockDim.x) v_cache[slot * vd + i] = vr[i];
 }
 
+// The same in 16-byte pieces, whatever the numbers: pk pieces of a token's keys, pv of its values.  4096 tokens of 512 + 512 bf16 numbers, us before /
+// here: 5.4 / 4.4, 32 of 1024 + 1024 4.2 / 2.9.
+__global__ __launch_bounds__(256) void paged_kv_write_pieces_kernel(u32x4* __restrict__ k_cache, u32x4* __restrict__ v_cache, const u32x4* __restrict__ k,
+                                                                    int64_t k_stride, const u32x4* __restrict__ v, int64_t v_stride,
+                                                                    const int64_t* __restrict__ slots, int64_t num_tokens, int pk, int pv,
+                                                                    int64_t num_slots) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, t = i / (pk + pv);
+  if (t >= num_tokens) return;
+  const int piece = (int)(i - t * (pk + pv));
+  const u32x4 x = piece < pk ? k[t * k_stride + piece] : v[t * v_stride + piece - pk];
+  const int64_t slot = slots[t];
+  if (slot < 0 || slot >= num_slots) return;
+  if (piece < pk) k_cache[slot * pk + piece] = x;
+  else v_cache[slot * pv + piece - pk] = x;
+}
+
 template <typename T>
 __device__ __forceinline__ float dot_row(const float* __restrict__ qsh, const typename T::storage* __restrict__ kr, int dim) {
   float d0 = 0.f, d1 = 0.f;
@@ -173,6 +189,16 @@ extern "C" int aphro_paged_kv_write(void* k_cache, void* v_cache, const void* k,
               "paged_kv_write: bad arguments");
   const int kd = kv_heads * dim, vd = kv_heads * vdim;
   APHRO_CHECK(k_stride >= kd && v_stride >= vd, "paged_kv_write: row strides smaller than the rows");
+  const int per = dtype == APHRO_BF16 ? 8 : 4;               // numbers of 16 bytes
+  const auto al16 = [](const void* ptr) { return ((uintptr_t)ptr & 15) == 0; };
+  const int64_t blocks = (num_tokens * ((kd + vd) / per) + 255) / 256;
+  if ((dtype == APHRO_BF16 || dtype == APHRO_F32) && kd % per == 0 && vd % per == 0 && k_stride % per == 0 && v_stride % per == 0 && al16(k_cache) &&
+      al16(v_cache) && al16(k) && al16(v) && blocks <= 0x7fffffff) {
+    hipLaunchKernelGGL(paged_kv_write_pieces_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (u32x4*)k_cache, (u32x4*)v_cache,
+                       (const u32x4*)k, k_stride / per, (const u32x4*)v, v_stride / per, slots, num_tokens, kd / per, vd / per, num_slots);
+    APHRO_LAUNCH_CHECK();
+    return APHRO_OK;
+  }
   MIX_DISPATCH_DTYPE(dtype, {
     typedef typename T::storage S;
     hipLaunchKernelGGL((paged_kv_write_kernel<T>), dim3((unsigned)num_tokens), dim3(128), 0, (hipStream_t)stream,

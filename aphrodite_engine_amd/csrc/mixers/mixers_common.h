@@ -126,7 +126,7 @@ __device__ __forceinline__ void lds_row(const float* p, float (&o)[NI]) {
 
 // out [rows, n] = x / rms(x over its group) * out_scale * weight * act(gate), x fp32 dense, groups of neighbouring columns; weight [n], or
 // [group] shared by the groups (``shared``), or NULL; gate [rows, n] or NULL, act 0 sigmoid, 1 silu.  False: not a form that the launch serves
-// (groups of 8 to 512 numbers, a power of two, 16-byte pieces).
+// (groups of whole 8s up to 8192, 16-byte pieces).
 bool group_rms_norm_launch(void* out, int64_t out_stride, const float* x, const void* weight, bool shared, const void* gate, int64_t gate_stride,
                            int64_t rows, int n, int group, float eps, float out_scale, int act, int dtype, hipStream_t stream);
 

@@ -69,7 +69,7 @@ __device__ __forceinline__ void sc_store8(typename T::storage* p, const float* v
 // first, then what the rows of the tile are (uniform over the workgroup), all at once, and the rows wait in the registers as they lay in
 // memory.  A tile whose taps lie in one segment turns every number to fp32 once.  With the segments looked up row by row between the rows'
 // stores and 4 rows a thread, 4 taps with silu, us before / here (the states' launch, 5, included): 6144 channels, 2000 rows beside 24 single
-// ones 30.3 / 27.2, 4096 rows 40.8 / 33.9, 32 single rows 15.3 / 9.9; 12288 channels, 2560 rows 47.0 / 37.5.
+// ones 30.3 / 22.2, 4096 rows 40.8 / 29.3, 32 single rows 15.3 / 9.4; 12288 channels, 2560 rows 47.0 / 33.8 (bf16 by the converter).
 template <typename T, int TAPS, int TOK>
 __global__ __launch_bounds__(256) void short_conv_vec8_kernel(
     typename T::storage* __restrict__ q_out, int64_t q_out_stride, typename T::storage* __restrict__ k_cache,
@@ -235,11 +235,11 @@ extern "C" int aphro_short_conv(void* q_out, int64_t q_out_stride, void* k_cache
   const auto al16 = [](const void* ptr) { return ((uintptr_t)ptr & 15) == 0; };
   const bool vec = taps >= 2 && taps <= 4 && (cq & 7) == 0 && (ck & 7) == 0 && (cv & 7) == 0 && (u_stride & 7) == 0 &&
                    (q_out_stride & 7) == 0 && al16(u) && al16(w) && al16(bias) && al16(q_out) && al16(k_cache) && al16(v_cache) && al16(state);
-  // rows a thread: 8 where that leaves two workgroups for every CU (each further row saves re-reading TAPS - 1 of them), else 2 (48 rows of
-  // 6144 channels 7.7 us, with 4 10.6)
+  // rows a thread: 4 where that leaves four workgroups for every CU, else 2 (48 rows of 6144 channels 7.7 us, with 4 10.6).  With 8 the chip is
+  // filled once and loads, sums and stores take turns: 2024 rows of 6144 24.8 us, with 4 22.2; 4096 rows 30.0 / 29.3
   const int threads = C / 8 >= 256 ? 256 : (C / 8 + 63) / 64 * 64;
   const unsigned parts = (unsigned)((C / 8 + threads - 1) / threads);
-  const bool tall = (num_tokens + 7) / 8 * parts >= 2 * device_cu_count();
+  const bool tall = (num_tokens + 3) / 4 * parts >= 4 * device_cu_count();
 #define SC_VEC_TOK(TAPS, TOK)                                                                                                  \
   hipLaunchKernelGGL((short_conv_vec8_kernel<T, TAPS, TOK>), dim3((unsigned)((num_tokens + TOK - 1) / TOK), parts), dim3(threads), 0, (hipStream_t)stream,  \
                      (S*)q_out, q_out_stride, (S*)k_cache,                                                                     \
@@ -247,7 +247,7 @@ extern "C" int aphro_short_conv(void* q_out, int64_t q_out_stride, void* k_cache
                      q_start, ctx_len, seq_of_token, num_tokens, cq, ck, cv, act)
 #define SC_VEC(TAPS)                 \
   do {                               \
-    if (tall) SC_VEC_TOK(TAPS, 8);   \
+    if (tall) SC_VEC_TOK(TAPS, 4);   \
     else SC_VEC_TOK(TAPS, 2);        \
   } while (0)
   MIX_DISPATCH_DTYPE(dtype, {

@@ -48,3 +48,20 @@ def test_embedding_rows(dtype, width):
     copy = torch.empty(5, width, device=DEV, dtype=dtype)
     got = mops.embed_scale(table, ids, 1.5, copy=copy)
     assert torch.equal(got, table[ids].float() * 1.5) and torch.equal(copy, got.to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("d,e,shift", [(128, 128, 0), (8, 24, 0), (20, 4, 0), (4, 6, 0), (64, 32, 1)])
+def test_paged_kv_write(dtype, d, e, shift):
+    """paged_kv_write in 16-byte pieces and, where rows are none, number by number: every slot gets its row, padding and slots outside none."""
+    from aphrodite_engine_amd import mixer_ops as mops
+    T, G, nb, bs = 37, 2, 9, 8
+    k, v = (torch.randn(T, G * n + 8 + shift, device=DEV).to(dtype)[:, shift:shift + G * n] for n in (d, e))
+    kc, vc = (torch.full((nb, bs, G, n), 7.0, device=DEV, dtype=dtype) for n in (d, e))
+    slots = torch.randperm(nb * bs, device=DEV)[:T].contiguous()
+    slots[5], slots[6] = -1, nb * bs
+    want_k, want_v = kc.view(-1, G * d).clone(), vc.view(-1, G * e).clone()
+    ok = [i for i in range(T) if i not in (5, 6)]
+    want_k[slots[ok]], want_v[slots[ok]] = k[ok], v[ok]
+    mops.paged_kv_write(kc, vc, k, v, slots)
+    assert torch.equal(kc.view(-1, G * d), want_k) and torch.equal(vc.view(-1, G * e), want_v)
