@@ -285,7 +285,7 @@ def flash_attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 # context_attention_fwd without host-side length hints: a workspace bound of new tokens + block-table capacity per sequence
 # is used without a device sync while it stays below this many bytes
 CONTEXT_ATTN_NOSYNC_WS_BYTES = 256 << 20
-CONTEXT_ATTN_GATHER_MIN_LEN = 1024     # (kept for callers that imported it: the third-generation kernel's threshold)
+CONTEXT_ATTN_GATHER_MIN_LEN = 1024     # (kept for callers that imported it)
 
 
 def context_attention_fwd(q, k, v, o, kv_cache_dtype: str, k_cache, v_cache, b_loc, b_start_loc,

@@ -446,378 +446,6 @@ __global__ __launch_bounds__(NWV * 64) void flash_attn_varlen_v2_kernel(FAParams
 }
 
 // ---------------------------------------------------------------------------
-// Third-generation prefill kernel (hd 128, sequences >= 1024): 8 waves x 32 query rows = 256 rows per workgroup,
-// 64-key tiles, 32x32x16 MFMA.  the second-generation kernel is VALU-issue bound at 7.4 VALU per
-// 16x16x32 MFMA; this one spends ~150 VALU per 32 MFMAs of 32 cycles:
-//   * swapped QK^T on 32x32 tiles (S^T = K . Q^T): a lane holds 32 of the 64 scores of ONE query row, so the row
-//     maximum / sum are 31 lane-local ops + one half-wave exchange (v_permlane32_swap), no LDS;
-//   * softmax in the log2 domain straight off the accumulators: p = exp2(fma(s, scale*log2e, -m)), 2 VALU per score;
-//   * P -> 16-bit with packed hardware converts, redistributed into PV B-operand fragments by 8 permlane32_swap per
-//     32 keys (the MFMA C layout interleaves the two half-waves' keys in groups of 4);
-//   * K and V tiles go global -> LDS with direct-to-LDS loads (no VGPR round trip, no address VALU in the loop),
-//     a 3-deep ring, one barrier per tile; the next tile's QK^T shares a straight-line block with this tile's softmax.  The LDS image is chosen on the SOURCE side (lane L of a 1 KiB piece
-//     fetches whatever must live at byte 16 L): K rows XOR-swizzled by key & 15 for conflict-free ds_read_b128
-//     fragments; V in [16-byte d-chunk][4 keys] order inside each 4-key piece, which makes every
-//     ds_read_b64_tr_b16 (transposing read: 4 keys of one d per lane) of a PV A-operand hit 64 distinct banks;
-//   * O leaves through a wave-private LDS transpose as full 256-byte rows.
-// Keys beyond the sequence are fetched as zeros by the buffer descriptor's bounds check.
-// ---------------------------------------------------------------------------
-
-
-template <typename T>
-__global__ __launch_bounds__(512) void flash_attn_varlen_v3_kernel(FAParams p) {
-  constexpr int HD = 128, BM = 256, BN = 64;
-  constexpr bool BF = __is_same(T, BFloat);
-  constexpr int KT = BN * HD * 2;           // bytes of one K (or V) tile: 16 KiB
-  constexpr int STAGE = 2 * KT;
-  extern __shared__ __attribute__((aligned(16))) unsigned char fa_smem[];   // ring of 3 x [K tile | V tile], then 8 x 8 KiB of Q fragments
-
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kh = lane >> 5, l31 = lane & 31;
-  // ---- which (sequence, head, 256-row query tile) is this workgroup -------------------------------------------------------
-  // Workgroup b runs on XCD b % 8 (round-robin dispatch).  All query heads of ONE kv head, and all their query tiles, go
-  // to the same XCD and walk the K/V tiles from key 0 upwards roughly in step: a K/V tile is pulled into that XCD's
-  // 4 MiB L2 once and the other workgroups hit it (K + V of one kv head at 8192 tokens = 4 MiB).  With the plain
-  // (tile, head, sequence) grid every XCD streamed every kv head: the staging alone ran at the 6 TB/s MALL/HBM rate and
-  // cost 0.37 of 1.06 ms at T = 8192 (tools/fa_lab.hip).  Within an XCD: heavy (late) query tiles first.
-  int head, seq, qt_rev;
-  {
-    const int G = p.num_heads / p.num_kv_heads;
-    const int per_group = G * p.nqt_max;                  // workgroups of one (sequence, kv head)
-    const int b = blockIdx.x;
-    int group, r;
-    if (p.xcd_remap) { group = (b % 8) + 8 * ((b / 8) / per_group); r = (b / 8) % per_group; }
-    else { group = b / per_group; r = b % per_group; }
-    seq = group / p.num_kv_heads;
-    head = (group % p.num_kv_heads) * G + r % G;
-    qt_rev = r / G;
-  }
-  const int kvh = head / (p.num_heads / p.num_kv_heads);
-  // queries [s0q, s0q + qlen) and keys [s0, s0 + len): the same rows for plain prefill; with a cached context in front
-  // (cu_seqlens_k given) the keys are context + new tokens and query row i sits at key position i + off, off = len - qlen
-  const int s0q = p.cu_seqlens[seq];
-  const int qlen = p.cu_seqlens[seq + 1] - s0q;
-  const int s0 = p.cu_seqlens_k ? p.cu_seqlens_k[seq] : s0q;
-  const int len = p.cu_seqlens_k ? p.cu_seqlens_k[seq + 1] - s0 : qlen;
-  const int off = len - qlen;
-  const int nqt = (qlen + BM - 1) / BM;
-  const int qt = nqt - 1 - qt_rev;            // heavy (late) tiles first
-  if (qt < 0) return;
-  const int q0 = qt * BM;
-  const int wq0 = q0 + 32 * wave;
-  const int qrow = wq0 + l31;
-
-  // ---- Q fragments (B operand of S^T = K . Q^T): lane (q = l31, kh) holds d = 16 ks + 8 kh .. + 7.  They live in LDS, not
-  // in 32 VGPRs: the lane that wrote a fragment is the one that reads it back (8 ds_read_b128 per tile), which is what
-  // lets two score tiles + the output accumulators + the P fragments fit in 256 registers without spills.
-  unsigned char* qlds = fa_smem + 3 * STAGE + wave * 8192;
-  const int qaddr = l31 * 256 + ((kh ^ (l31 & 15)) << 4);          // chunk 2 ks + kh of row l31, XOR-swizzled like K
-  {
-    const uint16_t* qp = (const uint16_t*)p.q + (size_t)(s0q + min(qrow, qlen - 1)) * p.q_stride + (size_t)head * HD + 8 * kh;
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks)
-      *reinterpret_cast<u32x4*>(qlds + (qaddr ^ (ks << 5))) = *reinterpret_cast<const u32x4*>(qp + 16 * ks);
-  }
-  const float slope2 = (p.alibi ? p.alibi[head] : 0.f) * 1.44269504088896f;
-  const float c2 = p.scale * 1.44269504088896f;
-
-  // ---- K / V staging: buffer descriptors over this sequence's rows of this kv head (reads past the end return 0) -------
-  const uint16_t* kbase = (const uint16_t*)p.k + (size_t)s0 * p.k_stride + (size_t)kvh * HD;
-  const uint16_t* vbase = (const uint16_t*)p.v + (size_t)s0 * p.v_stride + (size_t)kvh * HD;
-  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kbase), 0,
-      (uint32_t)(((size_t)(len - 1) * p.k_stride + HD) * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(vbase), 0,
-      (uint32_t)(((size_t)(len - 1) * p.v_stride + HD) * 2), 0x00020000);
-  // a wave stages pieces 2 wave, 2 wave + 1 (4 keys = 1 KiB each) of both tiles.
-  // K piece: lane L -> key 4 c + (L >> 4), LDS slot L & 15 holds d-chunk slot ^ (key & 15)
-  // V piece: lane L -> key 4 c + (L & 3), d-chunk L >> 2  (image [d-chunk][key] inside the piece)
-  int k_voff[2], v_voff[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int c = 2 * wave + j;
-    const int kk = 4 * c + (lane >> 4);
-    k_voff[j] = (int)(kk * p.k_stride * 2) + (((lane & 15) ^ (kk & 15)) << 4);
-    const int vk = 4 * c + (lane & 3);
-    v_voff[j] = (int)(vk * p.v_stride * 2) + ((lane >> 2) << 4);
-  }
-  auto stage = [&](int buf, int t0) {
-    unsigned char* sk = fa_smem + buf * STAGE;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int kv = k_voff[j], vv = v_voff[j];     // (local copies: see wna16_gemm_large.hip on the hipcc host-stub bug)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (fa_lds_ptr)(sk + (2 * wave + j) * 1024), 16, kv, (int)(t0 * p.k_stride * 2), 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (fa_lds_ptr)(sk + KT + (2 * wave + j) * 1024), 16, vv, (int)(t0 * p.v_stride * 2), 0, 0);
-    }
-  };
-  // fragment read addresses (lane-invariant parts)
-  //  K: key = 32 b + l31, d-chunk 2 ks + kh -> l31 * 256 + (((2 ks + kh) ^ (l31 & 15)) << 4) = kaddr ^ (ks << 5)
-  const int kaddr = l31 * 256 + ((kh ^ (l31 & 15)) << 4);
-  //  V (transposing read; 16-lane group g, lane i of it): piece 4 ks + 2 kh + h, key i >> 2 of it,
-  //  d = 32 db + 16 (g & 1) + 4 (i & 3)
-  const int vaddr = KT + (2 * kh) * 1024 + ((((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) * 4 + ((lane & 15) >> 2)) << 4)) + ((lane & 1) << 3);
-
-  f32x16 o[4];
-#pragma unroll
-  for (int db = 0; db < 4; ++db)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
-  float m_run = -1e30f, l_run = 0.f;          // log2-domain running maximum; this lane's share of the row sum
-
-  const int kv_end = p.causal ? min(len, q0 + BM + off) : len;
-  const int ntile = (kv_end + BN - 1) / BN;
-  // tiles this wave computes (causal: up to its diagonal), and how many of them need no masking for its 32 rows
-  const int L = p.causal ? min(ntile, (wq0 + off + 31) / BN + 1) : ntile;
-  const int F = slope2 != 0.f ? 0 : min(L, p.causal ? min((wq0 + off + 1) / BN, len / BN) : len / BN);
-
-  // ---- pieces of a tile ------------------------------------------------------------------------------------------------------
-  // S^T = K . Q^T of tile `it` into dst: lane (q = l31) gets keys 32 b + 8 (r >> 2) + 4 kh + (r & 3).  The two 32-key
-  // blocks are two independent accumulation chains, interleaved so that no MFMA waits for its predecessor.
-  auto do_qk = [&](int it, f32x16 (&dst)[2]) __attribute__((always_inline)) {
-    const unsigned char* sk = fa_smem + (it % 3) * STAGE;
-    const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    // (the addresses are made opaque per tile: otherwise hipcc hoists the 16 XOR-ed fragment addresses x 3 ring slots
-    //  out of the tile loop and SPILLS them -- one v_xor per read is cheaper than a scratch reload)
-    int ka = kaddr, qa = qaddr;
-    asm volatile("" : "+v"(ka), "+v"(qa));
-    // fragments of k-step ks + 1 are read while the two MFMAs of step ks run (left alone hipcc issues each read right in
-    // front of its MFMA and waits lgkmcnt(0): ~100 exposed cycles per pair)
-    u32x4 fr[2][3];
-    auto rd = [&](int ks, u32x4 (&f)[3]) __attribute__((always_inline)) {
-      f[0] = *reinterpret_cast<const u32x4*>(qlds + (qa ^ (ks << 5)));
-      f[1] = *reinterpret_cast<const u32x4*>(sk + (ka ^ (ks << 5)));
-      f[2] = *reinterpret_cast<const u32x4*>(sk + 8192 + (ka ^ (ks << 5)));
-    };
-    rd(0, fr[0]);
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      if (ks < 7) rd(ks + 1, fr[(ks + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);
-      dst[0] = fa_mfma32<T>(fr[ks & 1][1], fr[ks & 1][0], ks == 0 ? zero : dst[0]);
-      dst[1] = fa_mfma32<T>(fr[ks & 1][2], fr[ks & 1][0], ks == 0 ? zero : dst[1]);
-    }
-  };
-  // exchange a value with the lane holding the other 32 keys of the same row
-  auto other_half = [&](float x) __attribute__((always_inline)) {
-    const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x), false, false);
-    return kh ? __builtin_bit_cast(float, (unsigned)sw[0]) : __builtin_bit_cast(float, (unsigned)sw[1]);
-  };
-  // probabilities (in src) -> PV B-operand fragments: k-slot 2 b + j holds tile keys 32 b + 16 j + 8 kh .. + 7 of row l31
-  auto make_pf = [&](const f32x16 (&src)[2], u32x4 (&pf)[4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int g0 = 8 * j, g1 = 8 * j + 4;       // accumulator quads 2 j and 2 j + 1
-        const uint32_t lo0 = pack2_16<BF>(src[b][g0], src[b][g0 + 1]), hi0 = pack2_16<BF>(src[b][g0 + 2], src[b][g0 + 3]);
-        const uint32_t lo1 = pack2_16<BF>(src[b][g1], src[b][g1 + 1]), hi1 = pack2_16<BF>(src[b][g1 + 2], src[b][g1 + 3]);
-        const auto s_lo = __builtin_amdgcn_permlane32_swap(lo0, lo1, false, false);
-        const auto s_hi = __builtin_amdgcn_permlane32_swap(hi0, hi1, false, false);
-        pf[2 * b + j] = u32x4{(uint32_t)s_lo[0], (uint32_t)s_hi[0], (uint32_t)s_lo[1], (uint32_t)s_hi[1]};
-      }
-  };
-  // online softmax of an UNMASKED tile, straight-line (no branches: it is scheduled together with the next tile's QK^T).
-  // Returns the factor the running output must be scaled with.
-  auto softmax_fast = [&](f32x16 (&src)[2], u32x4 (&pf)[4]) __attribute__((always_inline)) -> float {
-    float mx = __builtin_fmaxf(src[0][0], src[1][0]);
-#pragma unroll
-    for (int r = 1; r < 16; ++r) mx = __builtin_fmaxf(mx, __builtin_fmaxf(src[0][r], src[1][r]));   // -> v_max3_f32
-    mx *= c2;                                      // scale > 0: the maximum commutes with it
-    mx = __builtin_fmaxf(mx, other_half(mx));
-    const float m_new = __builtin_fmaxf(m_run, mx);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    m_run = m_new;
-    float lsum0 = 0.f, lsum1 = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      src[0][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(src[0][r], c2, -m_new));
-      src[1][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(src[1][r], c2, -m_new));
-      lsum0 += src[0][r];
-      lsum1 += src[1][r];
-    }
-    l_run = l_run * alpha + (lsum0 + lsum1);
-    make_pf(src, pf);
-    return alpha;
-  };
-  // QK^T of tile it + 1 (into nxt) and the softmax of an unmasked tile (cur -> pf) as ONE hand-interleaved stream: per
-  // k-step two MFMAs, then a slice of the softmax VALU that runs in their shadow; sched_barrier keeps hipcc from
-  // regrouping them into an MFMA block and a VALU block (which is what every compiler-driven attempt produced).
-  auto qk_softmax_fast = [&](int it_next, f32x16 (&nxt)[2], f32x16 (&cur)[2], u32x4 (&pf)[4]) __attribute__((always_inline)) -> float {
-    const unsigned char* sk = fa_smem + (it_next % 3) * STAGE;
-    const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    int ka = kaddr, qa = qaddr;
-    asm volatile("" : "+v"(ka), "+v"(qa));
-    u32x4 fr[2][3];
-    auto rd = [&](int ks, u32x4 (&f)[3]) __attribute__((always_inline)) {
-      f[0] = *reinterpret_cast<const u32x4*>(qlds + (qa ^ (ks << 5)));
-      f[1] = *reinterpret_cast<const u32x4*>(sk + (ka ^ (ks << 5)));
-      f[2] = *reinterpret_cast<const u32x4*>(sk + 8192 + (ka ^ (ks << 5)));
-    };
-    float mx = 0.f, m_new = 0.f, alpha = 1.f, lsum = 0.f;
-    rd(0, fr[0]);
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      if (ks < 7) rd(ks + 1, fr[(ks + 1) & 1]);
-      nxt[0] = fa_mfma32<T>(fr[ks & 1][1], fr[ks & 1][0], ks == 0 ? zero : nxt[0]);
-      nxt[1] = fa_mfma32<T>(fr[ks & 1][2], fr[ks & 1][0], ks == 0 ? zero : nxt[1]);
-      if (ks == 0) {
-        mx = __builtin_fmaxf(cur[0][0], cur[1][0]);
-#pragma unroll
-        for (int r = 1; r < 8; ++r) mx = __builtin_fmaxf(mx, __builtin_fmaxf(cur[0][r], cur[1][r]));
-      } else if (ks == 1) {
-#pragma unroll
-        for (int r = 8; r < 16; ++r) mx = __builtin_fmaxf(mx, __builtin_fmaxf(cur[0][r], cur[1][r]));
-        mx *= c2;
-        mx = __builtin_fmaxf(mx, other_half(mx));
-        m_new = __builtin_fmaxf(m_run, mx);
-        alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        m_run = m_new;
-      } else if (ks < 6) {
-        const int b = (ks - 2) >> 1, r0 = ((ks - 2) & 1) * 8;
-#pragma unroll
-        for (int r = r0; r < r0 + 8; ++r) {
-          cur[b][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(cur[b][r], c2, -m_new));
-          lsum += cur[b][r];
-        }
-      } else {
-        const int b = ks - 6;
-        if (b == 0) l_run = l_run * alpha + lsum;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int g0 = 8 * j, g1 = 8 * j + 4;
-          const uint32_t lo0 = pack2_16<BF>(cur[b][g0], cur[b][g0 + 1]), hi0 = pack2_16<BF>(cur[b][g0 + 2], cur[b][g0 + 3]);
-          const uint32_t lo1 = pack2_16<BF>(cur[b][g1], cur[b][g1 + 1]), hi1 = pack2_16<BF>(cur[b][g1 + 2], cur[b][g1 + 3]);
-          const auto s_lo = __builtin_amdgcn_permlane32_swap(lo0, lo1, false, false);
-          const auto s_hi = __builtin_amdgcn_permlane32_swap(hi0, hi1, false, false);
-          pf[2 * b + j] = u32x4{(uint32_t)s_lo[0], (uint32_t)s_hi[0], (uint32_t)s_lo[1], (uint32_t)s_hi[1]};
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    return alpha;
-  };
-  // the general form: key >= len, key > q (causal), ALiBi
-  auto softmax_edge = [&](int it, f32x16 (&src)[2], u32x4 (&pf)[4]) __attribute__((always_inline)) -> float {
-    const int t0 = it * BN;
-    float mx = -1e30f;
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = t0 + 32 * b + 8 * (r >> 2) + 4 * kh + (r & 3);
-        float x = src[b][r] * c2 + slope2 * (float)(key - (qrow + off));
-        const int lim = p.causal ? min(qrow + off, len - 1) : len - 1;
-        x = key <= lim ? x : -1e30f;
-        src[b][r] = x;
-        mx = __builtin_fmaxf(mx, x);
-      }
-    mx = __builtin_fmaxf(mx, other_half(mx));
-    const float m_new = __builtin_fmaxf(m_run, mx);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    m_run = m_new;
-    float lsum = 0.f;
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float e = __builtin_amdgcn_exp2f(src[b][r] - m_new);
-        e = src[b][r] > -1e29f ? e : 0.f;
-        src[b][r] = e;
-        lsum += e;
-      }
-    l_run = l_run * alpha + lsum;
-    make_pf(src, pf);
-    return alpha;
-  };
-  // O^T += V^T . P^T : A fragment of (d block db, k-slot ks) = two transposing reads
-  auto do_pv = [&](int it, const u32x4 (&pf)[4]) __attribute__((always_inline)) {
-    int va = vaddr + (it % 3) * STAGE;
-    asm volatile("" : "+v"(va));
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int db = 0; db < 4; ++db) {
-        const unsigned char* vb = fa_smem + va + (4 * ks) * 1024 + db * 256;
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)vb);
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(vb + 1024));
-        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
-        o[db] = fa_mfma32<T>(u32x4{l2[0], l2[1], h2[0], h2[1]}, pf[ks], o[db]);
-      }
-  };
-
-  // ---- the tile loop ---------------------------------------------------------------------------------------------------------
-  // Iteration `it` (one barrier): QK^T of tile it + 1 || softmax of tile it, then PV of tile it.  The next tile's MFMAs are
-  // independent of this tile's softmax VALU, so one straight-line block holds both (measured on the phase-by-phase form:
-  // QK^T 1280 + softmax 1224 + PV 1032 cycles per tile with NOTHING overlapping, whatever the pairing of waves).
-  // Ring of 3 tile buffers: at the top of iteration it every wave has finished tile it - 1 (the barrier), tiles it and
-  // it + 1 are being read, tile it + 2 is written.
-  // (Rotating the three phases of a tile between the two waves of a SIMD -- one wave's softmax VALU beside the other's MFMAs --
-  // measured 0.852 / 0.837 ms against 0.794 unrotated at T = 8192 and is not in the tree: tools/lab_patches/flash_attn.hip.patch.)
-  f32x16 s_a[2], s_b[2];
-  stage(0, 0);
-  if (ntile > 1) stage(1, BN);
-  if (ntile > 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  if (L > 0) do_qk(0, s_a);
-  auto step = [&](int it, f32x16 (&s_cur)[2], f32x16 (&s_nxt)[2]) __attribute__((always_inline)) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this wave's pieces of tile it + 1 (issued one iteration ago)
-    __builtin_amdgcn_s_barrier();
-    if (it + 2 < ntile) stage((it + 2) % 3, (it + 2) * BN);
-    if (it >= L) return;                                   // causal: this wave's rows are done (it still stages its pieces)
-    u32x4 pf[4];
-    float alpha;
-    // QK^T of the NEXT tile is issued ahead of this tile's softmax: its MFMAs are independent of the softmax VALU
-    // (unconditional: past this wave's last tile it multiplies stale ring data into a buffer nobody reads -- keeping the
-    //  branch out puts these MFMAs and the softmax VALU in ONE scheduling region)
-    if (it < F) {
-      alpha = qk_softmax_fast(it + 1, s_nxt, s_cur, pf);
-    } else {
-      do_qk(it + 1, s_nxt);
-      alpha = softmax_edge(it, s_cur, pf);
-    }
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-      for (int db = 0; db < 4; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-    }
-    do_pv(it, pf);
-  };
-  for (int it = 0; it < ntile; it += 2) {
-    step(it, s_a, s_b);
-    if (it + 1 < ntile) step(it + 1, s_b, s_a);
-  }
-  __syncthreads();                                         // every wave is done with the K / V buffers
-
-  // ---- normalise, transpose through LDS (wave-private 8 KiB: 32 rows x 256 B), store whole rows -----------------------------
-  float l = l_run;
-  {
-    const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, l), __builtin_bit_cast(unsigned, l), false, false);
-    l = __builtin_bit_cast(float, (unsigned)sw[0]) + __builtin_bit_cast(float, (unsigned)sw[1]);
-  }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  unsigned char* region = fa_smem + wave * 8192;
-#pragma unroll
-  for (int db = 0; db < 4; ++db)
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      // d = 32 db + 8 g4 + 4 kh .. + 3  ->  8-byte chunk c8 = 8 db + 2 g4 + kh of row l31; 16-byte chunk XOR (row & 15)
-      const int c8 = 8 * db + 2 * g4 + kh;
-      const u32x2 v = {pack2_16<BF>(o[db][4 * g4] * inv, o[db][4 * g4 + 1] * inv),
-                       pack2_16<BF>(o[db][4 * g4 + 2] * inv, o[db][4 * g4 + 3] * inv)};
-      *reinterpret_cast<u32x2*>(region + l31 * 256 + ((c8 ^ ((l31 & 15) << 1)) << 3)) = v;
-    }
-  uint16_t* obase = (uint16_t*)p.out + (size_t)(s0q + wq0) * p.o_stride + (size_t)head * HD;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = i * 4 + (lane >> 4), c16 = lane & 15;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(region + row * 256 + ((c16 ^ (row & 15)) << 4));
-    if (wq0 + row < qlen) *reinterpret_cast<u32x4*>(obase + (size_t)row * p.o_stride + c16 * 8) = v;
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Prefill WITH cached context (the context_attention_fwd role,
 // aphrodite/attention/ops/prefix_prefill.py:696-858, kernel :58-255): every new
 // token attends to the sequence's cached context, read from the PAGED KV cache
@@ -1010,12 +638,12 @@ __global__ __launch_bounds__(256) void context_attn_kernel(CAParams p) {
 using namespace aphro;
 
 // ---------------------------------------------------------------------------
-// Prefill with cached context on the third-generation tile machine: the context of every sequence is
+// Prefill with cached context on the prompt kernels: the context of every sequence is
 // gathered ONCE from the paged cache into contiguous [token][kv head][hd] rows (dequantised like
 // prefix_prefill.py:131-134,178-181: float(fp8) * scale rounded to the query type), the new tokens' k / v are appended,
-// and flash_attn_varlen_v3_kernel runs over keys = context + new with the query rows offset by the context length.
+// and fa_dispatch's kernels run over keys = context + new with the query rows offset by the context length.
 // The gather is a streaming copy (2 x the context bytes); the attention then reads K/V tiles with direct-to-LDS loads
-// instead of per-element cache gathers.  hd 128, no sliding window; everything else stays on context_attn_kernel.
+// instead of per-element cache gathers.
 // ---------------------------------------------------------------------------
 __global__ void ca_prefix_kernel(const int32_t* __restrict__ seq_lens, int32_t* __restrict__ cu_k, int batch) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
@@ -1101,31 +729,22 @@ extern "C" int aphro_context_attention(void* out, const void* q, const void* k, 
 }
 
 
-// One dispatcher for the three prefill kernel generations (p fully set up except nqt_max / xcd_remap): third generation
-// for head 128, sequences >= 1024, no sliding window; second for head 64 / 128 (always when the keys carry a context
-// offset: its 64-key tiles are what the gathered-context path wants); first generation for the rest.
+// One dispatcher for the prefill kernels (p fully set up except nqt_max / xcd_remap): head 128 without a sliding window runs on 32 x 32 tiles
+// (flash_attn_v4.hip, flash_attn_short.hip); second generation for head 64 and windowed head 128 from 512 query rows on (with a context from
+// 128, its 64-key tiles are what the gathered-context path wants); first generation for the rest.
 static int fa_dispatch(FAParams p, int head_size, int dtype, int batch, int max_query_len, int max_key_len, hipStream_t st) {
-  if (head_size == 128 && max_key_len >= 1024 && p.window <= 0 && !APHRO_LAB_ENV_INT("APHRO_FA_NO_V3", 0)) {
-    p.nqt_max = (max_query_len + 255) / 256;
-    p.xcd_remap = (batch * p.num_kv_heads) % 8 == 0 && !knobs().fa_no_xcd;
-    // fourth generation (one wave per SIMD, two 32-row blocks per wave: flash_attn_v4.hip) from 4096 keys on (measured on
-    // T = 8192 / 4096 / 2048 / 1111 causal, Hq 32 / Hkv 8: 0.583 / 0.174 / 0.081 / 0.046 ms against 0.62 / 0.182 / 0.078 /
-    // 0.044 ms of the third generation); APHRO_FA_V4_MIN_KEYS=<n>: threshold (a huge n: third generation always)
-    if (max_key_len >= knobs().fa_v4_min_keys) return fa_v4_launch(p, dtype, batch, st);
-    dim3 grid3((unsigned)(p.nqt_max * p.num_heads * batch));
-    static bool attr_set_dev[APHRO_MAX_DEVICES] = {}; bool& attr_set = attr_set_dev[device_slot()];
-    if (!attr_set) {
-      if (hipFuncSetAttribute((const void*)flash_attn_varlen_v3_kernel<Half>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840) != hipSuccess ||
-          hipFuncSetAttribute((const void*)flash_attn_varlen_v3_kernel<BFloat>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840) != hipSuccess) {
-        set_error("flash attention: cannot raise the dynamic LDS limit");
-        return APHRO_ERR_LAUNCH;
-      }
-      attr_set = true;
+  if (head_size == 128 && p.window <= 0) {
+    // fourth generation (one wave per SIMD, two 32-row blocks per wave) from 4096 keys on; APHRO_FA_V4_MIN_KEYS=<n>: threshold
+    if (max_key_len >= 1024 && max_key_len >= knobs().fa_v4_min_keys) {
+      p.nqt_max = (max_query_len + 255) / 256;
+      p.xcd_remap = (batch * p.num_kv_heads) % 8 == 0 && !knobs().fa_no_xcd;
+      return fa_v4_launch(p, dtype, batch, st);
     }
-    if (dtype == APHRO_F16) hipLaunchKernelGGL((flash_attn_varlen_v3_kernel<Half>), grid3, dim3(512), 163840, st, p);
-    else hipLaunchKernelGGL((flash_attn_varlen_v3_kernel<BFloat>), grid3, dim3(512), 163840, st, p);
-    APHRO_LAUNCH_CHECK();
-    return APHRO_OK;
+    p.nqt_max = 0; p.xcd_remap = 0;
+    if (fa_short_launch(p, dtype, batch, max_query_len, max_key_len, st)) {
+      APHRO_LAUNCH_CHECK();
+      return APHRO_OK;
+    }
   }
   p.nqt_max = 0; p.xcd_remap = 0;
   // two 16-row query tiles per wave (128-row workgroups) once the sequences are long enough to
@@ -1165,8 +784,7 @@ extern "C" size_t aphro_context_attention_workspace_bytes(int64_t total_kv_token
 
 // Same arguments as aphro_context_attention plus: max_seq_len = max(seq_lens) (context + new), total_kv_tokens >=
 // sum(seq_lens), workspace.  Head sizes 64 / 96 / 128 / 256, ALiBi, sliding window: the context is gathered once and the
-// prefill tile machines run over context + new tokens (third generation for head 128 / >= 1024 keys / no window, second
-// for head 64 / 128, first for the rest) -- round 3: the scalar-gather aphro_context_attention kernel is no longer on any
+// prompt kernels run over context + new tokens (fa_dispatch): the scalar-gather aphro_context_attention kernel is no longer on any
 // path the Python op takes.
 extern "C" int aphro_context_attention_gathered(void* out, const void* q, const void* k, const void* v, const void* k_cache,
                                                 const void* v_cache, const int32_t* block_tables, const int32_t* q_start_loc,

@@ -15,8 +15,8 @@ struct FAParams {
   int64_t q_stride, k_stride, v_stride;
   float scale;
   int causal;
-  int nqt_max, xcd_remap;   // third-generation kernel: query tiles per sequence in the grid; kv-head -> XCD placement
-  const int32_t* cu_seqlens_k;   // third-generation kernel: key rows per sequence when they differ from the query rows
+  int nqt_max, xcd_remap;   // fourth-generation kernel: query tiles per sequence in the grid; kv-head -> XCD placement
+  const int32_t* cu_seqlens_k;   // key rows per sequence when they differ from the query rows
   int64_t o_stride;              // ... and the output row stride (elements)
   int window;                    // first / second generation kernels: sliding window (keys > query position - window), 0 = off
 };
@@ -48,6 +48,9 @@ __device__ __forceinline__ u32x4 fa_make_rsrc(const void* base, uint32_t bytes) 
   return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
                (uint32_t)__builtin_amdgcn_readfirstlane(bytes), 0x00020000u};
 }
+
+// rows of 128, fewer keys than the fourth generation's (flash_attn_short.hip): false where it does not serve the call
+bool fa_short_launch(const FAParams& p, int dtype, int batch, int max_query_len, int max_key_len, hipStream_t st);
 
 // fourth-generation prefill kernel (flash_attn_v4.hip): p fully set up incl. nqt_max / xcd_remap
 int fa_v4_launch(const FAParams& p, int dtype, int batch, hipStream_t st);

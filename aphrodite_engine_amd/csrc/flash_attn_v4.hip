@@ -2,7 +2,7 @@
 // next-round 1b): ONE wave per SIMD.  4 waves x 64 query rows = 256 rows per workgroup, 64-key tiles, 32x32x16 MFMA,
 // the whole 512-register file per wave.
 //
-// Why (measured on the third-generation kernel, 8 waves x 32 rows, 0.71 ms at T = 8192 = 5.4 k cycles per tile against
+// Why (measured on the kernel before it, since deleted, 8 waves x 32 rows, 0.71 ms at T = 8192 = 5.4 k cycles per tile against
 // 2 k cycles of MFMA per SIMD): every wave there needs QK^T 1280 + softmax 1224 + PV 1032 issue cycles per tile, two such
 // waves share a SIMD's issue port and matrix pipe, and each re-reads its Q fragments from LDS.  Here a wave owns TWO
 // 32-row query blocks, half a tile apart in the schedule, so that every group of 32 MFMAs carries the softmax of exactly
@@ -18,8 +18,7 @@
 //     piece every fourth step (an LDS-DMA instruction holds the issuing wave for 100-200 cycles);
 //   * the LDS fragments of a step are requested 2 same-kind steps before their MFMAs.
 // LDS images, swapped QK^T (S^T = K . Q^T so that a lane holds the scores of ONE query row), the probability -> PV operand
-// redistribution (permlane32_swap) and the O transpose through LDS are those of the third-generation kernel
-// (flash_attn.hip).  Masked tiles (diagonal, sequence end, ALiBi), the first and the last tile of a wave take a
+// redistribution (permlane32_swap) and the O transpose through LDS are that kernel's.  Masked tiles (diagonal, sequence end, ALiBi), the first and the last tile of a wave take a
 // straight-line path of the same arithmetic.
 #include "flash_attn_common.h"
 
@@ -356,7 +355,7 @@ void flash_attn_varlen_v4_kernel(FAParams p) {
   // Every body runs all 64 MFMAs: at t = 0 the PV of "tile -1" multiplies zeros, at this wave's last tile the S0 of tile
   // t + 1 is computed and never used (a real tile of a later wave, or a stale finite one) -- two loops, one straight-line
   // body each (a loop mixing bodies, or bodies with optional pieces, makes hipcc shuffle and spill the 192 accumulator
-  // registers at every join: measured 2 x slower than the third-generation kernel).
+  // registers at every join: measured 2 x slower than 8 waves x 32 rows).
   const int t_fast = min(F, L);
   int t = 0;
   for (; t < t_fast; ++t) {

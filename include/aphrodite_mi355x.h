@@ -440,7 +440,7 @@ int aphro_context_attention(void* out, const void* q, const void* k, const void*
                             int kv_dtype, void* stream);
 
 /* The same op for long prompts (head_size 128, no sliding window): the cached context is gathered once into contiguous
- * rows (workspace) and the third-generation prefill kernel (256-row workgroups, 32x32 MFMA, direct-to-LDS K/V) runs over
+ * rows (workspace) and the prefill kernels (32x32 MFMA, direct-to-LDS K/V) run over
  * context + new tokens.  max_seq_len = max(seq_lens), total_kv_tokens >= sum(seq_lens).  Round 3: every head size of
  * aphro_context_attention (64 / 96 / 128 / 256), ALiBi and sliding_window (> 0: keys within the window, prefix_prefill.py:
  * 756-760) -- the second / first generation tile machines take the shapes the third does not. */

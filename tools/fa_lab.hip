@@ -5,6 +5,7 @@
 // input (T tokens, Hq 32 / Hkv 8 / hd 128, causal) and compares their outputs element by element.
 #include "bin/csrc_lab/flash_attn.hip"
 #include "bin/csrc_lab/flash_attn_v4.hip"
+#include "bin/csrc_lab/flash_attn_short.hip"
 #include "bin/csrc_lab/runtime.hip"
 #include <cmath>
 #include <cstring>
