@@ -1022,14 +1022,18 @@ static size_t large_scratch_bytes(const LargePlan& pl, int64_t M, int64_t N) {
   return pl.ksplit > 1 ? (size_t)pl.ksplit * M * N * sizeof(float) : 0;
 }
 
-// stream-K: clear the flag words, point the kernel at them
+// stream-K: point the kernel at its flag words, cleared where it cuts tiles
 static int large_bind_scratch(Wna16LargeParams& p, const LargePlan& pl, char* ws, hipStream_t st) {
   p.streamk = pl.streamk; p.grid = pl.grid; p.ksplit = pl.ksplit; p.flags = nullptr; p.partial = (float*)ws;
   if (pl.streamk) {
     p.flags = (unsigned*)ws;
     p.partial = (float*)(ws + LARGE_FLAG_BYTES);
-    hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(LARGE_FLAG_BYTES / 4), 0, st, p.flags);
-    APHRO_LAUNCH_CHECK();
+    // (no tile is cut where the workgroups divide the tiles, as in fp8_gemm_large.hip)
+    const int64_t tiles = (int64_t)((p.M + 128 * pl.wm - 1) / (128 * pl.wm)) * (p.N / (64 * pl.wn));
+    if (tiles % pl.grid != 0) {
+      hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(LARGE_FLAG_BYTES / 4), 0, st, p.flags);
+      APHRO_LAUNCH_CHECK();
+    }
   }
   return APHRO_OK;
 }
