@@ -596,6 +596,32 @@ def wna16_gemm_large_strip(a: torch.Tensor, strip: torch.Tensor, qzeros: torch.T
     return out
 
 
+def wna16_linear_add_norm(a: torch.Tensor, qweight: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor, zero_offset: int, strip: bool,
+                          residual: torch.Tensor, weight: torch.Tensor, epsilon: float) -> Optional[torch.Tensor]:
+    """fused_add_rms_norm(a . dequant(W), residual, weight) where the product runs on the tile machine with K slices, the norm in the launch
+    that sums them: the normed rows, residual updated in place, the same bits; None (and nothing done) for any other call.  ``strip``: qweight is
+    the strip-major copy."""
+    m, k = a.shape
+    n, groups = scales.shape[1], scales.shape[0]
+    lib = _lib.lib()
+    if a.dtype != scales.dtype or weight.dtype != a.dtype or residual.dtype != a.dtype or not residual.is_contiguous() or residual.numel() != m * n \
+            or residual.data_ptr() % 16 != 0 or weight.data_ptr() % 16 != 0 or not weight.is_contiguous() \
+            or not wna16_large_ok(m, n, k, groups) or switch("APHRO_WNA16_NO_LARGE") \
+            or not wna16_prefers_large(m, n, k, a.dtype, groups, strip=strip) \
+            or not lib.aphro_wna16_gemm_large_add_norm_supported(m, n, k, groups, _dt(a)):
+        return None
+    _require_cuda(a, qweight, qzeros, scales, residual, weight)
+    if a.stride(1) != 1 or a.stride(0) % 8 != 0 or a.data_ptr() % 16 != 0:
+        a = a.contiguous()
+    out = torch.empty((m, n), dtype=a.dtype, device=a.device)
+    nbytes = lib.aphro_wna16_gemm_large_workspace_bytes(m, n, k, groups, _dt(a))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=a.device)
+    check(lib.aphro_wna16_gemm_large_add_norm(a.data_ptr(), qweight.data_ptr(), qzeros.data_ptr(), scales.data_ptr(), out.data_ptr(),
+                                              residual.data_ptr(), weight.data_ptr(), float(epsilon), ws.data_ptr(), nbytes, m, n, k, groups,
+                                              a.stride(0), zero_offset, _dt(a), 32 if strip else 0, _stream()), "wna16_gemm_large_add_norm")
+    return out
+
+
 def wna16_linear_strip(a: torch.Tensor, strip: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor,
                        zero_offset: int, strip_m: int = 32) -> torch.Tensor:
     """[M, N] = a . dequant(W) for ANY M when the strip-major copy is the only resident copy of W (model.enable_one_copy):

@@ -4,20 +4,9 @@
 //   rotary_embedding                kernels/pos_encoding_kernels.cu:10-160
 // One workgroup per token, 16-byte vector accesses, fp32 math, wave64 reductions.
 #include "common.h"
+#include "row_norm.h"
 
 namespace aphro {
-
-__device__ __forceinline__ float block_sum(float v, float* red) {
-  v = wave_sum(v);
-  const int nw = blockDim.x >> 6;
-  if (nw == 1) return v;
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  float t = 0.f;
-  for (int w = 0; w < nw; ++w) t += red[w];
-  __syncthreads();
-  return t;
-}
 
 // ADD: residual' = input + residual (stored), input' = norm(residual') * w  (in place)
 template <typename T, bool ADD>
@@ -152,15 +141,6 @@ __global__ void rotary_kernel(const int64_t* __restrict__ positions, uint16_t* _
 }  // namespace aphro
 
 using namespace aphro;
-
-static int norm_threads(int hidden) {
-  // same thread -> element mapping as add_rms_norm_pack_kernel (fused_decode.hip): the
-  // sum-of-squares reduction order, hence every output bit, is shared by the two paths
-  int nv = hidden / 8;
-  int t = nv <= 1024 ? nv : (nv + 1) / 2;
-  t = (t + 63) / 64 * 64;
-  return t < 64 ? 64 : (t > 1024 ? 1024 : t);
-}
 
 extern "C" int aphro_rms_norm(void* out, const void* input, const void* weight, float eps, int64_t num_tokens,
                               int hidden, int64_t in_stride, int dtype, void* stream) {

@@ -1104,7 +1104,8 @@ extern "C" size_t aphro_wna16_gemm_large_strip_workspace_bytes(int64_t M, int64_
 // with saturation, scales and output stay bf16).  Act-order: pass the activations already gathered (a[:, perm]).
 static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const uint32_t* qzeros, const void* scales,
                                  void* c, void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K,
-                                 int64_t groups, int64_t lda, int zero_offset, int dtype, int silu, void* stream, int strip_m = 0) {
+                                 int64_t groups, int64_t lda, int zero_offset, int dtype, int silu, void* stream, int strip_m = 0,
+                                 void* residual = nullptr, const void* norm_weight = nullptr, float norm_eps = 0.f) {
   hipStream_t st = (hipStream_t)stream;
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "wna16_gemm_large: dtype must be f16 or bf16");
   APHRO_CHECK(groups > 0 && K % groups == 0, "wna16_gemm_large: K=%ld not divisible by groups=%ld", (long)K, (long)groups);
@@ -1160,11 +1161,14 @@ static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const 
                   "wna16_gemm_large_strip: multiply-shift division fails at %u (nseg %d, nwv %d)", x, p.st_nseg, p.st_nwv);
   }
   const Wna16RowsPlan rp = rows_plan(pl, M, N, K, gs, dtype);
+  APHRO_CHECK(!norm_weight || (rp.mb > 0 && rp.ksplit > 1 && N <= 16384), "wna16_gemm_large_add_norm: M=%ld N=%ld K=%ld has no summed K slices",
+              (long)M, (long)N, (long)K);
   if (rp.mb > 0) {
     Wna16RowsParams q = {};
     q.a = p.a; q.lda = p.lda; q.qw = p.qw; q.qz = p.qz; q.sc = p.sc; q.c = p.c; q.partial = (float*)ws;
     q.M = p.M; q.N = p.N; q.K = p.K; q.group_size = p.group_size; q.zero_offset = zero_offset;
     q.ksplit = rp.ksplit; q.silu = silu; q.bf16 = p.out_bf16;
+    q.residual = (uint16_t*)residual; q.norm_weight = (const uint16_t*)norm_weight; q.norm_eps = norm_eps;
     APHRO_CHECK(strip_m == 0 || wna16_strip_fill(q.strip, strip_m, N, K, groups),
                 "wna16_gemm_large_strip: no strip-major form for M class %d, N=%ld, K=%ld, groups=%ld", strip_m, (long)N, (long)K, (long)groups);
     return wna16_rows_launch(q, rp, st);
@@ -1219,6 +1223,24 @@ extern "C" int aphro_wna16_gemm_large_strip(const void* a, const uint32_t* q_wei
   APHRO_CHECK(strip_m >= 1 && strip_m <= 64, "wna16_gemm_large_strip: strip_m=%ld", (long)strip_m);
   return wna16_gemm_large_impl(a, q_weight_strip, qzeros, scales, c, workspace, workspace_bytes, M, N, K, groups, lda, zero_offset, dtype,
                                silu ? 1 : 0, stream, (int)strip_m);
+}
+
+// aphro_wna16_gemm_large (strip_m == 0) / _strip followed by fused_add_rms_norm, where the GEMM ends in a sum over K slices: the norm is that
+// launch's.  c [M, N] = norm(residual') * norm_weight, residual' = residual + product, in place; the same bits.  1 if the shape is served, else 0: aphro_wna16_gemm_large_add_norm_supported.
+extern "C" int aphro_wna16_gemm_large_add_norm_supported(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype) {
+  if (M <= 0 || groups <= 0 || K % groups != 0 || K % 64 != 0 || (K / groups) % 64 != 0 || N % 128 != 0 || N > 16384) return 0;
+  const Wna16RowsPlan rp = rows_plan(large_plan(M, N, K, K / groups), M, N, K, K / groups, dtype);
+  return rp.mb > 0 && rp.ksplit > 1;
+}
+extern "C" int aphro_wna16_gemm_large_add_norm(const void* a, const uint32_t* q_weight, const uint32_t* qzeros, const void* scales, void* c,
+                                               void* residual, const void* norm_weight, float eps, void* workspace, size_t workspace_bytes,
+                                               int64_t M, int64_t N, int64_t K, int64_t groups, int64_t lda, int zero_offset, int dtype,
+                                               int64_t strip_m, void* stream) {
+  APHRO_CHECK(strip_m >= 0 && strip_m <= 64, "wna16_gemm_large_add_norm: strip_m=%ld", (long)strip_m);
+  APHRO_CHECK(residual && norm_weight && (((uintptr_t)residual | (uintptr_t)norm_weight | (uintptr_t)c) % 16) == 0,
+              "wna16_gemm_large_add_norm: c, residual and norm_weight must be 16-byte aligned");
+  return wna16_gemm_large_impl(a, q_weight, qzeros, scales, c, workspace, workspace_bytes, M, N, K, groups, lda, zero_offset, dtype, 0, stream,
+                               (int)strip_m, residual, norm_weight, eps);
 }
 
 extern "C" int aphro_wna16_gemm_large_silu_supported(int64_t M, int64_t N, int64_t K, int64_t groups) {

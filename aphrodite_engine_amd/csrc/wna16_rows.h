@@ -16,6 +16,10 @@ struct Wna16RowsParams {
   int M, N, K, lda;
   int group_size, zero_offset, ksplit, silu;
   int bf16;               // scales and results are bf16 (else f16)
+  // RMS norm behind summed K slices (ksplit > 1): residual' = residual + product, c = norm(residual') * norm_weight
+  uint16_t* residual;
+  const uint16_t* norm_weight;      // (null: none)
+  float norm_eps;
   int tiles_m, tiles_n;   // (filled by the launch)
   Wna16StripGeom strip;
 };

@@ -891,22 +891,26 @@ class LlamaDecoderLayer(nn.Module):
             d = tensor_model_parallel_all_reduce(d)
         return d
 
-    def forward(self, positions, hidden, residual, kv_cache, attn_metadata, cos_sin):
+    def forward(self, positions, hidden, residual, kv_cache, attn_metadata, cos_sin, next_norm=None):
+        """``next_norm``: the norm weight behind this layer (the next layer's first, or the model's last).  With it the returned rows are added
+        to the residual and normed already, and so are ``hidden``, except in the first layer (residual None)."""
         eps = self.cfg.rms_norm_eps
         if residual is None:
             residual = hidden
             normed = torch.empty_like(hidden)
             ops.rms_norm(normed, hidden, self.input_layernorm, eps)
             hidden = normed
-        else:
+        elif next_norm is None:
             ops.fused_add_rms_norm(hidden, residual, self.input_layernorm, eps)
         qkv = self.qkv_proj(hidden)
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
         attn_out = self._attend(positions, q, k, v, kv_cache, attn_metadata, cos_sin)
-        hidden = self._row_parallel(self.o_proj, attn_out)
-        ops.fused_add_rms_norm(hidden, residual, self.post_attention_layernorm, eps)
+        hidden = self._row_parallel(self.o_proj, attn_out, residual, self.post_attention_layernorm)
         if self.is_moe:
-            return self.moe_block(hidden), residual
+            hidden = self.moe_block(hidden)
+            if next_norm is not None:
+                ops.fused_add_rms_norm(hidden, residual, next_norm, eps)
+            return hidden, residual
         il = self.gate_up_interleaved is not None and not self.gate_up_keep_original
         if il and hidden.shape[0] > 64 and not self.has_bias and not switch("APHRO_PREFILL_NO_SILU_EPILOGUE") \
                 and not switch("APHRO_WNA16_NO_LARGE"):
@@ -918,25 +922,34 @@ class LlamaDecoderLayer(nn.Module):
                     act = ops.wna16_gemm_large_strip(hidden, qw, qz, sc, zo, silu=True)
                 else:
                     act = ops.wna16_gemm_large_silu(hidden, qw, qz, sc, zo)
-                hidden = self.down_proj(act)
-                if self.tp > 1:
-                    hidden = tensor_model_parallel_all_reduce(hidden)
-                return hidden, residual
+                return self._row_parallel(self.down_proj, act, residual, next_norm), residual
         gate_up = self.gate_up_proj(hidden)
         act = torch.empty(gate_up.shape[0], gate_up.shape[1] // 2, dtype=gate_up.dtype,
                           device=gate_up.device)
         # ONE copy of the gate_up weights: once SiluAndMul rides in the decode GEMM's epilogue the parameters hold the
         # interleaved (gate_j, up_j) column order, and the op-by-op / prompt-sized path pairs the columns in the activation
         ops.silu_and_mul(act, gate_up, interleaved=self.gate_up_interleaved is not None and not self.gate_up_keep_original)
-        return self._row_parallel(self.down_proj, act), residual
+        return self._row_parallel(self.down_proj, act, residual, next_norm), residual
 
-    def _row_parallel(self, lin: QuantLinear, x: torch.Tensor) -> torch.Tensor:
+    def _row_parallel(self, lin: QuantLinear, x: torch.Tensor, residual: torch.Tensor, norm: Optional[torch.Tensor]) -> torch.Tensor:
         """RowParallelLinear.forward (linear.py:1136-1150): this rank's partial product, the all-reduce over the TP group,
-        then the bias -- once, not per rank."""
+        then the bias -- once, not per rank.  ``norm``: then fused_add_rms_norm with these weights, in the product's own last launch where it
+        has one over whole sums."""
         if self.tp == 1:
-            return lin(x)
-        out = tensor_model_parallel_all_reduce(lin(x, add_bias=False))
-        return out if lin.bias is None else out + lin.bias
+            if norm is not None and lin.bias is None and x.shape[0] > 64 and isinstance(lin.quant_config, (GPTQConfig, AWQConfig)):
+                fp = lin.fast_params()
+                if fp is not None:
+                    out = ops.wna16_linear_add_norm(x, *fp, getattr(lin, "qweight_strip_major", False), residual, norm, self.cfg.rms_norm_eps)
+                    if out is not None:
+                        return out
+            out = lin(x)
+        else:
+            out = tensor_model_parallel_all_reduce(lin(x, add_bias=False))
+            if lin.bias is not None:
+                out = out + lin.bias
+        if norm is not None:
+            ops.fused_add_rms_norm(out, residual, norm, self.cfg.rms_norm_eps)
+        return out
 
 
 class LlamaForCausalLM(nn.Module):
@@ -1082,9 +1095,9 @@ class LlamaForCausalLM(nn.Module):
             return hidden
         residual = None
         for i, layer in enumerate(self.layers):
+            behind = self.layers[i + 1].input_layernorm if i + 1 < len(self.layers) else self.norm
             hidden, residual = layer(positions, hidden, residual, kv_caches[i],
-                                     attn_metadata, self.cos_sin)
-        ops.fused_add_rms_norm(hidden, residual, self.norm, self.cfg.rms_norm_eps)
+                                     attn_metadata, self.cos_sin, behind)
         return hidden
 
     # ---- what the engine (engine.py) asks of a model ------------------------------------------------------------------

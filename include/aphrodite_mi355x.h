@@ -736,6 +736,13 @@ int aphro_wna16_gemm_large_strip(const void* a, const uint32_t* q_weight_strip, 
                                  void* c, void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K,
                                  int64_t groups, int64_t lda, int zero_offset, int dtype, int silu, int64_t strip_m,
                                  void* stream);
+/* aphro_wna16_gemm_large (strip_m == 0) or _strip followed by aphro_fused_add_rms_norm, the norm in the launch that sums the GEMM's K slices:
+ * c = norm(residual + product) * norm_weight, residual in place; same bits, same workspace.  Served where the GEMM slices K (supported == 1). */
+int aphro_wna16_gemm_large_add_norm_supported(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype);
+int aphro_wna16_gemm_large_add_norm(const void* a, const uint32_t* q_weight, const uint32_t* qzeros, const void* scales, void* c,
+                                    void* residual, const void* norm_weight, float eps, void* workspace, size_t workspace_bytes,
+                                    int64_t M, int64_t N, int64_t K, int64_t groups, int64_t lda, int zero_offset, int dtype,
+                                    int64_t strip_m, void* stream);
 
 /* The op-level decode GEMM (`_C::gptq_gemm` / `_C::awq_gemm` at M <= 32, torch_bindings.cpp:229-243; the role of
  * gemm_half_q_half_gptq_4bit_kernel, q_gemm.cu:190-326, which also reads row-major `a` and writes [M, N] in one launch) in
