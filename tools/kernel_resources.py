@@ -15,8 +15,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Wno-unused-function", "-Wno-unused-variable", "-Wno-pass-failed",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 _VF, _KP = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], ["-mllvm", "-amdgpu-kernarg-preload-count=14"]
-EXTRA = {"paged_attention.hip": _VF + _KP, "flash_attn.hip": _VF, "wna16_moe_tile.hip": _VF, "wna16_gemm_resident.hip": _VF + _KP,
-         "fp8_gemm_resident.hip": _KP, "fp8_gemm_stream.hip": _KP, "wna16_gemm.hip": _KP}      # (the Makefile's per-file EXTRA)
+EXTRA = {"paged_attention.hip": _VF + _KP, "flash_attn.hip": _VF, "flash_attn_short.hip": _VF, "wna16_moe_tile.hip": _VF,
+         "wna16_gemm_resident.hip": _VF + _KP, "fp8_gemm_resident.hip": _KP, "fp8_gemm_stream.hip": _KP, "wna16_gemm.hip": _KP}      # (the Makefile's per-file EXTRA)
 
 
 def demangle(names):
