@@ -165,13 +165,14 @@ __device__ __forceinline__ typename T::storage from_f32_exact(float f) {
 // Division of many numbers by one: the reciprocal once, then q = v r and two corrections by the exact remainder (Markstein's theorem: with r and
 // the first correction within half and one unit in the last place, the second is the rounded quotient) -- 6 operations for the 11 of a division
 // that has to scale its operands, one of them a quarter as fast.  The bits of v / s for finite v whose quotient is not below 2^-40 of all; smaller
-// ones stay as small, and keep their sign.  ``plain`` says that s is in the range where nothing overflows or underflows on the way.
+// ones stay as small, and keep their sign.  ``plain`` says that nothing overflows or underflows on the way: s is in range, and so is the largest
+// |v| times r.  ``most``: that |v|, or 0 where s was made from it and no bound has lowered it since.
 struct Divisor {
   float s, r;
   bool plain;
 };
-__device__ __forceinline__ Divisor divisor(float s, bool finite) {
-  return {s, 1.0f / s, (bool)__builtin_amdgcn_readfirstlane(finite && s >= 0x1p-60f && s <= 0x1p60f)};
+__device__ __forceinline__ Divisor divisor(float s, float most) {
+  return {s, 1.0f / s, (bool)__builtin_amdgcn_readfirstlane(s >= 0x1p-60f && s <= 0x1p60f && most <= 0x1p40f * s)};
 }
 __device__ __forceinline__ float divide_plain(float v, const Divisor& d) {
   float q = v * d.r;

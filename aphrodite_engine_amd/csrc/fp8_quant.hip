@@ -222,12 +222,12 @@ __global__ __launch_bounds__(256) void per_token_quant_wave_kernel(uint8_t* __re
     }
   }
   m = wave_max(m);
-  const bool finite = m <= 3.402823466e38f;
+  const float most = m;                               // (an upper bound on the scale leaves quotients as large as they are)
   if (scale_ub) m = __builtin_fminf(m, *scale_ub);
   const float min_sf = 1.0f / (FP8_MAX * 512.f);
   const float s = __builtin_fmaxf(m / FP8_MAX, min_sf);
   if (lane == 0) scales[tok] = s;
-  const Divisor by = divisor(s, finite);
+  const Divisor by = divisor(s, most);
   uint32_t* o = reinterpret_cast<uint32_t*>(out + tok * hidden);
 #pragma unroll
   for (int j = 0; j < NQ; ++j) {

@@ -174,7 +174,7 @@ __global__ void add_rms_norm_quant_kernel(const uint16_t* __restrict__ input, co
     scale = __builtin_fmaxf(amax / FQ_MAX, 1.0f / (FQ_MAX * 512.f));
   }
   if (threadIdx.x == 0) scale_out[tok] = scale;
-  const Divisor by = divisor(scale, true);            // (a number that is not finite makes the scale so)
+  const Divisor by = divisor(scale, 0.f);            // (a number that is not finite makes the scale so)
 #pragma unroll
   for (int it = 0; it < 2; ++it) {
     const int i = threadIdx.x + it * blockDim.x;
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(VPT <= 4 ? 1024 : 512) void silu_mul_quant_kernel(c
     scale = __builtin_fmaxf(amax / FQ_MAX, 1.0f / (FQ_MAX * 512.f));
   }
   if (threadIdx.x == 0) scale_out[tok] = scale;
-  const Divisor by = divisor(scale, true);            // (a number that is not finite makes the scale so)
+  const Divisor by = divisor(scale, 0.f);            // (a number that is not finite makes the scale so)
 #pragma unroll
   for (int it = 0; it < VPT; ++it) {
     const int i = threadIdx.x + it * blockDim.x;

@@ -407,6 +407,24 @@ def test_per_token_fp8_quant_prompt_sized(ops, dtype, M, K):
     assert torch.equal(q.view(torch.uint8), q2)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M", [200, 256])
+@pytest.mark.parametrize("ub", [1e-3, 0.5, 300.0])
+def test_per_token_fp8_quant_far_above_the_bound(ops, dtype, M, ub):
+    """Numbers so far above the bound that their quotient is no fp32 number saturate with their own sign, in the workgroup-a-row form and in
+    the wave-a-row one, and rows without such numbers keep every bit."""
+    rng = np.random.default_rng(M)
+    x = ((rng.random((M, 516)) - 0.5) * 60).astype(np.float32)
+    x[3, 5], x[3, 6], x[4, 0], x[9, 515] = -3e36, 3e36, -1e34, -np.inf
+    x[11, 1], x[12, 2], x[13, 3] = -3.3e38, -2.0 ** 41, 2.0 ** 39
+    xt = t(x, dtype)
+    q, s = ops.scaled_fp8_quant(xt, scale_ub=torch.tensor([ub], device=DEV), use_per_token_if_dynamic=True)
+    with np.errstate(over="ignore"):
+        rq, rs = of8.dynamic_per_token_scaled_fp8_quant(xt.float().cpu().numpy(), ub)
+    np.testing.assert_array_equal(s.cpu().numpy(), rs)
+    np.testing.assert_array_equal(q.view(torch.uint8).cpu().numpy(), rq)
+
+
 @pytest.mark.parametrize("M", [1, 16, 33, 64, 90])
 @pytest.mark.parametrize("K,N", [(256, 64), (1024, 256), (4096, 32)])
 @pytest.mark.parametrize("per_token,per_channel", [(False, False), (True, True)])
