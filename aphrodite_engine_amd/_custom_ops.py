@@ -19,6 +19,7 @@ import os
 from typing import List, Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad as _forward_ad
 
 from .switches import switch
 from . import _lib
@@ -1774,7 +1775,9 @@ _transforms, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._ge
 
 
 def _launchable(*tensors) -> bool:
-    """Tensors whose memory a kernel may be launched on right away: nothing records, traces or batches what happens to them."""
+    """Tensors whose memory a kernel may be launched on right away: nothing records, traces, differentiates or batches what happens to them."""
+    if _forward_ad._current_level >= 0:                  # (a dual tensor is a plain one that needs no gradient)
+        return False
     grad = torch.is_grad_enabled()
     for t in tensors:
         if type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad):

@@ -99,3 +99,15 @@ def test_other_forms_go_to_torch():
         assert torch.equal(ops.dense_linear(a, b), F.linear(a, b))
     y = torch.func.vmap(lambda r: ops.dense_linear(r, w))(x.view(4, 2, 128))
     assert torch.allclose(y.reshape(8, 128).float(), F.linear(x, w).float(), rtol=2e-2, atol=2e-2)
+
+
+def test_forward_mode_keeps_its_tangent():
+    x, w = _operands(8, 128, 128, torch.bfloat16, 5)
+    tx, tw = _operands(8, 128, 128, torch.bfloat16, 6)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual
+        unpack = torch.autograd.forward_ad.unpack_dual
+        for f in (ops.dense_linear, ops.dense_logits):
+            assert torch.equal(unpack(f(dual(x, tx), w)).tangent.float(), F.linear(tx, w).float())
+            assert torch.equal(unpack(f(x, dual(w, tw))).tangent.float(), F.linear(x, tw).float())
+    assert ops.dense_rows(x, w) is not None
