@@ -1782,7 +1782,8 @@ def _launchable(*tensors) -> bool:
     for t in tensors:
         if type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad):
             return False
-    return not (_dispatch_modes() or _function_modes() or _transforms() or _tracing() or torch.compiler.is_compiling())
+    return not (_dispatch_modes() or _function_modes() or _transforms() or _tracing() or torch.compiler.is_compiling()
+                or torch.is_autocast_enabled())          # (autocast chooses a product's types)
 
 
 @functools.lru_cache(4096)

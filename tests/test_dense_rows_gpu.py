@@ -111,3 +111,12 @@ def test_forward_mode_keeps_its_tangent():
             assert torch.equal(unpack(f(dual(x, tx), w)).tangent.float(), F.linear(tx, w).float())
             assert torch.equal(unpack(f(x, dual(w, tw))).tangent.float(), F.linear(x, tw).float())
     assert ops.dense_rows(x, w) is not None
+
+
+def test_autocast_chooses_the_type():
+    x, w = _operands(8, 128, 128, torch.bfloat16, 7)
+    with torch.autocast("cuda", dtype=torch.float16):
+        got = ops.dense_linear(x, w)
+        assert got.dtype == torch.float16 and torch.equal(got, F.linear(x, w))
+        with torch.autocast("cuda", enabled=False):
+            assert ops.dense_linear(x, w).dtype == torch.bfloat16
