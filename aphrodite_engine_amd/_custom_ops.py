@@ -2264,6 +2264,8 @@ def cutlass_scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor,
     odt = _lib.F16 if out_dtype == torch.float16 else _lib.BF16
     sa = scale_a.reshape(-1).float()
     sb = scale_b.reshape(-1).float()
+    if rows and (sa.numel() not in (1, m) or sb.numel() not in (1, n)):
+        raise RuntimeError("cutlass_scaled_mm: scale_a must have 1 or M elements, scale_b 1 or N")
     a_tok = 1 if sa.numel() > 1 else 0
     b_ch = 1 if sb.numel() > 1 else 0
     most = m if rows else 64

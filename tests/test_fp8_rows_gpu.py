@@ -71,3 +71,13 @@ def test_rope_cache_of_scaled_slabs(kv, dtype, nslab, rows):
         results.append((q, k, v))
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("m", [65, 100, 192, 300])
+def test_scales_of_another_length_are_refused(m):
+    a, w = torch.zeros(m, 256, device="cuda").to(torch.float8_e4m3fn), torch.zeros(512, 256, device="cuda").to(torch.float8_e4m3fn)
+    one = lambda n: torch.ones(n, device="cuda")
+    for sa, sb in ((one(m - 1), one(512)), (one(m + 1), one(1)), (one(2), one(1)), (one(m), one(511)), (one(1), one(2))):
+        with pytest.raises(RuntimeError, match="scale_a must have 1 or M elements"):
+            ops.cutlass_scaled_mm(a, w.t(), sa, sb, torch.bfloat16)
+    assert not ops.cutlass_scaled_mm(a, w.t(), one(m), one(512), torch.bfloat16).any()
