@@ -128,9 +128,10 @@ struct RowsTile {
     int slot = 0, fetch = NS - 1;
     for (int s = 0; s < n; ++s) {
       // step s has landed when at most the loads of the NS - 2 steps behind it are outstanding; past the barrier every wave is through
-      // with step s - 1, whose stage the loads issued now take
-      if (s + NS - 2 < n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * LPS) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      // with step s - 1 -- its fragments are in registers (lgkmcnt: nothing else keeps a product, and the wait for its operands, ahead of the
+      // barrier) -- whose stage the loads issued now take
+      if (s + NS - 2 < n) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * LPS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       if (s + NS - 1 < n) issue(s + NS - 1, fetch);
