@@ -25,7 +25,12 @@ struct RowsPlan { int mt, nt, ksplit; };
 //  * 160 tiles of 64 rows and more: K in one piece ([11264, 2048], 16: 12.4, split 14.5).
 //  * else one workgroup a CU, or two where one a CU would leave more than an eighth of the CUs idle ([6144, 4096], 16: 5 slices 15.2);
 //    a slice has at least 4 steps.
-//  * from 65 rows of x on, 128 rows of w also with K split while a slice keeps 12 steps: [4096, 11008], 128: 30.3 against 33.5.
+//  * from 65 rows of x on, 128 rows of w also with K split while a slice keeps 10 steps: [4096, 11008], 128: 30.3 against 33.5; and in place of
+//    K in one piece where that gives work to more CUs ([10240, 8192], 65 / 128 / 192: 57 / 67 / 90 in one piece of 64 rows, 39 / 43 / 54 in
+//    three of 128).
+//  * from 129 rows of x on a 64-row tile's stages leave room for one workgroup a CU (rows_dispatch), so that more than 256 of them run in two
+//    rounds: no second workgroup a CU, and 128 rows of w above 256 tiles.  FP8, raw sums, 129 / 160 / 192 rows: [6144, 4096] 15.2 / 16.6 / 18.3 in 5
+//    slices, 12.5 / 13.2 / 14.6 in 2; [17408, 4096] 39.6 / 41.1 / 45.5 by 64, 29.3 / 30.5 / 31.4 by 128.
 inline RowsPlan rows_plan(int64_t M, int64_t w_rows, int64_t row_bytes) {
   RowsPlan plan;
   const int t64 = (int)((w_rows + 63) / 64), t128 = (int)((w_rows + 127) / 128), steps = (int)(row_bytes / 128);
@@ -40,13 +45,19 @@ inline RowsPlan rows_plan(int64_t M, int64_t w_rows, int64_t row_bytes) {
   if (mt <= 4) {
     plan.nt = t128 >= 160 && (mt > 2 || t64 < 480) ? 2 : 1;
     plan.ksplit = t64 >= 160 ? 1 : split(t64, true);
-  } else if (t128 >= 160 || t64 >= 160) {
-    plan.nt = t128 >= 160 ? 2 : 1;
+    return plan;
+  }
+  const bool lone = plan.mt > 8;
+  const int k2 = split(t128, false);
+  const bool long_slices = steps / k2 >= 10;
+  if (t128 >= 160 || (lone && t64 > 256)) {
+    plan.nt = 2;
     plan.ksplit = 1;
+  } else if (t64 >= 160 && (t128 * k2 <= t64 || !long_slices)) {
+    plan.nt = plan.ksplit = 1;
   } else {
-    const int k2 = split(t128, false);
-    plan.nt = steps / k2 >= 12 ? 2 : 1;
-    plan.ksplit = plan.nt == 2 ? k2 : split(t64, true);
+    plan.nt = long_slices ? 2 : 1;
+    plan.ksplit = long_slices ? k2 : split(t64, !lone);
   }
   return plan;
 }
@@ -142,12 +153,14 @@ struct RowsTile {
   }
 };
 
-// f(MT, NT, WR, NS) for a plan.  Stages: as many as let two workgroups share a CU's 160 KB (64 rows of w: three or two); where 256 CUs' worth of
-// 128-row tiles is all there is ([22016, 4096], 65 rows and more), one workgroup of eight waves a CU with deeper stages.
+// f(MT, NT, WR, NS) for a plan.  Stages: as many as let two workgroups share a CU's 160 KB; from 129 rows of x on, three with 64 rows of w, and one
+// workgroup a CU (two stages and two workgroups: [6144, 4096] FP8, 160 rows, 5 slices 13.7 us, this in 2 slices 13.2).  128-row tiles that all
+// run at once with one workgroup a CU ([22016, 4096], 65 rows and more) get eight waves and deeper stages, more tiles than CUs two stages:
+// bf16 [37888, 3584], 65 / 160 rows 73 / 99 us deep, 68 / 93 with two; [62000, 4096], 65 / 160 rows 111 / 133 and 115 / 126.
 template <typename F>
 int rows_dispatch(const RowsPlan& plan, int tiles_n, F&& f) {
 #define ROWS(MT, NT, WR, NS) f(std::integral_constant<int, MT>{}, std::integral_constant<int, NT>{}, std::integral_constant<int, WR>{}, std::integral_constant<int, NS>{})
-  const bool many = tiles_n >= 512;
+  const bool many = tiles_n >= 512 || (tiles_n > 256 && (plan.mt > 8 || tiles_n < 448));
   if (plan.nt == 1) {
     switch (plan.mt) {
       case 1: return ROWS(1, 1, 1, 5);

@@ -6,7 +6,7 @@
 // rows, from 65 on the prompt kernel); raw slabs last:
 //   [28672, 4096]   30.7 / 32.5 / 36.8  (59.7 / 33.4 / 38.2)      29.9 / 32.9 / 35.9
 //   [4096, 14336]   18.7 / 22.2 / 27.1  (36.8 / 25.3 / 30.4)      15.3 / 17.6 / 20.9
-//   [6144, 4096]    14.4 / 17.9 / 24.5  (17.0 / 18.8 / 22.9)       9.6 / 12.6 / 18.3
+//   [6144, 4096]    14.4 / 17.9 / 19.8  (17.0 / 18.8 / 22.9)       9.6 / 12.6 / 14.7
 //   [4096, 4096]    11.1 / 14.8 / 18.9  (12.7 / 19.2 / 22.8)       6.6 /  9.4 / 10.5
 // (a result in 16 bits over several K slices pays a second launch; the same bits as before at every shape measured)
 #include "dense_rows.h"
@@ -156,12 +156,9 @@ extern "C" int aphro_fp8_gemm_rows_ksplit(int64_t M, int64_t N, int64_t K) {
   return rows_plan(M, N, K).ksplit;
 }
 
-// Whether aphro_scaled_mm_fp8 is the faster op for 65 rows and more: everywhere but where a 16-bit result over several K slices of more than 64
-// column tiles meets many rows ([6144, 4096], 128 / 160 / 192 rows: 17.9 / 22.2 / 24.5 us, the prompt kernel 18.8 / 21.6 / 22.9).
-extern "C" int aphro_fp8_gemm_rows_preferred(int64_t M, int64_t N, int64_t K) {
-  const int split = M > 64 ? aphro_fp8_gemm_rows_ksplit(M, N, K) : 0;
-  return split == 1 || (split > 1 && (M <= 128 || N <= 4096));
-}
+// Whether aphro_scaled_mm_fp8 is the faster op for 65 rows and more: wherever it is served ([6144, 4096], the closest, 65 / 128 / 160 / 192 rows:
+// 14.1 / 17.8 / 18.1 / 19.6 us, the prompt kernel 16.8 / 18.5 / 21.0 / 22.6).
+extern "C" int aphro_fp8_gemm_rows_preferred(int64_t M, int64_t N, int64_t K) { return M > 64 && aphro_fp8_gemm_rows_ksplit(M, N, K) > 0; }
 
 extern "C" int aphro_fp8_gemm_rows(const void* a, const void* w, const float* a_scales, const float* b_scales, const void* bias, void* out,
                                    float* slabs, size_t slabs_bytes, int64_t M, int64_t N, int64_t K, int a_scale_per_token,

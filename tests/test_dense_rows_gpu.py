@@ -26,7 +26,9 @@ def _close(got, want, dtype, k):
 # (rows, columns, k): every row tile, its first and last row; tiles of 64 and 128 columns with remainders; K split and not, uneven slices
 SHAPES = [(1, 8, 64), (1, 4096, 11008), (16, 2048, 5632), (17, 2056, 832), (32, 6144, 4096), (33, 72, 1024), (48, 11264, 512), (49, 20552, 256),
           (64, 30736, 320), (65, 1000, 4096), (96, 11272, 256), (97, 4104, 11008), (128, 22016, 256), (129, 2048, 7680), (160, 65544, 128),
-          (177, 22024, 192), (192, 520, 2112), (192, 65536, 64)]
+          (177, 22024, 192), (192, 520, 2112), (192, 65536, 64),
+          # one workgroup a CU from 129 rows on; few long slices of 128 columns; more 128-column tiles than CUs
+          (150, 18952, 192), (140, 8328, 1024), (70, 10248, 1280), (100, 10248, 2048), (100, 37896, 64), (180, 37896, 128), (65, 62008, 64)]
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)

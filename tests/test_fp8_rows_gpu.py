@@ -10,7 +10,9 @@ from aphrodite_engine_amd import _lib
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(33, 16, 128), (48, 6144, 4096), (49, 4096, 14336), (64, 28672, 512), (65, 1040, 2048), (96, 10304, 1024), (97, 4096, 4096),
-          (128, 20496, 256), (150, 6144, 4096), (160, 4096, 14336), (161, 28672, 384), (192, 528, 8192), (192, 65552, 128)]
+          (128, 20496, 256), (150, 6144, 4096), (160, 4096, 14336), (161, 28672, 384), (192, 528, 8192), (192, 65552, 128),
+          # one workgroup a CU from 129 rows on; few long slices of 128 columns; more 128-column tiles than CUs
+          (129, 6144, 4096), (150, 18960, 256), (140, 8336, 1024), (100, 10256, 4096), (100, 37904, 128), (180, 37904, 256)]
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)
