@@ -1831,9 +1831,15 @@ def dense_rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
     return out
 
 
+@functools.lru_cache(4096)
+def _dense_rows_preferred(*sizes) -> bool:
+    return bool(_lib.lib().aphro_dense_rows_preferred(*sizes))
+
+
 def dense_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """torch.nn.functional.linear, on ``dense_rows`` where that serves the call."""
-    out = dense_rows(x, weight, bias)
+    """torch.nn.functional.linear, on ``dense_rows`` where that serves the call and is the faster one."""
+    few = x.shape[0] <= 64 or weight.dim() != 2 or _dense_rows_preferred(x.shape[0], *weight.shape)
+    out = dense_rows(x, weight, bias) if few else None
     return torch.nn.functional.linear(x, weight, bias) if out is None else out
 
 

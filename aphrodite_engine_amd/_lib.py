@@ -118,6 +118,7 @@ SIGNATURES = {
     "aphro_fp8_gemm_rows_ksplit": (I, [L, L, L]),
     "aphro_fp8_gemm_rows_preferred": (I, [L, L, L]),
     "aphro_fp8_gemm_rows": (I, [P, P, P, P, P, P, P, Z, L, L, L, I, I, I, P]),
+    "aphro_dense_rows_preferred": (I, [L, L, L]),
     "aphro_dense_rows_slab_floats": (L, [L, L, L, L, L, I]),
     "aphro_dense_rows": (I, [P, L, P, L, P, L, P, P, L, L, L, L, I, I, I, P]),
     "aphro_lm_head_argmax_supported": (I, [L, L, L, L, I]),

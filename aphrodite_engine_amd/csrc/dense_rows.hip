@@ -19,7 +19,8 @@
 //   [11264, 2048]   12.4 / 14.9   13.2 / 15.0   15.4 / 16.2   21.2 / 18.8   26.9 / 26.5
 //   [22016, 4096]   39.5 / 50.5   40.5 / 40.8   43.2 / 43.1   51.2 / 44.7   57.6 / 58.2   (gated: without the 3.5 us of an activation launch)
 //   [128256, 4096]  177 / 186     184 / 195     188 / 208     206 / 233     240 / 294
-// and the call costs the host a third of torch's 24 us.  From 193 rows on two row tiles re-read w and the library is ahead.
+// and the call costs the host a third of torch's 24 us.  From 193 rows on two row tiles re-read w and the library is ahead, from 65 rows on
+// with some wide weights too: aphro_dense_rows_preferred.
 #include "dense_rows.h"
 #include "mixers/mixers_common.h"
 
@@ -178,6 +179,24 @@ extern "C" int64_t aphro_dense_rows_slab_floats(int64_t M, int64_t N, int64_t K,
   const int64_t rows = act >= 0 ? 2 * N : N;
   const RowsPlan plan = rows_plan(M, rows, 2 * K);
   return plan.ksplit > 1 ? plan.ksplit * M * rows : 0;
+}
+
+// Whether the product is the faster one, by the GPU's time, against the library's.  Up to 64 rows of x, narrow weights (the library's host time
+// alone is what those take) and sliced K it is, or within a tenth.  Where K is in one piece, w large and rows many, it is not
+//  * with 64-column tiles, which bring x through LDS twice as often: [12288, 4096], 65 / 128 / 192 rows 31.5 / 37.0 / 48.6 us, library 30.3 / 33.0 /
+//    41.8, [18944, 3584], 96 rows 49 and 37;
+//  * with 128-column tiles that leave more than a tenth of the CUs idle in their last round, from 97 rows on: [22016, 4096], 128 / 160 rows 53 / 58,
+//    library 47 / 53, [28672, 4096] 59 / 62 and 55 / 58, [57344, 8192] 199 / 207 and 191 / 191 (at 65 and 80 rows 45 / 47 and 46 / 46, 54 / 55 and 54 /
+//    64, 183 / 188 and 186 / 178); where more than a third idle, from 65 on ([37888, 3584], 65 / 80 rows 68 / 70 and 65 / 62).
+// [32000, 4096] to [32000, 5120], [62000, 4096], [128256, 4096] and [128256, 8192] fill the CUs: ahead of the library or level with it.
+extern "C" int aphro_dense_rows_preferred(int64_t M, int64_t N, int64_t K) {
+  if (!rows_fits(M, N, 2 * K, 2 * K, 2 * K, false)) return 0;
+  if (M <= 64 || K < 2560 || N * K < 40000000) return 1;
+  const RowsPlan plan = rows_plan(M, N, 2 * K);
+  if (plan.ksplit > 1) return 1;
+  if (plan.nt == 1) return 0;
+  const int64_t tiles = (N + 127) / 128, cus = (tiles + 255) / 256 * 256;
+  return M > 96 ? tiles * 10 >= cus * 9 : tiles * 3 >= cus * 2;
 }
 
 extern "C" int aphro_dense_rows(void* out, int64_t ldo, const void* x, int64_t lda, const void* weight, int64_t ldw, const void* bias,

@@ -998,7 +998,9 @@ int aphro_lm_head_argmax(const void* hidden, int64_t lda, const void* weight, in
 /* out[M, N] = x[M, K] . weight[N, K]^T (+ bias[N]) for up to 192 rows, 16-bit operands, fp32 sums rounded once (out_f32: the rounded
  * values widened).  act 0 (silu) / 1 (gelu, tanh form): weight is [2 N, K] and out = act(x . weight[:N]^T) * (x . weight[N:]^T), no bias;
  * act -1: none.  K % 64 == 0, N % 8 == 0, strides in elements, lda and ldw multiples of 8, operands 16-byte aligned.
- * aphro_dense_rows_slab_floats: fp32 scratch the call needs (0: none), -1 where the form is not served. */
+ * aphro_dense_rows_slab_floats: fp32 scratch the call needs (0: none), -1 where the form is not served.
+ * aphro_dense_rows_preferred: whether it is the faster one against a library product (no activation), for a caller who has both. */
+int aphro_dense_rows_preferred(int64_t M, int64_t N, int64_t K);
 int64_t aphro_dense_rows_slab_floats(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int act);
 int aphro_dense_rows(void* out, int64_t ldo, const void* x, int64_t lda, const void* weight, int64_t ldw, const void* bias, float* slabs,
                      int64_t slab_floats, int64_t M, int64_t N, int64_t K, int act, int out_f32, int dtype, void* stream);

@@ -122,3 +122,10 @@ def test_autocast_chooses_the_type():
         assert got.dtype == torch.float16 and torch.equal(got, F.linear(x, w))
         with torch.autocast("cuda", enabled=False):
             assert ops.dense_linear(x, w).dtype == torch.bfloat16
+
+
+@pytest.mark.parametrize("m,n,k", [(100, 28672, 4096), (70, 12288, 4096)])
+def test_wide_weights_go_to_torch(m, n, k):
+    x, w = _operands(m, n, k, torch.bfloat16, 8)
+    assert torch.equal(ops.dense_linear(x, w), F.linear(x, w))
+    assert torch.equal(ops.dense_linear(x[:40], w), ops.dense_rows(x[:40], w))

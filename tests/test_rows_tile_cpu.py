@@ -19,3 +19,13 @@ def test_slices_of_tiles_that_have_a_cu_to_themselves():
     # 64-column tiles times slices: up to 256 from 129 rows on, up to 512 below
     for n, k, few, many in ((6144, 4096, 5, 2), (9216, 1024, 2, 1), (4608, 3584, 7, 3)):
         assert [slices(m, n, k) for m in (128, 129, 192)] == [few, many, many]
+
+
+def test_wide_weights_that_the_library_serves_better():
+    from aphrodite_engine_amd import _lib
+    ours = lambda m, n, k: bool(_lib.lib().aphro_dense_rows_preferred(m, n, k))
+    assert all(ours(m, n, k) for m in (1, 64) for n, k in ((12288, 4096), (22016, 4096), (57344, 8192)))
+    assert not any(ours(m, n, k) for m in (65, 128, 192) for n, k in ((11264, 4096), (12288, 4096), (15360, 5120), (18944, 3584), (37888, 3584)))
+    assert all(ours(65, n, 4096) and ours(96, n, 4096) and not ours(97, n, 4096) for n in (22016, 28672))
+    assert all(ours(m, n, k) for m in (65, 97, 192) for n, k in ((32000, 4096), (128256, 4096), (4096, 14336), (10240, 8192), (11264, 2048)))
+    assert not ours(193, 4096, 4096) and not ours(16, 4096, 4100)
