@@ -1772,6 +1772,12 @@ def argmax_rows(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Te
 
 _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
 _transforms, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+_hooks_of_all, _pre_hooks_of_all = torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks
+
+
+def unhooked(module: torch.nn.Module) -> bool:
+    """Nothing listens to the module's call: what its forward does may be done without calling it."""
+    return not (module._forward_hooks or module._forward_pre_hooks or _hooks_of_all or _pre_hooks_of_all)
 
 
 def _launchable(*tensors) -> bool:

@@ -209,7 +209,8 @@ class GatedMLP(nn.Module):
 
     def inner(self, h: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """What the output product reads, into ``out`` [T, ff] (dense rows, any row stride) if given."""
-        few = ops.dense_rows(h, self.gate_up.weight, act=self.act, out=out)
+        lin = self.gate_up
+        few = ops.dense_rows(h, lin.weight, act=self.act, out=out) if lin.quant_method is None and lin.bias is None and ops.unhooked(lin) else None
         return mops.act_and_mul(self.gate_up(h), self.act, out) if few is None else few
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
