@@ -936,7 +936,8 @@ class LlamaDecoderLayer(nn.Module):
         then the bias -- once, not per rank.  ``norm``: then fused_add_rms_norm with these weights, in the product's own last launch where it
         has one over whole sums."""
         if self.tp == 1:
-            if norm is not None and lin.bias is None and x.shape[0] > 64 and isinstance(lin.quant_config, (GPTQConfig, AWQConfig)):
+            if norm is not None and lin.bias is None and x.shape[0] > 64 and isinstance(lin.quant_config, (GPTQConfig, AWQConfig)) \
+                    and ops.unhooked(lin):
                 fp = lin.fast_params()
                 if fp is not None:
                     out = ops.wna16_linear_add_norm(x, *fp, getattr(lin, "qweight_strip_major", False), residual, norm, self.cfg.rms_norm_eps)

@@ -32,3 +32,37 @@ def test_gate_and_up(rows):
         assert torch.equal(mlp(h), plain)
         mlp.gate_up.bias = torch.nn.Parameter(torch.full((1024, ), -50.0, dtype=torch.bfloat16, device=DEV))       # (shuts every gate)
         assert mlp(h).abs().max() < 1e-6
+
+
+def _llama(quant, layers=2, kv="auto", dtype=torch.float16):
+    import dataclasses
+    from aphrodite_engine_amd import model as M
+    cfg = dataclasses.replace(M.LLAMA3_8B, num_hidden_layers=layers, vocab_size=512, max_position_embeddings=512)
+    model = M.LlamaForCausalLM(cfg, quant, dtype, kv)
+    model.init_synthetic(torch.device(DEV))
+    return M, cfg, model
+
+
+def _decode(M, cfg, model, rows, kv="auto", dtype=torch.float16):
+    meta, pos, blocks = M.make_decode_metadata(rows, [5 + i % 40 for i in range(rows)], 16, DEV)
+    caches = M.make_kv_caches(cfg, blocks, 16, dtype, kv, DEV, seed=5)
+    ids = torch.arange(rows, device=DEV)
+    return lambda: model(ids, pos, caches, meta)
+
+
+@pytest.mark.parametrize("rows", [70, 150])
+def test_int4_output_projections(rows):
+    from aphrodite_engine_amd.quantization.gptq import GPTQConfig
+    with torch.no_grad():
+        M, cfg, model = _llama(GPTQConfig(4, 128, False))
+        step, seen = _decode(M, cfg, model, rows), []
+        plain = step()
+        handles = [getattr(layer, name).register_forward_hook(lambda module, args, out: seen.append(module))
+                   for layer in model.layers for name in ("o_proj", "down_proj")]
+        assert torch.equal(step(), plain) and seen == [lin for layer in model.layers for lin in (layer.o_proj, layer.down_proj)]
+        for h in handles:
+            h.remove()
+        handle = model.layers[0].o_proj.register_forward_hook(lambda module, args, out: out * 2)
+        assert not torch.equal(step(), plain)
+        handle.remove()
+        assert torch.equal(step(), plain)
