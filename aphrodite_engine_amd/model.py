@@ -1095,10 +1095,16 @@ class LlamaForCausalLM(nn.Module):
             ops.fused_add_rms_norm(hidden, residual, self.norm, self.cfg.rms_norm_eps)
             return hidden
         residual = None
+        if all(type(layer).forward is LlamaDecoderLayer.forward and ops.unhooked(layer) for layer in self.layers):
+            for i, layer in enumerate(self.layers):
+                behind = self.layers[i + 1].input_layernorm if i + 1 < len(self.layers) else self.norm
+                hidden, residual = layer(positions, hidden, residual, kv_caches[i],
+                                         attn_metadata, self.cos_sin, behind)
+            return hidden
+        # somebody looks at the layers' results: rows as they come, their norm in front of the next layer
         for i, layer in enumerate(self.layers):
-            behind = self.layers[i + 1].input_layernorm if i + 1 < len(self.layers) else self.norm
-            hidden, residual = layer(positions, hidden, residual, kv_caches[i],
-                                     attn_metadata, self.cos_sin, behind)
+            hidden, residual = layer(positions, hidden, residual, kv_caches[i], attn_metadata, self.cos_sin)
+        ops.fused_add_rms_norm(hidden, residual, self.norm, self.cfg.rms_norm_eps)
         return hidden
 
     # ---- what the engine (engine.py) asks of a model ------------------------------------------------------------------

@@ -66,3 +66,30 @@ def test_int4_output_projections(rows):
         assert not torch.equal(step(), plain)
         handle.remove()
         assert torch.equal(step(), plain)
+
+
+@pytest.mark.parametrize("rows", [70, 150])
+def test_layers(rows):
+    """A hook on a layer, and a class of its own in a layer's place, see rows that no norm has touched."""
+    from aphrodite_engine_amd import _custom_ops as ops
+    from aphrodite_engine_amd.quantization.gptq import GPTQConfig
+    with torch.no_grad():
+        M, cfg, model = _llama(GPTQConfig(4, 128, False))
+        step, seen = _decode(M, cfg, model, rows), []
+        plain = step()
+        handle = model.layers[1].register_forward_hook(lambda module, args, out: seen.append([t.clone() for t in out]))
+        assert torch.equal(step(), plain)
+        handle.remove()
+        (hidden, residual), = seen
+        ops.fused_add_rms_norm(hidden, residual, model.norm, cfg.rms_norm_eps)
+        assert torch.equal(hidden, plain)
+
+        class Counted(M.LlamaDecoderLayer):
+            calls = 0
+
+            def forward(self, positions, hidden, residual, kv_cache, attn_metadata, cos_sin):
+                Counted.calls += 1
+                return super().forward(positions, hidden, residual, kv_cache, attn_metadata, cos_sin)
+
+        model.layers[0].__class__ = Counted
+        assert torch.equal(step(), plain) and Counted.calls == 1
