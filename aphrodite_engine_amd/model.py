@@ -702,8 +702,12 @@ class LlamaDecoderLayer(nn.Module):
 
     def fused_decode_fp8_rows_ok(self, m: int) -> bool:
         """``fused_decode_fp8_ok``, and beyond its 64 rows whatever the few-rows product leaves as slabs (up to 192)."""
-        return self.fused_decode_fp8_ok(min(m, 64)) and (m <= 64 or all(ops.fp8_gemm_ksplit(m, lin.out_features, lin.in_features) > 0
-                                                                        for lin in self.linears()))
+        return self.fused_decode_fp8_ok(min(m, 64)) and (m <= 64 or self.unhooked() and all(
+            ops.fp8_gemm_ksplit(m, lin.out_features, lin.in_features) > 0 for lin in self.linears()))
+
+    def unhooked(self) -> bool:
+        """No hook listens to the layer's call or to its projections'."""
+        return ops.unhooked(self) and all(ops.unhooked(lin) for lin in self.linears())
 
     def _channel_scale(self, lin) -> torch.Tensor:
         ws = lin.weight_scale
@@ -1086,7 +1090,8 @@ class LlamaForCausalLM(nn.Module):
                 _, _, out = ops.fused_add_rms_norm_quant_fp8(None, prev[0], prev[1], prev[2], residual, True,
                                                              self.norm, self.cfg.rms_norm_eps, want_out=True)
             return out
-        if hidden.shape[0] > 64 and all(l.fused_prefill_fp8_ok() for l in self.layers):
+        if hidden.shape[0] > 64 and all(l.fused_prefill_fp8_ok() for l in self.layers) \
+                and (attn_metadata.num_decode_tokens == 0 or all(l.unhooked() for l in self.layers)):
             # FP8 W8A8 batches of prompts, or of more decoded rows than the fused decode step takes: norm + quant and SiluAndMul + quant fused (forward_prefill_fp8)
             residual = torch.empty_like(hidden)
             for i, layer in enumerate(self.layers):

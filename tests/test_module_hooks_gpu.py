@@ -93,3 +93,16 @@ def test_layers(rows):
 
         model.layers[0].__class__ = Counted
         assert torch.equal(step(), plain) and Counted.calls == 1
+
+
+@pytest.mark.parametrize("rows", [100, 200])
+def test_fp8_steps_of_many_decoded_rows(rows):
+    from aphrodite_engine_amd.quantization.fp8 import CompressedTensorsW8A8Fp8Config
+    with torch.no_grad():
+        M, cfg, model = _llama(CompressedTensorsW8A8Fp8Config("channel", is_static_input_scheme=False), dtype=torch.bfloat16)
+        step, seen = _decode(M, cfg, model, rows, dtype=torch.bfloat16), []
+        plain = step()
+        for module in (model.layers[1], model.layers[0].o_proj):
+            handle = module.register_forward_hook(lambda module, args, out: seen.append(module))
+            assert torch.equal(step(), plain) and seen.pop() is module and not seen
+            handle.remove()
