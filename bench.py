@@ -579,6 +579,18 @@ def prefill_section(cfg):
 
 
 
+def sdpa_varlen(q, k, v, cu_seqlens, max_seqlen, softmax_scale, causal=True, alibi_slopes=None, window_size=None, out=None):
+    """ops.flash_attn_varlen by torch's SDPA, for one sequence (prefill_e2e_section's prompt): the library arm's attention."""
+    import torch.nn.functional as F
+    # [T, H, D] -> [1, H, T, D]; GQA inside SDPA
+    assert cu_seqlens.numel() == 2 and alibi_slopes is None and (window_size is None or window_size[0] < 0)
+    o = F.scaled_dot_product_attention(q.transpose(0, 1).unsqueeze(0), k.transpose(0, 1).unsqueeze(0),
+                                       v.transpose(0, 1).unsqueeze(0), is_causal=causal, scale=softmax_scale,
+                                       enable_gqa=True)
+    o = o.squeeze(0).transpose(0, 1)
+    return o.contiguous() if out is None else out.copy_(o)
+
+
 def prefill_e2e_section(T=8192, library=True, which=("int4", "fp8")):
     """End-to-end prefill (time to first token) of ONE 8192-token prompt -- BASELINE configs[2]'s sequence length -- through
     this package's Llama-3-8B, GPTQ int4 g128 (configs[1]'s model) and compressed-tensors FP8 W8A8 + FP8 KV:
@@ -591,7 +603,6 @@ def prefill_e2e_section(T=8192, library=True, which=("int4", "fp8")):
     (quantization/utils/w8a8_utils.py:130,165), torch SDPA (flash / CK) for the causal attention -- a stated baseline,
     never the target.  frac = time at the dense MFMA peaks (GEMMs at 2.5 PF f16 / 5 PF fp8, attention at 2.5 PF) / time."""
     import dataclasses
-    import torch.nn.functional as F
     from aphrodite_engine_amd import _custom_ops as ops
     from aphrodite_engine_amd import model as M
     from aphrodite_engine_amd.attention.backend import MI355XAttentionMetadata
@@ -600,14 +611,6 @@ def prefill_e2e_section(T=8192, library=True, which=("int4", "fp8")):
     dev = torch.device("cuda", torch.cuda.current_device())
     BS = 16
     out = {}
-
-    def sdpa_varlen(q, k, v, cu_seqlens, max_seqlen, softmax_scale, causal=True, alibi_slopes=None, window_size=None):
-        # one sequence (this section's prompt): [T, H, D] -> [1, H, T, D]; GQA inside SDPA
-        assert cu_seqlens.numel() == 2 and alibi_slopes is None and (window_size is None or window_size[0] < 0)
-        o = F.scaled_dot_product_attention(q.transpose(0, 1).unsqueeze(0), k.transpose(0, 1).unsqueeze(0),
-                                           v.transpose(0, 1).unsqueeze(0), is_causal=causal, scale=softmax_scale,
-                                           enable_gqa=True)
-        return o.squeeze(0).transpose(0, 1).contiguous()
 
     def one(name, qc, kv, gemm_peak):
         cfg = dataclasses.replace(M.LLAMA3_8B, max_position_embeddings=max(8192, T))
