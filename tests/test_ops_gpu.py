@@ -1056,8 +1056,8 @@ def test_flash_attn_varlen_long(ops, dtype, Hq, Hkv, D, causal, alibi):
 def test_flash_attn_varlen_sliding_window(ops, dtype, Hq, Hkv, D, left):
     """Prefill with a sliding window, as ROCmFlashAttentionImpl hands it to flash_attn_varlen_func (window_size = (left, left),
     causal; rocm_flash_attn.py:321-322, 497-507): query i sees keys i - left .. i.  Short and long sequences (both tile
-    machines that take a window, and the head-128 / >= 1024-key shape that would otherwise go to the window-less third
-    generation), windows of one key, around the 64-key tile edge, and wider than every sequence (= plain causal)."""
+    machines that take a window, and the head-128 / >= 1024-key shape that would otherwise go to a window-less
+    kernel), windows of one key, around the 64-key tile edge, and wider than every sequence (= plain causal)."""
     rng = np.random.default_rng(Hq * 5 + D + left)
     lens = [1, 63, 64, 65, 200, 33, 700, 1100]
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
@@ -1079,10 +1079,10 @@ def test_flash_attn_varlen_sliding_window(ops, dtype, Hq, Hkv, D, left):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal", [True, False])
-def test_flash_attn_varlen_v3_kv_head_placement(ops, dtype, causal):
-    """Third-generation prefill kernel with (sequences x kv heads) a multiple of 8: the kv-head -> XCD placement of the
-    workgroups is active (all query heads / query tiles of one kv head on one XCD).  Ragged lengths around the 256-row and
-    64-key tile edges, GQA 2:1, vs the oracle; the unplaced grid (APHRO_FA_NO_XCD) must give the same bits."""
+def test_flash_attn_varlen_v4_kv_head_placement(ops, dtype, causal):
+    """Fourth-generation prefill kernel (the one that places its workgroups; forced on from 1024 keys) with (sequences x kv heads) a
+    multiple of 8: all query heads / query tiles of one kv head on one XCD.  Ragged lengths around the 256-row and 64-key tile edges, GQA
+    2:1, vs the oracle; the unplaced grid (APHRO_FA_NO_XCD) must give the same bits."""
     import os
     rng = np.random.default_rng(5)
     Hq, Hkv, D = 16, 8, 128
@@ -1093,12 +1093,15 @@ def test_flash_attn_varlen_v3_kv_head_placement(ops, dtype, causal):
     q, k, v = qkv.split([Hq * D, Hkv * D, Hkv * D], dim=-1)
     q, k, v = q.view(T, Hq, D), k.view(T, Hkv, D), v.view(T, Hkv, D)
     scale = float(D ** -0.5)
-    got = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, causal=causal)
-    os.environ["APHRO_FA_NO_XCD"] = "1"; ops.reload_env()
+    os.environ["APHRO_FA_V4_MIN_KEYS"] = "1024"; ops.reload_env()
     try:
+        got = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, causal=causal)
+        os.environ["APHRO_FA_NO_XCD"] = "1"; ops.reload_env()
         plain = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, causal=causal)
     finally:
-        del os.environ["APHRO_FA_NO_XCD"]; ops.reload_env()
+        for name in ("APHRO_FA_V4_MIN_KEYS", "APHRO_FA_NO_XCD"):
+            os.environ.pop(name, None)
+        ops.reload_env()
     assert torch.equal(got, plain)
     ref = oa.varlen_causal_attention(q, k, v, cu, scale, causal=causal)
     tol = 2e-3 if dtype == torch.float16 else 1.6e-2
@@ -1111,7 +1114,7 @@ def test_flash_attn_varlen_v3_kv_head_placement(ops, dtype, causal):
 def test_flash_attn_varlen_v4(ops, dtype, causal, alibi, Hq, Hkv):
     """Fourth-generation prefill kernel (one wave per SIMD, two 32-row query blocks per wave, defer-max; flash_attn_v4.hip),
     forced on from 1024 keys: ragged lengths around the 256-row / 64-key tile edges, sequences of one to five tiles next to
-    long ones, GQA, ALiBi (every tile masked), non-causal -- vs the fp64 oracle and vs the third-generation kernel."""
+    long ones, GQA, ALiBi (every tile masked), non-causal -- vs the fp64 oracle and vs the kernel below its key count (flash_attn_short.hip)."""
     import os
     rng = np.random.default_rng(11 + Hq)
     D = 128
@@ -1127,14 +1130,14 @@ def test_flash_attn_varlen_v4(ops, dtype, causal, alibi, Hq, Hkv):
     os.environ["APHRO_FA_V4_MIN_KEYS"] = "1024"; ops.reload_env()
     try:
         got = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, **kw)
-        os.environ["APHRO_FA_V4_MIN_KEYS"] = str(1 << 30); ops.reload_env()       # third generation always
-        third = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, **kw)
+        os.environ["APHRO_FA_V4_MIN_KEYS"] = str(1 << 30); ops.reload_env()       # flash_attn_short.hip always
+        short = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, **kw)
     finally:
         os.environ.pop("APHRO_FA_V4_MIN_KEYS", None); ops.reload_env()
     ref = oa.varlen_causal_attention(q, k, v, cu, scale, causal=causal, alibi_slopes=slopes)
     tol = 2e-3 if dtype == torch.float16 else 1.6e-2
     np.testing.assert_allclose(got.float().cpu().numpy(), ref, atol=tol, rtol=tol)
-    np.testing.assert_allclose(got.float().cpu().numpy(), third.float().cpu().numpy(), atol=tol, rtol=tol)
+    np.testing.assert_allclose(got.float().cpu().numpy(), short.float().cpu().numpy(), atol=tol, rtol=tol)
 
 
 def test_flash_attn_varlen_v4_defer_max_rescale(ops):
