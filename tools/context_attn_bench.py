@@ -1,6 +1,5 @@
 #!/usr/bin/env python3
-"""Round 3: prefill with cached context outside the third-generation kernel's sweet spot (head 128, >= 1024 keys, no
-window): gather-once + second / first generation tile machines (the default) vs the round-1 scalar-gather kernel
+"""Prefill with cached context: gather-once + the prompt kernels (the default) vs the scalar-gather kernel
 (APHRO_CA_NO_GATHER=1).  HIP events over 10 calls."""
 import json
 import os
@@ -18,7 +17,7 @@ CASES = [  # name, batch, ctx, new, Hq, Hkv, D, window
     ("hd64: 4 x (2048 cached + 512 new)", 4, 2048, 512, 32, 8, 64, None),
     ("hd96: 4 x (1024 cached + 512 new)", 4, 1024, 512, 24, 8, 96, None),
     ("hd256: 2 x (1024 cached + 512 new)", 2, 1024, 512, 8, 4, 256, None),
-    ("hd128 long (third generation): 6144 cached + 2048 new", 1, 6144, 2048, 32, 8, 128, None),
+    ("hd128 long: 6144 cached + 2048 new", 1, 6144, 2048, 32, 8, 128, None),
 ]
 
 
