@@ -4,7 +4,7 @@
 //   * A workgroup owns 64 or 128 rows of w and ALL rows of x, so x crosses L2 M / 64 or M / 128 times as often as w.  (A first form with one
 //     16-row tile of w per workgroup and fragments straight from global memory read x 2-4 times as often as w: 36 us where this one
 //     takes 23 on [4096, 11008] with 32 rows.)
-//   * Both operands go through LDS in steps of 64 k by LDS-DMA, 8 rows of a full 128-byte line per instruction, 2 to 5 steps ahead; chunk
+//   * Both operands go through LDS in steps of 64 k by LDS-DMA, 8 rows of a full 128-byte line per instruction, 1 to 5 steps ahead; chunk
 //     j of row r lies at j ^ (r & 7), which leaves the fragment reads without bank conflicts.  One barrier a step.
 //   * Few column tiles: K is split over workgroups, each slice's sums go to a slab, a second small launch adds the slabs in order (no state
 //     between calls, the same bits every time).

@@ -10,7 +10,8 @@
 // causal): against 64-row workgroups with V transposed number by number, below 512 keys, 300 tokens 18.8 / 13.7, five prompts of 107 to 430 39.4 /
 // 20.4; against the second generation's 128 rows a workgroup, 1000 tokens 45.5 / 30.8, five of 600 61.9 / 39.1, three of 1000 94 / 53; against the
 // third's 256 rows (deleted), 1111 tokens 45.2 / 35.5, 3000 116.7 / 101.8, three of 1500 107 / 90, six of 1300 161 / 128.  The fourth: 4096 tokens
-// 176 / 187, 8192 596 / 604, but 5000 267 / 247.  Below 64 keys the first is the faster (six of 26 tokens 6.1 / 7.4).
+// 176 / 187, 8192 596 / 604, but 5000 267 / 247: the line at 4096 keys does not look at how full the last of its 256-row tiles is.  Below 64 keys the
+// first is the faster (six of 26 tokens 6.1 / 7.4).
 // Loads hidden from hipcc, which otherwise waits for the next tile in front of the transposing reads: no faster (three of 1000 tokens 53 / 55).
 #include "common.h"
 #include "flash_attn_common.h"

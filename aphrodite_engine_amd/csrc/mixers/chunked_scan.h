@@ -148,7 +148,7 @@ __device__ __forceinline__ u16x8 load8_bits(const uint16_t* __restrict__ row, in
   return w;
 }
 
-// An fp32 number as the sum of three bf16 ones, exactly (8 + 8 + 8 bits of its 24): a product with a bf16 number is then three products on the
+// An fp32 number as the sum of three bf16 ones, exactly (8 + 8 + 8 bits of its 24; below about 2^-110 the last bits fall out of bf16's range): a product with a bf16 number is then three products on the
 // 16-bit matrix cores, each exact, for a quarter of the time of the fp32 ones.  What is not finite stays in the first part.
 __device__ __forceinline__ void split3(float x, uint16_t (&p)[3]) {
   const uint32_t u = __builtin_bit_cast(uint32_t, x);
