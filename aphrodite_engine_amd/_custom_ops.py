@@ -1780,16 +1780,19 @@ def unhooked(module: torch.nn.Module) -> bool:
     return not (module._forward_hooks or module._forward_pre_hooks or _hooks_of_all or _pre_hooks_of_all)
 
 
+_grad_enabled, _autocast, _compiling, _plain = torch.is_grad_enabled, torch.is_autocast_enabled, torch.compiler.is_compiling, \
+    frozenset((torch.Tensor, torch.nn.Parameter))
+
+
 def _launchable(*tensors) -> bool:
     """Tensors whose memory a kernel may be launched on right away: nothing records, traces, differentiates or batches what happens to them."""
-    if _forward_ad._current_level >= 0:                  # (a dual tensor is a plain one that needs no gradient)
+    if _forward_ad._current_level >= 0 or _autocast():   # (a dual tensor is a plain one that needs no gradient; autocast chooses a product's types)
         return False
-    grad = torch.is_grad_enabled()
+    grad = _grad_enabled()
     for t in tensors:
-        if type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad):
+        if type(t) not in _plain or (grad and t.requires_grad):
             return False
-    return not (_dispatch_modes() or _function_modes() or _transforms() or _tracing() or torch.compiler.is_compiling()
-                or torch.is_autocast_enabled())          # (autocast chooses a product's types)
+    return not (_dispatch_modes() or _function_modes() or _transforms() or _tracing() or _compiling())
 
 
 @functools.lru_cache(4096)
