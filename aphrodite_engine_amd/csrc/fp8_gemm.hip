@@ -451,10 +451,15 @@ static int fp8_gemm_common(Fp8GemmParams p, bool a8, int dtype, void* workspace,
 
 using namespace aphro;
 
+// Enough for calls of fewer rows too: the few-rows plan changes behind 64 and 128 rows, and a taller batch may have fewer K slices.
 extern "C" size_t aphro_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  const int64_t m = M < 64 ? M : 64;
-  const size_t few = (size_t)8 * m * N * sizeof(float), rows = (size_t)aphro_fp8_gemm_rows_ksplit(M, N, K) * M * N * sizeof(float);
-  return rows > few ? rows : few;
+  size_t most = (size_t)8 * (M < 64 ? M : 64) * N;
+  for (int64_t m : {64, 128, 192}) {
+    if (m > M) m = M;
+    const size_t rows = (size_t)aphro_fp8_gemm_rows_ksplit(m, N, K) * m * N;
+    if (rows > most) most = rows;
+  }
+  return most * sizeof(float);
 }
 
 extern "C" int aphro_scaled_mm_fp8(void* out, const void* a, const void* b, const float* a_scales,

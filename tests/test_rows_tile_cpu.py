@@ -29,3 +29,13 @@ def test_wide_weights_that_the_library_serves_better():
     assert all(ours(65, n, 4096) and ours(96, n, 4096) and not ours(97, n, 4096) for n in (22016, 28672))
     assert all(ours(m, n, k) for m in (65, 97, 192) for n, k in ((32000, 4096), (128256, 4096), (4096, 14336), (10240, 8192), (11264, 2048)))
     assert not ours(193, 4096, 4096) and not ours(16, 4096, 4100)
+
+
+def test_a_workspace_for_many_rows_serves_fewer():
+    from aphrodite_engine_amd import _lib
+    lib = _lib.lib()
+    for n in (1024, 1280, 4096, 4608, 6144, 7168, 9216, 10240, 17408, 28672):
+        for k in (1024, 2048, 4096, 8192, 28672):
+            sizes = [lib.aphro_fp8_gemm_workspace_bytes(m, n, k) for m in range(1, 301)]
+            assert sizes == sorted(sizes)
+            assert all(sizes[m - 1] >= 4 * m * n * lib.aphro_fp8_gemm_rows_ksplit(m, n, k) for m in range(33, 193))
