@@ -12,10 +12,15 @@
 //     waves' at once, behind the barrier, made the waves wait for the address unit with the matrix cores idle (28672 x 4096, 150 rows:
 //     48.9 -> 41.8 us).
 //   * K slices write the accumulators as they lie in the registers, 1 KiB a store; a second kernel sums them in the order of K.
-// Bound by the activations' way into LDS and the MFMAs together: 1.2 us per K tile of 160 rows on every CU, 0.53 us of it MFMA.
+//   * what a wave issues is the other limit: with the scalar arithmetic of a tile's addresses (57 operations), its zero points' 64-bit
+//     addresses and the fragment reads of a step in one place, the first four waves of a CU needed 1 205 cycles a tile alone, and the
+//     other four, behind them, as many again beside their MFMAs.  Running offsets, groups by one multiplication, empty buffers behind the
+//     slice and one MFMA, one read or load and three or four operations of the unpacking a slot: 19 scalar operations of 143 in all.
+// Bound by MFMAs, which pull the clock to 1.65 GHz: 1 670 cycles per K tile of 160 rows (1 900 before), 1 280 of them MFMA.
 // Layer of Llama-3-8B at 150 rows, four GEMMs with their slab sums: 192 -> 114 us (qkv 40.4 -> 24, o 27.3 -> 17, gate_up 76 -> 42,
 // down 48 -> 31); at 65 rows 128 -> 79; at 1300 rows 756 -> 629 us.
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "row_norm.h"
@@ -31,25 +36,11 @@ __device__ __forceinline__ uint32_t rw_and_or(uint32_t a, uint32_t mask, uint32_
   asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(mask), "v"(orv));
   return r;
 }
-// one exllama dword -> 8 f16: (1024 + q) - (1024 + z), exact, and times the scale where SCALED (one rounding)
-template <bool SCALED>
-__device__ __forceinline__ f16x8 rw_dq8(uint32_t w, f16x2 zh, f16x2 zh16, f16x2 sc) {
-  const f16x2 inv16 = {(f16)0.0625f, (f16)0.0625f};
-  const uint32_t magic = 0x64006400u;
-  const uint32_t q0 = rw_and_or(w, 0x000f000fu, magic);
-  const uint32_t q1 = rw_and_or(w, 0x00f000f0u, magic);
-  const uint32_t w8 = w >> 8;
-  const uint32_t q2 = rw_and_or(w8, 0x000f000fu, magic);
-  const uint32_t q3 = rw_and_or(w8, 0x00f000f0u, magic);
-  f16x2 d0 = __builtin_bit_cast(f16x2, q0) - zh;
-  f16x2 d1 = __builtin_bit_cast(f16x2, q1) * inv16 + zh16;
-  f16x2 d2 = __builtin_bit_cast(f16x2, q2) - zh;
-  f16x2 d3 = __builtin_bit_cast(f16x2, q3) * inv16 + zh16;
-  if constexpr (SCALED) d0 *= sc, d1 *= sc, d2 *= sc, d3 *= sc;
-  u32x4 r = {__builtin_bit_cast(uint32_t, d0), __builtin_bit_cast(uint32_t, d1), __builtin_bit_cast(uint32_t, d2),
-             __builtin_bit_cast(uint32_t, d3)};
-  return __builtin_bit_cast(f16x8, r);
-}
+// f(integral_constant 0), .. f(integral_constant N - 1)
+template <typename F, int... I>
+__device__ __forceinline__ void rw_unroll_(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void rw_unroll(F&& f) { rw_unroll_(f, std::make_integer_sequence<int, N>{}); }
 
 constexpr int RW_BN = 128, RW_BK = 128, RW_STAGES = 4;
 constexpr int rw_pass(int mb) { return (mb + 1) / 2; }      // 32-row blocks whose K groups meet in LDS at a time
@@ -88,9 +79,9 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   const int tn = lin % p.tiles_n, rest = lin / p.tiles_n, tm = rest % p.tiles_m, ks = rest / p.tiles_m;
   const int m0 = tm * MB * 32, n0 = tn * RW_BN;
   const int T = p.K / RW_BK, t0 = ks * T / p.ksplit, t1 = (ks + 1) * T / p.ksplit;
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a) + (size_t)m0 * p.lda, 0,
-                                                                      (uint32_t)((size_t)(p.M - m0) * p.lda * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qw), 0, (uint32_t)((size_t)(p.K >> 3) * p.N * 4), 0x00020000);
+  __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a) + (size_t)m0 * p.lda, 0,
+                                                                (uint32_t)((size_t)(p.M - m0) * p.lda * 2), 0x00020000);
+  __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qw), 0, (uint32_t)((size_t)(p.K >> 3) * p.N * 4), 0x00020000);
   // ---- activations: one DMA instruction = 4 rows of 256 B, rows 32 apart from one to the next; LDS slot s of row r holds the row's
   // slot s ^ (r & 15).  Rows from M on read zeros (the buffer ends there); 32-row blocks that begin behind M read the last one that does
   // not, because a scalar offset past the buffer's end is not certain to fail the range check.  Nobody stores either. ------------------
@@ -99,49 +90,91 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   // ---- weights: the lane's columns are col and col + 1 (MFMA row i of block nb is column 2 i + nb) -------------------------------
   const int col = n0 + wn * 64 + 2 * l31;
   uint32_t w_voff, mult = 0;
-  if constexpr (STRIP) w_voff = wna16_strip_col(p.strip, col & ~3, mult) + (uint32_t)(col & 3) + mult * 64u * (uint32_t)kh;
+  if constexpr (STRIP) w_voff = wna16_strip_col(p.strip, col & ~3, mult) + (uint32_t)(col & 3) + mult * (64u * (uint32_t)kh + 16u * (uint32_t)kg);
   else w_voff = (uint32_t)((kg * 4 + kh) * p.N + col);
   w_voff *= 4u;
-  const uint32_t* scp = reinterpret_cast<const uint32_t*>(p.sc + col);
-  const uint32_t* zp = p.qz + (col >> 3);
+  const uint32_t mult4 = mult * 4u;
+  __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.sc), 0, (uint32_t)(p.K / p.group_size * p.N * 2), 0x00020000);
+  __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qz), 0, (uint32_t)(p.K / p.group_size * (p.N >> 3) * 4), 0x00020000);
+  const int sc_voff = col * 2, z_voff = (col >> 3) * 4;
   const int zshift = (col & 7) * 4;
   const int first_k = t0 * RW_BK + kg * 32, first_grp = first_k / p.group_size, first_in = first_k - first_grp * p.group_size;
-  int t_load = t0, grp = first_grp, in_group = first_in;  // the tile the next load fetches; its group, the k inside the group
-  const int grp_step = RW_BK / p.group_size, grp_rest = RW_BK - grp_step * p.group_size;
+  // Where the next load fetches, scalar: k of the wave's part (its group by a multiplication), the tiles until a chunk of the strip-major copy or
+  // the slice ends.  Behind the slice's end the buffers are empty: the loop stays straight-line code, and nothing is fetched.
+  const uint32_t sc_row = (uint32_t)p.N * 2u;
+  uint32_t k_load = (uint32_t)(t0 * RW_BK + kg * 32), sc_off, z_off;
+  uint32_t w_off, w_vrun = w_voff, a_run = (uint32_t)a_voff + (uint32_t)t0 * (RW_BK * 2);
+  int t_load = t0, event;
+  auto place = [&] {
+    if constexpr (STRIP) {
+      uint32_t chunk, R;
+      wna16_strip_row(p.strip, (uint32_t)t_load * 16u, chunk, R);
+      w_off = chunk * 4u;
+      w_vrun = w_voff + __umul24(mult4, R);
+      event = min(p.strip.nseg - (int)(R >> 8), t1 - t_load);
+    } else {
+      w_off = (uint32_t)t_load * 64u * (uint32_t)p.N;
+      event = t1 - t_load;
+    }
+  };
+  auto groups = [&] {
+    const uint32_t g = (uint32_t)(((uint64_t)k_load * p.inv_group) >> 32);
+    sc_off = g * sc_row;
+    z_off = sc_off >> 2;
+  };
+  place();
+  groups();
   u32x2 wr[3][2];
   uint32_t scr[3], zr[3];
-  auto load_w = [&](auto set) {
+  auto load_meta = [&](auto set) {
     constexpr int S = decltype(set)::value;
-    if constexpr (!EXACT) scr[S] = scp[(size_t)grp * (p.N >> 1)];
-    zr[S] = zp[(size_t)grp * (p.N >> 3)];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      if constexpr (STRIP) {
-        uint32_t chunk, R;
-        wna16_strip_row(p.strip, (uint32_t)(t_load * 16 + kg * 4), chunk, R);
-        wr[S][j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, (int)(w_voff + mult * (R + 128u * j) * 4u), (int)(chunk * 4u), 0));
+    if constexpr (!EXACT) scr[S] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, sc_voff, (int)sc_off, 0);
+    zr[S] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rz, z_voff, (int)z_off, 0);
+  };
+  auto load_w = [&](auto set, int j) {
+    constexpr int S = decltype(set)::value;
+    if constexpr (STRIP)
+      wr[S][j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, (int)(j ? w_vrun + mult4 * 128u : w_vrun), (int)w_off, 0));
+    else
+      wr[S][j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, (int)w_voff, (int)w_off + 2 * j * p.N * 4, 0));
+  };
+  auto load_a = [&](uint32_t st, int i) {
+    const int voff = (int)a_run;                           // (a local copy: see wna16_gemm_large.hip)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_ptr)(smem + st + (i * 8 + wave) * 1024), 16, voff,
+                                             (int)((uint32_t)min(i, last_block) * 64u * (uint32_t)p.lda), 0, 0);
+  };
+  auto advance_groups = [&] { k_load += RW_BK; groups(); };
+  auto advance_tile = [&] {
+    ++t_load;
+    a_run += RW_BK * 2;
+    if constexpr (STRIP) w_vrun += mult4 * 256u;
+    else w_off += 64u * (uint32_t)p.N;
+    if (__builtin_expect(--event == 0, 0)) {
+      if (t_load == t1) {
+        ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a) + (size_t)m0 * p.lda, 0, 0, 0x00020000);
+        rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qw), 0, 0, 0x00020000);
+        rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.sc), 0, 0, 0x00020000);
+        rz = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qz), 0, 0, 0x00020000);
+        event = 0x7fffffff;
       } else {
-        wr[S][j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, (int)w_voff, (t_load * 16 + 2 * j) * p.N * 4, 0));
+        place();
       }
     }
   };
-  auto load_a = [&](int st, int i) {
-    const int voff = a_voff;                               // (a local copy: see wna16_gemm_large.hip)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void_ptr)(smem + st * STAGE + (i * 8 + wave) * 1024), 16, voff,
-                                             (int)((uint32_t)t_load * (RW_BK * 2) + (uint32_t)min(i, last_block) * 64u * (uint32_t)p.lda), 0, 0);
+  // EXACT: one tile on, behind the slice's end not, without a branch (one among the sums costs registers, here more than there are)
+  auto stay = [&] {
+    t_load = min(t_load + 1, t1 - 1);
+    k_load = (uint32_t)(t_load * RW_BK + kg * 32);
+    a_run = (uint32_t)a_voff + (uint32_t)t_load * (RW_BK * 2);
+    place();
+    groups();
   };
-  auto advance = [&] {
-    ++t_load;
-    grp += grp_step;
-    in_group += grp_rest;
-    if (in_group >= p.group_size) { in_group -= p.group_size; ++grp; }
-    if (t_load == t1) { t_load = t0; grp = first_grp; in_group = first_in; }      // (behind the last tile: straight-line code)
-  };
-  auto load = [&](auto set, int st) {
-    load_w(set);
+  auto load = [&](auto set, uint32_t st) {
+    load_w(set, 0);
+    load_w(set, 1);
+    load_meta(set);
 #pragma unroll
     for (int i = 0; i < MB; ++i) load_a(st, i);
-    advance();
   };
   constexpr int LOADS = MB + (EXACT ? 3 : 4);              // memory instructions of one load()
   f32x16 acc[2][MB], total[EXACT ? 2 : 1][EXACT ? MB : 1];
@@ -169,6 +202,7 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
     }
     asm volatile("" ::: "memory");                         // (ahead of the loads that are counted)
   }
+  const int grp_step = RW_BK / p.group_size, grp_rest = RW_BK - grp_step * p.group_size;
   int tile_grp = first_grp, tile_in = first_in;             // of the tile being multiplied
   auto fold = [&] {
     const unsigned char* row = sc_lds + (tile_grp - slice_grp) * (RW_BN * 2) + wn * 128 + kh * 16;
@@ -194,73 +228,102 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   f16x8 wf[2][2];
   f16x2 zh[2], zh16[2], sv[2];
   const uint32_t a_base = (uint32_t)l31 * 256u;
-  auto read_a = [&](int stage, int j, u32x4 (&x)[MB]) {
-    const unsigned char* sa = smem + stage * STAGE + (a_base + (((uint32_t)(kg * 4 + 2 * j + kh) ^ (uint32_t)(l31 & 15)) << 4));
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) x[mb] = *reinterpret_cast<const u32x4*>(sa + mb * 8192);
-  };
-  auto meta = [&](auto set) {
+  const uint32_t a_read[2] = {a_base + (((uint32_t)(kg * 4 + kh) ^ (uint32_t)(l31 & 15)) << 4),
+                              a_base + (((uint32_t)(kg * 4 + 2 + kh) ^ (uint32_t)(l31 & 15)) << 4)};
+  auto read_a = [&](uint32_t st, int j, int mb) { af[j][mb] = *reinterpret_cast<const u32x4*>(smem + st + a_read[j] + mb * 8192); };
+  auto meta = [&](auto set, int nb) {
     constexpr int S = decltype(set)::value;
+    uint16_t sb = 0;
+    if constexpr (!EXACT) sb = (uint16_t)(nb ? scr[S] >> 16 : scr[S]);
+    const int z = (int)((zr[S] >> (zshift + 4 * nb)) & 0xf) + p.zero_offset;
+    const f16 s16 = BF16 ? (f16)bf16_bits_to_f32(sb) : __builtin_bit_cast(f16, sb);
+    const f16 a16 = __builtin_bit_cast(f16, (uint16_t)(0x6400 | z));       // 1024 + z
+    const f16 b16 = (f16)960.f - a16;                                      // -64 - z
+    sv[nb] = f16x2{s16, s16};
+    zh[nb] = f16x2{a16, a16};
+    zh16[nb] = f16x2{b16, b16};
+  };
+  f16x2 diff[2][4];
+  uint32_t high[2], biased[2][4];
+  // the weights of a step, an exllama dword a column: (1024 + q) - (1024 + z), exact, and times the scale (one rounding; EXACT: not here), in
+  // pieces of 3 or 4 operations
+  auto unpack_piece = [&](auto set, auto step, auto piece) {
+    constexpr int S = decltype(set)::value, J = decltype(step)::value, P = decltype(piece)::value, nb = P >> 2, q = P & 3;
+    const f16x2 inv16 = {(f16)0.0625f, (f16)0.0625f};
+    const uint32_t magic = 0x64006400u;
+    const uint32_t w = wr[S][J][nb];
+    if constexpr (q == 0) {
+      biased[nb][0] = rw_and_or(w, 0x000f000fu, magic);
+      biased[nb][1] = rw_and_or(w, 0x00f000f0u, magic);
+      high[nb] = w >> 8;
+    } else if constexpr (q == 1) {
+      biased[nb][2] = rw_and_or(high[nb], 0x000f000fu, magic);
+      biased[nb][3] = rw_and_or(high[nb], 0x00f000f0u, magic);
+      diff[nb][0] = __builtin_bit_cast(f16x2, biased[nb][0]) - zh[nb];
+    } else if constexpr (q == 2) {
+      diff[nb][1] = __builtin_bit_cast(f16x2, biased[nb][1]) * inv16 + zh16[nb];
+      diff[nb][2] = __builtin_bit_cast(f16x2, biased[nb][2]) - zh[nb];
+      diff[nb][3] = __builtin_bit_cast(f16x2, biased[nb][3]) * inv16 + zh16[nb];
+    } else {
+      f16x2 d[4];
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
-      uint16_t sb = 0;
-      if constexpr (!EXACT) sb = (uint16_t)(nb ? scr[S] >> 16 : scr[S]);
-      const int z = (int)((zr[S] >> (zshift + 4 * nb)) & 0xf) + p.zero_offset;
-      const f16 s16 = BF16 ? (f16)bf16_bits_to_f32(sb) : __builtin_bit_cast(f16, sb);
-      const f16 a16 = __builtin_bit_cast(f16, (uint16_t)(0x6400 | z));       // 1024 + z
-      const f16 b16 = (f16)960.f - a16;                                      // -64 - z
-      sv[nb] = f16x2{s16, s16};
-      zh[nb] = f16x2{a16, a16};
-      zh16[nb] = f16x2{b16, b16};
+      for (int i = 0; i < 4; ++i) d[i] = EXACT ? diff[nb][i] : diff[nb][i] * sv[nb];
+      wf[J][nb] = __builtin_bit_cast(f16x8, u32x4{__builtin_bit_cast(uint32_t, d[0]), __builtin_bit_cast(uint32_t, d[1]),
+                                                  __builtin_bit_cast(uint32_t, d[2]), __builtin_bit_cast(uint32_t, d[3])});
     }
   };
   auto unpack = [&](auto set, auto step) {
-    constexpr int S = decltype(set)::value, J = decltype(step)::value;
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb) wf[J][nb] = rw_dq8<!EXACT>(wr[S][J][nb], zh[nb], zh16[nb], sv[nb]);
+    rw_unroll<8>([&](auto piece) { unpack_piece(set, step, piece); });
   };
-  auto multiply = [&](auto step) {
+  auto multiply = [&](auto step, int i) {
     constexpr int J = decltype(step)::value;
     const f32x16 zero = {};
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
-        acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[J][nb], __builtin_bit_cast(f16x8, af[J][mb]), EXACT && J == 0 ? zero : acc[nb][mb], 0, 0, 0);
+    const int mb = i >> 1, nb = i & 1;
+    acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[J][nb], __builtin_bit_cast(f16x8, af[J][mb]), EXACT && J == 0 ? zero : acc[nb][mb], 0, 0, 0);
   };
-  int stage = 0;                                           // of the tile being multiplied
+  uint32_t before = 3 * STAGE, here = 0;                   // stages of the tile ahead of the one being multiplied, and of that one
   auto tile = [&](auto set, auto more) {
-    constexpr int S = decltype(set)::value;
-    read_a(stage, 1, af[1]);
-    unpack(set, std::integral_constant<int, 1>{});
-    multiply(std::integral_constant<int, 0>{});
-    if constexpr (decltype(more)::value) {
-      // the next tile has landed once at most the loads of ONE load(), the tile after it, are outstanding; past the barrier every wave
-      // is through with the tile BEFORE this one, whose stage the loads issued now take
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(LOADS) : "memory");
-      __builtin_amdgcn_s_barrier();
-    }
-    const int fetch = (stage + 3) & 3;
-    stage = (stage + 1) & 3;
-    read_a(stage, 0, af[0]);
-    meta(std::integral_constant<int, (S + 1) % 3>{});
-    unpack(std::integral_constant<int, (S + 1) % 3>{}, std::integral_constant<int, 0>{});
-    if constexpr (decltype(more)::value) {
-      // the loads go out between the MFMAs: all waves' at once would wait for one another with the matrix cores idle
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-          acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[1][nb], __builtin_bit_cast(f16x8, af[1][mb]), acc[nb][mb], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0x86);
-        if (mb == 0) load_w(set);
-        load_a(fetch, mb);
-        __builtin_amdgcn_sched_barrier(0x86);
-      }
-      advance();
-    } else {
-      multiply(std::integral_constant<int, 1>{});
-    }
+    constexpr int S = decltype(set)::value, SLOTS = 2 * MB;
+    constexpr bool MORE = decltype(more)::value;
+    constexpr std::integral_constant<int, 0> step0{};
+    constexpr std::integral_constant<int, 1> step1{};
+    constexpr std::integral_constant<int, (S + 1) % 3> next{};
+    if constexpr (MORE && EXACT) stay();
+    // A slot: one MFMA and what fits its 64 cycles (two waves share a matrix pipe).  First 16 k: the others' fragments are read, their
+    // weights unpacked; scalars one tile on.
+    rw_unroll<SLOTS>([&](auto slot) {
+      constexpr int I = decltype(slot)::value, P0 = I * 8 / SLOTS, P1 = (I + 1) * 8 / SLOTS;
+      multiply(step0, I);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (I < MB) read_a(here, 1, I);
+      if constexpr (MORE && !EXACT && I == 1) advance_groups();
+      if constexpr (MORE && !EXACT && I == 3) advance_tile();
+      rw_unroll<P1 - P0>([&](auto i) { unpack_piece(set, step1, std::integral_constant<int, P0 + decltype(i)::value>{}); });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    // the next tile has landed once at most the loads of the one behind it are outstanding; past the barrier every wave is through with the
+    // tile BEFORE this one, whose stage the loads issued now take
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(LOADS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint32_t fetch = before;
+    before = here;
+    here = here == 3 * STAGE ? 0 : here + STAGE;
+    __builtin_amdgcn_sched_barrier(0);
+    // the loads go out between the MFMAs: all waves' at once would wait for one another with the matrix cores idle
+    rw_unroll<SLOTS>([&](auto slot) {
+      constexpr int I = decltype(slot)::value, P0 = I < 1 ? 0 : (I - 1) * 8 / (SLOTS - 1), P1 = I * 8 / (SLOTS - 1);
+      multiply(step1, I);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (I < MB) read_a(here, 0, I);
+      if constexpr (MORE && I < 2) load_w(set, I);
+      if constexpr (MORE && I == 2) load_meta(set);
+      if constexpr (I == 1) meta(next, 0);
+      if constexpr (I == SLOTS / 2) meta(next, 1);
+      if constexpr (MORE && I >= SLOTS - MB) load_a(fetch, I - (SLOTS - MB));
+      rw_unroll<P1 - P0>([&](auto i) { unpack_piece(next, step0, std::integral_constant<int, P0 + decltype(i)::value>{}); });
+      __builtin_amdgcn_sched_barrier(0);
+    });
     if constexpr (EXACT) {
       fold();
       __builtin_amdgcn_sched_barrier(0);                   // (the next tile's sums would be a second set of accumulators)
@@ -269,19 +332,31 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   constexpr std::integral_constant<int, 0> set0{};
   constexpr std::integral_constant<int, 1> set1{};
   constexpr std::integral_constant<int, 2> set2{};
+  auto advance = [&] {
+    if constexpr (EXACT) {
+      stay();
+    } else {
+      advance_groups();
+      advance_tile();
+    }
+  };
   load(set0, 0);
   asm volatile("" ::: "memory");                           // (the counted waits rely on the order of the loads)
-  load(set1, 1);
+  advance();
+  load(set1, STAGE);
   asm volatile("" ::: "memory");
-  load(set2, 2);
+  advance();
+  load(set2, 2 * STAGE);
   if constexpr (EXACT) {
 #pragma unroll
     for (int i = 0; i < SC_LOADS; ++i) reinterpret_cast<uint32_t*>(sc_lds)[threadIdx.x + 512 * i] = sc_reg[i];
   }
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(2 * LOADS) : "memory");
   __builtin_amdgcn_s_barrier();
-  read_a(0, 0, af[0]);
-  meta(set0);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) read_a(0, 0, mb);
+  meta(set0, 0);
+  meta(set0, 1);
   unpack(set0, std::integral_constant<int, 0>{});
   int left = t1 - t0;
   for (; left >= 3; left -= 3) {
@@ -289,12 +364,10 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
     tile(set1, std::true_type{});
     tile(set2, std::true_type{});
   }
-  // The last one or two tiles, in flight or landed.  They issue no loads: ones that nobody reads are dropped by the compiler, and a
-  // counted wait behind them would let a tile's own activations be outstanding.
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
+  // the last one or two tiles, whose loads the loop has issued
   if (left > 0) tile(set0, std::false_type{});
   if (left > 1) tile(set1, std::false_type{});
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   // ---- the four K groups meet in LDS: the wave of group g ends with quad g of every block, columns 16 g + 8 kh + 2 r + nb ----------
   constexpr int RM = rw_pass(MB);
   auto& sum = [&]() -> f32x16 (&)[2][MB] {
@@ -449,13 +522,17 @@ __global__ void wna16_rows_norm_kernel(Wna16RowsParams p, int pad_rows) {
   }
 }
 
+static uint32_t rw_inv_group(int64_t gs) { return (uint32_t)((0x100000000ll + gs - 1) / gs); }
+// whether k * inv_group >> 32 is k / group_size for all k < K: but for odd groups of a K of 65536 and more it always is
+static bool rw_groups_exact(int64_t K, int64_t gs) { return (rw_inv_group(gs) * gs - 0x100000000ll) * K < 0x100000000ll; }
+
 // Tile height and K slices by the time they are expected to take (MI355X, ns; within 10 % of what was measured for 65 .. 4096 rows of
 // Llama-3-8B's and -70B's matrices): rounds of workgroups over the CUs, each 170 + 200 per 32-row block and K tile and 4.7 us around
 // them, and the slabs written and read again at 2.2 TB/s behind 3 us.  4096 x 14336, 150 rows: one slice 115 us, two 56, four 35, eight
 // 30; 4096 x 4096, 150 rows: five blocks and five slices 20.7, twice three blocks and four slices 18.0 us.
 Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t gs, int64_t slab_bytes, int64_t other_ns) {
   Wna16RowsPlan best = {0, 1, false};
-  if (M <= 64 || M > 4096 || N % RW_BN || K % RW_BK || gs % 64) return best;
+  if (M <= 64 || M > 4096 || N % RW_BN || K % RW_BK || gs % 64 || !rw_groups_exact(K, gs)) return best;
   const int cus = device_cu_count();
   const int64_t T = K / RW_BK;
   int64_t best_ns = other_ns;
@@ -475,7 +552,7 @@ Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t gs, int64
 // The EXACT form, 65 to 128 rows: two tiles of 64.  K slices by the time they are expected to take, as above; a slice's groups fit its LDS.
 Wna16RowsPlan wna16_rows_plan_exact(int64_t M, int64_t N, int64_t K, int64_t gs, int64_t slab_bytes) {
   Wna16RowsPlan best = {0, 1, true};
-  if (M <= 64 || M > 128 || N % RW_BN || K % RW_BK || gs % 64) return best;
+  if (M <= 64 || M > 128 || N % RW_BN || K % RW_BK || gs % 64 || !rw_groups_exact(K, gs)) return best;
   const int cus = device_cu_count();
   const int64_t T = K / RW_BK, tiles = 2 * (N / RW_BN);
   int64_t best_ns = -1;
@@ -495,6 +572,7 @@ template <int MB, bool BF16, bool STRIP, bool EXACT>
 static int rows_launch(Wna16RowsParams p, hipStream_t st) {
   p.tiles_m = (p.M + MB * 32 - 1) / (MB * 32);
   p.tiles_n = p.N / RW_BN;
+  p.inv_group = rw_inv_group(p.group_size);
   static bool attr_set_dev[APHRO_MAX_DEVICES] = {}; bool& attr_set = attr_set_dev[device_slot()];
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)wna16_gemm_rows_kernel<MB, BF16, STRIP, EXACT>, hipFuncAttributeMaxDynamicSharedMemorySize,

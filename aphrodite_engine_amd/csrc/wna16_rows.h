@@ -20,7 +20,8 @@ struct Wna16RowsParams {
   uint16_t* residual;
   const uint16_t* norm_weight;      // (null: none)
   float norm_eps;
-  int tiles_m, tiles_n;   // (filled by the launch)
+  int tiles_m, tiles_n;   // (filled by the launch, like the next)
+  uint32_t inv_group;     // ceil(2^32 / group_size): the group of every k of the matrix by a multiplication
   Wna16StripGeom strip;
 };
 
