@@ -14,8 +14,7 @@
 //   * K slices write the accumulators as they lie in the registers, 1 KiB a store; a second kernel sums them in the order of K.
 //   * what a wave issues is the other limit: with the scalar arithmetic of a tile's addresses (57 operations), its zero points' 64-bit
 //     addresses and the fragment reads of a step in one place, the first four waves of a CU needed 1 205 cycles a tile alone, and the
-//     other four, behind them, as many again beside their MFMAs.  Running offsets, groups by one multiplication, empty buffers behind the
-//     slice and one MFMA, one read or load and three or four operations of the unpacking a slot: 19 scalar operations of 143 in all.
+//     other four, behind them, as many again beside their MFMAs.  Running offsets, groups by one multiplication and one MFMA, one read or load and three or four operations of the unpacking a slot: 19 scalar operations of 143 in all.
 // Bound by MFMAs, which pull the clock to 1.65 GHz: 1 670 cycles per K tile of 160 rows (1 900 before), 1 280 of them MFMA.
 // Layer of Llama-3-8B at 150 rows, four GEMMs with their slab sums: 192 -> 114 us (qkv 40.4 -> 24, o 27.3 -> 17, gate_up 76 -> 42,
 // down 48 -> 31); at 65 rows 128 -> 79; at 1300 rows 756 -> 629 us.
@@ -79,9 +78,9 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   const int tn = lin % p.tiles_n, rest = lin / p.tiles_n, tm = rest % p.tiles_m, ks = rest / p.tiles_m;
   const int m0 = tm * MB * 32, n0 = tn * RW_BN;
   const int T = p.K / RW_BK, t0 = ks * T / p.ksplit, t1 = (ks + 1) * T / p.ksplit;
-  __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a) + (size_t)m0 * p.lda, 0,
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a) + (size_t)m0 * p.lda, 0,
                                                                 (uint32_t)((size_t)(p.M - m0) * p.lda * 2), 0x00020000);
-  __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qw), 0, (uint32_t)((size_t)(p.K >> 3) * p.N * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qw), 0, (uint32_t)((size_t)(p.K >> 3) * p.N * 4), 0x00020000);
   // ---- activations: one DMA instruction = 4 rows of 256 B, rows 32 apart from one to the next; LDS slot s of row r holds the row's
   // slot s ^ (r & 15).  Rows from M on read zeros (the buffer ends there); 32-row blocks that begin behind M read the last one that does
   // not, because a scalar offset past the buffer's end is not certain to fail the range check.  Nobody stores either. ------------------
@@ -94,13 +93,13 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
   else w_voff = (uint32_t)((kg * 4 + kh) * p.N + col);
   w_voff *= 4u;
   const uint32_t mult4 = mult * 4u;
-  __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.sc), 0, (uint32_t)(p.K / p.group_size * p.N * 2), 0x00020000);
-  __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qz), 0, (uint32_t)(p.K / p.group_size * (p.N >> 3) * 4), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.sc), 0, (uint32_t)(p.K / p.group_size * p.N * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qz), 0, (uint32_t)(p.K / p.group_size * (p.N >> 3) * 4), 0x00020000);
   const int sc_voff = col * 2, z_voff = (col >> 3) * 4;
   const int zshift = (col & 7) * 4;
   const int first_k = t0 * RW_BK + kg * 32, first_grp = first_k / p.group_size, first_in = first_k - first_grp * p.group_size;
   // Where the next load fetches, scalar: k of the wave's part (its group by a multiplication), the tiles until a chunk of the strip-major copy or
-  // the slice ends.  Behind the slice's end the buffers are empty: the loop stays straight-line code, and nothing is fetched.
+  // the slice ends.
   const uint32_t sc_row = (uint32_t)p.N * 2u;
   uint32_t k_load = (uint32_t)(t0 * RW_BK + kg * 32), sc_off, z_off;
   uint32_t w_off, w_vrun = w_voff, a_run = (uint32_t)a_voff + (uint32_t)t0 * (RW_BK * 2);
@@ -150,12 +149,14 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
     if constexpr (STRIP) w_vrun += mult4 * 256u;
     else w_off += 64u * (uint32_t)p.N;
     if (__builtin_expect(--event == 0, 0)) {
-      if (t_load == t1) {
-        ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a) + (size_t)m0 * p.lda, 0, 0, 0x00020000);
-        rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qw), 0, 0, 0x00020000);
-        rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.sc), 0, 0, 0x00020000);
-        rz = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.qz), 0, 0, 0x00020000);
-        event = 0x7fffffff;
+      if (t_load == t1) {                                    // the slice's end: the last tile again, which nobody reads
+        --t_load;
+        k_load -= RW_BK;
+        a_run -= RW_BK * 2;
+        if constexpr (STRIP) w_vrun -= mult4 * 256u;
+        else w_off -= 64u * (uint32_t)p.N;
+        groups();
+        event = 1;
       } else {
         place();
       }
