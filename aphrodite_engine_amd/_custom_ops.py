@@ -2090,9 +2090,10 @@ def wna16_moe_tile_ksplit(blocks: int, n: int, k: int, groups: int, block_m: int
 
 def wna16_moe_tile(a: torch.Tensor, sorted_slots: Optional[torch.Tensor], numel: int, topk: int, qweight: torch.Tensor, qzeros: torch.Tensor,
                    scales: torch.Tensor, expert_ids: torch.Tensor, num_tokens_post_pad: torch.Tensor, m_pad: int, block_m: int,
-                   zero_offset: int, silu: bool) -> torch.Tensor:
+                   zero_offset: int, silu: bool, row_slots: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Grouped expert GEMM of prompt-sized batches (csrc/wna16_moe_tile.hip): a [rows, K] f16 (or bf16 with bf16 scales, widened first);
-    silu -> f16 activations [m_pad, N/2], else fp32 slabs [S, m_pad, N]."""
+    silu -> f16 activations [m_pad, N/2], else fp32 slabs [S, m_pad, N].  row_slots: the sorted slots
+    of every padded row, experts in order; pieces of padding are left out."""
     lib = _lib.lib()
     k, n, groups = qweight.shape[1] * 8, qweight.shape[2], scales.shape[1]
     ks = wna16_moe_tile_ksplit(m_pad // block_m, n, k, groups, block_m, silu)
@@ -2106,6 +2107,12 @@ def wna16_moe_tile(a: torch.Tensor, sorted_slots: Optional[torch.Tensor], numel:
         a = f
     act = torch.empty((m_pad, n // 2), dtype=torch.float16, device=a.device) if silu else None
     out = None if silu else torch.empty((ks, m_pad, n), dtype=torch.float32, device=a.device)
+    if row_slots is not None:
+        check(lib.aphro_wna16_moe_tile_padded(a.data_ptr(), a.shape[0], a.stride(0), _ptr(sorted_slots), row_slots.data_ptr(), numel, topk,
+                                              qweight.data_ptr(), qzeros.data_ptr(), scales.data_ptr(), expert_ids.data_ptr(),
+                                              num_tokens_post_pad.data_ptr(), _ptr(act), _ptr(out), m_pad, n, k, groups, ks, block_m, zero_offset,
+                                              _dt(scales), _stream()), "wna16_moe_tile_padded")
+        return act if silu else out
     check(lib.aphro_wna16_moe_tile(a.data_ptr(), a.shape[0], a.stride(0), _ptr(sorted_slots), numel, topk, qweight.data_ptr(), qzeros.data_ptr(),
                                    scales.data_ptr(), expert_ids.data_ptr(), num_tokens_post_pad.data_ptr(), _ptr(act), _ptr(out), m_pad, n, k,
                                    groups, ks, block_m, zero_offset, _dt(scales), _stream()), "wna16_moe_tile")

@@ -72,6 +72,7 @@ SIGNATURES = {
     "aphro_wna16_gemm_grouped": (I, [P, P, P, P, P, P, P, P, Z, P, L, L, L, L, I, I, P]),
     "aphro_wna16_moe_tile_ksplit": (I, [L, L, L, L, I, I]),
     "aphro_wna16_moe_tile": (I, [P, L, L, P, L, I, P, P, P, P, P, P, P, L, L, L, L, I, I, I, I, P]),
+    "aphro_wna16_moe_tile_padded": (I, [P, L, L, P, P, L, I, P, P, P, P, P, P, P, L, L, L, L, I, I, I, I, P]),
     "aphro_moe_rows_to_f16": (I, [P, P, L, L, L, P]),
     "aphro_moe_route_align_blocks": (I, [P, P, P, L, P, P, P, P, P, L, I, I, I, I, I, P]),
     "aphro_moe_combine": (I, [P, P, I, L, P, P, L, I, L, I, P]),

@@ -127,10 +127,9 @@ class Wna16Experts:
         self.inter = self.w2[0].shape[1] * 8
 
 
-# Prompt-sized batches: from MOE_TILE_ROWS slots per expert on (the average; moe_tile_rows) the experts run on the tile GEMM, in blocks of 64 rows, and of 128
-# from MOE_TILE_WIDE on.  Mixtral-8x7B's experts (8, top 2), decode kernel / 64 / 128 in us: 64 tokens 251 / 280 / 475, 96 tokens 325 / 257 / 434,
-# 160 tokens 451 / 258 / 448, 512 tokens 1268 / 540 / 632, 2048 tokens 4900 / 1760 / 1806, 4096 tokens - / 3354 / 3334.
-MOE_TILE_ROWS, MOE_TILE_WIDE = 24, 768
+# Prompt-sized batches: from MOE_TILE_ROWS slots per expert on (the average; moe_tile_rows) the experts run on the tile GEMM, in tiles of 128 rows, of
+# which 32-row pieces without a row are left out, or of 64 (moe_tile_align).
+MOE_TILE_ROWS, MOE_TILE_PAIRS, MOE_TILE_WIDE = 24, 60, 768
 
 
 def moe_tile_rows(experts: "Wna16Experts") -> int:
@@ -147,18 +146,32 @@ def moe_tile_block(slots: int, experts: Wna16Experts, dtype: torch.dtype, a_byte
     """Rows of a block of the tile GEMM for a batch of ``slots`` (token, expert) pairs whose activations span ``a_bytes``; 0: the decode
     kernel's batch or shape."""
     e = experts.num_experts
-    if slots < moe_tile_rows(experts) * e or dtype != experts.w13[2].dtype:
+    if slots < moe_tile_rows(experts) * e:
         return 0
     bm = 64 if slots < MOE_TILE_WIDE * e else 128
-    blocks = (slots + e * (bm - 1) + bm - 1) // bm
-    if max(a_bytes, blocks * bm * experts.inter * 2) >= 2 ** 32 - 1:       # rows of either GEMM by 32-bit offsets: Mixtral's from 74 000 tokens on
-        return 0
-    for (qw, _, sc), k, silu in ((experts.w13, experts.hidden, True), (experts.w2, experts.inter, False)):
-        # (what the decode kernel refuses stays refused whatever the batch)
-        if ops.wna16_moe_tile_ksplit(blocks, qw.shape[2], k, sc.shape[1], bm, silu) <= 0 \
-                or ops.wna16_grouped_ksplit(blocks * bm, qw.shape[2], k, sc.shape[1]) <= 0:
-            return 0
-    return bm
+    return bm if _tile_served(slots, experts, bm, dtype, a_bytes) else 0
+
+
+def _tile_served(slots: int, experts: Wna16Experts, bm: int, dtype: torch.dtype, a_bytes: int) -> bool:
+    blocks = (slots + experts.num_experts * (bm - 1) + bm - 1) // bm
+    # rows of either GEMM go by 32-bit offsets: Mixtral's from 74 000 tokens on; what the decode kernel refuses stays refused whatever the batch
+    return (dtype == experts.w13[2].dtype and max(a_bytes, (slots + experts.num_experts * 127 + 127) // 128 * 128 * experts.inter * 2) < 2 ** 32 - 1
+            and all(ops.wna16_moe_tile_ksplit(blocks, qw.shape[2], k, sc.shape[1], bm, silu) > 0
+                    and ops.wna16_grouped_ksplit(blocks * bm, qw.shape[2], k, sc.shape[1]) > 0
+                    for (qw, _, sc), k, silu in ((experts.w13, experts.hidden, True), (experts.w2, experts.inter, False))))
+
+
+def moe_tile_align(slots: int, experts: Wna16Experts, dtype: torch.dtype, a_bytes: int = 0) -> int:
+    """Rows of the blocks that a batch is aligned in for the tile GEMM; 0: the decode kernel's batch or shape.  Two thirds of moe_tile_rows are enough
+    for tiles that leave out padding (us, decode kernel / tile at 16 slots an expert and more: 8 x 4096 x 14336 243 / 209, at 20 286 / 205, at 24 321 /
+    222; 16 x 4096 x 4096 139 / 139, 4 x 4096 x 14336 132 / 119; at 32 slots 8 x 4096 x 3584 108 / 85, 4 x 2048 x 8192 71 / 64; at
+    12 and 8 slots the decode kernel is ahead).  Blocks of 64 while most experts have no more rows, and where only those are served
+    (Mixtral-8x7B, both GEMMs, 64 / 128: 100 tokens 183 / 193, 160 235 / 254, 220 262 / 285, 300 370 / 332)."""
+    e = experts.num_experts
+    bm = moe_tile_block(slots, experts, dtype, a_bytes)
+    if bm == 0 and slots * 3 >= moe_tile_rows(experts) * e * 2 and slots < MOE_TILE_PAIRS * e:
+        return 64 if _tile_served(slots, experts, 64, dtype, a_bytes) else 0
+    return 128 if bm == 64 and slots >= MOE_TILE_PAIRS * e and _tile_served(slots, experts, 128, dtype, a_bytes) else bm
 
 
 def _tile_experts(hidden_states, experts: Wna16Experts, topk: int, topk_weights, sorted_ids, expert_ids, post_pad, inv, bm: int,
@@ -166,8 +179,8 @@ def _tile_experts(hidden_states, experts: Wna16Experts, topk: int, topk_weights,
     """Both expert GEMMs on the tile kernel, rows aligned in blocks of ``bm``."""
     m_pad = (sorted_ids.numel() + bm - 1) // bm * bm
     numel = hidden_states.shape[0] * topk
-    act = ops.wna16_moe_tile(hidden_states, sorted_ids, numel, topk, *experts.w13, expert_ids, post_pad, m_pad, bm, experts.zero_offset, True)
-    slabs = ops.wna16_moe_tile(act, None, numel, topk, *experts.w2, expert_ids, post_pad, m_pad, bm, experts.zero_offset, False)
+    act = ops.wna16_moe_tile(hidden_states, sorted_ids, numel, topk, *experts.w13, expert_ids, post_pad, m_pad, bm, experts.zero_offset, True, sorted_ids)
+    slabs = ops.wna16_moe_tile(act, None, numel, topk, *experts.w2, expert_ids, post_pad, m_pad, bm, experts.zero_offset, False, sorted_ids)
     if defer_combine:
         return DeferredCombine(slabs, inv, topk_weights.contiguous(), hidden_states.dtype)
     return ops.moe_combine(slabs, inv, topk_weights.contiguous(), hidden_states.dtype)
@@ -184,7 +197,7 @@ def fused_wna16_moe(hidden_states: torch.Tensor, experts: Wna16Experts, gating_o
     m = hidden_states.shape[0]
     e = experts.num_experts
     packed = None
-    bm = moe_tile_block(m * topk, experts, hidden_states.dtype, m * hidden_states.stride(0) * 2) if aligned is None else 0
+    bm = moe_tile_align(m * topk, experts, hidden_states.dtype, m * hidden_states.stride(0) * 2) if aligned is None else 0
     if bm:
         if topk_ids is not None:
             sorted_ids, expert_ids, post_pad, inv = moe_align_block_size(topk_ids, bm, e, want_inverse=True)

@@ -862,6 +862,12 @@ int aphro_wna16_moe_tile(const void* a, int64_t rows, int64_t lda, const int32_t
                          const uint32_t* q_weight, const uint32_t* qzeros, const void* scales, const int32_t* expert_ids,
                          const int32_t* num_tokens_post_pad, void* act, float* out, int64_t m_pad, int64_t N, int64_t K,
                          int64_t groups, int ksplit, int block_m, int zero_offset, int dtype, void* stream);
+/* The same where the caller knows the padding: row_slots holds numel and more in the padded rows behind an
+ * expert's (sorted_slots of the alignment), and whole 32-row pieces of those are neither computed nor written. */
+int aphro_wna16_moe_tile_padded(const void* a, int64_t rows, int64_t lda, const int32_t* sorted_slots, const int32_t* row_slots, int64_t numel,
+                                int topk, const uint32_t* q_weight, const uint32_t* qzeros, const void* scales,
+                                const int32_t* expert_ids, const int32_t* num_tokens_post_pad, void* act, float* out, int64_t m_pad, int64_t N,
+                                int64_t K, int64_t groups, int ksplit, int block_m, int zero_offset, int dtype, void* stream);
 /* bf16 rows as f16, saturating, dense [rows, K]. */
 int aphro_moe_rows_to_f16(const void* a, void* out, int64_t rows, int64_t K, int64_t lda, void* stream);
 /* aphro_moe_route_align in two launches over 256 tokens a workgroup: <= 16 experts, any number of tokens.  counts: 16 int32 per 256 tokens. */
