@@ -1137,7 +1137,7 @@ static SplitWs g_split_ws[APHRO_MAX_DEVICES];
 // Buffers are NEVER freed or moved once handed out: a HIP graph captured earlier has their raw pointers baked into its
 // kernel nodes, and the reference's model runner captures many batch sizes and keeps running eager decode beside them
 // (growth after capture used to hipFree what a captured graph still writes to).  The first use allocates for
-// the largest plan the launcher makes by itself (groups x want < 3 CUs, want <= 8); a forced APHRO_PA_SPLITS plan that
+// the largest plan the launcher makes by itself (groups x want <= CUs, want <= 8); a forced APHRO_PA_SPLITS plan that
 // needs more gets NEW, larger buffers and the old ones stay alive for the life of the process.
 static bool split_workspace(size_t groups, size_t floats, hipStream_t st, SplitWs** ws_out) {
   static std::mutex mu;                        // host threads racing on first use / growth
@@ -1230,14 +1230,19 @@ static int paged_attention_impl(void* out, void* out_packed, float* exp_sums, fl
     // v1 form: one workgroup per (seq, kv head) walks the whole sequence
     nw = max_seq_len > 256 ? 8 : 4;
     while (nw > 4 && (size_t)nw * (32 + p.nh_lds * head_size) * 4 > 96 * 1024) nw >>= 1;
-    // ... or nsplit workgroups share it (split-KV inside the launch) when (seq, kv head) groups alone leave CUs idle:
-    // aim at ~2 workgroups per CU, at least 8 pairs (256 tokens) per run.  APHRO_PA_SPLITS=n forces n (1 = off).
+    // ... or nsplit workgroups share it (split-KV inside the launch) when (seq, kv head) groups alone leave CUs idle: as many as give every CU one
+    // (eight waves of 164 registers and more are all that a CU holds), at most eight, about three 32-token pairs a run.  The hand-over takes
+    // 2 to 3 us, a pair 0.25 us of an unsplit workgroup, so two runs pay from 28 pairs on, four from 13, eight from 10.  us a layer against
+    // unsplit, this plan / up to two workgroups a CU with 8 pairs a run: one sequence of 330 / 611 / 1000 tokens -1.3 / -4.7 / -6.2, -0.1 / -2.0 /
+    // -5.9; eight of 500 / 1500 / 2500 -0.8 / -6.4 / -14.0, 0 / -2.5 / -10.7; 16 of 600 / 1500 0 / -5.3, 1.8 / -2.3; 24 of 700 0, 5.8.
+    // APHRO_PA_SPLITS=n forces n (1 = off).
     if (gqa <= 16 && head_size == 128 && (block_size == 16 || block_size == 32)) {
       const int64_t groups = (int64_t)num_seqs * num_kv_heads;
-      const int cus = device_cu_count();
-      int want = groups >= cus ? 1 : (int)((2 * cus + groups - 1) / groups);
-      const int max_pairs = (max_seq_len + 31) / 32;
-      if (want > max_pairs / 8) want = max_pairs / 8;
+      const int cus = device_cu_count(), pairs = (max_seq_len + 31) / 32;
+      int want = groups * 2 > cus ? 1 : (int)(cus / groups);
+      want = want > 8 ? 8 : want;
+      if (want > pairs / 3 + 1) want = pairs / 3 + 1;
+      if (pairs < 8 + 80 / (want * want)) want = 1;
       if (knobs().pa_splits > 0) want = knobs().pa_splits;
       want = want > 8 ? 8 : want;
       if (want > 1) {
