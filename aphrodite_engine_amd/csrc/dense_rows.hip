@@ -86,10 +86,10 @@ __device__ __forceinline__ void dr_store(const DenseRowsParams& p, int m, int n,
   }
 }
 
-template <typename T, int MT, int NT, int WR, int NS, int ACT>
+template <typename T, int MT, int NT, int WR, int NS, int ACT, bool STREAM>
 __global__ __launch_bounds__(256 * WR) void dense_rows_kernel(DenseRowsParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  RowsTile<DenseRowsProduct<T>, MT, NT, WR, NS, (ACT >= 0)> tile;
+  RowsTile<DenseRowsProduct<T>, MT, NT, WR, NS, (ACT >= 0), STREAM> tile;
   tile.run(p.op, smem);
   const int M = p.op.M, N = p.op.N, ks = tile.ks, g = tile.g;
 #pragma unroll
@@ -146,14 +146,26 @@ __global__ __launch_bounds__(256) void dense_rows_reduce_kernel(DenseRowsParams 
   dr_store<T>(p, m, col, v);
 }
 
+// Whether w takes the non-temporal hint (RowsTile) above 48 rows of x, up to which it always does: with 40 steps of 64 k a slice and more, up to
+// 128 rows.  us without / with it, f16, weights from memory: [128256, 4096], 16 / 64 / 96 / 192 rows 187 / 198 / 212 / 254 and 167 / 192 / 211 / 253;
+// [28672, 4096], 16 / 64 / 128 / 150 rows 50.5 / 51.4 / 57.9 / 59.5 and 46.7 / 47.9 / 56.8 / 60.1; [10240, 8192], 42 steps, 32 / 65 / 128 rows 38.1 /
+// 37.9 / 42.6 and 35.2 / 35.5 / 41.8.  Short slices lose with many rows: [4096, 14336], 28 steps, 16 / 48 / 96 / 128 rows 24.9 / 26.8 / 30.4 / 33.2
+// and 22.1 / 25.3 / 32.2 / 35.6; [6144, 4096], 12 steps, 16 / 64 / 128 rows 14.3 / 17.6 / 20.5 and 13.5 / 19.0 / 23.4.  (FP8, half the bytes of x a step,
+// is ahead or level with it everywhere: fp8_gemm_rows.hip.)  A w that stays in the 256 MB last-level cache from call to call is slower with it
+// ([32000, 2048] alone, 16 rows: 20.2 and 25.6; twelve of [2048, 2048], 101 MB: 8.1 and 7.7); a model's weights do not stay there.
+inline bool dense_rows_stream(const RowsOperands& op) { return op.M <= 48 || (op.M <= 128 && op.row_bytes >= 40 * 128 * op.ksplit); }
+
 template <typename T, int ACT>
 static int dense_rows_run(DenseRowsParams p, const RowsPlan& plan, hipStream_t st) {
   p.op.tiles_n = (int)(((ACT < 0 ? (int64_t)p.op.N : 2 * (int64_t)p.op.N) + 64 * plan.nt - 1) / (64 * plan.nt));
   p.op.ksplit = plan.ksplit;
   const int rc = rows_dispatch(plan, p.op.tiles_n, [&](auto mt, auto nt, auto wr, auto ns) {
     constexpr int MT = decltype(mt)::value, NT = decltype(nt)::value, WR = decltype(wr)::value, NS = decltype(ns)::value;
-    constexpr size_t lds = RowsTile<DenseRowsProduct<T>, MT, NT, WR, NS, (ACT >= 0)>::LDS;
-    auto kern = dense_rows_kernel<T, MT, NT, WR, NS, ACT>;
+    constexpr size_t lds = RowsTile<DenseRowsProduct<T>, MT, NT, WR, NS, (ACT >= 0), true>::LDS;
+    auto kern = dense_rows_kernel<T, MT, NT, WR, NS, ACT, (MT <= 8)>;
+    if constexpr (MT >= 4 && MT <= 8) {
+      if (!dense_rows_stream(p.op)) kern = dense_rows_kernel<T, MT, NT, WR, NS, ACT, false>;
+    }
     if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
       set_error("dense_rows: cannot raise the dynamic LDS limit to %zu", lds);
       return (int)APHRO_ERR_LAUNCH;

@@ -4,10 +4,11 @@
 // (fp8_gemm.hip's contract); a slab per K slice, added in order.
 // Measured, us, weights from memory, graph replay, [N, K] with 64 / 128 / 192 rows; in brackets the kernels before (fp8_gemm.hip's two passes of 32
 // rows, from 65 on the prompt kernel); raw slabs last:
-//   [28672, 4096]   30.7 / 32.5 / 36.8  (59.7 / 33.4 / 38.2)      29.9 / 32.9 / 35.9
-//   [4096, 14336]   18.7 / 22.2 / 27.1  (36.8 / 25.3 / 30.4)      15.3 / 17.6 / 20.9
-//   [6144, 4096]    14.4 / 17.9 / 19.8  (17.0 / 18.8 / 22.9)       9.6 / 12.6 / 14.7
-//   [4096, 4096]    11.1 / 14.8 / 18.9  (12.7 / 19.2 / 22.8)       6.6 /  9.4 / 10.5
+//   [28672, 4096]   30.7 / 32.5 / 36.8  (59.7 / 33.4 / 38.2)      27.8 / 30.8 / 35.0
+//   [4096, 14336]   18.7 / 22.2 / 27.1  (36.8 / 25.3 / 30.4)      13.3 / 17.0 / 21.1
+//   [6144, 4096]    14.4 / 17.9 / 19.8  (17.0 / 18.8 / 22.9)       9.2 / 12.4 / 14.5
+//   [4096, 4096]    11.1 / 14.8 / 18.9  (12.7 / 19.2 / 22.8)       7.0 /  9.1 / 10.4
+// (raw slabs: with the non-temporal hint on w's loads; without it 29.5 / 32.3 / 36.6, 14.0 / 17.5 / 21.3, 9.3 / 12.3 / 14.6 and 7.1 / 9.3 / 10.4)
 // (a result in 16 bits over several K slices pays a second launch; the same bits as before at every shape measured)
 #include "dense_rows.h"
 
@@ -80,7 +81,7 @@ __device__ __forceinline__ void fr_store(const Fp8RowsParams& p, int m, int n, f
 template <typename T, int MT, int NT, int WR, int NS>
 __global__ __launch_bounds__(256 * WR) void fp8_gemm_rows_kernel(Fp8RowsParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  RowsTile<Fp8RowsProduct, MT, NT, WR, NS, false> tile;
+  RowsTile<Fp8RowsProduct, MT, NT, WR, NS, false, true> tile;
   tile.run(p.op, smem);
   constexpr int MTW = MT / WR;
   const int m0 = tile.wr * MTW * 16 + tile.c, n0 = tile.n0 + 16 * tile.wc + 4 * tile.g, M = p.op.M, N = p.op.N;
@@ -130,7 +131,7 @@ static int fp8_rows_run(const Fp8RowsParams& p, const RowsPlan& plan, hipStream_
       set_error("fp8_gemm_rows: fewer than 33 rows");
       return (int)APHRO_ERR_INVALID;
     } else {
-      constexpr size_t lds = RowsTile<Fp8RowsProduct, MT, NT, WR, NS, false>::LDS;
+      constexpr size_t lds = RowsTile<Fp8RowsProduct, MT, NT, WR, NS, false, true>::LDS;
       auto kern = fp8_gemm_rows_kernel<T, MT, NT, WR, NS>;
       if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
         set_error("fp8_gemm_rows: cannot raise the dynamic LDS limit to %zu", lds);

@@ -10,6 +10,8 @@
 //     chunks XOR-swizzled by the row pair so that the 8-byte B-fragment reads are bank-conflict free; a ring of 8 segments
 //     (16 KiB) per wave = 128 KiB in flight per CU, no register touched on the way in (fp8_gemm_fast_kernel holds 2 macro
 //     steps = 16 KiB per WAVE GROUP in registers and measures 0.43 of the roofline on the gate_up matrix);
+//     The loads carry the non-temporal hint (SILU form, us without / with it, [28672, 4096] 1 / 16 / 32 rows 24.7 / 27.3 /
+//     30.5 and 22.6 / 25.3 / 28.6; [22016, 4096] 21.1 / 23.5 / 26.7 and 19.1 / 21.8 / 25.2);
 //   * hand-counted vmcnt waits (hipcc does not order a ds_read after the LDS-DMA that fills it), B-fragment reads in inline
 //     asm, an LDS-only workgroup barrier per tile (see lm_head.hip);
 //   * K reduction over the waves through LDS once per tile, epilogue in the reference's order sa * (sb * acc) (+ bias).
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_stream_kernel(const uint8_t* 
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
       const int vo = voff_w[it];
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (f8s_lds_ptr)(dst + it * 1024), 16, vo, so, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (f8s_lds_ptr)(dst + it * 1024), 16, vo, so, 0, 2);
     }
   };
   const int tok = tid >> 4, col = tid & 15;

@@ -12,6 +12,9 @@
 //     ring holds KS 128-k segments = one tile ahead of the one it computes: 16 KiB in flight per wave, 128 KiB per CU.
 //     hipcc does not order a ds_read after the LDS-DMA that fills its source: the waits are written by hand (loads return
 //     in order; stores between them can only make a wait return earlier for the stores' own sake -- see below).
+//     They carry the non-temporal hint, as they pass the caches once: us without / with it, f16, weights from memory,
+//     [128256, 4096] 1 / 32 rows 179 / 178 and 169 / 171, [151936, 2048] 117 / 116 and 105, [32000, 2048] 32.6 / 34.2 and
+//     31.0 / 33.1 (a plain read of the first by one workgroup per CU: 172 and 154).
 //   * K reduction over the waves through LDS once per tile; the thread that owns (token, column) of the tile rounds the sum
 //     to the activation dtype (the value the reference's argmax sees), optionally stores it, and keeps a running
 //     (max, index); at the end the workgroup's best per token goes to a partial buffer (write-through), a ticket is taken,
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(512, 1) void lm_head_argmax_kernel(LmHeadParams p) 
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       const int vo = voff_w[it];                    // (local copy: hipcc host-stub bug, see wna16_gemm_large.hip)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lmh_lds_ptr)(ring + s * SEGB + it * 1024), 16, vo, so, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lmh_lds_ptr)(ring + s * SEGB + it * 1024), 16, vo, so, 0, 2);
     }
   };
 

@@ -1,0 +1,62 @@
+"""Which form a decode batch takes: runs of keys shared by workgroups against one workgroup a (sequence, kv head) on both sides of the plan's
+lines, and few-rows products whose weights take the non-temporal hint on both sides of theirs."""
+import os
+
+import pytest
+import torch
+
+from aphrodite_engine_amd import _custom_ops as ops
+
+pytestmark = pytest.mark.gpu
+
+
+# (sequences, kv heads, longest): the last length without runs and the first with them for up to eight, four and two of them; more groups than
+# half the CUs; the longest
+@pytest.mark.parametrize("seqs,hkv,longest", [(1, 8, 352), (1, 8, 353), (1, 1, 600), (8, 8, 384), (8, 8, 385), (9, 8, 500), (16, 8, 864), (16, 8, 865),
+                                              (17, 8, 1100), (3, 2, 5000)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_runs_of_keys(seqs, hkv, longest, dtype):
+    g = torch.Generator(device="cuda").manual_seed(seqs * longest)
+    D, BS, rep = 128, 16, 4
+    bps = (longest + BS - 1) // BS
+    q = torch.randn(seqs, hkv * rep, D, generator=g, device="cuda").to(dtype)
+    kc = torch.randn(seqs * bps + 2, hkv, D // 8, BS, 8, generator=g, device="cuda").to(dtype)
+    vc = torch.randn(seqs * bps + 2, hkv, D, BS, generator=g, device="cuda").to(dtype)
+    table = torch.randperm(seqs * bps + 2, generator=g, device="cuda")[:seqs * bps].int().view(seqs, bps)
+    lens = torch.randint(1, longest + 1, (seqs,), generator=g, device="cuda").int()
+    lens[seqs - 1] = longest
+
+    def run():
+        out = torch.full_like(q, float("nan"))
+        ops.paged_attention_v1(out, q, kc, vc, hkv, D ** -0.5, table, lens, BS, longest, None, "auto", 1.0, 1.0)
+        return out
+
+    got, again = run(), run()
+    old = os.environ.get("APHRO_PA_SPLITS")
+    try:
+        os.environ["APHRO_PA_SPLITS"] = "1"
+        ops.reload_env()
+        want = run().double()
+    finally:
+        if old is None:
+            del os.environ["APHRO_PA_SPLITS"]
+        else:
+            os.environ["APHRO_PA_SPLITS"] = old
+        ops.reload_env()
+    # a probability is rounded to the type against another maximum in each form (u of the largest value each), and so is the result
+    u = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    assert bool(((got.double() - want).abs() <= 2 * u * (float(vc.abs().max()) + want.abs())).all())
+    assert torch.equal(got, again)
+
+
+# 48 / 49 and 128 / 129 rows; 39 and 40 steps of 64 k in one piece, in slices of 40, and in short ones
+@pytest.mark.parametrize("m", [16, 48, 49, 64, 65, 96, 97, 128, 129])
+@pytest.mark.parametrize("n,k", [(20488, 2496), (20488, 2560), (6152, 10240), (4104, 2048)])
+def test_streamed_weights(m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, generator=g, device="cuda").half()
+    w = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).half()
+    want = x.double() @ w.double().t()
+    got = ops.dense_rows(x, w)
+    # one rounding to the type, and fp32 sums of k products whose terms' sizes add up to about sqrt(k) times the result's
+    assert bool(((got.double() - want).abs() <= 2.0 ** -11 * want.abs() + k * 2.0 ** -24 * 4.0).all())
