@@ -623,6 +623,41 @@ def wna16_linear_add_norm(a: torch.Tensor, qweight: torch.Tensor, qzeros: torch.
     return out
 
 
+def wna16_linear_rotary_cache(a: torch.Tensor, qweight: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor, zero_offset: int, strip: bool,
+                              positions: torch.Tensor, num_heads: int, num_kv_heads: int, head_size: int, cos_sin_cache: torch.Tensor,
+                              key_cache: torch.Tensor, value_cache: torch.Tensor, slot_mapping: torch.Tensor, kv_cache_dtype: str, k_scale: float,
+                              v_scale: float) -> Optional[torch.Tensor]:
+    """rotary_embedding_and_cache of the q, k and v columns of a . dequant(W) where the product runs on the tile machine with K slices, in the launch
+    that sums them: the projection with its queries and keys turned, the same bits; None (and nothing done) for any other call.  ``strip``: qweight
+    is the strip-major copy."""
+    m, k = a.shape
+    n, groups = scales.shape[1], scales.shape[0]
+    lib = _lib.lib()
+    if a.dtype != scales.dtype or n != (num_heads + 2 * num_kv_heads) * head_size or not wna16_large_ok(m, n, k, groups) \
+            or switch("APHRO_WNA16_NO_LARGE") or not wna16_prefers_large(m, n, k, a.dtype, groups, strip=strip) \
+            or not lib.aphro_wna16_gemm_large_rotary_cache_supported(m, n, k, groups, _dt(a)):
+        return None
+    _require_cuda(a, qweight, qzeros, scales, positions, cos_sin_cache, key_cache, value_cache, slot_mapping)
+    dt, kv, slots = _dt(a), _kv(kv_cache_dtype), slot_mapping.flatten()
+    if not (cos_sin_cache.dtype == a.dtype and slots.dtype == torch.int64 and positions.dtype == torch.int64 and positions.is_contiguous()
+            and positions.numel() == m and slots.numel() == m and cos_sin_cache.is_contiguous() and key_cache.is_contiguous()
+            and value_cache.is_contiguous() and value_cache.shape[3] == key_cache.shape[3] and key_cache.shape[1] == num_kv_heads
+            and all(t.data_ptr() % 16 == 0 for t in (cos_sin_cache, key_cache, value_cache))
+            and _rotary_cache_served(head_size, cos_sin_cache.shape[1], True, key_cache.shape[3], key_cache.shape[4], dt, kv)):
+        return None
+    if a.stride(1) != 1 or a.stride(0) % 8 != 0 or a.data_ptr() % 16 != 0:
+        a = a.contiguous()
+    qkv = torch.empty((m, n), dtype=a.dtype, device=a.device)
+    nbytes = lib.aphro_wna16_gemm_large_workspace_bytes(m, n, k, groups, dt)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=a.device)
+    check(lib.aphro_wna16_gemm_large_rotary_cache(a.data_ptr(), qweight.data_ptr(), qzeros.data_ptr(), scales.data_ptr(), qkv.data_ptr(),
+                                                  ws.data_ptr(), nbytes, m, k, groups, a.stride(0), zero_offset, dt, 32 if strip else 0,
+                                                  positions.data_ptr(), cos_sin_cache.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
+                                                  slots.data_ptr(), num_heads, num_kv_heads, head_size, key_cache.shape[3], kv, float(k_scale),
+                                                  float(v_scale), _stream()), "wna16_gemm_large_rotary_cache")
+    return qkv
+
+
 def wna16_linear_strip(a: torch.Tensor, strip: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor,
                        zero_offset: int, strip_m: int = 32) -> torch.Tensor:
     """[M, N] = a . dequant(W) for ANY M when the strip-major copy is the only resident copy of W (model.enable_one_copy):

@@ -115,6 +115,8 @@ SIGNATURES = {
     "aphro_wna16_gemm_large_strip": (I, [P, P, P, P, P, P, Z, L, L, L, L, L, I, I, I, L, P]),
     "aphro_wna16_gemm_large_add_norm_supported": (I, [L, L, L, L, I]),
     "aphro_wna16_gemm_large_add_norm": (I, [P, P, P, P, P, P, P, F, P, Z, L, L, L, L, L, I, I, L, P]),
+    "aphro_wna16_gemm_large_rotary_cache_supported": (I, [L, L, L, L, I]),
+    "aphro_wna16_gemm_large_rotary_cache": (I, [P, P, P, P, P, P, Z, L, L, L, L, I, I, L, P, P, P, P, P, I, I, I, I, I, F, F, P]),
     "aphro_wna16_gemm_rowmajor_supported": (I, [L, L, L, L, I]),
     "aphro_fp8_gemm_rows_ksplit": (I, [L, L, L]),
     "aphro_fp8_gemm_rows_preferred": (I, [L, L, L]),

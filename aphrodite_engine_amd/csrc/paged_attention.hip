@@ -25,6 +25,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "rotary_cache.h"
 
 namespace aphro {
 
@@ -939,14 +940,17 @@ __global__ __launch_bounds__(256) void reshape_and_cache_window_kernel(
 // launch: a workgroup owns 16 consecutive tokens of one kv head, or of QH query heads.  Keys turn on their way into LDS and leave from there;
 // where the 16 slots are 16 places of one block, values leave as whole 16-byte pieces, else number by number, and keys as pieces either way.
 // Same operations as rotary_kernel followed by reshape_and_cache_kernel, same bits.
+// SLABS: the rows come as a projection's K slices, which are summed in order, rounded, and written with the rest: a launch less than
+// the sum by itself (wna16_rows_reduce_kernel's bits).  int4 steps, us, sum and rotation / here: 150 scattered tokens 5.2 + 7.4 / 9.5, a step of 16
+// layers 4125 / 4045.
 // Bound by memory.  us of the two launches / here (32 heads on 8 of 128): 33 scattered tokens 3.8 + 3.6 / 5.4, 150 4.0 + 6.6 / 6.3; 2150 tokens of
 // prompts 12.3 + 6.3 / 10.2; 8192, bf16 and an FP8 cache, 37.7 + 17.7 / 36.4.
-template <typename T, int KV, int HD>
+template <typename T, int KV, int HD, bool SLABS>
 __global__ __launch_bounds__(256) void rotary_cache_kernel(
     const int64_t* __restrict__ positions, typename T::storage* __restrict__ query, typename T::storage* __restrict__ key,
-    const typename T::storage* __restrict__ value, const typename T::storage* __restrict__ cos_sin, void* __restrict__ key_cache,
+    typename T::storage* __restrict__ value, const typename T::storage* __restrict__ cos_sin, void* __restrict__ key_cache,
     void* __restrict__ value_cache, const int64_t* __restrict__ slot_mapping, int64_t num_tokens, int num_heads, int num_kv_heads, int block_size,
-    int64_t q_stride, int64_t k_stride, int64_t v_stride, float k_scale, float v_scale) {
+    int64_t q_stride, int64_t k_stride, int64_t v_stride, float k_scale, float v_scale, const float* __restrict__ slabs, int nslab, int64_t slab_stride) {
   using S = typename T::storage;
   constexpr int W = 16;                               // tokens of a workgroup
   constexpr int X = KV == 0 ? 8 : 16;                 // numbers of a 16-byte cache piece
@@ -957,8 +961,30 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(
   __shared__ int64_t s_slot[W];
   const int64_t t0 = (int64_t)blockIdx.x * W;
   const int nt = (int)(num_tokens - t0 < W ? num_tokens - t0 : W);
-  auto turn = [&](const S* row, int64_t pos, int c, u16x8& xo8, u16x8& yo8) {
-    const u16x8 x = *reinterpret_cast<const u16x8*>(row + 8 * c), y = *reinterpret_cast<const u16x8*>(row + HALF + 8 * c);
+  // numbers 8 c .. + 7 of a head of token t and their partners; ``col``: the head's first column
+  auto fetch = [&](const S* row, int64_t t, int col, int c, u16x8& x, u16x8& y) {
+    if constexpr (!SLABS) {
+      x = *reinterpret_cast<const u16x8*>(row + 8 * c);
+      y = *reinterpret_cast<const u16x8*>(row + HALF + 8 * c);
+    } else {
+      const float* src = slabs + t * ((num_heads + 2 * num_kv_heads) * HD) + col + 8 * c;
+      f32x4 a[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a[q] = *reinterpret_cast<const f32x4*>(src + (q >> 1) * HALF + (q & 1) * 4);
+#pragma unroll 4
+      for (int s = 1; s < nslab; ++s)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] += *reinterpret_cast<const f32x4*>(src + s * slab_stride + (q >> 1) * HALF + (q & 1) * 4);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        x[i] = T::from_f32(a[i >> 2][i & 3]);
+        y[i] = T::from_f32(a[2 + (i >> 2)][i & 3]);
+      }
+    }
+  };
+  auto turn = [&](const S* row, int64_t t, int col, int64_t pos, int c, u16x8& xo8, u16x8& yo8) {
+    u16x8 x, y;
+    fetch(row, t, col, c, x, y);
     const u16x8 cs = *reinterpret_cast<const u16x8*>(cos_sin + pos * HD + 8 * c), sn = *reinterpret_cast<const u16x8*>(cos_sin + pos * HD + HALF + 8 * c);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -976,7 +1002,7 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(
       if (h >= num_heads) continue;
       S* row = query + t * q_stride + (int64_t)h * HD;
       u16x8 xo, yo;
-      turn(row, positions[t], c, xo, yo);
+      turn(row, t, h * HD, positions[t], c, xo, yo);
       *reinterpret_cast<u16x8*>(row + 8 * c) = xo;
       *reinterpret_cast<u16x8*>(row + HALF + 8 * c) = yo;
     }
@@ -984,20 +1010,30 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(
   }
   const int h = blockIdx.y;
   if (threadIdx.x < W) s_slot[threadIdx.x] = threadIdx.x < nt ? slot_mapping[t0 + threadIdx.x] : -1;
-  for (int i = threadIdx.x; i < nt * CPH; i += 256) {
-    const int c = i % CPH, j = i / CPH;
-    S* row = key + (t0 + j) * k_stride + (int64_t)h * HD;
+  for (int i = threadIdx.x; i < (SLABS ? 2 : 1) * nt * CPH; i += 256) {
+    const int c = i % CPH, j = SLABS ? i / CPH % nt : i / CPH;
     u16x8 xo, yo;
-    turn(row, positions[t0 + j], c, xo, yo);
+    if (SLABS && i >= nt * CPH) {                     // values
+      S* row = value + (t0 + j) * v_stride + (int64_t)h * HD;
+      fetch(row, t0 + j, (num_heads + num_kv_heads + h) * HD, c, xo, yo);
+      *reinterpret_cast<u16x8*>(row + 8 * c) = xo;
+      *reinterpret_cast<u16x8*>(row + HALF + 8 * c) = yo;
+      *reinterpret_cast<u16x8*>(sv + j * P + 8 * c) = xo;
+      *reinterpret_cast<u16x8*>(sv + j * P + HALF + 8 * c) = yo;
+      continue;
+    }
+    S* row = key + (t0 + j) * k_stride + (int64_t)h * HD;
+    turn(row, t0 + j, (num_heads + h) * HD, positions[t0 + j], c, xo, yo);
     *reinterpret_cast<u16x8*>(row + 8 * c) = xo;
     *reinterpret_cast<u16x8*>(row + HALF + 8 * c) = yo;
     *reinterpret_cast<u16x8*>(sk + j * P + 8 * c) = xo;
     *reinterpret_cast<u16x8*>(sk + j * P + HALF + 8 * c) = yo;
   }
-  for (int i = threadIdx.x; i < nt * (HD / 8); i += 256) {
-    const int pc = i % (HD / 8), j = i / (HD / 8);
-    *reinterpret_cast<u32x4*>(sv + j * P + 8 * pc) = *reinterpret_cast<const u32x4*>(value + (t0 + j) * v_stride + (int64_t)h * HD + 8 * pc);
-  }
+  if constexpr (!SLABS)
+    for (int i = threadIdx.x; i < nt * (HD / 8); i += 256) {
+      const int pc = i % (HD / 8), j = i / (HD / 8);
+      *reinterpret_cast<u32x4*>(sv + j * P + 8 * pc) = *reinterpret_cast<const u32x4*>(value + (t0 + j) * v_stride + (int64_t)h * HD + 8 * pc);
+    }
   __syncthreads();
   auto cvt4 = [](const S* p, int step, float scale) -> uint32_t {      // four numbers, ``step`` apart (a division, not a reciprocal)
     return f32x2_to_fp8<KV == 2>(T::to_f32(p[0]) / scale, T::to_f32(p[step]) / scale) |
@@ -1046,6 +1082,30 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(
     if constexpr (KV == 0) ((S*)value_cache)[dst] = sv[j * P + d];
     else ((uint8_t*)value_cache)[dst] = (uint8_t)f32x2_to_fp8<KV == 2>(T::to_f32(sv[j * P + d]) / v_scale, 0.f);
   }
+}
+
+template <typename T, int KV, int HD, bool SLABS>
+static int rotary_cache_run(const RotaryCacheCall& c, hipStream_t st) {
+  constexpr int QH = HD == 128 ? 2 : 4;
+  using S = typename T::storage;
+  const dim3 grid((unsigned)((c.num_tokens + 15) / 16), (unsigned)(c.num_kv_heads + (c.num_heads + QH - 1) / QH));
+  hipLaunchKernelGGL((rotary_cache_kernel<T, KV, HD, SLABS>), grid, dim3(256), 0, st, c.positions, (S*)c.query, (S*)c.key, (S*)c.value,
+                     (const S*)c.cos_sin, c.key_cache, c.value_cache, c.slot_mapping, c.num_tokens, c.num_heads, c.num_kv_heads, c.block_size,
+                     c.q_stride, c.k_stride, c.v_stride, c.k_scale, c.v_scale, c.slabs, c.nslab, c.slab_stride);
+  APHRO_LAUNCH_CHECK();
+  return APHRO_OK;
+}
+template <typename T, int KV>
+static int rotary_cache_head(const RotaryCacheCall& c, hipStream_t st) {
+  if (c.slabs) return c.head_size == 128 ? rotary_cache_run<T, KV, 128, true>(c, st) : rotary_cache_run<T, KV, 64, true>(c, st);
+  return c.head_size == 128 ? rotary_cache_run<T, KV, 128, false>(c, st) : rotary_cache_run<T, KV, 64, false>(c, st);
+}
+int rotary_cache_launch(const RotaryCacheCall& c, hipStream_t st) {
+  if (c.num_tokens == 0) return APHRO_OK;
+  const bool half = c.dtype == APHRO_F16;
+  if (c.kv_dtype == APHRO_KV_AUTO) return half ? rotary_cache_head<Half, 0>(c, st) : rotary_cache_head<BFloat, 0>(c, st);
+  if (c.kv_dtype == APHRO_KV_FP8_E4M3) return half ? rotary_cache_head<Half, 1>(c, st) : rotary_cache_head<BFloat, 1>(c, st);
+  return half ? rotary_cache_head<Half, 2>(c, st) : rotary_cache_head<BFloat, 2>(c, st);
 }
 
 template <typename T, int KV, bool TO_FP8>
@@ -1428,23 +1488,12 @@ extern "C" int aphro_rotary_cache(const int64_t* positions, void* query, void* k
   const auto al16 = [](const void* ptr) { return ((uintptr_t)ptr & 15) == 0; };
   APHRO_CHECK(num_heads > 0 && num_kv_heads > 0 && ((q_stride | k_stride | v_stride) & 7) == 0 && al16(query) && al16(key) && al16(value) &&
                   al16(cos_sin_cache) && al16(key_cache) && al16(value_cache), "rotary_cache: rows of 16-byte pieces, aligned");
-  if (num_tokens == 0) return APHRO_OK;
-  const int qh = head_size == 128 ? 2 : 4;
-  const dim3 grid((unsigned)((num_tokens + 15) / 16), (unsigned)(num_kv_heads + (num_heads + qh - 1) / qh));
-#define APHRO_RTC(TT, KVV, HDV)                                                                                                       \
-  hipLaunchKernelGGL((rotary_cache_kernel<TT, KVV, HDV>), grid, dim3(256), 0, (hipStream_t)stream, positions, (TT::storage*)query,     \
-                     (TT::storage*)key, (const TT::storage*)value, (const TT::storage*)cos_sin_cache, key_cache, value_cache, slot_mapping, num_tokens, \
-                     num_heads, num_kv_heads, block_size, q_stride, k_stride, v_stride, k_scale, v_scale)
-#define APHRO_RTC_H(TT, KVV) do { if (head_size == 128) APHRO_RTC(TT, KVV, 128); else APHRO_RTC(TT, KVV, 64); } while (0)
-#define APHRO_RTC_T(KVV) do { if (dtype == APHRO_F16) APHRO_RTC_H(Half, KVV); else APHRO_RTC_H(BFloat, KVV); } while (0)
-  if (kv_dtype == APHRO_KV_AUTO) APHRO_RTC_T(0);
-  else if (kv_dtype == APHRO_KV_FP8_E4M3) APHRO_RTC_T(1);
-  else APHRO_RTC_T(2);
-#undef APHRO_RTC_T
-#undef APHRO_RTC_H
-#undef APHRO_RTC
-  APHRO_LAUNCH_CHECK();
-  return APHRO_OK;
+  RotaryCacheCall r = {};
+  r.positions = positions; r.query = query; r.key = key; r.value = const_cast<void*>(value); r.cos_sin = cos_sin_cache;
+  r.key_cache = key_cache; r.value_cache = value_cache; r.slot_mapping = slot_mapping; r.num_tokens = num_tokens; r.num_heads = num_heads;
+  r.num_kv_heads = num_kv_heads; r.head_size = head_size; r.block_size = block_size; r.q_stride = q_stride; r.k_stride = k_stride;
+  r.v_stride = v_stride; r.dtype = dtype; r.kv_dtype = kv_dtype; r.k_scale = k_scale; r.v_scale = v_scale;
+  return rotary_cache_launch(r, (hipStream_t)stream);
 }
 
 extern "C" int aphro_reshape_and_cache(const void* key, const void* value, void* key_cache,

@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "rotary_cache.h"
 #include "wna16_rows.h"
 
 namespace aphro {
@@ -1105,7 +1106,8 @@ extern "C" size_t aphro_wna16_gemm_large_strip_workspace_bytes(int64_t M, int64_
 static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const uint32_t* qzeros, const void* scales,
                                  void* c, void* workspace, size_t workspace_bytes, int64_t M, int64_t N, int64_t K,
                                  int64_t groups, int64_t lda, int zero_offset, int dtype, int silu, void* stream, int strip_m = 0,
-                                 void* residual = nullptr, const void* norm_weight = nullptr, float norm_eps = 0.f) {
+                                 void* residual = nullptr, const void* norm_weight = nullptr, float norm_eps = 0.f,
+                                 RotaryCacheCall* rotary = nullptr) {
   hipStream_t st = (hipStream_t)stream;
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "wna16_gemm_large: dtype must be f16 or bf16");
   APHRO_CHECK(groups > 0 && K % groups == 0, "wna16_gemm_large: K=%ld not divisible by groups=%ld", (long)K, (long)groups);
@@ -1163,15 +1165,22 @@ static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const 
   const Wna16RowsPlan rp = rows_plan(pl, M, N, K, gs, dtype);
   APHRO_CHECK(!norm_weight || (rp.mb > 0 && rp.ksplit > 1 && N <= 16384), "wna16_gemm_large_add_norm: M=%ld N=%ld K=%ld has no summed K slices",
               (long)M, (long)N, (long)K);
+  APHRO_CHECK(!rotary || (rp.mb > 0 && rp.ksplit > 1), "wna16_gemm_large_rotary_cache: M=%ld N=%ld K=%ld has no summed K slices", (long)M, (long)N, (long)K);
   if (rp.mb > 0) {
     Wna16RowsParams q = {};
     q.a = p.a; q.lda = p.lda; q.qw = p.qw; q.qz = p.qz; q.sc = p.sc; q.c = p.c; q.partial = (float*)ws;
     q.M = p.M; q.N = p.N; q.K = p.K; q.group_size = p.group_size; q.zero_offset = zero_offset;
     q.ksplit = rp.ksplit; q.silu = silu; q.bf16 = p.out_bf16;
+    q.row_slabs = norm_weight || rotary;
     q.residual = (uint16_t*)residual; q.norm_weight = (const uint16_t*)norm_weight; q.norm_eps = norm_eps;
     APHRO_CHECK(strip_m == 0 || wna16_strip_fill(q.strip, strip_m, N, K, groups),
                 "wna16_gemm_large_strip: no strip-major form for M class %d, N=%ld, K=%ld, groups=%ld", strip_m, (long)N, (long)K, (long)groups);
-    return wna16_rows_launch(q, rp, st);
+    const int rc = wna16_rows_launch(q, rp, st);
+    if (rc != APHRO_OK || !rotary) return rc;
+    rotary->slabs = q.partial;
+    rotary->nslab = rp.ksplit;
+    rotary->slab_stride = (M + rp.mb * 32 - 1) / (rp.mb * 32) * (rp.mb * 32) * N;
+    return rotary_cache_launch(*rotary, st);
   }
   if (large_two_pass(pl, M, N, K, gs)) {
     // pass 1: the weights dequantised once into f16 W^T [N, K] (same numerics as the in-loop dequantisation: same bits out)
@@ -1241,6 +1250,37 @@ extern "C" int aphro_wna16_gemm_large_add_norm(const void* a, const uint32_t* q_
               "wna16_gemm_large_add_norm: c, residual and norm_weight must be 16-byte aligned");
   return wna16_gemm_large_impl(a, q_weight, qzeros, scales, c, workspace, workspace_bytes, M, N, K, groups, lda, zero_offset, dtype, 0, stream,
                                (int)strip_m, residual, norm_weight, eps);
+}
+
+// aphro_wna16_gemm_large (strip_m == 0) / _strip of a qkv projection followed by aphro_rotary_cache on its columns, where the GEMM ends in a sum
+// over K slices: the rotation and the cache write are that launch's.  qkv [M, (num_heads + 2 num_kv_heads) head_size] as the two leave it, the
+// same bits.  1 if the shape is served, else 0: aphro_wna16_gemm_large_rotary_cache_supported (the geometry: aphro_rotary_cache_supported).
+extern "C" int aphro_wna16_gemm_large_rotary_cache_supported(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype) {
+  if (M <= 0 || groups <= 0 || K % groups != 0 || K % 64 != 0 || (K / groups) % 64 != 0 || N % 128 != 0) return 0;
+  const Wna16RowsPlan rp = rows_plan(large_plan(M, N, K, K / groups), M, N, K, K / groups, dtype);
+  return rp.mb > 0 && rp.ksplit > 1;
+}
+extern "C" int aphro_wna16_gemm_large_rotary_cache(const void* a, const uint32_t* q_weight, const uint32_t* qzeros, const void* scales, void* qkv,
+                                                   void* workspace, size_t workspace_bytes, int64_t M, int64_t K, int64_t groups, int64_t lda,
+                                                   int zero_offset, int dtype, int64_t strip_m, const int64_t* positions, const void* cos_sin_cache,
+                                                   void* key_cache, void* value_cache, const int64_t* slot_mapping, int num_heads, int num_kv_heads,
+                                                   int head_size, int block_size, int kv_dtype, float k_scale, float v_scale, void* stream) {
+  APHRO_CHECK(strip_m >= 0 && strip_m <= 64, "wna16_gemm_large_rotary_cache: strip_m=%ld", (long)strip_m);
+  APHRO_CHECK(aphro_rotary_cache_supported(head_size, head_size, 1, block_size, kv_dtype == APHRO_KV_AUTO ? 8 : 16, dtype, kv_dtype),
+              "wna16_gemm_large_rotary_cache: heads of %d, blocks of %d, types %d / %d are not served", head_size, block_size, dtype, kv_dtype);
+  APHRO_CHECK(num_heads > 0 && num_kv_heads > 0 &&
+                  (((uintptr_t)qkv | (uintptr_t)cos_sin_cache | (uintptr_t)key_cache | (uintptr_t)value_cache) % 16) == 0,
+              "wna16_gemm_large_rotary_cache: qkv and the caches must be 16-byte aligned");
+  const int64_t N = (int64_t)(num_heads + 2 * num_kv_heads) * head_size, esz = 2;
+  RotaryCacheCall r = {};
+  r.positions = positions; r.query = qkv; r.key = (char*)qkv + (int64_t)num_heads * head_size * esz;
+  r.value = (char*)r.key + (int64_t)num_kv_heads * head_size * esz;
+  r.cos_sin = cos_sin_cache; r.key_cache = key_cache; r.value_cache = value_cache; r.slot_mapping = slot_mapping;
+  r.num_tokens = M; r.num_heads = num_heads; r.num_kv_heads = num_kv_heads; r.head_size = head_size; r.block_size = block_size;
+  r.q_stride = r.k_stride = r.v_stride = N;
+  r.dtype = dtype; r.kv_dtype = kv_dtype; r.k_scale = k_scale; r.v_scale = v_scale;
+  return wna16_gemm_large_impl(a, q_weight, qzeros, scales, qkv, workspace, workspace_bytes, M, N, K, groups, lda, zero_offset, dtype, 0, stream,
+                               (int)strip_m, nullptr, nullptr, 0.f, &r);
 }
 
 extern "C" int aphro_wna16_gemm_large_silu_supported(int64_t M, int64_t N, int64_t K, int64_t groups) {

@@ -423,7 +423,7 @@ __global__ __launch_bounds__(512) void wna16_gemm_rows_kernel(Wna16RowsParams p)
       if (row >= p.M) continue;
       const int c0 = n0 + wn * 64 + 16 * kg + 8 * kh;
       const f32x4 x = own[0][i], y = own[1][i];
-      if (p.ksplit > 1 && p.norm_weight) {                   // rows of N, which the norm reads whole
+      if (p.ksplit > 1 && p.row_slabs) {                     // rows of N, which a norm or a rotation reads whole
         float* o = p.partial + ((size_t)ks * p.tiles_m * (MB * 32) + row) * p.N + c0;
         *reinterpret_cast<f32x4*>(o) = f32x4{x[0], y[0], x[1], y[1]};
         *reinterpret_cast<f32x4*>(o + 4) = f32x4{x[2], y[2], x[3], y[3]};
@@ -589,7 +589,7 @@ static int rows_launch(Wna16RowsParams p, hipStream_t st) {
     using T16 = std::conditional_t<BF16, BFloat, Half>;
     hipLaunchKernelGGL(wna16_rows_norm_kernel<T16>, dim3(p.M), dim3(norm_threads(p.N)), 0, st, p, p.tiles_m * MB * 32);
     APHRO_LAUNCH_CHECK();
-  } else if (p.ksplit > 1) {
+  } else if (p.ksplit > 1 && !p.row_slabs) {
     hipLaunchKernelGGL(wna16_rows_reduce_kernel<BF16>, dim3(p.tiles_m * p.tiles_n * MB * 2), dim3(256), 0, st, p, MB);
     APHRO_LAUNCH_CHECK();
   }

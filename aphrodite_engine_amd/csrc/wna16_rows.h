@@ -13,6 +13,7 @@ struct Wna16RowsParams {
   const uint16_t* sc;     // [G, N]
   uint16_t* c;            // [M, N], [M, N / 2] with SiluAndMul
   float* partial;         // slabs when ksplit > 1
+  int row_slabs;          // K slices stay in partial, [ksplit][M rounded up to tiles][N], for a launch behind this one (with a norm: that one)
   int M, N, K, lda;
   int group_size, zero_offset, ksplit, silu;
   int bf16;               // scales and results are bf16 (else f16)

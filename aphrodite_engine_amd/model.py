@@ -857,10 +857,23 @@ class LlamaDecoderLayer(nn.Module):
                 return False
         return True
 
-    def _attend(self, positions, q, k, v, kv_cache, attn_metadata, cos_sin):
-        """Rotary embedding, cache write and attention of a projection's rows."""
-        cached = False
-        if kv_cache is not None and kv_cache.numel() > 0:
+    def _project_rotated(self, hidden, positions, kv_cache, attn_metadata, cos_sin) -> Optional[torch.Tensor]:
+        """The qkv projection with its rotary embedding and cache write done where the launch that sums its K slices can do them, else None."""
+        lin = self.qkv_proj
+        if kv_cache is None or kv_cache.numel() == 0:
+            return None
+        fp = self._int4_words(lin, hidden)
+        if fp is None:
+            return None
+        from .attention.paged_attn import PagedAttention
+        key_cache, value_cache = PagedAttention.split_kv_cache(kv_cache, self.num_kv_heads, self.head_dim)
+        return ops.wna16_linear_rotary_cache(hidden, *fp, getattr(lin, "qweight_strip_major", False), positions, self.num_heads, self.num_kv_heads,
+                                             self.head_dim, cos_sin, key_cache, value_cache, attn_metadata.slot_mapping, self.attn.kv_cache_dtype,
+                                             self.k_scale, self.v_scale)
+
+    def _attend(self, positions, q, k, v, kv_cache, attn_metadata, cos_sin, cached=False):
+        """Rotary embedding, cache write (``cached``: both done) and attention of a projection's rows."""
+        if not cached and kv_cache is not None and kv_cache.numel() > 0:
             from .attention.paged_attn import PagedAttention
             key_cache, value_cache = PagedAttention.split_kv_cache(kv_cache, self.num_kv_heads, self.head_dim)
             cached = ops.rotary_embedding_and_cache(positions, q, k, v, self.head_dim, cos_sin, True, key_cache, value_cache,
@@ -906,9 +919,12 @@ class LlamaDecoderLayer(nn.Module):
             hidden = normed
         elif next_norm is None:
             ops.fused_add_rms_norm(hidden, residual, self.input_layernorm, eps)
-        qkv = self.qkv_proj(hidden)
+        qkv = self._project_rotated(hidden, positions, kv_cache, attn_metadata, cos_sin)
+        cached = qkv is not None
+        if not cached:
+            qkv = self.qkv_proj(hidden)
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
-        attn_out = self._attend(positions, q, k, v, kv_cache, attn_metadata, cos_sin)
+        attn_out = self._attend(positions, q, k, v, kv_cache, attn_metadata, cos_sin, cached)
         hidden = self._row_parallel(self.o_proj, attn_out, residual, self.post_attention_layernorm)
         if self.is_moe:
             hidden = self.moe_block(hidden)
@@ -935,14 +951,20 @@ class LlamaDecoderLayer(nn.Module):
         ops.silu_and_mul(act, gate_up, interleaved=self.gate_up_interleaved is not None and not self.gate_up_keep_original)
         return self._row_parallel(self.down_proj, act, residual, next_norm), residual
 
+    @staticmethod
+    def _int4_words(lin: QuantLinear, x: torch.Tensor):
+        """lin.fast_params() where a batch beyond the decode kernels may be multiplied without lin's own call, else None."""
+        if lin.bias is None and x.shape[0] > 64 and isinstance(lin.quant_config, (GPTQConfig, AWQConfig)) and ops.unhooked(lin):
+            return lin.fast_params()
+        return None
+
     def _row_parallel(self, lin: QuantLinear, x: torch.Tensor, residual: torch.Tensor, norm: Optional[torch.Tensor]) -> torch.Tensor:
         """RowParallelLinear.forward (linear.py:1136-1150): this rank's partial product, the all-reduce over the TP group,
         then the bias -- once, not per rank.  ``norm``: then fused_add_rms_norm with these weights, in the product's own last launch where it
         has one over whole sums."""
         if self.tp == 1:
-            if norm is not None and lin.bias is None and x.shape[0] > 64 and isinstance(lin.quant_config, (GPTQConfig, AWQConfig)) \
-                    and ops.unhooked(lin):
-                fp = lin.fast_params()
+            if norm is not None:
+                fp = self._int4_words(lin, x)
                 if fp is not None:
                     out = ops.wna16_linear_add_norm(x, *fp, getattr(lin, "qweight_strip_major", False), residual, norm, self.cfg.rms_norm_eps)
                     if out is not None:

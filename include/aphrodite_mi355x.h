@@ -743,6 +743,15 @@ int aphro_wna16_gemm_large_add_norm(const void* a, const uint32_t* q_weight, con
                                     void* residual, const void* norm_weight, float eps, void* workspace, size_t workspace_bytes,
                                     int64_t M, int64_t N, int64_t K, int64_t groups, int64_t lda, int zero_offset, int dtype,
                                     int64_t strip_m, void* stream);
+/* aphro_wna16_gemm_large (strip_m == 0) or _strip of a qkv projection followed by aphro_rotary_cache on its columns, the rotation and the cache write
+ * in the launch that sums the GEMM's K slices: qkv [M, (num_heads + 2 num_kv_heads) head_size] as the two leave it, same bits, same workspace.
+ * Served where the GEMM slices K (supported == 1) and aphro_rotary_cache_supported. */
+int aphro_wna16_gemm_large_rotary_cache_supported(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype);
+int aphro_wna16_gemm_large_rotary_cache(const void* a, const uint32_t* q_weight, const uint32_t* qzeros, const void* scales, void* qkv,
+                                        void* workspace, size_t workspace_bytes, int64_t M, int64_t K, int64_t groups, int64_t lda,
+                                        int zero_offset, int dtype, int64_t strip_m, const int64_t* positions, const void* cos_sin_cache,
+                                        void* key_cache, void* value_cache, const int64_t* slot_mapping, int num_heads, int num_kv_heads,
+                                        int head_size, int block_size, int kv_dtype, float k_scale, float v_scale, void* stream);
 
 /* The op-level decode GEMM (`_C::gptq_gemm` / `_C::awq_gemm` at M <= 32, torch_bindings.cpp:229-243; the role of
  * gemm_half_q_half_gptq_4bit_kernel, q_gemm.cu:190-326, which also reads row-major `a` and writes [M, N] in one launch) in
