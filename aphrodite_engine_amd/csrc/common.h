@@ -263,12 +263,20 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// gate / (1 + e^-gate) for a gate of 16 bits: one reciprocal and one exact correction in place of a division, the same value once it is rounded to
+// the gate's type, for each of the 65536 gates of either (9 instructions for 16: they weigh in SiluAndMul's quantising form, 8192 x 28672 128 -> 118 us,
+// and in the products' epilogues; int4 gate_up of 32 rows 15.2 -> 14.8).  The denominator goes in a quarter of its size, so that its reciprocal is a normal number wherever the quotient is not zero.
+__device__ __forceinline__ float silu_quotient(float gate) {
+  const float d = 1.0f + __expf(-gate), y = 0.25f * __builtin_amdgcn_rcpf(0.25f * d), q = gate * y;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, gate), y, q), d, gate);
+}
+
 // round(round(silu(gate)) * up) in the activation type T, on T-rounded inputs
 // (activation_kernels.cu:14-17, 25-28).  Shared by silu_and_mul, silu_and_mul_pack and the
 // fused GEMM epilogue so that the three paths are bit-identical.
 template <typename T>
 __device__ __forceinline__ uint16_t silu_mul_bits(float gate, float up) {
-  const float s = T::to_f32(T::from_f32(gate / (1.0f + __expf(-gate))));
+  const float s = T::to_f32(T::from_f32(silu_quotient(gate)));
   return from_f32_exact<T>(s * up);
 }
 

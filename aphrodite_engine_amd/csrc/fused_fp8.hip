@@ -205,8 +205,9 @@ __global__ __launch_bounds__(VPT <= 4 ? 1024 : 512) void silu_mul_quant_kernel(c
   float amax = 0.f;
   auto load = [&](int it) {                            // past the row's end: its last piece once more, so that no load hangs on a branch
     const int i = threadIdx.x + it * blockDim.x, at = 8 * (i < nv ? i : nv - 1);
-    x[it & 1] = *reinterpret_cast<const u16x8*>(a + at);
-    y[it & 1] = *reinterpret_cast<const u16x8*>(b + at);
+    // (the non-temporal hint: 8192 rows of 28672, 470 MB, 142 us without and 128 with it; level where the rows are still in the last-level cache)
+    x[it & 1] = __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(a + at));
+    y[it & 1] = __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(b + at));
   };
   load(0);
 #pragma unroll
