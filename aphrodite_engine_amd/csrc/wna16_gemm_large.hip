@@ -1054,8 +1054,9 @@ static Wna16RowsPlan rows_exact_plan(int64_t M, int64_t N, int64_t K, int64_t gs
 }
 
 // The tile of wna16_gemm_rows.hip, up to 4096 rows: always where this file would take one workgroup per tile (4096 x 4096: 150 rows
-// 27.3 -> 18.3 us, 1300 rows 78 -> 56 us), and beside the stream-K form where its last round is full enough (28672 x 4096: 300 rows
-// 127 -> 82 us, 1300 rows 341 -> 326 us; 2048 rows 450 against 489 us: stays).  Its K slices are its own, of any whole K tiles up to 36 MiB of slabs;
+// 27.3 -> 18.3 us, 1300 rows 78 -> 56 us), and beside the stream-K form where it is expected to be ahead (us, stream-K / here: 28672 x 4096,
+// 300 rows 131 / 84, 400 134 / 124, 1100 308 / 278, 1340 362 / 337, 1600 423 / 375, 2600 656 / 621; 6144 x 4096, 1340 rows 94 / 80; 4096 x 14336, 3000
+// rows 345 / 331.  28672 x 4096, 700 rows 193 / 201, 2048 468 / 487, 4096 893 / 948: stays).  Its K slices are its own, of any whole K tiles up to 36 MiB of slabs;
 // this file's are ranges of whole groups, of which 11008 or 9728 rows of K have few divisors and one group per column none (4096 x 11008 at 65
 // / 150 / 300 rows with slices bound to this file's 53 / 54 / 54 us, without 21 / 28 / 40 us).
 static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype) {
@@ -1065,11 +1066,11 @@ static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_
     if (exact.mb > 0) return exact;
   }
   int64_t other_ns = -1;
-  if (pl.streamk) {            // 1.9 us per 256 x 256 x 64 of a CU's even share, 18 us around them
-    const int64_t units = (M + 255) / 256 * ((N + 255) / 256) * (K / 64);
-    other_ns = 18000 + units * 1900 / pl.grid;
+  if (pl.streamk) {            // 1.93 us per 256 x 256 x 64 of a CU's even share, 6 us per tile of it, 18 us around them
+    const int64_t tiles = (M + 255) / 256 * ((N + 255) / 256);
+    other_ns = 18000 + (tiles * (K / 64) * 1930 + tiles * 6000) / pl.grid;
   }
-  return wna16_rows_plan(M, N, K, gs, pl.streamk ? 0 : 36ll << 20, other_ns < 0 ? -1 : other_ns * 97 / 100);
+  return wna16_rows_plan(M, N, K, gs, pl.streamk ? 0 : 36ll << 20, other_ns);
 }
 
 static size_t large_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype, int strip_m) {
