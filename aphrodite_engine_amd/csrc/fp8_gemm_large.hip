@@ -10,15 +10,13 @@
 //     SOURCE address, read back with conflict-free ds_read_b128 (two per operand fragment).
 //   * 2 LDS stages of 64 KiB (256 x 256 x 128 tile) or 3 stages of 48 KiB (narrower tiles): the next K tile's loads
 //     are in flight under the current tile's 16 MFMAs per wave.
-//   * STREAM-K: one persistent workgroup per CU; the (tile, K tile) units are dealt out in equal contiguous ranges, so
-//     (a) there is no last partial round of tiles, and (b) the workgroups reach their tile boundaries at different
-//     times -- measured on the one-workgroup-per-tile form, all 256 CUs storing their 128 KiB of C at the same moment
-//     ran at 1.7 TB/s with every MFMA idle: a quarter of the kernel at K = 4096.  A tile whose K range is cut between
-//     workgroups is finished by the one that owns its k = 0 end: the others publish their fp32 accumulators
-//     (write-through stores + one flag word each, no fences) and the owner adds them in workgroup order
-//     (deterministic).  Small grids (< 128 tiles) keep the one-workgroup-per-(tile, K slice) form with fp32 slabs.
-//     Co-residency: an owner only waits for its successor, which publishes as soon as it has started -- progress is
-//     guaranteed while more than half of the CUs are available to this launch; the wait is bounded (5 s, then trap).
+//   * PERSISTENT forms, one workgroup per CU, where the plan (fp8_large_plan) finds them ahead of one workgroup per tile: workgroups that
+//     reach their tile boundaries at different times do not all store their 128 KiB of C at the same moment (1.7 TB/s with every MFMA idle).
+//     Stream-K deals the (tile, K tile) units out in equal contiguous ranges; the eight-phase kernel deals out whole tiles and, first, slices of
+//     the tiles that are left over.  A tile whose K range is cut between workgroups is finished by the one that owns its k = 0 end: the others
+//     publish their fp32 accumulators (write-through stores + one flag word each, no fences) and the owner adds them in workgroup order
+//     (deterministic).  Co-residency: an owner only waits for the workgroups that follow it, four at most, which publish as the first thing
+//     they do -- progress is guaranteed while more than half of the CUs are available to this launch; the wait is bounded (5 s, then trap).
 //   * results leave through a wave-private LDS transpose as full 128-byte row segments (epi_put / epi_flush, common.h).
 // Workgroup = WN x WM waves, wave tile = 128 rows (m) x 64 columns (n), K tile = 128.
 //
@@ -27,7 +25,7 @@
 // compute phase = one C quadrant of a wave (64 m x 32 n x 128 k = 4 MFMAs, 256 matrix cycles), the two waves of every SIMD
 // run one barrier apart so that one is in its MFMA cluster while the other issues its fragment reads and LDS-DMA, and the
 // direct-to-LDS loads stay in flight across the barriers behind COUNTED vmcnt waits (three half-tiles ahead).  The older
-// two-stage kernel (one vmcnt(0) + barrier per K tile) keeps the narrower tiles.
+// two-stage kernel (one vmcnt(0) + barrier per K tile) keeps the narrower tiles and short K.
 #include <algorithm>
 #include <type_traits>
 
@@ -49,7 +47,8 @@ struct Fp8LargeParams {
   int M, N, K;
   int a_per_token, b_per_channel, out_bf16;
   int tiles_m, tiles_n;
-  int streamk;             // 1: persistent grid, equal unit ranges; 0: one workgroup per (tile, K slice)
+  int streamk;             // 1: persistent grid (equal unit ranges; the 256 x 256 tile: whole tiles and slices of the rest); 0: one workgroup per (tile, K slice)
+  int slices;              // fp8_gemm_large8_kernel: K slices of each tile left over when every workgroup has had as many whole ones
   int ksplit;              // streamk == 0: K slices (blockIdx.y), fp32 slabs + reduce kernel when > 1
   float* partial;          // streamk == 0: [ksplit][M][N];  streamk == 1: [grid] accumulator images (see publish)
   unsigned* flags;         // streamk == 1: [grid] "image published", zeroed by the host before the launch where the grid cuts tiles
@@ -83,10 +82,9 @@ struct F8Units {
 // lane holds, for row m = mb*32 + l31, columns nb*32 + 8 q + 4 kh + (0..3), q = reg >> 2
 template <int NWAVE, bool BF16OUT>
 __device__ __forceinline__ void fp8_large_finish(const Fp8LargeParams& p, f32x16 (&acc)[2][4], unsigned char* smem,
-                                                 const F8Units& un, const __amdgpu_buffer_rsrc_t rp, bool head, bool tail,
-                                                 int w, int tile, int ktiles_total, int m0, int n0, int wave, int wm,
+                                                 int merge_end, const __amdgpu_buffer_rsrc_t rp, bool head, bool tail,
+                                                 int w, int m0, int n0, int wave, int wm,
                                                  int wn, int lane, unsigned long long* stamp = nullptr) {
-  const int G = un.G;
   const int kh = lane >> 5, l31 = lane & 31;
   if (p.streamk && !head) {
     // not the owner of this tile (always a workgroup's FIRST segment): publish the accumulators as they sit in the
@@ -107,10 +105,9 @@ __device__ __forceinline__ void fp8_large_finish(const Fp8LargeParams& p, f32x16
     return;
   }
   if (p.streamk && !tail) {
-    // owner of a tile whose K range continues in the following workgroups (always the LAST segment): add their images
-    // in workgroup order.  They were published long ago unless the whole tile is being computed right now.
-    const int64_t tile_end = (int64_t)(tile + 1) * ktiles_total;
-    for (int j = w + 1; j < G && un.begin(j) < tile_end; ++j) {
+    // owner of a tile whose K range continues in the following workgroups, up to merge_end: add their images in workgroup
+    // order.  Publishing is the first thing that they do.
+    for (int j = w + 1; j < merge_end; ++j) {
       if (threadIdx.x == 0) {
         // Bounded: workgroup j publishes its first segment right after it starts, so this only waits long if j is not
         // resident yet.  Progress needs two consecutive logical workgroups resident at some point, i.e. more than half
@@ -358,7 +355,10 @@ __global__ __launch_bounds__(WM * WN * 64) void fp8_gemm_large_kernel(Fp8LargePa
     }
     if constexpr (STAGES == 3) __syncthreads();      // every wave is done with the stage buffers
 
-    fp8_large_finish<NWAVE, BF16OUT>(p, acc, smem, un, rp, head, tail, w, tile, ktiles_total, m0, n0, wave, wm, wn, lane);
+    int merge_end = w + 1;
+    if (p.streamk && head && !tail)
+      while (merge_end < G && un.begin(merge_end) < (int64_t)(tile + 1) * ktiles_total) ++merge_end;
+    fp8_large_finish<NWAVE, BF16OUT>(p, acc, smem, merge_end, rp, head, tail, w, m0, n0, wave, wm, wn, lane);
   }
 }
 
@@ -394,6 +394,8 @@ __device__ __forceinline__ void f8_touch(u32x4& x) { asm volatile("" : "+v"(x));
 // The segment start is a raw barrier (no vmcnt(0): the previous tile's C stores drain under the next tile's loads).
 // Lab-only ablations of V = 2 (WRONG results, timing only): 4 = no LDS-DMA in the K loop, 5 = no fragment reads in the K
 // loop, 6 = no barriers in the K loop, 7 = MFMAs only.
+constexpr int F8_GROUP_M = 4;
+
 template <bool BF16OUT, int V>
 __global__ __launch_bounds__(512) void fp8_gemm_large8_kernel(Fp8LargeParams p) {
   constexpr int VS = V >= 4 ? 2 : V;                // schedule variant
@@ -412,12 +414,13 @@ __global__ __launch_bounds__(512) void fp8_gemm_large8_kernel(Fp8LargeParams p) 
   const int ktiles_total = p.K / BK;
   const int ntiles = p.tiles_m * p.tiles_n;
   const int G = gridDim.x;
-  const int64_t U = (int64_t)ntiles * ktiles_total;
-  F8Units un;
-  un.U = U; un.G = G;
   const int w = xcd_contiguous(blockIdx.x, G);
-  int u = (int)un.begin(w);
-  const int u_end = (int)un.begin(w + 1);
+  // every workgroup has ``full`` whole tiles; the tiles that are left go first, in slices of K that run side by side
+  const int full = ntiles / G, rest = (ntiles - full * G) * p.slices;
+  // the slices are dealt to the XCDs evenly, each a run of them (on as few XCDs as they fill, [3584, 18944], 2500 rows: 279 us, 140 tiles on four)
+  const int xcd = blockIdx.x % 8, on_xcd = blockIdx.x / 8;
+  const int part = xcd * (rest / 8) + min(xcd, rest % 8) + on_xcd;
+  const bool sliced = on_xcd < rest / 8 + (xcd < rest % 8 ? 1 : 0);
 
   const __amdgpu_buffer_rsrc_t ra = f8_rsrc(p.a, (uint32_t)((size_t)p.M * p.K));
   const __amdgpu_buffer_rsrc_t rb = f8_rsrc(p.w, (uint32_t)((size_t)p.N * p.K));
@@ -438,15 +441,20 @@ __global__ __launch_bounds__(512) void fp8_gemm_large8_kernel(Fp8LargeParams p) 
     }
 
   bool first_segment = true;
-  int seg_no = -1;
-  while (u < u_end) {
-    const int tile = u / ktiles_total;
-    const int k0 = u - tile * ktiles_total;
-    int k1 = min(ktiles_total, k0 + (u_end - u));
-    u += k1 - k0;
+  for (int round = sliced ? -1 : 0; round < full; ++round) {
+    int tile = round * G + w, k0 = 0, k1 = ktiles_total;
+    if (round < 0) {
+      const int slice = part % p.slices;
+      tile = full * G + part / p.slices;
+      k0 = slice * ktiles_total / p.slices;
+      k1 = (slice + 1) * ktiles_total / p.slices;
+    }
     const bool head = k0 == 0, tail = k1 == ktiles_total;
     if (p.debug == 2) k1 = k0 + 1;
-    const int tm = tile / p.tiles_n, tn = tile % p.tiles_n;
+    // four row panels at a time: the tiles that an XCD's workgroups run together share rows of both operands
+    const int group = tile / (F8_GROUP_M * p.tiles_n), in_group = tile - group * F8_GROUP_M * p.tiles_n;
+    const int rows = min(F8_GROUP_M, p.tiles_m - group * F8_GROUP_M);
+    const int tm = group * F8_GROUP_M + in_group % rows, tn = in_group / rows;
     const int m0 = tm * BM, n0 = tn * BN;
     unsigned long long* stamp = nullptr;
 #define F8_STAMP(i)
@@ -630,7 +638,7 @@ __global__ __launch_bounds__(512) void fp8_gemm_large8_kernel(Fp8LargeParams p) 
 #undef F8_BAR
 #undef F8_LGKM0
     F8_STAMP(2)
-    fp8_large_finish<NWAVE, BF16OUT>(p, acc, smem, un, rp, head, tail, w, tile, ktiles_total, m0, n0, wave, wm, wn, lane, stamp);
+    fp8_large_finish<NWAVE, BF16OUT>(p, acc, smem, part + p.slices, rp, head, tail, part, m0, n0, wave, wm, wn, lane, stamp);
     if (stamp) stamp[7] = __builtin_amdgcn_s_memrealtime();
 #undef F8_STAMP
   }
@@ -700,37 +708,61 @@ static int launch_fp8_large(const Fp8LargeParams& p, int grid_x, hipStream_t st)
 
 using namespace aphro;
 
-struct Fp8LargePlan { int wm, wn, tiles_m, tiles_n, streamk, grid, ksplit; };
+struct Fp8LargePlan { int wm, wn, tiles_m, tiles_n, streamk, grid, ksplit, eight, slices; };
 
 static int cu_count() { return device_cu_count(); }
 
-// Stream-K (one persistent workgroup per CU) when the biggest tile the shape allows still gives >= 128 tiles: then
-// every workgroup gets at least half a tile's K loop and a tile is cut between at most 3 workgroups.  Below that: one
-// workgroup per tile, narrower tiles and up to 8 K slices (fp32 slabs) so that ~200+ workgroups exist.
+// The form by the time it is expected to take (MI355X, ns).  Of the forms measured for 158 sizes (200 to 8192 rows, N 1280 to 37888, K 512 to
+// 18944) the one taken is 0.7 % behind the best on average.  us:
+//  * one workgroup per tile, or per tile and K slice: rounds over the CUs, a last one that is not full 0.68 of a full one and 0.27 by how full it
+//    is; a step of K is slower the more CUs run it; slabs are written and read again at 3 TB/s.  Few tiles: small ones without slices ([6144, 4096],
+//    520 rows: 128 x 128 29.6, 256 x 128 35.1 and in two slices 53.8; 1100 rows of [4096, 4096] 128 x 256 34.6, 256 x 128 in two slices 56.6).
+//  * stream-K of 256 x 128 tiles for some sizes of few tiles and long K ([4096, 14336], 520 rows: 61.9, in slices 77.6; [8192, 8192], 480 rows 45.3),
+//    of 256 x 256 for fewer than 16 K tiles and many rows ([28672, 1024], 8192 rows: 310, 256 x 128 364).
+//  * the eight-phase kernel on 256 x 256 tiles, whole ones and the rest in up to four slices each, from 16 K tiles on (below that its longer
+//    prologue costs more than its K loop gains: K = 512 / 1024 29.6 / 47.4, the two-stage kernel 25.8 / 43.6).  Equal unit ranges instead, cut wherever
+//    they end, put the workgroups of an XCD at different places of K, where they share nothing in its L2 ([28672, 4096], 5000 / 6500 / 8192
+//    rows 526 / 762 / 762, here 461 / 590 / 722, the last by the order of the tiles; [4096, 14336], 6500 rows 414 / 309).
 static Fp8LargePlan fp8_large_plan(int64_t M, int64_t N, int64_t K) {
-  Fp8LargePlan pl;
-  pl.wm = M > 128 ? 2 : 1;
-  const int64_t rows = (M + 128 * pl.wm - 1) / (128 * pl.wm);
-  const int mode = APHRO_LAB_ENV_INT("APHRO_FP8_LARGE_STREAMK", -1);
-  const int64_t big_tiles = N % 256 == 0 ? rows * (N / 256) : rows * (N / 128);
-  pl.streamk = (mode >= 0 ? mode : (big_tiles >= 128)) && device_coresident_cu_count() > 0;
-  pl.ksplit = 1;
-  if (pl.streamk) {
-    pl.wn = N % 256 == 0 ? 4 : 2;
-    pl.grid = cu_count();
-  } else {
-    pl.wn = (N % 256 == 0 && rows * (N / 256) >= 200) ? 4 : 2;
-    const int64_t tiles = rows * (N / (64 * pl.wn));
-    for (int s = 2; s <= 8; ++s) {
-      if (tiles * pl.ksplit >= 200) break;
-      if (K % (s * 128) == 0 && K / s >= 1024) pl.ksplit = s;
+  const int cus = cu_count();
+  const bool resident = device_coresident_cu_count() > 0;
+  const int64_t T = K / 128;
+  Fp8LargePlan best = {};
+  int64_t best_ns = -1;
+  auto offer = [&](int wm, int wn, int streamk, int ksplit, int eight, int slices, int64_t ns) {
+    if (best_ns >= 0 && ns >= best_ns) return;
+    best_ns = ns;
+    best.wm = wm; best.wn = wn; best.streamk = streamk; best.ksplit = ksplit; best.eight = eight; best.slices = slices;
+    best.tiles_m = (int)((M + 128 * wm - 1) / (128 * wm));
+    best.tiles_n = (int)(N / (64 * wn));
+    best.grid = streamk ? cus : best.tiles_m * best.tiles_n;
+  };
+  auto tiles_of = [&](int wm, int wn) { return (M + 128 * wm - 1) / (128 * wm) * (N / (64 * wn)); };
+  constexpr int64_t STEP[2][2] = {{655, 750}, {775, 1170}}, AROUND[2][2] = {{5750, 7705}, {6550, 8360}}, CROWD[2][2] = {{15, 35}, {27, 30}};
+  for (int wm = 1; wm <= 2; ++wm)
+    for (int wn = 2; wn <= (N % 256 == 0 ? 4 : 2); wn += 2)
+      for (int ks = 1; ks <= 8; ++ks) {
+        if (K % (ks * 128) != 0 || (ks > 1 && K / ks < 1024)) continue;
+        const int a = wm - 1, b = wn / 4;
+        const int64_t wgs = tiles_of(wm, wn) * ks, full = wgs / cus, rest = wgs % cus, busy = full ? cus : rest;
+        const int64_t round = AROUND[a][b] + (full ? 120 * wm * wn : 0) + T / ks * STEP[a][b] * (100 * cus + CROWD[a][b] * busy) / (100 * cus);
+        const int64_t last = rest == 0 ? 0 : full == 0 ? round : round * (68 * cus + 27 * rest) / (100 * cus);
+        offer(wm, wn, 0, ks, 0, 1, full * round + last + (ks > 1 ? 3555 + ks * M * N * 4 / 2985 : 0));
+      }
+  // Stream-K: a tile is cut into five at most, and EVERY workgroup has K tiles of its own -- the owner of a cut tile waits for each that follows it,
+  // and one without any would never publish.
+  if (resident && tiles_of(2, 2) >= 64 && tiles_of(2, 2) * T >= 4 * cus) offer(2, 2, 1, 1, 0, 1, 17925 + tiles_of(2, 2) * (T * 1010 + 1215) / cus);
+  if (resident && N % 256 == 0 && K < 2048 && tiles_of(2, 4) >= 128 && tiles_of(2, 4) * T >= 4 * cus)
+    offer(2, 4, 1, 1, 0, 1, 6220 + (tiles_of(2, 4) % cus ? tiles_of(2, 4) * T * 2275 / cus + 13260 : tiles_of(2, 4) * T * 2100 / cus));
+  if (resident && N % 256 == 0 && K >= 2048) {
+    const int64_t tiles = tiles_of(2, 4), full = tiles / cus, rest = tiles % cus;
+    for (int s = 1; s <= 4 && (s == 1 || rest * s <= cus); ++s) {
+      const int64_t steps = T * 830 * (100 * cus + 56 * (full ? cus : rest * s)) / (100 * cus), round = 9585 + steps;
+      const int64_t last = rest == 0 ? 0 : s > 1 ? 9585 + steps / s + 13290 : full == 0 ? round : round * (78 * cus + 24 * rest) / (100 * cus);
+      offer(2, 4, 1, 1, 1, s, full * round + last);
     }
-    { const int s = APHRO_LAB_ENV_INT("APHRO_FP8_LARGE_KSPLIT", 0); if (s >= 1 && K % (s * 128) == 0) pl.ksplit = s; }
-    pl.grid = (int)tiles;
   }
-  pl.tiles_m = (int)rows;
-  pl.tiles_n = (int)(N / (64 * pl.wn));
-  return pl;
+  return best;
 }
 
 constexpr size_t FP8_LARGE_FLAG_BYTES = 4096;
@@ -766,32 +798,21 @@ extern "C" int aphro_scaled_mm_fp8_large(void* out, const void* a, const void* b
   p.bias = (const uint16_t*)bias; p.c = (uint16_t*)out;
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
   p.a_per_token = a_scale_per_token; p.b_per_channel = b_scale_per_channel; p.out_bf16 = out_dtype == APHRO_BF16;
-  p.tiles_m = pl.tiles_m; p.tiles_n = pl.tiles_n; p.streamk = pl.streamk; p.ksplit = pl.ksplit;
+  p.tiles_m = pl.tiles_m; p.tiles_n = pl.tiles_n; p.streamk = pl.streamk; p.ksplit = pl.ksplit; p.slices = pl.slices;
   p.flags = nullptr; p.partial = (float*)workspace;
   p.debug = APHRO_LAB_ENV_INT("APHRO_FP8_LARGE_DEBUG", 0);
   if (pl.streamk) {
     p.flags = (unsigned*)workspace;
     p.partial = (float*)((char*)workspace + FP8_LARGE_FLAG_BYTES);
-    // no tile is cut where the workgroups divide the tiles: nothing is published or waited for then (the launch in front: 5 us; prompts of 8192
-    // rows on 4096 to 28672 columns are such: four layers' products 9458 -> 9327 us with all else in the step)
-    if ((int64_t)pl.tiles_m * pl.tiles_n % pl.grid != 0) {
+    // no tile is cut where the workgroups divide the tiles, or the eight-phase kernel does not slice what is left: nothing is published or waited
+    // for then (the launch in front: 5 us; prompts of 8192 rows on 4096 to 28672 columns are such: four layers' products 9458 -> 9327 us)
+    if ((int64_t)pl.tiles_m * pl.tiles_n % pl.grid != 0 && !(pl.eight && pl.slices == 1)) {
       hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(FP8_LARGE_FLAG_BYTES / 4), 0, st, p.flags);
       APHRO_LAUNCH_CHECK();
     }
   }
   int rc;
-  // eight-phase schedule from 16 K tiles per output tile up: below that the longer prologue (seven half-tiles, the stagger
-  // barriers) costs more than the K loop gains (K = 512 / 1024: 29.6 / 47.4 us against 25.8 / 43.6 for the two-stage kernel)
-  const int eight_lab = APHRO_LAB_ENV_INT("APHRO_FP8_LARGE_8PHASE", -1);
-  const int eight = eight_lab >= 0 ? eight_lab : (K >= 2048 ? 2 : 0);
-  if (pl.wm == 2 && pl.wn == 4 && pl.streamk && eight) {
-    switch (eight) {
-#define F8_V(v) case v: rc = p.out_bf16 ? launch_fp8_large8_t<true, v>(p, pl.grid, st) : launch_fp8_large8_t<false, v>(p, pl.grid, st); break;
-      F8_V(2)
-#undef F8_V
-      default: set_error("scaled_mm_fp8_large: unknown schedule variant %d", eight); return APHRO_ERR_INVALID;
-    }
-  }
+  if (pl.eight) rc = p.out_bf16 ? launch_fp8_large8_t<true, 2>(p, pl.grid, st) : launch_fp8_large8_t<false, 2>(p, pl.grid, st);
   else if (pl.wm == 2) rc = pl.wn == 4 ? launch_fp8_large<2, 4, 2>(p, pl.grid, st) : launch_fp8_large<2, 2, 3>(p, pl.grid, st);
   else rc = pl.wn == 4 ? launch_fp8_large<1, 4, 3>(p, pl.grid, st) : launch_fp8_large<1, 2, 3>(p, pl.grid, st);
   if (rc != APHRO_OK) return rc;
