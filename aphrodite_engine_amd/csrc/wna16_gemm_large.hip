@@ -46,6 +46,7 @@ struct Wna16LargeParams {
   // stream-K form (see fp8_gemm_large.hip): one persistent workgroup per CU, equal (tile, K tile) unit ranges; `partial`
   // then holds the accumulator images [grid][NWAVE * 32 KiB] and `flags` one "image published" word per workgroup
   int streamk, grid;      // grid: persistent workgroups (= CUs)
+  int slices;             // wna16_gemm_large8_kernel: K slices of each tile left over when every workgroup has had as many whole ones
   unsigned* flags;
   // W8A16 form (template WFP8): e4m3 weights [N, K] (K-contiguous), per-tensor / per-channel fp32 scales applied in the
   // epilogue, optional bias in the output type.  qw / qz / sc / group_size / zero_offset are unused then.
@@ -121,8 +122,8 @@ __device__ __forceinline__ f16x8 dq8_scaled(uint32_t w, f16x2 zh, f16x2 zh16, f1
 // + converted + stored (owner), or written as an fp32 slab (split-K form).  Shared by both kernels.
 template <int NWAVE, bool WFP8>
 __device__ __forceinline__ void wna16_large_finish(const Wna16LargeParams& p, f32x16 (&acc)[2][4], unsigned char* smem,
-                                                   const __amdgpu_buffer_rsrc_t rp, bool head, bool tail, int w, int GW, int64_t U,
-                                                   int tile, int ktiles_total, int m0, int n0, int wave, int wm, int wn, int lane) {
+                                                   const __amdgpu_buffer_rsrc_t rp, bool head, bool tail, int w, int merge_end, int m0,
+                                                   int n0, int wave, int wm, int wn, int lane) {
   const int kh = lane >> 5, l31 = lane & 31;
   // ---- what happens to the accumulators: lane holds, for row m = mb*32 + l31, columns nb*32 + 8 q + 4 kh + (0..3) ----------
   if (p.streamk && !head) {
@@ -144,10 +145,9 @@ __device__ __forceinline__ void wna16_large_finish(const Wna16LargeParams& p, f3
     return;
   }
   if (p.streamk && !tail) {
-    // owner of a tile whose K range continues in the following workgroups (always the LAST segment): add their images in
+    // owner of a tile whose K range continues in the following workgroups, up to merge_end: add their images in
     // workgroup order (deterministic).  Bounded wait, see fp8_gemm_large.hip.
-    const int64_t tile_end = (int64_t)(tile + 1) * ktiles_total;
-    for (int j = w + 1; j < GW && j * U / GW < tile_end; ++j) {
+    for (int j = w + 1; j < merge_end; ++j) {
       if (threadIdx.x == 0) {
         const unsigned long long t0 = wall_clock64();
         while (__hip_atomic_load(p.flags + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
@@ -501,7 +501,10 @@ __global__ __launch_bounds__(WM * WN * 64) void wna16_gemm_large_kernel(Wna16Lar
   }
 
   if constexpr (STAGES == 3) __syncthreads();      // every wave is done with the stage buffers
-  wna16_large_finish<NWAVE, WFP8>(p, acc, smem, rp, head, tail, w, GW, U, tile, ktiles_total, m0, n0, wave, wm, wn, lane);
+  int merge_end = w + 1;
+  if (p.streamk && head && !tail)
+    while (merge_end < GW && merge_end * U / GW < (int64_t)(tile + 1) * ktiles_total) ++merge_end;
+  wna16_large_finish<NWAVE, WFP8>(p, acc, smem, rp, head, tail, w, merge_end, m0, n0, wave, wm, wn, lane);
   }   // segments
 }
 
@@ -535,6 +538,8 @@ __device__ __forceinline__ void lg_lds_write128(uint32_t addr, const u32x4& v) {
 }
 __device__ __forceinline__ void lg_touch(u32x4& x) { asm volatile("" : "+v"(x)); }
 
+constexpr int LG_GROUP_M = 4;
+
 template <bool BF16OUT, bool WDMA = false, bool STRIP = false>
 __global__ __launch_bounds__(512) void wna16_gemm_large8_kernel(Wna16LargeParams p) {
   static_assert(!(WDMA && STRIP), "the two-pass form reads f16 W^T: the strip-major order is pass 1's business");
@@ -551,14 +556,17 @@ __global__ __launch_bounds__(512) void wna16_gemm_large8_kernel(Wna16LargeParams
   const int ktiles_total = p.K / BK;
   const int ntiles = p.tiles_m * p.tiles_n;
   const int GW = gridDim.x;
-  const int64_t U = (int64_t)ntiles * ktiles_total;
   auto xcd_contiguous = [](int bid, int n) {
     const int q = n / 8, r = n % 8, xcd = bid % 8, k = bid / 8;
     return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + k;
   };
   const int w = xcd_contiguous(blockIdx.x, GW);
-  int u = (int)(w * U / GW);
-  const int u_end = (int)((w + 1) * U / GW);
+  // every workgroup has ``full`` whole tiles; the tiles that are left go first, in slices of K that run side by side, dealt to the XCDs evenly
+  // (fp8_gemm_large8_kernel's way)
+  const int full = ntiles / GW, rest = (ntiles - full * GW) * p.slices;
+  const int xcd = blockIdx.x % 8, on_xcd = blockIdx.x / 8;
+  const int part = xcd * (rest / 8) + min(xcd, rest % 8) + on_xcd;
+  const bool sliced = on_xcd < rest / 8 + (xcd < rest % 8 ? 1 : 0);
 
   const __amdgpu_buffer_rsrc_t ra = lg_rsrc(p.a, (uint32_t)((size_t)p.M * p.lda * 2));
   const __amdgpu_buffer_rsrc_t rb = WDMA ? lg_rsrc(p.wt, (uint32_t)((size_t)p.N * p.K * 2))
@@ -584,13 +592,18 @@ __global__ __launch_bounds__(512) void wna16_gemm_large8_kernel(Wna16LargeParams
   const int zshift = (lane & 1) * 16;               // this thread's four zero-point nibbles inside its qzeros dword
 
   bool first_segment = true;
-  while (u < u_end) {
-    const int tile = u / ktiles_total;
-    const int k0 = u - tile * ktiles_total;
-    const int k1 = min(ktiles_total, k0 + (u_end - u));
-    u += k1 - k0;
+  for (int round = sliced ? -1 : 0; round < full; ++round) {
+    int tile = round * GW + w, k0 = 0, k1 = ktiles_total;
+    if (round < 0) {
+      const int slice = part % p.slices;
+      tile = full * GW + part / p.slices;
+      k0 = slice * ktiles_total / p.slices;
+      k1 = (slice + 1) * ktiles_total / p.slices;
+    }
     const bool head = k0 == 0, tail = k1 == ktiles_total;
-    const int tm = tile / p.tiles_n, tn = tile % p.tiles_n;
+    const int group = tile / (LG_GROUP_M * p.tiles_n), in_group = tile - group * LG_GROUP_M * p.tiles_n;   // four row panels at a time
+    const int rows = min(LG_GROUP_M, p.tiles_m - group * LG_GROUP_M);
+    const int tm = group * LG_GROUP_M + in_group % rows, tn = in_group / rows;
     const int m0 = tm * BM, n0 = tn * BN;
     if (!first_segment) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_s_barrier(); }
     first_segment = false;
@@ -821,7 +834,7 @@ __global__ __launch_bounds__(512) void wna16_gemm_large8_kernel(Wna16LargeParams
     }
 #undef LG_BAR
 #undef LG_LGKM0
-    wna16_large_finish<NWAVE, false>(p, acc, smem, rp, head, tail, w, GW, U, tile, ktiles_total, m0, n0, wave, wm, wn, lane);
+    wna16_large_finish<NWAVE, false>(p, acc, smem, rp, head, tail, part, part + p.slices, m0, n0, wave, wm, wn, lane);
   }
 }
 
@@ -1008,7 +1021,9 @@ static LargePlan large_plan(int64_t M, int64_t N, int64_t K, int64_t gs) {
 // Two-pass form (dequantise-transpose once per call, then the eight-phase schedule with the weights by LDS-DMA): where every
 // weight would otherwise be dequantised by >= TWO_PASS_ROW_TILES row-tile workgroups and the shape runs the eight-phase
 // stream-K plan.  Costs K x N f16 of workspace per call.  APHRO_WNA16_LARGE_TWO_PASS=0/1 forces (tests compare the two forms' bits).
-constexpr int64_t TWO_PASS_MIN_M = 6144;      // (M = 4096: the fused form is 2-4 % faster on all four Llama-3-8B shapes; 8192: 4-14 % slower)
+// (us, fused / two passes: 28672 x 4096, 2560 rows 572 / 564, 3072 673 / 653, 4096 857 / 813, 6100 1293 / 1204; 4096 x 14336, 3500 rows 391 / 358;
+// 6144 x 4096, 3072 rows 168 / 164, 5000 243 / 227; 4096 x 4096, 3072 rows 114 / 106; 8192 x 8192, 4096 rows 480 / 446)
+constexpr int64_t TWO_PASS_MIN_M = 3072;
 static bool large_two_pass(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs) {
   const int force = knobs().wna16_large_two_pass;
   const int eight = knobs().wna16_large_8phase >= 0 ? knobs().wna16_large_8phase : (K >= 2048 ? 1 : 0);
@@ -1023,15 +1038,38 @@ static size_t large_scratch_bytes(const LargePlan& pl, int64_t M, int64_t N) {
   return pl.ksplit > 1 ? (size_t)pl.ksplit * M * N * sizeof(float) : 0;
 }
 
-// stream-K: point the kernel at its flag words, cleared where it cuts tiles
-static int large_bind_scratch(Wna16LargeParams& p, const LargePlan& pl, char* ws, hipStream_t st) {
+// (the eight-phase schedule on the 256 x 256 stream-K tile from 32 K tiles per output tile up; APHRO_WNA16_LARGE_8PHASE=0/1 forces)
+static bool large_eight(const LargePlan& pl, int64_t K) {
+  const int eight = knobs().wna16_large_8phase >= 0 ? knobs().wna16_large_8phase : (K >= 2048 ? 1 : 0);
+  return pl.wm == 2 && pl.wn == 4 && pl.streamk && eight;
+}
+
+// The eight-phase kernel's slices of the tiles left over, and the time (ns) that it is expected to take: whole tiles and, in front, the rest in up
+// to four slices (equal unit ranges, cut wherever they end, keep the workgroups of an XCD from sharing rows of the operands in its L2; two passes, us
+// before / now: 28672 x 4096, 6500 / 7200 rows 1553 / 1710 and 1324 / 1390, 6144 x 4096, 6500 rows 409 / 301, 4096 x 4096, 6500 rows 268 / 210; fused
+// it is level, 3000 rows of 4096 x 4096 121 / 115, 1340 of 28672 x 4096 362 / 370).
+struct LargeRounds { int slices; int64_t ns; };
+static LargeRounds large_rounds(int64_t tiles, int64_t T, int64_t cus, bool two_pass) {
+  const int64_t full = tiles / cus, rest = tiles % cus, step = two_pass ? 1600 : 1930, round = 6000 + T * step;
+  LargeRounds best = {1, -1};
+  for (int s = 1; s <= 4 && (s == 1 || (rest * s <= cus && T / s >= 4)); ++s) {
+    const int64_t last = s > 1 ? 6000 + T * step / s + 13290 : round * (full ? 78 * cus + 24 * rest : 56 * cus + 42 * rest) / (100 * cus);
+    const int64_t ns = full * round + (rest ? last : 0);
+    if (best.ns < 0 || ns < best.ns) best = {s, ns};
+  }
+  return best;
+}
+
+// stream-K: point the kernel at its flag words, cleared where it cuts tiles.  eight: the kernel is wna16_gemm_large8_kernel
+static int large_bind_scratch(Wna16LargeParams& p, const LargePlan& pl, char* ws, bool eight, hipStream_t st) {
   p.streamk = pl.streamk; p.grid = pl.grid; p.ksplit = pl.ksplit; p.flags = nullptr; p.partial = (float*)ws;
   if (pl.streamk) {
     p.flags = (unsigned*)ws;
     p.partial = (float*)(ws + LARGE_FLAG_BYTES);
-    // (no tile is cut where the workgroups divide the tiles, as in fp8_gemm_large.hip)
+    // (no tile is cut where the workgroups divide the tiles, or the eight-phase kernel does not slice what is left, as in fp8_gemm_large.hip)
     const int64_t tiles = (int64_t)((p.M + 128 * pl.wm - 1) / (128 * pl.wm)) * (p.N / (64 * pl.wn));
-    if (tiles % pl.grid != 0) {
+    p.slices = eight ? large_rounds(tiles, p.K / 64, pl.grid, p.wt != nullptr).slices : 1;
+    if (tiles % pl.grid != 0 && !(eight && p.slices == 1)) {
       hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(LARGE_FLAG_BYTES / 4), 0, st, p.flags);
       APHRO_LAUNCH_CHECK();
     }
@@ -1040,12 +1078,6 @@ static int large_bind_scratch(Wna16LargeParams& p, const LargePlan& pl, char* ws
 }
 
 extern "C" int aphro_wna16_strip_geometry(int64_t M, int64_t N, int64_t K, int64_t groups, int* geom);      // wna16_gemm_resident.hip
-
-// (the eight-phase schedule on the 256 x 256 stream-K tile from 32 K tiles per output tile up; APHRO_WNA16_LARGE_8PHASE=0/1 forces)
-static bool large_eight(const LargePlan& pl, int64_t K) {
-  const int eight = knobs().wna16_large_8phase >= 0 ? knobs().wna16_large_8phase : (K >= 2048 ? 1 : 0);
-  return pl.wm == 2 && pl.wn == 4 && pl.streamk && eight;
-}
 
 // 65 to 128 float16 rows of a matrix below 2^25 weights belong to the decode kernels otherwise, which round no weight: nor does the tile's EXACT form.
 static Wna16RowsPlan rows_exact_plan(int64_t M, int64_t N, int64_t K, int64_t gs) {
@@ -1066,9 +1098,11 @@ static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_
     if (exact.mb > 0) return exact;
   }
   int64_t other_ns = -1;
-  if (pl.streamk) {            // 1.93 us per 256 x 256 x 64 of a CU's even share, 6 us per tile of it, 18 us around them
+  if (pl.streamk) {            // (the first of two passes writes the weights at 0.43 ps each)
     const int64_t tiles = (M + 255) / 256 * ((N + 255) / 256);
-    other_ns = 18000 + (tiles * (K / 64) * 1930 + tiles * 6000) / pl.grid;
+    const bool two_pass = large_two_pass(pl, M, N, K, gs);
+    if (large_eight(pl, K)) other_ns = large_rounds(tiles, K / 64, pl.grid, two_pass).ns + (two_pass ? 3000 + N * K * 43 / 100000 : 0);
+    else other_ns = 18000 + (tiles * (K / 64) * 1930 + tiles * 6000) / pl.grid;
   }
   return wna16_rows_plan(M, N, K, gs, pl.streamk ? 0 : 36ll << 20, other_ns);
 }
@@ -1197,7 +1231,7 @@ static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const 
     p.wt = (const uint16_t*)ws;
     ws += ((size_t)N * K * 2 + 255) / 256 * 256;
   }
-  if (int rcb = large_bind_scratch(p, pl, ws, st)) return rcb;
+  if (int rcb = large_bind_scratch(p, pl, ws, large_eight(pl, K), st)) return rcb;
   int rc;
   // eight-phase schedule on the 256 x 256 stream-K tile from 32 K tiles per output tile up (APHRO_WNA16_LARGE_8PHASE=0/1 forces)
   if (large_eight(pl, K)) rc = launch_large8(p, st);
@@ -1335,7 +1369,7 @@ extern "C" int aphro_fp8_w8a16_gemm_large(void* out, const void* a, const void* 
   p.out_bf16 = dtype == APHRO_BF16; p.scale_bf16 = 0;
   const LargePlan pl = large_plan(M, N, K, 64);
   p.tiles_m = p.tiles_n = 0;
-  if (int rcb = large_bind_scratch(p, pl, (char*)workspace + (dtype == APHRO_BF16 ? ((size_t)M * K * 2 + 255) / 256 * 256 : 0), st)) return rcb;
+  if (int rcb = large_bind_scratch(p, pl, (char*)workspace + (dtype == APHRO_BF16 ? ((size_t)M * K * 2 + 255) / 256 * 256 : 0), false, st)) return rcb;
   p.w8 = (const uint8_t*)w; p.w_scales = w_scales; p.w_per_channel = w_scale_per_channel; p.bias = (const uint16_t*)bias;
   int rc;
   if (pl.wm == 2) rc = pl.wn == 4 ? launch_large<2, 4, true>(p, st) : launch_large<2, 2, true>(p, st);
