@@ -529,7 +529,7 @@ static bool rw_groups_exact(int64_t K, int64_t gs) { return (rw_inv_group(gs) * 
 
 // Tile height and K slices by the time they are expected to take (MI355X, ns; within 10 % of what was measured for 65 .. 4096 rows of
 // Llama-3-8B's and -70B's matrices): rounds of workgroups over the CUs, each 170 + 200 per 32-row block and K tile and 4.7 us around
-// them, a last one that is not full 0.7 of that and 0.3 by how full it is (few workgroups run at a higher clock and have the memory to
+// them, a last one that is not full 0.74 of that and 0.26 by how full it is (few workgroups run at a higher clock and have the memory to
 // themselves), and the slabs written and read again at 2.2 TB/s behind 3 us.  Of the forms measured for 150 to 4096 rows of 28672 x 4096, 6144 x
 // 4096, 4096 x 4096 and 4096 x 14336 the one taken is 0.1 % behind the best on average (a last round counted whole: 2.2 %).  us: 6144 x 4096,
 // 150 rows: five blocks and four slices 24.3, three and two 21.1; 900 rows, five blocks in 1.1 rounds 69.8, three in 1.9 59.6; 4096 x 14336, 150
@@ -546,7 +546,7 @@ Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t gs, int64
       const int64_t slabs = tiles_m * mb * 32 * N * 4 * ks;
       if (ks > 1 && slabs > slab_bytes) break;
       const int64_t full = tiles * ks / cus, rest = tiles * ks % cus, round = (T + ks - 1) / ks * (170 + 200 * mb) + 4700;
-      const int64_t ns = full * round + (rest ? round * (7 * cus + 3 * rest) / (10 * cus) : 0) + (ks > 1 ? 3000 + slabs * 45 / 100000 : 0);
+      const int64_t ns = full * round + (rest ? round * (74 * cus + 26 * rest) / (100 * cus) : 0) + (ks > 1 ? 3000 + slabs * 45 / 100000 : 0);
       if (best_ns < 0 || ns < best_ns) { best = {mb, ks, false}; best_ns = ns; }
     }
   }
