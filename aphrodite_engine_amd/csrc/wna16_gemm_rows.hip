@@ -531,7 +531,7 @@ static bool rw_groups_exact(int64_t K, int64_t gs) { return (rw_inv_group(gs) * 
 // Llama-3-8B's and -70B's matrices): rounds of workgroups over the CUs, each 170 + 200 per 32-row block and K tile and 4.7 us around
 // them, a last one that is not full 0.74 of that and 0.26 by how full it is (few workgroups run at a higher clock and have the memory to
 // themselves), and the slabs written and read again at 2.2 TB/s behind 3 us.  Of the forms measured for 150 to 4096 rows of 28672 x 4096, 6144 x
-// 4096, 4096 x 4096 and 4096 x 14336 the one taken is 0.1 % behind the best on average (a last round counted whole: 2.2 %).  us: 6144 x 4096,
+// 4096, 4096 x 4096 and 4096 x 14336 the one taken is 0.2 % behind the best on average (a last round counted whole: 2.2 %).  us: 6144 x 4096,
 // 150 rows: five blocks and four slices 24.3, three and two 21.1; 900 rows, five blocks in 1.1 rounds 69.8, three in 1.9 59.6; 4096 x 14336, 150
 // rows: one slice 82, two 49, four 32; 4096 x 4096, 150 rows: five blocks and four slices 20.6, three and three 18.2.
 Wna16RowsPlan wna16_rows_plan(int64_t M, int64_t N, int64_t K, int64_t gs, int64_t slab_bytes, int64_t other_ns) {
