@@ -31,7 +31,10 @@ struct RowsPlan { int mt, nt, ksplit; };
 //  * from 129 rows of x on a 64-row tile's stages leave room for one workgroup a CU (rows_dispatch), so that more than 256 of them run in two
 //    rounds: no second workgroup a CU, and 128 rows of w above 256 tiles.  FP8, raw sums, 129 / 160 / 192 rows: [6144, 4096] 15.2 / 16.6 / 18.3 in 5
 //    slices, 12.5 / 13.2 / 14.6 in 2; [17408, 4096] 39.6 / 41.1 / 45.5 by 64, 29.3 / 30.5 / 31.4 by 128.
-inline RowsPlan rows_plan(int64_t M, int64_t w_rows, int64_t row_bytes) {
+//  * 16-bit products of 65 to 160 rows of x on weights of two rounds and more of 256 rows a workgroup, the last nine tenths full, K >= 2560: those
+//    (``wide``), which read x through LDS half as often ([128256, 4096], 65 / 96 / 128 / 160 rows 192 / 198 / 208 / 229 by 128 rows, 176 / 180 / 184 /
+//    212 here; 176 rows 243 / 256; rounds less full lose: [32768, 4096], 128 rows 64 / 82, [151552, 2048], 150 rows 165 / 174).
+inline RowsPlan rows_plan(int64_t M, int64_t w_rows, int64_t row_bytes, bool wide = false) {
   RowsPlan plan;
   const int t64 = (int)((w_rows + 63) / 64), t128 = (int)((w_rows + 127) / 128), steps = (int)(row_bytes / 128);
   const int mt = (int)((M + 15) / 16);
@@ -45,6 +48,12 @@ inline RowsPlan rows_plan(int64_t M, int64_t w_rows, int64_t row_bytes) {
   if (mt <= 4) {
     plan.nt = t128 >= 160 && (mt > 2 || t64 < 480) ? 2 : 1;
     plan.ksplit = t64 >= 160 ? 1 : split(t64, true);
+    return plan;
+  }
+  const int t256 = (int)((w_rows + 255) / 256), rounds = (t256 + 255) / 256;
+  if (wide && plan.mt <= 10 && rounds >= 2 && t256 * 10 >= rounds * 256 * 9 && row_bytes >= 40 * 128) {
+    plan.nt = 4;
+    plan.ksplit = 1;
     return plan;
   }
   const bool lone = plan.mt > 8;
@@ -154,11 +163,11 @@ struct RowsTile {
   }
 };
 
-// f(MT, NT, WR, NS) for a plan.  Stages: as many as let two workgroups share a CU's 160 KB; from 129 rows of x on, three with 64 rows of w, and one
+// f(MT, NT, WR, NS) for a plan (WIDE: of those that may have 256 rows of w).  Stages: as many as let two workgroups share a CU's 160 KB; from 129 rows of x on, three with 64 rows of w, and one
 // workgroup a CU (two stages and two workgroups: [6144, 4096] FP8, 160 rows, 5 slices 13.7 us, this in 2 slices 13.2).  128-row tiles that all
 // run at once with one workgroup a CU ([22016, 4096], 65 rows and more) get eight waves and deeper stages, more tiles than CUs two stages:
 // bf16 [37888, 3584], 65 / 160 rows 73 / 99 us deep, 68 / 93 with two; [62000, 4096], 65 / 160 rows 111 / 133 and 115 / 126.
-template <typename F>
+template <bool WIDE, typename F>
 int rows_dispatch(const RowsPlan& plan, int tiles_n, F&& f) {
 #define ROWS(MT, NT, WR, NS) f(std::integral_constant<int, MT>{}, std::integral_constant<int, NT>{}, std::integral_constant<int, WR>{}, std::integral_constant<int, NS>{})
   const bool many = tiles_n >= 512 || (tiles_n > 256 && (plan.mt > 8 || tiles_n < 448));
@@ -172,6 +181,15 @@ int rows_dispatch(const RowsPlan& plan, int tiles_n, F&& f) {
       case 8: return ROWS(8, 1, 1, 3);
       case 10: return ROWS(10, 1, 1, 3);
       default: return ROWS(12, 1, 1, 3);
+    }
+  }
+  if constexpr (WIDE) {
+    if (plan.nt == 4) {
+      switch (plan.mt) {
+        case 6: return ROWS(6, 4, 2, 3);
+        case 8: return ROWS(8, 4, 2, 3);
+        default: return ROWS(10, 4, 2, 3);
+      }
     }
   }
   switch (plan.mt) {

@@ -159,7 +159,7 @@ template <typename T, int ACT>
 static int dense_rows_run(DenseRowsParams p, const RowsPlan& plan, hipStream_t st) {
   p.op.tiles_n = (int)(((ACT < 0 ? (int64_t)p.op.N : 2 * (int64_t)p.op.N) + 64 * plan.nt - 1) / (64 * plan.nt));
   p.op.ksplit = plan.ksplit;
-  const int rc = rows_dispatch(plan, p.op.tiles_n, [&](auto mt, auto nt, auto wr, auto ns) {
+  const int rc = rows_dispatch<(ACT < 0)>(plan, p.op.tiles_n, [&](auto mt, auto nt, auto wr, auto ns) {
     constexpr int MT = decltype(mt)::value, NT = decltype(nt)::value, WR = decltype(wr)::value, NS = decltype(ns)::value;
     constexpr size_t lds = RowsTile<DenseRowsProduct<T>, MT, NT, WR, NS, (ACT >= 0), true>::LDS;
     auto kern = dense_rows_kernel<T, MT, NT, WR, NS, ACT, (MT <= 8)>;
@@ -189,7 +189,7 @@ extern "C" int64_t aphro_dense_rows_slab_floats(int64_t M, int64_t N, int64_t K,
       !rows_fits(M, N, 2 * K, 2 * lda, 2 * ldw, act >= 0))
     return -1;
   const int64_t rows = act >= 0 ? 2 * N : N;
-  const RowsPlan plan = rows_plan(M, rows, 2 * K);
+  const RowsPlan plan = rows_plan(M, rows, 2 * K, act < 0);
   return plan.ksplit > 1 ? plan.ksplit * M * rows : 0;
 }
 
@@ -204,7 +204,7 @@ extern "C" int64_t aphro_dense_rows_slab_floats(int64_t M, int64_t N, int64_t K,
 extern "C" int aphro_dense_rows_preferred(int64_t M, int64_t N, int64_t K) {
   if (!rows_fits(M, N, 2 * K, 2 * K, 2 * K, false)) return 0;
   if (M <= 64 || K < 2560 || N * K < 40000000) return 1;
-  const RowsPlan plan = rows_plan(M, N, 2 * K);
+  const RowsPlan plan = rows_plan(M, N, 2 * K, true);
   if (plan.ksplit > 1) return 1;
   if (plan.nt == 1) return 0;
   const int64_t tiles = (N + 127) / 128, cus = (tiles + 255) / 256 * 256;
@@ -226,7 +226,7 @@ extern "C" int aphro_dense_rows(void* out, int64_t ldo, const void* x, int64_t l
   p.op.a = (const uint8_t*)x; p.op.w = (const uint8_t*)weight; p.op.M = (int)M; p.op.N = (int)N; p.op.row_bytes = (int)(2 * K);
   p.op.lda = (int)(2 * lda); p.op.ldw = (int)(2 * ldw);
   p.bias = (const uint16_t*)bias; p.out = out; p.slabs = slabs; p.ldo = (int)ldo; p.out_f32 = out_f32;
-  const RowsPlan plan = rows_plan(M, act >= 0 ? 2 * N : N, 2 * K);
+  const RowsPlan plan = rows_plan(M, act >= 0 ? 2 * N : N, 2 * K, act < 0);
   hipStream_t st = (hipStream_t)stream;
 #define DR_ACT(TT) (act < 0 ? dense_rows_run<TT, -1>(p, plan, st) : act == 0 ? dense_rows_run<TT, 0>(p, plan, st) : dense_rows_run<TT, 1>(p, plan, st))
   return dtype == APHRO_F16 ? DR_ACT(Half) : DR_ACT(BFloat);

@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256) void fp8_rows_reduce_kernel(Fp8RowsParams p) {
 
 template <typename T>
 static int fp8_rows_run(const Fp8RowsParams& p, const RowsPlan& plan, hipStream_t st) {
-  const int rc = rows_dispatch(plan, p.op.tiles_n, [&](auto mt, auto nt, auto wr, auto ns) {
+  const int rc = rows_dispatch<false>(plan, p.op.tiles_n, [&](auto mt, auto nt, auto wr, auto ns) {
     constexpr int MT = decltype(mt)::value, NT = decltype(nt)::value, WR = decltype(wr)::value, NS = decltype(ns)::value;
     if constexpr (MT < 3) {
       set_error("fp8_gemm_rows: fewer than 33 rows");

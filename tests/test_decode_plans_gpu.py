@@ -60,3 +60,22 @@ def test_streamed_weights(m, n, k):
     got = ops.dense_rows(x, w)
     # one rounding to the type, and fp32 sums of k products whose terms' sizes add up to about sqrt(k) times the result's
     assert bool(((got.double() - want).abs() <= 2.0 ** -11 * want.abs() + k * 2.0 ** -24 * 4.0).all())
+
+
+# 256 rows of w a workgroup, two rounds of them: every height of x's tile, its first and last row, a ragged last tile; one row past it, a round less
+# full and K below the line, which go the other way
+@pytest.mark.parametrize("m,n,k", [(65, 124936, 2560), (96, 124936, 2560), (97, 131072, 2560), (128, 124936, 2560), (129, 124936, 2560), (160, 124936, 2560),
+                                   (161, 124936, 2560), (96, 110000, 2560), (96, 124936, 2496)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_wide_heads(m, n, k, dtype):
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+    w = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).to(dtype)
+    bias = torch.randn(n, generator=g, device="cuda").to(dtype)
+    u = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    got, biased, wide = ops.dense_rows(x, w), ops.dense_rows(x, w, bias), ops.dense_rows(x, w, f32=True)
+    assert torch.equal(wide, got.float())
+    for part in range(0, n, 32768):                      # one rounding to the type, and fp32 sums of k products
+        want = x.double() @ w[part:part + 32768].double().t()
+        for out, off in ((got, 0.0), (biased, bias[part:part + 32768].double())):
+            assert bool(((out[:, part:part + 32768].double() - (want + off)).abs() <= u * (want + off).abs() + k * 2.0 ** -24 * 4.0).all())
