@@ -202,15 +202,15 @@ class GatedMLP(nn.Module):
 
     def __init__(self, width: int, ff: int, act: int, dtype, prefix: str = "", down: bool = True):
         super().__init__()
-        from .model import QuantLinear
-        self.act, self.ff = act, ff
+        from .model import QuantLinear, plain_call
+        self.act, self.ff, self.plain_call = act, ff, plain_call
         self.gate_up = QuantLinear(width, [ff, ff], None, dtype, prefix=prefix + "gate_up")
         self.down = QuantLinear(ff, [width], None, dtype, prefix=prefix + "down") if down else None
 
     def inner(self, h: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """What the output product reads, into ``out`` [T, ff] (dense rows, any row stride) if given."""
         lin = self.gate_up
-        few = ops.dense_rows(h, lin.weight, act=self.act, out=out) if lin.quant_method is None and lin.bias is None and ops.unhooked(lin) else None
+        few = ops.dense_rows(h, lin.weight, act=self.act, out=out) if self.plain_call(lin) and lin.quant_method is None and lin.bias is None else None
         return mops.act_and_mul(self.gate_up(h), self.act, out) if few is None else few
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:

@@ -26,10 +26,10 @@ from .distributed import (DeferredAllReduce, defer_all_reduce,
                           get_tensor_model_parallel_rank,
                           get_tensor_model_parallel_world_size,
                           tensor_model_parallel_all_reduce)
-from .quantization.awq import AWQConfig
+from .quantization.awq import AWQConfig, CDNA4AWQLinearMethod
 from .quantization.base_config import QuantizationConfig
-from .quantization.fp8 import CompressedTensorsW8A8Fp8Config, Fp8Config
-from .quantization.gptq import GPTQConfig
+from .quantization.fp8 import CDNA4Fp8LinearMethod, CompressedTensorsW8A8Fp8Config, CompressedTensorsW8A8Fp8Method, Fp8Config
+from .quantization.gptq import CDNA4GPTQLinearMethod, GPTQConfig
 
 
 @dataclass
@@ -702,12 +702,12 @@ class LlamaDecoderLayer(nn.Module):
 
     def fused_decode_fp8_rows_ok(self, m: int) -> bool:
         """``fused_decode_fp8_ok``, and beyond its 64 rows whatever the few-rows product leaves as slabs (up to 192)."""
-        return self.fused_decode_fp8_ok(min(m, 64)) and (m <= 64 or self.unhooked() and all(
+        return self.fused_decode_fp8_ok(min(m, 64)) and (m <= 64 or self.plain() and all(
             ops.fp8_gemm_ksplit(m, lin.out_features, lin.in_features) > 0 for lin in self.linears()))
 
-    def unhooked(self) -> bool:
-        """No hook listens to the layer's call or to its projections'."""
-        return ops.unhooked(self) and all(ops.unhooked(lin) for lin in self.linears())
+    def plain(self) -> bool:
+        """The layer's call and its projections' may be done without calling them."""
+        return plain_call(self) and all(plain_call(lin) for lin in self.linears())
 
     def _channel_scale(self, lin) -> torch.Tensor:
         ws = lin.weight_scale
@@ -932,7 +932,7 @@ class LlamaDecoderLayer(nn.Module):
                 ops.fused_add_rms_norm(hidden, residual, next_norm, eps)
             return hidden, residual
         il = self.gate_up_interleaved is not None and not self.gate_up_keep_original
-        if il and hidden.shape[0] > 64 and not self.has_bias and not switch("APHRO_PREFILL_NO_SILU_EPILOGUE") \
+        if il and hidden.shape[0] > 64 and not self.has_bias and plain_call(self.gate_up_proj) and not switch("APHRO_PREFILL_NO_SILU_EPILOGUE") \
                 and not switch("APHRO_WNA16_NO_LARGE"):
             # prompt-sized batches on the interleaved copy: SiluAndMul in the GEMM's epilogue (same bits, no [M, 2 I] round trip)
             qw, qz, sc, zo = self.gate_up_interleaved
@@ -954,7 +954,7 @@ class LlamaDecoderLayer(nn.Module):
     @staticmethod
     def _int4_words(lin: QuantLinear, x: torch.Tensor):
         """lin.fast_params() where a batch beyond the decode kernels may be multiplied without lin's own call, else None."""
-        if lin.bias is None and x.shape[0] > 64 and isinstance(lin.quant_config, (GPTQConfig, AWQConfig)) and ops.unhooked(lin):
+        if x.shape[0] > 64 and plain_call(lin) and lin.bias is None and isinstance(lin.quant_config, (GPTQConfig, AWQConfig)):
             return lin.fast_params()
         return None
 
@@ -977,6 +977,20 @@ class LlamaDecoderLayer(nn.Module):
         if norm is not None:
             ops.fused_add_rms_norm(out, residual, norm, self.cfg.rms_norm_eps)
         return out
+
+
+# What a projection's or a layer's call does as this package wrote it
+_OWN_CALLS = frozenset((QuantLinear.forward, LlamaDecoderLayer.forward, CDNA4GPTQLinearMethod.apply, CDNA4AWQLinearMethod.apply,
+                        CDNA4Fp8LinearMethod.apply, CompressedTensorsW8A8Fp8Method.apply))
+
+
+def plain_call(module: nn.Module) -> bool:
+    """A call of the projection or layer does what this package wrote and nobody listens to it: a kernel that also does what follows may stand in for
+    it.  Not so for a class or a ``forward`` of somebody's own in its place, or a quant method of their own."""
+    if type(module).forward not in _OWN_CALLS or "forward" in vars(module) or type(module).__call__ is not nn.Module.__call__:
+        return False
+    method = getattr(module, "quant_method", None)
+    return (method is None or (type(method).apply in _OWN_CALLS and "apply" not in vars(method))) and ops.unhooked(module)
 
 
 class LlamaForCausalLM(nn.Module):
@@ -1113,7 +1127,7 @@ class LlamaForCausalLM(nn.Module):
                                                              self.norm, self.cfg.rms_norm_eps, want_out=True)
             return out
         if hidden.shape[0] > 64 and all(l.fused_prefill_fp8_ok() for l in self.layers) \
-                and (attn_metadata.num_decode_tokens == 0 or all(l.unhooked() for l in self.layers)):
+                and (attn_metadata.num_decode_tokens == 0 or all(l.plain() for l in self.layers)):
             # FP8 W8A8 batches of prompts, or of more decoded rows than the fused decode step takes: norm + quant and SiluAndMul + quant fused (forward_prefill_fp8)
             residual = torch.empty_like(hidden)
             for i, layer in enumerate(self.layers):
@@ -1122,7 +1136,7 @@ class LlamaForCausalLM(nn.Module):
             ops.fused_add_rms_norm(hidden, residual, self.norm, self.cfg.rms_norm_eps)
             return hidden
         residual = None
-        if all(type(layer).forward is LlamaDecoderLayer.forward and ops.unhooked(layer) for layer in self.layers):
+        if all(plain_call(layer) for layer in self.layers):
             for i, layer in enumerate(self.layers):
                 behind = self.layers[i + 1].input_layernorm if i + 1 < len(self.layers) else self.norm
                 hidden, residual = layer(positions, hidden, residual, kv_caches[i],

@@ -106,3 +106,49 @@ def test_fp8_steps_of_many_decoded_rows(rows):
             handle = module.register_forward_hook(lambda module, args, out: seen.append(module))
             assert torch.equal(step(), plain) and seen.pop() is module and not seen
             handle.remove()
+
+
+@pytest.mark.parametrize("rows", [70, 150])
+@pytest.mark.parametrize("name", ["qkv_proj", "o_proj", "gate_up_proj", "down_proj"])
+def test_a_projection_of_ones_own(rows, name):
+    """A class, or a forward, in a projection's place is called: its result counts."""
+    from aphrodite_engine_amd.quantization.gptq import GPTQConfig
+    with torch.no_grad():
+        M, cfg, model = _llama(GPTQConfig(4, 128, False))
+        if name == "gate_up_proj":                          # (the form whose columns are interleaved for the product's own SiluAndMul)
+            assert model.layers[0].enable_fused_silu(32, keep_original=False)
+        step, calls = _decode(M, cfg, model, rows), []
+        plain, lin = step(), getattr(model.layers[0], name)
+
+        class Own(M.QuantLinear):
+            scale = 1
+
+            def forward(self, x, add_bias=True):
+                calls.append(x.shape[0])
+                return super().forward(x, add_bias) * self.scale
+
+        lin.__class__ = Own
+        assert torch.equal(step(), plain) and calls == [rows]
+        Own.scale = 2
+        assert not torch.equal(step(), plain) and calls == [rows] * 2
+        lin.__class__ = M.QuantLinear
+        lin.forward = lambda x, add_bias=True: (calls.append("instance"), M.QuantLinear.forward(lin, x, add_bias))[1]
+        assert torch.equal(step(), plain) and calls[2:] == ["instance"]
+
+
+@pytest.mark.parametrize("rows", [100, 190])
+def test_an_fp8_projection_of_ones_own(rows):
+    from aphrodite_engine_amd.quantization.fp8 import CompressedTensorsW8A8Fp8Config
+    with torch.no_grad():
+        M, cfg, model = _llama(CompressedTensorsW8A8Fp8Config("channel", is_static_input_scheme=False), dtype=torch.bfloat16)
+        step, calls = _decode(M, cfg, model, rows, dtype=torch.bfloat16), []
+        step()
+
+        class Own(M.QuantLinear):
+            def forward(self, x, add_bias=True):
+                calls.append(x.shape[0])
+                return super().forward(x, add_bias)
+
+        model.layers[1].qkv_proj.__class__ = Own
+        step()
+        assert calls == [rows]
