@@ -712,6 +712,17 @@ struct Fp8LargePlan { int wm, wn, tiles_m, tiles_n, streamk, grid, ksplit, eight
 
 static int cu_count() { return device_cu_count(); }
 
+static int64_t fp8_large_tiles(int64_t M, int64_t N, int wm, int wn) { return (M + 128 * wm - 1) / (128 * wm) * (N / (64 * wn)); }
+static bool fp8_large_slices(int64_t K, int ks) { return K % (ks * 128) == 0 && (ks == 1 || K / ks >= 1024); }
+static size_t fp8_large_images(int wm, int wn) { return (size_t)cu_count() * wm * wn * 32 * 1024; }
+// Stream-K of 128 wm x 64 wn tiles: a tile is cut into five at most, and EVERY workgroup has K tiles of its own -- the owner of a cut tile waits for
+// each that follows it, and one without any would never publish.
+static bool fp8_large_streams(int64_t M, int64_t N, int64_t K, int wn) {
+  const int64_t tiles = fp8_large_tiles(M, N, 2, wn);
+  return device_coresident_cu_count() > 0 && tiles * (K / 128) >= 4 * cu_count() && (wn == 2 ? tiles >= 64 : N % 256 == 0 && K < 2048 && tiles >= 128);
+}
+static bool fp8_large_eight(int64_t N, int64_t K) { return device_coresident_cu_count() > 0 && N % 256 == 0 && K >= 2048; }
+
 // The form by the time it is expected to take (MI355X, ns).  Of the forms measured for 158 sizes (200 to 8192 rows, N 1280 to 37888, K 512 to
 // 18944) the one taken is 0.7 % behind the best on average.  us:
 //  * one workgroup per tile, or per tile and K slice: rounds over the CUs, a last one that is not full 0.68 of a full one and 0.27 by how full it
@@ -725,7 +736,6 @@ static int cu_count() { return device_cu_count(); }
 //    rows 526 / 762 / 762, here 461 / 590 / 722, the last by the order of the tiles; [4096, 14336], 6500 rows 414 / 309).
 static Fp8LargePlan fp8_large_plan(int64_t M, int64_t N, int64_t K) {
   const int cus = cu_count();
-  const bool resident = device_coresident_cu_count() > 0;
   const int64_t T = K / 128;
   Fp8LargePlan best = {};
   int64_t best_ns = -1;
@@ -737,24 +747,22 @@ static Fp8LargePlan fp8_large_plan(int64_t M, int64_t N, int64_t K) {
     best.tiles_n = (int)(N / (64 * wn));
     best.grid = streamk ? cus : best.tiles_m * best.tiles_n;
   };
-  auto tiles_of = [&](int wm, int wn) { return (M + 128 * wm - 1) / (128 * wm) * (N / (64 * wn)); };
+  auto tiles_of = [&](int wm, int wn) { return fp8_large_tiles(M, N, wm, wn); };
   constexpr int64_t STEP[2][2] = {{655, 750}, {775, 1170}}, AROUND[2][2] = {{5750, 7705}, {6550, 8360}}, CROWD[2][2] = {{15, 35}, {27, 30}};
   for (int wm = 1; wm <= 2; ++wm)
     for (int wn = 2; wn <= (N % 256 == 0 ? 4 : 2); wn += 2)
       for (int ks = 1; ks <= 8; ++ks) {
-        if (K % (ks * 128) != 0 || (ks > 1 && K / ks < 1024)) continue;
+        if (!fp8_large_slices(K, ks) || (ks > 1 && (size_t)ks * M * N * 4 > fp8_large_images(2, 4))) continue;
         const int a = wm - 1, b = wn / 4;
         const int64_t wgs = tiles_of(wm, wn) * ks, full = wgs / cus, rest = wgs % cus, busy = full ? cus : rest;
         const int64_t round = AROUND[a][b] + (full ? 120 * wm * wn : 0) + T / ks * STEP[a][b] * (100 * cus + CROWD[a][b] * busy) / (100 * cus);
         const int64_t last = rest == 0 ? 0 : full == 0 ? round : round * (68 * cus + 27 * rest) / (100 * cus);
         offer(wm, wn, 0, ks, 0, 1, full * round + last + (ks > 1 ? 3555 + ks * M * N * 4 / 2985 : 0));
       }
-  // Stream-K: a tile is cut into five at most, and EVERY workgroup has K tiles of its own -- the owner of a cut tile waits for each that follows it,
-  // and one without any would never publish.
-  if (resident && tiles_of(2, 2) >= 64 && tiles_of(2, 2) * T >= 4 * cus) offer(2, 2, 1, 1, 0, 1, 17925 + tiles_of(2, 2) * (T * 1010 + 1215) / cus);
-  if (resident && N % 256 == 0 && K < 2048 && tiles_of(2, 4) >= 128 && tiles_of(2, 4) * T >= 4 * cus)
+  if (fp8_large_streams(M, N, K, 2)) offer(2, 2, 1, 1, 0, 1, 17925 + tiles_of(2, 2) * (T * 1010 + 1215) / cus);
+  if (fp8_large_streams(M, N, K, 4))
     offer(2, 4, 1, 1, 0, 1, 6220 + (tiles_of(2, 4) % cus ? tiles_of(2, 4) * T * 2275 / cus + 13260 : tiles_of(2, 4) * T * 2100 / cus));
-  if (resident && N % 256 == 0 && K >= 2048) {
+  if (fp8_large_eight(N, K)) {
     const int64_t tiles = tiles_of(2, 4), full = tiles / cus, rest = tiles % cus;
     for (int s = 1; s <= 4 && (s == 1 || rest * s <= cus); ++s) {
       const int64_t steps = T * 830 * (100 * cus + 56 * (full ? cus : rest * s)) / (100 * cus), round = 9585 + steps;
@@ -767,11 +775,20 @@ static Fp8LargePlan fp8_large_plan(int64_t M, int64_t N, int64_t K) {
 
 constexpr size_t FP8_LARGE_FLAG_BYTES = 4096;
 
-// Bytes of scratch aphro_scaled_mm_fp8_large needs: stream-K flags + accumulator images, or the fp32 split-K slabs.
-extern "C" size_t aphro_scaled_mm_fp8_large_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  const Fp8LargePlan pl = fp8_large_plan(M, N, K);
-  if (pl.streamk) return FP8_LARGE_FLAG_BYTES + (size_t)pl.grid * pl.wm * pl.wn * 32 * 1024;
+// Bytes of scratch a plan needs: stream-K flags + accumulator images, or the fp32 split-K slabs.
+static size_t fp8_large_scratch(const Fp8LargePlan& pl, int64_t M, int64_t N) {
+  if (pl.streamk) return FP8_LARGE_FLAG_BYTES + fp8_large_images(pl.wm, pl.wn);
   return pl.ksplit > 1 ? (size_t)pl.ksplit * M * N * sizeof(float) : 0;
+}
+// What aphro_scaled_mm_fp8_large needs at most for M rows or fewer: whoever sizes once for the most rows is served below, where the plan may need
+// more than there (4096 x 4096: nothing at 2048 rows, 34 MB at 430).
+extern "C" size_t aphro_scaled_mm_fp8_large_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  size_t most = 0;
+  for (int ks = 2; ks <= 8; ++ks)
+    if (fp8_large_slices(K, ks)) most = std::min((size_t)ks * M * N * sizeof(float), fp8_large_images(2, 4));
+  if (M > 0 && fp8_large_streams(M, N, K, 2)) most = std::max(most, FP8_LARGE_FLAG_BYTES + fp8_large_images(2, 2));
+  if (M > 0 && (fp8_large_streams(M, N, K, 4) || fp8_large_eight(N, K))) most = std::max(most, FP8_LARGE_FLAG_BYTES + fp8_large_images(2, 4));
+  return most;
 }
 
 // out[M, N] = a_scales (.) (a[M, K] . b[N, K]^T) (.) b_scales + bias; e4m3 operands, any M (meant for M > 64).
@@ -788,7 +805,7 @@ extern "C" int aphro_scaled_mm_fp8_large(void* out, const void* a, const void* b
   if (M == 0) return APHRO_OK;
   const Fp8LargePlan pl = fp8_large_plan(M, N, K);
   APHRO_CHECK((int64_t)pl.tiles_m * pl.tiles_n * (K / 128) < 0x7fffffff, "scaled_mm_fp8_large: too many work units");
-  const size_t need = aphro_scaled_mm_fp8_large_workspace_bytes(M, N, K);
+  const size_t need = fp8_large_scratch(pl, M, N);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
     set_error("scaled_mm_fp8_large: workspace %zu < %zu bytes", workspace_bytes, need);
     return APHRO_ERR_WORKSPACE;

@@ -302,7 +302,7 @@ int aphro_scaled_mm_fp8(void* out, const void* a, const void* b,
  * cutlass sm89/sm90 kernels' role (cutlass_w8a8/scaled_mm_c3x.cu, scaled_mm_c2x.cu), which
  * on ROCm the reference hands to torch._scaled_mm (w8a8_utils.py:130-183).
  * N % 128 == 0, K % 128 == 0.  workspace: aphro_scaled_mm_fp8_large_workspace_bytes (split-K
- * slabs for small grids; may be 0). */
+ * slabs or accumulator images; may be 0), which serves every call of M rows or fewer. */
 size_t aphro_scaled_mm_fp8_large_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int aphro_scaled_mm_fp8_large(void* out, const void* a, const void* b,
                               const float* a_scales, const float* b_scales,

@@ -51,3 +51,19 @@ def test_captured_slices_replay():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want) and torch.equal(run(), want)
+
+
+# (rows that the workspace is sized for, rows, columns, k): the form of the most rows needs less than that of the fewer, or nothing
+@pytest.mark.parametrize("most,m,n,k", [(2048, 430, 4096, 4096), (2688, 1281, 6144, 4096), (640, 257, 22016, 4096), (895, 300, 4096, 4096),
+                                        (1552, 1300, 4224, 8192), (5392, 3000, 4224, 4096)])
+def test_a_workspace_for_many_rows_serves_fewer(most, m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randint(-2, 3, (m, k), generator=g, device="cuda").to(torch.float8_e4m3fn)
+    b = torch.randint(-2, 3, (n, k), generator=g, device="cuda").to(torch.float8_e4m3fn)
+    one = torch.ones(1, device="cuda")
+    lib = _lib.lib()
+    out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    ws = torch.full((lib.aphro_scaled_mm_fp8_large_workspace_bytes(most, n, k),), 0x7f, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.aphro_scaled_mm_fp8_large(out.data_ptr(), a.data_ptr(), b.data_ptr(), one.data_ptr(), one.data_ptr(), None, ws.data_ptr(), ws.numel(), m, n, k,
+                                             0, 0, _lib.BF16, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out, (a.float() @ b.float().t()).to(torch.bfloat16))

@@ -39,3 +39,13 @@ def test_a_workspace_for_many_rows_serves_fewer():
             sizes = [lib.aphro_fp8_gemm_workspace_bytes(m, n, k) for m in range(1, 301)]
             assert sizes == sorted(sizes)
             assert all(sizes[m - 1] >= 4 * m * n * lib.aphro_fp8_gemm_rows_ksplit(m, n, k) for m in range(33, 193))
+
+
+def test_a_prompt_workspace_for_many_rows_serves_fewer():
+    from aphrodite_engine_amd import _lib
+    size = _lib.lib().aphro_scaled_mm_fp8_large_workspace_bytes
+    rows = [*range(1, 400), *range(400, 3000, 37), *range(3000, 9000, 211)]
+    for n in (128, 1280, 4096, 4224, 6144, 22016, 28672, 37888):
+        for k in (128, 1024, 2048, 4096, 11008, 14336):
+            sizes = [size(m, n, k) for m in rows]
+            assert sizes == sorted(sizes) and sizes[-1] <= 4096 + 256 * 8 * 32 * 1024
