@@ -151,6 +151,7 @@ SIGNATURES = {
     "aphro_lm_head_argmax": (I, [P, L, P, L, P, L, P, L, L, L, I, P]),
     "aphro_wna16_gemm_rowmajor": (I, [P, L, P, P, P, P, P, Z, L, L, L, L, I, I, I, P]),
     "aphro_convert_fp8": (I, [P, P, L, F, I, I, I, P]),
+    "aphro_paged_attention_runs": (I, [I, I, I, I, I, I]),
     "aphro_paged_attention": (I, [P, P, P, P, P, P, P, I, I, I, I, F, P, P, I, I, I, P,
                                   L, L, L, I, I, F, F, I, P]),
     "aphro_static_scaled_fp8_quant": (I, [P, P, P, L, L, I, P]),

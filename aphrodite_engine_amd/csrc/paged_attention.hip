@@ -1187,6 +1187,26 @@ static int dispatch_pa(const PAParams& p, int num_seqs, int parts, int nw, int h
 
 using namespace aphro;
 
+constexpr int PA_SPLIT_PAIRS = 16, PA_MAX_RUNS = 8;
+// Runs of keys that the v1 form cuts a (sequence, kv head) into, each a workgroup's (split-KV inside the launch): as many as give every CU one (eight
+// waves of 164 registers and more are all that a CU holds), at most eight, about three 32-token pairs a run.  The hand-over takes 2 to 3 us, a pair
+// 0.25 us of an unsplit workgroup: two runs pay from 28 pairs on.  us a layer against unsplit, this plan / up to two workgroups a CU with 8 pairs a
+// run: one sequence of 611 / 1000 tokens -4.7 / -6.2, -2.0 / -5.9; eight of 500 / 1500 / 2500 -0.8 / -6.4 / -14.0, 0 / -2.5 / -10.7; 16 of 600 / 1500
+// 0 / -5.3, 1.8 / -2.3; 24 of 700 0, 5.8.  Below PA_SPLIT_PAIRS more runs would still gain up to 0.9 us (eight sequences of 400 tokens 9.8 and 9.3),
+// but such calls may overlap on several streams: the runs' scratch is one a device.
+static int pa_runs(int64_t groups, int gqa, int head_size, int block_size, int max_seq_len) {
+  if (gqa > 16 || head_size != 128 || (block_size != 16 && block_size != 32) || groups < 1) return 1;
+  const int cus = device_cu_count(), pairs = (max_seq_len + 31) / 32;
+  int want = groups * 2 > cus ? 1 : (int)(cus / groups);
+  want = want > PA_MAX_RUNS ? PA_MAX_RUNS : want;
+  if (want > pairs / 3 + 1) want = pairs / 3 + 1;
+  return pairs < PA_SPLIT_PAIRS || pairs < 8 + 80 / (want * want) ? 1 : want;
+}
+extern "C" int aphro_paged_attention_runs(int num_seqs, int num_heads, int num_kv_heads, int head_size, int block_size, int max_seq_len) {
+  if (num_kv_heads < 1 || num_heads < num_kv_heads) return 1;
+  return pa_runs((int64_t)num_seqs * num_kv_heads, num_heads / num_kv_heads, head_size, block_size, max_seq_len);
+}
+
 // Per-device workspace of the split form: tickets (zero between launches) + the runs' partial results.  Owned by the
 // library (hipMalloc on first use / growth, never during a stream capture: a capturing call that finds it too small runs
 // unsplit).  The decode attention launches of a process are stream-ordered (one compute stream per worker, as in the
@@ -1290,27 +1310,16 @@ static int paged_attention_impl(void* out, void* out_packed, float* exp_sums, fl
     // v1 form: one workgroup per (seq, kv head) walks the whole sequence
     nw = max_seq_len > 256 ? 8 : 4;
     while (nw > 4 && (size_t)nw * (32 + p.nh_lds * head_size) * 4 > 96 * 1024) nw >>= 1;
-    // ... or nsplit workgroups share it (split-KV inside the launch) when (seq, kv head) groups alone leave CUs idle: as many as give every CU one
-    // (eight waves of 164 registers and more are all that a CU holds), at most eight, about three 32-token pairs a run.  The hand-over takes
-    // 2 to 3 us, a pair 0.25 us of an unsplit workgroup, so two runs pay from 28 pairs on, four from 13, eight from 10.  us a layer against
-    // unsplit, this plan / up to two workgroups a CU with 8 pairs a run: one sequence of 330 / 611 / 1000 tokens -1.3 / -4.7 / -6.2, -0.1 / -2.0 /
-    // -5.9; eight of 500 / 1500 / 2500 -0.8 / -6.4 / -14.0, 0 / -2.5 / -10.7; 16 of 600 / 1500 0 / -5.3, 1.8 / -2.3; 24 of 700 0, 5.8.
-    // APHRO_PA_SPLITS=n forces n (1 = off).
-    if (gqa <= 16 && head_size == 128 && (block_size == 16 || block_size == 32)) {
-      const int64_t groups = (int64_t)num_seqs * num_kv_heads;
-      const int cus = device_cu_count(), pairs = (max_seq_len + 31) / 32;
-      int want = groups * 2 > cus ? 1 : (int)(cus / groups);
-      want = want > 8 ? 8 : want;
-      if (want > pairs / 3 + 1) want = pairs / 3 + 1;
-      if (pairs < 8 + 80 / (want * want)) want = 1;
-      if (knobs().pa_splits > 0) want = knobs().pa_splits;
-      want = want > 8 ? 8 : want;
-      if (want > 1) {
-        SplitWs* ws = nullptr;
-        if (split_workspace((size_t)groups, (size_t)groups * want * (16 * head_size + 32), st, &ws)) {
-          p.nsplit = want; p.split_scratch = ws->scratch; p.split_counter = ws->counter;
-          parts = want;
-        }
+    // ... or nsplit workgroups share it (pa_runs).  APHRO_PA_SPLITS=n forces n (1 = off).
+    const int64_t groups = (int64_t)num_seqs * num_kv_heads;
+    int want = pa_runs(groups, gqa, head_size, block_size, max_seq_len);
+    if (gqa <= 16 && head_size == 128 && (block_size == 16 || block_size == 32) && knobs().pa_splits > 0)
+      want = knobs().pa_splits > PA_MAX_RUNS ? PA_MAX_RUNS : knobs().pa_splits;
+    if (want > 1) {
+      SplitWs* ws = nullptr;
+      if (split_workspace((size_t)groups, (size_t)groups * want * (16 * head_size + 32), st, &ws)) {
+        p.nsplit = want; p.split_scratch = ws->scratch; p.split_counter = ws->counter;
+        parts = want;
       }
     }
   } else {

@@ -214,7 +214,13 @@ int aphro_convert_fp8(void* dst, const void* src, int64_t numel, float scale,
  * the v1 form (no scratch); otherwise exp_sums/max_logits [S,Hq,P] fp32 and
  * tmp_out [S,Hq,P,hd] (dtype) with P = ceil(max_seq_len/partition_size) are
  * written exactly as the reference defines them (attention_kernels.cu:350-358)
- * and merged into out.  alibi_slopes fp32 [Hq] or NULL. */
+ * and merged into out.  alibi_slopes fp32 [Hq] or NULL.
+ * Few long sequences in the v1 form and the forms below are cut into runs of keys
+ * (aphro_paged_attention_runs > 1), whose partial results go through ONE scratch a
+ * device that the library owns: two such launches on a device, replays of captured
+ * ones among them, must not run at the same time.  Calls of up to 480 keys, and
+ * those with partition_size > 0, use no scratch of the library's. */
+int aphro_paged_attention_runs(int num_seqs, int num_heads, int num_kv_heads, int head_size, int block_size, int max_seq_len);
 int aphro_paged_attention(void* out, float* exp_sums, float* max_logits,
                           void* tmp_out, const void* query, const void* key_cache,
                           const void* value_cache, int num_seqs, int num_heads,
