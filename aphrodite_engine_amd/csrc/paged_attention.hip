@@ -83,6 +83,7 @@ struct PAParams {
   // output -- no second launch, nobody waits.  Fills the chip when num_seqs x num_kv_heads << CUs (a TP8 shard of
   // Llama-3-70B has ONE kv head per GPU: 64 workgroups at bs 64).
   int nsplit;                    // 0 / 1: off
+  int extra;                     // > 0: the runs are dealt out by the sequences' lengths (pa_take_run), nsplit the most of one sequence
   float* split_scratch;          // [num_seqs * Hkv][nsplit][16 * HD + 32]
   unsigned* split_counter;       // [num_seqs * Hkv], zero between launches (the merging workgroup resets it)
 };
@@ -143,6 +144,80 @@ __device__ __forceinline__ u32x2 fp8x4_to_T(uint32_t w) {
   return r;
 }
 
+// The largest of 64 lanes' numbers >= 0.
+__device__ __forceinline__ int pa_wave_max(int v) {
+#define PA_MAX_STEP(ctrl) v = max(v, __builtin_amdgcn_update_dpp(0, v, ctrl, 0xf, 0xf, false))
+  PA_MAX_STEP(0x111); PA_MAX_STEP(0x112); PA_MAX_STEP(0x114); PA_MAX_STEP(0x118);      // row_shr 1, 2, 4, 8: a row's last lane has the row's
+  PA_MAX_STEP(0x142); PA_MAX_STEP(0x143);                                              // row_bcast 15, 31: lane 63 has all of them
+#undef PA_MAX_STEP
+  return __builtin_amdgcn_readlane(v, 63);
+}
+// Which run of which sequence workgroup y of n + extra takes: every sequence has one, and the longest share the extra ones.  The longest is cut in as
+// many runs (up to eight, if it has PA_SPLIT_PAIRS and more) as let every sequence have runs of that length or less: sequences of one length get one
+// number of them.  Every wave looks at all lengths, Q a lane, by itself.  false: an extra workgroup without a run.
+constexpr int PA_SPLIT_PAIRS = 16, PA_MAX_RUNS = 8, PA_MAX_DEALT = 256;
+struct PaRun { int seq, part, runs, seq_len; };
+template <int Q>
+__device__ __forceinline__ bool pa_take_run(const int32_t* seq_lens, int n, int extra, int y, PaRun& r) {
+  const int lane = threadIdx.x & 63;
+  int len[Q], pairs[Q], most = 0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    len[q] = 64 * q + lane < n ? seq_lens[64 * q + lane] : 0;
+    pairs[q] = (len[q] + 31) >> 5;
+    most = max(most, pairs[q]);
+  }
+  const int longest = pa_wave_max(most);
+  auto longer = [&](int than) {
+    int c = 0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) c += __builtin_popcountll(__ballot(pairs[q] > than));
+    return c;
+  };
+  int size = longest;                                   // pairs of a run at most
+  if (longest >= PA_SPLIT_PAIRS) {
+#pragma unroll
+    for (int j = 2; j <= PA_MAX_RUNS; ++j) {
+      const int t = (int)((unsigned)(longest + j - 1) / (unsigned)j);
+      int more = 0;
+#pragma unroll
+      for (int k = 1; k < j; ++k) more += longer(k * t);
+      if (more > extra || j > longest / 3 + 1) break;
+      if (j > 2 || longest >= 28) size = t;
+    }
+  }
+  r.seq = y;
+  r.part = 0;
+  if (y >= n) {
+    int e = y - n, k = 1;
+    for (; k < PA_MAX_RUNS; ++k) {
+      const int c = longer(k * size);
+      if (e < c) break;
+      e -= c;
+    }
+    if (k == PA_MAX_RUNS) return false;
+    r.part = k;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      uint64_t mask = __ballot(pairs[q] > k * size);
+      const int c = __builtin_popcountll(mask);
+      if (e >= 0 && e < c) {
+        for (int i = 0; i < e; ++i) mask &= mask - 1;
+        r.seq = 64 * q + __builtin_ctzll(mask);
+      }
+      e -= c;
+    }
+  }
+  r.seq_len = 0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if ((r.seq >> 6) == q) r.seq_len = __builtin_amdgcn_readlane(len[q], r.seq & 63);
+  r.runs = 1;
+#pragma unroll
+  for (int k = 1; k < PA_MAX_RUNS; ++k) r.runs += ((r.seq_len + 31) >> 5) > k * size ? 1 : 0;
+  return true;
+}
+
 // KV: 0 = cache holds T, 1 = e4m3, 2 = e5m2.   HD: head size.  BS: block size.
 // ROPE: the fused rotary + cache-write form (a separate instantiation: the plain kernel must not
 // pay for the extra live state -- measured +1.4 us per launch when it was a runtime branch)
@@ -189,11 +264,17 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t*
   const int g = lane >> 4;
   const int c = lane & 15;
   const int kvh = blockIdx.x;
-  const int seq = blockIdx.y;
-  const int part = blockIdx.z;
   const int gqa = p.num_heads / p.num_kv_heads;
-  constexpr bool split = SPLIT;
-  const int seq_len = p.seq_lens[seq];       // (a template parameter: the unsplit instantiations keep their register budget)
+  constexpr bool split = SPLIT;              // (a template parameter: the unsplit instantiations keep their register budget)
+  PaRun run = {(int)blockIdx.y, (int)blockIdx.z, p.nsplit, 0};
+  if (split && p.extra > 0) {
+    const int n = (int)gridDim.y - p.extra;
+    if (!(n <= 64 ? pa_take_run<1>(p.seq_lens, n, p.extra, (int)blockIdx.y, run) : pa_take_run<PA_MAX_DEALT / 64>(p.seq_lens, n, p.extra, (int)blockIdx.y, run)))
+      return;
+  } else {
+    run.seq_len = p.seq_lens[run.seq];
+  }
+  const int seq = run.seq, part = run.part, seq_len = run.seq_len, runs = run.runs;
   // fp8 copy of the output (scaled-slab form only): the scale is fetched HERE, a whole kernel ahead of its use -- at the
   // store it would be a serial global load (and a reload after every byte store, which may alias it)
   float q8_inv = 0.f;
@@ -202,7 +283,7 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t*
     asm volatile("" : "+v"(q8_inv));
   }
   // split form: equal runs of 32-token pairs per workgroup of the (sequence, kv-head) group
-  const int split_pp = split ? (((seq_len + 31) >> 5) + p.nsplit - 1) / p.nsplit : 0;
+  const int split_pp = split ? (((seq_len + 31) >> 5) + runs - 1) / runs : 0;
   const int psz = split ? max(split_pp, 1) * 32 : (p.partition_size > 0 ? p.partition_size : 0x7fffffe0);
   const int pstart = part * psz;
   const bool empty_run = pstart >= seq_len;
@@ -639,7 +720,7 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t*
     __syncthreads();
     constexpr int SLOT = 16 * HD + 32;      // floats per (group, run) slot of split_scratch: O [16][HD], then (m, l) [16]
     float* const grp_scratch = split ? p.split_scratch + ((size_t)seq * p.num_kv_heads + kvh) * p.nsplit * SLOT : nullptr;
-    if (split) {
+    if (split && runs > 1) {
       // ---- this run's unnormalised (O, m, l) -> scratch (write-through), ticket, and only the last arriver goes on -----
       if (!empty_run) {
         float* slot = grp_scratch + (size_t)part * SLOT;
@@ -668,7 +749,7 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t*
       if (threadIdx.x == 0) {
         const unsigned old = __hip_atomic_fetch_add(p.split_counter + (size_t)seq * p.num_kv_heads + kvh, 1u, __ATOMIC_RELAXED,
                                                     __HIP_MEMORY_SCOPE_AGENT);
-        kv_flag = (old == (unsigned)p.nsplit - 1u) ? 2 : 3;
+        kv_flag = (old == (unsigned)runs - 1u) ? 2 : 3;
       }
       __syncthreads();
       if (kv_flag != 2) return;
@@ -679,19 +760,19 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t*
     for (int idx = threadIdx.x; idx < nh * HD; idx += NW * 64) {
       const int h = idx / HD, d = idx - h * HD;
       float M = -1e30f, L = 0.f, acc = 0.f;
-      if (split) {
+      if (split && runs > 1) {
         // merge the runs (all loads of a thread in flight together, one wait): out = sum_z O_z e^(m_z - M) / (sum_z l_z e^(m_z - M) + 1e-6)
         float mz[8], lz[8], az[8];
 #pragma unroll
         for (int q4 = 0; q4 < 2; ++q4) {
           float m4[4] = {-1e30f, -1e30f, -1e30f, -1e30f}, l4[4] = {0.f, 0.f, 0.f, 0.f}, a4[4] = {0.f, 0.f, 0.f, 0.f};
-          if (4 * q4 < p.nsplit) {            // (uniform) runs 4 q4 .. 4 q4 + 3; a run that does not exist reads run 0's slot
+          if (4 * q4 < runs) {                // (uniform) runs 4 q4 .. 4 q4 + 3; a run that does not exist reads run 0's slot
             const float* pm[4];
             const float* pa[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               const int z = 4 * q4 + j;
-              const bool ok = z < p.nsplit && z * psz < seq_len;
+              const bool ok = z < runs && z * psz < seq_len;
               const float* slot = grp_scratch + (size_t)(ok ? z : 0) * SLOT;
               pm[j] = slot + 16 * HD + 2 * h;
               pa[j] = slot + h * HD + d;
@@ -700,7 +781,7 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t*
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               const int z = 4 * q4 + j;
-              if (!(z < p.nsplit && z * psz < seq_len)) { m4[j] = -1e30f; l4[j] = 0.f; a4[j] = 0.f; }
+              if (!(z < runs && z * psz < seq_len)) { m4[j] = -1e30f; l4[j] = 0.f; a4[j] = 0.f; }
             }
           }
 #pragma unroll
@@ -1126,7 +1207,7 @@ __global__ void convert_fp8_kernel(void* __restrict__ dst, const void* __restric
 // ---------------------------------------------------------------------------
 template <typename T, int KV, int HD, int BS, int ROPE = 0>
 static int launch_pa(const PAParams& p, int num_seqs, int parts, int nw, hipStream_t st) {
-  dim3 grid((unsigned)p.num_kv_heads, (unsigned)num_seqs, (unsigned)parts);
+  dim3 grid((unsigned)p.num_kv_heads, (unsigned)(num_seqs + p.extra), (unsigned)parts);
   size_t lds = ((size_t)nw * 16 * 2 + (size_t)nw * p.nh_lds * HD) * sizeof(float);
 #define APHRO_PA_LAUNCH(NWV, SPL)                                                                   \
   {                                                                                                 \
@@ -1187,24 +1268,37 @@ static int dispatch_pa(const PAParams& p, int num_seqs, int parts, int nw, int h
 
 using namespace aphro;
 
-constexpr int PA_SPLIT_PAIRS = 16, PA_MAX_RUNS = 8;
 // Runs of keys that the v1 form cuts a (sequence, kv head) into, each a workgroup's (split-KV inside the launch): as many as give every CU one (eight
 // waves of 164 registers and more are all that a CU holds), at most eight, about three 32-token pairs a run.  The hand-over takes 2 to 3 us, a pair
 // 0.25 us of an unsplit workgroup: two runs pay from 28 pairs on.  us a layer against unsplit, this plan / up to two workgroups a CU with 8 pairs a
 // run: one sequence of 611 / 1000 tokens -4.7 / -6.2, -2.0 / -5.9; eight of 500 / 1500 / 2500 -0.8 / -6.4 / -14.0, 0 / -2.5 / -10.7; 16 of 600 / 1500
 // 0 / -5.3, 1.8 / -2.3; 24 of 700 0, 5.8.  Below PA_SPLIT_PAIRS more runs would still gain up to 0.9 us (eight sequences of 400 tokens 9.8 and 9.3),
 // but such calls may overlap on several streams: the runs' scratch is one a device.
-static int pa_runs(int64_t groups, int gqa, int head_size, int block_size, int max_seq_len) {
-  if (gqa > 16 || head_size != 128 || (block_size != 16 && block_size != 32) || groups < 1) return 1;
+//
+// DEALT from PA_DEAL_PAIRS and a quarter of the CUs (in groups) on: the host knows the longest length only, and under a graph not even that, so the
+// launch has as many workgroups more as CUs are idle (three a kv head at least) and pa_take_run gives them to the longest sequences.  us a layer of an
+// int4 step, 16-bit keys, 8 kv heads, runs by the longest length alone / dealt: one sequence of 8192 keys among 11 / 23 / 30 of 300 53.1 / 23.4, 92.0 /
+// 25.5, 92.8 / 44.2; 10 / 17 of 1000 to 4000 28.9 / 26.3, 55.0 / 41.2, 24 59.9 / 61.6; of one length, 16 / 24 / 31 of 4096 49.3 / 50.2, 69.2 / 70.9, 88.2 /
+// 88.7; 12 / 24 of 600 captured for 8192 14.0 / 15.8, 17.0 / 17.9.  FP8 keys: 10 to 31 of one length +0.3 to +1.1, one of 8192 among 23 66.9 / 22.1.  Below
+// the lines it costs more than it gives: eight of 1500 15.0 / 15.5, 24 of 300 to 1200 21.4 / 23.2.
+struct PaPlan { int runs, extra; };
+constexpr int PA_DEAL_PAIRS = 64;
+static PaPlan pa_plan(int num_seqs, int num_kv_heads, int gqa, int head_size, int block_size, int max_seq_len) {
+  const int64_t groups = (int64_t)num_seqs * num_kv_heads;
+  if (gqa > 16 || head_size != 128 || (block_size != 16 && block_size != 32) || groups < 1) return {1, 0};
   const int cus = device_cu_count(), pairs = (max_seq_len + 31) / 32;
+  if (pairs >= PA_DEAL_PAIRS && groups * 4 > cus && groups < cus && num_seqs <= PA_MAX_DEALT) {
+    const int idle = (int)(cus - groups) / num_kv_heads;
+    return {PA_MAX_RUNS, idle > 3 ? idle : 3};
+  }
   int want = groups * 2 > cus ? 1 : (int)(cus / groups);
   want = want > PA_MAX_RUNS ? PA_MAX_RUNS : want;
   if (want > pairs / 3 + 1) want = pairs / 3 + 1;
-  return pairs < PA_SPLIT_PAIRS || pairs < 8 + 80 / (want * want) ? 1 : want;
+  return {pairs < PA_SPLIT_PAIRS || pairs < 8 + 80 / (want * want) ? 1 : want, 0};
 }
 extern "C" int aphro_paged_attention_runs(int num_seqs, int num_heads, int num_kv_heads, int head_size, int block_size, int max_seq_len) {
   if (num_kv_heads < 1 || num_heads < num_kv_heads) return 1;
-  return pa_runs((int64_t)num_seqs * num_kv_heads, num_heads / num_kv_heads, head_size, block_size, max_seq_len);
+  return pa_plan(num_seqs, num_kv_heads, num_heads / num_kv_heads, head_size, block_size, max_seq_len).runs;
 }
 
 // Per-device workspace of the split form: tickets (zero between launches) + the runs' partial results.  Owned by the
@@ -1217,7 +1311,7 @@ static SplitWs g_split_ws[APHRO_MAX_DEVICES];
 // Buffers are NEVER freed or moved once handed out: a HIP graph captured earlier has their raw pointers baked into its
 // kernel nodes, and the reference's model runner captures many batch sizes and keeps running eager decode beside them
 // (growth after capture used to hipFree what a captured graph still writes to).  The first use allocates for
-// the largest plan the launcher makes by itself (groups x want <= CUs, want <= 8); a forced APHRO_PA_SPLITS plan that
+// the largest plan the launcher makes by itself (groups < CUs, up to eight slots each); a forced APHRO_PA_SPLITS plan that
 // needs more gets NEW, larger buffers and the old ones stay alive for the life of the process.
 static bool split_workspace(size_t groups, size_t floats, hipStream_t st, SplitWs** ws_out) {
   static std::mutex mu;                        // host threads racing on first use / growth
@@ -1235,7 +1329,7 @@ static bool split_workspace(size_t groups, size_t floats, hipStream_t st, SplitW
       ws.groups = g2;
     }
     if (ws.floats < floats) {
-      const size_t bound = (size_t)3 * device_cu_count() * (16 * 128 + 32);
+      const size_t bound = (size_t)PA_MAX_RUNS * device_cu_count() * (16 * 128 + 32);
       const size_t f2 = floats < bound ? bound : floats * 2;
       float* fresh = nullptr;
       if (hipMalloc((void**)&fresh, f2 * sizeof(float)) != hipSuccess) return false;
@@ -1304,22 +1398,22 @@ static int paged_attention_impl(void* out, void* out_packed, float* exp_sums, fl
   const int gqa = num_heads / num_kv_heads;
   p.nh_lds = gqa < 16 ? gqa : 16;
   int parts = 1, nw;
-  p.nsplit = 0; p.split_scratch = nullptr; p.split_counter = nullptr;
+  p.nsplit = 0; p.extra = 0; p.split_scratch = nullptr; p.split_counter = nullptr;
   if (partition_size == 0) {
     p.partition_size = 0; p.max_parts = 0; p.write_direct = 1;
     // v1 form: one workgroup per (seq, kv head) walks the whole sequence
     nw = max_seq_len > 256 ? 8 : 4;
     while (nw > 4 && (size_t)nw * (32 + p.nh_lds * head_size) * 4 > 96 * 1024) nw >>= 1;
-    // ... or nsplit workgroups share it (pa_runs).  APHRO_PA_SPLITS=n forces n (1 = off).
-    const int64_t groups = (int64_t)num_seqs * num_kv_heads;
-    int want = pa_runs(groups, gqa, head_size, block_size, max_seq_len);
+    // ... or nsplit workgroups share it (pa_plan).  APHRO_PA_SPLITS=n forces n (1 = off).
+    const size_t groups = (size_t)num_seqs * num_kv_heads;
+    PaPlan plan = pa_plan(num_seqs, num_kv_heads, gqa, head_size, block_size, max_seq_len);
     if (gqa <= 16 && head_size == 128 && (block_size == 16 || block_size == 32) && knobs().pa_splits > 0)
-      want = knobs().pa_splits > PA_MAX_RUNS ? PA_MAX_RUNS : knobs().pa_splits;
-    if (want > 1) {
+      plan = {knobs().pa_splits > PA_MAX_RUNS ? PA_MAX_RUNS : knobs().pa_splits, 0};
+    if (plan.runs > 1) {
       SplitWs* ws = nullptr;
-      if (split_workspace((size_t)groups, (size_t)groups * want * (16 * head_size + 32), st, &ws)) {
-        p.nsplit = want; p.split_scratch = ws->scratch; p.split_counter = ws->counter;
-        parts = want;
+      if (split_workspace(groups, groups * plan.runs * (16 * head_size + 32), st, &ws)) {
+        p.nsplit = plan.runs; p.extra = plan.extra; p.split_scratch = ws->scratch; p.split_counter = ws->counter;
+        parts = plan.extra > 0 ? 1 : plan.runs;
       }
     }
   } else {
