@@ -1431,6 +1431,28 @@ def sample_top_k_top_p(logits: torch.Tensor, temperature: Optional[torch.Tensor]
 
 
 # --------------------------------------------------------------------------
+# weights that pass the caches once a step, or stay there
+# --------------------------------------------------------------------------
+LAST_LEVEL_CACHE = 256 << 20
+
+
+def mark_weights(model: torch.nn.Module) -> None:
+    """Says of all of a model's weights (``streamed``) whether they come from memory at every step, as in a model larger than the last-level cache.
+    Whoever knows better -- a small model between the steps of a large one -- sets the attribute himself.  A weight without it comes from
+    memory if it is larger than that cache."""
+    weights = dict(model.named_parameters())
+    own_head = "head" in weights or "lm_head" in weights                   # (then a step reads a few rows of the embedding)
+    total = sum(w.numel() * w.element_size() for name, w in weights.items() if not (own_head and name.startswith("embed")))
+    for w in weights.values():
+        w.streamed = total > LAST_LEVEL_CACHE
+
+
+def _weight_flags(weight: torch.Tensor) -> int:
+    streamed = getattr(weight, "streamed", None)
+    return 0 if streamed is None else _lib.WEIGHTS_STREAMED if streamed else _lib.WEIGHTS_CACHED
+
+
+# --------------------------------------------------------------------------
 # FP8 (W8A8, per-token dynamic) decode fast path
 # --------------------------------------------------------------------------
 def fp8_gemm_ksplit(m: int, n: int, k: int) -> int:
@@ -1450,8 +1472,8 @@ def scaled_mm_fp8_slabs(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     if ks <= 0:
         raise RuntimeError(f"scaled_mm_fp8_slabs: shape M={m} N={n} K={k} not served")
     slabs = torch.empty((ks, m, n), dtype=torch.float32, device=a.device)
-    check(lib.aphro_scaled_mm_fp8_slabs(a.data_ptr(), b.data_ptr(), slabs.data_ptr(), slabs.numel() * 4,
-                                        m, n, k, _stream()), "scaled_mm_fp8_slabs")
+    check(lib.aphro_scaled_mm_fp8_slabs_flags(a.data_ptr(), b.data_ptr(), slabs.data_ptr(), slabs.numel() * 4,
+                                              m, n, k, _weight_flags(b), _stream()), "scaled_mm_fp8_slabs")
     return slabs
 
 
@@ -1657,7 +1679,7 @@ def fp8_gemm_silu_quant(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor,
         raise RuntimeError("fp8_gemm_silu_quant: bias must be [N] in the activation dtype")
     check(_lib.lib().aphro_fp8_gemm_stream_silu_quant(
         a.data_ptr(), k, b.data_ptr(), sa.data_ptr(), sb.data_ptr(), _ptr(bias), q.data_ptr(), static_scale.data_ptr(),
-        m, n, k, 1 if sa.numel() > 1 else 0, 1 if sb.numel() > 1 else 0, _dt_of(dtype), _stream()), "fp8_gemm_silu_quant")
+        m, n, k, 1 if sa.numel() > 1 else 0, 1 if sb.numel() > 1 else 0, _dt_of(dtype) | _weight_flags(b), _stream()), "fp8_gemm_silu_quant")
     return q
 
 
@@ -1871,7 +1893,7 @@ def dense_rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
         return None
     slabs = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
     check(_lib.lib().aphro_dense_rows(out.data_ptr(), max(out.stride(0), N), xp, lda, wp, ldw, bp, None if slabs is None else slabs.data_ptr(), need,
-                                      M, N, K, act, int(f32), dt, _raw_stream(dev)), "dense_rows")
+                                      M, N, K, act, int(f32), dt | _weight_flags(weight), _raw_stream(dev)), "dense_rows")
     return out
 
 
@@ -1918,7 +1940,7 @@ def lm_head_argmax(hidden: torch.Tensor, weight: torch.Tensor, vocab_size: Optio
         raise RuntimeError("lm_head_argmax: logits_out must be [M, >= V] of the activation dtype with contiguous rows")
     check(_lib.lib().aphro_lm_head_argmax(hidden.data_ptr(), hidden.stride(0), weight.data_ptr(), weight.stride(0),
                                           _ptr(logits_out), logits_out.stride(0) if logits_out is not None else 0,
-                                          out.data_ptr(), m, k, v, _dt(hidden), _stream()), "lm_head_argmax")
+                                          out.data_ptr(), m, k, v, _dt(hidden) | _weight_flags(weight), _stream()), "lm_head_argmax")
     return out
 
 
@@ -2333,7 +2355,7 @@ def cutlass_scaled_mm(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor,
         check(lib.aphro_scaled_mm_fp8(
             out[m0:].data_ptr(), a[m0:].data_ptr(), b.data_ptr(),
             sa_blk.data_ptr(), sb.data_ptr(), _ptr(bias), ws.data_ptr(),
-            ws.numel(), rows, n, k, a_tok, b_ch, odt, _stream()),
+            ws.numel(), rows, n, k, a_tok, b_ch, odt | _weight_flags(b), _stream()),
             "cutlass_scaled_mm")
     return out
 

@@ -34,6 +34,7 @@ SIGNATURES = {
                                               L, L, I, I, F, F, P]),
     "aphro_fp8_gemm_ksplit": (I, [L, L, L]),
     "aphro_scaled_mm_fp8_slabs": (I, [P, P, P, Z, L, L, L, P]),
+    "aphro_scaled_mm_fp8_slabs_flags": (I, [P, P, P, Z, L, L, L, I, P]),
     "aphro_fused_add_rms_norm_quant_fp8": (I, [P, P, I, P, P, I, I, P, I, P, F, P, P, P, L, I, I, P]),
     "aphro_silu_and_mul_quant_fp8": (I, [P, P, P, P, L, I, I, P]),
     "aphro_fused_add_rms_norm_quant_fp8_static": (I, [P, P, I, P, P, I, I, P, I, P, F, P, P, P, L, I, I, P, P]),
@@ -244,6 +245,7 @@ MIXERS_SIGNATURES = {
 
 OK = 0
 F16, BF16, F32 = 0, 1, 2
+WEIGHTS_STREAMED, WEIGHTS_CACHED = 0x100, 0x200          # or-ed into a dtype
 KV_AUTO, KV_FP8_E4M3, KV_FP8_E5M2 = 0, 1, 2
 
 _lib = None

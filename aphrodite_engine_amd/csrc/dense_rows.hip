@@ -146,25 +146,26 @@ __global__ __launch_bounds__(256) void dense_rows_reduce_kernel(DenseRowsParams 
   dr_store<T>(p, m, col, v);
 }
 
-// Whether w takes the non-temporal hint (RowsTile) above 48 rows of x, up to which it always does: with 40 steps of 64 k a slice and more, up to
+// Whether a w that passes the caches once (weights_streamed) takes the non-temporal hint (RowsTile) above 48 rows of x, up to which it does: with 40 steps of 64 k a slice and more, up to
 // 128 rows.  us without / with it, f16, weights from memory: [128256, 4096], 16 / 64 / 96 / 192 rows 187 / 198 / 212 / 254 and 167 / 192 / 211 / 253;
 // [28672, 4096], 16 / 64 / 128 / 150 rows 50.5 / 51.4 / 57.9 / 59.5 and 46.7 / 47.9 / 56.8 / 60.1; [10240, 8192], 42 steps, 32 / 65 / 128 rows 38.1 /
 // 37.9 / 42.6 and 35.2 / 35.5 / 41.8.  Short slices lose with many rows: [4096, 14336], 28 steps, 16 / 48 / 96 / 128 rows 24.9 / 26.8 / 30.4 / 33.2
 // and 22.1 / 25.3 / 32.2 / 35.6; [6144, 4096], 12 steps, 16 / 64 / 128 rows 14.3 / 17.6 / 20.5 and 13.5 / 19.0 / 23.4.  (FP8, half the bytes of x a step,
-// is ahead or level with it everywhere: fp8_gemm_rows.hip.)  A w that stays in the 256 MB last-level cache from call to call is slower with it
-// ([32000, 2048] alone, 16 rows: 20.2 and 25.6; twelve of [2048, 2048], 101 MB: 8.1 and 7.7); a model's weights do not stay there.
+// is ahead or level with it everywhere: fp8_gemm_rows.hip.)  Weights that stay in the last-level cache from call to call, 180 to 260 MB in all, without /
+// with it, 16 and 48 rows: [2048, 2048] 8.1 / 8.1 and 9.5 / 9.5, [4096, 4096] 9.8 / 10.8 and 10.9 / 12.7, [11008, 4096] 15.4 / 19.8 and 20.5 / 24.7,
+// [32000, 2048] 21.1 / 27.1 and 22.2 / 28.7; one more of the latter, from memory, 30.6 / 27.7 and 31.8 / 29.9.  FP8 [28672, 4096], 64 rows 20.7 / 29.2.
 inline bool dense_rows_stream(const RowsOperands& op) { return op.M <= 48 || (op.M <= 128 && op.row_bytes >= 40 * 128 * op.ksplit); }
 
 template <typename T, int ACT>
-static int dense_rows_run(DenseRowsParams p, const RowsPlan& plan, hipStream_t st) {
+static int dense_rows_run(DenseRowsParams p, const RowsPlan& plan, bool streamed, hipStream_t st) {
   p.op.tiles_n = (int)(((ACT < 0 ? (int64_t)p.op.N : 2 * (int64_t)p.op.N) + 64 * plan.nt - 1) / (64 * plan.nt));
   p.op.ksplit = plan.ksplit;
   const int rc = rows_dispatch<(ACT < 0)>(plan, p.op.tiles_n, [&](auto mt, auto nt, auto wr, auto ns) {
     constexpr int MT = decltype(mt)::value, NT = decltype(nt)::value, WR = decltype(wr)::value, NS = decltype(ns)::value;
     constexpr size_t lds = RowsTile<DenseRowsProduct<T>, MT, NT, WR, NS, (ACT >= 0), true>::LDS;
-    auto kern = dense_rows_kernel<T, MT, NT, WR, NS, ACT, (MT <= 8)>;
-    if constexpr (MT >= 4 && MT <= 8) {
-      if (!dense_rows_stream(p.op)) kern = dense_rows_kernel<T, MT, NT, WR, NS, ACT, false>;
+    auto kern = dense_rows_kernel<T, MT, NT, WR, NS, ACT, false>;
+    if constexpr (MT <= 8) {
+      if (streamed && dense_rows_stream(p.op)) kern = dense_rows_kernel<T, MT, NT, WR, NS, ACT, true>;
     }
     if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
       set_error("dense_rows: cannot raise the dynamic LDS limit to %zu", lds);
@@ -214,6 +215,7 @@ extern "C" int aphro_dense_rows_preferred(int64_t M, int64_t N, int64_t K) {
 extern "C" int aphro_dense_rows(void* out, int64_t ldo, const void* x, int64_t lda, const void* weight, int64_t ldw, const void* bias,
                                 float* slabs, int64_t slab_floats, int64_t M, int64_t N, int64_t K, int act, int out_f32, int dtype,
                                 void* stream) {
+  const bool streamed = weights_streamed(weights_flags(dtype), (size_t)(act >= 0 ? 2 * N : N) * K * 2);
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "dense_rows: dtype must be f16 or bf16");
   const int64_t need = aphro_dense_rows_slab_floats(M, N, K, lda, ldw, act);
   APHRO_CHECK(need >= 0, "dense_rows: M=%ld N=%ld K=%ld lda=%ld ldw=%ld is not served", (long)M, (long)N, (long)K, (long)lda, (long)ldw);
@@ -228,7 +230,7 @@ extern "C" int aphro_dense_rows(void* out, int64_t ldo, const void* x, int64_t l
   p.bias = (const uint16_t*)bias; p.out = out; p.slabs = slabs; p.ldo = (int)ldo; p.out_f32 = out_f32;
   const RowsPlan plan = rows_plan(M, act >= 0 ? 2 * N : N, 2 * K, act < 0);
   hipStream_t st = (hipStream_t)stream;
-#define DR_ACT(TT) (act < 0 ? dense_rows_run<TT, -1>(p, plan, st) : act == 0 ? dense_rows_run<TT, 0>(p, plan, st) : dense_rows_run<TT, 1>(p, plan, st))
+#define DR_ACT(TT) (act < 0 ? dense_rows_run<TT, -1>(p, plan, streamed, st) : act == 0 ? dense_rows_run<TT, 0>(p, plan, streamed, st) : dense_rows_run<TT, 1>(p, plan, streamed, st))
   return dtype == APHRO_F16 ? DR_ACT(Half) : DR_ACT(BFloat);
 #undef DR_ACT
 }

@@ -406,13 +406,14 @@ static int run_fp8(Fp8GemmParams p, const Fp8Plan& pl, hipStream_t st) {
 
 static int fp8_gemm_common(Fp8GemmParams p, bool a8, int dtype, void* workspace, size_t workspace_bytes,
                            hipStream_t st) {
+  const int flags = a8 ? weights_flags(dtype) : 0;
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "fp8 gemm: output dtype must be f16 or bf16");
   APHRO_CHECK(p.K % 128 == 0, "fp8 gemm: K=%d must be a multiple of 128", p.K);
   APHRO_CHECK(p.N % 16 == 0, "fp8 gemm: N=%d must be a multiple of 16", p.N);
   // W8A8 from 33 rows on: one pass over the weight (fp8_gemm_rows.hip)
   if (a8 && p.lda == p.K && aphro_fp8_gemm_rows_ksplit(p.M, p.N, p.K) > 0 && ((uintptr_t)p.c % 8) == 0 && ((uintptr_t)workspace % 16) == 0)
     return aphro_fp8_gemm_rows(p.a, p.w, p.a_scales, p.b_scales, p.bias, p.force_partial ? nullptr : p.c, (float*)workspace, workspace_bytes,
-                               p.M, p.N, p.K, p.a_per_token, p.b_per_channel, dtype, (void*)st);
+                               p.M, p.N, p.K, p.a_per_token, p.b_per_channel, dtype | flags, (void*)st);
   APHRO_CHECK(p.M <= 64, "fp8 gemm: M=%d exceeds 64 rows per call", p.M);
   if (p.M == 0) return APHRO_OK;
   // W8A8 at <= 32 rows: the LDS-DMA streaming kernel (fp8_gemm_stream.hip) where it tiles the shape -- directly to `c` when
@@ -429,7 +430,7 @@ static int fp8_gemm_common(Fp8GemmParams p, bool a8, int dtype, void* workspace,
       }
       return aphro_fp8_gemm_stream(p.a, p.lda, p.w, p.a_scales, p.b_scales, p.bias, p.force_partial ? nullptr : p.c,
                                    p.force_partial ? (float*)workspace : nullptr, workspace_bytes, p.M, p.N, p.K,
-                                   p.a_per_token, p.b_per_channel, dtype, (void*)st);
+                                   p.a_per_token, p.b_per_channel, dtype | flags, (void*)st);
     }
   }
   Fp8Plan pl = make_fp8_plan(p.M, p.N, p.K, a8);
@@ -488,12 +489,17 @@ extern "C" int aphro_fp8_gemm_ksplit(int64_t M, int64_t N, int64_t K) {
 
 extern "C" int aphro_scaled_mm_fp8_slabs(const void* a, const void* b, float* partials, size_t partial_bytes,
                                          int64_t M, int64_t N, int64_t K, void* stream) {
+  return aphro_scaled_mm_fp8_slabs_flags(a, b, partials, partial_bytes, M, N, K, 0, stream);
+}
+extern "C" int aphro_scaled_mm_fp8_slabs_flags(const void* a, const void* b, float* partials, size_t partial_bytes,
+                                               int64_t M, int64_t N, int64_t K, int flags, void* stream) {
+  APHRO_CHECK((flags & ~(APHRO_WEIGHTS_STREAMED | APHRO_WEIGHTS_CACHED)) == 0, "scaled_mm: flags=%d", flags);
   APHRO_CHECK(((uintptr_t)a % 16) == 0 && ((uintptr_t)b % 16) == 0, "scaled_mm: operands must be 16-byte aligned");
   Fp8GemmParams p;
   p.a = a; p.w = (const uint8_t*)b; p.a_scales = nullptr; p.b_scales = nullptr; p.bias = nullptr; p.c = nullptr;
   p.M = (int)M; p.N = (int)N; p.K = (int)K; p.lda = (int)K;
   p.a_per_token = 0; p.b_per_channel = 0; p.force_partial = 1;
-  return fp8_gemm_common(p, true, APHRO_F16, partials, partial_bytes, (hipStream_t)stream);
+  return fp8_gemm_common(p, true, APHRO_F16 | flags, partials, partial_bytes, (hipStream_t)stream);
 }
 
 extern "C" int aphro_fp8_w8a16_gemm(void* out, const void* a, const void* w, const float* w_scales,

@@ -8,7 +8,7 @@
 //   [4096, 14336]   18.7 / 22.2 / 27.1  (36.8 / 25.3 / 30.4)      13.3 / 17.0 / 21.1
 //   [6144, 4096]    14.4 / 17.9 / 19.8  (17.0 / 18.8 / 22.9)       9.2 / 12.4 / 14.5
 //   [4096, 4096]    11.1 / 14.8 / 18.9  (12.7 / 19.2 / 22.8)       7.0 /  9.1 / 10.4
-// (raw slabs: with the non-temporal hint on w's loads; without it 29.5 / 32.3 / 36.6, 14.0 / 17.5 / 21.3, 9.3 / 12.3 / 14.6 and 7.1 / 9.3 / 10.4)
+// (raw slabs: with the non-temporal hint on w's loads, as where weights_streamed; without it 29.5 / 32.3 / 36.6, 14.0 / 17.5 / 21.3, 9.3 / 12.3 / 14.6 and 7.1 / 9.3 / 10.4)
 // (a result in 16 bits over several K slices pays a second launch; the same bits as before at every shape measured)
 #include "dense_rows.h"
 
@@ -78,10 +78,10 @@ __device__ __forceinline__ void fr_store(const Fp8RowsParams& p, int m, int n, f
   *reinterpret_cast<u16x4*>(p.out + (size_t)m * p.op.N + n) = o;
 }
 
-template <typename T, int MT, int NT, int WR, int NS>
+template <typename T, int MT, int NT, int WR, int NS, bool STREAM>
 __global__ __launch_bounds__(256 * WR) void fp8_gemm_rows_kernel(Fp8RowsParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  RowsTile<Fp8RowsProduct, MT, NT, WR, NS, false, true> tile;
+  RowsTile<Fp8RowsProduct, MT, NT, WR, NS, false, STREAM> tile;
   tile.run(p.op, smem);
   constexpr int MTW = MT / WR;
   const int m0 = tile.wr * MTW * 16 + tile.c, n0 = tile.n0 + 16 * tile.wc + 4 * tile.g, M = p.op.M, N = p.op.N;
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void fp8_rows_reduce_kernel(Fp8RowsParams p) {
 }
 
 template <typename T>
-static int fp8_rows_run(const Fp8RowsParams& p, const RowsPlan& plan, hipStream_t st) {
+static int fp8_rows_run(const Fp8RowsParams& p, const RowsPlan& plan, bool streamed, hipStream_t st) {
   const int rc = rows_dispatch<false>(plan, p.op.tiles_n, [&](auto mt, auto nt, auto wr, auto ns) {
     constexpr int MT = decltype(mt)::value, NT = decltype(nt)::value, WR = decltype(wr)::value, NS = decltype(ns)::value;
     if constexpr (MT < 3) {
@@ -132,7 +132,7 @@ static int fp8_rows_run(const Fp8RowsParams& p, const RowsPlan& plan, hipStream_
       return (int)APHRO_ERR_INVALID;
     } else {
       constexpr size_t lds = RowsTile<Fp8RowsProduct, MT, NT, WR, NS, false, true>::LDS;
-      auto kern = fp8_gemm_rows_kernel<T, MT, NT, WR, NS>;
+      auto kern = streamed ? fp8_gemm_rows_kernel<T, MT, NT, WR, NS, true> : fp8_gemm_rows_kernel<T, MT, NT, WR, NS, false>;
       if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
         set_error("fp8_gemm_rows: cannot raise the dynamic LDS limit to %zu", lds);
         return (int)APHRO_ERR_LAUNCH;
@@ -164,6 +164,7 @@ extern "C" int aphro_fp8_gemm_rows_preferred(int64_t M, int64_t N, int64_t K) { 
 extern "C" int aphro_fp8_gemm_rows(const void* a, const void* w, const float* a_scales, const float* b_scales, const void* bias, void* out,
                                    float* slabs, size_t slabs_bytes, int64_t M, int64_t N, int64_t K, int a_scale_per_token,
                                    int b_scale_per_channel, int dtype, void* stream) {
+  const bool streamed = weights_streamed(weights_flags(dtype), (size_t)N * K);
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "fp8_gemm_rows: output dtype must be f16 or bf16");
   const int split = aphro_fp8_gemm_rows_ksplit(M, N, K);
   APHRO_CHECK(split > 0, "fp8_gemm_rows: M=%ld N=%ld K=%ld is not served", (long)M, (long)N, (long)K);
@@ -185,5 +186,5 @@ extern "C" int aphro_fp8_gemm_rows(const void* a, const void* w, const float* a_
   p.op.ksplit = plan.ksplit;
   p.a_scales = a_scales; p.b_scales = b_scales; p.bias = (const uint16_t*)bias; p.out = (uint16_t*)out; p.slabs = slabs;
   p.a_per_token = a_scale_per_token; p.b_per_channel = b_scale_per_channel;
-  return dtype == APHRO_F16 ? fp8_rows_run<Half>(p, plan, (hipStream_t)stream) : fp8_rows_run<BFloat>(p, plan, (hipStream_t)stream);
+  return dtype == APHRO_F16 ? fp8_rows_run<Half>(p, plan, streamed, (hipStream_t)stream) : fp8_rows_run<BFloat>(p, plan, streamed, (hipStream_t)stream);
 }

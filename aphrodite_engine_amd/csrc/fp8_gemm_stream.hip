@@ -10,7 +10,7 @@
 //     chunks XOR-swizzled by the row pair so that the 8-byte B-fragment reads are bank-conflict free; a ring of 8 segments
 //     (16 KiB) per wave = 128 KiB in flight per CU, no register touched on the way in (fp8_gemm_fast_kernel holds 2 macro
 //     steps = 16 KiB per WAVE GROUP in registers and measures 0.43 of the roofline on the gate_up matrix);
-//     The loads carry the non-temporal hint (SILU form, us without / with it, [28672, 4096] 1 / 16 / 32 rows 24.7 / 27.3 /
+//     The loads carry the non-temporal hint where the weights pass the caches once (weights_streamed; SILU form, us without / with it, [28672, 4096] 1 / 16 / 32 rows 24.7 / 27.3 /
 //     30.5 and 22.6 / 25.3 / 28.6; [22016, 4096] 21.1 / 23.5 / 26.7 and 19.1 / 21.8 / 25.2);
 //   * hand-counted vmcnt waits (hipcc does not order a ds_read after the LDS-DMA that fills it), B-fragment reads in inline
 //     asm, an LDS-only workgroup barrier per tile (see lm_head.hip);
@@ -56,7 +56,7 @@ __device__ __forceinline__ void f8s_static_for(F&& f) {
 __device__ __forceinline__ void f8s_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // KS: 128-k segments per wave and K slice (K = gridDim.y x 8 waves x KS x 128).  MT: 16-token tiles.
-template <typename T, int MT, int KS, bool SILU = false>
+template <typename T, int MT, int KS, bool STREAM, bool SILU = false>
 __global__ __launch_bounds__(512, 1) void fp8_gemm_stream_kernel(const uint8_t* w, const uint8_t* a, int M, int N, int K,
                                                                  int lda, int tiles, Fp8StreamParams p_in) {
   // (leading scalars: preloaded into SGPRs, Makefile -amdgpu-kernarg-preload-count; p_in carries the rest)
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_stream_kernel(const uint8_t* 
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
       const int vo = voff_w[it];
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (f8s_lds_ptr)(dst + it * 1024), 16, vo, so, 0, 2);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (f8s_lds_ptr)(dst + it * 1024), 16, vo, so, 0, STREAM ? 2 : 0);
     }
   };
   const int tok = tid >> 4, col = tid & 15;
@@ -236,6 +236,7 @@ extern "C" int aphro_fp8_gemm_stream_ksplit(int64_t M, int64_t N, int64_t K) {
 extern "C" int aphro_fp8_gemm_stream(const void* a, int64_t lda, const void* w, const float* a_scales, const float* b_scales,
                                      const void* bias, void* out, float* slabs, size_t slabs_bytes, int64_t M, int64_t N,
                                      int64_t K, int a_scale_per_token, int b_scale_per_channel, int dtype, void* stream) {
+  const bool streamed = weights_streamed(weights_flags(dtype), (size_t)N * K);
   const int split = aphro_fp8_gemm_stream_ksplit(M, N, K);
   APHRO_CHECK(split > 0, "fp8_gemm_stream: M=%ld N=%ld K=%ld is not served", (long)M, (long)N, (long)K);
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "fp8_gemm_stream: output dtype must be f16 or bf16");
@@ -256,7 +257,7 @@ extern "C" int aphro_fp8_gemm_stream(const void* a, int64_t lda, const void* w, 
   dim3 grid((unsigned)gx, (unsigned)split);
 #define L(TT, MTV, KSV)                                                                                            \
   {                                                                                                                \
-    auto kern = fp8_gemm_stream_kernel<TT, MTV, KSV>;                                                              \
+    auto kern = streamed ? fp8_gemm_stream_kernel<TT, MTV, KSV, true> : fp8_gemm_stream_kernel<TT, MTV, KSV, false>; \
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) { \
       set_error("fp8_gemm_stream: cannot raise the dynamic LDS limit to %zu", lds);                                \
       return APHRO_ERR_LAUNCH;                                                                                     \
@@ -294,6 +295,7 @@ extern "C" int aphro_fp8_gemm_stream_silu_quant(const void* a, int64_t lda, cons
                                                 const float* q_scale, int64_t M, int64_t N, int64_t K,
                                                 int a_scale_per_token, int b_scale_per_channel, int dtype,
                                                 void* stream) {
+  const bool streamed = weights_streamed(weights_flags(dtype), (size_t)N * K);
   APHRO_CHECK(aphro_fp8_gemm_stream_silu_supported(M, N, K), "fp8_gemm_stream_silu_quant: M=%ld N=%ld K=%ld is not served",
               (long)M, (long)N, (long)K);
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "fp8_gemm_stream_silu_quant: dtype must be f16 or bf16");
@@ -311,7 +313,7 @@ extern "C" int aphro_fp8_gemm_stream_silu_quant(const void* a, int64_t lda, cons
   dim3 grid((unsigned)gx, 1);
 #define L(TT, MTV, KSV)                                                                                            \
   {                                                                                                                \
-    auto kern = fp8_gemm_stream_kernel<TT, MTV, KSV, true>;                                                        \
+    auto kern = streamed ? fp8_gemm_stream_kernel<TT, MTV, KSV, true, true> : fp8_gemm_stream_kernel<TT, MTV, KSV, false, true>; \
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) { \
       set_error("fp8_gemm_stream_silu_quant: cannot raise the dynamic LDS limit to %zu", lds);                     \
       return APHRO_ERR_LAUNCH;                                                                                     \

@@ -12,7 +12,7 @@
 //     ring holds KS 128-k segments = one tile ahead of the one it computes: 16 KiB in flight per wave, 128 KiB per CU.
 //     hipcc does not order a ds_read after the LDS-DMA that fills its source: the waits are written by hand (loads return
 //     in order; stores between them can only make a wait return earlier for the stores' own sake -- see below).
-//     They carry the non-temporal hint, as they pass the caches once: us without / with it, f16, weights from memory,
+//     They carry the non-temporal hint where the weights pass the caches once (weights_streamed): us without / with it, f16, from memory,
 //     [128256, 4096] 1 / 32 rows 179 / 178 and 169 / 171, [151936, 2048] 117 / 116 and 105, [32000, 2048] 32.6 / 34.2 and
 //     31.0 / 33.1 (a plain read of the first by one workgroup per CU: 172 and 154).
 //   * K reduction over the waves through LDS once per tile; the thread that owns (token, column) of the tile rounds the sum
@@ -64,7 +64,7 @@ __device__ __forceinline__ void lmh_lds_barrier() { asm volatile("s_waitcnt lgkm
 __device__ __forceinline__ bool lmh_better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
 
 // KS: 128-k segments per wave (K = 8 waves x KS x 128).  MT: 16-token tiles (M <= 16 MT).
-template <typename T, int MT, int KS>
+template <typename T, int MT, int KS, bool STREAM>
 __global__ __launch_bounds__(512, 1) void lm_head_argmax_kernel(LmHeadParams p) {
   constexpr int NWV = 8;
   constexpr int SEGB = 16 * 256;                    // one staged segment: [16 rows][16 chunks of 8 k]
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(512, 1) void lm_head_argmax_kernel(LmHeadParams p) 
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       const int vo = voff_w[it];                    // (local copy: hipcc host-stub bug, see wna16_gemm_large.hip)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lmh_lds_ptr)(ring + s * SEGB + it * 1024), 16, vo, so, 0, 2);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lmh_lds_ptr)(ring + s * SEGB + it * 1024), 16, vo, so, 0, STREAM ? 2 : 0);
     }
   };
 
@@ -270,6 +270,7 @@ extern "C" int aphro_lm_head_argmax(const void* hidden, int64_t lda, const void*
                                     int64_t ldl, int64_t* out_ids, int64_t M, int64_t K, int64_t V, int dtype,
                                     void* stream) {
   hipStream_t st = (hipStream_t)stream;
+  const bool streamed = weights_streamed(weights_flags(dtype), (size_t)V * ldw * 2);
   APHRO_CHECK(aphro_lm_head_argmax_supported(M, K, V, ldw, dtype), "lm_head_argmax: M=%ld K=%ld V=%ld ldw=%ld dtype=%d is not served",
               (long)M, (long)K, (long)V, (long)ldw, dtype);
   APHRO_CHECK(((uintptr_t)hidden % 16) == 0 && ((uintptr_t)weight % 16) == 0 && lda % 8 == 0 && lda >= K && out_ids != nullptr,
@@ -292,7 +293,7 @@ extern "C" int aphro_lm_head_argmax(const void* hidden, int64_t lda, const void*
   const size_t lds = (size_t)8 * ks * 4096 + (size_t)8 * 16 * mt * 17 * sizeof(float);
 #define LMH(TT, MTV, KSV)                                                                                          \
   {                                                                                                                \
-    auto kern = lm_head_argmax_kernel<TT, MTV, KSV>;                                                               \
+    auto kern = streamed ? lm_head_argmax_kernel<TT, MTV, KSV, true> : lm_head_argmax_kernel<TT, MTV, KSV, false>; \
     if (lds > 64 * 1024 &&                                                                                         \
         hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) { \
       set_error("lm_head_argmax: cannot raise the dynamic LDS limit to %zu", lds);                                 \

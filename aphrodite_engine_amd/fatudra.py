@@ -204,6 +204,7 @@ class FatudraForCausalLM(nn.Module):
     def finalize(self):
         for layer in self.layers:
             layer.mix.finalize()
+        ops.mark_weights(self)
         return self
 
     @torch.no_grad()

@@ -115,6 +115,7 @@ class FekotarForCausalLM(nn.Module):
     def finalize(self):
         for layer in self.layers:
             layer.mix.finalize()
+        ops.mark_weights(self)
         return self
 
     @torch.no_grad()

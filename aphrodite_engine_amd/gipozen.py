@@ -154,6 +154,7 @@ class GipozenForCausalLM(nn.Module):
                 layer.mlp.finalize()
             layer.gain1, layer.gain2 = float(layer.norm1), float(layer.norm2)
         self.final_gain = float(self.final_norm)
+        ops.mark_weights(self)
         return self
 
     @torch.no_grad()

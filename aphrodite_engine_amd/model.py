@@ -1061,6 +1061,7 @@ class LlamaForCausalLM(nn.Module):
                     lin.quant_method.process_weights_after_loading(lin)
             if layer.is_moe:
                 layer.experts.quant_method.process_weights_after_loading(layer.experts)
+        ops.mark_weights(self)
         return self
 
     def weight_bytes_per_layer(self, active_expert_fraction: float = 1.0) -> int:

@@ -265,6 +265,7 @@ class NukezenForCausalLM(nn.Module):
     def finalize(self):
         for layer in self.own.values():
             layer.mix.finalize()
+        ops.mark_weights(self)
         return self
 
     @torch.no_grad()

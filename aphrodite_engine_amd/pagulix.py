@@ -162,6 +162,7 @@ class PagulixForCausalLM(nn.Module):
             layer.hc1.finalize()
             if layer.hc2 is not None:
                 layer.hc2.finalize()
+        ops.mark_weights(self)
         return self
 
     @torch.no_grad()

@@ -203,6 +203,7 @@ class VivisunForCausalLM(nn.Module):
             for n in layer.norms():
                 n.finalize()
         self.final_norm.finalize()
+        ops.mark_weights(self)
         return self
 
     @torch.no_grad()

@@ -31,6 +31,12 @@ extern "C" {
 #define APHRO_F16 0
 #define APHRO_BF16 1
 #define APHRO_F32 2
+/* Or-ed into the dtype of aphro_dense_rows, aphro_lm_head_argmax, aphro_scaled_mm_fp8, aphro_fp8_gemm_stream, aphro_fp8_gemm_stream_silu_quant and
+ * aphro_fp8_gemm_rows, or given to aphro_scaled_mm_fp8_slabs_flags: whether the weight comes from memory at every call, as in a model larger than
+ * the 256 MB last-level cache, or stays in that cache from call to call (a small model, a draft model between its own steps).  Neither: weights of
+ * more than 256 MB come from memory.  The results are the same. */
+#define APHRO_WEIGHTS_STREAMED 0x100
+#define APHRO_WEIGHTS_CACHED 0x200
 /* KV-cache dtypes ("auto" | "fp8"=="fp8_e4m3" | "fp8_e5m2"), OCP encodings */
 #define APHRO_KV_AUTO 0
 #define APHRO_KV_FP8_E4M3 1
@@ -472,6 +478,8 @@ int aphro_fp8_gemm_ksplit(int64_t M, int64_t N, int64_t K);
 int aphro_scaled_mm_fp8_slabs(const void* a, const void* b, float* partials,
                               size_t partial_bytes, int64_t M, int64_t N, int64_t K,
                               void* stream);
+int aphro_scaled_mm_fp8_slabs_flags(const void* a, const void* b, float* partials, size_t partial_bytes, int64_t M, int64_t N, int64_t K, int flags,
+                                    void* stream);
 
 /* [slab reduce + dequant] + fused_add_rms_norm (layernorm_kernels.cu:200-240) +
  * dynamic_per_token_scaled_fp8_quant (fp8/common.cu:201-256).  input (T) XOR slabs

@@ -79,3 +79,34 @@ def test_wide_heads(m, n, k, dtype):
         want = x.double() @ w[part:part + 32768].double().t()
         for out, off in ((got, 0.0), (biased, bias[part:part + 32768].double())):
             assert bool(((out[:, part:part + 32768].double() - (want + off)).abs() <= u * (want + off).abs() + k * 2.0 ** -24 * 4.0).all())
+
+
+def test_marked_weights_give_the_same_results():
+    """Every kernel that takes the hint, with it, without it and by the weight's size."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    f8 = lambda *s: (torch.randn(*s, generator=g, device="cuda") * 0.1).to(torch.float8_e4m3fn)
+
+    def same(weight, call):
+        outs = []
+        for mark in (None, True, False):
+            if mark is None:
+                weight.__dict__.pop("streamed", None)
+            else:
+                weight.streamed = mark
+            outs.append(call(weight))
+        assert outs[0].isfinite().all() and outs[0].any() and torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+    for m in (1, 16, 40, 64, 100, 150):
+        x = torch.randn(m, 2560, generator=g, device="cuda").half()
+        same((torch.randn(20488, 2560, generator=g, device="cuda") * 0.02).half(), lambda w: ops.dense_rows(x, w))
+    x = torch.randn(20, 2048, generator=g, device="cuda").bfloat16()
+    same(torch.randn(32008, 2048, generator=g, device="cuda").bfloat16(), lambda w: ops.lm_head_argmax(x, w))
+    sb, one = torch.rand(16384, generator=g, device="cuda") + 0.5, torch.ones(1, device="cuda")
+    for m in (7, 32, 64, 128, 192):                          # (the stream kernel up to 32 rows, the few-rows one from 33 on)
+        a, sa = f8(m, 1024), torch.rand(m, 1, generator=g, device="cuda") + 0.5
+        w = f8(16384, 1024).t()
+        same(w, lambda w: ops.cutlass_scaled_mm(a, w, sa, sb, torch.float16))
+        same(w, lambda w: ops.scaled_mm_fp8_slabs(a, w))
+        if m <= 32:
+            assert ops.fp8_gemm_silu_quant_supported(m, 16384, 1024)
+            same(w, lambda w: ops.fp8_gemm_silu_quant(a, w, sa, sb, one, torch.float16).float())
