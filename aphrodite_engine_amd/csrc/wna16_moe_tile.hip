@@ -401,8 +401,8 @@ using namespace aphro;
 
 // K slices of the second GEMM for up to `blocks` row blocks, of which padding takes some four: the mean of the rounds of workgroups over the CUs
 // with and without a started one counting as whole, each round 1 us per K tile and 6 us around them, and the slabs.  Mixtral-8x7B, us with one /
-// two / four: 100 tokens 104 / 61 / 66, 362 183 / 116 / 123, 700 205 / 208 / 219, 1000 361 / 296 / 283, 3000 823 / 763 / 775.  0: the shape is not
-// served.
+// two / four: 100 tokens 104 / 61 / 66, 362 183 / 116 / 123, 700 205 / 208 / 219, 1000 361 / 296 / 283, 3000 823 / 763 / 775.  A slice has 179 groups
+// at most in blocks of 64 rows and 102 in blocks of 128: more have not been measured (the kernel would stage them in turn).  0: the shape is not served.
 static int moe_tile_ksplit(int64_t blocks, int64_t N, int64_t K, int64_t groups, int block_m, int silu) {
   if (groups <= 0 || K % groups != 0 || N % MT_BN != 0 || (block_m != 64 && block_m != 128)) return 0;
   if (K / groups % 128 != 0 || K / 8 * N * 4 > 0xffffffffll) return 0;

@@ -155,7 +155,7 @@ def moe_tile_block(slots: int, experts: Wna16Experts, dtype: torch.dtype, a_byte
 def _tile_served(slots: int, experts: Wna16Experts, bm: int, dtype: torch.dtype, a_bytes: int) -> bool:
     blocks = (slots + experts.num_experts * (bm - 1) + bm - 1) // bm
     # rows of either GEMM go by 32-bit offsets: Mixtral's from 74 000 tokens on; what the decode kernel refuses stays refused whatever the batch
-    return (dtype == experts.w13[2].dtype and max(a_bytes, (slots + experts.num_experts * 127 + 127) // 128 * 128 * experts.inter * 2) < 2 ** 32 - 1
+    return (dtype == experts.w13[2].dtype and max(a_bytes, blocks * bm * experts.inter * 2) < 2 ** 32 - 1
             and all(ops.wna16_moe_tile_ksplit(blocks, qw.shape[2], k, sc.shape[1], bm, silu) > 0
                     and ops.wna16_grouped_ksplit(blocks * bm, qw.shape[2], k, sc.shape[1]) > 0
                     for (qw, _, sc), k, silu in ((experts.w13, experts.hidden, True), (experts.w2, experts.inter, False))))
@@ -169,7 +169,8 @@ def moe_tile_align(slots: int, experts: Wna16Experts, dtype: torch.dtype, a_byte
     (Mixtral-8x7B, both GEMMs, 64 / 128: 100 tokens 183 / 193, 160 235 / 254, 220 262 / 285, 300 370 / 332)."""
     e = experts.num_experts
     bm = moe_tile_block(slots, experts, dtype, a_bytes)
-    if bm == 0 and slots * 3 >= moe_tile_rows(experts) * e * 2 and slots < MOE_TILE_PAIRS * e:
+    least = moe_tile_rows(experts) * e
+    if bm == 0 and (slots >= least or (slots * 3 >= least * 2 and slots < MOE_TILE_PAIRS * e)):
         return 64 if _tile_served(slots, experts, 64, dtype, a_bytes) else 0
     return 128 if bm == 64 and slots >= MOE_TILE_PAIRS * e and _tile_served(slots, experts, 128, dtype, a_bytes) else bm
 

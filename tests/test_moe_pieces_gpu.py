@@ -64,3 +64,28 @@ def test_which_batches_are_aligned_how():
     experts = SimpleNamespace(num_experts=8, hidden=4096, inter=14336, w13=w(4096, 28672), w2=w(14336, 4096))
     align = lambda slots: M.moe_tile_align(slots, experts, torch.float16)
     assert [align(s) for s in (127, 128, 479, 480, 8192)] == [0, 64, 64, 128, 128]
+
+
+def test_batches_that_only_blocks_of_64_serve():
+    """128 groups in front of the activation: blocks of 128 rows hold 102, and the largest batches of such experts take those of 64."""
+    from types import SimpleNamespace
+    from aphrodite_engine_amd import moe as M
+    w = lambda k, n: tuple(torch.empty(8, r, c, dtype=t, device="meta") for r, c, t in
+                           ((k // 8, n, torch.int32), (k // 128, n // 8, torch.int32), (k // 128, n, torch.float16)))
+    experts = SimpleNamespace(num_experts=8, hidden=16384, inter=4096, w13=w(16384, 8192), w2=w(4096, 16384))
+    align = lambda slots: M.moe_tile_align(slots, experts, torch.float16)
+    assert [align(s) for s in (127, 128, 480, 767 * 8, 768 * 8, 20000)] == [0, 64, 64, 64, 64, 64]
+
+    experts, a, b = _experts(2, 16384, 512, 128, 0)
+    g = torch.Generator(device=DEV).manual_seed(0)
+    tokens, ids = 1600, torch.randint(0, 2, (1600,), generator=g, device=DEV)
+    assert M.moe_tile_align(tokens, experts, torch.float16) == 64
+    x = torch.randn(tokens, 16384, generator=g, device=DEV).half()
+    logits, weight = torch.zeros(tokens, 2, device=DEV).half(), torch.rand(tokens, 1, generator=g, device=DEV) + 0.5
+    got = M.fused_wna16_moe(x, experts, logits, 1, True, weight, ids[:, None].to(torch.int32))
+    want = torch.zeros(tokens, 16384, dtype=torch.float64, device=DEV)
+    for i in range(2):
+        rows = ids == i
+        gate, up = (x[rows].double() @ _dense(a[i], 128)).chunk(2, -1)
+        want[rows] = (torch.nn.functional.silu(gate) * up) @ _dense(b[i], 128) * weight[rows].double()
+    assert float((got.double() - want).norm() / want.norm()) < 1.5e-3        # (as above)
