@@ -284,8 +284,8 @@ __device__ __forceinline__ float silu_quotient(float gate) {
 }
 
 // round(round(silu(gate)) * up) in the activation type T, on T-rounded inputs
-// (activation_kernels.cu:14-17, 25-28).  Shared by silu_and_mul, silu_and_mul_pack and the
-// fused GEMM epilogue so that the three paths are bit-identical.
+// (activation_kernels.cu:14-17, 25-28): of the quantising form and the products' epilogues.  silu_and_mul and
+// silu_and_mul_pack (glue.hip, fused_decode.hip), which memory bounds, divide: the two have to agree in every bit.
 template <typename T>
 __device__ __forceinline__ uint16_t silu_mul_bits(float gate, float up) {
   const float s = T::to_f32(T::from_f32(silu_quotient(gate)));
