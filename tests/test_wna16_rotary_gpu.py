@@ -31,8 +31,11 @@ def test_same_bits(dtype, kv, heads, kv_heads, hd, block, k, m, slots):
     for words, strip in forms:
         kc1, vc1, kc2, vc2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
         got = call(ops, a, words, qz, sc, strip, pos, heads, kv_heads, hd, cs, kc1, vc1, sm, kv)
+        served = ops.wna16_prefers_large(m, n, k, dtype, k // 128, strip=strip) and bool(
+            ops._lib.lib().aphro_wna16_gemm_large_rotary_cache_supported(m, n, k, k // 128, ops._dt(a)))
+        assert (got is not None) == served and (served or m not in (129, 150))       # (every head size, type and order of the weights)
         if got is None:                                     # (this order of the weights goes to other kernels)
-            assert not kc1.any() and not vc1.any() and (m, k) != (150, 4096)
+            assert not kc1.any() and not vc1.any()
             continue
         want = ops.wna16_linear_strip(a, words, qz, sc, 1) if strip else ops.wna16_gemm(a, qw, qz, sc, None, 1)
         assert ops.rotary_embedding_and_cache(pos, *parts(want, heads, kv_heads, hd), hd, cs, True, kc2, vc2, sm, kv, 0.5, 2.0)
