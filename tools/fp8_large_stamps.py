@@ -1,7 +1,7 @@
-"""Lab: s_memtime stamps of the stream-K fp8 GEMM's segments (APHRO_FP8_LARGE_DEBUG=4)."""
+"""Lab: s_memtime stamps of the segments of the persistent fp8 GEMM that the plan takes for the size (APHRO_FP8_LARGE_DEBUG=4): the eight-phase kernel's
+whole tiles and slices where the size has them (the default has); the forms without persistent workgroups leave no stamps."""
 import os, sys
 os.environ["APHRO_FP8_LARGE_DEBUG"] = "4"
-os.environ["APHRO_FP8_LARGE_STREAMK"] = "1"
 import torch
 from aphrodite_engine_amd import _custom_ops as ops
 DEV = "cuda"
