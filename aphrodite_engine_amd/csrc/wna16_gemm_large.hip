@@ -1081,9 +1081,10 @@ static int large_bind_scratch(Wna16LargeParams& p, const LargePlan& pl, char* ws
 extern "C" int aphro_wna16_strip_geometry(int64_t M, int64_t N, int64_t K, int64_t groups, int* geom);      // wna16_gemm_resident.hip
 
 // 65 to 128 float16 rows of a matrix below 2^25 weights belong to the decode kernels otherwise, which round no weight: nor does the tile's EXACT form.
-static Wna16RowsPlan rows_exact_plan(int64_t M, int64_t N, int64_t K, int64_t gs) {
+constexpr int64_t ROWS_SLAB_BYTES = 36ll << 20;
+static Wna16RowsPlan rows_exact_plan(int64_t M, int64_t N, int64_t K, int64_t gs, int64_t slab_bytes = ROWS_SLAB_BYTES) {
   if (M > 128 || N * K >= (1 << 25) || knobs().wna16_large_8phase >= 0 || knobs().wna16_large_two_pass >= 0) return {0, 1, false};
-  return wna16_rows_plan_exact(M, N, K, gs, 36ll << 20);
+  return wna16_rows_plan_exact(M, N, K, gs, slab_bytes);
 }
 
 // The tile of wna16_gemm_rows.hip, up to 4096 rows: always where this file would take one workgroup per tile (4096 x 4096: 150 rows
@@ -1092,10 +1093,10 @@ static Wna16RowsPlan rows_exact_plan(int64_t M, int64_t N, int64_t K, int64_t gs
 // rows 345 / 331.  28672 x 4096, 700 rows 193 / 201, 2048 468 / 487, 4096 893 / 948: stays).  Its K slices are its own, of any whole K tiles up to 36 MiB of slabs;
 // this file's are ranges of whole groups, of which 11008 or 9728 rows of K have few divisors and one group per column none (4096 x 11008 at 65
 // / 150 / 300 rows with slices bound to this file's 53 / 54 / 54 us, without 21 / 28 / 40 us).
-static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype) {
+static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype, int64_t slab_bytes = ROWS_SLAB_BYTES) {
   if (knobs().wna16_large_8phase >= 0 || knobs().wna16_large_two_pass >= 0) return {0, 1, false};      // a switch names this file's forms
   if (dtype == APHRO_F16) {
-    const Wna16RowsPlan exact = rows_exact_plan(M, N, K, gs);
+    const Wna16RowsPlan exact = rows_exact_plan(M, N, K, gs, slab_bytes);
     if (exact.mb > 0) return exact;
   }
   int64_t other_ns = -1;
@@ -1105,13 +1106,23 @@ static Wna16RowsPlan rows_plan(const LargePlan& pl, int64_t M, int64_t N, int64_
     if (large_eight(pl, K)) other_ns = large_rounds(tiles, K / 64, pl.grid, two_pass).ns + (two_pass ? 3000 + N * K * 43 / 100000 : 0);
     else other_ns = 18000 + (tiles * (K / 64) * 1930 + tiles * 6000) / pl.grid;
   }
-  return wna16_rows_plan(M, N, K, gs, pl.streamk ? 0 : 36ll << 20, other_ns);
+  return wna16_rows_plan(M, N, K, gs, pl.streamk ? 0 : slab_bytes, other_ns);
+}
+// The tile for a call whose workspace holds ``room`` bytes of slabs: fewer K slices where those of the plan do not fit.  A caller may have sized once
+// for more rows, whose plan has fewer slabs than these rows' or none (one group per column, 6144 x 4096: 200 rows nothing, 65 rows 6 MB).  The
+// same products and roundings of weights; mb == 0: no such form.
+static Wna16RowsPlan rows_plan_within(const Wna16RowsPlan& plan, const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs, int dtype, int64_t room) {
+  if (plan.mb == 0 || pl.streamk || (int64_t)wna16_rows_slab_bytes(plan, M, N) <= room) return plan;
+  const Wna16RowsPlan fewer = rows_plan(pl, M, N, K, gs, dtype, room);
+  return fewer.exact == plan.exact ? fewer : Wna16RowsPlan{0, 1, false};
 }
 
+// the f16 copy of bf16 activations
+static size_t large_copy_bytes(int64_t M, int64_t K, int dtype) { return dtype == APHRO_BF16 ? ((size_t)M * K * 2 + 255) / 256 * 256 : 0; }
 static size_t large_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype, int strip_m) {
   if (groups <= 0 || K % groups != 0) return 0;
   const LargePlan pl = large_plan(M, N, K, K / groups);
-  size_t b = dtype == APHRO_BF16 ? ((size_t)M * K * 2 + 255) / 256 * 256 : 0;
+  size_t b = large_copy_bytes(M, K, dtype);
   if (large_two_pass(pl, M, N, K, K / groups)) b += ((size_t)N * K * 2 + 255) / 256 * 256;      // f16 W^T of the two-pass form
   (void)strip_m;              // (every plan addresses the strip-major copy in place: nothing is rebuilt)
   const size_t slabs = wna16_rows_slab_bytes(rows_plan(pl, M, N, K, K / groups, dtype), M, N), other = large_scratch_bytes(pl, M, N);
@@ -1156,10 +1167,15 @@ static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const 
   const LargePlan pl = large_plan(M, N, K, gs);
   APHRO_CHECK(!silu || pl.streamk || pl.ksplit == 1, "wna16_gemm_large_silu: shape M=%ld N=%ld K=%ld is K-sliced (no SiluAndMul epilogue)",
               (long)M, (long)N, (long)K);
-  const size_t need = large_workspace_bytes(M, N, K, groups, dtype, strip_m);
-  if (need > 0 && (workspace == nullptr || workspace_bytes < need)) {
-    set_error("wna16_gemm_large: workspace %zu < %zu bytes", workspace_bytes, need);
-    return APHRO_ERR_WORKSPACE;
+  Wna16RowsPlan rp = rows_plan(pl, M, N, K, gs, dtype);
+  const size_t need = large_workspace_bytes(M, N, K, groups, dtype, strip_m), given = workspace ? workspace_bytes : 0;
+  if (given < need) {
+    const size_t copy = large_copy_bytes(M, K, dtype);
+    if (given >= copy) rp = rows_plan_within(rp, pl, M, N, K, gs, dtype, (int64_t)(given - copy));
+    if (given < copy || rp.mb == 0 || pl.streamk || ((norm_weight || rotary) && rp.ksplit == 1)) {
+      set_error("wna16_gemm_large: workspace %zu < %zu bytes", workspace_bytes, need);
+      return APHRO_ERR_WORKSPACE;
+    }
   }
   Wna16LargeParams p;
   p.silu = silu;
@@ -1171,7 +1187,7 @@ static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const 
                        (uint16_t*)ws, (int)M, (int)K, (int)lda);
     APHRO_LAUNCH_CHECK();
     p.a = (const uint16_t*)ws; p.lda = (int)K;
-    ws += ((size_t)M * K * 2 + 255) / 256 * 256;
+    ws += large_copy_bytes(M, K, dtype);
   }
   p.qw = q_weight; p.qz = qzeros; p.sc = (const uint16_t*)scales; p.c = (uint16_t*)c;
   p.M = (int)M; p.N = (int)N; p.K = (int)K; p.group_size = (int)gs; p.zero_offset = zero_offset;
@@ -1198,7 +1214,6 @@ static int wna16_gemm_large_impl(const void* a, const uint32_t* q_weight, const 
       APHRO_CHECK(((x * p.st_inv_nseg) >> 16) == x / p.st_nseg && ((x * p.st_inv_nwv) >> 16) == x / p.st_nwv,
                   "wna16_gemm_large_strip: multiply-shift division fails at %u (nseg %d, nwv %d)", x, p.st_nseg, p.st_nwv);
   }
-  const Wna16RowsPlan rp = rows_plan(pl, M, N, K, gs, dtype);
   APHRO_CHECK(!norm_weight || (rp.mb > 0 && rp.ksplit > 1 && N <= 16384), "wna16_gemm_large_add_norm: M=%ld N=%ld K=%ld has no summed K slices",
               (long)M, (long)N, (long)K);
   APHRO_CHECK(!rotary || (rp.mb > 0 && rp.ksplit > 1), "wna16_gemm_large_rotary_cache: M=%ld N=%ld K=%ld has no summed K slices", (long)M, (long)N, (long)K);

@@ -664,7 +664,8 @@ int aphro_custom_ar_init_loopback(void** fa_out, void* signal, void* scratch, si
  * q_weight [K/8, N] in the exllama-shuffled order, qzeros [G, N/8], scales [G, N] in `dtype`; c [M, N] in `dtype`.
  * N % 128 == 0, K % 64 == 0, group size % 64 == 0.  Act-order: pass activations already gathered (a[:, perm]).
  * workspace: aphro_wna16_gemm_large_workspace_bytes (f16 copy of bf16 activations, saturating; fp32 split-K slabs when
- * the tile grid alone would not cover the chip). */
+ * the tile grid alone would not cover the chip).  The size is that of M rows; fewer rows may ask for more slabs.  Up to 4096 rows
+ * the product takes fewer K slices where a smaller workspace holds no more. */
 size_t aphro_wna16_gemm_large_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t groups, int dtype);
 /* 65 to 128 float16 rows of a matrix below 2^25 weights: K tiles of 128 that a CU has to do (a further round of workgroups counts as
  * eight) in the form of aphro_wna16_gemm_large that multiplies exact integers and scales fp32 sums; 0: no such form for the call. */

@@ -60,3 +60,24 @@ def test_w8a16_clears_its_flags(m, n, k):
                                                   _lib.F16, torch.cuda.current_stream().cuda_stream), "gemm")
     for got in replayed(call, out, ws):
         assert torch.equal(got, want)
+
+
+# (rows that the workspace is sized for, rows, columns, k, groups): the most rows ask for fewer slabs than the fewer, or none; 65 to 128 float16 rows
+# keep their own form
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("most,m,n,k,groups", [(200, 65, 6144, 4096, 1), (256, 128, 6144, 4096, 1), (300, 150, 4096, 4096, 1), (300, 257, 4096, 4096, 1), (257, 129, 4096, 11008, 86),
+                                               (257, 100, 4096, 11008, 86), (1024, 200, 6144, 4096, 32)])
+def test_a_workspace_for_other_rows_serves_with_fewer_slices(most, m, n, k, groups, dtype):
+    lib, dt = _lib.lib(), _lib.F16 if dtype == torch.float16 else _lib.BF16
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a = torch.randint(-1, 2, (m, k), generator=g, device=DEV).to(dtype)
+    qw, w = weights(n, k, g)
+    qz = torch.full((groups, n // 8), 0x77777777, dtype=torch.int32, device=DEV)
+    sc = torch.ones(groups, n, dtype=dtype, device=DEV)
+    size = lambda rows: lib.aphro_wna16_gemm_large_workspace_bytes(rows, n, k, groups, dt)
+    assert size(most) < size(m)
+    ws = torch.full((size(most) + 256,), 0x7f, dtype=torch.uint8, device=DEV)        # (256 bytes that no call may write)
+    out = torch.empty(m, n, dtype=dtype, device=DEV)
+    _lib.check(lib.aphro_wna16_gemm_large(a.data_ptr(), qw.data_ptr(), qz.data_ptr(), sc.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel() - 256, m, n, k,
+                                          groups, k, 1, dt, torch.cuda.current_stream().cuda_stream), "gemm")
+    assert torch.equal(out, (a.float() @ w.float()).to(dtype)) and bool((ws[-256:] == 0x7f).all())
