@@ -223,16 +223,17 @@ __device__ __forceinline__ bool pa_take_run(const int32_t* seq_lens, int n, int 
 // pay for the extra live state -- measured +1.4 us per launch when it was a runtime branch)
 // Kernel arguments: the head of the dependent chain (sequence length -> block table -> K/V addresses) and the sizes every
 // address needs come first and as scalars, so that they are preloaded into SGPRs (Makefile: -amdgpu-kernarg-preload-count);
-// p_in carries the rest, its copies of the leading fields are not read.
+// p_in carries the rest, its copies of the leading fields are not read.  partition_or_extra: the split form has no partitions, and whether its runs are
+// dealt stands ahead of the sequence length (read from p_in: 0.1 us a launch longer, an int4 step of one row 2 of 885).
 template <typename T, int KV, int HD, int BS, int NW, int ROPE, bool SPLIT = false>
 __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t* seq_lens, const int32_t* block_tables,
                                                                   const void* kc_, const void* vc_, const float* qkv_slabs,
                                                                   int num_heads, int num_kv_heads, int max_blocks_per_seq,
-                                                                  int partition_size, PAParams p_in) {
+                                                                  int partition_or_extra, PAParams p_in) {
   PAParams p = p_in;
   p.seq_lens = seq_lens; p.block_tables = block_tables; p.kc = kc_; p.vc = vc_; p.qkv_slabs = qkv_slabs;
   p.num_heads = num_heads; p.num_kv_heads = num_kv_heads; p.max_blocks_per_seq = max_blocks_per_seq;
-  p.partition_size = partition_size;
+  (SPLIT ? p.extra : p.partition_size) = partition_or_extra;
   constexpr bool FP8 = KV != 0;
   constexpr bool E5M2 = KV == 2;
   constexpr int XB = 16;                        // bytes per K chunk
@@ -1215,7 +1216,7 @@ static int launch_pa(const PAParams& p, int num_seqs, int parts, int nw, hipStre
     if (lds > 64 * 1024)                                                                            \
       (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
     hipLaunchKernelGGL(kern, grid, dim3(NWV * 64), lds, st, p.seq_lens, p.block_tables, p.kc, p.vc, p.qkv_slabs,        \
-                       p.num_heads, p.num_kv_heads, p.max_blocks_per_seq, p.partition_size, p);                  \
+                       p.num_heads, p.num_kv_heads, p.max_blocks_per_seq, SPL ? p.extra : p.partition_size, p);                  \
   }
   if constexpr (HD == 128 && (BS == 16 || BS == 32)) {   // the split form is instantiated for the serving geometry only
     if (p.nsplit > 1) {
