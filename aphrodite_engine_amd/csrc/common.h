@@ -277,7 +277,8 @@ __device__ __forceinline__ float wave_max(float v) {
 
 // gate / (1 + e^-gate) for a gate of 16 bits: one reciprocal and one exact correction in place of a division, the same value once it is rounded to
 // the gate's type, for each of the 65536 gates of either (9 instructions for 16: they weigh in SiluAndMul's quantising form, 8192 x 28672 128 -> 118 us,
-// and in the products' epilogues; int4 gate_up of 32 rows 15.2 -> 14.8).  The denominator goes in a quarter of its size, so that its reciprocal is a normal number wherever the quotient is not zero.
+// and in the products' epilogues; int4 gate_up of 32 rows 15.2 -> 14.8).  The denominator goes in a quarter of its size, so that its reciprocal is a normal number
+// wherever the quotient is not zero.
 __device__ __forceinline__ float silu_quotient(float gate) {
   const float d = 1.0f + __expf(-gate), y = 0.25f * __builtin_amdgcn_rcpf(0.25f * d), q = gate * y;
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, gate), y, q), d, gate);

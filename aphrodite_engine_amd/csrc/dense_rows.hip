@@ -146,8 +146,8 @@ __global__ __launch_bounds__(256) void dense_rows_reduce_kernel(DenseRowsParams 
   dr_store<T>(p, m, col, v);
 }
 
-// Whether a w that passes the caches once (weights_streamed) takes the non-temporal hint (RowsTile) above 48 rows of x, up to which it does: with 40 steps of 64 k a slice and more, up to
-// 128 rows.  us without / with it, f16, weights from memory: [128256, 4096], 16 / 64 / 96 / 192 rows 187 / 198 / 212 / 254 and 167 / 192 / 211 / 253;
+// Whether a w that passes the caches once (weights_streamed) takes the non-temporal hint (RowsTile) above 48 rows of x, up to which it does: with 40
+// steps of 64 k a slice and more, up to 128 rows.  us without / with it, f16, weights from memory: [128256, 4096], 16 / 64 / 96 / 192 rows 187 / 198 / 212 / 254 and 167 / 192 / 211 / 253;
 // [28672, 4096], 16 / 64 / 128 / 150 rows 50.5 / 51.4 / 57.9 / 59.5 and 46.7 / 47.9 / 56.8 / 60.1; [10240, 8192], 42 steps, 32 / 65 / 128 rows 38.1 /
 // 37.9 / 42.6 and 35.2 / 35.5 / 41.8.  Short slices lose with many rows: [4096, 14336], 28 steps, 16 / 48 / 96 / 128 rows 24.9 / 26.8 / 30.4 / 33.2
 // and 22.1 / 25.3 / 32.2 / 35.6; [6144, 4096], 12 steps, 16 / 64 / 128 rows 14.3 / 17.6 / 20.5 and 13.5 / 19.0 / 23.4.  (FP8, half the bytes of x a step,

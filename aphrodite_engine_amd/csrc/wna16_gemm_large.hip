@@ -1023,7 +1023,8 @@ static LargePlan large_plan(int64_t M, int64_t N, int64_t K, int64_t gs) {
 // stream-K plan.  Costs K x N f16 of workspace per call.  APHRO_WNA16_LARGE_TWO_PASS=0/1 forces (tests compare the two forms' bits).
 // (us, fused / two passes: 28672 x 4096, 2560 rows 572 / 564, 3072 673 / 653, 4096 857 / 813, 6100 1293 / 1204; 4096 x 14336, 3500 rows 391 / 358;
 // 6144 x 4096, 3072 rows 168 / 164, 5000 243 / 227; 4096 x 4096, 3072 rows 114 / 106; 8192 x 8192, 4096 rows 480 / 446.  Up to 4096 rows the
-// workspace stays without the copy of the weights all the same: its size there is promised to callers)
+// workspace stays without the copy of the weights all the same: its size there is promised to callers, not measured.  From 4097 to 6143 rows, fused
+// before there were whole tiles, the copy is up to 235 MB more of it)
 constexpr int64_t TWO_PASS_MIN_M = 4097;
 static bool large_two_pass(const LargePlan& pl, int64_t M, int64_t N, int64_t K, int64_t gs) {
   const int force = knobs().wna16_large_two_pass;

@@ -14,7 +14,8 @@
 //   * K slices write the accumulators as they lie in the registers, 1 KiB a store; a second kernel sums them in the order of K.
 //   * what a wave issues is the other limit: with the scalar arithmetic of a tile's addresses (57 operations), its zero points' 64-bit
 //     addresses and the fragment reads of a step in one place, the first four waves of a CU needed 1 205 cycles a tile alone, and the
-//     other four, behind them, as many again beside their MFMAs.  Running offsets, groups by one multiplication and one MFMA, one read or load and three or four operations of the unpacking a slot: 19 scalar operations of 143 in all.
+//     other four, behind them, as many again beside their MFMAs.  Running offsets, groups by one multiplication and one MFMA, one read or
+//     load and three or four operations of the unpacking a slot: 19 scalar operations of 143 in all.
 // Bound by MFMAs, which pull the clock to 1.65 GHz: 1 670 cycles per K tile of 160 rows (1 900 before), 1 280 of them MFMA.
 // Layer of Llama-3-8B at 150 rows, four GEMMs with their slab sums: 192 -> 114 us (qkv 40.4 -> 24, o 27.3 -> 17, gate_up 76 -> 42,
 // down 48 -> 31); at 65 rows 128 -> 79; at 1300 rows 756 -> 629 us.
@@ -530,7 +531,8 @@ static bool rw_groups_exact(int64_t K, int64_t gs) { return (rw_inv_group(gs) * 
 // Tile height and K slices by the time they are expected to take (MI355X, ns; within 10 % of what was measured for 65 .. 4096 rows of
 // Llama-3-8B's and -70B's matrices): rounds of workgroups over the CUs, each 170 + 200 per 32-row block and K tile and 4.7 us around
 // them, a last one that is not full 0.74 of that and 0.26 by how full it is (few workgroups run at a higher clock and have the memory to
-// themselves), and the slabs written and read again at 2.2 TB/s behind 3 us.  Of the forms measured for 150 to 4096 rows of 28672 x 4096, 6144 x
+// themselves; 0.7 and 0.3 fit better by 0.1 %, but take fewer than four slices at 150 rows of 4096 x 4096 with one group per column, whose
+// workspace is promised), and the slabs written and read again at 2.2 TB/s behind 3 us.  Of the forms measured for 150 to 4096 rows of 28672 x 4096, 6144 x
 // 4096, 4096 x 4096 and 4096 x 14336 the one taken is 0.2 % behind the best on average (a last round counted whole: 2.2 %).  us: 6144 x 4096,
 // 150 rows: five blocks and four slices 24.3, three and two 21.1; 900 rows, five blocks in 1.1 rounds 69.8, three in 1.9 59.6; 4096 x 14336, 150
 // rows: one slice 82, two 49, four 32; 4096 x 4096, 150 rows: five blocks and four slices 20.6, three and three 18.2.
