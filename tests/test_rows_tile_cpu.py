@@ -49,3 +49,17 @@ def test_a_prompt_workspace_for_many_rows_serves_fewer():
         for k in (128, 1024, 2048, 4096, 11008, 14336):
             sizes = [size(m, n, k) for m in rows]
             assert sizes == sorted(sizes) and sizes[-1] <= 4096 + 256 * 8 * 32 * 1024
+
+
+def test_int4_products_whose_workspace_is_too_small_for_their_form_stay_refused():
+    """(Refused on the host, ahead of any launch.)  Tiles that workgroups share, a copy of bf16 rows that does not fit, slices that a norm sums."""
+    from aphrodite_engine_amd import _lib
+    lib, p = _lib.lib(), 1 << 20
+    size = lambda m, n, k, dt: lib.aphro_wna16_gemm_large_workspace_bytes(m, n, k, k // 128, dt)
+    call = lambda m, n, k, dt, ws, room: lib.aphro_wna16_gemm_large(p, p, p, p, p, ws, room, m, n, k, k // 128, k, 1, dt, None)
+    refused = -3                                             # APHRO_ERR_WORKSPACE
+    for m, n, k, dt, room in ((4096, 28672, 4096, _lib.F16, size(4096, 28672, 4096, _lib.F16) - 1), (150, 4096, 4096, _lib.BF16, 150 * 4096 * 2 - 1),
+                              (8192, 4096, 4096, _lib.F16, 1 << 20), (150, 4096, 4096, _lib.BF16, 0)):
+        assert call(m, n, k, dt, p if room else None, room) == refused
+    assert lib.aphro_wna16_gemm_large_add_norm_supported(150, 4096, 4096, 32, _lib.F16)
+    assert lib.aphro_wna16_gemm_large_add_norm(p, p, p, p, p, p, p, 1e-5, p, 160 * 4096 * 4, 150, 4096, 4096, 32, 4096, 1, _lib.F16, 0, None) == refused
