@@ -42,7 +42,7 @@ struct PAParams {
   const float* alibi;
   int num_heads, num_kv_heads;
   int max_blocks_per_seq;
-  int partition_size;  // tokens per grid.z slice (multiple of 32) ; 0 -> whole sequence
+  int partition_size;  // tokens per grid.z slice (multiple of 32) ; 0 -> whole sequence ; < 0: whole sequences, longest first (plain form)
   int max_parts;       // P of the scratch tensors (0 in v1 form)
   int nh_lds;          // query heads per kv head held in the LDS merge buffer (<= 16)
   int write_direct;    // 1: write `out` (single partition) ; 0: write scratch
@@ -218,6 +218,44 @@ __device__ __forceinline__ bool pa_take_run(const int32_t* seq_lens, int n, int 
   return true;
 }
 
+// The ``rank``-th longest of n sequences, by tile pairs and then by number: found by bisection over the pairs, a ballot per 64 sequences and step.
+template <int Q>
+__device__ __forceinline__ int pa_by_length(const int32_t* seq_lens, int n, int rank, int& seq_len) {
+  const int lane = threadIdx.x & 63;
+  int len[Q], pairs[Q], most = 0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    len[q] = 64 * q + lane < n ? seq_lens[64 * q + lane] : 0;
+    pairs[q] = 64 * q + lane < n ? (len[q] + 31) >> 5 : -1;
+    most = max(most, pairs[q]);
+  }
+  int lo = 0, hi = pa_wave_max(most);                   // the pairs of the one looked for
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    int c = 0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) c += __builtin_popcountll(__ballot(pairs[q] > mid));
+    if (c > rank) lo = mid + 1; else hi = mid;
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q) rank -= __builtin_popcountll(__ballot(pairs[q] > lo));
+  int seq = 0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    uint64_t mask = __ballot(pairs[q] == lo);
+    const int c = __builtin_popcountll(mask);
+    if (rank >= 0 && rank < c) {
+      for (int i = 0; i < rank; ++i) mask &= mask - 1;
+      seq = 64 * q + __builtin_ctzll(mask);
+    }
+    rank -= c;
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if ((seq >> 6) == q) seq_len = __builtin_amdgcn_readlane(len[q], seq & 63);
+  return seq;
+}
+
 // KV: 0 = cache holds T, 1 = e4m3, 2 = e5m2.   HD: head size.  BS: block size.
 // ROPE: the fused rotary + cache-write form (a separate instantiation: the plain kernel must not
 // pay for the extra live state -- measured +1.4 us per launch when it was a runtime branch)
@@ -272,6 +310,8 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(const int32_t*
     const int n = (int)gridDim.y - p.extra;
     if (!(n <= 64 ? pa_take_run<1>(p.seq_lens, n, p.extra, (int)blockIdx.y, run) : pa_take_run<PA_MAX_DEALT / 64>(p.seq_lens, n, p.extra, (int)blockIdx.y, run)))
       return;
+  } else if (!split && ROPE == 0 && p.partition_size < 0) {
+    run.seq = pa_by_length<PA_MAX_DEALT / 64>(p.seq_lens, (int)gridDim.y, (int)blockIdx.y, run.seq_len);
   } else {
     run.seq_len = p.seq_lens[run.seq];
   }
@@ -1402,8 +1442,15 @@ static int paged_attention_impl(void* out, void* out_packed, float* exp_sums, fl
   p.nsplit = 0; p.extra = 0; p.split_scratch = nullptr; p.split_counter = nullptr;
   if (partition_size == 0) {
     p.partition_size = 0; p.max_parts = 0; p.write_direct = 1;
-    // v1 form: one workgroup per (seq, kv head) walks the whole sequence
-    nw = max_seq_len > 256 ? 8 : 4;
+    // v1 form: one workgroup per (seq, kv head) walks the whole sequence.  Eight waves of 164 registers are all that a CU holds, of four three
+    // workgroups: where there are more of them than CUs, a workgroup's start (three dependent loads) and merge then lie behind the others' streams.
+    // us a decode step of four layers, 8 kv heads, 16-bit keys, eight waves / four: 34 sequences of 300 543 / 526, 33 / 40 / 65 of 1040 618 / 605, 631 /
+    // 625, 819 / 800, 64 of 400 606 / 593; the fused forms over FP8 keys (127 registers: two workgroups of eight) keep eight, 64 of 400 561 / 566.
+    // From three workgroups a CU on they do not all run at once, and the sequences go from the longest to the shortest (pa_by_length), so that a
+    // launch does not end on a long one: 150 sequences of 375 to 1500, a layer, eight waves / four / longest first 115 / 111 / 102 us (5.0 -> 5.7 TB/s).
+    const int64_t wgs = (int64_t)num_seqs * num_kv_heads, cus = device_cu_count();
+    nw = max_seq_len > 256 && (wgs <= cus || (qkv_slabs != nullptr && kv_dtype != APHRO_KV_AUTO)) ? 8 : 4;
+    if (qkv_slabs == nullptr && wgs >= 3 * cus && num_seqs <= PA_MAX_DEALT) p.partition_size = -1;
     while (nw > 4 && (size_t)nw * (32 + p.nh_lds * head_size) * 4 > 96 * 1024) nw >>= 1;
     // ... or nsplit workgroups share it (pa_plan).  APHRO_PA_SPLITS=n forces n (1 = off).
     const size_t groups = (size_t)num_seqs * num_kv_heads;
