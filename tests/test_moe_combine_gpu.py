@@ -1,0 +1,27 @@
+"""Routed weights and the sum over a token's choices (moe_combine): every number of slabs that has a kernel of its own and others, odd numbers of choices,
+rows at the edges of a workgroup's columns -- the same bits as the sums in the order that the operation states."""
+import pytest
+import torch
+
+from aphrodite_engine_amd import _custom_ops as ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("tokens,topk,nslab,n", [(1, 1, 1, 4), (3, 2, 2, 1020), (32, 2, 4, 4096), (5, 3, 3, 1028), (2, 5, 4, 2052), (17, 8, 7, 260),
+                                                 (65, 3, 1, 1024), (300, 2, 2, 512)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_combine(tokens, topk, nslab, n, dtype):
+    g = torch.Generator(device=DEV).manual_seed(tokens * n + nslab)
+    rows = tokens * topk + 7
+    slabs = torch.randn(nslab, rows, n, generator=g, device=DEV)
+    inv = torch.randperm(rows, generator=g, device=DEV)[:tokens * topk].int()
+    w = torch.rand(tokens, topk, generator=g, device=DEV)
+    y = slabs[0]
+    for s in range(1, nslab):
+        y = y + slabs[s]
+    acc = torch.zeros(tokens, n, device=DEV)
+    for k in range(topk):
+        acc = acc + (y[inv.view(tokens, topk)[:, k].long()] * w[:, k:k + 1]).to(dtype).float()
+    assert torch.equal(ops.moe_combine(slabs, inv, w, dtype), acc.to(dtype))
