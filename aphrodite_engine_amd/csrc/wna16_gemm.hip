@@ -379,6 +379,181 @@ __global__ __launch_bounds__(FNW * 64, (VEC * MT >= 8) ? 2 : 3) void wna16_gemm_
   wna16_epilogue<T, VEC, MT, FNW>(p, red, cacc, lane, wave, g, m0, ncol, by);
 }
 
+// Grouped form for chains of 4 to 8 segments a wave: workgroups that stay, two a CU.  A workgroup takes an equal share of the (16-row tile, K slice,
+// 64-column tile) units, neighbours in that order, and keeps the tile's activations -- the A fragments of its waves' segments, NSEG * 16 registers --
+// from unit to unit; the next unit's first weights are on their way before this one's sums meet.  wna16_gemm_kernel reads a byte of activations a byte
+// of weights from L2 again for every 64 columns, and each of its workgroups starts anew behind three dependent loads: 8 experts of 4096 x
+// 28672 (502 MB with scales), 16-row tiles, random weights 99 us against 72.5 for the same weights only read; here 82 (6.1 TB/s).
+// 8 x 14336 x 4096 in four K slices 54 -> 46.5 (read 37).  The units are dealt so that an XCD's are
+// neighbours (its L2 fetches its own tiles' activations only: 2 us of the 46.5) and that units over an equal share go to one workgroup of a CU,
+// not both (four tiles of the first 55 -> 49).  Two segments of weights ahead, with spills: 8 us more.  Same products in the same order as wna16_gemm_kernel: same bits.
+template <typename T, int NSEG>
+__global__ __launch_bounds__(FNW * 64, 2) void wna16_experts_kernel(Wna16Params p) {
+  constexpr int AUX_NT = 2;
+  extern __shared__ __attribute__((aligned(16))) float red2[];          // [2][FNW][4][64][4]: units alternate, one barrier each
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  const int ntiles = p.N >> 6, mtiles = p.M >> 4;
+  const int units = min((*p.num_post_pad + 15) >> 4, mtiles) * p.ksplit * ntiles;
+  // workgroup b of grid (a multiple of 8) stands at (b % 8) * grid / 8 + b / 8; of the units over an equal share, b < rest take one each
+  const int each = units / (int)gridDim.x, rest = units - each * (int)gridDim.x;
+  const int xcd = (int)blockIdx.x & 7, idx = (int)blockIdx.x >> 3, more_each = rest >> 3, more_xcds = rest & 7;
+  const int more_here = more_each + (xcd < more_xcds ? 1 : 0);
+  int unit = (xcd * ((int)gridDim.x >> 3) + idx) * each + xcd * more_each + min(xcd, more_xcds) + min(idx, more_here);
+  const int end = unit + each + (idx < more_here ? 1 : 0);
+  if (unit >= end) return;
+  const int ngroups = p.K / p.group_size;
+  const uint32_t wbytes = (uint32_t)((size_t)(p.K >> 3) * p.N * 4), sbytes = (uint32_t)((size_t)ngroups * p.N * 2),
+                 zbytes = (uint32_t)((size_t)ngroups * (p.N >> 3) * 4);
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.apk, (uint32_t)((size_t)(p.K >> 7) * 4 * mtiles * 1024));
+  const int roww = p.N * 4, abytes = mtiles * 1024;
+  const int voff_w = (4 * g * p.N + 4 * c) * 4, zshift = ((4 * c) & 7) * 4;
+  const float zoff = (float)p.zero_offset;
+  const f16x8 ones = {(f16)1.f, (f16)1.f, (f16)16.f, (f16)16.f, (f16)1.f, (f16)1.f, (f16)16.f, (f16)16.f};
+  const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+
+  struct Unit {
+    __amdgpu_buffer_rsrc_t w, s, z;         // of no bytes where there is nothing to read: the loads return zeros
+    int mt, by, col, seg0, valid;
+  };
+  auto unit_at = [&](int u, bool there) {
+    Unit r;
+    const int a = u / ntiles;
+    r.col = (u - a * ntiles) << 6;
+    r.mt = a / p.ksplit;
+    r.by = a - r.mt * p.ksplit;
+    r.seg0 = (r.by * FNW + wave) * NSEG;
+    const int e = p.expert_ids[r.mt];
+    r.valid = e >= 0;
+    const size_t e0 = r.valid ? (size_t)e : 0;
+    there = there && r.valid;
+    r.w = make_rsrc(p.qw + e0 * p.w_estride, there ? wbytes : 0);
+    r.s = make_rsrc(p.sc + e0 * p.s_estride, there ? sbytes : 0);
+    r.z = make_rsrc(p.qz + e0 * p.z_estride, there ? zbytes : 0);
+    return r;
+  };
+  u32x4 af[NSEG][4];
+  uint32_t w[2][4][4];
+  u32x2 sc2[2];                              // raw scales and zero words (see SegMeta)
+  uint32_t zw[2];
+  auto load_a = [&](const Unit& t) {
+#pragma unroll
+    for (int s = 0; s < NSEG; ++s)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) af[s][u] = __builtin_amdgcn_raw_buffer_load_b128(ra, (t.mt * 64 + lane) * 16, ((t.seg0 + s) * 4 + u) * abytes, 0);
+#pragma unroll
+    for (int s = 0; s < NSEG; ++s)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {         // (the nibbles that weigh 16x: see wna16_gemm_kernel)
+        asm("v_pk_mul_f16 %0, %1, %2" : "=v"(af[s][u][1]) : "v"(af[s][u][1]), "s"(0x2c002c00u));
+        asm("v_pk_mul_f16 %0, %1, %2" : "=v"(af[s][u][3]) : "v"(af[s][u][3]), "s"(0x2c002c00u));
+      }
+  };
+  auto load_w = [&](uint32_t (&wd)[4][4], const Unit& t, int s) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(t.w, voff_w, ((t.seg0 + s) * 16 + u) * roww + t.col * 4, AUX_NT);
+      wd[u][0] = v[0]; wd[u][1] = v[1]; wd[u][2] = v[2]; wd[u][3] = v[3];
+    }
+  };
+  auto load_meta = [&](u32x2& sc, uint32_t& z, const Unit& t, int s) {
+    const int grp = (t.seg0 + s) >> p.gshift;
+    z = __builtin_amdgcn_raw_buffer_load_b32(t.z, (c >> 1) * 4, (grp * (p.N >> 3) + (t.col >> 3)) * 4, 0);
+    sc = __builtin_amdgcn_raw_buffer_load_b64(t.s, c * 8, (grp * p.N + t.col) * 2, 0);
+  };
+
+  Unit cur = unit_at(unit, true);
+  load_w(w[0], cur, 0);
+  load_meta(sc2[0], zw[0], cur, 0);
+  load_a(cur);
+  float* red = red2;
+  for (;;) {
+    const bool more = unit + 1 < end;
+    const Unit nxt = unit_at(more ? unit + 1 : unit, more);
+    f32x4 cacc[4] = {zero4, zero4, zero4, zero4};
+#pragma unroll
+    for (int s = 0; s < NSEG; ++s) {
+      // (one buffer ahead; the scales first: what is waited for in order)
+      if (s + 1 < NSEG) {
+        load_meta(sc2[(s + 1) & 1], zw[(s + 1) & 1], cur, s + 1);
+        load_w(w[(s + 1) & 1], cur, s + 1);
+      } else {
+        load_meta(sc2[(s + 1) & 1], zw[(s + 1) & 1], nxt, 0);
+        load_w(w[(s + 1) & 1], nxt, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      f32x4 acc[4], rs;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const f16x8 a = __builtin_bit_cast(f16x8, af[s][u]);
+        rs = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ones, u == 0 ? zero4 : rs, 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const uint32_t wv = w[s & 1][u][t], w8 = wv >> 8;
+          const u32x4 bq = {wv & 0x000f000fu, wv & 0x00f000f0u, w8 & 0x000f000fu, w8 & 0x00f000f0u};
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(f16x8, bq), u == 0 ? zero4 : acc[t], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float z = (float)((zw[s & 1] >> (zshift + 4 * t)) & 0xf) + zoff;
+        const float sf = T::to_f32((uint16_t)(sc2[s & 1][t >> 1] >> (16 * (t & 1))));
+        const float s24 = sf * 16777216.f;
+        const float nzs = -z * sf;
+        cacc[t] = __builtin_elementwise_fma(acc[t], f32x4{s24, s24, s24, s24}, cacc[t]);
+        cacc[t] = __builtin_elementwise_fma(rs, f32x4{nzs, nzs, nzs, nzs}, cacc[t]);
+      }
+    }
+    // a barrier for what lies in LDS only: the next unit's loads stay on their way
+#pragma unroll
+    for (int t = 0; t < 4; ++t) *reinterpret_cast<f32x4*>(&red[((wave * 4 + t) * 64 + lane) * 4]) = cacc[t];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int row = 16 * cur.mt + 4 * g + wave, ncol = cur.col + 4 * c;
+    float v[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float sum = 0.f;
+#pragma unroll
+      for (int w2 = 0; w2 < FNW; ++w2) sum += red[((w2 * 4 + t) * 64 + lane) * 4 + wave];
+      v[t] = sum;
+    }
+    if (cur.valid) {
+      if (p.act_packed) {                    // SiluAndMul of (gate, up) pairs, as in wna16_epilogue
+        const int j = ncol >> 1, seg = j >> 7, gg = (j & 127) >> 5, u = (j & 31) >> 3;
+        uint16_t* dst = p.act_packed + ((((size_t)seg * 4 + u) * mtiles + cur.mt) * 64 + gg * 16 + (row & 15)) * 8 + (j & 7);
+        uint16_t o[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          o[q] = silu_mul_bits<T>(T::to_f32(T::from_f32(v[2 * q])), T::to_f32(T::from_f32(v[2 * q + 1])));
+          if constexpr (!__is_same(T, Half)) o[q] = bf16_bits_to_f16_bits_sat(o[q]);
+        }
+        *reinterpret_cast<uint32_t*>(dst) = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
+      } else if (p.ksplit == 1 && !p.force_partial) {
+        *reinterpret_cast<u16x4*>(p.c + (size_t)row * p.N + ncol) = u16x4{T::from_f32(v[0]), T::from_f32(v[1]), T::from_f32(v[2]), T::from_f32(v[3])};
+      } else {
+        *reinterpret_cast<f32x4*>(p.partial + ((size_t)cur.by * p.M + row) * p.N + ncol) = f32x4{v[0], v[1], v[2], v[3]};
+      }
+    }
+    if (!more) break;
+    ++unit;
+    const bool other = nxt.mt != cur.mt || nxt.by != cur.by;
+    cur = nxt;
+    if (other) load_a(cur);
+    red = red == red2 ? red2 + FNW * 4 * 64 * 4 : red2;
+    if constexpr (NSEG & 1) {                // the next unit's first segment lies in the other buffer
+      sc2[0] = sc2[1];
+      zw[0] = zw[1];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) w[0][u][t] = w[1][u][t];
+    }
+  }
+}
+
 // Generic path (any group size that is a multiple of 32): per-segment loads.
 // VEC = dwords per lane per k-step (4 -> 64-column tile, 2 -> 32, 1 -> 16)
 // MT  = 16-row m-tiles (1 or 2)
@@ -708,11 +883,32 @@ static Wna16Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t gs, int64_t 
   return pl;
 }
 
+// Workgroups of wna16_experts_kernel where the grouped form runs on it: where there is room for more than a unit each (of the rows that the caller makes
+// room for an eighth or less may be there: one token of Mixtral has room for eight tiles and fills two).  us, wna16_gemm_kernel / this one, two
+// tiles of 14336 x 4096 14.8 / 14.5, four 27.2 / 22.9; of 4096 x 28672 27.0 / 24.8, 50.6 / 41.8.
+static int experts_grid(const Wna16Params& p, const Wna16Plan& pl) {
+  const int grid = 2 * device_cu_count() / 8 * 8;
+  return grid > 0 && pl.vec == 4 && pl.mt == 1 && pl.nseg >= 4 && (int64_t)(p.M / 16) * pl.ksplit * (p.N / 64) > grid ? grid : 0;
+}
+
 template <typename T, int VEC, int MT>
 static void launch_wna16(const Wna16Params& p_in, const Wna16Plan& pl, hipStream_t st) {
   const Wna16Params& p = p_in;
   dim3 grid((unsigned)(p.N / (16 * VEC)), (unsigned)pl.ksplit, (unsigned)((p.M + 16 * MT - 1) / (16 * MT)));
   if (pl.fast) {
+    if constexpr (VEC == 4 && MT == 1) {
+      if (const int wgs = p.expert_ids != nullptr ? experts_grid(p, pl) : 0; wgs > 0) {
+        const size_t lds = (size_t)2 * FNW * 4 * 64 * 4 * sizeof(float);
+#define APHRO_EXPERTS(NS) hipLaunchKernelGGL((wna16_experts_kernel<T, NS>), dim3((unsigned)wgs), dim3(FNW * 64), lds, st, p)
+        switch (pl.nseg) {
+          case 8: APHRO_EXPERTS(8); break;
+          case 7: APHRO_EXPERTS(7); break;
+          default: APHRO_EXPERTS(4); break;
+        }
+#undef APHRO_EXPERTS
+        return;
+      }
+    }
     if constexpr (VEC >= 2) {
       Wna16Params p = p_in;
       const unsigned per = pl.ksplit > 1 && 8 % pl.ksplit == 0 ? 8u / (unsigned)pl.ksplit : 0u;
