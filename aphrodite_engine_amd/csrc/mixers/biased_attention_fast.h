@@ -759,24 +759,31 @@ constexpr size_t p32_lds(int qt) { return 4 * P32_TILE + (size_t)2 * qt * 4 * p3
 // query heads of one kv head (QT = 4, 2, 1: as many as divide its heads), a wave 32 rows of one head.  Against dba_prefill_kernel a
 // fragment read from LDS feeds 32 columns instead of 16, K and V go from the cache to LDS without a stop in registers (V by whole rows,
 // its transpose is the transposing LDS read's), the temperature and the bias are one FMA on a score whose four biases are one aligned
-// LDS read, the output is rescaled only when some row's maximum moved, and one barrier a tile does.  Two workgroups share a CU.
+// LDS read, the output is rescaled only when some row's maximum moved, and one barrier a tile does.  Two workgroups of one group share a CU.
 // Workgroups are numbered over the row tiles that the segments have, not over the longest segment's times their number: decoded rows
 // beside a prompt portion cost none.
-// Bound by a tile's chain of steps (products, softmax, products, 2 us) more than by any unit: without its exponentials, its products or its
-// loads it is 5 to 30 % faster each.  us before / after: 16 heads on 4, 4096 rows with bias 327 / 157, without 317 / 135; 2000 rows
-// behind 1024 keys, window 1024 84 / 42, with cap and bias 151 / 98; 32 heads on 8, three segments of 900 to 1400 rows with gate 147 / 82,
-// eight of 9 rows 35 / 21; 48 rows 20 / 20 (the launch).  Loads by 64-bit addresses instead of buffer offsets: 160 for 157; loads between the
+// Bound by a tile's chain of steps (products, softmax, products: 2 us where a workgroup is alone on its CU, 1.1 where two share it) more than by any unit:
+// without its exponentials, its products or its loads it is 5 to 30 % faster each.  us before / after: 16 heads on 4, 4096 rows with bias 327 / 157,
+// without 317 / 135; 2000 rows behind 1024 keys, window 1024 84 / 42, with cap and bias 151 / 98; 32 heads on 8, three segments of 900 to 1400 rows
+// with gate 147 / 82, eight of 9 rows 35 / 21; 48 rows 20 / 20 (the launch).  Nothing in a step waits for the tile on its way before its products
+// are done (block table entries and biases are asked for ahead of it and looked at in the next step, q is waited for where hipcc sees it), lane
+// offsets of whole tiles are constants, the halves' maxima meet without LDS: 143 -> 127, 122 -> 103, 91 -> 79, 69 -> 67 for the first, second, fourth
+// and fifth of these, 32 heads on 8 of 8192 rows 591 -> 553.  GROUPS = 2: two such groups of waves take a row tile's key tiles in turn, each in
+// LDS of its own, and their sums meet at the end: half the chain (the launch says where).  The groups' own barriers, counted in LDS, in place of the
+// workgroup's: 3 % slower.  Loads by 64-bit addresses instead of buffer offsets: 160 for 157; loads between the
 // products: 170 to 208 (hipcc waits for them in front of the next LDS read).  V in the order [4 keys][16 bytes] of flash_attn.hip, for which four neighbouring
 // lanes read four rows: 192 for 164; fragments as hipcc orders them: 164 for 160; tiles begun at another key by every workgroup: no change.
-template <int QT, int FORM>
-__global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
+template <int QT, int FORM, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS, 2) void dba_prefill32_kernel(DBAParams p) {
   constexpr bool EXT = FORM == DBA_MASKED;
   constexpr int D = 128, R = p32_rows(QT), BP = p32_pitch(QT), NB = (QT * (R + 63) + 255) / 256;
   constexpr float LOG2E = 1.4426950408889634f;
-  extern __shared__ __attribute__((aligned(16))) unsigned char dba_smem[];
+  extern __shared__ __attribute__((aligned(16))) unsigned char dba_room[];
+  const int group = GROUPS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = threadIdx.x & 255;
+  unsigned char* const dba_smem = dba_room + group * p32_lds(QT);
   float* bias_lds = reinterpret_cast<float*>(dba_smem + 4 * P32_TILE);      // [2][QT][4 copies][BP]
   const int lane = threadIdx.x & 63, kh = lane >> 5, l31 = lane & 31;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);      // of the group's four
   // ---- head unit and rank among the row tiles (numbering over the XCDs: see dba_prefill_kernel) ------------------------------------
   int unit, rank;
   {
@@ -826,22 +833,40 @@ __global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
   const uint32_t span = (uint32_t)(in_block ? p.block_size : p.num_blocks * p.block_size) * row_bytes - kvh * D * 2;
   const unsigned char* kb = reinterpret_cast<const unsigned char*>(p.k_cache) + kvh * D * 2;
   const unsigned char* vb = reinterpret_cast<const unsigned char*>(p.v_cache) + kvh * D * 2;
-  // block of the wave's 16 keys of the tile at t0 where they share one (past the last key: the last key's)
-  auto block_of = [&](int t0) {
-    if (p.bs_shift < 4) return 0;
-    const int blk = bt[min(t0 + 16 * wave, (nk - 1) & ~15) >> p.bs_shift];
+  // block of the wave's 16 keys of the tile at t0 where they share one (past the last key: the last key's): the table's entry as it lies, looked at a
+  // tile later -- a look at once would wait for the tile on its way, which left ahead of it
+  auto entry_of = [&](int t0) { return p.bs_shift < 4 ? 0 : bt[min(t0 + 16 * wave, (nk - 1) & ~15) >> p.bs_shift]; };
+  auto block_of = [&](int entry) {
+    const int blk = __builtin_amdgcn_readfirstlane(entry);
     return blk < 0 || blk >= p.num_blocks ? 0 : blk;         // never read outside the pool
   };
-  auto fetch = [&](int buf, int t0, int blk, int j) {        // four keys of K and of V
-    const int key = min(t0 + 16 * wave + 4 * j + (lane >> 4), nk - 1);
-    const uint32_t at = (uint32_t)(in_block ? key & (p.block_size - 1) : dba_slot(p, bt, key)) * row_bytes;
+  // where the wave's 16 keys all exist, lane offsets are the same in every tile
+  const int lrow = lane >> 4, vlane = lrow * (int)row_bytes + (((lane & 15) ^ (lrow << 2)) << 4);
+  int klane[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) klane[j] = lrow * (int)row_bytes + (((lane & 15) ^ (4 * j + lrow)) << 4);
+  auto fetch = [&](int buf, int t0, int blk) {               // a tile's 16 keys of the wave, K and V
+    unsigned char* dst = dba_smem + buf * 2 * P32_TILE + wave * 4096;
     const int64_t base = in_block ? (int64_t)blk * p.block_size * row_bytes : 0;
-    unsigned char* dst = dba_smem + buf * 2 * P32_TILE + wave * 4096 + j * 1024;
-    const int ko = (int)(at + (((lane & 15) ^ (4 * j + (lane >> 4))) << 4)), vo = (int)(at + (((lane & 15) ^ ((lane >> 4) << 2)) << 4));
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(kb + base), 0, span, 0x00020000),
-                                             (dba_lds_ptr)dst, 16, ko, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(vb + base), 0, span, 0x00020000),
-                                             (dba_lds_ptr)(dst + P32_TILE), 16, vo, 0, 0, 0);
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(kb + base), 0, span, 0x00020000),
+                                 rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(vb + base), 0, span, 0x00020000);
+    if (in_block && t0 + 16 * wave + 16 <= nk) {
+      const uint32_t first = (uint32_t)((t0 + 16 * wave) & (p.block_size - 1)) * row_bytes;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (dba_lds_ptr)(dst + j * 1024), 16, klane[j], first + 4 * j * row_bytes, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (dba_lds_ptr)(dst + P32_TILE + j * 1024), 16, vlane, first + 4 * j * row_bytes, 0, 0);
+      }
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int key = min(t0 + 16 * wave + 4 * j + lrow, nk - 1);
+      const uint32_t at = (uint32_t)(in_block ? key & (p.block_size - 1) : dba_slot(p, bt, key)) * row_bytes;
+      const int ko = (int)(at + (((lane & 15) ^ (4 * j + lrow)) << 4)), vo = (int)(at + (((lane & 15) ^ (lrow << 2)) << 4));
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (dba_lds_ptr)(dst + j * 1024), 16, ko, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (dba_lds_ptr)(dst + P32_TILE + j * 1024), 16, vo, 0, 0, 0);
+    }
   };
   // ---- bias of a tile: entry x of a head's window is the distance (ctx + q0 - t0 + R - 1) - x; a row reads 4 neighbours at a time, and
   // the copy shifted by its own misalignment makes them 16 aligned bytes -----------------------------------------------------------------
@@ -849,19 +874,19 @@ __global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
   auto bias_load = [&](int t0) {
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      const int x = threadIdx.x + 256 * i, h = x / (R + 63), e = x - h * (R + 63);
+      const int x = tid + 256 * i, h = x / (R + 63), e = x - h * (R + 63);
       const int dist = ctx + q0 - t0 + R - 1 - e;
-      bias_reg[i] = h < QT ? p.bias_lut[(int64_t)(unit * QT + h) * p.lut_len + min(max(dist, 0), p.lut_len - 1)] * LOG2E : 0.f;
+      bias_reg[i] = p.bias_lut[(int64_t)(unit * QT + min(h, QT - 1)) * p.lut_len + min(max(dist, 0), p.lut_len - 1)];
     }
   };
   auto bias_store = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      const int x = threadIdx.x + 256 * i, h = x / (R + 63), e = x - h * (R + 63);
+      const int x = tid + 256 * i, h = x / (R + 63), e = x - h * (R + 63);
       if (h < QT)
 #pragma unroll
         for (int c = 0; c < 4; ++c)
-          if (e >= c) bias_lds[((buf * QT + h) * 4 + c) * BP + e - c] = bias_reg[i];
+          if (e >= c) bias_lds[((buf * QT + h) * 4 + c) * BP + e - c] = bias_reg[i] * LOG2E;
     }
   };
   const int bx = R - 1 - (qrow - q0), bias_at = (t * 4 + (bx & 3)) * BP + (bx & ~3) + 4 * kh;
@@ -875,28 +900,31 @@ __global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
   // transposing read of 4 keys x 16 columns by 16 lanes: lane i asks for 8 bytes of key i >> 2 and gets column i of the four keys
   const int vk = (lane & 15) >> 2;
   const int vaddr = P32_TILE + kh * 1024 + vk * 256 + (vk << 6) + (((lane >> 4) & 1) << 5) + ((lane & 3) << 3);
-  {
-    const int b0 = block_of(t_first);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) fetch(0, t_first, b0, j);
-  }
-  if (p.bias_lut) {
-    bias_load(t_first);
-    bias_store(0);
-  }
-  int blk = block_of(t_first + P32_BN), buf = 0;
-  for (int t0 = t_first; t0 < nk; t0 += P32_BN, buf ^= 1) {
-    // this wave's part of the tile is there, and it is through with the other buffer
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    const bool more = t0 + P32_BN < nk;
-    if (more) {                                              // in flight during this tile's products
-      if (p.bias_lut) bias_load(t0 + P32_BN);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) fetch(buf ^ 1, t0 + P32_BN, blk, j);
-      blk = block_of(t0 + 2 * P32_BN);
+  constexpr int STEP = P32_BN * GROUPS;                      // the groups take a row tile's key tiles in turn
+  const int g_first = t_first + P32_BN * group;
+  if (g_first < nk) {
+    fetch(0, g_first, block_of(entry_of(g_first)));
+    if (p.bias_lut) {
+      bias_load(g_first);
+      bias_store(0);
     }
-    if (t0 <= ctx + row0 + 31 && !(EXT && t0 + P32_BN <= lo_wave0)) {      // some key of the tile is seen by some row of the wave
+  }
+  int entry = entry_of(g_first + STEP), buf = 0;
+  for (int t0 = g_first; t0 - P32_BN * group < nk; t0 += STEP, buf ^= 1) {      // (as often in every group: the barrier is the workgroup's)
+    // this wave's part of the tile is there, and it is through with the other buffer
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);                      // vmcnt(0) lgkmcnt(0), where hipcc sees it: it waits for q once, not in every tile
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const bool more = t0 + STEP < nk;
+    if (more) {                                              // in flight during this tile's products
+      const int blk = block_of(entry);
+      entry = entry_of(t0 + 2 * STEP);
+      if (p.bias_lut) bias_load(t0 + STEP);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(buf ^ 1, t0 + STEP, blk);
+    }
+    if ((GROUPS == 1 || t0 < nk) && t0 <= ctx + row0 + 31 && !(EXT && t0 + P32_BN <= lo_wave0)) {      // some key of the tile is seen by some row of the wave
       const unsigned char* sb = dba_smem + buf * 2 * P32_TILE;
       // (the order is fixed by hand: left to itself hipcc reads one pair of fragments, waits for it, multiplies, and so on)
       f32x16 s[2];
@@ -972,7 +1000,12 @@ __global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[b][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      {                                                      // the other half's largest, without LDS
+        const uint32_t mb = __builtin_bit_cast(uint32_t, mx);
+        const auto sw = __builtin_amdgcn_permlane32_swap(mb, mb, false, false);
+        const uint32_t low = sw[0], high = sw[1];            // (hipcc takes element 0 for either where one is bit-cast in place)
+        mx = fmaxf(__builtin_bit_cast(float, low), __builtin_bit_cast(float, high));
+      }
       const float m_new = fmaxf(m_run, mx);
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;
@@ -1012,6 +1045,28 @@ __global__ __launch_bounds__(256, 2) void dba_prefill32_kernel(DBAParams p) {
     if (more && p.bias_lut) bias_store(buf ^ 1);
   }
   float l = l_run + __shfl_xor(l_run, 32, 64);
+  if constexpr (GROUPS > 1) {                                // the second group's sums join the first's
+    f32x4* const ro = reinterpret_cast<f32x4*>(dba_room + p32_lds(QT)) + wave * 16 * 64 + lane;
+    float* const rm = reinterpret_cast<float*>(dba_room + p32_lds(QT) + 4 * P32_TILE) + wave * 128 + lane;
+    __syncthreads();
+    if (group == 1) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ro[64 * i] = f32x4{o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1], o[i >> 2][4 * (i & 3) + 2], o[i >> 2][4 * (i & 3) + 3]};
+      rm[0] = m_run;
+      rm[64] = l;
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float m1 = rm[0], M = fmaxf(m_run, m1), a0 = __builtin_amdgcn_exp2f(m_run - M), a1 = __builtin_amdgcn_exp2f(m1 - M);
+    m_run = M;
+    l = l * a0 + rm[64] * a1;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const f32x4 x = ro[64 * i];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[i >> 2][4 * (i & 3) + r] = o[i >> 2][4 * (i & 3) + r] * a0 + x[r] * a1;
+    }
+  }
   if (qrow >= len) return;
   float f = (l > 0.f ? 1.f / l : 0.f) * p.out_scale;
   if (EXT && p.sink) {                                       // one more term of the denominator, without a value
@@ -1063,29 +1118,40 @@ static void launch_prefill_dk(const DBAParams& p, dim3 grid, hipStream_t st) {
   }
 }
 
-template <int QT, int FORM>
+template <int QT, int FORM, int GROUPS>
 static void launch_prefill32(const DBAParams& p0, int64_t num_tokens, int num_seqs, hipStream_t st) {
   DBAParams p = p0;
   constexpr int R = p32_rows(QT);
   const int64_t most = num_tokens / R + (num_tokens / p.min_len < num_seqs ? num_tokens / p.min_len : num_seqs);     // row tiles there can be
   const int64_t blocks = (most * (p.heads / QT) + 7) / 8 * 8;
-  p.snake = num_seqs == 1 && blocks <= 2 * device_cu_count();
+  p.snake = GROUPS == 1 && num_seqs == 1 && blocks <= 2 * device_cu_count();
+  constexpr size_t lds = GROUPS * p32_lds(QT);
   static bool attr_set_dev[APHRO_MAX_DEVICES] = {}; bool& attr_set = attr_set_dev[device_slot()];
   if (!attr_set)
-    attr_set = hipFuncSetAttribute((const void*)dba_prefill32_kernel<QT, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p32_lds(QT)) == hipSuccess;
-  hipLaunchKernelGGL((dba_prefill32_kernel<QT, FORM>), dim3((unsigned)blocks), dim3(256), p32_lds(QT), st, p);
+    attr_set = hipFuncSetAttribute((const void*)dba_prefill32_kernel<QT, FORM, GROUPS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+  hipLaunchKernelGGL((dba_prefill32_kernel<QT, FORM, GROUPS>), dim3((unsigned)blocks), dim3(256 * GROUPS), lds, st, p);
 }
 
 template <int FORM>
-void dba_prefill_launch(const DBAParams& p0, int64_t num_tokens, int max_q_len, int num_seqs, hipStream_t st) {
+void dba_prefill_launch(const DBAParams& p0, int64_t num_tokens, int max_q_len, int num_seqs, int max_keys, hipStream_t st) {
   // 16-byte loads into LDS want aligned caches (rows are 256 bytes times the kv heads); their 32-bit offsets a block below 4 GiB, or the
   // whole cache where blocks are no multiples of 16 keys
   const int64_t span = (p0.bs_shift >= 4 ? 1 : p0.num_blocks) * p0.block_size * (int64_t)p0.kv_heads * 256;
   if (p0.dim == 128 && p0.vdim == 128 && (((uintptr_t)p0.k_cache | (uintptr_t)p0.v_cache) & 15) == 0 && span < (1ll << 32)) {
     const int per_kv = p0.heads / p0.kv_heads;
-    if (per_kv % 4 == 0) launch_prefill32<4, FORM>(p0, num_tokens, num_seqs, st);
-    else if (per_kv % 2 == 0) launch_prefill32<2, FORM>(p0, num_tokens, num_seqs, st);
-    else launch_prefill32<1, FORM>(p0, num_tokens, num_seqs, st);
+    const int qt = per_kv % 4 == 0 ? 4 : per_kv % 2 == 0 ? 2 : 1;
+    // Two groups of waves a row tile where a launch lasts as long as its longest chain of key tiles: where the row tiles would leave every CU one workgroup
+    // at the most, or two of which one segment's have anything from one key tile to all (no window that evens them out).  us, one group / two: 16 heads
+    // on 4, 1000 rows with bias 32 / 26, 2000 behind 1024 keys with cap and bias 79 / 61, 4096 rows 103 / 85, 3000 behind 3000 147 / 145, under a
+    // window of 1024 50 / 53; 32 heads on 8, 1200 rows 40 / 30, 2500 85 / 90, three segments of 700 33 / 36.
+    const int64_t tiles = (num_tokens + p32_rows(qt) - 1) / p32_rows(qt) * (p0.heads / qt), cus = device_cu_count();
+    const bool spread = 2 * (int64_t)max_q_len > num_tokens && (p0.window == 0 || 2 * (int64_t)p0.window > max_q_len) && (p0.chunk == 0 || 2 * (int64_t)p0.chunk > max_q_len);
+    const bool two = max_keys >= 256 && (tiles <= cus || (tiles <= 2 * cus && spread));
+#define P32(QT) (two ? launch_prefill32<QT, FORM, 2>(p0, num_tokens, num_seqs, st) : launch_prefill32<QT, FORM, 1>(p0, num_tokens, num_seqs, st))
+    if (qt == 4) P32(4);
+    else if (qt == 2) P32(2);
+    else P32(1);
+#undef P32
     return;
   }
   DBAParams p = p0;
