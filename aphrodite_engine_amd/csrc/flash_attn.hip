@@ -729,24 +729,13 @@ extern "C" int aphro_context_attention(void* out, const void* q, const void* k, 
 }
 
 
-// One dispatcher for the prefill kernels (p fully set up except nqt_max / xcd_remap): head 128 without a sliding window runs on 32 x 32 tiles
-// (flash_attn_v4.hip, flash_attn_short.hip); second generation for head 64 and windowed head 128 from 512 query rows on (with a context from
+// One dispatcher for the prefill kernels: head 128 without a sliding window runs on 32 x 32 tiles (flash_attn_short.hip); second generation for head 64 and windowed head 128 from 512 query rows on (with a context from
 // 128, its 64-key tiles are what the gathered-context path wants); first generation for the rest.
 static int fa_dispatch(FAParams p, int head_size, int dtype, int batch, int max_query_len, int max_key_len, hipStream_t st) {
-  if (head_size == 128 && p.window <= 0) {
-    // fourth generation (one wave per SIMD, two 32-row blocks per wave) from 4096 keys on; APHRO_FA_V4_MIN_KEYS=<n>: threshold
-    if (max_key_len >= 1024 && max_key_len >= knobs().fa_v4_min_keys) {
-      p.nqt_max = (max_query_len + 255) / 256;
-      p.xcd_remap = (batch * p.num_kv_heads) % 8 == 0 && !knobs().fa_no_xcd;
-      return fa_v4_launch(p, dtype, batch, st);
-    }
-    p.nqt_max = 0; p.xcd_remap = 0;
-    if (fa_short_launch(p, dtype, batch, max_query_len, max_key_len, st)) {
-      APHRO_LAUNCH_CHECK();
-      return APHRO_OK;
-    }
+  if (head_size == 128 && fa_short_launch(p, dtype, batch, max_query_len, max_key_len, st)) {
+    APHRO_LAUNCH_CHECK();
+    return APHRO_OK;
   }
-  p.nqt_max = 0; p.xcd_remap = 0;
   // two 16-row query tiles per wave (128-row workgroups) once the sequences are long enough to
   // fill the chip with them; head 256 keeps one tile (registers)
   const bool offset_keys = p.cu_seqlens_k != nullptr;
@@ -856,7 +845,7 @@ static int fa_varlen_entry(void* out, const void* q, const void* k, const void* 
   p.num_heads = num_heads; p.num_kv_heads = num_kv_heads;
   p.q_stride = q_stride; p.k_stride = k_stride; p.v_stride = v_stride;
   p.scale = scale; p.causal = causal;
-  p.cu_seqlens_k = nullptr; p.o_stride = (int64_t)num_heads * head_size; p.nqt_max = 0; p.xcd_remap = 0;
+  p.cu_seqlens_k = nullptr; p.o_stride = (int64_t)num_heads * head_size;
   p.window = window > 0 ? window : 0;
   return fa_dispatch(p, head_size, dtype, batch, max_seqlen, max_seqlen, (hipStream_t)stream);
 }

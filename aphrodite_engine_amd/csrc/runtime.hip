@@ -22,7 +22,6 @@ static Knobs read_knobs() {
   Knobs k;
   k.pa_splits = env_i("APHRO_PA_SPLITS", 0);
   k.fa_v4_min_keys = env_i("APHRO_FA_V4_MIN_KEYS", 4096);
-  k.fa_no_xcd = env_i("APHRO_FA_NO_XCD", 0);
   k.fp8_stream_all = env_i("APHRO_FP8_STREAM_ALL", 0);
   k.wna16_stream = env_i("APHRO_WNA16_STREAM", 1);
   k.wna16_op_no_resident = env_i("APHRO_WNA16_OP_NO_RESIDENT", 0);

@@ -1,6 +1,6 @@
 #!/bin/bash
-# The kernel sources WITH their lab branches (per-wave stamps, timing-only ablations, schedule variants: PA_LAB, FA4_LAB,
-# F8_LAB, ABL_*, LMH_*, FA_TRAIL, ...) -- removed from the product tree in round 6 -- as a scratch copy under tools/bin/csrc_lab/:
+# The kernel sources WITH their lab branches (per-wave stamps, timing-only ablations, schedule variants: PA_LAB,
+# F8_LAB, ABL_*, LMH_*, ...) -- removed from the product tree in round 6 -- as a scratch copy under tools/bin/csrc_lab/:
 # the product sources + tools/lab_patches/*.patch.  The torch-free harnesses (tools/*.hip) and lab library builds include / compile
 # from there:   bash tools/apply_lab_patches.sh && make -C tools/bin/csrc_lab LAB=1 EXTRA=-DPA_LAB ...
 set -e
