@@ -248,6 +248,27 @@ F16, BF16, F32 = 0, 1, 2
 WEIGHTS_STREAMED, WEIGHTS_CACHED = 0x100, 0x200          # or-ed into a dtype
 KV_AUTO, KV_FP8_E4M3, KV_FP8_E5M2 = 0, 1, 2
 
+ENTRY_CALLS_PATH = os.path.join(_HERE, "lib", "aphrodite_entry_calls.so")
+
+
+def _bind_calls(l, signatures) -> None:
+    """Functions of ``l`` as Python functions that convert their arguments by the declared types (csrc_torch/entry_calls.cpp), in place of ctypes'
+    own calls, which stay for whatever is not a plain number, for names that it does not have, and where it is not built."""
+    if not os.path.exists(ENTRY_CALLS_PATH):
+        return
+    import importlib.machinery
+    import importlib.util
+    name = "aphrodite_entry_calls"
+    loader = importlib.machinery.ExtensionFileLoader(name, ENTRY_CALLS_PATH)
+    calls = importlib.util.module_from_spec(importlib.util.spec_from_file_location(name, ENTRY_CALLS_PATH, loader=loader))
+    loader.exec_module(calls)
+    for name in signatures:
+        fn = getattr(l, name)
+        call = calls.bind(name, ctypes.cast(fn, c_void_p).value, fn)
+        if call is not None:
+            setattr(l, name, call)
+
+
 _lib = None
 
 
@@ -269,6 +290,7 @@ def lib():
             raise ImportError(f"{LIB_PATH} does not export {name}") from e
         fn.restype = res
         fn.argtypes = args
+    _bind_calls(l, SIGNATURES)
     _lib = l
     return l
 
@@ -303,6 +325,7 @@ def mixers_lib():
             raise ImportError(f"{MIXERS_LIB_PATH} does not export {name}") from e
         fn.restype = res
         fn.argtypes = args
+    _bind_calls(l, MIXERS_SIGNATURES)
     _mixers = l
     return l
 
