@@ -28,15 +28,16 @@ __device__ __forceinline__ int wave_incl_sum(int v, int lane) {
   return v;
 }
 
-__device__ __forceinline__ int chunks_of(int n, int min_len) { return n >= min_len ? (n + CHUNK - 1) / CHUNK : 0; }
+// (In what follows a unit is a chunk, or a group of chunks of one segment.)
+__device__ __forceinline__ int chunks_of(int n, int min_len, int unit = CHUNK) { return n >= min_len ? (n + unit - 1) / unit : 0; }
 
 // Chunk ``id`` of the batch's segments of at least min_len tokens, counted in order -> segment s and chunk c of it; false: there are
 // fewer.  Every wave of a workgroup works it out for itself (64 segments a step).
-__device__ __forceinline__ bool locate_chunk(int id, const int32_t* __restrict__ q_len, int num_seqs, int min_len, int& s, int& c) {
+__device__ __forceinline__ bool locate_chunk(int id, const int32_t* __restrict__ q_len, int num_seqs, int min_len, int& s, int& c, int unit = CHUNK) {
   const int lane = threadIdx.x & 63;
   int before = 0;
   for (int s0 = 0; s0 < num_seqs; s0 += 64) {
-    const int cnt = s0 + lane < num_seqs ? chunks_of(q_len[s0 + lane], min_len) : 0;
+    const int cnt = s0 + lane < num_seqs ? chunks_of(q_len[s0 + lane], min_len, unit) : 0;
     const int incl = wave_incl_sum(cnt, lane) + before;
     const uint64_t past = __ballot(incl > id);
     if (past) {
@@ -51,17 +52,17 @@ __device__ __forceinline__ bool locate_chunk(int id, const int32_t* __restrict__
 }
 
 // Number of chunks ahead of segment s.
-__device__ __forceinline__ int chunks_before(int s, const int32_t* __restrict__ q_len, int min_len) {
+__device__ __forceinline__ int chunks_before(int s, const int32_t* __restrict__ q_len, int min_len, int unit = CHUNK) {
   const int lane = threadIdx.x & 63;
   int sum = 0;
-  for (int s0 = 0; s0 < s; s0 += 64) sum += __shfl(wave_incl_sum(s0 + lane < s ? chunks_of(q_len[s0 + lane], min_len) : 0, lane), 63, 64);
+  for (int s0 = 0; s0 < s; s0 += 64) sum += __shfl(wave_incl_sum(s0 + lane < s ? chunks_of(q_len[s0 + lane], min_len, unit) : 0, lane), 63, 64);
   return __builtin_amdgcn_readfirstlane(sum);
 }
 
 // The most chunks that num_tokens rows in num_seqs segments can hold.
-inline int64_t max_chunks(int64_t num_tokens, int num_seqs, int min_len) {
+inline int64_t max_chunks(int64_t num_tokens, int num_seqs, int min_len, int unit = CHUNK) {
   const int64_t longs = num_tokens / min_len;
-  return num_tokens / CHUNK + (longs < num_seqs ? longs : num_seqs);
+  return num_tokens / unit + (longs < num_seqs ? longs : num_seqs);
 }
 
 // A call's chunks run in spans of as many as the workspace holds, the state between them in the state tensors (fp32, as the chunks carry it: the
@@ -69,8 +70,8 @@ inline int64_t max_chunks(int64_t num_tokens, int num_seqs, int min_len) {
 // the segment's chunk 0 would lie in the span's arrays.
 constexpr int64_t SPAN_BYTES = 256 << 20;       // 38 chunks of 32 heads of the delta rule's 128 x 128, the widest: enough for the chip.  16384 tokens in spans
 // against all at once: delta rule 16 / 32 heads 1712 / 2687 -> 1748 / 2682 us, state space of 64 heads 1227 -> 1310 us
-__device__ __forceinline__ bool span_of(int s, int nc, const int32_t* __restrict__ q_len, int min_len, int chunk0, int span, int& begin, int& end, int64_t& first) {
-  const int64_t rel = (int64_t)chunks_before(s, q_len, min_len) - chunk0;
+__device__ __forceinline__ bool span_of(int s, int nc, const int32_t* __restrict__ q_len, int min_len, int chunk0, int span, int& begin, int& end, int64_t& first, int unit = CHUNK) {
+  const int64_t rel = (int64_t)chunks_before(s, q_len, min_len, unit) - chunk0;
   first = rel;
   begin = rel < 0 ? (int)-rel : 0;
   end = rel + nc > span ? (int)(span - rel) : nc;

@@ -13,9 +13,8 @@
 // What bounds it: the fp32 products (the matrix pipe is busy half of the time in launches 1 and 3) and the states between the chunks
 // (written once, read and written once, read once: dim x vdim x 4 bytes a chunk and head).  A scan is bound by the latency of its
 // token chain.  One portion of 4096 tokens, scan -> chunks: decay 8 x 64 x 128 1106 -> 60 us, mLSTM 4 x 128 x 256 2170 -> 113 us, state
-// space 64 x 128 x 64 1476 -> 274 us (128 heads: 1482 -> 575 us).  With mLSTM's and the state space's bf16 inputs on the 16-bit units (the *16
-// kernels): mLSTM 4096 tokens 112 -> 95 us, state space 2000 tokens 146 -> 111, three portions of 300, 128 heads 171 -> 137; error against 64
-// bits 4.8e-7 -> 2.5e-7 and 1.05e-7 -> 0.94e-7.
+// space 64 x 128 x 64 1476 -> 274 us (128 heads: 1482 -> 575 us).  mLSTM's and the state space's bf16 inputs go to the 16-bit units, several chunks of a
+// segment to a workgroup (the *16 kernels).
 // Outputs lie as the products leave them: scores as K Q^T and results as V^T P^T, so that a score's registers are the next product's
 // operand and a lane holds four neighbouring value columns of one token.  Row pitches are 4 floats over a multiple of 32: the
 // eight lanes that a 16-byte LDS access serves at a time fall on all 32 banks.
@@ -30,6 +29,7 @@ constexpr int OMC_PITCH = CHUNK + 4;
 struct OMChunk {
   OuterMemory p;
   int min_len;            // segments shorter than this are the scan's
+  int group;              // chunks that a workgroup takes in turn (bf16 inputs' kernels; 1 elsewhere): below, and where states are numbered, a chunk is a group of so many
   int chunk0, span;       // the chunks of these launches (below: [chunks] of one span)
   int vpad;               // vdim rounded up to 16
   float* u;               // [chunks, heads, vpad, DP] U, then the state ahead of the chunk
@@ -216,104 +216,207 @@ __global__ __launch_bounds__(256) void om_chunk_update_kernel(OMChunk a) {
   }
 }
 
-// The same where keys and values enter as the bf16 numbers they are (mLSTM, state space): U = sum_j k_j (w_j v_j)^T with the second factor in
-// three bf16 parts.  Keys that are not finite would meet a part that is zero: such a chunk multiplies in fp32, from the same LDS.
-template <int MODE, int DP, bool VEC>
-__global__ __launch_bounds__(256) void om_chunk_update16_kernel(OMChunk a) {
-  constexpr int PITCH = CHUNK + 8;
-  __shared__ __attribute__((aligned(16))) uint16_t kt[DP * PITCH];
-  __shared__ __attribute__((aligned(16))) uint16_t vt[3][OMC_COLS * PITCH];
-  __shared__ float ws[CHUNK];
-  const OuterMemory& p = a.p;
-  int s, c;
-  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
-  const int slot = p.slot_of_seq[s];
-  if (slot < 0 || slot >= p.num_slots) return;
-  const int h = blockIdx.y, c0 = blockIdx.z * OMC_COLS, hk = MODE == 2 ? h / (p.heads / p.qk_heads) : h;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int cnt = min(CHUNK, p.q_len[s] - c * CHUNK);
-  const int64_t row0 = (int64_t)p.q_start[s] + c * CHUNK;
-  const int64_t row = row0 + min(lane, cnt - 1);
-  const uint16_t* kr = (const uint16_t*)p.k + row * p.k_stride + (int64_t)hk * p.dim;
-  const uint16_t* vr = (const uint16_t*)p.v + row * p.v_stride + (int64_t)h * p.vdim + c0;
-  u16x8 kx[DP / 32], vx[OMC_COLS / 32];
+// The same where keys, queries and values enter as the bf16 numbers they are (mLSTM, state space), a workgroup taking a.group chunks of a segment in
+// turn: the states that go through memory are those between groups.  Products are on the 16-bit units, one factor in three bf16 parts.  A wave owns 16 value
+// columns: what it multiplies its state and its values with (queries, keys, weights) comes from LDS, the state stays in its registers -- a lane has, of
+// one column, the eight neighbouring rows 32 kk + 8 lg + (0..7), which are its part of the next product's operand as they lie (the keys' rows lie in
+// LDS in the order that gives this: key_row).  Numbers that are not finite would meet a part that is zero: a chunk with any multiplies in fp32.
+// What bounds it: the vector units (splits, weights, the copy to LDS: some 1200 instructions a wave and chunk beside 130 matrix ones).  Against a workgroup
+// a chunk, whose states (32 KB each) made 250 of the 370 MB that 64 heads and 2000 tokens moved and whose state products were fp32: state space 64 heads
+// 2000 tokens 111 -> 74 us, 4096 216 -> 117, 128 heads 4096 499 -> 211, mLSTM 4 x 128 x 256 4096 95 -> 66; error against 64 bits of outputs 1.6e-7 ->
+// 1.2e-7, of states 8.4e-8 -> 8.3e-8.  Without branches at the use of
+// every number that may not be finite, and with masks and bits two at a time: 90 -> 74 at the first of these.
+constexpr int OMG_PITCH = CHUNK + 8;
+constexpr __device__ __forceinline__ int key_row(int d) { return (d & ~31) | ((d & 4) << 2) | ((d & 24) >> 1) | (d & 3); }
+// Is a number not finite?  The largest of the bits without sign, two a step.
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void largest_bits(u16x2& m, u32x4 w) {
 #pragma unroll
-  for (int it = 0; it < DP / 32; ++it) kx[it] = load8_bits<VEC>(kr, wave * (DP / 4) + it * 8, p.dim);
+  for (int i = 0; i < 4; ++i) m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w[i] & 0x7fff7fffu));
+}
+__device__ __forceinline__ bool odd_bits(u16x2 m) { return max(m[0], m[1]) >= 0x7f80; }
+// Eight neighbouring rows of a lane's token into LDS; row(i) is the place of the i-th.
+template <typename F>
+__device__ __forceinline__ void put_rows(uint16_t* at, u32x4 w, F row) {
 #pragma unroll
-  for (int it = 0; it < OMC_COLS / 32; ++it) vx[it] = load8_bits<VEC>(vr, wave * (OMC_COLS / 4) + it * 8, p.vdim - c0);
-  double la;
-  float b;
-  chunk_gate<BFloat, MODE>(a, h, row0, lane, cnt, la, b);
-  const double g = wave_incl_sum(la, lane), gend = __shfl(g, 63, 64);
-  const float w = exp2_d(gend - g) * b, all = exp2_d(gend);
-  if (blockIdx.z == 0 && tid == 0) a.total[(int64_t)blockIdx.x * p.heads + h] = all;
-  if (tid < CHUNK) ws[tid] = lane < cnt ? w : 0.f;
-  bool odd = false;                                                      // a key that is not finite
+  for (int i = 0; i < 4; ++i) {
+    at[row(2 * i) * OMG_PITCH] = (uint16_t)w[i];
+    at[row(2 * i + 1) * OMG_PITCH] = (uint16_t)(w[i] >> 16);
+  }
+}
+// split3 of eight finite numbers.
+__device__ __forceinline__ void split3_finite(const float (&x)[8], u16x8 (&part)[3]) {
+  u32x4 h, m, l;
 #pragma unroll
-  for (int it = 0; it < DP / 32; ++it)
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t a0 = __builtin_bit_cast(uint32_t, x[2 * i]), b0 = __builtin_bit_cast(uint32_t, x[2 * i + 1]);
+    const float ra = x[2 * i] - __builtin_bit_cast(float, a0 & 0xffff0000u), rb = x[2 * i + 1] - __builtin_bit_cast(float, b0 & 0xffff0000u);
+    const uint32_t a1 = __builtin_bit_cast(uint32_t, ra), b1 = __builtin_bit_cast(uint32_t, rb);
+    const float la = ra - __builtin_bit_cast(float, a1 & 0xffff0000u), lb = rb - __builtin_bit_cast(float, b1 & 0xffff0000u);
+    h[i] = __builtin_amdgcn_perm(b0, a0, 0x07060302u);
+    m[i] = __builtin_amdgcn_perm(b1, a1, 0x07060302u);
+    l[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, lb), __builtin_bit_cast(uint32_t, la), 0x07060302u);
+  }
+  part[0] = __builtin_bit_cast(u16x8, h), part[1] = __builtin_bit_cast(u16x8, m), part[2] = __builtin_bit_cast(u16x8, l);
+}
+// A wave's state S (rows 32 kk + 8 lg + 4 hf + r of its column) after a chunk: S decays by ``all`` and takes the chunk's tokens, values weighted by ws.  The
+// tokens' sum starts from zero and meets S once: added to S product by product, S was rounded six times a chunk (error against 64 bits 1.01e-7 for 0.85e-7).
+template <int DP>
+__device__ __forceinline__ void group_update(f32x4 (&S)[DP / 32][2], const uint16_t* kt, const u16x8 (&v)[CHUNK / 32], const float* ws, float all, bool odd, int li, int lg) {
+  float x[CHUNK / 32][8], z = 0.f;                                       // (z is not zero: a weighted value that is not finite)
+#pragma unroll
+  for (int jj = 0; jj < CHUNK / 32; ++jj) {
+    const f32x4 w0 = *reinterpret_cast<const f32x4*>(&ws[32 * jj + 8 * lg]), w1 = *reinterpret_cast<const f32x4*>(&ws[32 * jj + 8 * lg + 4]);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const uint16_t x = lane < cnt ? kx[it][i] : (uint16_t)0;
-      odd |= (x & 0x7f80u) == 0x7f80u;
-      kt[(wave * (DP / 4) + it * 8 + i) * PITCH + lane] = x;
+      x[jj][i] = BFloat::to_f32(v[jj][i]) * (i < 4 ? w0[i] : w1[i - 4]);
+      z = fmaf(x[jj][i], 0.f, z);
     }
+  }
+  const uint16_t* kr = kt + li * OMG_PITCH + 8 * lg;
+  f32x4 U[DP / 16] = {};
+  if (odd || __any(z != 0.f)) {
 #pragma unroll
-  for (int it = 0; it < OMC_COLS / 32; ++it)
+    for (int jj = 0; jj < CHUNK / 32; ++jj)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      uint16_t part[3];
-      split3(lane < cnt ? BFloat::to_f32(vx[it][i]) * w : 0.f, part);
+      for (int kk = 0; kk < DP / 16; ++kk) {
+        const u16x8 av = *reinterpret_cast<const u16x8*>(&kr[kk * 16 * OMG_PITCH + 32 * jj]);
 #pragma unroll
-      for (int n = 0; n < 3; ++n) vt[n][(wave * (OMC_COLS / 4) + it * 8 + i) * PITCH + lane] = part[n];
-    }
-  odd = __syncthreads_or(odd);
-  const int li = lane & 15, lg = lane >> 4;
-  const int nct = min(OMC_COLS / 16, (p.vdim - c0 + 15) >> 4);
-  constexpr int DT = DP / 64;                              // 16-row tiles of a wave
-  f32x4 acc[DT][OMC_COLS / 16] = {};
+        for (int m = 0; m < 8; ++m) U[kk] = mfma4(BFloat::to_f32(av[m]), x[jj][m], U[kk]);
+      }
+  } else {
+    u16x8 high[CHUNK / 32];                                              // the first parts: last, when the small ones are in
 #pragma unroll
-  for (int kk = 0; kk < CHUNK / 32; ++kk) {
-    u16x8 av[DT];
+    for (int jj = 0; jj < CHUNK / 32; ++jj) {
+      u16x8 part[3];
+      split3_finite(x[jj], part);
+      high[jj] = part[0];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) av[dt] = *reinterpret_cast<const u16x8*>(&kt[((wave * DT + dt) * 16 + li) * PITCH + 32 * kk + 8 * lg]);
+      for (int kb = 0; kb < DP / 16; kb += 4) {
+        u16x8 av[4];
 #pragma unroll
-    for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
-      if (ct >= nct) break;
-      u16x8 bv[3];
+        for (int kk = 0; kk < 4; ++kk) av[kk] = *reinterpret_cast<const u16x8*>(&kr[(kb + kk) * 16 * OMG_PITCH + 32 * jj]);
 #pragma unroll
-      for (int n = 0; n < 3; ++n) bv[n] = *reinterpret_cast<const u16x8*>(&vt[n][(ct * 16 + li) * PITCH + 32 * kk + 8 * lg]);
-      if (!odd) {
+        for (int n = 2; n >= 1; --n)
 #pragma unroll
-        for (int n = 2; n >= 0; --n)
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) acc[dt][ct] = mfma16(av[dt], bv[n], acc[dt][ct]);
-      } else {
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-          const float x = (BFloat::to_f32(bv[2][m]) + BFloat::to_f32(bv[1][m])) + BFloat::to_f32(bv[0][m]);
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) acc[dt][ct] = mfma4(BFloat::to_f32(av[dt][m]), x, acc[dt][ct]);
-        }
+          for (int kk = 0; kk < 4; ++kk) U[kb + kk] = mfma16(av[kk], part[n], U[kb + kk]);
       }
     }
+#pragma unroll
+    for (int jj = 0; jj < CHUNK / 32; ++jj)
+#pragma unroll
+      for (int kk = 0; kk < DP / 16; ++kk) U[kk] = mfma16(*reinterpret_cast<const u16x8*>(&kr[kk * 16 * OMG_PITCH + 32 * jj]), high[jj], U[kk]);
   }
-  float* u = a.u + (((int64_t)blockIdx.x * p.heads + h) * a.vpad + c0) * DP;
 #pragma unroll
-  for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
-    if (ct >= nct) break;
+  for (int kk = 0; kk < DP / 16; ++kk)
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-      *reinterpret_cast<f32x4*>(&u[(ct * 16 + li) * DP + (wave * DT + dt) * 16 + 4 * lg]) = acc[dt][ct];
+    for (int r = 0; r < 4; ++r) S[kk >> 1][kk & 1][r] = fmaf(all, S[kk >> 1][kk & 1][r], U[kk][r]);
+}
+// The normaliser's number of key row tid.
+__device__ __forceinline__ float group_update_n(float sum, const uint16_t* kt, const float* ws, float all, int tid) {
+  float add = 0.f;
+  for (int t = 0; t < CHUNK; t += 8) {
+    const u16x8 x = *reinterpret_cast<const u16x8*>(&kt[key_row(tid) * OMG_PITCH + t]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) add += BFloat::to_f32(x[i]) * ws[t + i];
   }
-  if (MODE == 1 && blockIdx.z == 0 && tid < DP) {
-    float sum = 0.f;
-    for (int t = 0; t < CHUNK; t += 8) {
-      const u16x8 x = *reinterpret_cast<const u16x8*>(&kt[tid * PITCH + t]);
+  return all * sum + add;
+}
+// What a workgroup of the two kernels below works on.  Workgroups that read the same keys and queries -- the heads of a key head, the column blocks of
+// a head -- follow each other on one XCD, whose L2 then holds them; pairs of group and key head go round the XCDs.
+struct OMGroup {
+  int x, h, hk, c0, chunks, tokens;    // group's number in the launch, head, key head, first column, chunks and tokens of the group
+  int64_t row0;                        // its first token
+};
+__host__ __device__ __forceinline__ int om_key_heads(const OuterMemory& p) { return p.mode == 2 ? p.qk_heads : p.heads; }
+__device__ __forceinline__ bool locate_group(const OMChunk& a, OMGroup& w) {
+  const OuterMemory& p = a.p;
+  const int key_heads = om_key_heads(p), heads = p.heads / key_heads, blocks = (p.vdim + OMC_COLS - 1) / OMC_COLS;
+  const int idx = blockIdx.x >> 3, pair = idx / (heads * blocks) * 8 + (blockIdx.x & 7), sub = idx % (heads * blocks);
+  if (pair >= a.span * key_heads) return false;
+  w.x = pair % a.span, w.hk = pair / a.span, w.h = w.hk * heads + sub / blocks, w.c0 = sub % blocks * OMC_COLS;
+  int s, g;
+  if (!locate_chunk(a.chunk0 + w.x, p.q_len, p.num_seqs, a.min_len, s, g, a.group * CHUNK)) return false;
+  const int slot = p.slot_of_seq[s], first = g * a.group * CHUNK;
+  if (slot < 0 || slot >= p.num_slots) return false;
+  w.tokens = min(a.group * CHUNK, p.q_len[s] - first);
+  w.chunks = (w.tokens + CHUNK - 1) / CHUNK;
+  w.row0 = (int64_t)p.q_start[s] + first;
+  return true;
+}
+
+template <int MODE, int DP, bool VEC>
+__global__ __launch_bounds__(256) void om_chunk_update16_kernel(OMChunk a) {
+  __shared__ __attribute__((aligned(16))) uint16_t kt[DP * OMG_PITCH];
+  __shared__ __attribute__((aligned(16))) uint16_t vt[OMC_COLS * OMG_PITCH];
+  __shared__ __attribute__((aligned(16))) float ws[4][CHUNK];
+  __shared__ float alls[4];
+  const OuterMemory& p = a.p;
+  OMGroup g;
+  if (!locate_group(a, g)) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, lg = lane >> 4;
+  const int nct = min(OMC_COLS / 16, (p.vdim - g.c0 + 15) >> 4);
+  const uint16_t* kb = (const uint16_t*)p.k + (int64_t)g.hk * p.dim;
+  const uint16_t* vb = (const uint16_t*)p.v + (int64_t)g.h * p.vdim + g.c0;
+  const u32x4 zeros = {};
+  u32x4 kx[DP / 32], vx[OMC_COLS / 32];
+  auto fetch = [&](int c) {                                              // lane = token; the waves divide the key rows and the columns
+    const int64_t row = g.row0 + min(c * CHUNK + lane, g.tokens - 1);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sum += BFloat::to_f32(x[i]) * ws[t + i];
+    for (int it = 0; it < DP / 32; ++it) kx[it] = __builtin_bit_cast(u32x4, load8_bits<VEC>(kb + row * p.k_stride, wave * (DP / 4) + it * 8, p.dim));
+#pragma unroll
+    for (int it = 0; it < OMC_COLS / 32; ++it) vx[it] = __builtin_bit_cast(u32x4, load8_bits<VEC>(vb + row * p.v_stride, wave * (OMC_COLS / 4) + it * 8, p.vdim - g.c0));
+  };
+  fetch(0);
+  f32x4 S[DP / 32][2] = {};
+  float sn = 0.f;
+  float total = 1.f;
+  for (int c = 0; c < g.chunks; ++c) {
+    if ((c & 3) == 0) {                                                  // the gates of four chunks, one a wave
+      double la;
+      float b;
+      chunk_gate<BFloat, MODE>(a, g.h, g.row0 + (c + wave) * CHUNK, lane, g.tokens - (c + wave) * CHUNK, la, b);
+      const double gi = wave_incl_sum(la, lane), gend = __shfl(gi, 63, 64);
+      ws[wave][lane] = exp2_d(gend - gi) * b;
+      if (lane == 0) alls[wave] = exp2_d(gend);
     }
-    a.un[((int64_t)blockIdx.x * p.heads + h) * DP + tid] = sum;
+    if ((c + 1) * CHUNK > g.tokens && c * CHUNK + lane >= g.tokens) {
+#pragma unroll
+      for (int it = 0; it < DP / 32; ++it) kx[it] = zeros;
+#pragma unroll
+      for (int it = 0; it < OMC_COLS / 32; ++it) vx[it] = zeros;
+    }
+    u16x2 top = {};
+#pragma unroll
+    for (int it = 0; it < DP / 32; ++it) {
+      largest_bits(top, kx[it]);
+      put_rows(kt + lane, kx[it], [&](int i) { return key_row(wave * (DP / 4) + it * 8 + i); });
+    }
+#pragma unroll
+    for (int it = 0; it < OMC_COLS / 32; ++it)
+      put_rows(vt + lane, vx[it], [&](int i) { return wave * (OMC_COLS / 4) + it * 8 + i; });
+    bool odd = odd_bits(top);
+    odd = __builtin_amdgcn_readfirstlane(__syncthreads_or(odd));
+    if (c + 1 < g.chunks) fetch(c + 1);
+    total *= alls[c & 3];
+    if (wave < nct) {
+      u16x8 v[CHUNK / 32];
+#pragma unroll
+      for (int jj = 0; jj < CHUNK / 32; ++jj) v[jj] = *reinterpret_cast<const u16x8*>(&vt[(wave * 16 + li) * OMG_PITCH + 32 * jj + 8 * lg]);
+      group_update<DP>(S, kt, v, ws[c & 3], alls[c & 3], odd, li, lg);
+    }
+    if (MODE == 1 && g.c0 == 0 && tid < DP) sn = group_update_n(sn, kt, ws[c & 3], alls[c & 3], tid);
+    lds_barrier();
   }
+  const int64_t at = (int64_t)g.x * p.heads + g.h;
+  if (g.c0 == 0 && tid == 0) a.total[at] = total;
+  if (MODE == 1 && g.c0 == 0 && tid < DP) a.un[at * DP + tid] = sn;
+  if (wave >= nct) return;
+  float* u = a.u + (at * a.vpad + g.c0 + wave * 16 + li) * DP + 8 * lg;
+#pragma unroll
+  for (int kk = 0; kk < DP / 32; ++kk)
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) *reinterpret_cast<f32x4*>(u + 32 * kk + 4 * hf) = S[kk][hf];
 }
 
 // ---- 2. the state through the chunks -------------------------------------------------------------------------------------------------
@@ -327,7 +430,8 @@ __global__ __launch_bounds__(64) void om_chunk_carry_kernel(OMChunk a) {
   if (n < a.min_len || slot < 0 || slot >= p.num_slots) return;
   int begin, nc;
   int64_t first;
-  if (!span_of(s, (n + CHUNK - 1) / CHUNK, p.q_len, a.min_len, a.chunk0, a.span, begin, nc, first)) return;
+  const int unit = a.group * CHUNK;
+  if (!span_of(s, (n + unit - 1) / unit, p.q_len, a.min_len, a.chunk0, a.span, begin, nc, first, unit)) return;
   const bool fresh = begin == 0 && p.ctx_len[s] == 0;
   first += begin, nc -= begin;                             // (chunks are numbered from the span's first from here on)
   const int x = blockIdx.x * 64 + threadIdx.x, quads = a.vpad * (DP / 4);
@@ -575,176 +679,262 @@ __global__ __launch_bounds__(256) void om_chunk_out_kernel(OMChunk a) {
   }
 }
 
-// The same where keys, queries and values enter as the bf16 numbers they are (mLSTM, state space): scores are bf16 products as they stand, the
-// weights that meet the values go in three bf16 parts; only the state's product stays on the fp32 units.
+// The outputs of a group of chunks (bf16 inputs; om_chunk_update16_kernel above says how the work lies).  Per chunk: a wave's 16 queries against the keys --
+// the weights go to LDS in three bf16 parts, where the keys were --, then every wave's own columns: state times all queries, values times weights, and
+// the state after the chunk.  Which wave has which queries goes round: later ones see more tokens.
 template <int MODE, int DP, bool VEC>
-__global__ __launch_bounds__(256, MODE == 2 ? 4 : 3) void om_chunk_out16_kernel(OMChunk a) {
-  constexpr int KP = DP + 8, VP = CHUNK + 8, SCORES = CHUNK * (CHUNK + 1) * 4, KEYS = CHUNK * KP * 2;
-  __shared__ __attribute__((aligned(16))) unsigned char room[KEYS > SCORES ? KEYS : SCORES];      // keys; for values that are not finite, then: the scores
-  __shared__ __attribute__((aligned(16))) uint16_t vt[OMC_COLS * VP];
-  __shared__ double gs[CHUNK];
-  __shared__ float bs[CHUNK];
+__global__ __launch_bounds__(256, 2) void om_chunk_out16_kernel(OMChunk a) {
+  constexpr int KP = DP + 8, KEYS = CHUNK * KP * 2, PARTS = 3 * CHUNK * OMG_PITCH * 2;
+  static_assert(PARTS >= KEYS && PARTS >= CHUNK * (CHUNK + 1) * 4, "");
+  __shared__ __attribute__((aligned(16))) unsigned char room[PARTS];     // keys [token][row], then the weights' parts [3][query][token], or fp32 ones
+  __shared__ __attribute__((aligned(16))) uint16_t qs[CHUNK * KP];
+  __shared__ __attribute__((aligned(16))) uint16_t kt[DP * OMG_PITCH];
+  __shared__ __attribute__((aligned(16))) uint16_t vt[OMC_COLS * OMG_PITCH];
+  __shared__ double gs[4][CHUNK];
+  __shared__ __attribute__((aligned(16))) float bs[4][CHUNK], ws[4][CHUNK];
+  __shared__ float alls[4], ns[MODE == 1 ? DP : 1], invs[MODE == 1 ? CHUNK : 1];
   uint16_t* ks = reinterpret_cast<uint16_t*>(room);
+  uint16_t* pp = reinterpret_cast<uint16_t*>(room);
+  float* ps = reinterpret_cast<float*>(room);
   const OuterMemory& p = a.p;
-  int s, c;
-  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
-  const int slot = p.slot_of_seq[s];
-  if (slot < 0 || slot >= p.num_slots) return;
-  const int h = blockIdx.y, c0 = blockIdx.z * OMC_COLS, hk = MODE == 2 ? h / (p.heads / p.qk_heads) : h;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
-  const int cnt = min(CHUNK, p.q_len[s] - c * CHUNK);
-  const int64_t row0 = (int64_t)p.q_start[s] + c * CHUNK;
-  const int64_t row = row0 + min(lane, cnt - 1);
-  const uint16_t* kr = (const uint16_t*)p.k + row * p.k_stride + (int64_t)hk * p.dim;
-  const uint16_t* vr = (const uint16_t*)p.v + row * p.v_stride + (int64_t)h * p.vdim + c0;
-  u16x8 kx[DP / 32], vx[OMC_COLS / 32];
+  OMGroup g;
+  if (!locate_group(a, g)) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, lg = lane >> 4;
+  const int nct = min(OMC_COLS / 16, (p.vdim - g.c0 + 15) >> 4);
+  const uint16_t* kb = (const uint16_t*)p.k + (int64_t)g.hk * p.dim;
+  const uint16_t* qb = (const uint16_t*)p.q + (int64_t)g.hk * p.dim;
+  const uint16_t* vb = (const uint16_t*)p.v + (int64_t)g.h * p.vdim + g.c0;
+  const u32x4 zeros = {};
+  u32x4 kx[DP / 32], qx[DP / 32], vx[OMC_COLS / 32];
+  auto fetch = [&](int c) {                                              // lane = token; the waves divide the rows and the columns
+    const int64_t row = g.row0 + min(c * CHUNK + lane, g.tokens - 1);
 #pragma unroll
-  for (int it = 0; it < DP / 32; ++it) kx[it] = load8_bits<VEC>(kr, wave * (DP / 4) + it * 8, p.dim);
+    for (int it = 0; it < DP / 32; ++it) kx[it] = __builtin_bit_cast(u32x4, load8_bits<VEC>(kb + row * p.k_stride, wave * (DP / 4) + it * 8, p.dim));
 #pragma unroll
-  for (int it = 0; it < OMC_COLS / 32; ++it) vx[it] = load8_bits<VEC>(vr, wave * (OMC_COLS / 4) + it * 8, p.vdim - c0);
-  const int qt = (wave + blockIdx.x + blockIdx.y) & 3, qi = qt * 16 + li;      // (which queries a wave has: as above)
-  u16x8 q[DP / 32];
-  {
-    const uint16_t* qr = (const uint16_t*)p.q + (row0 + min(qi, cnt - 1)) * p.q_stride + (int64_t)hk * p.dim;
+    for (int it = 0; it < DP / 32; ++it) qx[it] = __builtin_bit_cast(u32x4, load8_bits<VEC>(qb + row * p.q_stride, wave * (DP / 4) + it * 8, p.dim));
 #pragma unroll
-    for (int kk = 0; kk < DP / 32; ++kk) q[kk] = load8_bits<VEC>(qr, 32 * kk + 8 * lg, p.dim);
-  }
-  const int nct = min(OMC_COLS / 16, (p.vdim - c0 + 15) >> 4);
-  const float* st = a.u + (((int64_t)blockIdx.x * p.heads + h) * a.vpad + c0) * DP;
-  f32x4 acc[OMC_COLS / 16] = {};
-#pragma unroll
-  for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
-    if (ct >= nct) break;
-    const float* sr = st + (ct * 16 + li) * DP + 8 * lg;
-#pragma unroll
-    for (int kk = 0; kk < DP / 32; ++kk) {
-      const f32x4 s0 = *reinterpret_cast<const f32x4*>(sr + 32 * kk), s1 = *reinterpret_cast<const f32x4*>(sr + 32 * kk + 4);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) acc[ct] = mfma4(s0[m], BFloat::to_f32(q[kk][m]), acc[ct]);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) acc[ct] = mfma4(s1[m], BFloat::to_f32(q[kk][4 + m]), acc[ct]);
-    }
-  }
-  bool odd = false;                                                      // a value that is not finite
-#pragma unroll
-  for (int it = 0; it < DP / 32; ++it)
-    *reinterpret_cast<u16x8*>(&ks[lane * KP + wave * (DP / 4) + it * 8]) = lane < cnt ? kx[it] : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-  for (int it = 0; it < OMC_COLS / 32; ++it)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint16_t x = lane < cnt ? vx[it][i] : (uint16_t)0;
-      odd |= (x & 0x7f80u) == 0x7f80u;
-      vt[(wave * (OMC_COLS / 4) + it * 8 + i) * VP + lane] = x;
-    }
-  if (wave == 0) {
-    double la;
-    float b;
-    chunk_gate<BFloat, MODE>(a, h, row0, lane, cnt, la, b);
-    gs[lane] = wave_incl_sum(la, lane);
-    bs[lane] = b;
-  }
-  odd = __syncthreads_or(odd);
-  const double gq = gs[qi];
-  const float scale = MODE == 1 ? p.q_scale : 1.f, eq = exp2_d(gq) * scale;
-#pragma unroll
-  for (int ct = 0; ct < OMC_COLS / 16; ++ct)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[ct][r] *= eq;
-  float nq = 0.f;                                                       // mLSTM: the lane's part of n . q
-  if constexpr (MODE == 1) {
-    const float* nb = a.un + ((int64_t)blockIdx.x * p.heads + h) * DP + 8 * lg;
+    for (int it = 0; it < OMC_COLS / 32; ++it) vx[it] = __builtin_bit_cast(u32x4, load8_bits<VEC>(vb + row * p.v_stride, wave * (OMC_COLS / 4) + it * 8, p.vdim - g.c0));
+  };
+  fetch(0);
+  const int64_t at = (int64_t)g.x * p.heads + g.h;
+  f32x4 S[DP / 32][2] = {};
+  if (wave < nct) {
+    const float* u = a.u + (at * a.vpad + g.c0 + wave * 16 + li) * DP + 8 * lg;
 #pragma unroll
     for (int kk = 0; kk < DP / 32; ++kk)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) nq += BFloat::to_f32(q[kk][i]) * nb[32 * kk + i];
-    nq *= eq;
+      for (int hf = 0; hf < 2; ++hf) S[kk][hf] = *reinterpret_cast<const f32x4*>(u + 32 * kk + 4 * hf);
   }
-  // the chunk's own tokens up to the query's, 32 a step: lane group lg has tokens 4 lg .. 4 lg + 3 of either half
-  f32x4 pr[CHUNK / 16];
+  float sn = 0.f;
+  if (MODE == 1 && tid < DP) ns[tid] = sn = a.un[at * DP + tid];
+  const float scale = MODE == 1 ? p.q_scale : 1.f, skip = MODE == 2 ? p.skip[g.h] : 0.f;
+  const int qt = (wave + g.x + g.h) & 3, qi = qt * 16 + li;
+  for (int c = 0; c < g.chunks; ++c) {
+    const int c4 = c & 3;
+    if (c4 == 0) {                                                       // the gates of four chunks, one a wave
+      double la;
+      float b;
+      chunk_gate<BFloat, MODE>(a, g.h, g.row0 + (c + wave) * CHUNK, lane, g.tokens - (c + wave) * CHUNK, la, b);
+      const double gi = wave_incl_sum(la, lane), gend = __shfl(gi, 63, 64);
+      gs[wave][lane] = gi;
+      bs[wave][lane] = b;
+      ws[wave][lane] = exp2_d(gend - gi) * b;
+      if (lane == 0) alls[wave] = exp2_d(gend);
+    }
+    const int cnt = min(CHUNK, g.tokens - c * CHUNK);
+    const int64_t row0 = g.row0 + c * CHUNK;
+    if (cnt < CHUNK && lane >= cnt) {
 #pragma unroll
-  for (int jp = 0; jp < CHUNK / 32; ++jp) {
-    if (2 * jp > qt) break;
-    u16x8 part[3];
+      for (int it = 0; it < DP / 32; ++it) kx[it] = qx[it] = zeros;
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int jt = 2 * jp + half;
-      f32x4 sc = {};
-      if (jt <= qt) {
+      for (int it = 0; it < OMC_COLS / 32; ++it) vx[it] = zeros;
+    }
+    u16x2 top = {};
+#pragma unroll
+    for (int it = 0; it < DP / 32; ++it) {
+      largest_bits(top, kx[it]);
+      largest_bits(top, qx[it]);
+      const int d = wave * (DP / 4) + it * 8;
+      *reinterpret_cast<u32x4*>(&ks[lane * KP + d]) = kx[it];
+      *reinterpret_cast<u32x4*>(&qs[lane * KP + d]) = qx[it];
+      put_rows(kt + lane, kx[it], [&](int i) { return key_row(d + i); });
+    }
+#pragma unroll
+    for (int it = 0; it < OMC_COLS / 32; ++it) {
+      largest_bits(top, vx[it]);
+      put_rows(vt + lane, vx[it], [&](int i) { return wave * (OMC_COLS / 4) + it * 8 + i; });
+    }
+    bool odd = odd_bits(top);                                            // a number that is not finite
+    odd = __builtin_amdgcn_readfirstlane(__syncthreads_or(odd));
+    if (c + 1 < g.chunks) fetch(c + 1);
+    // the wave's queries against the chunk's tokens up to them
+    const double gq = gs[c4][qi];
+    f32x4 pr[CHUNK / 16] = {};
+    int lj = li;                                                         // (not to be kept as sixteen masks from chunk to chunk)
+    asm("" : "+v"(lj));
+    float nq = 0.f;                                                      // mLSTM: the lane's part of n . q
+    {
+      u16x8 q[DP / 32];
+#pragma unroll
+      for (int kk = 0; kk < DP / 32; ++kk) q[kk] = *reinterpret_cast<const u16x8*>(&qs[qi * KP + 32 * kk + 8 * lg]);
+      if constexpr (MODE == 1) {
+#pragma unroll
+        for (int kk = 0; kk < DP / 32; ++kk)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) nq += BFloat::to_f32(q[kk][i]) * ns[32 * kk + 8 * lg + i];
+        nq *= exp2_d(gq) * scale;
+      }
+#pragma unroll
+      for (int jt = 0; jt < CHUNK / 16; ++jt) {
+        if (jt > qt) break;
+        const int last = jt == qt ? lj : CHUNK;
+        f32x4 sc = {};
 #pragma unroll
         for (int kk = 0; kk < DP / 32; ++kk) sc = mfma16(*reinterpret_cast<const u16x8*>(&ks[(jt * 16 + li) * KP + 32 * kk + 8 * lg]), q[kk], sc);
-      }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int j = jt * 16 + 4 * lg + r;
-        float w = 0.f;
-        if (j <= qi) w = sc[r] * scale * (exp2_d(gq - gs[j]) * bs[j]);
-        pr[jt][r] = w;
-        if (MODE == 1) nq += w;
-        uint16_t x[3];
-        split3(w, x);
-#pragma unroll
-        for (int n = 0; n < 3; ++n) part[n][4 * half + r] = x[n];
+        for (int r = 0; r < 4; ++r) {
+          const int j = jt * 16 + 4 * lg + r;
+          const float w = sc[r] * scale * (exp2_d(gq - gs[c4][j]) * bs[c4][j]);
+          pr[jt][r] = 4 * lg + r > last ? 0.f : w;
+          if (MODE == 1) nq += pr[jt][r];
+          if (MODE == 2 && 4 * lg + r == last) pr[jt][r] += skip;               // skip times the query's own value
+        }
       }
     }
-    if (!odd) {
-#pragma unroll
-      for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
-        if (ct >= nct) break;
-        const uint16_t* vp = &vt[(ct * 16 + li) * VP + 32 * jp + 4 * lg];
-        const u32x2 lo = *reinterpret_cast<const u32x2*>(vp), hi = *reinterpret_cast<const u32x2*>(vp + 16);
-        const u16x8 vv = __builtin_bit_cast(u16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
-#pragma unroll
-        for (int n = 2; n >= 0; --n) acc[ct] = mfma16(vv, part[n], acc[ct]);
-      }
+    if constexpr (MODE == 1) {
+      nq += __shfl_xor(nq, 16, 64);
+      nq += __shfl_xor(nq, 32, 64);
+      const float em = a.em[(int64_t)g.h * p.num_tokens + row0 + min(qi, cnt - 1)];
+      if (lg == 0) invs[qi] = fmaxf(fabsf(nq), em) + 1e-6f;
     }
-  }
-  if (odd) {
-    // zero times a value that is not finite is not zero: a token behind the query must not be multiplied at all
-    __syncthreads();                                                     // every wave is through with the keys
-    float* ps = reinterpret_cast<float*>(room);                          // [64 queries][64 + 1]
+    lds_barrier();                                                       // every wave is through with the keys
+    if (odd) {
 #pragma unroll
-    for (int jt = 0; jt < CHUNK / 16; ++jt)
-      if (jt <= qt)
+      for (int jt = 0; jt < CHUNK / 16; ++jt)
+        if (jt <= qt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ps[qi * (CHUNK + 1) + jt * 16 + 4 * lg + r] = pr[jt][r];
-    __syncthreads();
-#pragma unroll
-    for (int ct = 0; ct < OMC_COLS / 16; ++ct)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float sum = 0.f;
-        for (int j = 0; j <= qi; ++j) sum += ps[qi * (CHUNK + 1) + j] * BFloat::to_f32(vt[(ct * 16 + 4 * lg + r) * VP + j]);
-        acc[ct][r] += sum;
-      }
-  }
-  float inv = 1.f;
-  if constexpr (MODE == 1) {
-    nq += __shfl_xor(nq, 16, 64);
-    nq += __shfl_xor(nq, 32, 64);
-    const float em = a.em[(int64_t)h * p.num_tokens + row0 + min(qi, cnt - 1)];
-    inv = fmaxf(fabsf(nq), em) + 1e-6f;
-  }
-  if (qi >= cnt) return;
-  const float skip = MODE == 2 ? p.skip[h] : 0.f;
-  float* o = p.out + (row0 + qi) * ((int64_t)p.heads * p.vdim) + (int64_t)h * p.vdim + c0;
-#pragma unroll
-  for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
-    if (ct >= nct) break;
-    const int e = ct * 16 + 4 * lg;
-    f32x4 x = acc[ct];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      if (MODE == 1) x[r] = x[r] / inv;
-      if (MODE == 2) x[r] += skip * BFloat::to_f32(vt[(e + r) * VP + qi]);
-    }
-    if ((p.vdim & 3) == 0) {
-      if (c0 + e < p.vdim) *reinterpret_cast<f32x4*>(o + e) = x;
+          for (int r = 0; r < 4; ++r) ps[qi * (CHUNK + 1) + jt * 16 + 4 * lg + r] = pr[jt][r];
     } else {
+      float z = 0.f;                                                     // not zero: a sum beyond fp32's range
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (c0 + e + r < p.vdim) o[e + r] = x[r];
+      for (int jt = 0; jt < CHUNK / 16; ++jt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z = fmaf(pr[jt][r], 0.f, z);
+      const bool all = !__any(z != 0.f);
+#pragma unroll
+      for (int jp = 0; jp < CHUNK / 32; ++jp) {                          // (products take 32 tokens: zeros up to there)
+        if (2 * jp > qt) break;
+        const float x[8] = {pr[2 * jp][0], pr[2 * jp][1], pr[2 * jp][2], pr[2 * jp][3], pr[2 * jp + 1][0], pr[2 * jp + 1][1], pr[2 * jp + 1][2], pr[2 * jp + 1][3]};
+        u16x8 part[3];
+        if (all) split3_finite(x, part);
+        else
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            uint16_t t[3];
+            split3(x[i], t);
+#pragma unroll
+            for (int n = 0; n < 3; ++n) part[n][i] = t[n];
+          }
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+          const u32x4 w = __builtin_bit_cast(u32x4, part[n]);
+          uint16_t* at = &pp[(n * CHUNK + qi) * OMG_PITCH + 32 * jp + 4 * lg];
+          *reinterpret_cast<u32x2*>(at) = u32x2{w[0], w[1]};
+          *reinterpret_cast<u32x2*>(at + 16) = u32x2{w[2], w[3]};
+        }
+      }
     }
+    lds_barrier();
+    if (wave < nct) {
+      u16x8 v[CHUNK / 32];
+#pragma unroll
+      for (int jj = 0; jj < CHUNK / 32; ++jj) v[jj] = *reinterpret_cast<const u16x8*>(&vt[(wave * 16 + li) * OMG_PITCH + 32 * jj + 8 * lg]);
+      f32x4 acc[CHUNK / 16] = {};
+      float eq[CHUNK / 16];
+#pragma unroll
+      for (int t = 0; t < CHUNK / 16; ++t) eq[t] = exp2_d(gs[c4][t * 16 + li]) * scale;
+      float z = 0.f;                                                     // not zero: a state that is not finite
+#pragma unroll
+      for (int kk = 0; kk < DP / 32; ++kk)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) z = fmaf(S[kk][i >> 2][i & 3], 0.f, z);
+      if (odd || __any(z != 0.f)) {
+#pragma unroll
+        for (int kk = 0; kk < DP / 32; ++kk)
+#pragma unroll
+          for (int t = 0; t < CHUNK / 16; ++t) {
+            const u16x8 q = *reinterpret_cast<const u16x8*>(&qs[(t * 16 + li) * KP + 32 * kk + 8 * lg]);
+#pragma unroll
+            for (int m = 0; m < 8; ++m) acc[t] = mfma4(S[kk][m >> 2][m & 3], BFloat::to_f32(q[m]), acc[t]);
+          }
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < DP / 32; ++kk) {                           // what the state ahead of the chunk gives
+          u16x8 part[3], q[CHUNK / 16];
+          const float x[8] = {S[kk][0][0], S[kk][0][1], S[kk][0][2], S[kk][0][3], S[kk][1][0], S[kk][1][1], S[kk][1][2], S[kk][1][3]};
+          split3_finite(x, part);
+#pragma unroll
+          for (int t = 0; t < CHUNK / 16; ++t) q[t] = *reinterpret_cast<const u16x8*>(&qs[(t * 16 + li) * KP + 32 * kk + 8 * lg]);
+#pragma unroll
+          for (int n = 2; n >= 0; --n)
+#pragma unroll
+            for (int t = 0; t < CHUNK / 16; ++t) acc[t] = mfma16(part[n], q[t], acc[t]);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < CHUNK / 16; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[t][r] *= eq[t];
+      if (!odd) {
+#pragma unroll
+        for (int jj = 0; jj < CHUNK / 32; ++jj)
+#pragma unroll
+          for (int n = 2; n >= 0; --n)
+#pragma unroll
+            for (int t = 2 * jj; t < CHUNK / 16; ++t)
+              acc[t] = mfma16(v[jj], *reinterpret_cast<const u16x8*>(&pp[(n * CHUNK + t * 16 + li) * OMG_PITCH + 32 * jj + 8 * lg]), acc[t]);
+      } else {
+        // zero times a value that is not finite is not zero: a token behind the query must not be multiplied at all
+#pragma unroll
+        for (int t = 0; t < CHUNK / 16; ++t) {
+          const uint16_t* vr = &vt[(wave * 16 + 4 * lg) * OMG_PITCH];
+          f32x4 sum = {};
+#pragma unroll 1
+          for (int j = 0; j <= t * 16 + li; ++j) {
+            const float w = ps[(t * 16 + li) * (CHUNK + 1) + j];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[r] += w * BFloat::to_f32(vr[r * OMG_PITCH + j]);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[t][r] += sum[r];
+        }
+      }
+      const int e = wave * 16 + 4 * lg;
+      float* o = p.out + row0 * ((int64_t)p.heads * p.vdim) + (int64_t)g.h * p.vdim + g.c0 + e;
+#pragma unroll
+      for (int t = 0; t < CHUNK / 16; ++t) {
+        const int j = t * 16 + li;
+        f32x4 x = acc[t];
+        const float inv = MODE == 1 ? invs[j] : 1.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (MODE == 1) x[r] = x[r] / inv;
+        }
+        if (j >= cnt) continue;
+        float* oj = o + (int64_t)j * p.heads * p.vdim;
+        if ((p.vdim & 3) == 0) {
+          if (g.c0 + e < p.vdim) *reinterpret_cast<f32x4*>(oj) = x;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (g.c0 + e + r < p.vdim) oj[r] = x[r];
+        }
+      }
+      if (c + 1 < g.chunks) group_update<DP>(S, kt, v, ws[c4], alls[c4], odd, li, lg);
+    }
+    if (c + 1 == g.chunks) return;
+    if (MODE == 1 && tid < DP) ns[tid] = sn = group_update_n(sn, kt, ws[c4], alls[c4], tid);
+    lds_barrier();
   }
 }
 
@@ -762,18 +952,31 @@ static int64_t om_chunk_floats(const OuterMemory& p, int64_t chunks) {
   return n[0] + n[1] + n[2] + n[3];
 }
 
+// Chunks of a workgroup (bf16 mLSTM and state space): more of them cost parallelism, fewer the traffic of their states.  Measured, us, with 1 / 2 / 4 / 8 /
+// 16: state space 64 heads 300 tokens (320 workgroups of one chunk) 38 / 39 / 51, 600 (640) 56 / 50 / 55, 2000 (2048) 109 / 85 / 75 / 90,
+// 4096 (4160) 199 / 148 / 126 / 120 / 192; 128 heads 1024 (2176) 111 / 88 / 75 / 112, 4096 (8320) 484 / 294 / 235 / 211 / 200; mLSTM 4 x 128 x 256
+// 2000 (512) 50 / 51 / 61, 4096 (1040) 83 / 65 / 78, 16384 (4112) 275 / 209 / 176 / 160 / 238.  Chunks are counted from the tokens: beside a prompt the
+// bound over segments would count every decoded sequence as one.
+static int om_group_chunks(const OuterMemory& p) {
+  if (p.mode == 0 || p.dtype != APHRO_BF16) return 1;
+  const int64_t units = (p.num_tokens / CHUNK + 1) * p.heads * ((p.vdim + OMC_COLS - 1) / OMC_COLS);
+  return units < 600 ? 1 : units < 1200 ? 2 : units < 4000 ? 4 : 8;
+}
+
 template <typename T, int MODE, int DP, bool VEC>
 static void om_chunk_launch(OMChunk a, int64_t chunks) {
   const OuterMemory& p = a.p;
   const dim3 grid((unsigned)a.span, (unsigned)p.heads, (unsigned)((p.vdim + OMC_COLS - 1) / OMC_COLS));
+  const unsigned pairs = (unsigned)a.span * (unsigned)om_key_heads(p);
+  const dim3 grid16((pairs + 7) / 8 * 8 * (unsigned)(p.heads / om_key_heads(p)) * grid.z);
   const unsigned items = (unsigned)a.vpad * (DP / 4) + (MODE == 1 ? DP : 0);
   if (MODE == 1) hipLaunchKernelGGL((om_gates_kernel<T>), dim3((unsigned)p.num_seqs, (unsigned)p.heads), dim3(1024), 0, p.stream, a);
   for (; a.chunk0 < chunks; a.chunk0 += a.span) {
     constexpr bool B16 = sizeof(typename T::storage) == 2 && MODE != 0;
-    if constexpr (B16) hipLaunchKernelGGL((om_chunk_update16_kernel<MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
+    if constexpr (B16) hipLaunchKernelGGL((om_chunk_update16_kernel<MODE, DP, VEC>), grid16, dim3(256), 0, p.stream, a);
     else hipLaunchKernelGGL((om_chunk_update_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
     hipLaunchKernelGGL((om_chunk_carry_kernel<MODE, DP>), dim3((items + 63) / 64, (unsigned)p.heads, (unsigned)p.num_seqs), dim3(64), 0, p.stream, a);
-    if constexpr (B16) hipLaunchKernelGGL((om_chunk_out16_kernel<MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
+    if constexpr (B16) hipLaunchKernelGGL((om_chunk_out16_kernel<MODE, DP, VEC>), grid16, dim3(256), 0, p.stream, a);
     else hipLaunchKernelGGL((om_chunk_out_kernel<T, MODE, DP, VEC>), grid, dim3(256), 0, p.stream, a);
   }
 }
@@ -807,8 +1010,10 @@ extern "C" int aphro_outer_memory_chunked(float* out, const void* q, int64_t q_s
   if (rc != APHRO_OK) return rc;
   APHRO_CHECK(dim <= 128 && min_len > 0 && num_seqs <= 65535, "outer_memory_chunked: dim %d (<= 128), %d segments (<= 65535) from %d tokens on", dim, num_seqs, min_len);
   if (num_seqs == 1) min_len = 1;
-  const int64_t chunks = max_chunks(num_tokens, num_seqs, min_len);
+  int64_t chunks = max_chunks(num_tokens, num_seqs, min_len);
   APHRO_CHECK(chunks <= 0x3fffffff, "outer_memory_chunked: too many tokens");
+  a.group = om_group_chunks(p);
+  if (a.group > 1) chunks = max_chunks(num_tokens, num_seqs, min_len, a.group * CHUNK);
   const int64_t span = span_chunks(chunks, workspace_bytes, [&](int64_t m) { return om_chunk_floats(p, m); });
   APHRO_CHECK(((uintptr_t)out & 15) == 0 && (chunks == 0 || (workspace && ((uintptr_t)workspace & 15) == 0 && span > 0)),
               "outer_memory_chunked: a workspace of %lld bytes at least, 16-byte aligned, is needed", (long long)om_chunk_floats(p, 1) * 4);
