@@ -17,9 +17,16 @@
 //
 // What bounds it: the scan is bound by the latency of its token chain; here launch 2's chain is one of 64-token steps (two products of 64 x
 // dim x 16 and two barriers each), launches 1 and 3 have all chunks to fill the chip (launch 1 one workgroup a CU:
-// its rows of q, k and g take the LDS).  16 heads of 128 x 128, a decay per channel, one portion, scan -> chunks: 512 tokens 246 -> 88 us, 2048
-// tokens 1010 -> 210 us, 4096 tokens 2020 -> 404 us; a decay per head 1490 -> 357 us.  On the way, launch 2 at 2000 tokens: column blocks of a
-// head on different XCDs and barriers that wait for the operands in flight 100 us, neither 96 us, no early wait for the newest load 87 us.
+// its rows of q, k and g take the LDS).  16 heads of 128 x 128, a decay per channel, one portion: 512 tokens 85 -> 64 us (scan 193), 2000 tokens 198 -> 138,
+// 4096 tokens 394 -> 276 (a decay per head 355 -> 261); 32 heads of 64 x 64, 2000 tokens 178 -> 134.  What that took, launches 1 / 2 / 3 at 2000
+// tokens 82 / 88 / 39 us: matrices between the launches as rows, of which a load of 16 bytes a lane met another cache line in every lane of
+// four, so that the address unit, not the matrix pipe, was waited for (in fragments: launch 2 63, launch 3 30; launch 2's loads between its
+// products: 53); decays one after the other, each with a load of its own and log1pf (launch 1: 25 000 cycles of a chunk's 87 000, now 10 000); a block
+// with itself without LDS, values loaded ahead: 62.  Left in launch 1: 2 rounds of a workgroup a CU, 64 000 cycles each, half of them waits; in launch 2
+// 2 050 of a step's 3 600 cycles are fp32 products.
+#include <type_traits>
+#include <utility>
+
 #include "delta_rule.h"
 #include "chunked_scan.h"
 
@@ -32,16 +39,52 @@ struct GDChunk {
   int min_len;
   int chunk0, span;        // the chunks of these launches (below: [chunks] of one span)
   int vpad;                // vdim rounded up to 16
-  float* w;                // [chunks, heads, 64, DP]  T (Pi K)
-  float* qg;               // [chunks, heads, 64, DP]  Pi Q
-  float* kd;               // [chunks, heads, DP, 64]  (P_63 K)^T
-  float* bm;               // [chunks, heads, 64, 64]  q_i . P_ij k_j, zero above the diagonal of a block with itself, unwritten in later blocks
-  float* ut;               // [chunks, heads, vpad, 64] T V, then U
-  float* st;               // [chunks, heads, vpad, DP] the state ahead of the chunk
+  // Matrices lie in the fragments that the waves read, 1 KiB each with a lane's four numbers next to each other: lane (li, lg) = (l % 16, l / 16) of
+  // fragment (i, j) has row 16 i + li and columns 16 j + 4 lg + (0..3), or, of an array marked *, of fragment (i, 2 j + u) columns 32 j + 8 lg + 4 u + (0..3).
+  float* w;                // [chunks, heads] 64 x DP *   T (Pi K)
+  float* qg;               // [chunks, heads] 64 x DP *   Pi Q
+  float* kd;               // [chunks, heads] DP x 64     (P_63 K)^T
+  float* bm;               // [chunks, heads] 64 x 64     q_i . P_ij k_j, zero above the diagonal of a block with itself, unwritten in later blocks
+  float* ut;               // [chunks, heads] vpad x 64   T V, then U
+  float* st;               // [chunks, heads] vpad x DP * the state ahead of the chunk
   float* gam;              // [chunks, heads, DP]      Pi_63
   int32_t* bad_token;      // [chunks, heads]          first token that is not finite (64: none)
   int32_t* bad_value;      // [chunks, heads, vpad]    first value, or u, of the column that is not finite (64: none)
 };
+
+// Where, in an array marked *, the lane's columns 16 j + 4 lg + (0..3) of row 16 i + li begin.
+template <int DP>
+__device__ __forceinline__ int frag8(int i, int j, int li, int lg) { return (i * (DP / 16) + (j & ~1) + (lg & 1)) * 256 + (((j & 1) * 2 + (lg >> 1)) * 16 + li) * 4; }
+// x of lane I of the own sixteen.
+template <int I>
+__device__ __forceinline__ float of_lane16(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x150 + I, 0xf, 0xf, true));
+}
+// p += sum of x[.] of lane I of the own sixteen times e[.], and q with y.  (hipcc folds the lane's choice into a product, not into an FMA.  The s_nop: what a
+// lane's choice reads has to be two steps old.)
+template <int I>
+__device__ __forceinline__ void fma_of_lane16(float& p, const f32x4& x, float& q, const f32x4& y, const f32x4& e) {
+#define GDC_FMA(ACC, X, E) "v_fmac_f32_dpp " ACC ", " X ", " E " row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
+  asm("s_nop 1\n\t" GDC_FMA("%0", "%2", "%10") GDC_FMA("%1", "%6", "%10") GDC_FMA("%0", "%3", "%11") GDC_FMA("%1", "%7", "%11")
+      GDC_FMA("%0", "%4", "%12") GDC_FMA("%1", "%8", "%12") GDC_FMA("%0", "%5", "%13") GDC_FMA("%1", "%9", "%13")
+      : "+v"(p), "+v"(q)
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(e[0]), "v"(e[1]), "v"(e[2]), "v"(e[3]), "n"(I));
+#undef GDC_FMA
+}
+// a + b of the lanes 16 (32) apart, of a in the even sixteens (the first half), of b in the others.
+__device__ __forceinline__ float sum_swap16(float a, float b) {
+  const auto w = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  const uint32_t x = w[0], y = w[1];
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+__device__ __forceinline__ float sum_swap32(float a, float b) {
+  const auto w = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  const uint32_t x = w[0], y = w[1];
+  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+}
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+template <typename F, int... I>
+__device__ __forceinline__ void each16_(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
 
 template <int DP>
 constexpr size_t gd_prepare_lds() { return (3 * CHUNK * (DP + 4) + 2 * CHUNK * GDC_P + 4 * DP + CHUNK + 2 * (DP / 16) * CHUNK + CHUNK + 4) * sizeof(float); }
@@ -67,7 +110,6 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
   int s, c;
   if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
   const int slot = p.slot_of_seq[s];
-  if (slot < 0 || slot >= p.num_slots) return;
   const int h = blockIdx.y, hk = h / (p.heads / p.kv_heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
   const int cnt = min(CHUNK, p.q_len[s] - c * CHUNK);
@@ -87,8 +129,15 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
       load8<T, VEC>(kr, d, p.dim, k[it]);
       if constexpr (CHANNEL) load8<T, VEC>(ar, d, p.dim, g[it]);
     }
+    float bias[2][8];                                      // (loaded here, not where each is used: sixteen loads to wait for one after the other)
+    if constexpr (CHANNEL)
+#pragma unroll
+      for (int it = 0; it < 2; ++it)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) bias[it][i] = p.dt_bias[(int64_t)h * p.dim + min(wave * 16 + it * 8 + i, p.dim - 1)];
     const float raw_b = T::to_f32(((const ST*)p.b)[row * p.b_stride + h]);
     const float rate = -expf(p.a_log[h]);
+    if (slot < 0 || slot >= p.num_slots) return;
     float sq = 0.f, sk = 0.f;
 #pragma unroll
     for (int it = 0; it < 2; ++it)
@@ -113,7 +162,10 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
         const int d = wave * 16 + it * 8 + i;
         q[it][i] = live ? q[it][i] * fq : 0.f;
         k[it][i] = live ? k[it][i] * fk : 0.f;
-        if constexpr (CHANNEL) g[it][i] = d < p.dim && live ? expf(rate * softplus_f(g[it][i] + p.dt_bias[(int64_t)h * p.dim + d])) : 1.f;
+        if constexpr (CHANNEL) {
+          const float z = expf(rate * softplus_f(g[it][i] + bias[it][i]));
+          g[it][i] = d < p.dim && live ? z : 1.f;
+        }
         else g[it][i] = live ? gh : 1.f;
         bad |= !finite_f(k[it][i]) || !finite_f(g[it][i]);
       }
@@ -153,45 +205,54 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
     const int b0 = (wave & 3) * 16, r0 = (wave >> 2) * (DP / 2) + lg * PART;
 #pragma unroll 2
     for (int r = r0; r < r0 + PART; r += 4) {
+      // a lane's own rows; token i's numbers come from lane i of the sixteen inside the instruction that uses them (read from LDS by every lane: 17 300
+      // cycles for 12 700)
       const f32x4 kj = *reinterpret_cast<const f32x4*>(&kk[(b0 + li) * KP + r]);
+      const f32x4 gj = *reinterpret_cast<const f32x4*>(&gg[(b0 + li) * KP + r]);
+      const f32x4 qj = *reinterpret_cast<const f32x4*>(&qq[(b0 + li) * KP + r]);
       f32x4 e = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const f32x4 gi = *reinterpret_cast<const f32x4*>(&gg[(b0 + i) * KP + r]);
-        const f32x4 ki = *reinterpret_cast<const f32x4*>(&kk[(b0 + i) * KP + r]);
-        const f32x4 qi = *reinterpret_cast<const f32x4*>(&qq[(b0 + i) * KP + r]);
+      each16_([&](auto ii) {
+        constexpr int i = decltype(ii)::value;
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-          e[x] = i == li ? kj[x] : e[x] * gi[x];
-          la[i] += ki[x] * e[x];
-          lb[i] += qi[x] * e[x];
+          const float d = e[x] * of_lane16<i>(gj[x]);
+          e[x] = i == li ? kj[x] : d;
         }
-      }
+        fma_of_lane16<i>(la[i], kj, lb[i], qj, e);
+      }, std::make_integer_sequence<int, 16>{});
     }
+    // sums over the quarters; sixteens 0 and 2 keep L, 1 and 3 the scores, of tokens i = 0..7 (sixteens 0 and 1) and 8..15
+    float sum[8];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      la[i] += __shfl_xor(la[i], 16, 64);
-      lb[i] += __shfl_xor(lb[i], 16, 64);
-      la[i] += __shfl_xor(la[i], 32, 64);
-      lb[i] += __shfl_xor(lb[i], 32, 64);
-    }
+    for (int i = 0; i < 8; ++i) sum[i] = sum_swap32(sum_swap16(la[i], lb[i]), sum_swap16(la[i + 8], lb[i + 8]));
+    const int i0 = (lg >> 1) * 8;
     if constexpr (HALVES == 2) {
-      if (wave >= 4 && lg == 0)
+      float* half = tm + (b0 + (lane >> 2)) * GDC_P + (lane & 3) * 8;        // eight numbers of a lane, in rows of the block
+      if (wave >= 4)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) tm[(b0 + i) * GDC_P + li] = la[i], tm[(b0 + i) * GDC_P + 16 + li] = lb[i];
+        for (int u = 0; u < 2; ++u) *reinterpret_cast<f32x4*>(half + 4 * u) = f32x4{sum[4 * u], sum[4 * u + 1], sum[4 * u + 2], sum[4 * u + 3]};
       __syncthreads();
       if (wave < 4)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) la[i] += tm[(b0 + i) * GDC_P + li], lb[i] += tm[(b0 + i) * GDC_P + 16 + li];
+        for (int u = 0; u < 2; ++u) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(half + 4 * u);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sum[4 * u + i] += x[i];
+        }
       __syncthreads();
       for (int i = tid; i < CHUNK * 32; i += NW * 64) tm[(i >> 5) * GDC_P + (i & 31)] = 0.f;
     }
-    if (lg == 0 && wave < 4)
+    if (wave < 4) {
+      if (lg & 1) {
+        float* at = bmu + wave * 5 * 256 + (li >> 2) * 64 + (li & 3);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        if (i > li) lm[(b0 + i) * GDC_P + b0 + li] = bet[b0 + i] * la[i];
-        bmu[(b0 + i) * CHUNK + b0 + li] = i >= li ? lb[i] : 0.f;
+        for (int i = 0; i < 8; ++i) at[(i0 + i) * 4] = i0 + i >= li ? sum[i] : 0.f;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (i0 + i > li) lm[(b0 + i0 + i) * GDC_P + b0 + li] = bet[b0 + i0 + i] * sum[i];
       }
+    }
   }
   __syncthreads();
   // -- decays from a block's start and to its end, folded into q and k; thread = (channel, block)
@@ -239,15 +300,15 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
 #pragma unroll
         for (int y = 0; y < 4; ++y) {
           al = mfma4(ki[u][y], bj[u][y], al);
-          ab = mfma4(qi[u][y], bj[u][y], ab);
+          ab = mfma4(bj[u][y], qi[u][y], ab);             // (a lane: a query, four neighbouring keys)
         }
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = I * 16 + 4 * lg + r;
       lm[i * GDC_P + J * 16 + li] = bet[i] * al[r];
-      bmu[i * CHUNK + J * 16 + li] = ab[r];
     }
+    *reinterpret_cast<f32x4*>(&bmu[(I * 4 + J) * 256 + lane * 4]) = ab;
   }
   __syncthreads();
   // -- (1 + L)^-1: blocks on the diagonal by substitution (wave = block, lane = column), the others by products, one diagonal after the other
@@ -292,29 +353,44 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
     const int blk = lane >> 4;                              // lane = token; the waves divide the channels
     for (int it = 0; it < 4; ++it) {
       const int r = wave * 16 + it * 4;
-      f32x4 pre = {1.f, 1.f, 1.f, 1.f}, suf = pre;
-      for (int m = 0; m < 4; ++m) {
+      f32x4 pre = {1.f, 1.f, 1.f, 1.f};
+      for (int m = 0; m < 3; ++m) {
         const f32x4 d = *reinterpret_cast<const f32x4*>(&dd[m * DP + r]);
 #pragma unroll
-        for (int y = 0; y < 4; ++y) {
+        for (int y = 0; y < 4; ++y)
           if (m < blk) pre[y] *= d[y];
-          if (m > blk) suf[y] *= d[y];
-        }
       }
       f32x4 k = *reinterpret_cast<const f32x4*>(&kk[lane * KP + r]), q = *reinterpret_cast<const f32x4*>(&qq[lane * KP + r]);
-      const f32x4 e = *reinterpret_cast<const f32x4*>(&gg[lane * KP + r]);
 #pragma unroll
       for (int y = 0; y < 4; ++y) {
         k[y] *= pre[y];
         q[y] *= pre[y];
-        kd[(r + y) * CHUNK + lane] = e[y] * suf[y];
       }
       *reinterpret_cast<f32x4*>(&kk[lane * KP + r]) = k;
-      *reinterpret_cast<f32x4*>(&qg[lane * DP + r]) = q;
+      *reinterpret_cast<f32x4*>(&qg[frag8<DP>(blk, wave, li, it)]) = q;
+    }
+    {                                                       // the same of k to the chunk's end: a wave's sixteen channels, four neighbouring tokens a lane
+      float suf = 1.f;
+      for (int m = 3; m >= 0; --m) {
+        f32x4 e;
+#pragma unroll
+        for (int y = 0; y < 4; ++y) e[y] = gg[(16 * m + 4 * lg + y) * KP + wave * 16 + li] * suf;
+        *reinterpret_cast<f32x4*>(&kd[(wave * 4 + m) * 256 + lane * 4]) = e;
+        suf *= dd[m * DP + wave * 16 + li];
+      }
     }
     for (int r = tid; r < DP; r += NW * 64) a.gam[unit * DP + r] = (dd[r] * dd[DP + r]) * (dd[2 * DP + r] * dd[3 * DP + r]);
   }
   __syncthreads();
+  // (the first values are on their way meanwhile)
+  constexpr int LOADS = 8 / NW;
+  float x[LOADS][8];
+  auto values = [&](int c0) {
+    const ST* vr = (const ST*)p.v + row * p.v_stride + (int64_t)h * p.vdim + c0;
+#pragma unroll
+    for (int it = 0; it < LOADS; ++it) load8<T, VEC>(vr, (wave * LOADS + it) * 8, p.vdim - c0, x[it]);
+  };
+  values(0);
   // -- W^T = (Pi K)^T T^T: a wave's 16 channels x the tokens, four neighbouring channels a lane
   {
     f32x4 acc[4] = {};
@@ -332,16 +408,11 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
     }
     float* w = a.w + unit * CHUNK * DP;
 #pragma unroll
-    for (int it = 0; it < 4; ++it) *reinterpret_cast<f32x4*>(&w[(it * 16 + li) * DP + wave * 16 + 4 * lg]) = acc[it];
+    for (int it = 0; it < 4; ++it) *reinterpret_cast<f32x4*>(&w[frag8<DP>(it, wave, li, lg)]) = acc[it];
   }
   // -- T V, 64 value columns at a time: a wave takes 16 columns x the tokens (or every other 16 of them), four neighbouring tokens a lane
   float* vt = qq;
   for (int c0 = 0; c0 < p.vdim; c0 += 64) {
-    const ST* vr = (const ST*)p.v + row * p.v_stride + (int64_t)h * p.vdim + c0;
-    constexpr int LOADS = 8 / NW;
-    float x[LOADS][8];
-#pragma unroll
-    for (int it = 0; it < LOADS; ++it) load8<T, VEC>(vr, (wave * LOADS + it) * 8, p.vdim - c0, x[it]);
 #pragma unroll
     for (int it = 0; it < LOADS; ++it)
 #pragma unroll
@@ -354,10 +425,11 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
         if (lane == 0) bad_col[e] = mask ? __ffsll((unsigned long long)mask) - 1 : CHUNK;
       }
     __syncthreads();
+    if (c0 + 64 < p.vdim) values(c0 + 64);
     if (tid < 64 && c0 + tid < a.vpad) a.bad_value[unit * a.vpad + c0 + tid] = bad_col[tid];
     const int ct = wave & 3;
     if (c0 + ct * 16 < a.vpad) {
-      float* ut = a.ut + (unit * a.vpad + c0 + ct * 16 + li) * CHUNK;
+      float* ut = a.ut + (unit * a.vpad + c0 + ct * 16) * CHUNK + lane * 4;
 #pragma unroll
       for (int i = 0; i < 4 / HALVES; ++i) {
         const int it = HALVES == 2 ? 2 * i + (wave >> 2) : i;
@@ -368,7 +440,7 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
 #pragma unroll
           for (int y = 0; y < 4; ++y) acc = mfma4(t[y], vv[y], acc);
         }
-        *reinterpret_cast<f32x4*>(&ut[it * 16 + 4 * lg]) = acc;
+        *reinterpret_cast<f32x4*>(&ut[it * 256]) = acc;
       }
     }
     __syncthreads();
@@ -411,32 +483,30 @@ __global__ __launch_bounds__(256) void gd_chunk_carry_kernel(GDChunk a) {
       const int d = (wave * DT + dt) * 16 + 4 * lg + r;
       S[dt][r] = !fresh && d < p.dim && col < p.vdim ? sb[(int64_t)d * p.vdim] : 0.f;
     }
-  auto fetch = [&](int c, GDCarry<DP>& x) {
-    const int64_t unit = (first + min(c, nc - 1)) * p.heads + h;
-    const float* w = a.w + unit * CHUNK * DP + (wave * 16 + li) * DP + 8 * lg;
+  // a chunk's operands in pieces: the loads of the next chunk go out between this one's products, as 21 loads in a row hold the wave up for 1 250 cycles
+  auto unit_of = [&](int c) { return (first + min(c, nc - 1)) * p.heads + h; };
+  auto fetch_w = [&](int64_t unit, GDCarry<DP>& x, int k8, int u) {
+    x.w[k8][u] = *reinterpret_cast<const f32x4*>(a.w + unit * CHUNK * DP + wave * 16 * DP + (2 * k8 + u) * 256 + lane * 4);
+  };
+  auto fetch_kd = [&](int64_t unit, GDCarry<DP>& x, int dt, int k4) {
+    x.kd[dt][k4] = *reinterpret_cast<const f32x4*>(a.kd + unit * DP * CHUNK + (wave * DT + dt) * 16 * CHUNK + k4 * 256 + lane * 4);
+  };
+  auto fetch_rest = [&](int64_t unit, GDCarry<DP>& x) {
 #pragma unroll
-    for (int k8 = 0; k8 < DP / 32; ++k8)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) x.w[k8][u] = *reinterpret_cast<const f32x4*>(w + 32 * k8 + 4 * u);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const float* kd = a.kd + unit * DP * CHUNK + ((wave * DT + dt) * 16 + li) * CHUNK + 4 * lg;
-#pragma unroll
-      for (int k4 = 0; k4 < 4; ++k4) x.kd[dt][k4] = *reinterpret_cast<const f32x4*>(kd + 16 * k4);
-      x.gam[dt] = *reinterpret_cast<const f32x4*>(a.gam + unit * DP + (wave * DT + dt) * 16 + 4 * lg);
-    }
-    x.ut = *reinterpret_cast<const f32x4*>(a.ut + (unit * a.vpad + col) * CHUNK + wave * 16 + 4 * lg);
+    for (int dt = 0; dt < DT; ++dt) x.gam[dt] = *reinterpret_cast<const f32x4*>(a.gam + unit * DP + (wave * DT + dt) * 16 + 4 * lg);
+    x.ut = *reinterpret_cast<const f32x4*>(a.ut + (unit * a.vpad + c0) * CHUNK + wave * 256 + lane * 4);
     x.bad_token = a.bad_token[unit];
     x.bad_value = a.bad_value[unit * a.vpad + col];
   };
-  auto step = [&](int c, const GDCarry<DP>& x) {
+  auto step = [&](int c, const GDCarry<DP>& x, GDCarry<DP>& y) {
+    const int64_t next = unit_of(c + 1);
     const int64_t unit = (first + c) * p.heads + h;
-    float* st = a.st + (unit * a.vpad + col) * DP;
+    float* st = a.st + (unit * a.vpad + c0) * DP;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       const int d = (wave * DT + dt) * 16 + 4 * lg;
       *reinterpret_cast<f32x4*>(&ss[li * SP + d]) = S[dt];
-      *reinterpret_cast<f32x4*>(&st[d]) = S[dt];
+      *reinterpret_cast<f32x4*>(&st[frag8<DP>(0, wave * DT + dt, li, lg)]) = S[dt];
     }
     lds_barrier();
     f32x4 acc[2] = {}, sv[DP / 32][2];
@@ -448,9 +518,15 @@ __global__ __launch_bounds__(256) void gd_chunk_carry_kernel(GDChunk a) {
 #pragma unroll
     for (int k8 = 0; k8 < DP / 32; ++k8)
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int i = 0; i < 4; i += 2) {
 #pragma unroll
-        for (int y = 0; y < 4; ++y) acc[u] = mfma4(x.w[k8][u][y], sv[k8][u][y], acc[u]);
+        for (int m = i; m < i + 2; ++m)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) acc[u] = mfma4(x.w[k8][u][m], sv[k8][u][m], acc[u]);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_w(next, y, k8, i >> 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     f32x4 uv;
 #pragma unroll
     for (int r = 0; r < 4; ++r) uv[r] = x.ut[r] - (acc[0][r] + acc[1][r]);
@@ -463,7 +539,7 @@ __global__ __launch_bounds__(256) void gd_chunk_carry_kernel(GDChunk a) {
           uv[r] = 0.f;
         }
     }
-    *reinterpret_cast<f32x4*>(a.ut + (unit * a.vpad + col) * CHUNK + wave * 16 + 4 * lg) = uv;
+    *reinterpret_cast<f32x4*>(a.ut + (unit * a.vpad + c0) * CHUNK + wave * 256 + lane * 4) = uv;
     lds_barrier();
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -474,23 +550,38 @@ __global__ __launch_bounds__(256) void gd_chunk_carry_kernel(GDChunk a) {
     for (int k4 = 0; k4 < 4; ++k4) u4[k4] = *reinterpret_cast<const f32x4*>(&us[li * GDC_P + 16 * k4 + 4 * lg]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int k4 = 0; k4 < 4; ++k4)
+    for (int k4 = 0; k4 < 4; ++k4) {
 #pragma unroll
-      for (int y = 0; y < 4; ++y)
+      for (int i = 0; i < 4; i += 2) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) S[dt] = mfma4(x.kd[dt][k4][y], u4[k4][y], S[dt]);
+        for (int m = i; m < i + 2; ++m)
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) S[dt] = mfma4(x.kd[dt][k4][m], u4[k4][m], S[dt]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (DT == 2 || i == 0) fetch_kd(next, y, DT == 2 ? i >> 1 : 0, k4);
+        if (k4 == 3 && i == 0) fetch_rest(next, y);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
     if (x.bad_token < CHUNK || x.bad_value < CHUNK)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) S[dt] = f32x4{NAN, NAN, NAN, NAN};
   };
   GDCarry<DP> x0, x1;
-  fetch(0, x0);
+  {
+    const int64_t unit = unit_of(0);
+#pragma unroll
+    for (int k8 = 0; k8 < DP / 32; ++k8) fetch_w(unit, x0, k8, 0), fetch_w(unit, x0, k8, 1);
+#pragma unroll
+    for (int k4 = 0; k4 < 4; ++k4)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) fetch_kd(unit, x0, dt, k4);
+    fetch_rest(unit, x0);
+  }
   for (int c = 0; c < nc; c += 2) {
-    fetch(c + 1, x1);
-    step(c, x0);
+    step(c, x0, x1);
     if (c + 1 >= nc) break;
-    fetch(c + 2, x0);
-    step(c + 1, x1);
+    step(c + 1, x1, x0);
   }
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -520,21 +611,21 @@ __global__ __launch_bounds__(256) void gd_chunk_out_kernel(GDChunk a) {
 #pragma unroll
   for (int k8 = 0; k8 < DP / 32; ++k8)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) q[k8][u] = *reinterpret_cast<const f32x4*>(a.qg + unit * CHUNK * DP + tok * DP + 32 * k8 + 8 * lg + 4 * u);
+    for (int u = 0; u < 2; ++u) q[k8][u] = *reinterpret_cast<const f32x4*>(a.qg + unit * CHUNK * DP + qt * 16 * DP + (2 * k8 + u) * 256 + lane * 4);
 #pragma unroll
   for (int jt = 0; jt < 4; ++jt)
-    if (jt <= qt) b[jt] = *reinterpret_cast<const f32x4*>(a.bm + unit * CHUNK * CHUNK + tok * CHUNK + jt * 16 + 4 * lg);
+    if (jt <= qt) b[jt] = *reinterpret_cast<const f32x4*>(a.bm + unit * CHUNK * CHUNK + (qt * 4 + jt) * 256 + lane * 4);
   const int bad_token = a.bad_token[unit];
   float* o = p.out + ((int64_t)p.q_start[s] + c * CHUNK + tok) * ((int64_t)p.heads * p.vdim) + (int64_t)h * p.vdim + c0;
 #pragma unroll
   for (int ct = 0; ct < 4; ++ct) {
     if (ct >= nct) break;
-    const int64_t colrow = unit * a.vpad + c0 + ct * 16 + li;
+    const int64_t colrow = unit * a.vpad + c0 + ct * 16;
     f32x4 acc = {}, acc2 = {};
 #pragma unroll
     for (int k8 = 0; k8 < DP / 32; ++k8) {
-      const float* sp = a.st + colrow * DP + 32 * k8 + 8 * lg;
-      const f32x4 s0 = *reinterpret_cast<const f32x4*>(sp), s1 = *reinterpret_cast<const f32x4*>(sp + 4);
+      const float* sp = a.st + colrow * DP + k8 * 512 + lane * 4;
+      const f32x4 s0 = *reinterpret_cast<const f32x4*>(sp), s1 = *reinterpret_cast<const f32x4*>(sp + 256);
 #pragma unroll
       for (int y = 0; y < 4; ++y) acc = mfma4(s0[y], q[k8][0][y], acc);
 #pragma unroll
@@ -543,17 +634,18 @@ __global__ __launch_bounds__(256) void gd_chunk_out_kernel(GDChunk a) {
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt) {
       if (jt > qt) break;
-      const f32x4 u = *reinterpret_cast<const f32x4*>(a.ut + colrow * CHUNK + jt * 16 + 4 * lg);
+      const f32x4 u = *reinterpret_cast<const f32x4*>(a.ut + colrow * CHUNK + jt * 256 + lane * 4);
 #pragma unroll
       for (int y = 0; y < 4; ++y) acc = mfma4(u[y], b[jt][y], acc);
     }
     if (tok >= cnt) continue;
     const int e = ct * 16 + 4 * lg;
+    const i32x4 bad = *reinterpret_cast<const i32x4*>(&a.bad_value[unit * a.vpad + c0 + e]);
     f32x4 x;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       x[r] = acc[r] + acc2[r];
-      if (tok >= bad_token || tok >= a.bad_value[unit * a.vpad + c0 + e + r]) x[r] = NAN;
+      if (tok >= bad_token || tok >= bad[r]) x[r] = NAN;
     }
     if ((p.vdim & 3) == 0) {
       if (c0 + e < p.vdim) *reinterpret_cast<f32x4*>(o + e) = x;

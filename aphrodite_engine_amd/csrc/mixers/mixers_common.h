@@ -136,7 +136,15 @@ __device__ __forceinline__ float gelu_tanh_f(float z) {
   const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
   return 0.5f * z * (1.0f + tanhf(u));
 }
-__device__ __forceinline__ float softplus_f(float z) { return z > 20.f ? z : log1pf(expf(z)); }
+// log(1 + e^z) = max(z, 0) + 2 atanh(y), y = x / (2 + x), x = e^-|z|: y in two numbers, atanh by its series in y^2 (coefficients fitted by least squares
+// over y <= 1 / 3, 1e-10).  Largest error 2.04 x 2^-24, root mean square 0.47 (log1p(e^z) with both rounded correctly: 1.98, 0.46), a fifth of
+// log1pf's instructions and no branch.
+__device__ __forceinline__ float softplus_f(float z) {
+  const float x = expf(-fabsf(z)), d = x + 2.f, dl = x - (d - 2.f), r = __builtin_amdgcn_rcpf(d);
+  const float y = x * r, yl = fmaf(-y, dl, fmaf(-y, d, x)) * r, t = y * y;
+  const float s = fmaf(fmaf(fmaf(fmaf(0.12120297f, t, 0.10722389f), t, 0.14307591f), t, 0.19999473f), t, 0.33333337f);
+  return fmaxf(z, 0.f) + (2.f * y + fmaf(2.f * y * t, s, 2.f * yl));
+}
 // log(sigmoid(z)) without overflow on either side
 __device__ __forceinline__ float log_sigmoid_f(float z) {
   return fminf(z, 0.f) - log1pf(expf(-fabsf(z)));

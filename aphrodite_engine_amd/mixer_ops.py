@@ -873,14 +873,14 @@ DELTA_CHUNKED_FROM, DELTA_CHUNKED_MIN = 128, 32
 
 
 def delta_chunks_pay(tokens: int, segments: int, longest: int, heads: int, dim: int, vdim: int, channel: bool) -> bool:
-    """Whether the chunked delta rule is expected to be the faster by a tenth, from times measured on MI355X (420 batches of 1 to 64 segments of 96 to
-    2048 tokens, 4 to 48 heads of 64 x 64 to 96 x 192: none of those it takes is slower than the scan; 816 of 1 to 16 segments beside 1 to 56 single
-    tokens: four are, by 3 to 5 %, and the mean gain is 1.51 of 1.64 that the better form each time would give).  The scan is bound by the longest segment's
-    chain of tokens or, where there are many segments and heads, by what all tokens take of the vector ALUs; the chunks by their preparation,
-    a workgroup a CU, and their products, more work than the scan's but with a chain a tenth as long.  Scan / chunks in us: one segment of
-    512 tokens, 16 heads of 128, a decay per channel 246 / 88, per head 175 / 78; sixteen of 256 444 / 336, 274 / 298; sixteen of 256, 48 heads of
-    64 382 / 554, 284 / 455.  Segments too short for chunks, decoded rows beside prompt portions, are scanned whichever it is: at most twice as
-    many as ``longest`` goes into ``tokens`` count as long (four of 551 beside 24 rows, 32 heads of 128, a decay per channel 702 / 440; with
+    """Whether the chunked delta rule is expected to be the faster by a tenth, from times measured on MI355X (113 batches of 1 to 32 segments of 96 to
+    2048 tokens, 4 to 48 heads of 64 x 64 to 128 x 192: of those it takes one is slower than the scan, by 7 %; 132 of 1 to 16 segments beside 0 to 56 single
+    tokens: one is, by 8 %; the mean gains are 1.71 and 1.95 of 1.73 and 2.04 that the better form each time would give).  The scan is bound by the
+    longest segment's chain of tokens or, where there are many segments and heads, by what all tokens take of the vector ALUs; the chunks by their
+    preparation, a workgroup a CU, and their products, more work than the scan's but with a chain a tenth as long.  Scan / chunks in us: one segment
+    of 512 tokens, 16 heads of 128, a decay per channel 193 / 64, per head 173 / 61; sixteen of 256 340 / 260, 258 / 241; sixteen of 256, 48 heads of
+    64 286 / 420, 254 / 388.  Segments too short for chunks, decoded rows beside prompt portions, are scanned whichever it is: at most twice as
+    many as ``longest`` goes into ``tokens`` count as long (four of 551 beside 24 rows, 32 heads of 128, a decay per channel 557 / 340; with
     all 28 counted the scan was taken)."""
     wide = dim > 64
     chain = longest * ((0.48 if channel else 0.35) if wide else (0.34 if channel else 0.29))
@@ -892,8 +892,8 @@ def delta_chunks_pay(tokens: int, segments: int, longest: int, heads: int, dim: 
             work *= min(math.gcd(segments // 8, 32), segments / longs)
     scan = 8 + (chain ** 4 + work ** 4) ** 0.25
     units = (tokens / 64 + min(longs, tokens / 32) / 2) * heads                 # (segments that end in half a chunk, on the average)
-    prepare = (27.5 + 10 * channel if wide else 16 + 8 * channel) * math.ceil(units / 256)
-    chunks = 17.5 + (1.2 if wide else 0.6) * ((longest + 63) // 64) + prepare + (23 if wide else 17) * units * ((vdim + 63) // 64) / 256
+    prepare = (20.2 + 1.6 * channel if wide else 9.5 + 2.5 * channel) * math.ceil(units / 256)
+    chunks = 22 + (0.4 if wide else 0.6) * ((longest + 63) // 64) + prepare + (16 if wide else 13.5) * units * ((vdim + 63) // 64) / 256
     if 10 * tokens < 9 * segments * longest:                                    # (not all as long: some may be scanned beside them)
         chunks += 20 + max(0, segments - longs) * heads * ((vdim + 15) // 16) * 6e-3
     return 1.1 * chunks < scan
