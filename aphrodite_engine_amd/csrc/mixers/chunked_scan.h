@@ -12,6 +12,12 @@ constexpr int CHUNK = 64;
 // here lane group g = l / 16 brings four (or eight) NEIGHBOURING k per load and one of them per call.
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
+// A matrix of DP columns in the fragments that fp32 and 16-bit products read: 1 KiB each, a lane's four numbers next to each other.  Lane (li, lg) =
+// (l % 16, l / 16) of fragment (i, 2 j + u) has row 16 i + li, columns 32 j + 8 lg + 4 u + (0..3).  As rows, a load of 16 bytes a lane would meet another
+// cache line in every lane of four.  Here: where the lane's columns 16 j + 4 lg + (0..3) of row 16 i + li begin, as a 16 x 16 product leaves them.
+template <int DP>
+__device__ __forceinline__ int frag8(int i, int j, int li, int lg) { return (i * (DP / 16) + (j & ~1) + (lg & 1)) * 256 + (((j & 1) * 2 + (lg >> 1)) * 16 + li) * 4; }
+
 // A barrier for what lies in LDS only: __syncthreads() also waits for the loads from memory that are still on their way.
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -52,9 +52,6 @@ struct GDChunk {
   int32_t* bad_value;      // [chunks, heads, vpad]    first value, or u, of the column that is not finite (64: none)
 };
 
-// Where, in an array marked *, the lane's columns 16 j + 4 lg + (0..3) of row 16 i + li begin.
-template <int DP>
-__device__ __forceinline__ int frag8(int i, int j, int li, int lg) { return (i * (DP / 16) + (j & ~1) + (lg & 1)) * 256 + (((j & 1) * 2 + (lg >> 1)) * 16 + li) * 4; }
 // x of lane I of the own sixteen.
 template <int I>
 __device__ __forceinline__ float of_lane16(float x) {

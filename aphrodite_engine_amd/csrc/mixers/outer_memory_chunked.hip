@@ -17,7 +17,8 @@
 // segment to a workgroup (the *16 kernels).
 // Outputs lie as the products leave them: scores as K Q^T and results as V^T P^T, so that a score's registers are the next product's
 // operand and a lane holds four neighbouring value columns of one token.  Row pitches are 4 floats over a multiple of 32: the
-// eight lanes that a 16-byte LDS access serves at a time fall on all 32 banks.
+// eight lanes that a 16-byte LDS access serves at a time fall on all 32 banks.  The states lie in fragments: as rows of DP, the address unit took four times
+// as long over a load (state space 64 heads, 600 / 2000 / 4096 tokens 51 / 73 / 116 -> 46 / 67 / 111 us, decay 16 x 64 x 128, 4096 tokens 92 -> 89).
 #include "outer_memory.h"
 #include "chunked_scan.h"
 
@@ -32,7 +33,7 @@ struct OMChunk {
   int group;              // chunks that a workgroup takes in turn (bf16 inputs' kernels; 1 elsewhere): below, and where states are numbered, a chunk is a group of so many
   int chunk0, span;       // the chunks of these launches (below: [chunks] of one span)
   int vpad;               // vdim rounded up to 16
-  float* u;               // [chunks, heads, vpad, DP] U, then the state ahead of the chunk
+  float* u;               // [chunks, heads] vpad x DP in fragments (frag8): U, then the state ahead of the chunk
   float* un;              // mLSTM: [chunks, heads, DP], the same of the normaliser
   float* total;           // [chunks, heads] decay over the chunk
   float *la, *gb, *em;    // mLSTM: [heads, tokens] log decay, write strength, e^{-m}
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(256) void om_chunk_update_kernel(OMChunk a) {
     if (ct >= nct) break;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
-      *reinterpret_cast<f32x4*>(&u[(ct * 16 + li) * DP + (wave * DT + dt) * 16 + 4 * lg]) = acc[dt][ct];
+      *reinterpret_cast<f32x4*>(&u[frag8<DP>(ct, wave * DT + dt, li, lg)]) = acc[dt][ct];
   }
   if (MODE == 1 && blockIdx.z == 0 && tid < DP) {
     float sum = 0.f;
@@ -412,11 +413,11 @@ __global__ __launch_bounds__(256) void om_chunk_update16_kernel(OMChunk a) {
   if (g.c0 == 0 && tid == 0) a.total[at] = total;
   if (MODE == 1 && g.c0 == 0 && tid < DP) a.un[at * DP + tid] = sn;
   if (wave >= nct) return;
-  float* u = a.u + (at * a.vpad + g.c0 + wave * 16 + li) * DP + 8 * lg;
+  float* u = a.u + (at * a.vpad + g.c0 + wave * 16) * DP + lane * 4;
 #pragma unroll
   for (int kk = 0; kk < DP / 32; ++kk)
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf) *reinterpret_cast<f32x4*>(u + 32 * kk + 4 * hf) = S[kk][hf];
+    for (int hf = 0; hf < 2; ++hf) *reinterpret_cast<f32x4*>(u + (2 * kk + hf) * 256) = S[kk][hf];
 }
 
 // ---- 2. the state through the chunks -------------------------------------------------------------------------------------------------
@@ -451,14 +452,14 @@ __global__ __launch_bounds__(64) void om_chunk_carry_kernel(OMChunk a) {
     return;
   }
   if (x >= quads) return;
-  const int e = x / (DP / 4), d = (x % (DP / 4)) * 4;
+  const int l = x & 63, f = x >> 6, e = f / (DP / 16) * 16 + (l & 15), d = (f % (DP / 16) >> 1) * 32 + (l >> 4) * 8 + (f & 1) * 4;
   float* sb = p.state_s + ((int64_t)slot * p.heads + h) * p.dim * (int64_t)p.vdim + e;
   f32x4 S = {};
   if (!fresh && e < p.vdim)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (d + i < p.dim) S[i] = sb[(int64_t)(d + i) * p.vdim];
-  float* u = a.u + (first * p.heads + h) * a.vpad * (int64_t)DP + (int64_t)e * DP + d;
+  float* u = a.u + (first * p.heads + h) * a.vpad * (int64_t)DP + 4 * x;
   const int64_t step = (int64_t)p.heads * a.vpad * DP;
   constexpr int AHEAD = 8;
   f32x4 w[2][AHEAD];
@@ -540,10 +541,10 @@ __global__ __launch_bounds__(256) void om_chunk_out_kernel(OMChunk a) {
 #pragma unroll
   for (int ct = 0; ct < OMC_COLS / 16; ++ct) {
     if (ct >= nct) break;
-    const float* sr = st + (ct * 16 + li) * DP + 8 * lg;
+    const float* sr = st + ct * 16 * DP + lane * 4;
 #pragma unroll
     for (int kk = 0; kk < DP / 32; ++kk) {
-      const f32x4 s0 = *reinterpret_cast<const f32x4*>(sr + 32 * kk), s1 = *reinterpret_cast<const f32x4*>(sr + 32 * kk + 4);
+      const f32x4 s0 = *reinterpret_cast<const f32x4*>(sr + kk * 512), s1 = *reinterpret_cast<const f32x4*>(sr + kk * 512 + 256);
 #pragma unroll
       for (int m = 0; m < 4; ++m) acc[ct] = mfma4(s0[m], q[kk][m], acc[ct]);
 #pragma unroll
@@ -719,11 +720,11 @@ __global__ __launch_bounds__(256, 2) void om_chunk_out16_kernel(OMChunk a) {
   const int64_t at = (int64_t)g.x * p.heads + g.h;
   f32x4 S[DP / 32][2] = {};
   if (wave < nct) {
-    const float* u = a.u + (at * a.vpad + g.c0 + wave * 16 + li) * DP + 8 * lg;
+    const float* u = a.u + (at * a.vpad + g.c0 + wave * 16) * DP + lane * 4;
 #pragma unroll
     for (int kk = 0; kk < DP / 32; ++kk)
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) S[kk][hf] = *reinterpret_cast<const f32x4*>(u + 32 * kk + 4 * hf);
+      for (int hf = 0; hf < 2; ++hf) S[kk][hf] = *reinterpret_cast<const f32x4*>(u + (2 * kk + hf) * 256);
   }
   float sn = 0.f;
   if (MODE == 1 && tid < DP) ns[tid] = sn = a.un[at * DP + tid];
