@@ -25,34 +25,46 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-__device__ __forceinline__ int wave_incl_sum(int v, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(v, o, 64);
-    if (lane >= o) v += u;
-  }
+// Inclusive prefix sum over the wave: within sixteens, then the sixteens ahead (lane choices inside the instruction; by way of LDS the six steps took
+// 600 cycles of a chunk).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int from_lane(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false); }
+__device__ __forceinline__ int wave_incl_sum(int v) {
+  v += from_lane<0x111, 0xf>(v);       // row_shr 1, 2, 4, 8
+  v += from_lane<0x112, 0xf>(v);
+  v += from_lane<0x114, 0xf>(v);
+  v += from_lane<0x118, 0xf>(v);
+  v += from_lane<0x142, 0xa>(v);       // row_bcast 15 to rows 1 and 3, 31 to rows 2 and 3
+  v += from_lane<0x143, 0xc>(v);
   return v;
 }
 
 // (In what follows a unit is a chunk, or a group of chunks of one segment.)
 __device__ __forceinline__ int chunks_of(int n, int min_len, int unit = CHUNK) { return n >= min_len ? (n + unit - 1) / unit : 0; }
 
-// Chunk ``id`` of the batch's segments of at least min_len tokens, counted in order -> segment s and chunk c of it; false: there are
-// fewer.  Every wave of a workgroup works it out for itself (64 segments a step).
-__device__ __forceinline__ bool locate_chunk(int id, const int32_t* __restrict__ q_len, int num_seqs, int min_len, int& s, int& c, int unit = CHUNK) {
+// Chunk ``id`` of the batch's segments of at least min_len tokens, counted in order: segment s, chunk c of it, and what the segment is; false: there are
+// fewer.  Every wave of a workgroup works it out for itself (64 segments a step); what the segment is comes with the lengths, not behind them -- at the
+// start of a launch a load takes 1 700 cycles.
+struct ChunkPlace {
+  int s, c, len, start, slot;
+};
+template <typename P>
+__device__ __forceinline__ bool locate_chunk(int id, const P& p, int min_len, ChunkPlace& at, int unit = CHUNK) {
   const int lane = threadIdx.x & 63;
   int before = 0;
-  for (int s0 = 0; s0 < num_seqs; s0 += 64) {
-    const int cnt = s0 + lane < num_seqs ? chunks_of(q_len[s0 + lane], min_len, unit) : 0;
-    const int incl = wave_incl_sum(cnt, lane) + before;
+  for (int s0 = 0; s0 < p.num_seqs; s0 += 64) {
+    const int seg = min(s0 + lane, p.num_seqs - 1), len = p.q_len[seg], start = p.q_start[seg], slot = p.slot_of_seq[seg];
+    const int cnt = s0 + lane < p.num_seqs ? chunks_of(len, min_len, unit) : 0;
+    const int incl = wave_incl_sum(cnt) + before;
     const uint64_t past = __ballot(incl > id);
     if (past) {
       const int l = __ffsll((unsigned long long)past) - 1;
-      s = __builtin_amdgcn_readfirstlane(s0 + l);
-      c = __builtin_amdgcn_readfirstlane(id - (__shfl(incl, l, 64) - __shfl(cnt, l, 64)));
+      at.s = s0 + l;
+      at.c = id - (__builtin_amdgcn_readlane(incl, l) - __builtin_amdgcn_readlane(cnt, l));
+      at.len = __builtin_amdgcn_readlane(len, l), at.start = __builtin_amdgcn_readlane(start, l), at.slot = __builtin_amdgcn_readlane(slot, l);
       return true;
     }
-    before = __shfl(incl, 63, 64);
+    before = __builtin_amdgcn_readlane(incl, 63);
   }
   return false;
 }
@@ -61,7 +73,7 @@ __device__ __forceinline__ bool locate_chunk(int id, const int32_t* __restrict__
 __device__ __forceinline__ int chunks_before(int s, const int32_t* __restrict__ q_len, int min_len, int unit = CHUNK) {
   const int lane = threadIdx.x & 63;
   int sum = 0;
-  for (int s0 = 0; s0 < s; s0 += 64) sum += __shfl(wave_incl_sum(s0 + lane < s ? chunks_of(q_len[s0 + lane], min_len, unit) : 0, lane), 63, 64);
+  for (int s0 = 0; s0 < s; s0 += 64) sum += __builtin_amdgcn_readlane(wave_incl_sum(s0 + lane < s ? chunks_of(q_len[s0 + lane], min_len, unit) : 0), 63);
   return __builtin_amdgcn_readfirstlane(sum);
 }
 
@@ -101,13 +113,24 @@ inline int64_t span_workspace(int64_t chunks, F floats) {
 }
 
 // Inclusive prefix sum over the wave, in 64 bits: differences of two prefixes keep a small decay exact behind a large one.
-__device__ __forceinline__ double wave_incl_sum(double v, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const double u = __shfl_up(v, o, 64);
-    if (lane >= o) v += u;
-  }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double from_lane(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)from_lane<CTRL, ROWS>((int)(uint32_t)b), hi = (uint32_t)from_lane<CTRL, ROWS>((int)(uint32_t)(b >> 32));
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double wave_incl_sum(double v) {
+  v += from_lane<0x111, 0xf>(v);
+  v += from_lane<0x112, 0xf>(v);
+  v += from_lane<0x114, 0xf>(v);
+  v += from_lane<0x118, 0xf>(v);
+  v += from_lane<0x142, 0xa>(v);
+  v += from_lane<0x143, 0xc>(v);
   return v;
+}
+__device__ __forceinline__ double of_lane(double v, int l) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l));
 }
 
 // 2^t for a difference of two prefixes.  Rounding t to fp32 costs |t| 2^-24 of a factor of size 2^t: half an ulp of one at the most.

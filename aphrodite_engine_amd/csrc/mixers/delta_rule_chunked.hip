@@ -104,13 +104,13 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
   int* bad_col = (int*)(red + 2 * NW * CHUNK);   // [64]
   int* bad_tok = bad_col + CHUNK;          // [1]
   const GatedDelta& p = a.p;
-  int s, c;
-  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
-  const int slot = p.slot_of_seq[s];
+  ChunkPlace at;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p, a.min_len, at) || at.slot < 0 || at.slot >= p.num_slots) return;
+  const int c = at.c;
   const int h = blockIdx.y, hk = h / (p.heads / p.kv_heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
-  const int cnt = min(CHUNK, p.q_len[s] - c * CHUNK);
-  const int64_t row0 = (int64_t)p.q_start[s] + c * CHUNK, row = row0 + min(lane, cnt - 1);
+  const int cnt = min(CHUNK, at.len - c * CHUNK);
+  const int64_t row0 = (int64_t)at.start + c * CHUNK, row = row0 + min(lane, cnt - 1);
   const int64_t unit = (int64_t)blockIdx.x * p.heads + h;
   const bool live = lane < cnt;
   // -- q, k, g, beta: lane = token, the waves divide the key channels
@@ -134,7 +134,6 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
         for (int i = 0; i < 8; ++i) bias[it][i] = p.dt_bias[(int64_t)h * p.dim + min(wave * 16 + it * 8 + i, p.dim - 1)];
     const float raw_b = T::to_f32(((const ST*)p.b)[row * p.b_stride + h]);
     const float rate = -expf(p.a_log[h]);
-    if (slot < 0 || slot >= p.num_slots) return;
     float sq = 0.f, sk = 0.f;
 #pragma unroll
     for (int it = 0; it < 2; ++it)
@@ -594,13 +593,12 @@ __global__ __launch_bounds__(256) void gd_chunk_carry_kernel(GDChunk a) {
 template <int DP>
 __global__ __launch_bounds__(256) void gd_chunk_out_kernel(GDChunk a) {
   const GatedDelta& p = a.p;
-  int s, c;
-  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
-  const int slot = p.slot_of_seq[s];
-  if (slot < 0 || slot >= p.num_slots) return;
+  ChunkPlace at;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p, a.min_len, at) || at.slot < 0 || at.slot >= p.num_slots) return;
+  const int c = at.c;
   const int h = blockIdx.y, c0 = blockIdx.z * 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
-  const int cnt = min(CHUNK, p.q_len[s] - c * CHUNK);
+  const int cnt = min(CHUNK, at.len - c * CHUNK);
   const int64_t unit = (int64_t)blockIdx.x * p.heads + h;
   const int qt = (wave + blockIdx.x + blockIdx.y) & 3, tok = qt * 16 + li;       // (later tokens see more: the long tiles go round the SIMDs)
   const int nct = min(4, (p.vdim - c0 + 15) >> 4);
@@ -613,7 +611,7 @@ __global__ __launch_bounds__(256) void gd_chunk_out_kernel(GDChunk a) {
   for (int jt = 0; jt < 4; ++jt)
     if (jt <= qt) b[jt] = *reinterpret_cast<const f32x4*>(a.bm + unit * CHUNK * CHUNK + (qt * 4 + jt) * 256 + lane * 4);
   const int bad_token = a.bad_token[unit];
-  float* o = p.out + ((int64_t)p.q_start[s] + c * CHUNK + tok) * ((int64_t)p.heads * p.vdim) + (int64_t)h * p.vdim + c0;
+  float* o = p.out + ((int64_t)at.start + c * CHUNK + tok) * ((int64_t)p.heads * p.vdim) + (int64_t)h * p.vdim + c0;
 #pragma unroll
   for (int ct = 0; ct < 4; ++ct) {
     if (ct >= nct) break;

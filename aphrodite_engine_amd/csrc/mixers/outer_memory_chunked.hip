@@ -18,7 +18,9 @@
 // Outputs lie as the products leave them: scores as K Q^T and results as V^T P^T, so that a score's registers are the next product's
 // operand and a lane holds four neighbouring value columns of one token.  Row pitches are 4 floats over a multiple of 32: the
 // eight lanes that a 16-byte LDS access serves at a time fall on all 32 banks.  The states lie in fragments: as rows of DP, the address unit took four times
-// as long over a load (state space 64 heads, 600 / 2000 / 4096 tokens 51 / 73 / 116 -> 46 / 67 / 111 us, decay 16 x 64 x 128, 4096 tokens 92 -> 89).
+// as long over a load (state space 64 heads, 600 / 2000 / 4096 tokens 51 / 73 / 116 -> 46 / 67 / 111 us, decay 16 x 64 x 128, 4096 tokens 92 -> 89).  A
+// third of a launch is the way to its first numbers; with a segment's place beside its length, prefix sums without LDS and a fixed decay's
+// as multiples 42 / 66 / 103, 87.
 #include "outer_memory.h"
 #include "chunked_scan.h"
 
@@ -133,6 +135,13 @@ __device__ __forceinline__ void chunk_gate(const OMChunk& a, int h, int64_t row0
   }
 }
 
+// Sums of the log decays up to each lane's token: a fixed decay's are multiples.
+template <int MODE>
+__device__ __forceinline__ double chunk_decays(double la, int lane, int cnt) {
+  if constexpr (MODE == 0) return of_lane(la, 0) * (double)(min(lane, cnt - 1) + 1);
+  else return wave_incl_sum(la);
+}
+
 template <int MODE>
 __device__ __forceinline__ float act_k(float x) { return MODE == 0 ? silu_f(x) : x; }
 
@@ -143,14 +152,13 @@ __global__ __launch_bounds__(256) void om_chunk_update_kernel(OMChunk a) {
   __shared__ __attribute__((aligned(16))) float kt[DP * OMC_PITCH];
   __shared__ __attribute__((aligned(16))) float vt[OMC_COLS * OMC_PITCH];
   const OuterMemory& p = a.p;
-  int s, c;
-  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
-  const int slot = p.slot_of_seq[s];
-  if (slot < 0 || slot >= p.num_slots) return;
+  ChunkPlace at;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p, a.min_len, at) || at.slot < 0 || at.slot >= p.num_slots) return;
+  const int c = at.c;
   const int h = blockIdx.y, c0 = blockIdx.z * OMC_COLS, hk = MODE == 2 ? h / (p.heads / p.qk_heads) : h;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int cnt = min(CHUNK, p.q_len[s] - c * CHUNK);
-  const int64_t row0 = (int64_t)p.q_start[s] + c * CHUNK;
+  const int cnt = min(CHUNK, at.len - c * CHUNK);
+  const int64_t row0 = (int64_t)at.start + c * CHUNK;
   // lane = token; the four waves divide the key numbers and the value columns.  Every load is on its way before the first is used.
   const int64_t row = row0 + min(lane, cnt - 1);
   const ST* kr = (const ST*)p.k + row * p.k_stride + (int64_t)hk * p.dim;
@@ -163,7 +171,7 @@ __global__ __launch_bounds__(256) void om_chunk_update_kernel(OMChunk a) {
   double la;
   float b;
   chunk_gate<T, MODE>(a, h, row0, lane, cnt, la, b);
-  const double g = wave_incl_sum(la, lane), gend = __shfl(g, 63, 64);
+  const double g = chunk_decays<MODE>(la, lane, cnt), gend = of_lane(g, 63);
   float w = exp2_d(gend - g) * b, all = exp2_d(gend);
   if (MODE == 0 && p.decay[h] < 0.f) {
     if ((cnt - 1 - lane) & 1) w = -w;
@@ -336,13 +344,12 @@ __device__ __forceinline__ bool locate_group(const OMChunk& a, OMGroup& w) {
   const int idx = blockIdx.x >> 3, pair = idx / (heads * blocks) * 8 + (blockIdx.x & 7), sub = idx % (heads * blocks);
   if (pair >= a.span * key_heads) return false;
   w.x = pair % a.span, w.hk = pair / a.span, w.h = w.hk * heads + sub / blocks, w.c0 = sub % blocks * OMC_COLS;
-  int s, g;
-  if (!locate_chunk(a.chunk0 + w.x, p.q_len, p.num_seqs, a.min_len, s, g, a.group * CHUNK)) return false;
-  const int slot = p.slot_of_seq[s], first = g * a.group * CHUNK;
-  if (slot < 0 || slot >= p.num_slots) return false;
-  w.tokens = min(a.group * CHUNK, p.q_len[s] - first);
+  ChunkPlace at;
+  if (!locate_chunk(a.chunk0 + w.x, p, a.min_len, at, a.group * CHUNK) || at.slot < 0 || at.slot >= p.num_slots) return false;
+  const int first = at.c * a.group * CHUNK;
+  w.tokens = min(a.group * CHUNK, at.len - first);
   w.chunks = (w.tokens + CHUNK - 1) / CHUNK;
-  w.row0 = (int64_t)p.q_start[s] + first;
+  w.row0 = (int64_t)at.start + first;
   return true;
 }
 
@@ -377,7 +384,7 @@ __global__ __launch_bounds__(256) void om_chunk_update16_kernel(OMChunk a) {
       double la;
       float b;
       chunk_gate<BFloat, MODE>(a, g.h, g.row0 + (c + wave) * CHUNK, lane, g.tokens - (c + wave) * CHUNK, la, b);
-      const double gi = wave_incl_sum(la, lane), gend = __shfl(gi, 63, 64);
+      const double gi = wave_incl_sum(la), gend = of_lane(gi, 63);
       ws[wave][lane] = exp2_d(gend - gi) * b;
       if (lane == 0) alls[wave] = exp2_d(gend);
     }
@@ -504,14 +511,13 @@ __global__ __launch_bounds__(256) void om_chunk_out_kernel(OMChunk a) {
   __shared__ double gs[CHUNK];
   __shared__ float bs[CHUNK];
   const OuterMemory& p = a.p;
-  int s, c;
-  if (!locate_chunk(a.chunk0 + blockIdx.x, p.q_len, p.num_seqs, a.min_len, s, c)) return;
-  const int slot = p.slot_of_seq[s];
-  if (slot < 0 || slot >= p.num_slots) return;
+  ChunkPlace at;
+  if (!locate_chunk(a.chunk0 + blockIdx.x, p, a.min_len, at) || at.slot < 0 || at.slot >= p.num_slots) return;
+  const int c = at.c;
   const int h = blockIdx.y, c0 = blockIdx.z * OMC_COLS, hk = MODE == 2 ? h / (p.heads / p.qk_heads) : h;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
-  const int cnt = min(CHUNK, p.q_len[s] - c * CHUNK);
-  const int64_t row0 = (int64_t)p.q_start[s] + c * CHUNK;
+  const int cnt = min(CHUNK, at.len - c * CHUNK);
+  const int64_t row0 = (int64_t)at.start + c * CHUNK;
   const int64_t row = row0 + min(lane, cnt - 1);
   const ST* kr = (const ST*)p.k + row * p.k_stride + (int64_t)hk * p.dim;
   const ST* vr = (const ST*)p.v + row * p.v_stride + (int64_t)h * p.vdim + c0;
@@ -521,6 +527,13 @@ __global__ __launch_bounds__(256) void om_chunk_out_kernel(OMChunk a) {
   for (int it = 0; it < DP / 32; ++it) load8<T, VEC>(kr, wave * (DP / 4) + it * 8, p.dim, kx[it]);
 #pragma unroll
   for (int it = 0; it < OMC_COLS / 32; ++it) load8<T, VEC>(vr, wave * (OMC_COLS / 4) + it * 8, p.vdim - c0, vx[it]);
+  if (wave == 0) {                                                       // (while they are)
+    double la;
+    float b;
+    chunk_gate<T, MODE>(a, h, row0, lane, cnt, la, b);
+    gs[lane] = chunk_decays<MODE>(la, lane, cnt);
+    bs[lane] = b;
+  }
   // a wave's sixteen queries: lane li's query, eight neighbouring numbers a step.  Later queries see more tokens: the tiles go round the
   // waves from workgroup to workgroup, so that no SIMD has all the long ones.
   const int qt = (wave + blockIdx.x + blockIdx.y) & 3, qi = qt * 16 + li;
@@ -573,13 +586,6 @@ __global__ __launch_bounds__(256) void om_chunk_out_kernel(OMChunk a) {
       odd |= !finite_f(val);
       vt[(e + i) * OMC_PITCH + lane] = val;
     }
-  }
-  if (wave == 0) {
-    double la;
-    float b;
-    chunk_gate<T, MODE>(a, h, row0, lane, cnt, la, b);
-    gs[lane] = wave_incl_sum(la, lane);
-    bs[lane] = b;
   }
   odd = __syncthreads_or(odd);
   const bool neg = MODE == 0 && p.decay[h] < 0.f;
@@ -736,7 +742,7 @@ __global__ __launch_bounds__(256, 2) void om_chunk_out16_kernel(OMChunk a) {
       double la;
       float b;
       chunk_gate<BFloat, MODE>(a, g.h, g.row0 + (c + wave) * CHUNK, lane, g.tokens - (c + wave) * CHUNK, la, b);
-      const double gi = wave_incl_sum(la, lane), gend = __shfl(gi, 63, 64);
+      const double gi = wave_incl_sum(la), gend = of_lane(gi, 63);
       gs[wave][lane] = gi;
       bs[wave][lane] = b;
       ws[wave][lane] = exp2_d(gend - gi) * b;
