@@ -130,8 +130,16 @@ __device__ __forceinline__ void lds_row(const float* p, float (&o)[NI]) {
 bool group_rms_norm_launch(void* out, int64_t out_stride, const float* x, const void* weight, bool shared, const void* gate, int64_t gate_stride,
                            int64_t rows, int n, int group, float eps, float out_scale, int act, int dtype, hipStream_t stream);
 
-__device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + __expf(-z)); }
-__device__ __forceinline__ float silu_f(float z) { return z / (1.0f + __expf(-z)); }
+// n / (1 + e^-z): the reciprocal's product, one correction and the hardware's rules for zeros, infinities and NaN, without a division's scaling (ten
+// instructions for six): the same bits for every z from 1.2e-38 on, of 4 million over all exponents.  Both sides in quarters, as the reciprocal of
+// 2^126 and more would be taken for zero.  Where the vector units bound: decay memories of 4096 tokens, 16 heads, 86.6 -> 83.9 us, a convolution of
+// 2024 rows 18.5 -> 17.6.
+__device__ __forceinline__ float over_1_exp_f(float n, float z) {
+  const float d = fmaf(__expf(-z), 0.25f, 0.25f), m = 0.25f * n, r = __builtin_amdgcn_rcpf(d), q = m * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, d, m), r, q), d, m);
+}
+__device__ __forceinline__ float sigmoid_f(float z) { return over_1_exp_f(1.0f, z); }
+__device__ __forceinline__ float silu_f(float z) { return over_1_exp_f(z, z); }
 __device__ __forceinline__ float gelu_tanh_f(float z) {
   const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
   return 0.5f * z * (1.0f + tanhf(u));
