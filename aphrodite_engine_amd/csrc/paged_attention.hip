@@ -1066,7 +1066,8 @@ __global__ __launch_bounds__(256) void reshape_and_cache_window_kernel(
 // the sum by itself (wna16_rows_reduce_kernel's bits).  int4 steps, us, sum and rotation / here: 150 scattered tokens 5.2 + 7.4 / 9.5, a step of 16
 // layers 4125 / 4045.
 // Bound by memory.  us of the two launches / here (32 heads on 8 of 128): 33 scattered tokens 3.8 + 3.6 / 5.4, 150 4.0 + 6.6 / 6.3; 2150 tokens of
-// prompts 12.3 + 6.3 / 10.2; 8192, bf16 and an FP8 cache, 37.7 + 17.7 / 36.4.
+// prompts 12.3 + 6.3 / 10.2; 8192, bf16 and an FP8 cache, 37.7 + 17.7 / 36.4.  Places in the cache divided out once a token instead of at each store: 150
+// scattered tokens behind slabs, in a step of 16 layers, 8.6 / 7.7.
 template <typename T, int KV, int HD, bool SLABS>
 __global__ __launch_bounds__(256) void rotary_cache_kernel(
     const int64_t* __restrict__ positions, typename T::storage* __restrict__ query, typename T::storage* __restrict__ key,
@@ -1080,7 +1081,8 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(
   constexpr int QH = CPH >= 16 ? 1 : 16 / CPH;        // query heads: 256 threads' worth
   constexpr int P = HD + 8;                           // LDS row pitch
   __shared__ __attribute__((aligned(16))) S sk[W * P], sv[W * P];
-  __shared__ int64_t s_slot[W];
+  __shared__ int64_t s_head[W];                       // (block, kv head) of the token's slot, -1: padding
+  __shared__ int s_off[W];                            // its place in the block
   const int64_t t0 = (int64_t)blockIdx.x * W;
   const int nt = (int)(num_tokens - t0 < W ? num_tokens - t0 : W);
   // numbers 8 c .. + 7 of a head of token t and their partners; ``col``: the head's first column
@@ -1131,7 +1133,11 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(
     return;
   }
   const int h = blockIdx.y;
-  if (threadIdx.x < W) s_slot[threadIdx.x] = threadIdx.x < nt ? slot_mapping[t0 + threadIdx.x] : -1;
+  if (threadIdx.x < W) {                              // (divided once a token: 64-bit quotients at each store were a third of a decode batch's launch)
+    const int64_t slot = threadIdx.x < nt ? slot_mapping[t0 + threadIdx.x] : -1, blk = slot < 0 ? 0 : slot / block_size;
+    s_head[threadIdx.x] = slot < 0 ? -1 : blk * num_kv_heads + h;
+    s_off[threadIdx.x] = slot < 0 ? 0 : (int)(slot - blk * block_size);
+  }
   for (int i = threadIdx.x; i < (SLABS ? 2 : 1) * nt * CPH; i += 256) {
     const int c = i % CPH, j = SLABS ? i / CPH % nt : i / CPH;
     u16x8 xo, yo;
@@ -1163,9 +1169,8 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(
   };
   for (int i = threadIdx.x; i < (HD / X) * W; i += 256) {      // K: piece (d / X, token)
     const int px = i / W, j = i % W;
-    const int64_t slot = s_slot[j];
-    if (slot < 0) continue;                           // padding
-    const int64_t dst = (((slot / block_size * num_kv_heads + h) * (HD / X) + px) * block_size + slot % block_size) * X;
+    if (s_head[j] < 0) continue;                      // padding
+    const int64_t dst = ((s_head[j] * (HD / X) + px) * block_size + s_off[j]) * X;
     if constexpr (KV == 0) {
       *reinterpret_cast<u32x4*>((S*)key_cache + dst) = *reinterpret_cast<const u32x4*>(sk + j * P + px * X);
     } else {
@@ -1173,16 +1178,15 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(
       *reinterpret_cast<u32x4*>((uint8_t*)key_cache + dst) = u32x4{cvt4(p, 1, k_scale), cvt4(p + 4, 1, k_scale), cvt4(p + 8, 1, k_scale), cvt4(p + 12, 1, k_scale)};
     }
   }
-  bool run = nt == W && s_slot[0] >= 0 && (s_slot[0] % block_size) + W <= block_size && (s_slot[0] % block_size) % X == 0;
+  bool run = nt == W && s_head[0] >= 0 && s_off[0] + W <= block_size && s_off[0] % X == 0;
 #pragma unroll
-  for (int j = 1; j < W; ++j) run = run && s_slot[j] == s_slot[0] + j;
+  for (int j = 1; j < W; ++j) run = run && s_head[j] == s_head[0] && s_off[j] == s_off[0] + j;
   if (run) {
-    const int64_t blk = s_slot[0] / block_size;
-    const int off0 = (int)(s_slot[0] % block_size);
+    const int off0 = s_off[0];
     constexpr int VP = KV == 0 ? 2 : 1;               // V: a row's 16 tokens, 32 or 16 bytes
     for (int i = threadIdx.x; i < HD * VP; i += 256) {
       const int d = i / VP, part = i % VP;
-      const int64_t dst = ((blk * num_kv_heads + h) * HD + d) * block_size + off0;
+      const int64_t dst = (s_head[0] * HD + d) * block_size + off0;
       uint32_t w[4];
       if constexpr (KV == 0) {
 #pragma unroll
@@ -1198,9 +1202,8 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(
   }
   for (int i = threadIdx.x; i < nt * HD; i += 256) {
     const int j = i / HD, d = i % HD;
-    const int64_t slot = s_slot[j];
-    if (slot < 0) continue;
-    const int64_t dst = ((slot / block_size * num_kv_heads + h) * HD + d) * block_size + slot % block_size;
+    if (s_head[j] < 0) continue;
+    const int64_t dst = (s_head[j] * HD + d) * block_size + s_off[j];
     if constexpr (KV == 0) ((S*)value_cache)[dst] = sv[j * P + d];
     else ((uint8_t*)value_cache)[dst] = (uint8_t)f32x2_to_fp8<KV == 2>(T::to_f32(sv[j * P + d]) / v_scale, 0.f);
   }
