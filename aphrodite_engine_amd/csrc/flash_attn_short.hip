@@ -143,11 +143,10 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void flash_attn_short_kernel(FAPar
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[b][i] = 32 * b + 8 * (i >> 2) + (i & 3) <= last ? s[b][i] : -INFINITY;
     }
-    auto max3 = [](float a, float b, float c) __attribute__((always_inline)) {
-      float r;      // (one instruction: hipcc puts a canonicalising v_max in front of every fmaxf on an MFMA output)
-      asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-      return r;
-    };
+    // The scores are the products' results: what reads them first is where hipcc sees it, as it keeps the wait states between a product and its reader only
+    // there.  (One instruction for three numbers, without the canonicalising v_max that fmaxf has in front; a NaN makes its row NaN, as it does
+    // without.)
+    auto max3 = [](float a, float b, float c) __attribute__((always_inline)) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); };
     // a step of the online softmax: NB blocks of 32 keys from block b0 on; the running maximum moves for rows that are past it by more than 2^lazy
     auto softmax = [&](auto nb, int b0, float lazy) __attribute__((always_inline)) {
       constexpr int NB = decltype(nb)::value;
@@ -158,9 +157,9 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void flash_attn_short_kernel(FAPar
         m4[c] = max3(s[b][i0], s[b][i0 + 1], s[b][i0 + 2]);
         m4[c] = max3(m4[c], s[b][i0 + 3], s[b][i0 + 4]);
         m4[c] = max3(m4[c], s[b][i0 + 5], s[b][i0 + 6]);
-        m4[c] = fmaxf(m4[c], s[b][i0 + 7]);
+        m4[c] = __builtin_elementwise_maximum(m4[c], s[b][i0 + 7]);
       }
-      float mx = fmaxf(m4[0], m4[1]);
+      float mx = __builtin_elementwise_maximum(m4[0], m4[1]);
       if constexpr (NB == 2) mx = max3(mx, m4[2], m4[3]);
       const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
       const unsigned low = sw[0], high = sw[1];
