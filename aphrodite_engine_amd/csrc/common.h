@@ -19,6 +19,13 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
+// An A fragment whose B operand is int4 nibbles in place: nibbles 2, 3, 6 and 7 of a word lie four bits higher and weigh 16x, so their k carry 1/16.
+// (Where hipcc sees it: a product wants two wait states behind what wrote its operand, and next to inline asm hipcc does not keep them.)
+__device__ __forceinline__ f16x8 sixteenths(u32x4 a) {
+  constexpr f16 s = (f16)0.0625f;
+  return __builtin_bit_cast(f16x8, a) * f16x8{1, 1, s, s, 1, 1, s, s};
+}
+
 #define WAVE 64
 
 namespace aphro {

@@ -341,11 +341,7 @@ __global__ __launch_bounds__(FNW * 64, (VEC * MT >= 8) ? 2 : 3) void wna16_gemm_
       for (int i = 0; i < MT; ++i) {
         // nibbles 2,3,6,7 of a word are extracted in place (bits 4-7 of each half):
         // they weigh 16x, so those four k of the A fragment are scaled by 1/16
-        // (inline asm on the integer lanes: hipcc miscompiles a bitcast of one vector element)
-        u32x4 av = af[s % NA][u][i];
-        asm("v_pk_mul_f16 %0, %1, %2" : "=v"(av[1]) : "v"(av[1]), "s"(0x2c002c00u));
-        asm("v_pk_mul_f16 %0, %1, %2" : "=v"(av[3]) : "v"(av[3]), "s"(0x2c002c00u));
-        a[i] = __builtin_bit_cast(f16x8, av);
+        a[i] = sixteenths(af[s % NA][u][i]);
         rs[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], ones, u == 0 ? zero4 : rs[i], 0, 0, 0);
       }
 #pragma unroll
@@ -446,8 +442,7 @@ __global__ __launch_bounds__(FNW * 64, 2) void wna16_experts_kernel(Wna16Params 
     for (int s = 0; s < NSEG; ++s)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {         // (the nibbles that weigh 16x: see wna16_gemm_kernel)
-        asm("v_pk_mul_f16 %0, %1, %2" : "=v"(af[s][u][1]) : "v"(af[s][u][1]), "s"(0x2c002c00u));
-        asm("v_pk_mul_f16 %0, %1, %2" : "=v"(af[s][u][3]) : "v"(af[s][u][3]), "s"(0x2c002c00u));
+        af[s][u] = __builtin_bit_cast(u32x4, sixteenths(af[s][u]));
       }
   };
   auto load_w = [&](uint32_t (&wd)[4][4], const Unit& t, int s) {

@@ -337,8 +337,8 @@ __global__ __launch_bounds__(NWV * 64, NWV <= 4 ? 1 : 2) void wna16_gemm_residen
     for (int i = 0; i < MT; ++i) {
       u32x4 av = af[s][u][i];
       if constexpr (pass == 0) {
-        asm("v_pk_mul_f16 %0, %1, %2" : "=v"(av[1]) : "v"(av[1]), "s"(0x2c002c00u));
-        asm("v_pk_mul_f16 %0, %1, %2" : "=v"(av[3]) : "v"(av[3]), "s"(0x2c002c00u));
+        // (sixteenths() takes 2 to 6 registers more here, of all that there are, and spills; the s_nop: what a product reads has to be two states old)
+        asm("v_pk_mul_f16 %0, %2, %4\n\tv_pk_mul_f16 %1, %3, %4\n\ts_nop 1" : "=&v"(av[1]), "=v"(av[3]) : "v"(av[1]), "v"(av[3]), "s"(0x2c002c00u));
         af[s][u][i] = av;
       }
       a[i] = __builtin_bit_cast(f16x8, av);
@@ -756,10 +756,7 @@ __global__ __launch_bounds__(NWV * 64, MT) void wna16_gemm_stream_kernel(const u
     f16x8 a[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      u32x4 av = ar[B][i];
-      asm("v_pk_mul_f16 %0, %1, %2" : "=v"(av[1]) : "v"(av[1]), "s"(0x2c002c00u));
-      asm("v_pk_mul_f16 %0, %1, %2" : "=v"(av[3]) : "v"(av[3]), "s"(0x2c002c00u));
-      a[i] = __builtin_bit_cast(f16x8, av);
+      a[i] = sixteenths(ar[B][i]);
       rs[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], ones, u == 0 ? zero4 : rs[i], 0, 0, 0);
     }
     res_static_for<0, NT>([&](auto T_) {

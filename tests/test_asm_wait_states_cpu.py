@@ -12,9 +12,14 @@ import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "aphrodite_engine_amd", "csrc")
 PRODUCTS = ("v_mfma", "v_smfma")
-BEHIND_PRODUCT, BEHIND_ASM = 20, 2      # states: any product's result (16 passes and four) ahead of asm; asm's ahead of a product, a lane swap or choice
+BEHIND_ASM = 2                          # states between asm's result and a product, a lane swap or a lane choice that reads it
 
 Step = collections.namedtuple("Step", "line asm op text writes reads states")
+
+
+def _behind(product):
+    """States between a product and a vector instruction on its result: its passes and four.  16-bit products of 16x16x32 and 32x32x16 take 8 passes at most."""
+    return 12 if re.search(r"_(16x16x32|32x32x16)_b?f16", product) else 20
 
 
 def _registers(operand):
@@ -58,17 +63,17 @@ def _too_near(text):
                 ahead[i + 1].append(i)
 
         def writer(i, registers, which, states):
-            """A step that ``which`` picks and that wrote one of the registers fewer states ahead of step i, on some path."""
+            """A step that ``which`` picks and that wrote one of the registers fewer than ``states`` ahead of step i, on some path."""
             seen, todo = {}, [(i, 0, registers)]
             while todo:
                 j, d, left = todo.pop()
                 for k in ahead[j]:
                     s, e, rest = steps[k], d, left
                     if not isinstance(s, str):
-                        if s.writes & left and which(s):
+                        if s.writes & left and which(s) and d < states(s):
                             return s
                         e, rest = d + s.states, left - s.writes
-                    if rest and e < states and seen.get((k, rest), states) > e:
+                    if rest and e < 20 and seen.get((k, rest), 20) > e:
                         seen[k, rest] = e
                         todo.append((k, e, rest))
 
@@ -77,11 +82,11 @@ def _too_near(text):
                 continue
             w = None
             if s.asm:
-                w = writer(i, s.reads | s.writes, lambda x: x.op.startswith(PRODUCTS), BEHIND_PRODUCT)
+                w = writer(i, s.reads | s.writes, lambda x: x.op.startswith(PRODUCTS), lambda x: _behind(x.op))
             if not w and (s.op.startswith(PRODUCTS) or "permlane" in s.op):
-                w = writer(i, s.reads, lambda x: x.asm and x.op.startswith("v_") and not x.op.startswith(PRODUCTS), BEHIND_ASM)
+                w = writer(i, s.reads, lambda x: x.asm and x.op.startswith("v_") and not x.op.startswith(PRODUCTS), lambda x: BEHIND_ASM)
             if not w and "row_" in s.text:
-                w = writer(i, _registers(s.text.split(",")[1]), lambda x: x.asm and x.op.startswith("v_"), BEHIND_ASM)
+                w = writer(i, _registers(s.text.split(",")[1]), lambda x: x.asm and x.op.startswith("v_"), lambda x: BEHIND_ASM)
             if w:
                 found.append(f"{kernel}: '{w.text}' (line {w.line}) too near '{s.text}' (line {s.line})")
     return found
@@ -90,8 +95,9 @@ def _too_near(text):
 def test_the_count():
     def kernel(between, ahead="v_mfma_f32_32x32x16_bf16 v[0:15], v[20:23], v[24:27], 0", asm="v_max3_f32 v30, v3, v4, v5"):
         return f"_Zk:\n\t{ahead}\n{between}\t;;#ASMSTART\n\t{asm}\n\t;;#ASMEND\n\ts_endpgm\n"
-    far = "\ts_nop 15\n\ts_nop 3\n"
-    assert _too_near(kernel("")) and not _too_near(kernel(far)) and _too_near(kernel("\ts_nop 15\n\ts_nop 2\n"))
+    far = "\ts_nop 11\n"
+    assert _too_near(kernel("")) and not _too_near(kernel(far)) and _too_near(kernel("\ts_nop 10\n"))
+    assert _too_near(kernel(far, ahead="v_mfma_f32_32x32x2_f32 v[0:15], v20, v24, 0"))
     # a jump past the states, and a register written anew
     assert _too_near(kernel("\ts_cbranch_scc1 .L1\n" + far + ".L1:\n"))
     assert not _too_near(kernel("\tv_mov_b32_e32 v3, 0\n", asm="v_max3_f32 v30, v3, v31, v32"))
@@ -100,7 +106,7 @@ def test_the_count():
 
 
 @pytest.mark.skipif(not shutil.which("hipcc") and not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
-@pytest.mark.parametrize("name", ["flash_attn_short", "mixers/delta_rule_chunked"])
+@pytest.mark.parametrize("name", ["flash_attn_short", "wna16_gemm", "mixers/delta_rule_chunked"])
 def test_states_around_inline_asm(name, tmp_path):
     folder, file = os.path.split(os.path.join(CSRC, name))
     lines = subprocess.run(["make", "-n", "-B", f"build/{file}.o"], cwd=folder, check=True, capture_output=True, text=True).stdout.splitlines()
