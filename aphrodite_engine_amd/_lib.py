@@ -7,6 +7,7 @@ same way -- `aphrodite/_custom_ops.py:13-43` re-raises with a hint when
 """
 import ctypes
 import os
+import sysconfig
 from ctypes import c_float, c_int, c_int64, c_size_t, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -248,23 +249,37 @@ F16, BF16, F32 = 0, 1, 2
 WEIGHTS_STREAMED, WEIGHTS_CACHED = 0x100, 0x200          # or-ed into a dtype
 KV_AUTO, KV_FP8_E4M3, KV_FP8_E5M2 = 0, 1, 2
 
-ENTRY_CALLS_PATH = os.path.join(_HERE, "lib", "aphrodite_entry_calls.so")
+ENTRY_CALLS_PATH = os.path.join(_HERE, "lib", "aphrodite_entry_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
-def _bind_calls(l, signatures) -> None:
-    """Functions of ``l`` as Python functions that convert their arguments by the declared types (csrc_torch/entry_calls.cpp), in place of ctypes'
-    own calls, which stay for whatever is not a plain number, for names that it does not have, and where it is not built."""
+def _letters(res, args) -> str:
+    """A signature in ctypes' letters, the result's first ('?' for what has none)."""
+    letters = (getattr(t, "_type_", None) for t in (res, *args))
+    return "".join(c if isinstance(c, str) else "?" for c in letters)
+
+
+def _entry_calls():
+    """The module of typed calls (csrc_torch/entry_calls.cpp), or None where it is not built for this Python."""
     if not os.path.exists(ENTRY_CALLS_PATH):
-        return
+        return None
     import importlib.machinery
     import importlib.util
     name = "aphrodite_entry_calls"
     loader = importlib.machinery.ExtensionFileLoader(name, ENTRY_CALLS_PATH)
     calls = importlib.util.module_from_spec(importlib.util.spec_from_file_location(name, ENTRY_CALLS_PATH, loader=loader))
     loader.exec_module(calls)
-    for name in signatures:
+    return calls
+
+
+def _bind_calls(l, signatures) -> None:
+    """Functions of ``l`` as Python functions that convert their arguments by the declared types, in place of ctypes' own calls, which stay for whatever
+    is not a plain number, for names that the module does not have or that it was built with other types for, and where there is no such module."""
+    calls = _entry_calls()
+    if calls is None:
+        return
+    for name, (res, args) in signatures.items():
         fn = getattr(l, name)
-        call = calls.bind(name, ctypes.cast(fn, c_void_p).value, fn)
+        call = calls.bind(name, ctypes.cast(fn, c_void_p).value, fn, _letters(res, args))
         if call is not None:
             setattr(l, name, call)
 
@@ -280,8 +295,7 @@ def lib():
     if not os.path.exists(LIB_PATH):
         raise ImportError(
             f"{LIB_PATH} not found: the MI355X HIP library has not been built. "
-            "Run `python -c 'import __graft_entry__ as g; g.build()'` (or "
-            "`make -C aphrodite_engine_amd/csrc`). There is no CPU fallback.")
+            "Run `python -c 'import __graft_entry__ as g; g.build()'`. There is no CPU fallback.")
     l = ctypes.CDLL(LIB_PATH)
     for name, (res, args) in SIGNATURES.items():
         try:

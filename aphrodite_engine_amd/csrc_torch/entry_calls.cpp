@@ -2,7 +2,10 @@
 // them in Python's object model -- 20 to 45 arguments, 3 to 6 us a call where the launch itself takes 2.5.  Here the arguments are converted by the
 // declared types of the function, at compile time.
 // Measured on the host: 0.8 us against ctypes' 7.8 for the 40 arguments of the attention with a bias, 0.3 against 1.9 for 6 arguments.
-//   bind(name, address, call) -> the function at that address under the type that the header declares for the name, or None for a name not listed here
+//   bind(name, address, call, types) -> the function at that address under the type that the header declares for the name, or None for a name not listed
+//                                       here, or listed with other types than the caller's (ctypes' letters, the result's first): headers that moved on
+//                                       since this file was built leave such a name to ctypes
+//   names() -> the names listed here
 // The address comes from whoever loaded the library (_lib.py), so that nothing is linked and an overridden library path keeps its meaning; it is kept in
 // the returned function, so that two libraries can be bound side by side.
 // Whole numbers, None for a null pointer and numbers for floats are converted here, as ctypes converts them (whole numbers wrap); a call with anything
@@ -48,10 +51,20 @@ bool take(PyObject* o, T& out) {
   }
 }
 
+// ctypes' letter of a type
+template <typename T>
+constexpr char letter() {
+  if constexpr (std::is_pointer_v<T>) return 'P';
+  else if constexpr (std::is_floating_point_v<T>) return sizeof(T) == 4 ? 'f' : 'd';
+  else if constexpr (sizeof(T) == 4) return std::is_signed_v<T> ? 'i' : 'I';
+  else return sizeof(T) != 8 ? '?' : std::is_signed_v<T> ? 'l' : 'L';
+}
+
 template <typename F>
 struct Entry;
 template <typename R, typename... A>
 struct Entry<R (*)(A...)> {
+  static constexpr char types[] = {letter<R>(), letter<A>()..., 0};
   template <size_t... I>
   static PyObject* run(const Target* t, PyObject* const* args, std::index_sequence<I...>) {
     std::tuple<A...> a;
@@ -115,8 +128,9 @@ struct Entry<R (*)(A...)> {
   X(aphro_gated_delta_scan) X(aphro_gated_head_rms_norm) X(aphro_conv_rotary_supported) X(aphro_conv_rotary_qk_norm_kv_write) \
   X(aphro_short_conv_state) X(aphro_residual_tanh_norm) X(aphro_rotary_qk_norm_kv_write)
 
-#define X(name) {#name, (PyCFunction)(void (*)(void))&Entry<decltype(&name)>::call, METH_FASTCALL, nullptr},
-PyMethodDef rows[] = {CORE_ENTRIES(X) MIXER_ENTRIES(X)};
+struct Row { PyMethodDef def; const char* types; };
+#define X(name) {{#name, (PyCFunction)(void (*)(void))&Entry<decltype(&name)>::call, METH_FASTCALL, nullptr}, Entry<decltype(&name)>::types},
+Row rows[] = {CORE_ENTRIES(X) MIXER_ENTRIES(X)};
 #undef X
 
 void drop(PyObject* capsule) {
@@ -126,23 +140,34 @@ void drop(PyObject* capsule) {
 }
 
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (n != 3) return PyErr_Format(PyExc_TypeError, "bind(name, address, call)");
-  const char* name = PyUnicode_AsUTF8(args[0]);
-  if (!name) return nullptr;
+  if (n != 4) return PyErr_Format(PyExc_TypeError, "bind(name, address, call, types)");
+  const char *name = PyUnicode_AsUTF8(args[0]), *types = name ? PyUnicode_AsUTF8(args[3]) : nullptr;
+  if (!types) return nullptr;
   void* at = PyLong_AsVoidPtr(args[1]);
   if (!at) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "no address");
-  for (PyMethodDef& row : rows) {
-    if (strcmp(row.ml_name, name)) continue;
+  for (Row& row : rows) {
+    if (strcmp(row.def.ml_name, name)) continue;
+    if (strcmp(row.types, types)) break;
     PyObject* self = PyCapsule_New(new Target{at, Py_NewRef(args[2])}, nullptr, &drop);
     if (!self) return nullptr;
-    PyObject* call = PyCFunction_New(&row, self);
+    PyObject* call = PyCFunction_New(&row.def, self);
     Py_DECREF(self);
     return call;
   }
   Py_RETURN_NONE;
 }
 
-PyMethodDef methods[] = {{"bind", (PyCFunction)(void (*)(void))&bind, METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyObject* names(PyObject*, PyObject*) {
+  PyObject* list = PyList_New(0);
+  for (const Row& row : rows) {
+    PyObject* name = list ? PyUnicode_FromString(row.def.ml_name) : nullptr;
+    if (!name || PyList_Append(list, name)) Py_CLEAR(list);
+    Py_XDECREF(name);
+  }
+  return list;
+}
+
+PyMethodDef methods[] = {{"bind", (PyCFunction)(void (*)(void))&bind, METH_FASTCALL, nullptr}, {"names", &names, METH_NOARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "aphrodite_entry_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

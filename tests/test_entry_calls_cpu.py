@@ -26,10 +26,40 @@ def outcome(fn, args):
 
 
 def test_the_entry_points_are_bound():
-    for l, signatures in ((_lib.lib(), _lib.SIGNATURES), (_lib.mixers_lib(), _lib.MIXERS_SIGNATURES)):
-        bound = [n for n in signatures if type(getattr(l, n)).__name__ == "builtin_function_or_method"]
-        assert 2 * len(bound) > len(signatures)
-        assert all(getattr(l, n).__name__ == n for n in bound)
+    calls = _lib._entry_calls()
+    assert len(calls.names()) == len(set(calls.names())) >= 170
+    for name in calls.names():
+        fn = typed(name)
+        assert type(fn).__name__ == "builtin_function_or_method" and fn.__name__ == name
+
+
+@pytest.mark.parametrize("name", ["aphro_dense_rows_slab_floats", "aphro_rms_norm", "aphro_distance_bias_attention"])
+def test_other_types_than_the_module_was_built_with(name):
+    """Signatures and module that do not agree in one type, or in their number: the name stays with ctypes."""
+    calls, fn = _lib._entry_calls(), plain(name)
+    at, types = ctypes.cast(fn, ctypes.c_void_p).value, _lib._letters(fn.restype, fn.argtypes)
+    assert calls.bind(name, at, fn, types).__name__ == name
+    for i in range(len(types)):
+        for other in "PilLf?":
+            if other != types[i]:
+                assert calls.bind(name, at, fn, types[:i] + other + types[i + 1:]) is None
+    assert calls.bind(name, at, fn, types + "P") is None and calls.bind(name, at, fn, types[:-1]) is None
+
+
+def test_a_moved_signature_keeps_ctypes():
+    name = "aphro_dense_rows_slab_floats"
+    l = ctypes.CDLL(_lib.LIB_PATH)
+    moved = (ctypes.c_int, [ctypes.c_float] + _lib.SIGNATURES[name][1][1:])
+    getattr(l, name).restype, getattr(l, name).argtypes = moved
+    _lib._bind_calls(l, {name: moved})
+    assert not type(getattr(l, name)).__name__.startswith("builtin")
+
+
+def test_built_for_another_python(monkeypatch, tmp_path):
+    monkeypatch.setattr(_lib, "ENTRY_CALLS_PATH", str(tmp_path / "aphrodite_entry_calls.so"))
+    l = ctypes.CDLL(_lib.LIB_PATH)
+    _lib._bind_calls(l, {"aphro_rms_norm": _lib.SIGNATURES["aphro_rms_norm"]})
+    assert not type(l.aphro_rms_norm).__name__.startswith("builtin")
 
 
 SLAB = (32, 4096, 4096, 4096, 4096, -1)
