@@ -25,6 +25,14 @@ def test_silu_against_64_bits(low, high):
         assert ((silu(z).double() - want).abs() <= bound * 2.0 ** -24 * want.abs() + 2.0 ** -148).all()
 
 
+def test_silu_of_the_smallest():
+    """Half of z, rounded once, down to the least number there is."""
+    n = torch.cat([torch.arange(1, 4097), torch.logspace(12, 26.7, 4096, base=2, dtype=torch.float64).long()]).to(torch.int32)      # 1.4e-45 .. 5e-38
+    z = n.view(torch.float32).to(DEV).view(2, 4096)
+    for x in (z, -z):
+        assert torch.equal(silu(x), (x.double() / 2).float())
+
+
 def test_silu_of_edges():
     inf, nan = float("inf"), float("nan")
     z = torch.tensor([[0.0, -0.0, inf, -inf, nan, 3e38, -3e38, -89.0]], device=DEV)
