@@ -143,14 +143,14 @@ __device__ __forceinline__ float gelu_tanh_f(float z) {
   const float u = 0.7978845608028654f * (z + 0.044715f * z * z * z);
   return 0.5f * z * (1.0f + tanhf(u));
 }
-// log(1 + e^z) = max(z, 0) + 2 atanh(y), y = x / (2 + x), x = e^-|z|: y in two numbers, atanh by its series in y^2 (coefficients fitted by least squares
-// over y <= 1 / 3, 1e-10).  Largest error 2.04 x 2^-24, root mean square 0.47 (log1p(e^z) with both rounded correctly: 1.98, 0.46), a fifth of
-// log1pf's instructions and no branch.
+// log(1 + e^z) = max(z, 0) + 2 atanh(h / 2), h = x / (1 + x / 2), x = e^-|z|: h in two numbers, atanh by its series in h^2 (coefficients fitted by least
+// squares over h <= 2 / 3, 1e-10), the sum with what its first step rounds away (z = infinity leaves NaN there: -1 for it).  No branch.
 __device__ __forceinline__ float softplus_f(float z) {
-  const float x = expf(-fabsf(z)), d = x + 2.f, dl = x - (d - 2.f), r = __builtin_amdgcn_rcpf(d);
-  const float y = x * r, yl = fmaf(-y, dl, fmaf(-y, d, x)) * r, t = y * y;
-  const float s = fmaf(fmaf(fmaf(fmaf(0.12120297f, t, 0.10722389f), t, 0.14307591f), t, 0.19999473f), t, 0.33333337f);
-  return fmaxf(z, 0.f) + (2.f * y + fmaf(2.f * y * t, s, 2.f * yl));
+  const float x = expf(-fabsf(z)), d = fmaf(x, 0.5f, 1.f), dl = fmaf(x, 0.5f, 1.f - d), r = __builtin_amdgcn_rcpf(d);
+  const float h = x * r, hl = fmaf(-h, dl, fmaf(-h, d, x)) * r, t = h * h;
+  const float s = fmaf(fmaf(fmaf(fmaf(0.12120297f / 1024, t, 0.10722389f / 256), t, 0.14307591f / 64), t, 0.19999473f / 16), t, 0.33333337f / 4);
+  const float m = fmaxf(z, 0.f), a = fmaxf(m, h), b = fminf(m, h), sum = a + b;
+  return sum + (fmaxf(b - (sum - a), -1.f) + fmaf(h * t, s, hl));
 }
 // log(sigmoid(z)) without overflow on either side
 __device__ __forceinline__ float log_sigmoid_f(float z) {

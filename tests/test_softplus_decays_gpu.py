@@ -31,3 +31,25 @@ def test_decays_over_the_range_of_their_gates(monkeypatch, chunks, channel):
         # g = e^ln: an error of (softplus 2.1, exp of a_log 1.5, the product 0.5) x 2^-24 of ln, 1.5 x 2^-24 of g; below 2^-120 fp32 itself runs out
         bound = want * ((4.1 * ln.abs()).clamp(max=1e3) + 1.5) * 2.0 ** -24 + 2.0 ** -140
         assert (got[:, :, 0] - want).abs().le(bound).all(), (rate, ((got[:, :, 0] - want).abs() / bound).max())
+
+
+@pytest.mark.parametrize("low,high", [(-87.3, -20.0), (-20.0, -1.0), (-1.0, 0.0), (0.0, 0.54), (0.54, 20.0), (20.0, 1e4)])
+def test_softplus_against_64_bits(low, high):
+    """A state-space memory's first token writes softplus(step size) k v^T: with ones for k and v, softplus itself."""
+    from aphrodite_engine_amd import mixer_ops as mops
+    T, H, d = 256, 128, 16
+    g = torch.Generator(device=DEV).manual_seed(7)
+    z = torch.rand(T, H, generator=g, device=DEV) * (high - low) + low
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    one = torch.ones(T, H * d, device=DEV)
+    state = torch.zeros(mops.memory_state_shapes(T, H, d, d, mops.MEMORY_STATE_SPACE)[0], device=DEV)
+    zero = torch.zeros(H, device=DEV)
+    mops.outer_memory_scan(one[:, :d].contiguous(), one[:, :d].contiguous(), one, (state, ), i32(range(T)), i32(range(T)), i32([1] * T), i32([0] * T), H,
+                           mops.MEMORY_STATE_SPACE, gate_i=z, qk_heads=1, a_log=zero, dt_bias=zero, skip=zero)
+    got, x = state[:, :, 0, 0].double(), torch.exp(-z.double().abs())
+    want = z.double().clamp(min=0) + torch.log1p(x)
+    ulp = lambda v: torch.exp2(v.log2().floor() - 23).clamp(min=2.0 ** -149)
+    # rounded once itself; e^-|z| is right to a last place, of which 1 / (1 + x) arrives; what follows a number's first part rounds below 0.06 x 2^-24 of it
+    bound = ulp(want) / 2 + ulp(x.clamp(min=1e-45)) / (1 + x) + 0.06 * 2.0 ** -24 * torch.log1p(x)
+    err = (got - want).abs()
+    assert (err <= bound).all(), float((err / bound).max())
