@@ -260,8 +260,14 @@ static void fa_short_launch_t(const FAParams& p, int batch, int max_query_len, i
   // Two groups of waves a row tile where a launch lasts as long as its longest chain of key tiles: where the row tiles would leave every CU one workgroup
   // at the most, or two of which one prompt's have anything from one key tile to all.  us, one group / two, 32 heads on 8: 600 tokens 18.6 /
   // 16.4, 1500 40.8 / 32.6, 2000 55.3 / 51.7, two of 500 17.0 / 15.7; 8 heads on one, 8192 tokens 187 / 160, 4 on one, 16384 356 / 290.
+  // Behind cached keys a prompt's chains are the more alike the more keys there are, and two workgroups of one group that share a CU are then the faster
+  // (gather included): 32 on 8, 1300 rows behind 650 / 1300 / 2600 / 20800 keys 62 / 58, 78 / 82, 114 / 125, 596 / 645; 1480 behind 740 / 990 / 2220
+  // 68.4 / 67.5, 74.7 / 75.8, 110 / 117.  Long chains bear more: 8 on one, 4800 behind 4800 / 7200 / 14400 194 / 182, 240 / 247, 420 / 444, and where the
+  // CUs have two nearly all over any number: 6800 rows behind 6800 / 27200 313 / 297, 883 / 868.
   const int64_t tiles = (int64_t)batch * ((max_query_len + rows - 1) / rows) * (p.num_heads / qt), cus = device_cu_count();
-  const bool two = max_key_len >= 256 && (tiles <= cus || (batch == 1 && p.causal && tiles <= 2 * cus));
+  const int64_t cached = max((int64_t)max_key_len - max_query_len, (int64_t)0);
+  const bool uneven = 3 * cached <= 2 * (int64_t)max_query_len || (max_key_len >= 8192 && (3 * cached <= 4 * (int64_t)max_query_len || 5 * tiles >= 8 * cus));
+  const bool two = max_key_len >= 256 && (tiles <= cus || (batch == 1 && p.causal && tiles <= 2 * cus && uneven));
   const bool lng = max_key_len >= 1024 && max_key_len >= knobs().fa_v4_min_keys;
 #define APHRO_FAS(QT)                                                                                                                            \
   (two ? (lng ? fa_short_launch_g<T, QT, true, 2>(p, batch, max_query_len, st) : fa_short_launch_g<T, QT, false, 2>(p, batch, max_query_len, st)) \

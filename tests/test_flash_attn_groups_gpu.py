@@ -9,17 +9,17 @@ pytestmark = pytest.mark.gpu
 DEV, D = "cuda", 128
 
 
-def _check(out, q, k, v, cu, scale, causal, slopes, dtype):
+def _check(out, q, k, v, cu, scale, causal, slopes, dtype, cached=0):
     heads, rep = q.shape[1], q.shape[1] // k.shape[1]
     for a, b in zip(cu[:-1], cu[1:]):
         n = b - a
-        kk, vv = (x[a:b].double().repeat_interleave(rep, 1).transpose(0, 1) for x in (k, v))
+        kk, vv = (x[a:b + cached].double().repeat_interleave(rep, 1).transpose(0, 1) for x in (k, v))
         s = torch.matmul(q[a:b].double().transpose(0, 1), kk.transpose(1, 2).contiguous()) * scale
-        i = torch.arange(n, device=DEV)
+        i, j = torch.arange(cached, cached + n, device=DEV)[:, None], torch.arange(cached + n, device=DEV)[None]
         if slopes is not None:
-            s = s + slopes.double()[:, None, None] * (i[None] - i[:, None])
+            s = s + slopes.double()[:, None, None] * (j - i)
         if causal:
-            s = s.masked_fill(i[None] > i[:, None], float("-inf"))
+            s = s.masked_fill(j > i, float("-inf"))
         want = torch.matmul(torch.softmax(s, 2), vv).transpose(0, 1)
         # probabilities and results are rounded to the type: u of a value each, the probabilities' against values of up to the largest
         u = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
@@ -43,6 +43,27 @@ def test_forms(heads, kv, lens, causal, alibi, first, dtype):
     with ops.knob("APHRO_FA_V4_MIN_KEYS", first):
         out = ops.flash_attn_varlen(q, k, v, torch.tensor(cu, dtype=torch.int32, device=DEV), max(lens), D ** -0.5, causal=causal, alibi_slopes=slopes)
     _check(out, q, k, v, cu, D ** -0.5, causal, slopes, dtype)
+
+
+@pytest.mark.parametrize("heads,kv,rows,cached,first", [
+    (32, 8, 1300, 650, 4096), (32, 8, 1300, 1300, 4096), (32, 8, 1030, 686, 1024), (32, 8, 1030, 687, 1024), (32, 8, 300, 2000, 4096), (8, 8, 400, 79, 4096),
+    (8, 1, 3000, 6001, 4096), (4, 4, 1033, 8000, 4096)])
+def test_behind_cached_keys(heads, kv, rows, cached, first):
+    """One prompt behind cached keys, on both sides of where its chains count as uneven."""
+    g = torch.Generator(device=DEV).manual_seed(rows + cached)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+    q, k, v, bs = rnd(rows, heads, D), rnd(cached + rows, kv, D), rnd(cached + rows, kv, D), 16
+    blocks = (cached + bs - 1) // bs
+    order = torch.randperm(blocks + 1, generator=g, device=DEV)
+    kc, vc = torch.full((blocks + 1, kv, D // 8, bs, 8), float("nan"), device=DEV).bfloat16(), torch.full((blocks + 1, kv, D, bs), float("nan"), device=DEV).bfloat16()
+    at, off = order[torch.arange(cached, device=DEV) // bs], torch.arange(cached, device=DEV) % bs
+    kc[at, :, :, off], vc[at, :, :, off] = k[:cached].view(cached, kv, D // 8, 8), v[:cached]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    out = torch.empty_like(q)
+    with ops.knob("APHRO_FA_V4_MIN_KEYS", first):
+        ops.context_attention_fwd(q, k[cached:], v[cached:], out, "auto", kc, vc, order[None, :blocks].int().contiguous(), i32([0, rows]), i32([cached + rows]),
+                                  i32([cached]), rows, max_seq_len=cached + rows, total_kv_tokens=cached + rows)
+    _check(out, q, k, v, [0, rows], D ** -0.5, True, None, torch.bfloat16, cached)
 
 
 @pytest.mark.parametrize("first", [1024, 4096])
