@@ -42,9 +42,9 @@ int dba_decode_splits(int64_t rows, int64_t num_tokens, int units, int max_kv_le
 // The forms of the kernels, a translation unit each: causal with a gate per head at most; window / chunk, soft cap, sink and elementwise
 // gate, chosen at run time; causal with an elementwise gate.
 enum DBAForm { DBA_PLAIN = 0, DBA_MASKED = 1, DBA_GATED = 2 };
-// max_keys: the most keys that a row can see
+// max_keys: the most keys that a row can see; max_kv_len: the most that a sequence has (0: not known)
 template <int FORM>
-void dba_prefill_launch(const DBAParams& p, int64_t num_tokens, int max_q_len, int num_seqs, int max_keys, hipStream_t st);
+void dba_prefill_launch(const DBAParams& p, int64_t num_tokens, int max_q_len, int num_seqs, int max_keys, int max_kv_len, hipStream_t st);
 template <int FORM>
 void dba_decode_launch(const DBAParams& p, int64_t rows, int nsplit, hipStream_t st);
 constexpr int DBA_MAX_SPLITS = 8;       // workgroups that share a decoded row's keys

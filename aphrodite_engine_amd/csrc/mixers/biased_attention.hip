@@ -268,9 +268,9 @@ extern "C" int aphro_distance_bias_attention(void* out, int64_t out_stride, cons
     const int nsplit = workspace ? dba_decode_splits(likely, num_tokens, dba_decode_units(heads, kv_heads, dim, vdim), visible, workspace_floats, heads, vdim) : 1;
     if (pf && (all_long || dc)) {
       p.min_len = DBA_MFMA_MIN_LEN;
-      if (form == DBA_MASKED) dba_prefill_launch<DBA_MASKED>(p, num_tokens, max_q_len, num_seqs, visible, (hipStream_t)stream);
-      else if (form == DBA_GATED) dba_prefill_launch<DBA_GATED>(p, num_tokens, max_q_len, num_seqs, visible, (hipStream_t)stream);
-      else dba_prefill_launch<DBA_PLAIN>(p, num_tokens, max_q_len, num_seqs, visible, (hipStream_t)stream);
+      if (form == DBA_MASKED) dba_prefill_launch<DBA_MASKED>(p, num_tokens, max_q_len, num_seqs, visible, max_kv_len, (hipStream_t)stream);
+      else if (form == DBA_GATED) dba_prefill_launch<DBA_GATED>(p, num_tokens, max_q_len, num_seqs, visible, max_kv_len, (hipStream_t)stream);
+      else dba_prefill_launch<DBA_PLAIN>(p, num_tokens, max_q_len, num_seqs, visible, max_kv_len, (hipStream_t)stream);
       if (!all_long) {
         if (form == DBA_MASKED) dba_decode_launch<DBA_MASKED>(p, rows, nsplit, (hipStream_t)stream);
         else if (form == DBA_GATED) dba_decode_launch<DBA_GATED>(p, rows, nsplit, (hipStream_t)stream);

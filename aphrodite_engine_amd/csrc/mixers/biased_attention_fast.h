@@ -1133,7 +1133,7 @@ static void launch_prefill32(const DBAParams& p0, int64_t num_tokens, int num_se
 }
 
 template <int FORM>
-void dba_prefill_launch(const DBAParams& p0, int64_t num_tokens, int max_q_len, int num_seqs, int max_keys, hipStream_t st) {
+void dba_prefill_launch(const DBAParams& p0, int64_t num_tokens, int max_q_len, int num_seqs, int max_keys, int max_kv_len, hipStream_t st) {
   // 16-byte loads into LDS want aligned caches (rows are 256 bytes times the kv heads); their 32-bit offsets a block below 4 GiB, or the
   // whole cache where blocks are no multiples of 16 keys
   const int64_t span = (p0.bs_shift >= 4 ? 1 : p0.num_blocks) * p0.block_size * (int64_t)p0.kv_heads * 256;
@@ -1141,12 +1141,19 @@ void dba_prefill_launch(const DBAParams& p0, int64_t num_tokens, int max_q_len, 
     const int per_kv = p0.heads / p0.kv_heads;
     const int qt = per_kv % 4 == 0 ? 4 : per_kv % 2 == 0 ? 2 : 1;
     // Two groups of waves a row tile where a launch lasts as long as its longest chain of key tiles: where the row tiles would leave every CU one workgroup
-    // at the most, or two of which one segment's have anything from one key tile to all (no window that evens them out).  us, one group / two: 16 heads
-    // on 4, 1000 rows with bias 32 / 26, 2000 behind 1024 keys with cap and bias 79 / 61, 4096 rows 103 / 85, 3000 behind 3000 147 / 145, under a
-    // window of 1024 50 / 53; 32 heads on 8, 1200 rows 40 / 30, 2500 85 / 90, three segments of 700 33 / 36.
+    // at the most, or two of one segment with chains so unlike that all of them are worth at most 1.31 of the longest to a CU, and 0.86 of it to
+    // each.  us, one group / two (the two numbers): 16 heads on 4, fresh, 2800 rows 68 / 52 (0.7, 0.5), 4000 96 / 84 (1.0, 0.5); 2400 behind 4800 keys 189 /
+    // 181 (1.0, 0.83), 9600 322 / 328 (1.05, 0.9); 4000 behind 2000 154 / 151 (1.3, 0.67), 4000 211 / 219 (1.5, 0.75); windows: 2400 under 1024 42 / 31
+    // (0.9, 0.79), under 512 27 / 30 (1.05, 0.9), behind 2400 under 2048 75 / 81 (1.2, 1), 4000 under 2048 73 / 79 (1.5, 0.74); 32 on 8, 1200
+    // fresh 34 / 27, behind 1200 under 1024 44 / 50, 2000 fresh under 1024 43 / 48, three segments of 700 33 / 36.
     const int64_t tiles = (num_tokens + p32_rows(qt) - 1) / p32_rows(qt) * (p0.heads / qt), cus = device_cu_count();
-    const bool spread = 2 * (int64_t)max_q_len > num_tokens && (p0.window == 0 || 2 * (int64_t)p0.window > max_q_len) && (p0.chunk == 0 || 2 * (int64_t)p0.chunk > max_q_len);
-    const bool two = max_keys >= 256 && (tiles <= cus || (tiles <= 2 * cus && spread));
+    auto uneven = [&] {                                      // (with max_kv_len, the batch's, for the longest segment's: with longer ones beside it one group is taken)
+      const double n = max_q_len, ctx = max(max_kv_len - max_q_len, 0), most = p0.window > 0 ? fmin(ctx + n, p0.window) : ctx + n;
+      const double rise = fmin(fmax(most - ctx, 0.0), n);                             // rows whose chains grow
+      const double mean = (rise * (ctx + 0.5 * rise) + (n - rise) * most) / (n * most);      // of the longest
+      return 2 * n > num_tokens && (p0.chunk == 0 || 2.0 * p0.chunk > n) && mean <= 0.86 && tiles * mean <= 1.31 * cus;
+    };
+    const bool two = max_keys >= 256 && (tiles <= cus || (tiles <= 2 * cus && uneven()));
 #define P32(QT) (two ? launch_prefill32<QT, FORM, 2>(p0, num_tokens, num_seqs, st) : launch_prefill32<QT, FORM, 1>(p0, num_tokens, num_seqs, st))
     if (qt == 4) P32(4);
     else if (qt == 2) P32(2);

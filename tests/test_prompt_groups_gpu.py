@@ -14,7 +14,8 @@ CASES = [
     (16, 4, [(700, 33)], 16, dict(window=300)), (16, 4, [(0, 700)], 16, dict(window=130, sink=True)), (6, 3, [(0, 449)], 16, dict(gate=1)),
     (3, 3, [(129, 513)], 64, dict(gate=2)), (8, 2, [(0, 1000), (300, 9), (250, 1)], 16, dict(bias=True)), (16, 4, [(0, 640)], 16, dict(chunk=192)),
     (16, 4, [(10, 300)], 8, {}), (16, 4, [(0, 2100)], 16, dict(bias=True)), (32, 8, [(0, 2100)], 16, {}), (32, 8, [(0, 700)] * 4, 16, dict(gate=2)),
-    (16, 4, [(40, 200)], 16, dict(bias=True))]
+    (16, 4, [(40, 200)], 16, dict(bias=True)), (32, 8, [(2200, 1100)], 16, dict(bias=True)), (32, 8, [(5000, 1100)], 16, {}), (32, 8, [(0, 1100)], 16, dict(window=300)),
+    (32, 8, [(0, 1100)], 16, dict(window=400)), (32, 8, [(100, 1100), (3000, 1)], 16, {})]
 
 
 @pytest.mark.parametrize("heads,kv_heads,segs,bs,kw", CASES)
