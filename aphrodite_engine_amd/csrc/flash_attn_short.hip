@@ -249,7 +249,10 @@ static void fa_short_launch_g(const FAParams& p, int batch, int max_query_len, h
   constexpr int rows = 128 / QT;
   constexpr size_t lds = (size_t)GROUPS * 4 * FAS_TILE;
   auto kern = flash_attn_short_kernel<T, QT, LONG, GROUPS>;
-  if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if constexpr (lds > 64 * 1024) {
+    static bool attr_set_dev[APHRO_MAX_DEVICES] = {}; bool& attr_set = attr_set_dev[device_slot()];
+    if (!attr_set) attr_set = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+  }
   const dim3 grid((unsigned)(p.num_heads / QT), (unsigned)((max_query_len + rows - 1) / rows), (unsigned)batch);
   hipLaunchKernelGGL(kern, grid, dim3(256 * GROUPS), lds, st, p);
 }
