@@ -68,17 +68,6 @@ __device__ __forceinline__ void fma_of_lane16(float& p, const f32x4& x, float& q
       : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(e[0]), "v"(e[1]), "v"(e[2]), "v"(e[3]), "n"(I));
 #undef GDC_FMA
 }
-// a + b of the lanes 16 (32) apart, of a in the even sixteens (the first half), of b in the others.
-__device__ __forceinline__ float sum_swap16(float a, float b) {
-  const auto w = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
-  const uint32_t x = w[0], y = w[1];
-  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
-}
-__device__ __forceinline__ float sum_swap32(float a, float b) {
-  const auto w = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
-  const uint32_t x = w[0], y = w[1];
-  return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
-}
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 template <typename F, int... I>
 __device__ __forceinline__ void each16_(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
@@ -220,7 +209,7 @@ __global__ __launch_bounds__(DP * 4) void gd_chunk_prepare_kernel(GDChunk a) {
     // sums over the quarters; sixteens 0 and 2 keep L, 1 and 3 the scores, of tokens i = 0..7 (sixteens 0 and 1) and 8..15
     float sum[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) sum[i] = sum_swap32(sum_swap16(la[i], lb[i]), sum_swap16(la[i + 8], lb[i + 8]));
+    for (int i = 0; i < 8; ++i) sum[i] = swap_add32(swap_add16(la[i], lb[i]), swap_add16(la[i + 8], lb[i + 8]));
     const int i0 = (lg >> 1) * 8;
     if constexpr (HALVES == 2) {
       float* half = tm + (b0 + (lane >> 2)) * GDC_P + (lane & 3) * 8;        // eight numbers of a lane, in rows of the block
