@@ -32,7 +32,9 @@ def _check(out, q, k, v, cu, scale, causal, slopes, dtype, cached=0):
 @pytest.mark.parametrize("heads,kv,lens,causal,alibi,first", [
     (8, 2, [256], True, False, 4096), (8, 2, [257, 65], True, False, 4096), (32, 8, [1024], True, False, 4096), (32, 8, [2048], True, False, 4096),
     (32, 8, [2080], True, False, 4096), (6, 3, [321], False, False, 4096), (3, 3, [449, 1], True, True, 4096), (8, 2, [1100, 40, 700], True, False, 1024),
-    (32, 8, [1500], True, True, 1024), (4, 4, [1090], False, False, 1024), (32, 8, [1200, 1300, 64], True, False, 1024)])
+    (32, 8, [1500], True, True, 1024), (4, 4, [1090], False, False, 1024), (32, 8, [1200, 1300, 64], True, False, 1024),
+    (8, 2, [1057, 31, 32, 33], True, False, 1024), (8, 2, [1057, 31, 32, 33], False, False, 1024), (4, 4, [1089, 127, 128, 129], True, False, 1024),
+    (6, 3, [1025, 63, 64, 65, 1], True, False, 1024), (6, 3, [1025, 63, 64, 65, 1], False, True, 1024)])
 def test_forms(heads, kv, lens, causal, alibi, first, dtype):
     g = torch.Generator(device=DEV).manual_seed(sum(lens) + heads)
     t = sum(lens)

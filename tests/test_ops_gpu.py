@@ -720,7 +720,7 @@ def test_context_attention_fwd_long(ops, kv_cache_dtype, dtype, variant):
     tol = 2e-3 if dtype == torch.float16 else 1.6e-2
     np.testing.assert_allclose(out.float().cpu().numpy(), ref, atol=tol, rtol=tol)
     np.testing.assert_allclose(out_old.float().cpu().numpy(), ref, atol=tol, rtol=tol)
-    # the fourth-generation tile machine over the gathered context (query rows offset by the context length)
+    # the deferred maximum over the gathered context (query rows offset by the context length), from 1024 keys on
     os.environ["APHRO_FA_V4_MIN_KEYS"] = "1024"; ops.reload_env()
     try:
         out4 = torch.empty_like(out)
@@ -1079,14 +1079,13 @@ def test_flash_attn_varlen_sliding_window(ops, dtype, Hq, Hkv, D, left):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal", [True, False])
-def test_flash_attn_varlen_v4_kv_head_placement(ops, dtype, causal):
-    """Fourth-generation prefill kernel (the one that places its workgroups; forced on from 1024 keys) with (sequences x kv heads) a
-    multiple of 8: all query heads / query tiles of one kv head on one XCD.  Ragged lengths around the 256-row and 64-key tile edges, GQA
-    2:1, vs the oracle; the unplaced grid (APHRO_FA_NO_XCD) must give the same bits."""
+def test_flash_attn_varlen_deferred_maximum_tile_edges(ops, dtype, causal):
+    """Prompt attention with a deferred maximum (forced on from 1024 keys): a workgroup's rows are 64 of two query heads of a kv head, a tile 64 keys;
+    lengths on either side, vs the oracle."""
     import os
     rng = np.random.default_rng(5)
     Hq, Hkv, D = 16, 8, 128
-    lens = [1300, 257, 1024, 65]
+    lens = [1089, 63, 1024, 65, 257]
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     T = int(cu[-1])
     qkv = t(rng.standard_normal((T, (Hq + 2 * Hkv) * D)).astype(np.float32) * 0.7, dtype)
@@ -1096,13 +1095,8 @@ def test_flash_attn_varlen_v4_kv_head_placement(ops, dtype, causal):
     os.environ["APHRO_FA_V4_MIN_KEYS"] = "1024"; ops.reload_env()
     try:
         got = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, causal=causal)
-        os.environ["APHRO_FA_NO_XCD"] = "1"; ops.reload_env()
-        plain = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, causal=causal)
     finally:
-        for name in ("APHRO_FA_V4_MIN_KEYS", "APHRO_FA_NO_XCD"):
-            os.environ.pop(name, None)
-        ops.reload_env()
-    assert torch.equal(got, plain)
+        os.environ.pop("APHRO_FA_V4_MIN_KEYS", None); ops.reload_env()
     ref = oa.varlen_causal_attention(q, k, v, cu, scale, causal=causal)
     tol = 2e-3 if dtype == torch.float16 else 1.6e-2
     np.testing.assert_allclose(got.float().cpu().numpy(), ref, atol=tol, rtol=tol)
@@ -1111,14 +1105,13 @@ def test_flash_attn_varlen_v4_kv_head_placement(ops, dtype, causal):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal,alibi", [(True, False), (False, False), (True, True)])
 @pytest.mark.parametrize("Hq,Hkv", [(16, 8), (32, 8), (4, 4)])     # 2:1, the benched Llama-3-8B geometry (4:1), no grouping (GQA 1)
-def test_flash_attn_varlen_v4(ops, dtype, causal, alibi, Hq, Hkv):
-    """Fourth-generation prefill kernel (one wave per SIMD, two 32-row query blocks per wave, defer-max; flash_attn_v4.hip),
-    forced on from 1024 keys: ragged lengths around the 256-row / 64-key tile edges, sequences of one to five tiles next to
-    long ones, GQA, ALiBi (every tile masked), non-causal -- vs the fp64 oracle and vs the kernel below its key count (flash_attn_short.hip)."""
+def test_flash_attn_varlen_deferred_and_exact_maximum(ops, dtype, causal, alibi, Hq, Hkv):
+    """Prompt attention with a deferred maximum (forced on from 1024 keys) and with an exact one over the same prompts: ragged lengths, sequences of one
+    to ten key tiles next to long ones, GQA, ALiBi, non-causal -- vs the fp64 oracle and vs each other."""
     import os
     rng = np.random.default_rng(11 + Hq)
     D = 128
-    lens = [1300, 257, 1024, 65, 1, 640]        # (GQA 4:1 and > 2048 keys: the defer-max test below)
+    lens = [1300, 257, 1024, 65, 1, 640]        # (> 2048 keys: the test of rescaling below)
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     T = int(cu[-1])
     qkv = t(rng.standard_normal((T, (Hq + 2 * Hkv) * D)).astype(np.float32) * 0.7, dtype)
@@ -1130,18 +1123,18 @@ def test_flash_attn_varlen_v4(ops, dtype, causal, alibi, Hq, Hkv):
     os.environ["APHRO_FA_V4_MIN_KEYS"] = "1024"; ops.reload_env()
     try:
         got = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, **kw)
-        os.environ["APHRO_FA_V4_MIN_KEYS"] = str(1 << 30); ops.reload_env()       # flash_attn_short.hip always
-        short = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, **kw)
+        os.environ["APHRO_FA_V4_MIN_KEYS"] = str(1 << 30); ops.reload_env()       # exact at every length
+        exact = ops.flash_attn_varlen(q, k, v, t(cu), max(lens), scale, **kw)
     finally:
         os.environ.pop("APHRO_FA_V4_MIN_KEYS", None); ops.reload_env()
     ref = oa.varlen_causal_attention(q, k, v, cu, scale, causal=causal, alibi_slopes=slopes)
     tol = 2e-3 if dtype == torch.float16 else 1.6e-2
     np.testing.assert_allclose(got.float().cpu().numpy(), ref, atol=tol, rtol=tol)
-    np.testing.assert_allclose(got.float().cpu().numpy(), short.float().cpu().numpy(), atol=tol, rtol=tol)
+    np.testing.assert_allclose(got.float().cpu().numpy(), exact.float().cpu().numpy(), atol=tol, rtol=tol)
 
 
-def test_flash_attn_varlen_v4_defer_max_rescale(ops):
-    """The running maximum of the fourth-generation kernel moves only when a row's new maximum exceeds it by more than 2^8:
+def test_flash_attn_varlen_deferred_maximum_rescale(ops):
+    """A deferred running maximum moves only when a row's new maximum exceeds it by more than 2^8:
     keys whose scores jump far above everything before them (at a tile in the middle, at the diagonal tile, twice in a
     row) force that rescale of the output accumulators; rows that never trigger it sit next to rows that do."""
     import os
