@@ -75,7 +75,7 @@ inline int device_cu_count() {
 // tools/ scripts load through APHRODITE_MI355X_LIB) and is the constant `default` in the product.
 struct Knobs {
   int pa_splits;              // APHRO_PA_SPLITS=<n>: force the in-launch KV split count of decode attention (0: planned)
-  int fa_v4_min_keys;         // APHRO_FA_V4_MIN_KEYS=<n>: prompt attention, the running maximum is deferred from n keys on (default 4096, 1024 at least)
+  int fa_v4_min_keys;         // APHRO_FA_V4_MIN_KEYS=<n>: prompt attention, the running maximum is deferred from n keys on (default 4096, 1024 at least; the name is a former kernel's)
   int fp8_stream_all;         // APHRO_FP8_STREAM_ALL=1: the LDS-DMA FP8 decode kernel on every shape it tiles
   int wna16_stream;           // APHRO_WNA16_STREAM=0: the two-pass resident kernel instead of the single-pass stream kernel
   int wna16_op_no_resident;   // APHRO_WNA16_OP_NO_RESIDENT=1: op-level gptq_gemm as pack + GEMM + reduce (three launches)

@@ -6,16 +6,18 @@
 //     16-byte piece s ^ (j & 15), V's s ^ 4 (j & 3): fragment reads and transposing reads find their banks free.  Keys past the sequence's end are
 //     fetched as zeros (the buffer ends there) and masked.
 //   * the scale is the exponential's FMA; LONG (from 4096 keys on): one step of the online softmax a tile, and the maximum moves only for rows that are
-//     past it by more than 2^8, else a step is 32 keys and its largest probability exactly 1 (error against 64 bits, of the result's size, bf16: exact
-//     steps 0.00206 at 3000 keys and 0.00209 at 8192, LONG 0.00212 and 0.00215, the kernel that it replaced there 0.00215).
+//     past it by more than 2^8, else a step is 32 keys and its largest probability 1 up to the rounding of the scaled maximum, which the FMA's product
+//     does not share; a row's sum and its values take the same probability, before it is 16 bits (error against 64 bits, of the result's size, bf16: steps
+//     of 32 keys 0.00206 at 3000 keys and 0.00209 at 8192, LONG 0.00212 and 0.00215, the kernel that it replaced there 0.00215).
 //   * GROUPS = 2: two such groups of waves take the key tiles in turn, each in LDS of its own, and their sums meet at the end: half the chain.
 // Bound by a tile's chain of steps where a workgroup is alone on its CU (1.2 us: 32 products, the softmax), else by issue and power: at 8192 tokens the
-// matrix pipe is busy 60 % of the SIMDs' cycles, the vector ALUs 53 %, LDS 30 %, at 1.7 GHz.  us before / here, 32 heads on 8, causal: against
+// matrix pipe is busy 60 % of the SIMDs' cycles, the vector ALUs 53 %, LDS 30 %, at 1.7 GHz.  us before / here, 32 heads on 8, causal, bf16, the two in turn
+// on one card (others take 507 to 532 for 8192 tokens, 536 in f16, 491 for numbers a third as large: power): against
 // 64-row workgroups with V transposed number by number, 300 tokens 18.8 / 12.0; against 128-row ones, 1000 tokens 45.5 / 23.6; against one wave
 // a SIMD with 64 rows of the whole register file (deleted), 4096 tokens 174 / 159, 8192 601 / 558, 5000 261 / 210, two of 4096 324 / 276, 8 heads on one
 // 250 / 161.  Below 64 keys the first kernel of flash_attn.hip is the faster (six of 26 tokens 6.1 / 7.4).
 // No gain: loads hidden from hipcc, which otherwise waits for the next tile in front of the transposing reads (three of 1000 tokens 53 / 55); loads between
-// the products (8192 tokens 531 / 534); the next tile's scores between this one's exponentials (530 / 531); row sums as a product with ones (531 / 550).
+// the products (8192 tokens, on a faster card, 531 / 534); the next tile's scores between this one's exponentials (530 / 531); row sums as a product with ones (531 / 550).
 #include "common.h"
 #include "flash_attn_common.h"
 

@@ -132,7 +132,8 @@ bool group_rms_norm_launch(void* out, int64_t out_stride, const float* x, const 
 
 // n / (1 + e^-z): the reciprocal's product, one correction and the hardware's rules for zeros, infinities and NaN, without a division's scaling (ten
 // instructions for seven), and with a division's bits wherever n is not scaled: the reciprocal is a quarter's, as that of 2^126 and more would be
-// taken for zero.  Where the vector units bound: decay memories of 4096 tokens, 16 heads, 86.6 -> 83.9 us, a convolution of 2024 rows 18.5 -> 17.6.
+// taken for zero.  Every 257th of all floats: a division's bits.  Where the vector units bound: decay memories of 4096 tokens, 16 heads, 86.6 -> 83.9 us, a
+// convolution of 2024 rows 18.5 -> 17.6, with both sides scaled (six instructions, two bits less below 4.7e-38; the seventh: 88.6 -> 88.9 on one card).
 __device__ __forceinline__ float over_1_exp_f(float n, float z) {
   const float d = 1.0f + __expf(-z), r = 0.25f * __builtin_amdgcn_rcpf(0.25f * d), q = n * r;
   return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, d, n), r, q), d, n);
@@ -144,7 +145,8 @@ __device__ __forceinline__ float gelu_tanh_f(float z) {
   return 0.5f * z * (1.0f + tanhf(u));
 }
 // log(1 + e^z) = max(z, 0) + 2 atanh(h / 2), h = x / (1 + x / 2), x = e^-|z|: h in two numbers, atanh by its series in h^2 (coefficients fitted by least
-// squares over h <= 2 / 3, 1e-10), the sum with what its first step rounds away (z = infinity leaves NaN there: -1 for it).  No branch.
+// squares over h <= 2 / 3, 1e-10), the sum with what its first step rounds away (z = infinity leaves NaN there: -1 for it).  No branch.  Error against 64 bits, of the result, x 2^-24, largest and root mean square, log1pf(expf(z)) / here: over
+// [-20, 20] 2.26, 0.495 / 2.26, 0.491; [-1, -0.1] 1.80, 0.549 / 1.88, 0.551; [-0.1, 0.1] 1.66, 0.528 / 1.49, 0.479; [0.1, 1] 1.61, 0.517 / 1.39, 0.464.
 __device__ __forceinline__ float softplus_f(float z) {
   const float x = expf(-fabsf(z)), d = fmaf(x, 0.5f, 1.f), dl = fmaf(x, 0.5f, 1.f - d), r = __builtin_amdgcn_rcpf(d);
   const float h = x * r, hl = fmaf(-h, dl, fmaf(-h, d, x)) * r, t = h * h;

@@ -7,20 +7,22 @@
 //   3. om_chunk_out:    o of every chunk -- all chunks at once
 // and mLSTM's running maximum (a recurrence of its own, one number per head and token) is worked out ahead of them by om_gates.
 //
-// Everything is fp32, products on v_mfma_f32_16x16x4_f32 (what enters the recurrence is fp32 and stays so); G is summed in 64 bits, so that a small decay keeps its digits behind a large one.
-// Only the differences G_i - G_j <= 0 are exponentiated: nothing overflows however strong the decay.
+// What enters the recurrence is fp32 and stays so.  Decay memories, and inputs that are not bf16, multiply on v_mfma_f32_16x16x4_f32; mLSTM's and the state
+// space's bf16 queries, keys and values go to the 16-bit units as they are, against fp32 factors in three bf16 parts (the *16 kernels, several chunks
+// of a segment to a workgroup: how many goes by all tokens of the call, so that a segment's last bits may differ with what runs beside it).  G is
+// summed in 64 bits, so that a small decay keeps its digits behind a large one.  Only the differences G_i - G_j <= 0 are exponentiated: nothing overflows
+// however strong the decay.
 //
 // What bounds it: the fp32 products (the matrix pipe is busy half of the time in launches 1 and 3) and the states between the chunks
 // (written once, read and written once, read once: dim x vdim x 4 bytes a chunk and head).  A scan is bound by the latency of its
-// token chain.  One portion of 4096 tokens, scan -> chunks: decay 8 x 64 x 128 1106 -> 60 us, mLSTM 4 x 128 x 256 2170 -> 113 us, state
-// space 64 x 128 x 64 1476 -> 274 us (128 heads: 1482 -> 575 us).  mLSTM's and the state space's bf16 inputs go to the 16-bit units, several chunks of a
-// segment to a workgroup (the *16 kernels).
+// token chain.  One portion of 4096 tokens, scan -> chunks in fp32 -> here: decay 8 x 64 x 128 1106 -> 60 us, mLSTM 4 x 128 x 256 2170 -> 113 -> 64,
+// state space 64 x 128 x 64 1476 -> 274 -> 103 (128 heads: 1482 -> 575 -> 211).
 // Outputs lie as the products leave them: scores as K Q^T and results as V^T P^T, so that a score's registers are the next product's
 // operand and a lane holds four neighbouring value columns of one token.  Row pitches are 4 floats over a multiple of 32: the
 // eight lanes that a 16-byte LDS access serves at a time fall on all 32 banks.  The states lie in fragments: as rows of DP, the address unit took four times
 // as long over a load (state space 64 heads, 600 / 2000 / 4096 tokens 51 / 73 / 116 -> 46 / 67 / 111 us, decay 16 x 64 x 128, 4096 tokens 92 -> 89).  A
 // third of a launch is the way to its first numbers; with a segment's place beside its length, prefix sums without LDS and a fixed decay's
-// as multiples 42 / 66 / 103, 87.
+// as multiples 42 / 66 / 103, 87 (89 since silu keeps the last places of its smallest numbers, on a card that took 88.6 before).
 #include "outer_memory.h"
 #include "chunked_scan.h"
 

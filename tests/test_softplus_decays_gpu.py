@@ -28,8 +28,8 @@ def test_decays_over_the_range_of_their_gates(monkeypatch, chunks, channel):
         want = ln.exp().expand(H, d)
         got = state[0].double().cpu()
         assert torch.equal(got, got[:, :, :1].expand_as(got))
-        # g = e^ln: an error of (softplus 2.1, exp of a_log 1.5, the product 0.5) x 2^-24 of ln, 1.5 x 2^-24 of g; below 2^-120 fp32 itself runs out
-        bound = want * ((4.1 * ln.abs()).clamp(max=1e3) + 1.5) * 2.0 ** -24 + 2.0 ** -140
+        # g = e^ln: an error of (softplus 2.3, exp of a_log 1.5, the product 0.5) x 2^-24 of ln, 1.5 x 2^-24 of g; below 2^-120 fp32 itself runs out
+        bound = want * ((4.3 * ln.abs()).clamp(max=1e3) + 1.5) * 2.0 ** -24 + 2.0 ** -140
         assert (got[:, :, 0] - want).abs().le(bound).all(), (rate, ((got[:, :, 0] - want).abs() / bound).max())
 
 
