@@ -784,3 +784,12 @@ def test_when_the_delta_rule_runs_in_chunks():
     assert pay(2024, 25, 2000, 16, 128, 128, True)                       # a portion with decoded tokens beside it
     assert pay(2228, 28, 551, 32, 128, 128, True)                        # ... and four: the rows are not portions that end in half a chunk
     assert not pay(4096, 16, 256, 48, 64, 64, True) and not pay(8192, 32, 256, 32, 128, 128, False) and not pay(512, 4, 128, 32, 128, 128, False)
+
+
+def test_moe_combine_of_no_columns_is_refused():
+    """An error to the caller (and no division by the threads of no columns), as a call without tokens is none."""
+    from aphrodite_engine_amd import _lib
+    for columns in (0, -4, 6):
+        rc = _lib.lib().aphro_moe_combine(256, 256, 1, 16, 256, 256, 1, 1, columns, _lib.F16, None)
+        assert rc != _lib.OK and b"moe_combine" in _lib.lib().aphro_last_error()
+    assert _lib.lib().aphro_moe_combine(256, 256, 1, 16, 256, 256, 0, 1, 4096, _lib.F16, None) == _lib.OK
