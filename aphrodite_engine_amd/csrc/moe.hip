@@ -752,7 +752,6 @@ extern "C" int aphro_moe_combine(void* out, const float* slabs, int nslab, int64
   APHRO_CHECK(dtype == APHRO_F16 || dtype == APHRO_BF16, "moe_combine: dtype must be f16 or bf16");
   APHRO_CHECK(N > 0 && N % 4 == 0 && nslab >= 1, "moe_combine: bad shape");
   if (num_tokens == 0) return APHRO_OK;
-  APHRO_CHECK((N / 4 + 255) / 256 <= 65535, "moe_combine: rows are too long");
   if (dtype == APHRO_F16) launch_combine<Half>(out, slabs, nslab, m_pad * N, inv_pos, topk_weights, num_tokens, topk, N, (hipStream_t)stream);
   else launch_combine<BFloat>(out, slabs, nslab, m_pad * N, inv_pos, topk_weights, num_tokens, topk, N, (hipStream_t)stream);
   APHRO_LAUNCH_CHECK();

@@ -25,3 +25,10 @@ def test_combine(tokens, topk, nslab, n, dtype):
     for k in range(topk):
         acc = acc + (y[inv.view(tokens, topk)[:, k].long()] * w[:, k:k + 1]).to(dtype).float()
     assert torch.equal(ops.moe_combine(slabs, inv, w, dtype), acc.to(dtype))
+
+
+def test_rows_of_more_workgroups_than_16_bits_count():
+    n = 4 * 256 * 65536 + 4
+    slabs = torch.arange(n, dtype=torch.float32, device=DEV).remainder_(2048).view(1, 1, n)
+    out = ops.moe_combine(slabs, torch.zeros(1, dtype=torch.int32, device=DEV), torch.ones(1, 1, device=DEV), torch.float16)
+    assert torch.equal(out, slabs[0].half())
