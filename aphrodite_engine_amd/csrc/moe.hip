@@ -547,34 +547,48 @@ __global__ __launch_bounds__(256) void moe_route_gather_kernel(
 // out[t][:] = sum_k round_T(w[t][k] * y[pos(t, k)][:])   (fused_moe.py:520-542: routed weight applied to
 // the second GEMM's fp32 result, cast, then summed over top-k).  y = sum of `nslab` fp32 slabs
 // [nslab][m_pad][N] (split-K partials of the expert GEMM) -- rounded once, after the weight.
-// A thread has four columns of one token; the slabs of two choices are on their way together (NS of them a choice, known here: with a count known
-// at run time only every load waited for the one before it, and a workgroup went over the whole row: 32 tokens of 4096 columns, two choices of four slabs,
-// 10.0 -> 4.8 us; 3000 tokens, two of two, 40 both ways: 196 MB of slabs at the copy rate).
-template <typename T, int NS>
+// A thread has four columns of one token; the slabs of U choices are on their way together (NS of them a choice, known here, or 0: any number, four at a time.
+// With a count known at run time only every load waited for the one before it, and a workgroup went over the whole row: 32 tokens of 4096 columns, two
+// choices of four slabs, 10.0 -> 4.8 us; 3000 tokens, two of two, 40 both ways: 196 MB of slabs at the copy rate).  U is one where there is one choice (5725
+// tokens of 512 columns, seven slabs: 25.5 us where it was read twice and a slab behind the other, 15.9) and four for many choices of few slabs.
+template <typename T, int NS, int U>
 __global__ __launch_bounds__(256) void moe_combine_kernel(typename T::storage* __restrict__ out, const float* __restrict__ slabs,
                                                           int nslab, int64_t slab_stride, const int32_t* __restrict__ inv_pos,
                                                           const float* __restrict__ topk_weights, int topk, int N) {
   const int tok = blockIdx.x, c0 = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
   if (c0 >= N) return;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int kk = 0; kk < topk; kk += 2) {
-    f32x4 y[2][NS > 0 ? NS : 1];
-    float w[2];
+  for (int kk = 0; kk < topk; kk += U) {
+    f32x4 y[U][NS > 0 ? NS : 1];
+    float w[U];
+    const float* p0[U];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int k1 = kk + u < topk ? kk + u : kk;
-      const float* p0 = slabs + (size_t)inv_pos[(size_t)tok * topk + k1] * N + c0;
+      p0[u] = slabs + (size_t)inv_pos[(size_t)tok * topk + k1] * N + c0;
       w[u] = topk_weights[(size_t)tok * topk + k1];
-      if constexpr (NS > 0) {
 #pragma unroll
-        for (int s = 0; s < NS; ++s) y[u][s] = *reinterpret_cast<const f32x4*>(p0 + s * slab_stride);
-      } else {
-        y[u][0] = *reinterpret_cast<const f32x4*>(p0);
-        for (int s = 1; s < nslab; ++s) y[u][0] += *reinterpret_cast<const f32x4*>(p0 + s * slab_stride);
+      for (int s = 0; s < (NS > 0 ? NS : 1); ++s) y[u][s] = *reinterpret_cast<const f32x4*>(p0[u] + s * slab_stride);
+    }
+    if constexpr (NS == 0) {
+      int s = 1;
+      for (; s + 4 <= nslab; s += 4) {
+        f32x4 x[U][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[u][i] = *reinterpret_cast<const f32x4*>(p0[u] + (s + i) * slab_stride);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) y[u][0] += x[u][i];
       }
+      for (; s < nslab; ++s)
+#pragma unroll
+        for (int u = 0; u < U; ++u) y[u][0] += *reinterpret_cast<const f32x4*>(p0[u] + s * slab_stride);
     }
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       if (kk + u >= topk) break;
 #pragma unroll
       for (int s = 1; s < NS; ++s) y[u][0] += y[u][s];
@@ -587,21 +601,29 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(typename T::storage* _
   for (int j = 0; j < 4; ++j) o[j] = T::from_f32(acc[j]);
 }
 
+template <typename T, int NS>
+static void launch_combine_n(void* out, const float* slabs, int nslab, int64_t slab_stride, const int32_t* inv_pos, const float* topk_weights,
+                             int64_t num_tokens, int topk, int64_t N, hipStream_t st) {
+  const int threads = N / 4 >= 256 ? 256 : (int)((N / 4 + 63) / 64 * 64);
+  const dim3 grid((unsigned)num_tokens, (unsigned)((N / 4 + threads - 1) / threads));
+#define APHRO_COMBINE(U) \
+  hipLaunchKernelGGL((moe_combine_kernel<T, NS, U>), grid, dim3(threads), 0, st, (typename T::storage*)out, slabs, nslab, slab_stride, inv_pos, \
+                     topk_weights, topk, (int)N)
+  if (topk == 1) APHRO_COMBINE(1);
+  else if ((NS == 1 || NS == 2) && topk >= 4) APHRO_COMBINE((NS == 1 || NS == 2) ? 4 : 2);
+  else APHRO_COMBINE(2);
+#undef APHRO_COMBINE
+}
+
 template <typename T>
 static void launch_combine(void* out, const float* slabs, int nslab, int64_t slab_stride, const int32_t* inv_pos, const float* topk_weights,
                            int64_t num_tokens, int topk, int64_t N, hipStream_t st) {
-  const int threads = N / 4 >= 256 ? 256 : (int)((N / 4 + 63) / 64 * 64);
-  const dim3 grid((unsigned)num_tokens, (unsigned)((N / 4 + threads - 1) / threads));
-#define APHRO_COMBINE(NS) \
-  hipLaunchKernelGGL((moe_combine_kernel<T, NS>), grid, dim3(threads), 0, st, (typename T::storage*)out, slabs, nslab, slab_stride, inv_pos, \
-                     topk_weights, topk, (int)N)
   switch (nslab) {
-    case 1: APHRO_COMBINE(1); break;
-    case 2: APHRO_COMBINE(2); break;
-    case 4: APHRO_COMBINE(4); break;
-    default: APHRO_COMBINE(0); break;
+    case 1: launch_combine_n<T, 1>(out, slabs, nslab, slab_stride, inv_pos, topk_weights, num_tokens, topk, N, st); break;
+    case 2: launch_combine_n<T, 2>(out, slabs, nslab, slab_stride, inv_pos, topk_weights, num_tokens, topk, N, st); break;
+    case 4: launch_combine_n<T, 4>(out, slabs, nslab, slab_stride, inv_pos, topk_weights, num_tokens, topk, N, st); break;
+    default: launch_combine_n<T, 0>(out, slabs, nslab, slab_stride, inv_pos, topk_weights, num_tokens, topk, N, st); break;
   }
-#undef APHRO_COMBINE
 }
 
 }  // namespace aphro

@@ -10,7 +10,7 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("tokens,topk,nslab,n", [(1, 1, 1, 4), (3, 2, 2, 1020), (32, 2, 4, 4096), (5, 3, 3, 1028), (2, 5, 4, 2052), (17, 8, 7, 260),
-                                                 (65, 3, 1, 1024), (300, 2, 2, 512)])
+                                                 (65, 3, 1, 1024), (300, 2, 2, 512), (9, 1, 7, 512), (9, 2, 6, 512), (9, 1, 5, 516), (40, 6, 2, 512), (7, 5, 1, 2052)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_combine(tokens, topk, nslab, n, dtype):
     g = torch.Generator(device=DEV).manual_seed(tokens * n + nslab)
