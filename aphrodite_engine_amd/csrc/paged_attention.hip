@@ -1385,6 +1385,31 @@ static bool split_workspace(size_t groups, size_t floats, hipStream_t st, SplitW
   return true;
 }
 
+// Four waves a workgroup, or eight: eight waves of 164 registers are all that a CU holds, of four three workgroups: where there are more of them than CUs, a
+// workgroup's start (three dependent loads) and merge then lie behind the others' streams.  us a decode step of four layers, 8 kv heads, 16-bit keys, eight
+// waves / four: 34 sequences of 300 543 / 526, 33 / 40 / 65 of 1040 618 / 605, 631 / 625, 819 / 800, 64 of 400 606 / 593.
+// A long sequence of four waves takes longer where it ends a launch, though, and lengths are not known here.  Up to a quarter more workgroups than CUs the
+// plain form keeps eight above 640 keys (a launch, lengths of 0.3 to 1 times 1200, 33 sequences 23.1 / 27.0, even ones 32.4 / 30.3; of 800, seven batches 0.86 to
+// 1.06); the fused form from 1281 on (a step, 33 to 64 sequences of 450 to 1800 keys 0.95 to 0.99, of 1000 0.98 to 1.01); its form over FP8
+// keys (127 registers: two workgroups of eight) always, 64 of 400 561 / 566.  Heads of 64 (three workgroups of eight waves a CU) keep eight up to
+// three workgroups a CU: 17 to 32 sequences, 16 kv heads, 300 to 1500 keys 0.77 to 1.06 of eight's speed.  Heads of 256 gain always (1.1 to 1.4).
+static bool pa_four_waves(int64_t wgs, int head_size, int max_seq_len, bool fused, bool fused_fp8) {
+  const int64_t cus = device_cu_count();
+  if (wgs <= cus || fused_fp8) return false;
+  if (head_size > 128) return true;
+  if (head_size <= 64) return wgs >= 3 * cus;
+  return fused ? max_seq_len <= 1280 : max_seq_len <= 640 || 4 * wgs >= 5 * cus;
+}
+
+// From three workgroups a CU on they do not all run at once, and below that a long one may start late: the sequences go from the longest to the shortest
+// (pa_by_length), so that a launch does not end on a long one.  150 sequences of 375 to 1500, a layer, eight waves / four / longest first 115 / 111 / 102 us
+// (5.0 -> 5.7 TB/s); 48 of 360 to 1200 31.7 / 33.3 / 29.1.  Finding a sequence's rank is 2 us of a launch: up to 512 keys that is more than it gives
+// (150 of 150 19.0 / 22.2 in any order / longest first, of 45 to 150 15.7 / 16.9; 97 of 400 even 0.95, ragged 1.11), below three workgroups a CU up to 1023.
+static bool pa_longest_first(int64_t wgs, int max_seq_len) {
+  const int64_t cus = device_cu_count();
+  return wgs >= 3 * cus ? max_seq_len > 512 : 4 * wgs >= 5 * cus && max_seq_len >= 1024;
+}
+
 static int paged_attention_impl(void* out, void* out_packed, float* exp_sums, float* max_logits, void* tmp_out,
                                      const void* query, const void* key_cache, const void* value_cache,
                                      int num_seqs, int num_heads, int num_kv_heads, int head_size,
@@ -1445,15 +1470,11 @@ static int paged_attention_impl(void* out, void* out_packed, float* exp_sums, fl
   p.nsplit = 0; p.extra = 0; p.split_scratch = nullptr; p.split_counter = nullptr;
   if (partition_size == 0) {
     p.partition_size = 0; p.max_parts = 0; p.write_direct = 1;
-    // v1 form: one workgroup per (seq, kv head) walks the whole sequence.  Eight waves of 164 registers are all that a CU holds, of four three
-    // workgroups: where there are more of them than CUs, a workgroup's start (three dependent loads) and merge then lie behind the others' streams.
-    // us a decode step of four layers, 8 kv heads, 16-bit keys, eight waves / four: 34 sequences of 300 543 / 526, 33 / 40 / 65 of 1040 618 / 605, 631 /
-    // 625, 819 / 800, 64 of 400 606 / 593; the fused forms over FP8 keys (127 registers: two workgroups of eight) keep eight, 64 of 400 561 / 566.
-    // From three workgroups a CU on they do not all run at once, and the sequences go from the longest to the shortest (pa_by_length), so that a
-    // launch does not end on a long one: 150 sequences of 375 to 1500, a layer, eight waves / four / longest first 115 / 111 / 102 us (5.0 -> 5.7 TB/s).
-    const int64_t wgs = (int64_t)num_seqs * num_kv_heads, cus = device_cu_count();
-    nw = max_seq_len > 256 && (wgs <= cus || (qkv_slabs != nullptr && kv_dtype != APHRO_KV_AUTO)) ? 8 : 4;
-    if (qkv_slabs == nullptr && wgs >= 3 * cus && num_seqs <= PA_MAX_DEALT) p.partition_size = -1;
+    // v1 form: one workgroup per (seq, kv head) walks the whole sequence, of four waves up to 256 keys and where pa_four_waves says so.
+    const bool fused = qkv_slabs != nullptr;
+    const int64_t wgs = (int64_t)num_seqs * num_kv_heads;
+    nw = max_seq_len <= 256 || pa_four_waves(wgs, head_size, max_seq_len, fused, fused && kv_dtype != APHRO_KV_AUTO) ? 4 : 8;
+    if (!fused && nw == 4 && num_seqs <= PA_MAX_DEALT && pa_longest_first(wgs, max_seq_len)) p.partition_size = -1;
     while (nw > 4 && (size_t)nw * (32 + p.nh_lds * head_size) * 4 > 96 * 1024) nw >>= 1;
     // ... or nsplit workgroups share it (pa_plan).  APHRO_PA_SPLITS=n forces n (1 = off).
     const size_t groups = (size_t)num_seqs * num_kv_heads;

@@ -1,5 +1,5 @@
-"""Decode attention of more (sequence, kv head) pairs than the CUs hold at once: the sequences go from the longest to the shortest, in workgroups of
-four waves -- against attention in fp32 over the gathered pages."""
+"""Decode attention of more (sequence, kv head) pairs than CUs: workgroups of four waves or eight, the sequences in order or from the longest to the shortest, on
+both sides of where each is taken -- against attention in fp32 over the gathered pages."""
 import pytest
 import torch
 
@@ -27,7 +27,9 @@ def _cache(x, width):                                        # [n, pages, hkv, B
 
 @pytest.mark.parametrize("kind,n,hkv,rep,d,longest", [
     ("ragged", 97, 8, 4, 128, 700), ("ragged", 256, 3, 8, 128, 333), ("empty", 130, 8, 4, 128, 290), ("tied", 200, 4, 2, 64, 500),
-    ("even", 96, 8, 4, 128, 257), ("ragged", 257, 4, 1, 128, 300), ("ragged", 100, 8, 2, 256, 400), ("tied", 65, 12, 20, 128, 300)])
+    ("even", 96, 8, 4, 128, 257), ("ragged", 257, 4, 1, 128, 300), ("ragged", 100, 8, 2, 256, 400), ("tied", 65, 12, 20, 128, 300),
+    ("ragged", 256, 3, 8, 128, 533), ("empty", 130, 8, 4, 128, 590), ("tied", 200, 4, 2, 64, 700), ("even", 96, 8, 4, 128, 513), ("ragged", 100, 8, 2, 256, 600),
+    ("empty", 48, 8, 4, 128, 1100), ("ragged", 39, 8, 1, 128, 700), ("ragged", 40, 8, 2, 64, 600), ("ragged", 41, 8, 4, 128, 1023)])
 @pytest.mark.parametrize("dtype,kv", [(torch.float16, "auto"), (torch.bfloat16, "auto"), (torch.float16, "fp8")])
 def test_longest_first(kind, n, hkv, rep, d, longest, dtype, kv):
     g = torch.Generator(device=DEV).manual_seed(n + longest)
