@@ -340,11 +340,18 @@ struct OMGroup {
   int64_t row0;                        // its first token
 };
 __host__ __device__ __forceinline__ int om_key_heads(const OuterMemory& p) { return p.mode == 2 ? p.qk_heads : p.heads; }
+// A few pairs that do not come out even on the eight XCDs (a key head for all heads, or two): each is divided among the XCDs.  us, one key head for 128 heads
+// of 128 x 64, 277 tokens (two or three groups, of which an XCD had one each) 121 -> 87, for
+// 64 heads 219 tokens 34.6 -> 27.7, 2725 beside 280 in 25 short segments 137 -> 121.
+__host__ __device__ __forceinline__ bool om_split_pairs(int64_t pairs, int subs) { return pairs < 64 && pairs % 8 != 0 && subs >= 8; }
 __device__ __forceinline__ bool locate_group(const OMChunk& a, OMGroup& w) {
   const OuterMemory& p = a.p;
   const int key_heads = om_key_heads(p), heads = p.heads / key_heads, blocks = (p.vdim + OMC_COLS - 1) / OMC_COLS;
-  const int idx = blockIdx.x >> 3, pair = idx / (heads * blocks) * 8 + (blockIdx.x & 7), sub = idx % (heads * blocks);
-  if (pair >= a.span * key_heads) return false;
+  const int idx = blockIdx.x >> 3, per = om_split_pairs(a.span * key_heads, heads * blocks) ? (heads * blocks + 7) / 8 : heads * blocks;
+  int pair = idx / per, sub = idx % per;
+  if (per < heads * blocks) sub += (int)(blockIdx.x & 7) * per;
+  else pair = pair * 8 + (int)(blockIdx.x & 7);
+  if (pair >= a.span * key_heads || sub >= heads * blocks) return false;
   w.x = pair % a.span, w.hk = pair / a.span, w.h = w.hk * heads + sub / blocks, w.c0 = sub % blocks * OMC_COLS;
   ChunkPlace at;
   if (!locate_chunk(a.chunk0 + w.x, p, a.min_len, at, a.group * CHUNK) || at.slot < 0 || at.slot >= p.num_slots) return false;
@@ -977,7 +984,8 @@ static void om_chunk_launch(OMChunk a, int64_t chunks) {
   const OuterMemory& p = a.p;
   const dim3 grid((unsigned)a.span, (unsigned)p.heads, (unsigned)((p.vdim + OMC_COLS - 1) / OMC_COLS));
   const unsigned pairs = (unsigned)a.span * (unsigned)om_key_heads(p);
-  const dim3 grid16((pairs + 7) / 8 * 8 * (unsigned)(p.heads / om_key_heads(p)) * grid.z);
+  const unsigned subs = (unsigned)(p.heads / om_key_heads(p)) * grid.z;
+  const dim3 grid16(om_split_pairs(pairs, (int)subs) ? pairs * ((subs + 7) / 8) * 8 : (pairs + 7) / 8 * 8 * subs);
   const unsigned items = (unsigned)a.vpad * (DP / 4) + (MODE == 1 ? DP : 0);
   if (MODE == 1) hipLaunchKernelGGL((om_gates_kernel<T>), dim3((unsigned)p.num_seqs, (unsigned)p.heads), dim3(1024), 0, p.stream, a);
   for (; a.chunk0 < chunks; a.chunk0 += a.span) {
