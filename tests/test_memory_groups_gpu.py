@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 # (mode, heads, key heads, d, e): chunks * heads * blocks of 64 columns makes the group
 CASES = [(2, 64, 8, 100, 64, [597]), (2, 96, 4, 64, 60, [449]), (1, 16, 0, 128, 256, [610]),                      # two
          (2, 64, 8, 128, 64, [1281, 1, 65, 33]), (2, 80, 1, 40, 130, [400, 2, 129]), (1, 24, 0, 72, 200, [513, 256, 1]),    # four
-         (2, 64, 2, 128, 256, [1089]), (2, 64, 8, 64, 250, [513, 512, 40]), (1, 64, 0, 64, 256, [577, 1, 450])]      # eight
+         (2, 64, 2, 128, 256, [1089]), (2, 64, 8, 64, 250, [513, 512, 40]), (1, 64, 0, 64, 256, [577, 1, 450]),      # eight
+         (2, 12, 1, 64, 64, [700]), (2, 27, 3, 64, 40, [130, 70])]                                               # few key heads: a pair's heads over the XCDs
 
 
 @pytest.mark.parametrize("case", CASES)
